@@ -1,0 +1,666 @@
+"""What is measured of this engine: the steps that a program which serves requests has it do.
+
+A case is one model (a named configuration, perhaps with fewer layers: same layer sizes), an element type and a pass:
+
+- ``"step"``: one call of the step function on requests that are there already: ``decode`` requests bring one token each
+  behind contexts of ``context_lo`` to ``context_hi`` tokens, ``prompts`` requests bring portions of ``prompt_lo`` to
+  ``prompt_hi`` tokens behind ``behind`` cached ones. Afterwards the requests are taken back to where they stood, so a pass
+  can be repeated (only models without state and windows can be).
+- ``"serve"``: prompts come in, in one step, ``steps`` single-token steps follow, and the requests end. The tokens are given.
+- ``"generate"``: ``LLM.generate``, greedy: the scheduler, the sampler and the steps that it issues ahead.
+
+The first two return the float32 logits of every place that a program would sample from. Models with routed experts are
+left out: in bfloat16 any other order of a sum sends some token to another expert, and results of two correct programs
+can then not be compared. The layers of such a design whose feed-forward is dense are in.
+
+Token ids and weights are random, as in ``bench.py``: N(0, 0.02^2), norm weights 1 + N(0, 0.1^2), and the other parameters
+as the parts themselves draw them; but, as in trained models, what the layers add to the stream does not drown it: the output
+projections are drawn smaller by the root of twice the number of layers (norms behind a sublayer: a quarter), and in
+bfloat16 the embedding's rows have unit size. (Otherwise the stream is the last layers' rounding several times over, and two
+correct programs differ by 4 per cent. In 32 bits, where that does not matter, the rows stay small: a tied head would
+else hold the last token for the likeliest next one.)
+"""
+import copy
+import math
+import random
+
+import numpy as np
+import torch
+
+from nanohybrid_vlm_amd import LLM, SamplingParams
+from nanohybrid_vlm_amd.config.registry import named_shapes, resolve_architecture
+from nanohybrid_vlm_amd.engine.runner import StepEntry
+from nanohybrid_vlm_amd.parts.model import DecoderModel
+
+DEVICE = "cuda:0"
+DTYPES = {"bfloat16": torch.bfloat16, "float32": torch.float32}
+
+
+def _case(model, layers, mode, dtype="bfloat16", page=256, decode=0, context_lo=0, context_hi=0, prompts=0, prompt_lo=0, prompt_hi=0,
+          behind=0, steps=0):
+    return {"model": model, "layers": layers, "mode": mode, "dtype": dtype, "page": page, "decode": decode, "context_lo": context_lo,
+            "context_hi": context_hi, "prompts": prompts, "prompt_lo": prompt_lo, "prompt_hi": prompt_hi, "behind": behind, "steps": steps}
+
+
+def listed():
+    cases = [
+        # one user chatting with the smallest model: every launch of the step shows
+        ("one request, 0.6b", _case("0.6b", 28, "step", decode=1, context_lo=150, context_hi=150)),
+        # the benchmark's step: a few users after prompts of one length (a third of the layers)
+        ("8 requests, 8b", _case("8b", 12, "step", decode=8, context_lo=2048, context_hi=2048)),
+        # a loaded server: many users, every context another length
+        ("64 requests, 8b", _case("8b", 12, "step", decode=64, context_lo=97, context_hi=2048)),
+        # the benchmark's prompt
+        ("prompt of 2048, 8b", _case("8b", 12, "step", prompts=1, prompt_lo=2048, prompt_hi=2048)),
+        # continuous batching: portions of ragged prompts beside requests that decode
+        ("mixed, 8b", _case("8b", 12, "step", decode=13, context_lo=60, context_hi=1700, prompts=3, prompt_lo=90, prompt_hi=901)),
+        # a long document comes in by portions: attention over what is there already
+        ("portion at 14336, 8b", _case("8b", 12, "step", prompts=1, prompt_lo=2048, prompt_hi=2048, behind=14336)),
+        # a short question to a model of medium size, small pages, other users decoding: a step that replays a graph
+        ("short mixed, 4b", _case("4b", 12, "step", page=16, decode=4, context_lo=40, context_hi=700, prompts=1, prompt_lo=75, prompt_hi=75)),
+        # the 32-bit path: a prompt whose logits are compared with another implementation's
+        ("prompt of 517, 0.6b, 32 bits", _case("0.6b", 14, "step", dtype="float32", prompts=1, prompt_lo=517, prompt_hi=517)),
+        # the 32-bit path through the whole program: prompts to tokens
+        ("generate, 0.6b, 32 bits", _case("0.6b", 14, "generate", dtype="float32", prompts=6, prompt_lo=9, prompt_hi=130, steps=24)),
+        # attention beside a gated delta rule: prompts come in
+        ("prompts, pevazen", _case("pevazen-1b", 8, "serve", prompts=2, prompt_lo=701, prompt_hi=1500)),
+        # linear recurrences and windowed attention: short prompts, then decoding
+        ("serve 16, zigelorn", _case("zigelorn-1b", 8, "serve", prompts=16, prompt_lo=20, prompt_hi=200, steps=12)),
+        # attention over a cached latent and with a bias by distance: prompts beyond the window, then decoding
+        ("serve 5, gabelorn", _case("gabelorn-1b", 8, "serve", prompts=5, prompt_lo=150, prompt_hi=1300, steps=6)),
+    ]
+    return [dict(case, name=name) for name, case in cases]
+
+
+def draw(rng):
+    def spread(lo, hi):                                   # evenly over the logarithm
+        return min(hi, max(lo, int(round(math.exp(rng.uniform(math.log(lo), math.log(hi)))))))
+
+    page = rng.choice((16, 64, 256, 256))
+    kind = rng.choices(("decode", "prompt", "mixed", "portion", "float", "pevazen", "zigelorn", "gabelorn"),
+                       (3, 2, 2, 1, 2, 2, 1, 1))[0]
+    model, layers = rng.choice((("0.6b", 28), ("1.7b", rng.randint(6, 20)), ("4b", rng.randint(6, 16)), ("8b", rng.randint(4, 12))))
+    if kind == "decode":
+        n = spread(1, 64)
+        hi = spread(16, min(4000, 60000 // n))
+        return _case(model, layers, "step", page=page, decode=n, context_lo=spread(8, hi), context_hi=hi)
+    if kind == "prompt":
+        n = rng.choice((1, 1, 1, 2, 3, 5))
+        hi = spread(8, 3000 // n)
+        return _case(model, layers, "step", page=page, prompts=n, prompt_lo=spread(4, hi) if hi > 4 else hi, prompt_hi=hi)
+    if kind == "mixed":
+        n, hi, p = spread(1, 40), spread(30, 1500), rng.randint(1, 3)
+        top = spread(8, 2000 // p)
+        return _case(model, layers, "step", page=page, decode=n, context_lo=spread(8, hi), context_hi=hi, prompts=p,
+                     prompt_lo=spread(4, top), prompt_hi=top)
+    if kind == "portion":
+        n = spread(100, 2000)
+        return _case(model, layers, "step", page=page, prompts=1, prompt_lo=n, prompt_hi=n, behind=spread(500, 14000))
+    if kind == "float":
+        model, layers = rng.choice((("0.6b", rng.randint(4, 14)), ("1.7b", rng.randint(2, 6))))
+        way = rng.choice(("prompt", "decode", "generate"))
+        if way == "prompt":
+            n = spread(5, 500)
+            return _case(model, layers, "step", dtype="float32", page=page, prompts=1, prompt_lo=n, prompt_hi=n)
+        if way == "decode":
+            n, hi = spread(1, 24), spread(10, 400)
+            return _case(model, layers, "step", dtype="float32", page=page, decode=n, context_lo=spread(8, hi), context_hi=hi)
+        hi = spread(5, 130)
+        return _case(model, layers, "generate", dtype="float32", page=page, prompts=rng.randint(1, 6), prompt_lo=spread(4, hi),
+                     prompt_hi=hi, steps=rng.randint(4, 16))
+    n = spread(1, 24)
+    hi = spread(12, 2600 // n if kind == "pevazen" else 4000 // n)
+    return _case(kind + "-1b", rng.choice((4, 8)), "serve", page=page, prompts=n, prompt_lo=spread(4, hi), prompt_hi=hi,
+                 steps=rng.choice((0, rng.randint(1, 10))))
+
+
+# ------------------------------------------------------------------ what a case holds
+def config_of(case):
+    """config.json's contents."""
+    raw = copy.deepcopy(named_shapes()[case["model"]])
+    if "num_hidden_layers" in raw:
+        raw["num_hidden_layers"] = case["layers"]
+        return raw
+    raw["layers"] = raw["layers"][:case["layers"]]
+    dense = next(layer["mlp"] for layer in raw["layers"] if layer["mlp"]["kind"] == "dense")
+    for layer in raw["layers"]:
+        layer["mlp"] = dense
+    return raw
+
+
+def _lengths(count, lo, hi):
+    """``count`` lengths from ``lo`` to ``hi``, the longest among them: the same ones whenever they are asked for."""
+    rng = random.Random(1000003 * count + 1009 * lo + hi)
+    return ([hi] + [rng.randint(lo, hi) for _ in range(count - 1)])[:count]
+
+
+def requests_of(case):
+    """[(tokens that are cached before the pass, tokens that its first step brings)], one for each request."""
+    decoding = [(n, 1) for n in _lengths(case["decode"], case["context_lo"], case["context_hi"])]
+    return decoding + [(case["behind"], n) for n in _lengths(case["prompts"], case["prompt_lo"], case["prompt_hi"])]
+
+
+def tokens_of(case, seed, vocab):
+    """Every request's token ids: what is cached, what the first step brings, one for every single-token step."""
+    gen = torch.Generator().manual_seed(int(seed))
+    more = case["steps"] if case["mode"] == "serve" else 0
+    return [torch.randint(0, vocab, (a + n + more,), generator=gen).tolist() for a, n in requests_of(case)]
+
+
+def weights_of(config, seed, dtype):
+    """The model's parameters by their names in the built model, drawn on the device."""
+    gen = torch.Generator(device=DEVICE).manual_seed(int(seed))
+    out = {}
+
+    def put(name, shape, mean=0.0, std=0.02, dt=dtype):
+        out[name] = torch.empty(shape, dtype=dt, device=DEVICE).normal_(mean, std, generator=gen)
+
+    def wide(name, shape, mean, std):                     # parameters that are 32 bits whatever the run computes in
+        put(name, shape, mean, std, torch.float32)
+
+    small = 0.02 * (2 * (config.get("num_hidden_layers") or len(config["layers"]))) ** -0.5
+    rows = 0.02 if dtype == torch.float32 else 1.0
+    if "hidden_size" in config:
+        W, D, ff, vocab = config["hidden_size"], config["head_dim"], config["intermediate_size"], config["vocab_size"]
+        H, G = config["num_attention_heads"], config["num_key_value_heads"]
+        for i in range(config["num_hidden_layers"]):
+            p = f"layers.{i}."
+            put(p + "mixer.qkv.weight", ((H + 2 * G) * D, W))
+            put(p + "mixer.o.weight", (W, H * D), 0.0, small)
+            put(p + "feed_forward.gate_up.weight", (2 * ff, W))
+            put(p + "feed_forward.down.weight", (W, ff), 0.0, small)
+            for name, size in (("mixer.q_norm", D), ("mixer.k_norm", D), ("mixer_norm", W), ("feed_forward_norm", W)):
+                put(f"{p}{name}.weight", (size,), 1.0, 0.1)
+        put("final_norm.weight", (W,), 1.0, 0.1)
+        if not config["tie_word_embeddings"]:
+            put("head.weight", (vocab, W))
+        put("embed.weight", (vocab, W), 0.0, rows)
+        return out
+
+    W, vocab = config["width"], config["vocab"]
+    name = config["architecture"]
+    for i, layer in enumerate(config["layers"]):
+        p, m, ff = f"layers.{i}.", layer["mixer"], layer["mlp"]["ff"]
+        q = p + "mixer."
+        if name == "Pevazen":
+            a = m["left"] if layer["type"] == "parallel" else m
+            H, G, D, E = a["heads"], a["kv_heads"], a["dim"], a["vdim"]
+            left = q + ("left." if layer["type"] == "parallel" else "")
+            width = H * D + (0 if "kv_from" in a else G * (D + E))
+            put(left + "qkv.weight", (width, W))
+            put(left + "o.weight", (W, H * E), 0.0, small)
+            if layer["type"] == "attention":
+                put(left + "qkv.bias", (width,))
+            else:
+                r, right = m["right"], q + "right."
+                H, G, D, E = r["heads"], r["kv_heads"], r["dim"], r["vdim"]
+                channels = 2 * G * D + H * E
+                put(right + "in.weight", (channels + H, W))
+                wide(right + "conv.weight", (channels, r["conv"]), 0.0, 0.5)
+                put(right + "a1.weight", (r["decay_rank"], W))
+                put(right + "a2.weight", (H * D, r["decay_rank"]))
+                put(right + "g1.weight", (r["gate_rank"], W))
+                put(right + "g2.weight", (H * E, r["gate_rank"]))
+                wide(right + "dt_bias", (H * D,), -1.0, 1.0)
+                wide(right + "A_log", (H,), -1.0, 0.5)
+                wide(right + "norm.weight", (E,), 1.0, 0.1)
+                put(right + "o.weight", (W, H * E), 0.0, small)
+                wide(q + "left_out.weight", (W,), 1.0, 0.1)
+                wide(q + "right_out.weight", (W,), 1.0, 0.1)
+            wide(p + "norm.weight", (), 1.0, 0.1)
+            wide(p + "depth.weight", (i + 2,), 1.0 / (i + 2), 0.3 / (i + 2))
+            put(p + "feed_forward.gate_up.weight", (2 * ff, W))
+            put(p + "feed_forward.down.weight", (W, ff), 0.0, small)
+        elif name == "Zigelorn":
+            H, D = m["heads"], m["dim"]
+            n = H * D
+            if layer["type"] == "attention":
+                G = m["kv_heads"]
+                put(q + "qkv.weight", (n + G * D + H, W))
+                put(q + "qkv.bias", (n + G * D,))
+                wide(q + "q_norm.weight", (n,), 1.0, 0.1)
+                wide(q + "k_norm.weight", (G * D,), 1.0, 0.1)
+            elif layer["type"] == "retention":
+                put(q + "in.weight", (2 * n + 2 * H * m["vdim"], W))
+                n = H * m["vdim"]
+            else:
+                put(q + "in.weight", (4 * n + m["decay_rank"], W))
+                put(q + "w2.weight", (n, m["decay_rank"]))
+                wide(q + "mu", (5 * W,), 0.5, 0.2)
+                wide(q + "w0", (n,), -3.0, 1.5)
+                wide(q + "u", (H, D), 0.5, 0.3)
+                wide(q + "norm.weight", (n,), 1.0, 0.1)
+            put(q + "o.weight", (W, n))
+            put(p + "feed_forward.up.weight", (ff, W))
+            put(p + "feed_forward.down.weight", (W, ff))
+            for norm in ("mixer_norm", "mixer_out_norm", "feed_forward_norm", "feed_forward_out_norm"):
+                wide(f"{p}{norm}.weight", (W,), -0.75 if "out" in norm else 0.0, 0.1)
+        else:
+            H, D, E = m["heads"], m["dim"], m["vdim"]
+            if layer["type"] == "latent_attention":
+                R, C = m["rot_dim"], m["kv_rank"]
+                put(q + "down.weight", (H * (D + R) + C + R + H * E, W))
+                wide(q + "kv_norm.weight", (C,), 1.0, 0.1)
+                put(q + "uk.weight", (H * D, C))
+                put(q + "uv.weight", (H * E, C))
+            else:
+                put(q + "qkv.weight", (H * D + m["kv_heads"] * (D + E), W))
+                if m["v_mix"]:
+                    wide(q + "vmix", (), 0.4, 0.1)
+            wide(q + "sink", (H,), 0.0, 1.0)
+            put(q + "o.weight", (W, H * E), 0.0, small)
+            put(p + "feed_forward.gate_up.weight", (2 * ff, W))
+            put(p + "feed_forward.gate_up.bias", (2 * ff,))
+            put(p + "feed_forward.down.weight", (W, ff), 0.0, small)
+            put(p + "feed_forward.down.bias", (W,))
+            for norm in ("mixer_norm", "feed_forward_norm"):
+                put(f"{p}{norm}.weight", (W,), 1.0, 0.1)
+    if name == "Pevazen":
+        wide("embed_norm.weight", (), 1.0, 0.1)
+        wide("final_norm.weight", (), 1.0, 0.1)
+    elif name == "Zigelorn":
+        wide("final_norm.weight", (W,), 0.0, 0.1)
+    else:
+        put("final_norm.weight", (W,), 1.0, 0.1)
+    if name != "Zigelorn":
+        put("head.weight", (vocab, W))
+    put("embed.weight", (vocab, W), 0.0, rows)
+    return out
+
+
+# ------------------------------------------------------------------ the pass
+def prepare(case, seed):
+    """An engine with its model's weights, the requests' contexts in its cache, and the steps of the pass met once (a
+    server's engine has recorded its steps before the call that is measured)."""
+    config = config_of(case)
+    arch = resolve_architecture(config)
+    typed = arch.parse_config(config)
+    model = DecoderModel(arch.build_spec(typed), options={"residual_float32": True})
+    model.bind_all(weights_of(config, seed, DTYPES[case["dtype"]]))
+    requests, vocab = requests_of(case), model.spec.vocab_size
+    tokens = tokens_of(case, seed, vocab)
+    longest = max(a + n for a, n in requests) + case["steps"] + 1
+    pages = sum(-(-(a + n + case["steps"] + 1) // case["page"]) for a, n in requests)
+    llm = LLM("random weights", built_model=(arch, typed, model), dtype=case["dtype"], kvcache_block_size=case["page"],
+              num_kvcache_blocks=pages + 1, max_num_seqs=len(requests), max_model_len=max(4096, longest))
+    state = {"llm": llm, "case": case, "tokens": tokens, "requests": requests}
+    if case["mode"] == "step":
+        at = 0
+        while any(at < a for a, _ in requests):           # the contexts, 2,048 tokens of a request at a time
+            brought = [StepEntry(i, tokens[i][at:min(a, at + 2048)]) for i, (a, _) in enumerate(requests) if at < a]
+            while brought:
+                llm.runner.step(brought[:8])
+                brought = brought[8:]
+            at += 2048
+    run(state)
+    return state
+
+
+def run(state):
+    case, llm, tokens, requests = state["case"], state["llm"], state["tokens"], state["requests"]
+    runner = llm.runner
+    if case["mode"] == "generate":
+        greedy = SamplingParams(temperature=0.0, max_tokens=case["steps"], ignore_eos=True)
+        return {"tokens": np.array([r["token_ids"] for r in llm.generate(tokens, greedy, use_tqdm=False)])}
+    logits = [runner.step([StepEntry(i, tokens[i][a:a + n], [n - 1]) for i, (a, n) in enumerate(requests)])]
+    if case["mode"] == "step":
+        for i, (a, _) in enumerate(requests):
+            if a:
+                runner.cache.rewind(i, a)
+            else:
+                runner.finish(i)
+        return {"logits": logits}
+    for s in range(case["steps"]):
+        logits.append(runner.step([StepEntry(i, [tokens[i][a + n + s]], [0]) for i, (a, n) in enumerate(requests)]))
+    for i in range(len(requests)):
+        runner.finish(i)
+    return {"logits": logits}
+
+
+# ------------------------------------------------------------------ what a pass cannot do without
+def work(case):
+    config, requests = config_of(case), requests_of(case)
+    size = 2 if case["dtype"] == "bfloat16" else 4
+    if "hidden_size" in config:
+        W, ff, vocab, D = config["hidden_size"], config["intermediate_size"], config["vocab_size"], config["head_dim"]
+        H, G = config["num_attention_heads"], config["num_key_value_heads"]
+        layer = W * D * (2 * H + 2 * G) + 3 * W * ff
+        layers = [(layer, 2 * G * D, 4 * H * D, None, 0)] * config["num_hidden_layers"]
+    else:
+        # of every layer: matrix entries, cached entries a token, flops a pair of query and key, keys a query reads at
+        # most, entries of 32-bit state a request (read and written in each step; 6 flops a token and entry)
+        W, vocab, layers = config["width"], config["vocab"], []
+        for entry in config["layers"]:
+            m, ff = entry["mixer"], entry["mlp"]["ff"] * (2 if config["architecture"] == "Zigelorn" else 3) * W
+            a = m.get("left", m)
+            H, D, E, reach = a["heads"], a["dim"], a.get("vdim", a["dim"]), a.get("mask", {}).get("size")
+            if entry["type"] == "latent_attention":
+                C, R = m["kv_rank"], m["rot_dim"]
+                layers.append((ff + W * (H * (D + R) + C + R + 2 * H * E) + C * H * (D + E), C + R, 2 * H * (2 * C + R), reach, 0))
+            elif entry["type"] in ("wkv", "retention"):
+                rows = 4 * H * D + 2 * m.get("decay_rank", 0) + H * E
+                layers.append((ff + W * rows, 0, 0, None, H * D * E))
+            else:
+                G = a["kv_heads"]
+                own = 0 if "kv_from" in a else (1 if config["architecture"] == "Zigelorn" else 2)
+                entries = ff + W * D * (2 * H + own * G)
+                state = 0
+                if "right" in m:
+                    r = m["right"]
+                    entries += W * r["dim"] * (2 * r["kv_heads"] + 2 * r["heads"] + 2) + 2 * r["decay_rank"] * (W + r["heads"] * r["dim"])
+                    state = r["heads"] * r["dim"] * r["vdim"]
+                layers.append((entries, own * G * D, 4 * H * D, reach, state))
+    steps = [requests] + [[(a + n + s, 1) for a, n in requests] for s in range(max(0, case["steps"] - (case["mode"] == "generate")))]
+    total_bytes = total_flops = 0
+    for step in steps:
+        tokens, rows = sum(n for _, n in step), len(step)
+        total_bytes += vocab * W * size + tokens * W * size + rows * vocab * 4
+        total_flops += 2 * vocab * W * rows
+        for entries, cached, pair, reach, state in layers:
+            total_bytes += entries * size + tokens * cached * size + rows * state * 8
+            total_flops += 2 * entries * tokens + 6 * state * tokens
+            for a, n in step:
+                total_bytes += min(a, reach or a) * cached * size
+                if pair:
+                    seen = n * a + n * (n + 1) // 2
+                    total_flops += pair * (min(seen, n * reach) if reach else seen)
+    return {"bytes": total_bytes, "flops": total_flops}
+
+
+def tolerance(case):
+    if case["mode"] == "generate":
+        return {"rel": 0.0, "differ": 0.01}
+    # four times what the passes are off from 64 bits (2.4e-6; 0.0024 to 0.0096 in bfloat16)
+    return {"rel": 1e-5} if case["dtype"] == "float32" else {"rel": 0.03}
+
+
+# ------------------------------------------------------------------ the same in 64 bits
+class _Sequences:
+    """Whole sequences one after the other in one tensor's rows, and plain functions over them, all in float64."""
+
+    def __init__(self, lengths):
+        self.spans, at = [], 0
+        for n in lengths:
+            self.spans.append((at, n))
+            at += n
+        self.positions = torch.cat([torch.arange(n, device=DEVICE, dtype=torch.float64) for n in lengths])
+
+    def turn(self, x, dims, freqs, gain=1.0, sign=1.0):
+        """x [rows, heads, size]: entries i and i + dims / 2 of the first ``dims`` turn by position times freqs[i]."""
+        angle = sign * self.positions[:, None] * freqs
+        c, s = gain * angle.cos()[:, None], gain * angle.sin()[:, None]
+        u, v = x[..., :dims // 2], x[..., dims // 2:dims]
+        return torch.cat((u * c - v * s, v * c + u * s, x[..., dims:]), dim=-1)
+
+    def attend(self, q, k, v, scale, window=None, chunk=None, sink=None, slopes=None):
+        """q [rows, H, D], k [rows, G, D], v [rows, G, E]."""
+        H, G = q.shape[1], k.shape[1]
+        out = torch.empty(q.shape[0], H, v.shape[2], dtype=torch.float64, device=DEVICE)
+        for at, n in self.spans:
+            keys = k[at:at + n].permute(1, 2, 0)[:, None]                       # [G, 1, D, n]
+            values = v[at:at + n].permute(1, 0, 2)[:, None]                     # [G, 1, n, E]
+            for i in range(0, n, 512):
+                m = min(512, n - i)
+                here = q[at + i:at + i + m].permute(1, 0, 2).reshape(G, H // G, m, -1)
+                query, key = torch.arange(i, i + m, device=DEVICE)[:, None], torch.arange(n, device=DEVICE)[None]
+                hidden = key > query
+                if window is not None:
+                    hidden = hidden | (query - key >= window)
+                if chunk is not None:
+                    hidden = hidden | (query // chunk != key // chunk)
+                # (products of batches, the right operand dense: one group of heads at a time)
+                s = torch.stack([here[g].reshape(-1, here.shape[-1]) @ keys[g, 0].contiguous() for g in range(G)])
+                s = s.view(H, m, n) * scale
+                if slopes is not None:
+                    s = s - slopes[:, None, None] * (query - key).double()
+                s = s.masked_fill(hidden, -math.inf)
+                top = s.amax(-1, keepdim=True)
+                if sink is not None:
+                    top = torch.maximum(top, sink.view(H, 1, 1))
+                e = torch.exp(s - top)
+                below = e.sum(-1, keepdim=True)
+                if sink is not None:
+                    below = below + torch.exp(sink.view(H, 1, 1) - top)
+                e = (e / below).view(G, -1, n)
+                o = torch.stack([e[g] @ values[g, 0].contiguous() for g in range(G)])
+                out[at + i:at + i + m] = o.view(H, m, -1).permute(1, 0, 2)
+        return out
+
+    def padded(self, x):
+        """[sequences, longest, ...]: zeros behind a sequence's end."""
+        out = x.new_zeros(len(self.spans), max(n for _, n in self.spans), *x.shape[1:])
+        for i, (at, n) in enumerate(self.spans):
+            out[i, :n] = x[at:at + n]
+        return out
+
+    def packed(self, x):
+        return torch.cat([x[i, :n] for i, (_, n) in enumerate(self.spans)])
+
+    def recur(self, step, state, *inputs):
+        """``step(state, inputs of one token) -> (state, result)``, every sequence at once."""
+        inputs, results = [self.padded(x) for x in inputs], []
+        for t in range(inputs[0].shape[1]):
+            state, r = step(state, *(x[:, t] for x in inputs))
+            results.append(r)
+        return self.packed(torch.stack(results, dim=1))
+
+    def before(self, x, back=1):
+        """Every row's predecessor ``back`` places before it in its sequence, zeros before the first."""
+        out = torch.zeros_like(x)
+        for at, n in self.spans:
+            if n > back:
+                out[at + back:at + n] = x[at:at + n - back]
+        return out
+
+
+def _freqs(dims, base, factor=1.0):
+    return float(base) ** (-2.0 * torch.arange(dims // 2, dtype=torch.float64, device=DEVICE) / dims) / factor
+
+
+def _over_rms(x, eps):
+    return x / torch.sqrt(x.pow(2).mean(-1, keepdim=True) + eps)
+
+
+def _silu(z):
+    return z * torch.sigmoid(z)
+
+
+def _exact_qwen3(c, w, x, seqs):
+    D, H, G, eps = c["head_dim"], c["num_attention_heads"], c["num_key_value_heads"], c["rms_norm_eps"]
+    f = _freqs(D, c["rope_theta"])
+    for i in range(c["num_hidden_layers"]):
+        p = f"layers.{i}."
+        qkv = _over_rms(x, eps) * w(p + "mixer_norm.weight") @ w(p + "mixer.qkv.weight").T
+        q, k, v = (t.unflatten(-1, (-1, D)) for t in qkv.split([H * D, G * D, G * D], dim=-1))
+        q = seqs.turn(_over_rms(q, eps) * w(p + "mixer.q_norm.weight"), D, f)
+        k = seqs.turn(_over_rms(k, eps) * w(p + "mixer.k_norm.weight"), D, f)
+        x = x + seqs.attend(q, k, v, D ** -0.5).flatten(1) @ w(p + "mixer.o.weight").T
+        g, u = (_over_rms(x, eps) * w(p + "feed_forward_norm.weight") @ w(p + "feed_forward.gate_up.weight").T).chunk(2, dim=-1)
+        x = x + (_silu(g) * u) @ w(p + "feed_forward.down.weight").T
+    return _over_rms(x, eps) * w("final_norm.weight")
+
+
+def _exact_pevazen(c, w, x, seqs):
+    eps = c["norm"]["eps"]
+    x = _over_rms(x, eps) * w("embed_norm.weight")
+    results, lent = [x], {}
+    for i, layer in enumerate(c["layers"]):
+        p, m, both = f"layers.{i}.", layer["mixer"], layer["type"] == "parallel"
+        h = _over_rms(x, eps) * w(p + "norm.weight")
+        a, q = (m["left"], p + "mixer.left.") if both else (m, p + "mixer.")
+        H, G, D, E, rot = a["heads"], a["kv_heads"], a["dim"], a["vdim"], a["rot"]
+        f = _freqs(rot["dims"], rot["base"], (rot.get("scaling") or {}).get("factor", 1.0))
+        rows = h @ w(q + "qkv.weight").T
+        if not both:
+            rows = rows + w(q + "qkv.bias")
+        query = seqs.turn(rows[:, :H * D].unflatten(-1, (H, D)), rot["dims"], f)
+        fv = _freqs(E, rot["base"])
+        if "kv_from" in a:
+            k, v = lent[a["kv_from"]]
+        else:
+            k = seqs.turn(rows[:, H * D:(H + G) * D].unflatten(-1, (G, D)), rot["dims"], f)
+            v = rows[:, (H + G) * D:].unflatten(-1, (G, E))
+            if both:
+                v = seqs.turn(v, E, fv)
+            lent[i] = (k, v)
+        o = seqs.attend(query, k, v, a["scale"], chunk=a["mask"]["size"])
+        if both:
+            o = seqs.turn(o, E, fv, sign=-1.0)
+        mixed = o.flatten(1) @ w(q + "o.weight").T
+        if both:
+            r, q = m["right"], p + "mixer.right."
+            H, G, D, E = r["heads"], r["kv_heads"], r["dim"], r["vdim"]
+            rows, taps = h @ w(q + "in.weight").T, w(q + "conv.weight")
+            z, n = rows[:, :-H], taps.shape[1]
+            z = _silu(sum(taps[:, n - 1 - j] * (seqs.before(z, j) if j else z) for j in range(n)))
+            qq, kk, vv = z.split([G * D, G * D, H * E], dim=-1)
+            qq, kk = (t.unflatten(-1, (G, D)) for t in (qq, kk))
+            qq, kk = (t / torch.sqrt(t.pow(2).sum(-1, keepdim=True) + 1e-6) for t in (qq, kk))
+            qq, kk = (t.repeat_interleave(H // G, dim=1) for t in (qq * D ** -0.5, kk))
+            linear = (h @ w(q + "a1.weight").T) @ w(q + "a2.weight").T + w(q + "dt_bias")
+            decay = torch.exp(-torch.exp(w(q + "A_log"))[:, None] * torch.nn.functional.softplus(linear).unflatten(-1, (H, D)))
+
+            def step(S, q_, k_, v_, g_, b_):
+                S = g_[..., None] * S
+                u = b_[..., None] * (v_ - (S * k_[..., None]).sum(-2))
+                S = S + k_[..., None] * u[..., None, :]
+                return S, (S * q_[..., None]).sum(-2)
+
+            S = x.new_zeros(len(seqs.spans), H, D, E)
+            o = seqs.recur(step, S, qq, kk, vv.unflatten(-1, (H, E)), decay, torch.sigmoid(rows[:, -H:]))
+            gate = torch.sigmoid((h @ w(q + "g1.weight").T) @ w(q + "g2.weight").T).unflatten(-1, (H, E))
+            right = (_over_rms(o, eps) * w(q + "norm.weight") * gate).flatten(1) @ w(q + "o.weight").T
+            mixed = 0.5 * (_over_rms(mixed, eps) * w(p + "mixer.left_out.weight") + _over_rms(right, eps) * w(p + "mixer.right_out.weight"))
+        g, u = (h @ w(p + "feed_forward.gate_up.weight").T).chunk(2, dim=-1)
+        results.append(x + mixed + (_silu(g) * u) @ w(p + "feed_forward.down.weight").T)
+        x = sum(s * t for s, t in zip(w(p + "depth.weight"), results))
+    return _over_rms(x, eps) * w("final_norm.weight")
+
+
+def _yarn(rot):
+    """Frequencies scaled part by part, and the factor of cosines and sines."""
+    f, scaling, dims = _freqs(rot["dims"], rot["base"]), rot.get("scaling"), rot["dims"]
+    if not scaling:
+        return f, 1.0
+
+    def pair_of(turns):
+        return dims * math.log(scaling["original"] / (turns * 2.0 * math.pi)) / (2.0 * math.log(rot["base"]))
+
+    low, high = max(math.floor(pair_of(scaling["fast"])), 0), min(math.ceil(pair_of(scaling["slow"])), dims - 1)
+    share = ((torch.arange(dims // 2, dtype=torch.float64, device=DEVICE) - low) / max(high - low, 0.001)).clamp(0.0, 1.0)
+    return share * f / scaling["factor"] + (1.0 - share) * f, 1.0 + 0.1 * math.log(scaling["factor"])
+
+
+def _exact_zigelorn(c, w, x, seqs):
+    eps = c["norm"]["eps"]
+
+    def norm(t, name):
+        return _over_rms(t, eps) * (1.0 + w(name + ".weight"))
+
+    for i, layer in enumerate(c["layers"]):
+        p, m = f"layers.{i}.", layer["mixer"]
+        q, h, H, D = p + "mixer.", norm(x, p + "mixer_norm"), m["heads"], m["dim"]
+        if layer["type"] == "attention":
+            G, (f, gain) = m["kv_heads"], _yarn(m["rot"])
+            rows = h @ w(q + "qkv.weight").T
+            bias, n = w(q + "qkv.bias"), H * D
+            query, key = rows[:, :n] + bias[:n], rows[:, n:n + G * D] + bias[n:]
+            v = key.unflatten(-1, (G, D))
+            query = seqs.turn((_over_rms(query, eps) * w(q + "q_norm.weight")).unflatten(-1, (H, D)), m["rot"]["dims"], f, gain)
+            key = seqs.turn((_over_rms(key, eps) * w(q + "k_norm.weight")).unflatten(-1, (G, D)), m["rot"]["dims"], f, gain)
+            o = seqs.attend(query, key, v, m["scale"], window=m["mask"]["size"]) * torch.sigmoid(rows[:, n + G * D:])[..., None]
+            o = o.flatten(1)
+        elif layer["type"] == "retention":
+            E = m["vdim"]
+            query, key, v, gate = (h @ w(q + "in.weight").T).split([H * D, H * D, H * E, H * E], dim=-1)
+            f = _freqs(m["rot"]["dims"], m["rot"]["base"])
+            query = seqs.turn(query.unflatten(-1, (H, D)), m["rot"]["dims"], f)
+            key = seqs.turn(key.unflatten(-1, (H, D)), m["rot"]["dims"], f) * D ** -0.5
+            decay = torch.tensor(m["decay"], dtype=torch.float64, device=DEVICE)[:, None, None]
+
+            def step(S, q_, k_, v_):
+                S = decay * S + k_[..., None] * v_[..., None, :]
+                return S, (S * q_[..., None]).sum(-2)
+
+            o = seqs.recur(step, x.new_zeros(len(seqs.spans), H, D, E), query, key, v.unflatten(-1, (H, E)))
+            o = _over_rms(o, eps).flatten(1) * _silu(gate)
+        else:
+            n, W, before = H * D, x.shape[1], seqs.before(h)
+            rows, mu = w(q + "in.weight"), w(q + "mu").split(W)
+            r, k, v, gate, low = ((h + (before - h) * mu[j]) @ rows[j * n:min((j + 1) * n, rows.shape[0])].T for j in range(5))
+            linear = torch.tanh(low) @ w(q + "w2.weight").T + w(q + "w0")
+            r, k, v, decay = (t.unflatten(-1, (H, D)) for t in (r, k, v, torch.exp(-torch.exp(linear))))
+            bonus = w(q + "u")
+
+            def step(S, r_, k_, v_, g_):
+                pair = k_[..., None] * v_[..., None, :]
+                return g_[..., None] * S + pair, ((S + bonus[..., None] * pair) * r_[..., None]).sum(-2)
+
+            o = seqs.recur(step, x.new_zeros(len(seqs.spans), H, D, D), r, k, v, decay)
+            o = _over_rms(o, eps).flatten(1) * w(q + "norm.weight") * _silu(gate)
+        x = x + norm(o @ w(q + "o.weight").T, p + "mixer_out_norm")
+        h = norm(x, p + "feed_forward_norm")
+        z = torch.nn.functional.gelu(h @ w(p + "feed_forward.up.weight").T, approximate="tanh")
+        x = x + norm(z @ w(p + "feed_forward.down.weight").T, p + "feed_forward_out_norm")
+    return norm(x, "final_norm")
+
+
+def _exact_gabelorn(c, w, x, seqs):
+    eps, first = c["norm"]["eps"], None
+    for i, layer in enumerate(c["layers"]):
+        p, m = f"layers.{i}.", layer["mixer"]
+        q, H, D, E = p + "mixer.", m["heads"], m["dim"], m["vdim"]
+        h, sink = _over_rms(x, eps) * w(p + "mixer_norm.weight"), w(q + "sink")
+        if layer["type"] == "latent_attention":
+            R, C, rot = m["rot_dim"], m["kv_rank"], m["rot"]
+            query, latent, turned, gate = (h @ w(q + "down.weight").T).split([H * (D + R), C, R, H * E], dim=-1)
+            latent, f = _over_rms(latent, eps) * w(q + "kv_norm.weight"), _freqs(rot["dims"], rot["base"])
+            query = query.unflatten(-1, (H, D + R))
+            query = torch.cat((query[..., :D], seqs.turn(query[..., D:], rot["dims"], f)), dim=-1)
+            turned = seqs.turn(turned[:, None], rot["dims"], f).expand(-1, H, -1)
+            k = torch.cat(((latent @ w(q + "uk.weight").T).unflatten(-1, (H, D)), turned), dim=-1)
+            v = (latent @ w(q + "uv.weight").T).unflatten(-1, (H, E))
+            o = seqs.attend(query, k, v, m["scale"], window=m["mask"]["size"], sink=sink).flatten(1) * torch.sigmoid(gate)
+        else:
+            G, t = m["kv_heads"], m["q_temp"]
+            query, k, v = (h @ w(q + "qkv.weight").T).split([H * D, G * D, G * E], dim=-1)
+            warm = 1.0 + t["coef"] * torch.log(torch.floor((seqs.positions + 1) / t["every"]) + 1)
+            query = query.unflatten(-1, (H, D)) * warm[:, None, None]
+            k, v = k.unflatten(-1, (G, D)), v.unflatten(-1, (G, E))
+            if m["v_mix"] and first is not None:
+                share = w(q + "vmix")
+                v = (1 - share) * v + share * first
+            elif m["v_mix"]:
+                first = v
+            slopes = 2.0 ** (-8.0 * torch.arange(1, H + 1, dtype=torch.float64, device=DEVICE) / H)
+            o = seqs.attend(query, k, v, m["scale"], sink=sink, slopes=slopes).flatten(1)
+        x = x + o @ w(q + "o.weight").T
+        h, p = _over_rms(x, eps) * w(p + "feed_forward_norm.weight"), p + "feed_forward."
+        g, u = (h @ w(p + "gate_up.weight").T + w(p + "gate_up.bias")).chunk(2, dim=-1)
+        limit = layer["mlp"]["limit"]
+        g, u = g.clamp(max=limit), u.clamp(-limit, limit)
+        x = x + (g * torch.sigmoid(1.702 * g) * (u + 1)) @ w(p + "down.weight").T + w(p + "down.bias")
+    return _over_rms(x, eps) * w("final_norm.weight")
+
+
+def exact(case, seed):
+    if case["mode"] == "generate":
+        return None                                       # whole numbers
+    config = config_of(case)
+    stored = weights_of(config, seed, DTYPES[case["dtype"]])
+
+    def w(name):
+        return stored[name].double()
+
+    vocab = config.get("vocab_size") or config["vocab"]
+    tokens = tokens_of(case, seed, vocab)
+    seqs = _Sequences([len(t) for t in tokens])
+    x = stored["embed.weight"][torch.tensor([t for row in tokens for t in row], device=DEVICE)].double()
+    name = config.get("architecture", "Qwen3")
+    x = {"Qwen3": _exact_qwen3, "Pevazen": _exact_pevazen, "Zigelorn": _exact_zigelorn, "Gabelorn": _exact_gabelorn}[name](config, w, x, seqs)
+    head = (stored["head.weight"] if "head.weight" in stored else stored["embed.weight"]).double()
+    ends = [at + n - 1 for at, n in seqs.spans]
+    more = case["steps"] if case["mode"] == "serve" else 0
+    logits = [x[[e - more + s for e in ends]] @ head.T for s in range(more + 1)]
+    cap = config.get("logit_softcap")
+    return {"logits": [cap * torch.tanh(t / cap) for t in logits] if cap else logits}
