@@ -45,29 +45,29 @@ def _case(model, layers, mode, dtype="bfloat16", page=256, decode=0, context_lo=
 def listed():
     cases = [
         # one user chatting with the smallest model: every launch of the step shows
-        ("one request, 0.6b", _case("0.6b", 28, "step", decode=1, context_lo=150, context_hi=150)),
+        ("one request 0.6b", _case("0.6b", 28, "step", decode=1, context_lo=150, context_hi=150)),
         # the benchmark's step: a few users after prompts of one length (a third of the layers)
-        ("8 requests, 8b", _case("8b", 12, "step", decode=8, context_lo=2048, context_hi=2048)),
+        ("8 requests 8b", _case("8b", 12, "step", decode=8, context_lo=2048, context_hi=2048)),
         # a loaded server: many users, every context another length
-        ("64 requests, 8b", _case("8b", 12, "step", decode=64, context_lo=97, context_hi=2048)),
+        ("64 requests 8b", _case("8b", 12, "step", decode=64, context_lo=97, context_hi=2048)),
         # the benchmark's prompt
-        ("prompt of 2048, 8b", _case("8b", 12, "step", prompts=1, prompt_lo=2048, prompt_hi=2048)),
+        ("prompt of 2048 8b", _case("8b", 12, "step", prompts=1, prompt_lo=2048, prompt_hi=2048)),
         # continuous batching: portions of ragged prompts beside requests that decode
-        ("mixed, 8b", _case("8b", 12, "step", decode=13, context_lo=60, context_hi=1700, prompts=3, prompt_lo=90, prompt_hi=901)),
+        ("mixed 8b", _case("8b", 12, "step", decode=13, context_lo=60, context_hi=1700, prompts=3, prompt_lo=90, prompt_hi=901)),
         # a long document comes in by portions: attention over what is there already
-        ("portion at 14336, 8b", _case("8b", 12, "step", prompts=1, prompt_lo=2048, prompt_hi=2048, behind=14336)),
+        ("portion at 14336 8b", _case("8b", 12, "step", prompts=1, prompt_lo=2048, prompt_hi=2048, behind=14336)),
         # a short question to a model of medium size, small pages, other users decoding: a step that replays a graph
-        ("short mixed, 4b", _case("4b", 12, "step", page=16, decode=4, context_lo=40, context_hi=700, prompts=1, prompt_lo=75, prompt_hi=75)),
+        ("short mixed 4b", _case("4b", 12, "step", page=16, decode=4, context_lo=40, context_hi=700, prompts=1, prompt_lo=75, prompt_hi=75)),
         # the 32-bit path: a prompt whose logits are compared with another implementation's
-        ("prompt of 517, 0.6b, 32 bits", _case("0.6b", 14, "step", dtype="float32", prompts=1, prompt_lo=517, prompt_hi=517)),
+        ("prompt of 517 0.6b 32 bits", _case("0.6b", 14, "step", dtype="float32", prompts=1, prompt_lo=517, prompt_hi=517)),
         # the 32-bit path through the whole program: prompts to tokens
-        ("generate, 0.6b, 32 bits", _case("0.6b", 14, "generate", dtype="float32", prompts=6, prompt_lo=9, prompt_hi=130, steps=24)),
+        ("generate 0.6b 32 bits", _case("0.6b", 14, "generate", dtype="float32", prompts=6, prompt_lo=9, prompt_hi=130, steps=24)),
         # attention beside a gated delta rule: prompts come in
-        ("prompts, pevazen", _case("pevazen-1b", 8, "serve", prompts=2, prompt_lo=701, prompt_hi=1500)),
+        ("prompts pevazen", _case("pevazen-1b", 8, "serve", prompts=2, prompt_lo=701, prompt_hi=1500)),
         # linear recurrences and windowed attention: short prompts, then decoding
-        ("serve 16, zigelorn", _case("zigelorn-1b", 8, "serve", prompts=16, prompt_lo=20, prompt_hi=200, steps=12)),
+        ("serve 16 zigelorn", _case("zigelorn-1b", 8, "serve", prompts=16, prompt_lo=20, prompt_hi=200, steps=12)),
         # attention over a cached latent and with a bias by distance: prompts beyond the window, then decoding
-        ("serve 5, gabelorn", _case("gabelorn-1b", 8, "serve", prompts=5, prompt_lo=150, prompt_hi=1300, steps=6)),
+        ("serve 5 gabelorn", _case("gabelorn-1b", 8, "serve", prompts=5, prompt_lo=150, prompt_hi=1300, steps=6)),
     ]
     return [dict(case, name=name) for name, case in cases]
 
