@@ -1,8 +1,8 @@
-// y[M, N] = x[M, K] . w[N, K]^T (+ bias[N]) for any M, N, K, in float or bfloat16
+// y[M, N] = x[M, K] . w[N, K]^T (+ bias[N]) for any M, N, K, in bfloat16
 // with float accumulation. Every output element is summed over k = 0..K-1 in that
 // order by one thread, so a row's result does not depend on how many other rows
-// there are. This is the matrix product of the 32-bit path and the fallback of the
-// bfloat16 path for sizes that the faster kernels refuse.
+// there are. This is the fallback of the bfloat16 path for sizes that the faster
+// kernels refuse.
 #include "nhv_common.h"
 
 #define TM 64
@@ -72,8 +72,7 @@ extern "C" int nhv_gemm_generic(const void* x, const void* w, const void* bias, 
   hipStream_t s = (hipStream_t)stream;
 #define LAUNCH(TI, TO) \
   hipLaunchKernelGGL((gemm_generic_kernel<TI, TO>), grid, dim3(256), 0, s, (const TI*)x, (const TI*)w, (const TI*)bias, (TO*)y, M, N, K)
-  if (in_dtype == NHV_F32 && out_dtype == NHV_F32) LAUNCH(float, float);
-  else if (in_dtype == NHV_BF16 && out_dtype == NHV_BF16) LAUNCH(bf16_t, bf16_t);
+  if (in_dtype == NHV_BF16 && out_dtype == NHV_BF16) LAUNCH(bf16_t, bf16_t);
   else if (in_dtype == NHV_BF16 && out_dtype == NHV_F32) LAUNCH(bf16_t, float);
   else return nhv_fail("gemm: unsupported dtypes in=%d out=%d", in_dtype, out_dtype);
 #undef LAUNCH

@@ -18,8 +18,8 @@ import torch
 
 from . import library
 
-CORE_SOURCES = ["error.hip", "elementwise.hip", "gemm_generic.hip", "gemm_skinny_bf16.hip", "gemm_fewrows_bf16.hip", "attention_generic.hip",
-                "sampling.hip", "measure.hip", "stream_mixing.hip", "delta_rule.hip", "parallel_block.hip", "latent_attention.hip",
+CORE_SOURCES = ["error.hip", "elementwise.hip", "gemm_generic.hip", "gemm_float32.hip", "gemm_skinny_bf16.hip", "gemm_fewrows_bf16.hip",
+                "attention_generic.hip", "sampling.hip", "measure.hip", "stream_mixing.hip", "delta_rule.hip", "parallel_block.hip", "latent_attention.hip",
                 "routed_experts.hip", "hyper_streams.hip", "head_outputs.hip", "sandwich_norms.hip", "linear_recurrence.hip"]
 BLAS_SOURCES = ["error.hip", "gemm_library.hip"]                                                   # the vendor's matrix library, algorithm by number
 BLAS_LINK = ["-lhipblaslt"]
@@ -753,6 +753,8 @@ class NativeBackend:
                     self._call("nhv_gemm_skinny_bf16", _ptr(x[m0:m1]), _ptr(w), _ptr(bias), _ptr(out[m0:m1]),
                                m1 - m0, N, K, dtype_code(out), _stream())
                 return None
+        if x.dtype == torch.float32:
+            return self._call("nhv_gemm_float32", _ptr(x), _ptr(w), _ptr(bias), _ptr(out), M, N, K, _stream())
         self._call("nhv_gemm_generic", _ptr(x), _ptr(w), _ptr(bias), _ptr(out), M, N, K, dtype_code(x),
                    dtype_code(out), _stream())
 

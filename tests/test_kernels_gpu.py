@@ -244,6 +244,21 @@ def test_gated_linear(ops, M, I, K):
             backend.own_kernels_only = False
 
 
+@pytest.mark.parametrize("N,K", [(1, 1), (17, 130), (48, 16), (130, 20), (65, 516), (300, 2064), (16400, 36), (24000, 7)])
+def test_float32_linear_in_all_its_tiles(ops, N, K):
+    """Every tile that the number of rows and columns can choose, K below and beyond eight blocks of 16, ends inside a block of
+    16, rows off 16-byte boundaries: against float64 (a sum of K products of size 1 is off by K^(1/2) roundings of its own size,
+    K^(1/2), at most), and the same row bit for bit whatever the number of rows."""
+    x, w, b = rnd(520, K, seed=51), rnd(N, K, seed=52), rnd(N, seed=53)
+    ref = x.double() @ w.double().T + b.double()
+    last = None
+    for M in (520, 65, 64, 33, 17, 16, 1):
+        y = ops.linear(x[520 - M:].contiguous(), w, b)
+        torch.testing.assert_close(y.double(), ref[520 - M:], rtol=1e-6, atol=K * 2.0 ** -23 + 1e-6)
+        assert last is None or torch.equal(y, last[-M:])
+        last = y
+
+
 def test_linear_rows_do_not_depend_on_the_batch_in_float32(ops):
     x = rnd(70, 200, seed=7)
     w = rnd(150, 200, seed=8)
