@@ -1,0 +1,237 @@
+// Attention over the paged cache in float on the float matrix cores (v_mfma_f32_16x16x4_f32: every product and sum in 32 bits),
+// for key heads of a multiple of 16 entries and value heads of 64, 128, 192 or 256; masks and options are those of
+// attention_generic.hip, which takes the other sizes.
+//
+// Keys are taken in blocks of 64 aligned to absolute positions. Each block's maximum, sum and weighted values are computed by
+// themselves and merged in rising order, masked keys count as nothing, so a position's result depends neither on the batch
+// nor on the portion, nor on which wave took a block.
+//
+// A block of 4 waves owns 16 rows, a row being (token, one of the query heads that read one key/value head), of one request:
+// 8 tokens of a prompt where two heads share a key head, or one decoded token. The waves take the blocks of keys in turn;
+// after each round of four blocks the results meet in LDS and are merged. Scores come as S^T = K Q^T, whose layout is
+// that of the second product's right operand (O^T = V^T P^T), so the weights never leave their registers.
+// What bounds it: the chain of rounds of a row tile (32 KB of keys and values a wave and round at 128 entries) while the chip
+// is not full, else the matrix cores.
+#include "nhv_common.h"
+#include <math.h>
+
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+
+#define WAVES 4
+#define ROWS 16
+#define KEYS 64
+#define MAX_E 256
+#define MAX_D 512
+
+struct FloatAttention {
+  const float *q, *k, *v;
+  float* out;
+  const int *positions, *cu, *block_tables;
+  int max_blocks, Hq, Hkv, D, E, page_size;
+  float scale;
+  int window, chunk;
+  float cap;
+  int has_sink;
+  float sink;
+  const float *sinks, *slopes, *gate;
+  long long gate_ld;
+};
+
+__global__ __launch_bounds__(64 * WAVES) void attention_float32_kernel(FloatAttention a) {
+  extern __shared__ __attribute__((aligned(16))) float shared[];
+  const int D = a.D, E = a.E, group = a.Hq / a.Hkv;
+  float* qs = shared;                                    // [ROWS][D + 4]
+  float* part = qs + ROWS * (D + 4);                     // [WAVES][ROWS][E + 4]
+  float* stats = part + WAVES * ROWS * (E + 4);          // [WAVES][ROWS][2]: maximum and sum
+  const int kvh = blockIdx.y, req = blockIdx.z;
+  const int first = a.cu[req], rows = (a.cu[req + 1] - first) * group;
+  const int row0 = blockIdx.x * ROWS;
+  if (row0 >= rows) return;                              // (the same for the whole block)
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, r16 = lane & 15, g = lane >> 4;
+
+  // this lane's row: what it may read
+  const int row = row0 + r16;
+  const bool live = row < rows;
+  const int head = kvh * group + (live ? row % group : 0);
+  const int pos = live ? a.positions[first + row / group] : -1;
+  const int lo = !live ? 0x7fffffff : a.chunk > 0 ? pos - pos % a.chunk : a.window > 0 ? max(0, pos - a.window + 1) : 0;
+  int tile_lo = lo, tile_hi = pos;                       // the same in every lane afterwards
+#pragma unroll
+  for (int o = 8; o > 0; o >>= 1) {
+    tile_lo = min(tile_lo, __shfl_xor(tile_lo, o, NHV_WAVE));
+    tile_hi = max(tile_hi, __shfl_xor(tile_hi, o, NHV_WAVE));
+  }
+  const float slope = a.slopes && live ? a.slopes[head] : 0.f;
+  const int* table = a.block_tables + (size_t)req * a.max_blocks;
+
+  for (int i = threadIdx.x * 4; i < ROWS * D; i += 64 * WAVES * 4) {
+    const int r = i / D, d = i % D;
+    f32x4 v = {0.f, 0.f, 0.f, 0.f};
+    if (row0 + r < rows)
+      v = *reinterpret_cast<const f32x4*>(a.q + ((size_t)(first + (row0 + r) / group) * a.Hq + kvh * group + (row0 + r) % group) * D + d);
+    *reinterpret_cast<f32x4*>(&qs[r * (D + 4) + d]) = v;
+  }
+  __syncthreads();
+
+  // what a thread merges: 16 threads a row, entries c + 16 i
+  const int my_row = threadIdx.x >> 4, c = threadIdx.x & 15;
+  float M = -INFINITY, L = 0.f, total[MAX_E / 16];
+#pragma unroll
+  for (int i = 0; i < MAX_E / 16; ++i) total[i] = 0.f;
+
+  for (int round = tile_lo / KEYS * KEYS; round <= tile_hi; round += KEYS * WAVES) {
+    const int kb = round + wave * KEYS;
+    if (kb <= tile_hi) {
+      // lane l's own key of the block, and where it lies (-1: no row reads it)
+      const int own = kb + lane;
+      int slot = -1;
+      if (own >= tile_lo && own <= tile_hi) slot = table[own / a.page_size] * a.page_size + own % a.page_size;
+      f32x4 s[4];
+      const float* kr[4];
+#pragma unroll
+      for (int t = 0; t < 4; ++t) {
+        const int at = __shfl(slot, 16 * t + r16, NHV_WAVE);
+        kr[t] = at >= 0 ? a.k + ((size_t)at * a.Hkv + kvh) * D + 4 * g : nullptr;
+        s[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+      }
+#pragma unroll 4
+      for (int d = 0; d < D; d += 16) {
+        const f32x4 qf = *reinterpret_cast<const f32x4*>(&qs[r16 * (D + 4) + d + 4 * g]);
+        f32x4 kf[4];
+#pragma unroll
+        for (int t = 0; t < 4; ++t) kf[t] = kr[t] ? *reinterpret_cast<const f32x4*>(kr[t] + d) : f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+#pragma unroll
+          for (int t = 0; t < 4; ++t) s[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[t][j], qf[j], s[t], 0, 0, 0);
+      }
+      // s[t][i]: key kb + 16 t + 4 g + i against row r16
+      float m = -INFINITY;
+#pragma unroll
+      for (int t = 0; t < 4; ++t)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const int key = kb + 16 * t + 4 * g + i;
+          float z = s[t][i] * a.scale;
+          if (a.cap > 0.f) z = a.cap * tanhf(z / a.cap);
+          if (a.slopes) z = fmaf(-slope, (float)(pos - key), z);
+          s[t][i] = key >= lo && key <= pos ? z : -INFINITY;
+          m = fmaxf(m, s[t][i]);
+        }
+      m = fmaxf(m, __shfl_xor(m, 16, NHV_WAVE));
+      m = fmaxf(m, __shfl_xor(m, 32, NHV_WAVE));
+      const float base = m == -INFINITY ? 0.f : m;       // (no visible key: every weight is 0)
+      float l = 0.f;
+#pragma unroll
+      for (int t = 0; t < 4; ++t)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          s[t][i] = expf(s[t][i] - base);
+          l += s[t][i];
+        }
+      l += __shfl_xor(l, 16, NHV_WAVE);
+      l += __shfl_xor(l, 32, NHV_WAVE);
+      if (g == 0) {
+        stats[(wave * ROWS + r16) * 2] = m;
+        stats[(wave * ROWS + r16) * 2 + 1] = l;
+      }
+      // value entry h + 4 r + j of a chunk of 64 is row r of matrix tile j: one load of 16 bytes a key feeds four tiles
+      for (int h = 0; h < E; h += 64) {
+        f32x4 o[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) o[j] = f32x4{0.f, 0.f, 0.f, 0.f};
+        float odd = 0.f;                                 // not a number as soon as some value is infinite or none
+#pragma unroll
+        for (int t = 0; t < 4; ++t)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            const int at = __shfl(slot, 16 * t + 4 * g + i, NHV_WAVE);
+            const f32x4 vf = at >= 0 ? *reinterpret_cast<const f32x4*>(a.v + ((size_t)at * a.Hkv + kvh) * E + h + 4 * r16)
+                                     : f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+              odd = fmaf(vf[j], 0.f, odd);
+              o[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(vf[j], s[t][i], o[j], 0, 0, 0);
+            }
+          }
+        // o[j][i]: row r16, entry h + 16 g + 4 i + j
+        if (__any(odd != 0.f)) {
+          // a value that is no finite number: it must not reach the rows that do not read it (0 times it is not 0)
+#pragma unroll
+          for (int j = 0; j < 4; ++j) o[j] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+          for (int t = 0; t < 4; ++t)
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+              for (int gk = 0; gk < 4; ++gk) {
+                const int at = __shfl(slot, 16 * t + 4 * gk + i, NHV_WAVE);
+                const float p = __shfl(s[t][i], 16 * gk + r16, NHV_WAVE);
+                if (p != 0.f && at >= 0) {
+                  const float* vr = a.v + ((size_t)at * a.Hkv + kvh) * E + h + 16 * g;
+#pragma unroll
+                  for (int ii = 0; ii < 4; ++ii)
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) o[j][ii] = fmaf(p, vr[4 * ii + j], o[j][ii]);
+                }
+              }
+        }
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          *reinterpret_cast<f32x4*>(&part[(wave * ROWS + r16) * (E + 4) + h + 16 * g + 4 * i]) = f32x4{o[0][i], o[1][i], o[2][i], o[3][i]};
+      }
+    }
+    __syncthreads();
+    for (int p = 0; p < WAVES && round + p * KEYS <= tile_hi; ++p) {
+      const float m = stats[(p * ROWS + my_row) * 2], l = stats[(p * ROWS + my_row) * 2 + 1];
+      if (m == -INFINITY) continue;                      // this row reads no key of the block
+      const float top = fmaxf(M, m), old = expf(M - top), now = expf(m - top);
+      L = L * old + l * now;
+      M = top;
+#pragma unroll
+      for (int i = 0; i < MAX_E / 16; ++i)
+        if (16 * i < E) total[i] = total[i] * old + part[(p * ROWS + my_row) * (E + 4) + c + 16 * i] * now;
+    }
+    __syncthreads();
+  }
+
+  if (row0 + my_row >= rows) return;
+  const int t = first + (row0 + my_row) / group, h = kvh * group + (row0 + my_row) % group;
+  float after = 1.f;
+  if (a.has_sink || a.sinks) {                           // one more term of the denominator, without a value
+    const float z = a.sinks ? a.sinks[h] : a.sink;
+    const float top = fmaxf(M, z);
+    after = expf(M - top);
+    L = L * after + expf(z - top);
+  }
+  float inv = after / L;
+  if (a.gate) inv /= 1.0f + expf(-a.gate[(size_t)t * a.gate_ld + h]);
+  float* o = a.out + ((size_t)t * a.Hq + h) * E;
+#pragma unroll
+  for (int i = 0; i < MAX_E / 16; ++i)
+    if (16 * i < E) o[c + 16 * i] = total[i] * inv;
+}
+
+extern "C" int nhv_attention_float32(const void* q, const void* k_cache, const void* v_cache, void* out, const void* positions,
+                                     const void* cu_seqlens_q, const void* block_tables, int max_blocks, int B, int max_q_len, int Hq,
+                                     int Hkv, int D, int E, int page_size, float scale, int window, int chunk, float cap,
+                                     int has_sink, float sink, const void* sinks, const void* slopes, const void* gate, long long gate_ld,
+                                     void* stream) {
+  NHV_REQUIRE(cap >= 0.f && (!gate || gate_ld >= Hq), "attention: cap %g, gate rows %lld apart for %d heads", (double)cap, gate_ld, Hq);
+  NHV_REQUIRE(B > 0 && max_q_len > 0 && Hq > 0 && Hkv > 0 && page_size > 0 && max_blocks > 0,
+              "attention: bad sizes B=%d portion=%d Hq=%d Hkv=%d page=%d blocks=%d", B, max_q_len, Hq, Hkv, page_size, max_blocks);
+  NHV_REQUIRE(Hq % Hkv == 0, "attention: %d query heads are not a multiple of %d key heads", Hq, Hkv);
+  NHV_REQUIRE(D > 0 && D % 16 == 0 && D <= MAX_D && E > 0 && E % 64 == 0 && E <= MAX_E, "attention: head sizes %d and %d are not for this kernel", D, E);
+  NHV_REQUIRE(window >= 0 && chunk >= 0 && !(window > 0 && chunk > 0), "attention: window %d and chunk %d", window, chunk);
+  const long long tiles = ((long long)max_q_len * (Hq / Hkv) + ROWS - 1) / ROWS;
+  NHV_REQUIRE(B <= 65535 && Hkv <= 65535 && tiles < (1ll << 31), "attention: %d requests, %d key heads, portions of %d", B, Hkv, max_q_len);
+  const FloatAttention a = {(const float*)q, (const float*)k_cache, (const float*)v_cache, (float*)out, (const int*)positions,
+                            (const int*)cu_seqlens_q, (const int*)block_tables, max_blocks, Hq, Hkv, D, E, page_size, scale, window, chunk,
+                            cap, has_sink, sink, (const float*)sinks, (const float*)slopes, (const float*)gate, gate_ld};
+  const size_t lds = (ROWS * (D + 4) + WAVES * ROWS * (E + 4) + WAVES * ROWS * 2) * sizeof(float);
+  static const hipError_t allowed = hipFuncSetAttribute((const void*)attention_float32_kernel, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                                        (int)((ROWS * (MAX_D + 4) + WAVES * ROWS * (MAX_E + 4) + WAVES * ROWS * 2) * sizeof(float)));
+  if (allowed != hipSuccess) return nhv_fail("attention: %zu bytes of LDS are refused: %s", lds, hipGetErrorString(allowed));
+  hipLaunchKernelGGL(attention_float32_kernel, dim3((unsigned)tiles, Hkv, B), dim3(64 * WAVES), lds, (hipStream_t)stream, a);
+  NHV_LAUNCH_CHECK("attention_float32");
+  return 0;
+}

@@ -12,7 +12,8 @@
 // softmax's denominator (a sink: a key of a given score that has no value; one score for the layer, or one per head in
 // ``sinks``), and a gate per (token, head) whose sigmoid multiplies the head's result (read from rows ``gate_ld``
 // entries apart).
-// This is the attention of the 32-bit path and the fallback of the bfloat16 path.
+// This is the attention of the 32-bit path at head sizes that attention_float32.hip does not take, and the fallback of the
+// bfloat16 path.
 #include "nhv_common.h"
 #include <math.h>
 

@@ -19,7 +19,7 @@ import torch
 from . import library
 
 CORE_SOURCES = ["error.hip", "elementwise.hip", "gemm_generic.hip", "gemm_float32.hip", "gemm_skinny_bf16.hip", "gemm_fewrows_bf16.hip",
-                "attention_generic.hip", "sampling.hip", "measure.hip", "stream_mixing.hip", "delta_rule.hip", "parallel_block.hip", "latent_attention.hip",
+                "attention_generic.hip", "attention_float32.hip", "sampling.hip", "measure.hip", "stream_mixing.hip", "delta_rule.hip", "parallel_block.hip", "latent_attention.hip",
                 "routed_experts.hip", "hyper_streams.hip", "head_outputs.hip", "sandwich_norms.hip", "linear_recurrence.hip"]
 BLAS_SOURCES = ["error.hip", "gemm_library.hip"]                                                   # the vendor's matrix library, algorithm by number
 BLAS_LINK = ["-lhipblaslt"]
@@ -214,6 +214,12 @@ class NativeBackend:
                               _ptr(out), _ptr(batch.cu_seqlens_q), _ptr(batch.context_lens), _ptr(block_tables),
                               block_tables.shape[1], batch.num_requests, batch.max_q_len, Hq, Hkv, page_size,
                               ctypes.c_float(scale), window, *more, _stream(), lib=self.attention_lib(D))
+        # 32 bits: by the head sizes alone, so that one model's positions are always computed by one kernel
+        if (q.dtype == torch.float32 and D % 16 == 0 and D <= 512 and E % 64 == 0 and E <= 256 and batch.num_requests <= 65535
+                and Hkv <= 65535 and all(t.data_ptr() % 16 == 0 for t in (q, k_cache, v_cache))):
+            return self._call("nhv_attention_float32", _ptr(q), _ptr(k_cache), _ptr(v_cache), _ptr(out), _ptr(batch.positions),
+                              _ptr(batch.cu_seqlens_q), _ptr(block_tables), block_tables.shape[1], batch.num_requests, batch.max_q_len,
+                              Hq, Hkv, D, E, page_size, ctypes.c_float(scale), 0 if chunk else window, chunk, *options, _stream())
         self._call("nhv_paged_attention_generic", _ptr(q), _ptr(k_cache), _ptr(v_cache), _ptr(out),
                    _ptr(batch.token_req), _ptr(batch.positions), _ptr(block_tables), block_tables.shape[1], T, Hq, Hkv,
                    D, E, page_size, ctypes.c_float(scale), 0 if chunk else window, chunk, *options, dtype_code(q), _stream())

@@ -436,6 +436,67 @@ def test_paged_attention(ops, dtype, Hq, Hkv, D, page, window):
     torch.testing.assert_close(out.double().cpu(), ref, **t)
 
 
+@pytest.mark.parametrize("Hq,Hkv,D,E,page,reach,cap,sinks,slopes,gated", [
+    (2, 2, 64, 64, 16, None, None, None, False, False), (3, 1, 16, 64, 5, ("window", 70), None, "each", False, True),
+    (8, 1, 128, 128, 64, ("chunk", 50), 3.0, "one", False, False), (34, 2, 48, 192, 256, None, None, None, True, True),
+    (4, 4, 256, 256, 7, ("window", 1), None, "each", True, False), (2, 1, 512, 128, 8, ("chunk", 64), None, None, False, False),
+])
+def test_float32_attention_of_whole_tiles(ops, Hq, Hkv, D, E, page, reach, cap, sinks, slopes, gated):
+    """The kernel on the float matrix cores with every option: row tiles that end inside a token's heads, rounds of four blocks of
+    keys and their rests, against float64; the same bits for a token alone; and a value that is no number, which reaches the
+    rows that read it and no others."""
+    import dataclasses
+    lens, q_lens = [1, 64, 65, 300, 17, 513, 5, 257], [1, 64, 1, 43, 2, 30, 5, 1]
+    q, kc, _, batch, bt, ks, _, qs = _paged_setup(torch.float32, lens, q_lens, Hq, Hkv, D, page, seed=61)
+    g = torch.Generator().manual_seed(62)
+    vc = torch.full((*kc.shape[:3], E), float("nan"))
+    vs = [torch.randn(n, Hkv, E, generator=g) for n in lens]
+    for r, v in enumerate(vs):
+        for p in range(len(v)):
+            vc[bt[r, p // page], p % page] = v[p]
+    vc = vc.cuda()
+    rows = torch.randn(q.shape[0], Hq + 3, generator=g)
+    slope = torch.rand(Hq, generator=g) * 0.1 if slopes else None
+    sink = {None: None, "one": 0.7, "each": torch.randn(Hq, generator=g)}[sinks]
+    options = {"softcap": cap, "slopes": None if slope is None else slope.cuda(), "sink": sink.cuda() if sinks == "each" else sink,
+               "gate": (rows.cuda(), 2) if gated else None, **({reach[0]: reach[1]} if reach else {})}
+    out = ops.paged_attention(q, kc, vc, batch, bt, D ** -0.5, **options)
+    want, reads, at = [], [], 0
+    for r, (n, nq) in enumerate(zip(lens, q_lens)):
+        group = Hq // Hkv
+        pos, key = torch.arange(n - nq, n)[:, None], torch.arange(n)[None]
+        ok = key <= pos
+        if reach:
+            ok &= key > pos - reach[1] if reach[0] == "window" else key // reach[1] == pos // reach[1]
+        s = torch.einsum("qhd,khd->hqk", qs[r].double(), ks[r].double().repeat_interleave(group, 1)) * D ** -0.5
+        s = cap * torch.tanh(s / cap) if cap else s
+        s = s - slope.double()[:, None, None] * (pos - key) if slopes else s
+        s = s.masked_fill(~ok, float("-inf"))
+        if sinks:
+            s = torch.cat((s, torch.as_tensor(sink, dtype=torch.float64).expand(Hq)[:, None, None].expand(Hq, nq, 1)), -1)
+        o = torch.einsum("hqk,khd->qhd", torch.softmax(s, -1)[..., :n], vs[r].double().repeat_interleave(group, 1))
+        want.append(o * torch.sigmoid(rows[at:at + nq, 2:2 + Hq].double())[..., None] if gated else o)
+        reads.append(ok[:, n - 2:n - 1].any(-1) if n > 1 else torch.zeros(nq, dtype=torch.bool))
+        at += nq
+    torch.testing.assert_close(out.double().cpu(), torch.cat(want), rtol=1e-5, atol=1e-5)
+    last = dataclasses.replace(batch, num_tokens=1, num_requests=1, token_req=torch.zeros(1, dtype=torch.int32, device="cuda"),
+                               positions=batch.positions[-1:], cu_seqlens_q=torch.tensor([0, 1], dtype=torch.int32, device="cuda"),
+                               context_lens=batch.context_lens[-1:], max_q_len=1)
+    if gated:
+        options["gate"] = (rows[-1:].cuda(), 2)
+    alone = ops.paged_attention(q[-1:].contiguous(), kc, vc, last, bt[7:8].contiguous(), D ** -0.5, **options)
+    assert torch.equal(alone, out[-1:])
+    if gated:
+        options["gate"] = (rows.cuda(), 2)
+    for r, n in enumerate(lens):
+        if n > 1:
+            vc[bt[r, (n - 2) // page], (n - 2) % page] = float("inf")
+    spoilt = ops.paged_attention(q, kc, vc, batch, bt, D ** -0.5, **options)
+    hit = torch.cat(reads)
+    assert not torch.isfinite(spoilt[hit.cuda()]).any()
+    torch.testing.assert_close(spoilt[~hit.cuda()], out[~hit.cuda()], rtol=1e-5, atol=1e-5)
+
+
 @pytest.mark.parametrize("Hq,Hkv,D,page,window", [
     (4, 2, 16, 4, None), (6, 1, 32, 8, None), (5, 5, 48, 7, None), (3, 1, 80, 16, 9), (8, 2, 128, 64, None),
     (32, 8, 128, 256, None), (16, 1, 64, 5, 70), (7, 7, 112, 3, None), (2, 1, 256, 32, None), (12, 2, 96, 16, 300),
