@@ -2,26 +2,29 @@
 // for key heads of a multiple of 16 entries and value heads of 64, 128, 192 or 256; masks and options are those of
 // attention_generic.hip, which takes the other sizes.
 //
-// Keys are taken in blocks of 64 aligned to absolute positions. Each block's maximum, sum and weighted values are computed by
+// Keys are taken in blocks of 32 aligned to absolute positions. Each block's maximum, sum and weighted values are computed by
 // themselves and merged in rising order, masked keys count as nothing, so a position's result depends neither on the batch
 // nor on the portion, nor on which wave took a block.
 //
-// A block of 4 waves owns 16 rows, a row being (token, one of the query heads that read one key/value head), of one request:
+// A block of 8 waves owns 16 rows, a row being (token, one of the query heads that read one key/value head), of one request:
 // 8 tokens of a prompt where two heads share a key head, or one decoded token. The waves take the blocks of keys in turn;
-// after each round of four blocks the results meet in LDS and are merged. Scores come as S^T = K Q^T, whose layout is
+// after each round of eight blocks the results meet in LDS and are merged. Scores come as S^T = K Q^T, whose layout is
 // that of the second product's right operand (O^T = V^T P^T), so the weights never leave their registers.
-// What bounds it: the chain of rounds of a row tile (32 KB of keys and values a wave and round at 128 entries) while the chip
-// is not full, else the matrix cores.
+// What bounds it: the chain of rounds of a row tile, half of it matrix instructions, the rest exponentials and the merge, which
+// a block's barrier keeps from overlapping (next round's loads asked for before the merge: no faster). 16 heads on 8 key heads
+// of 128: a prompt of 517 tokens 55 us (four waves with blocks of 64 keys and conditional loads 63), six tokens after 100
+// 9 us (29), eight after 3,000 132 us.
 #include "nhv_common.h"
 #include <math.h>
 
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
-#define WAVES 4
+#define WAVES 8
 #define ROWS 16
-#define KEYS 64
+#define KEYS 32
+#define TILES (KEYS / 16)
 #define MAX_E 256
-#define MAX_D 512
+#define MAX_D 256
 
 struct FloatAttention {
   const float *q, *k, *v;
@@ -45,7 +48,7 @@ __global__ __launch_bounds__(64 * WAVES) void attention_float32_kernel(FloatAtte
   float* stats = part + WAVES * ROWS * (E + 4);          // [WAVES][ROWS][2]: maximum and sum
   const int kvh = blockIdx.y, req = blockIdx.z;
   const int first = a.cu[req], rows = (a.cu[req + 1] - first) * group;
-  const int row0 = blockIdx.x * ROWS;
+  const int row0 = (gridDim.x - 1 - blockIdx.x) * ROWS;  // (the tiles with the longest chains of keys first)
   if (row0 >= rows) return;                              // (the same for the whole block)
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, r16 = lane & 15, g = lane >> 4;
 
@@ -73,42 +76,66 @@ __global__ __launch_bounds__(64 * WAVES) void attention_float32_kernel(FloatAtte
   }
   __syncthreads();
 
-  // what a thread merges: 16 threads a row, entries c + 16 i
-  const int my_row = threadIdx.x >> 4, c = threadIdx.x & 15;
-  float M = -INFINITY, L = 0.f, total[MAX_E / 16];
+  // what a thread merges: 32 threads a row, entries c + 32 i
+  const int my_row = threadIdx.x / (4 * WAVES), c = threadIdx.x % (4 * WAVES);
+  float M = -INFINITY, L = 0.f, total[MAX_E / (4 * WAVES)];
 #pragma unroll
-  for (int i = 0; i < MAX_E / 16; ++i) total[i] = 0.f;
+  for (int i = 0; i < MAX_E / (4 * WAVES); ++i) total[i] = 0.f;
 
   for (int round = tile_lo / KEYS * KEYS; round <= tile_hi; round += KEYS * WAVES) {
     const int kb = round + wave * KEYS;
     if (kb <= tile_hi) {
-      // lane l's own key of the block, and where it lies (-1: no row reads it)
-      const int own = kb + lane;
-      int slot = -1;
-      if (own >= tile_lo && own <= tile_hi) slot = table[own / a.page_size] * a.page_size + own % a.page_size;
-      f32x4 s[4];
-      const float* kr[4];
+      // lane l's own key of the block, and where it lies. A key that no row reads is taken for the tile's last: its score is
+      // masked, and every load is without a condition (with one the compiler waits for all that are under way).
+      const int mine = kb + lane % KEYS, own = mine >= tile_lo && mine <= tile_hi ? mine : tile_hi;
+      const int slot = table[own / a.page_size] * a.page_size + own % a.page_size;
+      f32x4 s[TILES], kf[2][2][TILES], vf[TILES][4];
+      const float *kr[TILES], *vr[TILES][4];
 #pragma unroll
-      for (int t = 0; t < 4; ++t) {
-        const int at = __shfl(slot, 16 * t + r16, NHV_WAVE);
-        kr[t] = at >= 0 ? a.k + ((size_t)at * a.Hkv + kvh) * D + 4 * g : nullptr;
+      for (int t = 0; t < TILES; ++t) {
+        kr[t] = a.k + ((size_t)__shfl(slot, 16 * t + r16, NHV_WAVE) * a.Hkv + kvh) * D + 4 * g;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) vr[t][i] = a.v + ((size_t)__shfl(slot, 16 * t + 4 * g + i, NHV_WAVE) * a.Hkv + kvh) * E + 4 * r16;
         s[t] = f32x4{0.f, 0.f, 0.f, 0.f};
       }
-#pragma unroll 4
-      for (int d = 0; d < D; d += 16) {
-        const f32x4 qf = *reinterpret_cast<const f32x4*>(&qs[r16 * (D + 4) + d + 4 * g]);
-        f32x4 kf[4];
+      // keys two blocks of 16 entries ahead (the last one again where there are no two); the first 64 value entries at once
+      auto ask = [&](int buf, int d) {
 #pragma unroll
-        for (int t = 0; t < 4; ++t) kf[t] = kr[t] ? *reinterpret_cast<const f32x4*>(kr[t] + d) : f32x4{0.f, 0.f, 0.f, 0.f};
+        for (int u = 0; u < 2; ++u)
+#pragma unroll
+          for (int t = 0; t < TILES; ++t) kf[buf][u][t] = *reinterpret_cast<const f32x4*>(kr[t] + min(d + 16 * u, D - 16));
+      };
+      auto score = [&](int buf, int d, int u) {
+        const f32x4 qf = *reinterpret_cast<const f32x4*>(&qs[r16 * (D + 4) + d + 16 * u + 4 * g]);
 #pragma unroll
         for (int j = 0; j < 4; ++j)
 #pragma unroll
-          for (int t = 0; t < 4; ++t) s[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[t][j], qf[j], s[t], 0, 0, 0);
+          for (int t = 0; t < TILES; ++t) s[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[buf][u][t][j], qf[j], s[t], 0, 0, 0);
+      };
+      ask(0, 0);
+#pragma unroll
+      for (int t = 0; t < TILES; ++t)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) vf[t][i] = *reinterpret_cast<const f32x4*>(vr[t][i]);
+      int d = 0;
+      for (; d + 64 <= D; d += 64) {
+        ask(1, d + 32);
+        score(0, d, 0);
+        score(0, d, 1);
+        ask(0, d + 64);
+        score(1, d + 32, 0);
+        score(1, d + 32, 1);
+      }
+      if (d < D) {                                       // 16, 32 or 48 entries more
+        ask(1, d + 32);
+        score(0, d, 0);
+        if (d + 16 < D) score(0, d, 1);
+        if (d + 32 < D) score(1, d + 32, 0);
       }
       // s[t][i]: key kb + 16 t + 4 g + i against row r16
       float m = -INFINITY;
 #pragma unroll
-      for (int t = 0; t < 4; ++t)
+      for (int t = 0; t < TILES; ++t)
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
           const int key = kb + 16 * t + 4 * g + i;
@@ -123,7 +150,7 @@ __global__ __launch_bounds__(64 * WAVES) void attention_float32_kernel(FloatAtte
       const float base = m == -INFINITY ? 0.f : m;       // (no visible key: every weight is 0)
       float l = 0.f;
 #pragma unroll
-      for (int t = 0; t < 4; ++t)
+      for (int t = 0; t < TILES; ++t)
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
           s[t][i] = expf(s[t][i] - base);
@@ -135,24 +162,24 @@ __global__ __launch_bounds__(64 * WAVES) void attention_float32_kernel(FloatAtte
         stats[(wave * ROWS + r16) * 2] = m;
         stats[(wave * ROWS + r16) * 2 + 1] = l;
       }
-      // value entry h + 4 r + j of a chunk of 64 is row r of matrix tile j: one load of 16 bytes a key feeds four tiles
+      // value entry h + 4 r + j of a chunk of 64 is row r of matrix tile j: one load of 16 bytes a key feeds four tiles. The next
+      // chunk is asked for as this one is used up.
       for (int h = 0; h < E; h += 64) {
+        const int next = min(h + 64, E - 64);
         f32x4 o[4];
 #pragma unroll
         for (int j = 0; j < 4; ++j) o[j] = f32x4{0.f, 0.f, 0.f, 0.f};
         float odd = 0.f;                                 // not a number as soon as some value is infinite or none
 #pragma unroll
-        for (int t = 0; t < 4; ++t)
+        for (int t = 0; t < TILES; ++t)
 #pragma unroll
           for (int i = 0; i < 4; ++i) {
-            const int at = __shfl(slot, 16 * t + 4 * g + i, NHV_WAVE);
-            const f32x4 vf = at >= 0 ? *reinterpret_cast<const f32x4*>(a.v + ((size_t)at * a.Hkv + kvh) * E + h + 4 * r16)
-                                     : f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
-              odd = fmaf(vf[j], 0.f, odd);
-              o[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(vf[j], s[t][i], o[j], 0, 0, 0);
+              odd = fmaf(vf[t][i][j], 0.f, odd);
+              o[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(vf[t][i][j], s[t][i], o[j], 0, 0, 0);
             }
+            vf[t][i] = *reinterpret_cast<const f32x4*>(vr[t][i] + next);
           }
         // o[j][i]: row r16, entry h + 16 g + 4 i + j
         if (__any(odd != 0.f)) {
@@ -160,18 +187,18 @@ __global__ __launch_bounds__(64 * WAVES) void attention_float32_kernel(FloatAtte
 #pragma unroll
           for (int j = 0; j < 4; ++j) o[j] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-          for (int t = 0; t < 4; ++t)
+          for (int t = 0; t < TILES; ++t)
 #pragma unroll
             for (int i = 0; i < 4; ++i)
               for (int gk = 0; gk < 4; ++gk) {
                 const int at = __shfl(slot, 16 * t + 4 * gk + i, NHV_WAVE);
                 const float p = __shfl(s[t][i], 16 * gk + r16, NHV_WAVE);
-                if (p != 0.f && at >= 0) {
-                  const float* vr = a.v + ((size_t)at * a.Hkv + kvh) * E + h + 16 * g;
+                if (p != 0.f) {
+                  const float* row_v = a.v + ((size_t)at * a.Hkv + kvh) * E + h + 16 * g;
 #pragma unroll
                   for (int ii = 0; ii < 4; ++ii)
 #pragma unroll
-                    for (int j = 0; j < 4; ++j) o[j][ii] = fmaf(p, vr[4 * ii + j], o[j][ii]);
+                    for (int j = 0; j < 4; ++j) o[j][ii] = fmaf(p, row_v[4 * ii + j], o[j][ii]);
                 }
               }
         }
@@ -188,8 +215,8 @@ __global__ __launch_bounds__(64 * WAVES) void attention_float32_kernel(FloatAtte
       L = L * old + l * now;
       M = top;
 #pragma unroll
-      for (int i = 0; i < MAX_E / 16; ++i)
-        if (16 * i < E) total[i] = total[i] * old + part[(p * ROWS + my_row) * (E + 4) + c + 16 * i] * now;
+      for (int i = 0; i < MAX_E / (4 * WAVES); ++i)
+        if (4 * WAVES * i < E) total[i] = total[i] * old + part[(p * ROWS + my_row) * (E + 4) + c + 4 * WAVES * i] * now;
     }
     __syncthreads();
   }
@@ -207,8 +234,8 @@ __global__ __launch_bounds__(64 * WAVES) void attention_float32_kernel(FloatAtte
   if (a.gate) inv /= 1.0f + expf(-a.gate[(size_t)t * a.gate_ld + h]);
   float* o = a.out + ((size_t)t * a.Hq + h) * E;
 #pragma unroll
-  for (int i = 0; i < MAX_E / 16; ++i)
-    if (16 * i < E) o[c + 16 * i] = total[i] * inv;
+  for (int i = 0; i < MAX_E / (4 * WAVES); ++i)
+    if (4 * WAVES * i < E) o[c + 4 * WAVES * i] = total[i] * inv;
 }
 
 extern "C" int nhv_attention_float32(const void* q, const void* k_cache, const void* v_cache, void* out, const void* positions,

@@ -215,7 +215,7 @@ class NativeBackend:
                               block_tables.shape[1], batch.num_requests, batch.max_q_len, Hq, Hkv, page_size,
                               ctypes.c_float(scale), window, *more, _stream(), lib=self.attention_lib(D))
         # 32 bits: by the head sizes alone, so that one model's positions are always computed by one kernel
-        if (q.dtype == torch.float32 and D % 16 == 0 and D <= 512 and E % 64 == 0 and E <= 256 and batch.num_requests <= 65535
+        if (q.dtype == torch.float32 and D % 16 == 0 and D <= 256 and E % 64 == 0 and E <= 256 and batch.num_requests <= 65535
                 and Hkv <= 65535 and all(t.data_ptr() % 16 == 0 for t in (q, k_cache, v_cache))):
             return self._call("nhv_attention_float32", _ptr(q), _ptr(k_cache), _ptr(v_cache), _ptr(out), _ptr(batch.positions),
                               _ptr(batch.cu_seqlens_q), _ptr(block_tables), block_tables.shape[1], batch.num_requests, batch.max_q_len,

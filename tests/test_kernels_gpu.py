@@ -439,10 +439,10 @@ def test_paged_attention(ops, dtype, Hq, Hkv, D, page, window):
 @pytest.mark.parametrize("Hq,Hkv,D,E,page,reach,cap,sinks,slopes,gated", [
     (2, 2, 64, 64, 16, None, None, None, False, False), (3, 1, 16, 64, 5, ("window", 70), None, "each", False, True),
     (8, 1, 128, 128, 64, ("chunk", 50), 3.0, "one", False, False), (34, 2, 48, 192, 256, None, None, None, True, True),
-    (4, 4, 256, 256, 7, ("window", 1), None, "each", True, False), (2, 1, 512, 128, 8, ("chunk", 64), None, None, False, False),
+    (4, 4, 256, 256, 7, ("window", 1), None, "each", True, False), (2, 1, 240, 128, 8, ("chunk", 64), None, None, False, False),
 ])
 def test_float32_attention_of_whole_tiles(ops, Hq, Hkv, D, E, page, reach, cap, sinks, slopes, gated):
-    """The kernel on the float matrix cores with every option: row tiles that end inside a token's heads, rounds of four blocks of
+    """The kernel on the float matrix cores with every option: row tiles that end inside a token's heads, rounds of eight blocks of
     keys and their rests, against float64; the same bits for a token alone; and a value that is no number, which reaches the
     rows that read it and no others."""
     import dataclasses
