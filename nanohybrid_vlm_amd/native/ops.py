@@ -19,7 +19,7 @@ import torch
 from . import library
 
 CORE_SOURCES = ["error.hip", "elementwise.hip", "gemm_generic.hip", "gemm_float32.hip", "gemm_skinny_bf16.hip", "gemm_fewrows_bf16.hip",
-                "attention_generic.hip", "attention_float32.hip", "sampling.hip", "measure.hip", "stream_mixing.hip", "delta_rule.hip", "parallel_block.hip", "latent_attention.hip",
+                "attention_generic.hip", "attention_float32.hip", "sampling.hip", "measure.hip", "stream_mixing.hip", "delta_rule.hip", "delta_chunks.hip", "parallel_block.hip", "latent_attention.hip",
                 "routed_experts.hip", "hyper_streams.hip", "head_outputs.hip", "sandwich_norms.hip", "linear_recurrence.hip"]
 BLAS_SOURCES = ["error.hip", "gemm_library.hip"]                                                   # the vendor's matrix library, algorithm by number
 BLAS_LINK = ["-lhipblaslt"]
@@ -304,6 +304,24 @@ class NativeBackend:
         self._call("nhv_delta_rule", _ptr(q), _ptr(k), _ptr(v), _ptr(decay), _ptr(beta), _ptr(state), _ptr(out),
                    _ptr(batch.positions), _ptr(batch.cu_seqlens_q), _ptr(state_slots), batch.num_requests, H, G, D, E,
                    max(1, batch.max_q_len), decay.shape[2], _stream())
+
+    def delta_chunks(self, proj, taps, kept, a_lin, a_col, dt_bias, a_log, state, out, batch, state_slots, H, G, D, E, decay_dim):
+        """``delta_prepare`` and ``delta_rule`` for portions of prompts, 16 tokens at a time (``kept`` is only read)."""
+        T, B, C = proj.shape[0], batch.num_requests, 16
+        Dp, longest = -(-D // 16) * 16, max(1, batch.max_q_len)
+        places = T // C + B + 1
+        w = torch.empty((places, H, C, Dp), dtype=torch.float32, device=proj.device)
+        r, k = torch.empty_like(w), torch.empty_like(w)
+        v = torch.empty((places, H, E, C), dtype=torch.float32, device=proj.device)
+        b = torch.empty((places, H, C, C), dtype=torch.float32, device=proj.device)
+        decay = torch.empty((places, H, Dp), dtype=torch.float32, device=proj.device)
+        LL = ctypes.c_longlong
+        self._call("nhv_delta_chunks_prepare", _ptr(proj), dtype_code(proj), LL(proj.shape[1]), _ptr(taps), taps.shape[1], _ptr(kept),
+                   ctypes.c_void_p(a_lin.data_ptr() + 4 * a_col), LL(a_lin.shape[1]), _ptr(dt_bias), _ptr(a_log), _ptr(batch.positions),
+                   _ptr(batch.cu_seqlens_q), _ptr(state_slots), _ptr(w), _ptr(r), _ptr(k), _ptr(v), _ptr(b), _ptr(decay), B, H, G, D, E,
+                   decay_dim, longest, _stream())
+        self._call("nhv_delta_chunks", _ptr(w), _ptr(r), _ptr(k), _ptr(v), _ptr(b), _ptr(decay), _ptr(state), _ptr(out),
+                   _ptr(batch.positions), _ptr(batch.cu_seqlens_q), _ptr(state_slots), B, H, D, E, _stream())
 
     def gated_head_norm(self, o, gate, w, y, eps, gate_col=0, gate_act=0):
         """``gate`` [tokens, columns] float32: the gates of (t, h, e) from column ``gate_col`` on; ``gate_act`` 0: the
@@ -1651,6 +1669,7 @@ class WKV:
 
 FEW_TOKENS = 4                # up to so many tokens a request, a recurrence is one kernel from projections to gated read-out
 RECURRENCE_KEY_DIM = 256      # the largest key head that the recurrences take
+DELTA_CHUNK_TOKENS = 16       # from portions of so many tokens on, the delta rule takes sixteen tokens at a time
 
 
 def token_shift(h: torch.Tensor, mu: torch.Tensor, kept: torch.Tensor, batch: AttentionBatch, state_slots: torch.Tensor) -> torch.Tensor:
@@ -2044,7 +2063,7 @@ def gated_delta_rule(proj: torch.Tensor, a_lin: torch.Tensor | None, gate_lin: t
     order from and into ``state`` [slots, heads, value_dim, head_dim] (a request whose first token is at position 0
     starts from zero), then per head the read-out over its root mean square times ``norm_weight`` times
     f(gate_lin), f = ``gate_activation`` ("sigmoid", or "silu": z sigmoid(z)). Returns [tokens, heads * value_dim]
-    in ``out_dtype``. ``a_lin`` is overwritten with the decays. ``a_lin`` and ``gate_lin`` None: ``proj`` is float32
+    in ``out_dtype``. ``a_lin`` may be overwritten. ``a_lin`` and ``gate_lin`` None: ``proj`` is float32
     and holds them as further columns, q | k | v | beta | a | gate (one product made them all)."""
     T = proj.shape[0]
     H, G, D, E = num_heads, num_kv_heads, head_dim, value_dim
@@ -2080,10 +2099,6 @@ def gated_delta_rule(proj: torch.Tensor, a_lin: torch.Tensor | None, gate_lin: t
     _dense(batch.cu_seqlens_q, "gated_delta_rule: cu_seqlens_q", (B + 1,), torch.int32)
     _dense(state_slots, "gated_delta_rule: state_slots", (B,), torch.int32)
     dev = proj.device
-    q = torch.empty((T, G, D), dtype=torch.float32, device=dev)
-    k = torch.empty((T, G, D), dtype=torch.float32, device=dev)
-    v = torch.empty((T, H, E), dtype=torch.float32, device=dev)
-    beta = torch.empty((T, H), dtype=torch.float32, device=dev)
     o = torch.empty((T, H, E), dtype=torch.float32, device=dev)
     y = torch.empty((T, H * E), dtype=out_dtype, device=dev)
     dtype_code(y)
@@ -2091,18 +2106,29 @@ def gated_delta_rule(proj: torch.Tensor, a_lin: torch.Tensor | None, gate_lin: t
         return y
     b = backend()
     act = {"gate_act": 1} if gate_activation == "silu" else {}
-    if packed:
-        decay = torch.empty((T, H, Dd), dtype=torch.float32, device=dev)
-        b.delta_prepare(proj, taps, kept, proj, dt_bias, a_log, batch, state_slots, q, k, v, beta, H, G, D, E, decay=decay,
-                        a_col=C + H)
-    elif decay_per_head:
-        decay = a_lin.view(T, H, 1)
-        b.delta_prepare(proj, taps, kept, a_lin, dt_bias, a_log, batch, state_slots, q, k, v, beta, H, G, D, E, decay=decay)
+    # A run in 32 bits takes its tokens one by one whatever the portions, so that its results do not depend on how a prompt is
+    # cut; otherwise portions go sixteen tokens at a time (the sums within sixteen tokens are ordered differently).
+    if y.dtype != torch.float32 and batch.max_q_len >= DELTA_CHUNK_TOKENS and D <= RECURRENCE_KEY_DIM and hasattr(b, "delta_chunks"):
+        b.delta_chunks(proj, taps, kept, proj if packed else a_lin, C + H if packed else 0, dt_bias, a_log, state, o, batch, state_slots,
+                       H, G, D, E, Dd)
+        b.conv_state_update(proj, kept, n, batch, state_slots, C)
     else:
-        decay = a_lin.view(T, H, D)
-        b.delta_prepare(proj, taps, kept, a_lin, dt_bias, a_log, batch, state_slots, q, k, v, beta, H, G, D, E)
-    b.conv_state_update(proj, kept, n, batch, state_slots, C)
-    b.delta_rule(q, k, v, decay, beta, state, o, batch, state_slots)
+        q = torch.empty((T, G, D), dtype=torch.float32, device=dev)
+        k = torch.empty((T, G, D), dtype=torch.float32, device=dev)
+        v = torch.empty((T, H, E), dtype=torch.float32, device=dev)
+        beta = torch.empty((T, H), dtype=torch.float32, device=dev)
+        if packed:
+            decay = torch.empty((T, H, Dd), dtype=torch.float32, device=dev)
+            b.delta_prepare(proj, taps, kept, proj, dt_bias, a_log, batch, state_slots, q, k, v, beta, H, G, D, E, decay=decay,
+                            a_col=C + H)
+        elif decay_per_head:
+            decay = a_lin.view(T, H, 1)
+            b.delta_prepare(proj, taps, kept, a_lin, dt_bias, a_log, batch, state_slots, q, k, v, beta, H, G, D, E, decay=decay)
+        else:
+            decay = a_lin.view(T, H, D)
+            b.delta_prepare(proj, taps, kept, a_lin, dt_bias, a_log, batch, state_slots, q, k, v, beta, H, G, D, E)
+        b.conv_state_update(proj, kept, n, batch, state_slots, C)
+        b.delta_rule(q, k, v, decay, beta, state, o, batch, state_slots)
     if packed:
         b.gated_head_norm(o, proj, norm_weight, y.view(T, H, E), float(eps), gate_col=C + H + H * Dd, **act)
     else:

@@ -964,3 +964,63 @@ def test_attention_kernels_at_random_sizes(ops, Hq, Hkv, D, page, window, seed):
     out = ops.paged_attention(q, kc, vc, batch, bt, scale, window)
     torch.testing.assert_close(out.double().cpu(), _attention_reference(qs, ks, vs, lens, q_lens, scale, window),
                                **tol(torch.bfloat16))
+
+
+@pytest.mark.parametrize("H,G,D,E,taps,per_head,packed,lengths", [
+    (2, 1, 16, 16, 4, False, False, [16, 17]), (3, 3, 20, 5, 1, False, False, [40, 1, 31]), (2, 2, 128, 128, 4, False, False, [100]),
+    (4, 2, 72, 40, 5, True, True, [15, 33, 2]), (1, 1, 200, 24, 4, False, False, [64, 3]), (2, 1, 256, 100, 3, True, True, [19]),
+    (1, 1, 3, 3, 16, False, False, [50]),
+])
+def test_delta_rule_sixteen_tokens_at_a_time(ops, H, G, D, E, taps, per_head, packed, lengths):
+    """Portions that end inside a chunk and on its edge, beside requests of fewer tokens; a second portion goes on from the state
+    and the kept inputs of the first; weak and very strong decays. State and result against the recurrence token by token in
+    float64. The state is 32 bits: sums of 16 products a chunk of entries below 1 are off by some 16 roundings of 2^-24 each,
+    and a chunk's error decays or stays; the result is one bfloat16 rounding of what follows from it."""
+    import plain_pevazen as plain
+    from nanohybrid_vlm_amd.native.ops import AttentionBatch
+    g = torch.Generator().manual_seed(71)
+    C, Dd, B = 2 * G * D + H * E, 1 if per_head else D, len(lengths)
+    total = [n + 18 for n in lengths]                      # a portion of 18 more for every request
+    proj = [torch.randn(n, C + H, generator=g) for n in total]
+    a_lin = [3.0 * torch.randn(n, H * Dd, generator=g) for n in total]
+    a_lin[0][5:8] = 60.0                                   # decays that are zero in 32 bits
+    gates = [torch.randn(n, H * E, generator=g) for n in total]
+    tap, dt_bias = 0.6 * torch.randn(C, taps, generator=g), torch.randn(H * Dd, generator=g) - 0.5
+    a_log, norm = 0.5 * torch.randn(H, generator=g) - 0.5, 1.0 + 0.2 * torch.randn(E, generator=g)
+    kept = torch.full((B + 1, C, taps - 1), float("nan")).cuda()
+    state = torch.full((B + 1, H, E, D), float("nan")).cuda()
+    slots = torch.arange(B, 0, -1).to(torch.int32)
+    got = [[] for _ in lengths]
+    for lo, hi in (([0] * B, lengths), (lengths, total)):
+        at = [torch.arange(a, b) for a, b in zip(lo, hi)]
+        batch = AttentionBatch(num_tokens=sum(map(len, at)), num_requests=B,
+                               token_req=torch.repeat_interleave(torch.arange(B), torch.tensor([len(a) for a in at])).to(torch.int32).cuda(),
+                               positions=torch.cat(at).to(torch.int32).cuda(),
+                               cu_seqlens_q=torch.tensor([0] + [len(a) for a in at]).cumsum(0).to(torch.int32).cuda(),
+                               context_lens=torch.tensor(hi, dtype=torch.int32).cuda(), max_q_len=max(map(len, at)), max_context_len=max(hi))
+        rows = lambda x: torch.cat([t[a] for t, a in zip(x, at)]).cuda()
+        p, a, z = rows(proj), rows(a_lin), rows(gates)
+        y = ops.gated_delta_rule(torch.cat((p, a, z), 1) if packed else p, None if packed else a, None if packed else z, tap.cuda(),
+                                 dt_bias.cuda(), a_log.cuda(), norm.cuda(), 1e-5, kept, state, batch, slots.cuda(), H, G, D, E,
+                                 torch.bfloat16, decay_per_head=per_head)
+        for i, part in enumerate(y.float().cpu().split([len(a) for a in at])):
+            got[i].append(part)
+    for i, n in enumerate(total):
+        x = proj[i].double()
+        act = plain.silu(plain.causal_taps(x[:, :C], tap.double()))
+        unit = lambda t: t / torch.sqrt(t.pow(2).sum(-1, keepdim=True) + 1e-6)
+        q = unit(act[:, :G * D].view(n, G, D)).repeat_interleave(H // G, dim=1) * D ** -0.5
+        k = unit(act[:, G * D:2 * G * D].view(n, G, D)).repeat_interleave(H // G, dim=1)
+        v, beta = act[:, 2 * G * D:].view(n, H, E), torch.sigmoid(x[:, C:])
+        decay = torch.exp(-torch.exp(a_log.double())[None, :, None] * plain.softplus((a_lin[i] + dt_bias).double()).view(n, H, Dd)).expand(n, H, D)
+        S = torch.zeros(H, D, E, dtype=torch.float64)
+        want = []
+        for t in range(n):
+            S = decay[t][..., None] * S
+            u = beta[t][:, None] * (v[t] - torch.einsum("hde,hd->he", S, k[t]))
+            S = S + k[t][..., None] * u[:, None]
+            want.append(torch.einsum("hde,hd->he", S, q[t]))
+        torch.testing.assert_close(state[int(slots[i])].double().cpu(), S.transpose(1, 2), rtol=1e-5, atol=2e-6)
+        want = (plain.unit_rms(torch.stack(want), 1e-5) * norm * torch.sigmoid(gates[i].double()).view(n, H, E)).reshape(n, H * E)
+        torch.testing.assert_close(torch.cat(got[i]).double(), want, rtol=1e-2, atol=2e-3)
+    assert state[0].isnan().all()                          # a slot that no request holds is left alone
