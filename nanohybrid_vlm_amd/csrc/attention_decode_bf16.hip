@@ -1,8 +1,8 @@
 // Attention of single tokens over the paged cache in bfloat16, split over the keys.
 // Compiled for one head size: -DNHV_HEAD_DIM=<multiple of 16>.
 //
-// One wave works on (token, key/value head, up to 16 of the query heads that share it, split of
-// the keys). The query heads are the 16 columns of the MFMA tiles (more than 16 heads on one
+// A block works on (token, key/value head, up to 16 of the query heads that share it, split of
+// the keys), its waves on rounds of 32 keys in turn. The query heads are the 16 columns of the MFMA tiles (more than 16 heads on one
 // key/value head, as over a cached latent, are several waves that read the same keys):
 //   S^T[key, head]  = K[key, :] . Q[head, :]        K rows straight from the cache (v_mfma_f32_16x16x32_bf16)
 //   running maximum per head in float (two shuffles), sums kept per lane
@@ -15,8 +15,9 @@
 // product sums them, so P never leaves the registers, and a lane's outputs belong to
 // the head of its scores: rescaling needs no exchange. Splits are aligned to absolute
 // key positions. Each split writes its unnormalised output with (maximum, sum) in
-// float; a second kernel merges the splits in rising order. Keys that are not visible
-// are loaded as zeros (the cache's unused slots may hold anything).
+// float; a second kernel merges the splits in rising order (with one split the block
+// writes the result). Only visible keys are loaded (the cache's unused slots may hold
+// anything).
 // What a layer may ask for besides (the entry point ..._more): a cap on the scores (s <- cap tanh(s / cap), after the
 // scale; taken on the float scores where they leave the first product), a bias that grows with the distance (BIASED:
 // slopes[head] * (query position - key position) is taken off the float score after scale and cap), one more term
@@ -66,15 +67,34 @@ __device__ __forceinline__ int slot_of(const int* bt, int key, int page_size, in
 
 // CAPPED: the scores pass cap tanh(s scale / cap). cap_l2 = cap log2(e); tanh_k = 2 log2(e) scale / cap, so that
 // tanh(x) = 1 - 2 / (1 + exp(2 x)) costs one exp2 and one reciprocal (an overflowing exp2 gives the limit 1).
+// A block's waves take the rounds of its split in turn and meet in LDS at the end. One split in all: the block writes the
+// result itself and there is nothing to merge. Eight waves against one (a wave then is a split): 9.1 -> 6.1 us for one token
+// after 150 keys of 8 key heads, 57 -> 53 us for 32 after 2,050, where no merge follows; 23 -> 21.5 us for 8 after 2,050, where
+// one follows over a quarter as many splits. Two blocks fill a compute unit's LDS. (The next round's keys and values asked
+// for before this one is computed: more than 256 registers, one wave a SIMD, and 2 to 10 % more time.)
+constexpr int WAVES = D <= 128 ? 8 : 4;
+constexpr int TURN = D <= 64 ? 2 : 1;                       // rounds a wave takes before the next wave's: 16 KB and more of keys and values
+constexpr int OPITCH = D + 4;                               // floats a head in the waves' meeting place, which lies where a wave's V^T tile was
+constexpr int MEET = 16 * OPITCH * 4 + 16 * 2 * 4;          // bytes: 16 heads' sums, maxima and sums of weights
+constexpr int TILE = D * VPITCH * 2 > MEET ? D * VPITCH * 2 : MEET;
+
+struct Finish {                                             // what follows the sums: one more term in the denominator, a gate
+  float sink_l2;
+  const float* sinks;
+  const bf16_t* gate;
+  long long gate_ld;
+};
+
 template <bool CAPPED, bool BIASED>
-__global__ __launch_bounds__(64) void decode_attention_kernel(
+__global__ __launch_bounds__(64 * WAVES) void decode_attention_kernel(
     const bf16_t* __restrict__ q, const bf16_t* __restrict__ k_cache, const bf16_t* __restrict__ v_cache,
-    float* __restrict__ part_o, float* __restrict__ part_ml, const int* __restrict__ token_req,
+    float* __restrict__ part_o, float* __restrict__ part_ml, bf16_t* __restrict__ out, const int* __restrict__ token_req,
     const int* __restrict__ positions, const int* __restrict__ block_tables, int max_blocks, int Hq, int Hkv,
     int page_size, int page_shift, float scale_log2e, int window, int split_len, int n_splits, float cap_l2, float tanh_k,
-    const float* __restrict__ slopes) {
-  __shared__ __attribute__((aligned(16))) bf16_t vt_s[D * VPITCH];
-  const int lane = threadIdx.x;
+    const float* __restrict__ slopes, const Finish finish) {
+  __shared__ __attribute__((aligned(16))) char tiles_s[WAVES][TILE];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  bf16_t* vt_s = reinterpret_cast<bf16_t*>(tiles_s[wave]);
   // blocks go to the eight XCDs in turn by their linear index: with the split as the slowest index every XCD
   // gets the same share of each split (the last splits of a request are short or empty: as the fastest index,
   // four splits a request put all the long ones on half of the chip, 141 us against 108 us at 64 requests)
@@ -85,7 +105,7 @@ __global__ __launch_bounds__(64) void decode_attention_kernel(
   const int group = (int)((blockIdx.x + blockIdx.y + blockIdx.z) % gridDim.x);
   const int per_kv = (int)gridDim.x / Hkv;         // groups of up to 16 query heads on one key/value head
   const int kvh = group / per_kv;
-  const int head0 = kvh * (Hq / Hkv) + (group % per_kv) * 16;                  // this wave's query heads: head0 + (0 .. G - 1)
+  const int head0 = kvh * (Hq / Hkv) + (group % per_kv) * 16;                  // this block's query heads: head0 + (0 .. G - 1)
   const int G = min(16, Hq / Hkv - (group % per_kv) * 16);
   const int pos = positions[t];
   const int lo = nhv_first_key(pos, window);
@@ -108,37 +128,40 @@ __global__ __launch_bounds__(64) void decode_attention_kernel(
   floatx4 o[DTILES];                          // o[dt][j]: entry dt * 16 + 4 grp + j of head `col`
 #pragma unroll
   for (int dt = 0; dt < DTILES; ++dt) o[dt] = floatx4{0.f, 0.f, 0.f, 0.f};
-  const int ksub = lane / LPK, chunk = lane % LPK;       // this lane loads piece `chunk` of keys ksub * PASSES + (0..PASSES)
+  const int ksub = lane / LPK;                            // this lane loads piece `chunk` of keys ksub * PASSES + (0..PASSES)
+  const int chunk = lane % LPK;
   const bool chunk_live = chunk * 8 < D;
+  const int chunk_at = (chunk_live ? chunk : CHUNKS - 1) * 8;
 
-  for (int kb = (first / RK) * RK; kb <= last; kb += RK) {
-    // ---- all keys and values of the round are asked for before anything is computed (16 KB a wave at head size 128)
-    // (pages that are a power of two of at least 64 tokens hold a whole round: one look at the block table)
-    const bool one_page = page_shift >= 6;
-    const int round_base = one_page ? (bt[kb >> page_shift] << page_shift) : 0;
-    bf16x8 ka[KT][DSTEPS];
+  bf16x8 ka[KT][DSTEPS], vv[PASSES];
+  // All keys and values of a round are asked for before anything is computed (16 KB a wave at head size 128). A key that the
+  // split does not hold is taken for the nearest that it does: its score is masked, so its weight is 0, and no load hangs on
+  // a condition.
+  auto ask = [&](int kb) {
+    int base[KT];                                         // where the page of each 16 keys begins, if they lie in one page
+    if (page_shift >= 4) {
+#pragma unroll
+      for (int kt = 0; kt < KT; ++kt) base[kt] = bt[min(max(kb + kt * 16, first), last) >> page_shift] << page_shift;
+    }
+    auto slot = [&](int kt, int key) {
+      key = min(max(key, first), last);
+      if (page_shift < 4) return slot_of(bt, key, page_size, page_shift);
+      int at = base[0];
+#pragma unroll
+      for (int i = 1; i < KT; ++i) at = kt == i ? base[i] : at;
+      return at + (key & (page_size - 1));
+    };
 #pragma unroll
     for (int kt = 0; kt < KT; ++kt) {
-      const int key = kb + kt * 16 + col;
-      const bool ok = key >= first && key <= last;
-      int slot = 0;
-      if (ok) slot = one_page ? round_base + (key & (page_size - 1)) : slot_of(bt, key, page_size, page_shift);
-      const bf16_t* krow = k_cache + ((size_t)slot * Hkv + kvh) * D;
+      const bf16_t* krow = k_cache + ((size_t)slot(kt, kb + kt * 16 + col) * Hkv + kvh) * D;
 #pragma unroll
-      for (int s = 0; s < DSTEPS; ++s) {
-        const int d = s * 32 + grp * 8;
-        ka[kt][s] = (ok && d < D) ? load8(krow + d) : zero8();
-      }
+      for (int s = 0; s < DSTEPS; ++s) ka[kt][s] = load8(krow + (D % 32 ? min(s * 32 + grp * 8, D - 8) : s * 32 + grp * 8));   // (beyond D queries are zeros)
     }
-    bf16x8 vv[PASSES];
 #pragma unroll
-    for (int ps = 0; ps < PASSES; ++ps) {
-      const int key = kb + ksub * PASSES + ps;
-      const bool ok = chunk_live && key >= first && key <= last;
-      int slot = 0;
-      if (ok) slot = one_page ? round_base + (key & (page_size - 1)) : slot_of(bt, key, page_size, page_shift);
-      vv[ps] = ok ? load8(v_cache + ((size_t)slot * Hkv + kvh) * D + chunk * 8) : zero8();
-    }
+    for (int ps = 0; ps < PASSES; ++ps)
+      vv[ps] = load8(v_cache + ((size_t)slot(ksub * PASSES / 16, kb + ksub * PASSES + ps) * Hkv + kvh) * D + chunk_at);
+  };
+  auto round = [&](int kb) {
     // ---- scores
     floatx4 s4[KT];
 #pragma unroll
@@ -147,8 +170,9 @@ __global__ __launch_bounds__(64) void decode_attention_kernel(
 #pragma unroll
       for (int s = 0; s < DSTEPS; ++s) s4[kt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ka[kt][s], qb[s], s4[kt], 0, 0, 0);
     }
-    // ---- values into LDS, transposed: row d, columns = keys of the round
-    __syncthreads();                                   // the last round's tile has been read
+    // ---- values into LDS, transposed: row d, columns = keys of the round (the tile is this wave's own, and a wave's
+    // accesses to LDS are done in their order)
+    asm volatile("" ::: "memory");
     if (chunk_live) {
 #pragma unroll
       for (int pg = 0; pg < PASSES / KG; ++pg) {
@@ -205,7 +229,7 @@ __global__ __launch_bounds__(64) void decode_attention_kernel(
       }
     l_part = l_part * alpha + psum;
     m_run = m_new;
-    __syncthreads();                                   // the tile is written
+    asm volatile("" ::: "memory");
     // ---- O^T += V^T P^T
     // (the outputs are rescaled only when the reference has moved: a branch of the whole wave; written as a condition
     // inside the loop over the output tiles it became a multiply and a select for every output entry in every round)
@@ -233,19 +257,56 @@ __global__ __launch_bounds__(64) void decode_attention_kernel(
         o[dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(va, pa[a], o[dt], 0, 0, 0);
       }
     }
-  }
-  // ---- this split's result
+  };
+  for (int turn = first / RK * RK + wave * RK * TURN; turn <= last; turn += RK * TURN * WAVES)
+    for (int kb = turn; kb <= min(last, turn + RK * (TURN - 1)); kb += RK) {
+      ask(kb);
+      round(kb);
+    }
+  // ---- the waves meet: a wave's sums lie where its values lay
   l_part += __shfl_xor(l_part, 16, 64);
   l_part += __shfl_xor(l_part, 32, 64);
+  asm volatile("" ::: "memory");
   if (col < G) {
-    const size_t item = ((size_t)t * Hq + head0 + col) * n_splits + split;
-    if (grp == 0) {
-      part_ml[item * 2] = m_run;
-      part_ml[item * 2 + 1] = l_part;
-    }
+    float* mine = reinterpret_cast<float*>(vt_s) + col * OPITCH + grp * 4;
+    if (grp == 0) *reinterpret_cast<float2*>(reinterpret_cast<float*>(vt_s) + 16 * OPITCH + 2 * col) = make_float2(m_run, l_part);
 #pragma unroll
-    for (int dt = 0; dt < DTILES; ++dt)
-      *reinterpret_cast<float4*>(part_o + item * D + dt * 16 + grp * 4) = make_float4(o[dt][0], o[dt][1], o[dt][2], o[dt][3]);
+    for (int dt = 0; dt < DTILES; ++dt) *reinterpret_cast<floatx4*>(mine + dt * 16) = o[dt];
+  }
+  __syncthreads();
+  for (int i = threadIdx.x * 4; i < G * D; i += 64 * WAVES * 4) {
+    const int head = i / D, d = i % D;
+    float2 ml[WAVES];                                  // (a wave without a round: -inf, weight 0 and sums of 0)
+#pragma unroll
+    for (int w = 0; w < WAVES; ++w) ml[w] = *reinterpret_cast<const float2*>(reinterpret_cast<const float*>(tiles_s[w]) + 16 * OPITCH + 2 * head);
+    float m = ml[0].x;
+#pragma unroll
+    for (int w = 1; w < WAVES; ++w) m = fmaxf(m, ml[w].x);
+    float l = 0.f;
+    floatx4 sum = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int w = 0; w < WAVES; ++w) {
+      const float weight = __builtin_amdgcn_exp2f(ml[w].x - m);
+      l += ml[w].y * weight;
+      sum += *reinterpret_cast<const floatx4*>(reinterpret_cast<const float*>(tiles_s[w]) + head * OPITCH + d) * weight;
+    }
+    const size_t row = (size_t)t * Hq + head0 + head;
+    if (n_splits > 1) {
+      const size_t item = row * n_splits + split;
+      if (d == 0) {
+        part_ml[item * 2] = m;
+        part_ml[item * 2 + 1] = l;
+      }
+      *reinterpret_cast<floatx4*>(part_o + item * D + d) = sum;
+    } else {
+      l += exp2f((finish.sinks ? finish.sinks[head0 + head] * 1.4426950408889634f : finish.sink_l2) - m);   // (no sink: 0)
+      float inv = 1.0f / l;
+      if (finish.gate) inv /= 1.0f + expf(-(float)finish.gate[(size_t)t * finish.gate_ld + head0 + head]);
+      bf16x4 y;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) y[j] = (__bf16)(sum[j] * inv);
+      *reinterpret_cast<bf16x4*>(out + row * D + d) = y;
+    }
   }
 }
 
@@ -464,19 +525,21 @@ static int launch_decode_attention(const void* q, const void* k_cache, const voi
   dim3 grid(Hkv * ((Hq / Hkv + 15) / 16), T, n_splits);
   const float log2e = 1.4426950408889634f;
 #define NHV_DECODE_LAUNCH(CAPPED_, BIASED_)                                                                           \
-  hipLaunchKernelGGL((decode_attention_kernel<CAPPED_, BIASED_>), grid, dim3(64), 0, s, (const bf16_t*)q, (const bf16_t*)k_cache, \
-                     (const bf16_t*)v_cache, part_o, part_ml, (const int*)token_req,                                  \
+  hipLaunchKernelGGL((decode_attention_kernel<CAPPED_, BIASED_>), grid, dim3(64 * WAVES), 0, s, (const bf16_t*)q, (const bf16_t*)k_cache, \
+                     (const bf16_t*)v_cache, part_o, part_ml, (bf16_t*)out, (const int*)token_req,                    \
                      (const int*)positions, (const int*)block_tables, max_blocks, Hq, Hkv, page_size, page_shift,     \
                      scale * log2e, window, split_len, n_splits, cap * log2e, cap > 0.f ? 2.0f * log2e * scale / cap : 0.f, \
-                     (const float*)slopes)
+                     (const float*)slopes, finish)
+  const float sink_l2 = has_sink ? sink * log2e : -INFINITY;
+  const Finish finish = {sink_l2, (const float*)sinks, (const bf16_t*)gate, gate_ld};
   if (cap > 0.f && slopes) NHV_DECODE_LAUNCH(true, true);
   else if (cap > 0.f) NHV_DECODE_LAUNCH(true, false);
   else if (slopes) NHV_DECODE_LAUNCH(false, true);
   else NHV_DECODE_LAUNCH(false, false);
 #undef NHV_DECODE_LAUNCH
   NHV_LAUNCH_CHECK("decode_attention");
+  if (n_splits == 1) return 0;
   const unsigned items = (unsigned)((size_t)T * Hq);
-  const float sink_l2 = has_sink ? sink * log2e : -INFINITY;
 #define NHV_MERGE_ARGS (const float*)part_o, (const float*)part_ml, (bf16_t*)out, (const int*)positions, window, split_len, n_splits, Hq, \
                        sink_l2, (const float*)sinks, (const bf16_t*)gate, gate_ld
 #define NHV_MERGE_AT_ONCE(W_, NL_) \

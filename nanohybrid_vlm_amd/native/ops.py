@@ -525,24 +525,23 @@ class NativeBackend:
         span = min(self.planned_context, batch.max_context_len) if self.planned_context else batch.max_context_len
         if window:                                   # (a chunk comes as a negative window)
             span = min(span, abs(window) + 64)
-        # One wave per SIMD of the chip (about a thousand) is the fastest while that leaves splits of up to 256
-        # keys, half as many waves again from there on (a wave takes its keys one round after the other), and no
-        # split is longer than 1,024 keys. Measured at 2,176 and 8,192 keys, 1 to 64 requests, 8 key/value heads: the
-        # best split length is 64 to 128 keys for 8 x 2,176 keys in all, 256 for 32 x 2,176 (62 against 64 us with
-        # 512), 512 for 48 and 64 x 2,176 (110 against 118 us with 1,024) and for 16 x 8,192, 1,024 for 32 x 8,192.
-        want = max(1, T * Hkv * -(-(Hq // Hkv) // 16) * span // 1024)      # (a wave takes up to 16 heads of a key/value head)
-        want = min(want, max(256, want * 2 // 3))
-        # (splits of one round of 32 keys for one request of 2,100 keys, 525 waves: 3.64 against 3.66 ms a step; for two
-        # requests 3.77 against 3.75: not taken)
-        split_len = 64
-        while split_len * 2 <= want and split_len < 1024:
-            split_len *= 2
         # the splits cover the longest context this launch can meet: outside a graph the batch's own; inside one, what
         # the recorder says it will let the graph meet (``covered_context``: it replaces a graph before its contexts
         # outgrow that), not the bound of the block tables (max_model_len), whose splits would nearly all be empty blocks
         covered = batch.max_context_len
         if self.planned_context and self.covered_context:
             covered = min(covered, self.covered_context)
+        # A block of eight waves takes 256 keys in the time of 32. One split where the blocks fill the chip anyway (24 to 128
+        # requests of 8 key/value heads: no split faster) or where its rounds are over before a merge would be (one request of
+        # 16 heads, 150 keys: 6.2 us, two splits of 128 8.3; eight of 300 keys 8.4 against 9.9; one of 1,000 14.4 against
+        # 9.4). Else one block a compute unit, splits of at least 128 keys and not many more than 32 of them, which is what
+        # the merge takes at once (8 x 2,050 keys: 21.3 us with splits of 512, 23.7 with 384 or 256; 8 x 4,000: 31.5 with
+        # 1,024, 36.6 with 256; 1 x 9,000: 15.4 with 384, 19.5 with 256).
+        blocks = T * Hkv * -(-(Hq // Hkv) // 16)            # (a block takes up to 16 heads of a key/value head)
+        if blocks >= 192 or span <= 448:
+            split_len = -(-covered // 32) * 32
+        else:
+            split_len = max(128, 128 * round(max(span * blocks / 256, covered / 36) / 128))
         n_splits = -(-covered // split_len)
         part_o = torch.empty((T, Hq, n_splits, D), dtype=torch.float32, device=q.device)
         part_ml = torch.empty((T, Hq, n_splits, 2), dtype=torch.float32, device=q.device)
