@@ -74,6 +74,7 @@ __device__ __forceinline__ int slot_of(const int* bt, int key, int page_size, in
 // for before this one is computed: more than 256 registers, one wave a SIMD, and 2 to 10 % more time.)
 constexpr int WAVES = D <= 128 ? 8 : 4;
 constexpr int TURN = D <= 64 ? 2 : 1;                       // rounds a wave takes before the next wave's: 16 KB and more of keys and values
+constexpr int MOST_SORTED = 64;                             // up to so many tokens the longest contexts are taken first
 constexpr int OPITCH = D + 4;                               // floats a head in the waves' meeting place, which lies where a wave's V^T tile was
 constexpr int MEET = 16 * OPITCH * 4 + 16 * 2 * 4;          // bytes: 16 heads' sums, maxima and sums of weights
 constexpr int TILE = D * VPITCH * 2 > MEET ? D * VPITCH * 2 : MEET;
@@ -101,7 +102,39 @@ __global__ __launch_bounds__(64 * WAVES) void decode_attention_kernel(
   // and the key/value head turns with the token and the split: a head's keys are 2 D bytes out of every
   // 2 D Hkv bytes of a page, and an XCD that read one and the same head for every token took 4 to 5 % longer at
   // 32 and 64 requests (116 against 111 us at 64) than one whose blocks go over all heads
-  const int t = blockIdx.y, split = blockIdx.z;
+  int t = blockIdx.y;
+  const int split = blockIdx.z;
+  // One split and contexts of different lengths: the blocks that start first take the longest (after 100 to 2,000 keys: 64
+  // requests 68.7 -> 62.7 us, 40 requests 52.5 -> 43.6; for 128 what it costs is what it saves). Every block finds its token
+  // by counting, each wave against its share of the tokens (against all of them in one thread a token: 65 us).
+  if (n_splits == 1 && gridDim.y >= 16 && gridDim.y <= MOST_SORTED) {
+    static_assert(sizeof(int) * (2 * MOST_SORTED + 1) <= sizeof(tiles_s), "the tokens' numbers of keys do not fit the tiles");
+    int *keys_s = reinterpret_cast<int*>(tiles_s), *place_s = keys_s + MOST_SORTED, *chosen = place_s + MOST_SORTED;
+    const int T = gridDim.y, tid = threadIdx.x;
+    for (int i = tid; i < MOST_SORTED; i += 64 * WAVES) {
+      const int p = positions[min(i, T - 1)];
+      keys_s[i] = i < T ? p - nhv_first_key(p, window) : -1;
+      place_s[i] = 0;
+    }
+    __syncthreads();
+    const int share = (T + 4 * WAVES - 1) / (4 * WAVES) * 4, j0 = wave * share;
+    for (int i = lane; i < T; i += 64) {
+      const int keys = keys_s[i];
+      int before = 0;
+      for (int j = j0; j < min(j0 + share, T); j += 4) {
+        const int4 other = *reinterpret_cast<const int4*>(&keys_s[j]);
+        before += (other.x > keys || (other.x == keys && j < i)) + (other.y > keys || (other.y == keys && j + 1 < i)) +
+                  (other.z > keys || (other.z == keys && j + 2 < i)) + (other.w > keys || (other.w == keys && j + 3 < i));
+      }
+      if (before) atomicAdd(&place_s[i], before);
+    }
+    __syncthreads();
+    for (int i = tid; i < T; i += 64 * WAVES)
+      if (place_s[i] == t) *chosen = i;
+    __syncthreads();
+    t = *chosen;
+    __syncthreads();
+  }
   const int group = (int)((blockIdx.x + blockIdx.y + blockIdx.z) % gridDim.x);
   const int per_kv = (int)gridDim.x / Hkv;         // groups of up to 16 query heads on one key/value head
   const int kvh = group / per_kv;

@@ -531,6 +531,45 @@ def test_decode_attention_of_few_tokens_over_many_splits(ops, Hq, Hkv, D, page, 
         torch.testing.assert_close(out.double().cpu(), ref, **tol(torch.bfloat16))
 
 
+@pytest.mark.parametrize("T,Hq,Hkv,D,page,window", [(16, 4, 2, 128, 16, None), (64, 2, 1, 64, 8, None), (63, 2, 2, 128, 32, 40),
+                                                    (41, 1, 1, 256, 16, None), (30, 1, 1, 32, 7, None), (300, 1, 1, 16, 64, None)])
+def test_decode_attention_of_many_tokens_with_one_split(ops, T, Hq, Hkv, D, page, window):
+    """Blocks take the tokens in the order of their numbers of keys (equal ones among them), up to 64, and as they come beyond;
+    contexts from one key to some rounds of all waves; every token's result is its own."""
+    g = torch.Generator().manual_seed(81)
+    lens = torch.randint(1, 700 if T < 100 else 90, (T,), generator=g).tolist()
+    lens[0], lens[-1], lens[T // 2] = 1, max(lens), max(lens)
+    scale = D ** -0.5
+    q, kc, vc, batch, bt, ks, vs, qs = _paged_setup(torch.bfloat16, lens, [1] * T, Hq, Hkv, D, page, seed=82)
+    out = ops.paged_attention(q, kc, vc, batch, bt, scale, window)
+    ref = _attention_reference(qs, ks, vs, lens, [1] * T, scale, window)
+    torch.testing.assert_close(out.double().cpu(), ref, **tol(torch.bfloat16))
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("W", [8, 1000, 2048, 2056, 4104, 8192, 8200, 50])
+def test_depth_mix_in_all_its_widths(ops, dtype, W):
+    """Rows in one, two and four passes of 2,048 entries and what does not fit them; layers that read none to five results."""
+    T, eps = 5, 1e-5
+    x, gain = rnd(T, W, seed=91), torch.tensor(0.7, device="cuda")
+    results = torch.zeros(8, T, W, device="cuda")
+    want = [x.double()]
+    for i in range(6):
+        a, b, c = (rnd(T, W, dtype=dtype, seed=92 + 3 * i + j) for j in range(3))
+        wa, wb, w = rnd(W, seed=93, scale=0.1) + 1, rnd(W, seed=94, scale=0.1) + 1, rnd(i + 2, seed=95 + i, scale=0.5)
+        pair = i % 2 == 1
+        first = ops.NormedPairMean(a, wa, c, wb, eps) if pair else a
+        got, normed = ops.depth_mix(x, first, None if i == 2 else b, results, i, w, gain=gain, eps=eps)
+        unit = lambda t: t / torch.sqrt(t.pow(2).mean(-1, keepdim=True) + eps)
+        add = 0.5 * (unit(a.double()) * wa + unit(c.double()) * wb) if pair else a.double()
+        want.append(x.double() + add + (0 if i == 2 else b.double()))
+        ref = sum(w[j].double() * want[j] for j in range(i + 2))
+        torch.testing.assert_close(got.double(), ref, rtol=1e-5, atol=1e-5)
+        torch.testing.assert_close(results[i + 1].double(), want[-1], rtol=1e-5, atol=1e-5)
+        torch.testing.assert_close(normed.double(), unit(ref) * 0.7, **tol(dtype))
+        x = got
+
+
 @pytest.mark.parametrize("D,split_len,n_splits,window", [
     (128, 64, 5, None),      # one wave, four splits a lane
     (128, 64, 20, None),     # four waves, four splits a lane; the last waves' splits lie past every position but one
