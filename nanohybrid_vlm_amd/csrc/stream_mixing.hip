@@ -85,8 +85,129 @@ extern "C" int nhv_pair_norm_mean(const void* a, const void* wa, const void* b, 
 // as its weight is written to ``normed`` as well (what the next layer reads). With ``a2`` the first addend is not a but
 // half the sum of a and a2, each over its root mean square (pair_eps) times its weight vector wa, wb: what
 // nhv_pair_norm_mean would have written, unrounded.
+// Bound by the reads of the earlier results (row by row, 4 W bytes each). V entries a thread at a time, several results'
+// entries asked for before the first is used; a row stays in registers up to its norm (rows of up to PASSES 256 V
+// entries). 2,201 rows of 2,048 beside 1 to 8 earlier results: 32 us on the mean; one entry a thread and trip took 77.
+template <typename T, int V, int PASSES>
+__global__ __launch_bounds__(256) void depth_mix_kernel(const float* __restrict__ x, const T* __restrict__ a, const T* __restrict__ b,
+                                                        float* __restrict__ results, size_t plane, int index, const float* __restrict__ weights,
+                                                        float* __restrict__ out, const float* __restrict__ gain, T* __restrict__ normed, int W,
+                                                        float eps, const T* __restrict__ a2, const float* __restrict__ wa,
+                                                        const float* __restrict__ wb, float pair_eps) {
+  struct alignas(sizeof(T) * V) Pack { T e[V]; };
+  struct alignas(sizeof(float) * (V < 4 ? V : 4)) Four { float e[V < 4 ? V : 4]; };
+  constexpr int N4 = V < 4 ? 1 : V / 4, W4 = V < 4 ? V : 4;      // 16 bytes of floats at a time
+  __shared__ float scratch[16];
+  const size_t base = (size_t)blockIdx.x * W;
+  const int n = index + 2;
+  auto load = [&](const float* p, float* v) {
+#pragma unroll
+    for (int j = 0; j < N4; ++j) {
+      const Four f = *reinterpret_cast<const Four*>(p + j * W4);
+#pragma unroll
+      for (int k = 0; k < W4; ++k) v[j * W4 + k] = f.e[k];
+    }
+  };
+  auto store = [&](float* p, const float* v) {
+#pragma unroll
+    for (int j = 0; j < N4; ++j) {
+      Four f;
+#pragma unroll
+      for (int k = 0; k < W4; ++k) f.e[k] = v[j * W4 + k];
+      *reinterpret_cast<Four*>(p + j * W4) = f;
+    }
+  };
+  auto load_rows = [&](const T* p, float* v) {
+    const Pack f = *reinterpret_cast<const Pack*>(p);
+#pragma unroll
+    for (int k = 0; k < V; ++k) v[k] = to_f32(f.e[k]);
+  };
+  float ra = 1.f, rb = 0.f;
+  if (a2 != nullptr) {
+    float sa = 0.f, sb = 0.f;
+#pragma unroll
+    for (int p = 0; p < PASSES; ++p) {
+      const int i = (p * 256 + threadIdx.x) * V;
+      if (i >= W) continue;
+      float u[V], v[V];
+      load_rows(a + base + i, u);
+      load_rows(a2 + base + i, v);
+#pragma unroll
+      for (int k = 0; k < V; ++k) {
+        sa = fmaf(u[k], u[k], sa);
+        sb = fmaf(v[k], v[k], sb);
+      }
+    }
+    ra = 1.0f / sqrtf(block_sum(sa, scratch) / (float)W + pair_eps);
+    rb = 1.0f / sqrtf(block_sum(sb, scratch) / (float)W + pair_eps);
+  }
+  float ss = 0.f, sum[PASSES][V];
+#pragma unroll
+  for (int p = 0; p < PASSES; ++p) {
+    const int i = (p * 256 + threadIdx.x) * V;
+    if (i >= W) continue;
+    float xi[V], mine[V], t[V];
+    load(x + base + i, xi);
+    load_rows(a + base + i, mine);
+    if (a2 != nullptr) {
+      float ga[V], gb[V];
+      load_rows(a2 + base + i, t);
+      load(wa + i, ga);
+      load(wb + i, gb);
+#pragma unroll
+      for (int k = 0; k < V; ++k) mine[k] = 0.5f * (mine[k] * ra * ga[k] + t[k] * rb * gb[k]);
+    }
+    if (b != nullptr) {
+      load_rows(b + base + i, t);
+#pragma unroll
+      for (int k = 0; k < V; ++k) mine[k] += t[k];
+    }
+#pragma unroll
+    for (int k = 0; k < V; ++k) mine[k] += xi[k];
+    store(results + (size_t)(index + 1) * plane + base + i, mine);
+    if (index == 0) store(results + base + i, xi);
+    const float w0 = weights[0];
+    if (index == 0) {
+#pragma unroll
+      for (int k = 0; k < V; ++k) sum[p][k] = fmaf(w0, xi[k], 0.f);
+    } else {
+      load(results + base + i, t);
+#pragma unroll
+      for (int k = 0; k < V; ++k) sum[p][k] = fmaf(w0, t[k], 0.f);
+    }
+#pragma unroll 4
+    for (int j = 1; j + 1 < n; ++j) {
+      float r[V];
+      load(results + (size_t)j * plane + base + i, r);
+      const float wj = weights[j];
+#pragma unroll
+      for (int k = 0; k < V; ++k) sum[p][k] = fmaf(wj, r[k], sum[p][k]);
+    }
+    const float wn = weights[n - 1];
+#pragma unroll
+    for (int k = 0; k < V; ++k) {
+      sum[p][k] = fmaf(wn, mine[k], sum[p][k]);
+      ss = fmaf(sum[p][k], sum[p][k], ss);
+    }
+    store(out + base + i, sum[p]);
+  }
+  if (gain == nullptr) return;
+  const float total = block_sum(ss, scratch);
+  const float r = gain[0] / sqrtf(total / (float)W + eps);
+#pragma unroll
+  for (int p = 0; p < PASSES; ++p) {
+    const int i = (p * 256 + threadIdx.x) * V;
+    if (i >= W) continue;
+    Pack y;
+#pragma unroll
+    for (int k = 0; k < V; ++k) y.e[k] = from_f32<T>(sum[p][k] * r);
+    *reinterpret_cast<Pack*>(normed + base + i) = y;
+  }
+}
+
+// Rows that do not stay in a thread's registers, whose widths or addresses are not whole groups of entries, one entry at a time.
 template <typename T>
-__global__ void depth_mix_kernel(const float* __restrict__ x, const T* __restrict__ a, const T* __restrict__ b,
+__global__ void depth_mix_any_kernel(const float* __restrict__ x, const T* __restrict__ a, const T* __restrict__ b,
                                  float* __restrict__ results, size_t plane, int index, const float* __restrict__ weights,
                                  float* __restrict__ out, const float* __restrict__ gain, T* __restrict__ normed, int W,
                                  float eps, const T* __restrict__ a2, const float* __restrict__ wa,
@@ -132,15 +253,26 @@ extern "C" int nhv_depth_mix(const void* x, const void* a, const void* b, void* 
   NHV_REQUIRE(x != out, "depth_mix: the sum cannot be written over the stream it reads");
   NHV_REQUIRE(a2 == nullptr || (wa != nullptr && wb != nullptr), "depth_mix: a pair of addends without its weights");
   hipStream_t s = (hipStream_t)stream;
-  if (dtype == NHV_F32)
-    hipLaunchKernelGGL(depth_mix_kernel<float>, dim3(T), dim3(256), 0, s, (const float*)x, (const float*)a, (const float*)b,
-                       (float*)results, (size_t)plane, index, (const float*)weights, (float*)out, (const float*)gain,
-                       (float*)normed, W, eps, (const float*)a2, (const float*)wa, (const float*)wb, pair_eps);
-  else if (dtype == NHV_BF16)
-    hipLaunchKernelGGL(depth_mix_kernel<bf16_t>, dim3(T), dim3(256), 0, s, (const float*)x, (const bf16_t*)a, (const bf16_t*)b,
-                       (float*)results, (size_t)plane, index, (const float*)weights, (float*)out, (const float*)gain,
-                       (bf16_t*)normed, W, eps, (const bf16_t*)a2, (const float*)wa, (const float*)wb, pair_eps);
+  // eight entries a thread and pass: 32 bytes of floats, 16 of bfloat16
+  const uintptr_t places = (uintptr_t)x | (uintptr_t)a | (uintptr_t)b | (uintptr_t)results | (uintptr_t)out | (uintptr_t)normed |
+                           (uintptr_t)a2 | (uintptr_t)wa | (uintptr_t)wb;
+  const bool wide = W % 8 == 0 && W <= 4 * 2048 && plane % 8 == 0 && places % 32 == 0;
+#define LAUNCH_AS(KERNEL, TT)                                                                                          \
+  hipLaunchKernelGGL(KERNEL, dim3(T), dim3(256), 0, s, (const float*)x, (const TT*)a, (const TT*)b, (float*)results, (size_t)plane, \
+                     index, (const float*)weights, (float*)out, (const float*)gain, (TT*)normed, W, eps, (const TT*)a2,  \
+                     (const float*)wa, (const float*)wb, pair_eps)
+#define LAUNCH(TT)                                                          \
+  do {                                                                      \
+    if (!wide) LAUNCH_AS(depth_mix_any_kernel<TT>, TT);                     \
+    else if (W <= 2048) LAUNCH_AS((depth_mix_kernel<TT, 8, 1>), TT);        \
+    else if (W <= 2 * 2048) LAUNCH_AS((depth_mix_kernel<TT, 8, 2>), TT);    \
+    else LAUNCH_AS((depth_mix_kernel<TT, 8, 4>), TT);                       \
+  } while (0)
+  if (dtype == NHV_F32) LAUNCH(float);
+  else if (dtype == NHV_BF16) LAUNCH(bf16_t);
   else return nhv_fail("depth_mix: unknown dtype %d", dtype);
+#undef LAUNCH
+#undef LAUNCH_AS
   NHV_LAUNCH_CHECK("depth_mix");
   return 0;
 }
