@@ -8,7 +8,8 @@
 // The waves' sums meet in LDS and are added in the order of the waves, so the result does not depend
 // on timing. Rows of x beyond M and columns beyond K read as zero.
 //
-// Where all rows of x fit into LDS beside the sums (M (K + 8) 2 bytes of the 160 KB) a second kernel is used
+// Most products take one of two kernels in whose tiles nothing waits (tiles_plan() below). For the others: where all rows of
+// x fit into LDS beside the sums (M (K + 8) 2 bytes of the 160 KB) a second kernel is used
 // instead: a block copies x into LDS once (straight from memory, global_load_lds) and then walks over
 // tiles of w, tile after tile, one or two blocks per compute unit for the whole matrix. The rows of x
 // then cross from L2 to a compute unit once per call instead of once per tile: 5 to 25 % less time at
@@ -579,7 +580,332 @@ __global__ __launch_bounds__(64 * WAVES) void gemm_fewrows_passes_kernel(const b
   }
 }
 
+typedef __attribute__((__vector_size__(4 * sizeof(__bf16)))) __bf16 bf16x4;
+typedef __attribute__((__vector_size__(4 * sizeof(unsigned)))) unsigned uint4v;
+typedef __attribute__((__vector_size__(2 * sizeof(unsigned)))) unsigned uint2v;
+
+// Four neighbouring numbers as they lie in memory, in float32 or bfloat16 (a conversion where they are asked for would wait for
+// them, and so would a branch on the type): two loads of 8 bytes, which for bfloat16 are the same one. Without a pointer:
+// `some` is read and not used.
+struct Four {
+  uint2v lo, hi;
+  __device__ __forceinline__ void ask(const void* p, size_t at, int is_f32, const void* some) {
+    const char* from = p ? (const char*)p + at * (is_f32 ? 4 : 2) : (const char*)some;
+    lo = *reinterpret_cast<const uint2v*>(from);
+    hi = *reinterpret_cast<const uint2v*>(from + (is_f32 ? 8 : 0));
+  }
+  __device__ __forceinline__ float at(int j, int is_f32) const {
+    return __uint_as_float(is_f32 ? (j < 2 ? lo[j] : hi[j - 2]) : j % 2 ? lo[j / 2] & 0xffff0000u : lo[j / 2] << 16);
+  }
+};
+__device__ __forceinline__ void store4(bf16_t* p, const float (&v)[4]) {
+  bf16x4 y;
+#pragma unroll
+  for (int j = 0; j < 4; ++j) y[j] = (__bf16)v[j];
+  *reinterpret_cast<bf16x4*>(p) = y;
+}
+__device__ __forceinline__ void store4(float* p, const float (&v)[4]) { *reinterpret_cast<floatx4*>(p) = floatx4{v[0], v[1], v[2], v[3]}; }
+
+// A barrier for LDS alone: loads from memory stay under way.
+__device__ __forceinline__ void lds_barrier() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+  __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
+// What the two kernels below share. They are bound by the latency of a product's few loads where it is small and by the stream of
+// w where it is large: a tile is up to 16 rows of w (a multiple of 4, so that all 256 compute units have one); 16 waves share
+// K; a wave has AHEAD steps of 32 columns under way, AHEAD KB and matrix, which for most layers is its whole share. No load hangs
+// on a condition, a conversion or another load (each makes the compiler wait for all that are under way): rows and columns
+// beyond the matrix are read from the last ones inside, and columns are multiplied as zeros. Against the kernels further
+// down, which ask for two steps at a time and wait for the residual before the weights: 1,024 outputs of 2,048 and 3,072 columns
+// added to a residual at 1 row 6.4 -> 4.9 us and 8.5 -> 6.3, at 16 rows 8.0 -> 6.0 and 11.1 -> 8.0; 4,096 of 4,096 at 8 rows
+// 12.4 -> 10.4; 6,144 of 4,096 13.7 -> 12.2 and 15.4 -> 13.0 at 1 and 8; gated 9,728 of 2,560 26.3 -> 23.3, 3,072 of 1,024 at
+// 16 rows 9.9 -> 6.8.
+constexpr int TW = 16;                       // waves
+
+// x into LDS, [M][K + 8] (the 16 bytes between rows spread the rows over the banks): a wave's load brings 64 consecutive
+// 16-byte pieces of one row
+__device__ __forceinline__ void ask_x(const bf16_t* __restrict__ x, bf16_t* x_s, int M, int K, int wave, int lane) {
+  const int pieces_per_row = K / 8, loads_per_row = (pieces_per_row + 63) / 64;
+  for (int job = wave; job < M * loads_per_row; job += TW) {
+    const int m = job / loads_per_row, part = job % loads_per_row;
+    if (part * 64 + lane < pieces_per_row)
+      __builtin_amdgcn_global_load_lds((global_ptr)(x + (size_t)m * K + (part * 64 + lane) * 8), (lds_ptr)(x_s + m * (K + 8) + part * 512), 16, 0, 0);
+  }
+}
+// The wait for x alone, when YOUNGER loads have been asked for since (a fence would wait for all).
+template <int YOUNGER>
+__device__ __forceinline__ void wait_for_x() {
+  __builtin_amdgcn_sched_barrier(0);
+  asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(YOUNGER) : "memory");
+  __builtin_amdgcn_sched_barrier(0);
+}
+
+__device__ __forceinline__ bf16x8 masked(bf16x8 v, unsigned mask) { return (bf16x8)((uint4v)v & mask); }
+
+// A tile's sums of the waves (red[wave][matrix][lane]), added in the order of the waves; then the rows' scales, the biases, the gate.
+template <bool GLU, bool FUSED>
+__device__ __forceinline__ void add_waves(const Fusion& f, const floatx4 (*red)[GLU ? 2 : 1][64], const float* r_s, const Four* bias4, bool biased,
+                                          float (&out)[4], int lane) {
+  constexpr int NA = GLU ? 2 : 1, SIDE = 8 / NA;                     // (so many at once: the registers that are left)
+  floatx4 v[NA];
+#pragma unroll
+  for (int na = 0; na < NA; ++na) v[na] = floatx4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll 1
+  for (int wv = 0; wv < TW; wv += SIDE) {
+    floatx4 part[SIDE][NA];
+#pragma unroll
+    for (int i = 0; i < SIDE; ++i)
+#pragma unroll
+      for (int na = 0; na < NA; ++na) part[i][na] = red[wv + i][na][lane];
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int i = 0; i < SIDE; ++i)
+#pragma unroll
+      for (int na = 0; na < NA; ++na) v[na] += part[i][na];
+  }
+  const float rs = (FUSED && f.ss_in) ? r_s[lane & 15] : 1.0f;       // the row's scale, where x is a sum whose norm is due
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    float r = v[0][j] * rs, up = v[NA - 1][j] * rs;
+    if (biased) r += bias4[0].at(j, 0), up += bias4[NA - 1].at(j, 0);
+    if (GLU) r = nhv_gated(r, up, f.gate);
+    else if (f.plain_act) r = nhv_plain_act(r, f.plain_act);
+    out[j] = r;
+  }
+}
+
+// One tile a block. XLDS: x is brought to LDS, its loads before the first weights', and the wait before the first product is
+// for x alone; without, x comes from memory step by step beside w.
+template <int AHEAD, bool GLU, bool XLDS, bool FUSED, typename TOut>
+__global__ __launch_bounds__(64 * TW) void gemm_fewrows_tile_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ w,
+                                                                    const bf16_t* __restrict__ bias, TOut* __restrict__ y, int M, int N, int K,
+                                                                    int rows, int groups, const Fusion f) {
+  constexpr int NA = GLU ? 2 : 1;
+  extern __shared__ __attribute__((aligned(16))) unsigned char lds_raw[];
+  floatx4(*red)[NA][64] = reinterpret_cast<floatx4(*)[NA][64]>(lds_raw);       // [TW][NA][64]
+  bf16_t* x_s = reinterpret_cast<bf16_t*>(lds_raw + TW * NA * sizeof(floatx4) * 64);
+  __shared__ float r_s[16];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int col = lane & 15, grp = lane >> 4;
+  const int n0 = blockIdx.x * rows, n = n0 + grp * 4;
+  float share[SCALE_ROWS<TW>][SCALE_SHARES];
+  if constexpr (FUSED) ask_row_scales<TW>(f, share, M, wave, lane);
+  Four res, next_w, bias4[NA];               // what the wave that writes the tile needs beside the sums
+  if (wave == 0) {
+    const int n_in = min(n, N - 4);
+    if constexpr (FUSED && !GLU) {
+      res.ask(f.residual, (size_t)min(col, M - 1) * N + n_in, f.residual && f.residual_f32, w);
+      next_w.ask(f.next_w, n_in, f.next_w && f.next_w_f32, w);
+    }
+#pragma unroll
+    for (int na = 0; na < NA; ++na) bias4[na].ask(bias, (size_t)na * N + n_in, 0, w);
+  }
+  if constexpr (XLDS) ask_x(x, x_s, M, K, wave, lane);
+  const int k0 = wave * groups * AHEAD * 32 + grp * 8, k_end = min((wave + 1) * groups * AHEAD * 32, K);
+  const char *xb = reinterpret_cast<const char*>(x), *wb[2] = {reinterpret_cast<const char*>(w), reinterpret_cast<const char*>(w + (size_t)N * K)};
+  const unsigned xrow = (unsigned)min(col, M - 1) * K * 2, wrow = (unsigned)min(n0 + min(col, rows - 1), N - 1) * K * 2;
+  const bf16_t* xrow_s = x_s + min(col, M - 1) * (K + 8);
+  bf16x8 a[AHEAD][NA], b[AHEAD];
+  auto ask = [&](int u, int s) {
+    const unsigned k = (unsigned)min(k0 + s * 32, K - 8) * 2;
+#pragma unroll
+    for (int na = 0; na < NA; ++na) a[u][na] = *reinterpret_cast<const bf16x8*>(wb[na] + (wrow + k));
+    if constexpr (!XLDS) b[u] = *reinterpret_cast<const bf16x8*>(xb + (xrow + k));
+  };
+  asm volatile("" ::: "memory");
+  __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+  for (int u = 0; u < AHEAD; ++u) ask(u, u);
+  if constexpr (XLDS) wait_for_x<AHEAD * NA>();
+  floatx4 acc[NA];
+#pragma unroll
+  for (int na = 0; na < NA; ++na) acc[na] = floatx4{0.f, 0.f, 0.f, 0.f};
+  auto multiply = [&](int u, int s) {
+    const int k = k0 + s * 32;
+    const unsigned in = k < k_end ? ~0u : 0u;
+    bf16x8 bu = b[u];
+    if constexpr (XLDS) bu = *reinterpret_cast<const bf16x8*>(xrow_s + min(k, K - 8));
+    bu = masked(bu, in);
+#pragma unroll
+    for (int na = 0; na < NA; ++na) {
+      asm volatile("" : "+v"(a[u][na]));                             // (nothing of it is done before it is this step's turn)
+      acc[na] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(masked(a[u][na], in), bu, acc[na], 0, 0, 0);
+    }
+  };
+  int s = 0;
+  for (int g = 1; g < groups; ++g, s += AHEAD) {
+#pragma unroll
+    for (int u = 0; u < AHEAD; ++u) {
+      multiply(u, s + u);
+      ask(u, s + AHEAD + u);
+    }
+  }
+#pragma unroll
+  for (int u = 0; u < AHEAD; ++u) multiply(u, s + u);
+  if constexpr (FUSED) set_row_scales<TW>(f, share, r_s, M, K, wave, lane);
+#pragma unroll
+  for (int na = 0; na < NA; ++na) red[wave][na][lane] = acc[na];
+  lds_barrier();
+  if (wave > 0) return;
+
+  float out[4];
+  add_waves<GLU, FUSED>(f, red, r_s, bias4, bias != nullptr, out, lane);
+  const bool mine = col < M && grp * 4 < rows && n < N;
+  const size_t at = (size_t)col * N + n;
+  if (!FUSED || GLU || f.residual == nullptr) {
+    if (mine) store4(y + at, out);
+    return;
+  }
+  float sum[4], weighted[4], sq = 0.f;                               // (see emit_tile)
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    sum[j] = out[j] + res.at(j, f.residual_f32);
+    weighted[j] = sum[j] * (f.next_w ? next_w.at(j, f.next_w_f32) : 1.0f);
+    sq += mine ? sum[j] * sum[j] : 0.f;
+  }
+  if (mine) {
+    if (f.residual_f32) store4((float*)f.residual + at, sum);
+    else store4((bf16_t*)f.residual + at, sum);
+    store4(f.sum_out + at, weighted);
+  }
+  sq += __shfl_xor(sq, 16, 64);
+  sq += __shfl_xor(sq, 32, 64);
+  if (grp == 0 && col < M) f.ss_out[(size_t)col * gridDim.x + blockIdx.x] = sq;
+}
+
+// `rows` rows of w a block, in tiles of `height`, without biases and a residual: the next tile's weights are under way while a
+// tile is finished. (After the last one each lane asks for the matrix's first bytes instead: with a branch there the compiler
+// waits for all loads before it uses one.)
+template <int AHEAD, bool GLU, bool FUSED, typename TOut>
+__global__ __launch_bounds__(64 * TW) void gemm_fewrows_walk_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ w, TOut* __restrict__ y,
+                                                                    int M, int N, int K, int rows, int height, int groups, const Fusion f) {
+  constexpr int NA = GLU ? 2 : 1;
+  extern __shared__ __attribute__((aligned(16))) unsigned char lds_raw[];
+  floatx4(*red)[NA][64] = reinterpret_cast<floatx4(*)[NA][64]>(lds_raw);       // [2 TW][NA][64]: one tile's and the next one's
+  bf16_t* x_s = reinterpret_cast<bf16_t*>(lds_raw + 2 * TW * NA * sizeof(floatx4) * 64);
+  __shared__ float r_s[16];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int col = lane & 15, grp = lane >> 4;
+  float share[SCALE_ROWS<TW>][SCALE_SHARES];
+  if constexpr (FUSED) ask_row_scales<TW>(f, share, M, wave, lane);
+  ask_x(x, x_s, M, K, wave, lane);
+  const int k0 = wave * groups * AHEAD * 32 + grp * 8, k_end = min((wave + 1) * groups * AHEAD * 32, K);
+  const char* wb[2] = {reinterpret_cast<const char*>(w), reinterpret_cast<const char*>(w + (size_t)N * K)};
+  const bf16_t* xrow_s = x_s + min(col, M - 1) * (K + 8);
+  // (blocks side by side have tiles side by side: 2 % less time than with all of a block's rows in one place)
+  const int tiles = (rows + height - 1) / height;
+  auto height_of = [&](int tile) { return tile + 1 < tiles ? height : rows - (tiles - 1) * height; };
+  auto first_of = [&](int tile) { return tile * (int)gridDim.x * height + (int)blockIdx.x * height_of(tile); };
+  auto row_of = [&](int tile) { return (unsigned)min(first_of(tile) + min(col, height_of(tile) - 1), N - 1) * K * 2; };
+  int tile = 0, turn = 0, parity = 0, g = 0;
+  bf16x8 a[AHEAD][NA];
+  auto ask = [&](int u, unsigned at) {
+#pragma unroll
+    for (int na = 0; na < NA; ++na) a[u][na] = *reinterpret_cast<const bf16x8*>(wb[na] + at);
+  };
+  auto k_of = [&](int s) { return (unsigned)min(k0 + s * 32, K - 8) * 2; };
+  unsigned row = row_of(0);
+  asm volatile("" ::: "memory");
+  __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+  for (int u = 0; u < AHEAD; ++u) ask(u, row + k_of(u));
+  wait_for_x<AHEAD * NA>();
+  if constexpr (FUSED) set_row_scales<TW>(f, share, r_s, M, K, wave, lane);
+  floatx4 acc[NA];
+#pragma unroll
+  for (int na = 0; na < NA; ++na) acc[na] = floatx4{0.f, 0.f, 0.f, 0.f};
+  while (true) {
+    const bool last = g + 1 == groups, more = !last || (tile + 1 < tiles && first_of(tile + 1) < N);
+    const unsigned row_next = last ? row_of(tile + 1) : row;
+    const int s_next = last ? 0 : (g + 1) * AHEAD;
+#pragma unroll
+    for (int u = 0; u < AHEAD; ++u) {
+      const int k = k0 + (g * AHEAD + u) * 32;
+      const unsigned in = k < k_end ? ~0u : 0u;
+      const bf16x8 bu = masked(*reinterpret_cast<const bf16x8*>(xrow_s + min(k, K - 8)), in);
+#pragma unroll
+      for (int na = 0; na < NA; ++na) {
+        asm volatile("" : "+v"(a[u][na]));                           // (nothing of it is done before it is this step's turn)
+        acc[na] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(masked(a[u][na], in), bu, acc[na], 0, 0, 0);
+      }
+      ask(u, more ? row_next + k_of(s_next + u) : 0u);
+    }
+    ++g;
+    if (!last) continue;
+    floatx4(*my_red)[NA][64] = red + parity * TW;
+#pragma unroll
+    for (int na = 0; na < NA; ++na) {
+      my_red[wave][na][lane] = acc[na];
+      acc[na] = floatx4{0.f, 0.f, 0.f, 0.f};
+    }
+    lds_barrier();
+    if (wave == turn) {
+      float out[4];
+      add_waves<GLU, FUSED>(f, my_red, r_s, nullptr, false, out, lane);
+      const int n = first_of(tile) + grp * 4;
+      if (col < M && grp * 4 < height_of(tile) && n < N) store4(y + (size_t)col * N + n, out);
+    }
+    if (!more) break;
+    ++tile, row = row_next, g = 0, parity ^= 1, turn = turn + 1 == TW ? 0 : turn + 1;
+  }
+}
+
 constexpr size_t LDS_BYTES = 160 * 1024 - 64;      // (64 bytes are the rows' scales, which every kernel keeps beside)
+// How the kernels above are launched; ahead == 0 where they are not the ones to take.
+struct TilesPlan {
+  int ahead;
+  bool x_in_lds;
+  int rows, height, groups;                                 // rows of w a block and a tile
+  size_t lds;
+};
+static TilesPlan tiles_plan(bool glu, bool squares, bool biased, int M, int N, int K) {
+  TilesPlan p = {};
+  if (N % 4 || (size_t)N * K * sizeof(bf16_t) >> 32) return p;       // (four outputs a store; places in w are 32 bits)
+  // as many rows a block as give each of the 256 compute units the same (sums of squares go out by tiles of 16)
+  p.rows = squares ? 16 : 4 * ((N + 4 * 256 - 1) / (4 * 256));
+  const int tiles = (p.rows + 15) / 16;
+  p.height = 4 * ((p.rows + 4 * tiles - 1) / (4 * tiles));
+  const size_t sums = (size_t)(tiles > 1 ? 2 : 1) * TW * (glu ? 2 : 1) * 64 * sizeof(floatx4), x_bytes = (size_t)M * (K + 8) * 2;
+  p.x_in_lds = sums + x_bytes <= LDS_BYTES;
+  // The kernels below it is where a product of several tiles a block has biases or a residual, and where x does not fit into LDS,
+  // but for up to 8 rows on the whole chip (4,096 outputs of 12,288 columns at 8 rows 25.2 against 26.8 us; 3,584 of 18,944 on
+  // 224 units, where x beside w is too much for a unit, 36.4 against 33.9; 4,096 of 12,288 at 16 rows 31.4 against 30.7).
+  if (tiles > 1 && (biased || squares)) return p;
+  if (!p.x_in_lds && (glu || tiles > 1 || M > 8 || N <= 240 * p.rows)) return p;
+  p.lds = sums + (p.x_in_lds ? x_bytes : 0);
+  const int steps = ((K + 31) / 32 + 15) / 16;
+  int slots = 1 << 30;
+  for (int u : {2, 3, 4, 5, 6, 7, 8}) {            // the fewest steps in all, and as many at once as can be
+    if (u > (glu ? 5 : p.x_in_lds ? 8 : 6)) continue;
+    const int groups = (steps + u - 1) / u;
+    if (groups * u <= slots) p.ahead = u, p.groups = groups, slots = groups * u;
+  }
+  // So it is where a gated product walks over three tiles and more that come out even anyway (12,288 outputs of 4,096 columns at
+  // 4 rows: 38.0 against 39.1 us) or whose steps do not come out even here (18,944 of 3,584 at 8 rows: 53.3 against 54.6).
+  if (glu && tiles > 2 && (p.rows % 16 == 0 || slots != steps)) p.ahead = 0;
+  return p;
+}
+
+template <int AHEAD, bool GLU, bool XLDS, bool FUSED, typename TOut>
+static int launch_tiles(const TilesPlan& p, hipStream_t s, const void* x, const void* w, const void* bias, void* y, int M, int N, int K, const Fusion& f) {
+  // more than 64 KB of dynamic LDS has to be allowed once per kernel (and per process)
+  auto once = gemm_fewrows_tile_kernel<AHEAD, GLU, XLDS, FUSED, TOut>;
+  static const hipError_t allowed = hipFuncSetAttribute((const void*)once, hipFuncAttributeMaxDynamicSharedMemorySize, (int)LDS_BYTES);
+  if (allowed != hipSuccess) return nhv_fail("few-rows gemm: %s", hipGetErrorString(allowed));
+  const dim3 grid((N + p.rows - 1) / p.rows);
+  if (p.rows == p.height) {
+    hipLaunchKernelGGL(once, grid, dim3(64 * TW), p.lds, s, (const bf16_t*)x, (const bf16_t*)w, (const bf16_t*)bias, (TOut*)y, M, N, K,
+                       p.rows, p.groups, f);
+  } else if constexpr (XLDS) {
+    auto walk = gemm_fewrows_walk_kernel<AHEAD, GLU, FUSED, TOut>;
+    static const hipError_t allowed_too = hipFuncSetAttribute((const void*)walk, hipFuncAttributeMaxDynamicSharedMemorySize, (int)LDS_BYTES);
+    if (allowed_too != hipSuccess) return nhv_fail("few-rows gemm: %s", hipGetErrorString(allowed_too));
+    hipLaunchKernelGGL(walk, grid, dim3(64 * TW), p.lds, s, (const bf16_t*)x, (const bf16_t*)w, (TOut*)y, M, N, K, p.rows, p.height, p.groups, f);
+  }
+  return 0;
+}
 
 // The resident kernel's shape: waves, loads in flight and blocks per compute unit, from the best variants measured
 // (same shapes as below), and in how many pieces x comes; waves == 0 when this kernel is not the one to take.
@@ -758,6 +1084,19 @@ int nhv_gemm_fewrows_launch(bool glu, const void* x, const void* w, const void* 
     return 0;
   }
   if (fused && out_dtype != NHV_BF16) return nhv_fail("few-rows gemm: a product that takes over its neighbours' work gives bfloat16");
+  const TilesPlan tp = tiles_plan(glu, f.residual != nullptr, bias != nullptr, M, N, K);
+  const bool on_16 = (((uintptr_t)y | (uintptr_t)bias | (uintptr_t)f.residual | (uintptr_t)f.sum_out | (uintptr_t)f.next_w) & 15) == 0;
+#define NHV_TILES_CASE(AHEAD_, GLU_, XLDS_)                                                                            \
+  if (tp.ahead == AHEAD_ && glu == GLU_ && tp.x_in_lds == XLDS_ && on_16)                                             \
+    return fused                   ? launch_tiles<AHEAD_, GLU_, XLDS_, true, bf16_t>(tp, s, x, w, bias, y, M, N, K, f)   \
+           : out_dtype == NHV_BF16 ? launch_tiles<AHEAD_, GLU_, XLDS_, false, bf16_t>(tp, s, x, w, bias, y, M, N, K, f) \
+                                   : launch_tiles<AHEAD_, GLU_, XLDS_, false, float>(tp, s, x, w, bias, y, M, N, K, f);
+  NHV_TILES_CASE(2, true, true) NHV_TILES_CASE(3, true, true) NHV_TILES_CASE(4, true, true) NHV_TILES_CASE(5, true, true)
+  NHV_TILES_CASE(2, false, true) NHV_TILES_CASE(3, false, true) NHV_TILES_CASE(4, false, true) NHV_TILES_CASE(5, false, true)
+  NHV_TILES_CASE(6, false, true) NHV_TILES_CASE(7, false, true) NHV_TILES_CASE(8, false, true)
+  NHV_TILES_CASE(2, false, false) NHV_TILES_CASE(3, false, false) NHV_TILES_CASE(4, false, false) NHV_TILES_CASE(5, false, false)
+  NHV_TILES_CASE(6, false, false)
+#undef NHV_TILES_CASE
   const ResidentPlan rp = resident_plan(glu, M, N, K);
 #define NHV_RESIDENT_CASE(WV_, UN_, GLU_, PIECES_)                                                                     \
   if (rp.waves == WV_ && rp.unroll == UN_ && glu == GLU_ && (rp.nchunks > 1) == PIECES_)                              \

@@ -225,6 +225,49 @@ def test_few_rows_linear_bfloat16_in_all_its_variants(ops, M, N, K):
     assert torch.equal(ops.linear(x, w, out_dtype=torch.float32), ops.linear(x, w, out_dtype=torch.float32))
 
 
+@pytest.mark.parametrize("M,N,K", [
+    # one tile a block: of 4 rows, of 16, the last one cut off; a K of one piece, of part of the waves, of steps that do not come out even
+    (1, 4, 8), (3, 20, 40), (16, 1020, 520), (5, 1036, 1000), (2, 4096, 3592), (9, 4092, 4608), (16, 512, 9728),
+    # several tiles a block, even and not, and blocks at the end whose last tile lies beyond the matrix
+    (1, 4100, 264), (7, 6144, 3584), (16, 8200, 2560), (4, 9732, 1544), (3, 20484, 72),
+    # x beside w, and just not (LDS)
+    (8, 4096, 12288), (6, 3076, 16392), (4, 4092, 18440),
+])
+def test_tiles_of_few_rows_products(ops, M, N, K):
+    """Plain, activated, gated, with rows that lack their scales and added to a residual (bounds: float32 sums of K products of
+    size K^-1/2; one rounding to 8 bits, of values up to 8 where a residual is added)."""
+    b = ops.backend()
+    x, w = rnd(M, K, dtype=torch.bfloat16, seed=71), rnd(2 * N, K, dtype=torch.bfloat16, seed=72, scale=K ** -0.5)
+    bias, squares, eps = rnd(2 * N, dtype=torch.bfloat16, seed=73), rnd(M, 270, seed=74).abs() + 0.5, 1e-6
+    both = x.double() @ w.double().T
+    plain, wn = both[:, :N], w[:N].contiguous()
+    b.own_kernels_only = True
+    try:
+        torch.testing.assert_close(ops.linear(x, wn, out_dtype=torch.float32).double(), plain, rtol=1e-4, atol=2e-4)
+        torch.testing.assert_close(ops.linear(x, wn, bias[:N].contiguous()).double(), plain + bias[:N].double(), **tol(torch.bfloat16))
+        gated = lambda g, u: g * torch.sigmoid(g) * u
+        if 2 * N * K < 120_000_000:
+            torch.testing.assert_close(ops.gated_linear(x, w).double(), gated(plain, both[:, N:]), **tol(torch.bfloat16))
+    finally:
+        b.own_kernels_only = False
+    scale = torch.rsqrt(squares.double().sum(-1, keepdim=True) / K + eps)
+    out = torch.empty(M, N, dtype=torch.bfloat16, device="cuda")
+    b.fused_linear(x, wn, bias[:N].contiguous(), out, row_scales=(squares, eps))
+    torch.testing.assert_close(out.double(), plain * scale + bias[:N].double(), **tol(torch.bfloat16))
+    b.fused_linear(x, w, bias, out, gated=True, row_scales=(squares, eps))
+    want = both * scale + bias.double()
+    torch.testing.assert_close(out.double(), gated(want[:, :N], want[:, N:]), **tol(torch.bfloat16))
+    for dtype in DTYPES:
+        residual, next_w = rnd(M, N, dtype=dtype, seed=75), rnd(N, dtype=dtype, seed=76, scale=0.1) + 1
+        want = residual.double() + plain + bias[:N].double()
+        left = torch.empty(M, (N + 15) // 16, device="cuda")
+        b.fused_linear(x, wn, bias[:N].contiguous(), None, residual=residual, sum_out=out, ss_out=left, next_w=next_w)
+        torch.testing.assert_close(residual.double(), want, **(dict(rtol=1e-4, atol=2e-4) if dtype == torch.float32 else tol(dtype)))
+        torch.testing.assert_close(out.double(), want * next_w.double(), **tol(torch.bfloat16))
+        tiles = torch.nn.functional.pad(want, (0, -N % 16)).view(M, -1, 16).pow(2).sum(-1)
+        torch.testing.assert_close(left.double(), tiles, rtol=1e-3, atol=1e-3)
+
+
 @pytest.mark.parametrize("M,I,K", [(1, 112, 80), (5, 1001, 96), (16, 12288, 4096), (17, 160, 96), (64, 300, 1024),
                                    (4, 17408, 136), (16, 25600, 72), (13, 25000, 264), (16, 9000, 5120), (15, 520, 5384)])
 def test_gated_linear(ops, M, I, K):
