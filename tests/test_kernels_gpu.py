@@ -613,6 +613,29 @@ def test_depth_mix_in_all_its_widths(ops, dtype, W):
         x = got
 
 
+@pytest.mark.parametrize("rows_dtype,result_dtype", [(torch.bfloat16, torch.bfloat16), (torch.float32, torch.float32), (torch.bfloat16, torch.float32)])
+@pytest.mark.parametrize("W", [4, 1000, 1028, 2048, 2052, 4100, 8192, 8196, 16384, 16388, 1001])
+def test_sandwich_step_in_all_its_widths(ops, W, rows_dtype, result_dtype):
+    """One, two and four passes, full and not, and what is not read four at a time; both halves and either alone."""
+    T, ea, eb = 3, 1e-5, 1e-3
+    x, y, wa, wb = rnd(T, W, seed=81), rnd(T, W, dtype=result_dtype, seed=82), rnd(W, seed=83) + 1, rnd(W, seed=84) + 1
+    unit = lambda t, eps: t / torch.sqrt(t.pow(2).mean(-1, keepdim=True) + eps)
+    want = x.double() + unit(y.double(), eb) * wb.double()
+    stream = x.clone()
+    read = ops.sandwich_step(stream, read=(wa, ea), rows_dtype=rows_dtype)
+    torch.testing.assert_close(read.double(), unit(x.double(), ea) * wa.double(), **tol(rows_dtype))
+    assert torch.equal(stream, x)
+    both = ops.sandwich_step(stream, add=(y, wb, eb), read=(wa, ea), rows_dtype=rows_dtype)
+    torch.testing.assert_close(stream.double(), want, rtol=1e-5, atol=1e-5)
+    torch.testing.assert_close(both.double(), unit(want, ea) * wa.double(), **tol(rows_dtype))
+    alone = x.clone()
+    assert ops.sandwich_step(alone, add=(y, wb, eb)) is None
+    assert torch.equal(alone, stream)
+    # a token's result is its own, whatever the batch
+    one = x[1:2].clone()
+    assert torch.equal(ops.sandwich_step(one, add=(y[1:2].contiguous(), wb, eb), read=(wa, ea), rows_dtype=rows_dtype)[0], both[1])
+
+
 @pytest.mark.parametrize("D,split_len,n_splits,window", [
     (128, 64, 5, None),      # one wave, four splits a lane
     (128, 64, 20, None),     # four waves, four splits a lane; the last waves' splits lie past every position but one
