@@ -621,7 +621,7 @@ __device__ __forceinline__ void lds_barrier() {
 // down, which ask for two steps at a time and wait for the residual before the weights: 1,024 outputs of 2,048 and 3,072 columns
 // added to a residual at 1 row 6.4 -> 4.9 us and 8.5 -> 6.3, at 16 rows 8.0 -> 6.0 and 11.1 -> 8.0; 4,096 of 4,096 at 8 rows
 // 12.4 -> 10.4; 6,144 of 4,096 13.7 -> 12.2 and 15.4 -> 13.0 at 1 and 8; gated 9,728 of 2,560 26.3 -> 23.3, 3,072 of 1,024 at
-// 16 rows 9.9 -> 6.8.
+// 16 rows 9.9 -> 6.8, with biases 6,144 of 2,048 at 5 rows 16.9 -> 14.6.
 constexpr int TW = 16;                       // waves
 
 // x into LDS, [M][K + 8] (the 16 bytes between rows spread the rows over the banks): a wave's load brings 64 consecutive
@@ -646,7 +646,7 @@ __device__ __forceinline__ bf16x8 masked(bf16x8 v, unsigned mask) { return (bf16
 
 // A tile's sums of the waves (red[wave][matrix][lane]), added in the order of the waves; then the rows' scales, the biases, the gate.
 template <bool GLU, bool FUSED>
-__device__ __forceinline__ void add_waves(const Fusion& f, const floatx4 (*red)[GLU ? 2 : 1][64], const float* r_s, const Four* bias4, bool biased,
+__device__ __forceinline__ void add_waves(const Fusion& f, const floatx4 (*red)[GLU ? 2 : 1][64], const float* r_s, bool biased, const float (&bias)[GLU ? 2 : 1][4],
                                           float (&out)[4], int lane) {
   constexpr int NA = GLU ? 2 : 1, SIDE = 8 / NA;                     // (so many at once: the registers that are left)
   floatx4 v[NA];
@@ -669,7 +669,7 @@ __device__ __forceinline__ void add_waves(const Fusion& f, const floatx4 (*red)[
 #pragma unroll
   for (int j = 0; j < 4; ++j) {
     float r = v[0][j] * rs, up = v[NA - 1][j] * rs;
-    if (biased) r += bias4[0].at(j, 0), up += bias4[NA - 1].at(j, 0);
+    if (biased) r += bias[0][j], up += bias[NA - 1][j];
     if (GLU) r = nhv_gated(r, up, f.gate);
     else if (f.plain_act) r = nhv_plain_act(r, f.plain_act);
     out[j] = r;
@@ -750,8 +750,12 @@ __global__ __launch_bounds__(64 * TW) void gemm_fewrows_tile_kernel(const bf16_t
   lds_barrier();
   if (wave > 0) return;
 
-  float out[4];
-  add_waves<GLU, FUSED>(f, red, r_s, bias4, bias != nullptr, out, lane);
+  float out[4], bias_here[NA][4];
+#pragma unroll
+  for (int na = 0; na < NA; ++na)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) bias_here[na][j] = bias4[na].at(j, 0);
+  add_waves<GLU, FUSED>(f, red, r_s, bias != nullptr, bias_here, out, lane);
   const bool mine = col < M && grp * 4 < rows && n < N;
   const size_t at = (size_t)col * N + n;
   if (!FUSED || GLU || f.residual == nullptr) {
@@ -775,22 +779,22 @@ __global__ __launch_bounds__(64 * TW) void gemm_fewrows_tile_kernel(const bf16_t
   if (grp == 0 && col < M) f.ss_out[(size_t)col * gridDim.x + blockIdx.x] = sq;
 }
 
-// `rows` rows of w a block, in tiles of `height`, without biases and a residual: the next tile's weights are under way while a
-// tile is finished. (After the last one each lane asks for the matrix's first bytes instead: with a branch there the compiler
+// `rows` rows of w a block, in tiles of `height`, without a residual: the next tile's weights are under way while a tile is
+// finished, whose biases lie in LDS from the start (asked for tile by tile they would be waited for behind the weights). (After the last one each lane asks for the matrix's first bytes instead: with a branch there the compiler
 // waits for all loads before it uses one.)
-template <int AHEAD, bool GLU, bool FUSED, typename TOut>
-__global__ __launch_bounds__(64 * TW) void gemm_fewrows_walk_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ w, TOut* __restrict__ y,
-                                                                    int M, int N, int K, int rows, int height, int groups, const Fusion f) {
+template <int AHEAD, bool GLU, bool FUSED, bool BIASED, typename TOut>
+__global__ __launch_bounds__(64 * TW) void gemm_fewrows_walk_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ w,
+                                                                    const bf16_t* __restrict__ bias, TOut* __restrict__ y, int M, int N, int K, int rows, int height, int groups, const Fusion f) {
   constexpr int NA = GLU ? 2 : 1;
   extern __shared__ __attribute__((aligned(16))) unsigned char lds_raw[];
   floatx4(*red)[NA][64] = reinterpret_cast<floatx4(*)[NA][64]>(lds_raw);       // [2 TW][NA][64]: one tile's and the next one's
   bf16_t* x_s = reinterpret_cast<bf16_t*>(lds_raw + 2 * TW * NA * sizeof(floatx4) * 64);
+  float* bias_s = reinterpret_cast<float*>(x_s + M * (K + 8));                 // [NA][rows] and what a lane beyond the last tile reads
   __shared__ float r_s[16];
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int col = lane & 15, grp = lane >> 4;
   float share[SCALE_ROWS<TW>][SCALE_SHARES];
   if constexpr (FUSED) ask_row_scales<TW>(f, share, M, wave, lane);
-  ask_x(x, x_s, M, K, wave, lane);
   const int k0 = wave * groups * AHEAD * 32 + grp * 8, k_end = min((wave + 1) * groups * AHEAD * 32, K);
   const char* wb[2] = {reinterpret_cast<const char*>(w), reinterpret_cast<const char*>(w + (size_t)N * K)};
   const bf16_t* xrow_s = x_s + min(col, M - 1) * (K + 8);
@@ -800,6 +804,12 @@ __global__ __launch_bounds__(64 * TW) void gemm_fewrows_walk_kernel(const bf16_t
   auto first_of = [&](int tile) { return tile * (int)gridDim.x * height + (int)blockIdx.x * height_of(tile); };
   auto row_of = [&](int tile) { return (unsigned)min(first_of(tile) + min(col, height_of(tile) - 1), N - 1) * K * 2; };
   int tile = 0, turn = 0, parity = 0, g = 0;
+  unsigned bias_bits = 0;                                            // one a thread: NA rows are no more than the block's threads
+  if constexpr (BIASED) {
+    const int mine = min((int)threadIdx.x, NA * rows - 1), my_row = mine % rows;
+    bias_bits = reinterpret_cast<const unsigned short*>(bias)[(size_t)(mine / rows) * N + min(first_of(my_row / height) + my_row % height, N - 1)];
+  }
+  ask_x(x, x_s, M, K, wave, lane);
   bf16x8 a[AHEAD][NA];
   auto ask = [&](int u, unsigned at) {
 #pragma unroll
@@ -812,6 +822,7 @@ __global__ __launch_bounds__(64 * TW) void gemm_fewrows_walk_kernel(const bf16_t
 #pragma unroll
   for (int u = 0; u < AHEAD; ++u) ask(u, row + k_of(u));
   wait_for_x<AHEAD * NA>();
+  if constexpr (BIASED) if ((int)threadIdx.x < NA * rows) bias_s[threadIdx.x] = __uint_as_float(bias_bits << 16);
   if constexpr (FUSED) set_row_scales<TW>(f, share, r_s, M, K, wave, lane);
   floatx4 acc[NA];
 #pragma unroll
@@ -842,8 +853,12 @@ __global__ __launch_bounds__(64 * TW) void gemm_fewrows_walk_kernel(const bf16_t
     }
     lds_barrier();
     if (wave == turn) {
-      float out[4];
-      add_waves<GLU, FUSED>(f, my_red, r_s, nullptr, false, out, lane);
+      float out[4], bias_here[NA][4];
+#pragma unroll
+      for (int na = 0; na < NA; ++na)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) bias_here[na][j] = BIASED ? bias_s[na * rows + tile * height + grp * 4 + j] : 0.f;
+      add_waves<GLU, FUSED>(f, my_red, r_s, BIASED, bias_here, out, lane);
       const int n = first_of(tile) + grp * 4;
       if (col < M && grp * 4 < height_of(tile) && n < N) store4(y + (size_t)col * N + n, out);
     }
@@ -868,13 +883,14 @@ static TilesPlan tiles_plan(bool glu, bool squares, bool biased, int M, int N, i
   const int tiles = (p.rows + 15) / 16;
   p.height = 4 * ((p.rows + 4 * tiles - 1) / (4 * tiles));
   const size_t sums = (size_t)(tiles > 1 ? 2 : 1) * TW * (glu ? 2 : 1) * 64 * sizeof(floatx4), x_bytes = (size_t)M * (K + 8) * 2;
-  p.x_in_lds = sums + x_bytes <= LDS_BYTES;
-  // The kernels below it is where a product of several tiles a block has biases or a residual, and where x does not fit into LDS,
+  const size_t biases = tiles > 1 && biased ? ((glu ? 2 : 1) * p.rows + 16) * sizeof(float) : 0;
+  p.x_in_lds = sums + x_bytes + biases <= LDS_BYTES;
+  // The kernels below it is where a product of several tiles a block has a residual (or more biases than threads), and where x does not fit into LDS,
   // but for up to 8 rows on the whole chip (4,096 outputs of 12,288 columns at 8 rows 25.2 against 26.8 us; 3,584 of 18,944 on
   // 224 units, where x beside w is too much for a unit, 36.4 against 33.9; 4,096 of 12,288 at 16 rows 31.4 against 30.7).
-  if (tiles > 1 && (biased || squares)) return p;
+  if (tiles > 1 && (squares || biases > (64 * TW + 16) * sizeof(float))) return p;
   if (!p.x_in_lds && (glu || tiles > 1 || M > 8 || N <= 240 * p.rows)) return p;
-  p.lds = sums + (p.x_in_lds ? x_bytes : 0);
+  p.lds = sums + (p.x_in_lds ? x_bytes + biases : 0);
   const int steps = ((K + 31) / 32 + 15) / 16;
   int slots = 1 << 30;
   for (int u : {2, 3, 4, 5, 6, 7, 8}) {            // the fewest steps in all, and as many at once as can be
@@ -899,10 +915,14 @@ static int launch_tiles(const TilesPlan& p, hipStream_t s, const void* x, const 
     hipLaunchKernelGGL(once, grid, dim3(64 * TW), p.lds, s, (const bf16_t*)x, (const bf16_t*)w, (const bf16_t*)bias, (TOut*)y, M, N, K,
                        p.rows, p.groups, f);
   } else if constexpr (XLDS) {
-    auto walk = gemm_fewrows_walk_kernel<AHEAD, GLU, FUSED, TOut>;
-    static const hipError_t allowed_too = hipFuncSetAttribute((const void*)walk, hipFuncAttributeMaxDynamicSharedMemorySize, (int)LDS_BYTES);
-    if (allowed_too != hipSuccess) return nhv_fail("few-rows gemm: %s", hipGetErrorString(allowed_too));
-    hipLaunchKernelGGL(walk, grid, dim3(64 * TW), p.lds, s, (const bf16_t*)x, (const bf16_t*)w, (TOut*)y, M, N, K, p.rows, p.height, p.groups, f);
+    // (the biases' reads cost a product without any 1 % as a condition)
+    auto without = gemm_fewrows_walk_kernel<AHEAD, GLU, FUSED, false, TOut>, with = gemm_fewrows_walk_kernel<AHEAD, GLU, FUSED, true, TOut>;
+    static const hipError_t allowed_too[2] = {hipFuncSetAttribute((const void*)without, hipFuncAttributeMaxDynamicSharedMemorySize, (int)LDS_BYTES),
+                                              hipFuncSetAttribute((const void*)with, hipFuncAttributeMaxDynamicSharedMemorySize, (int)LDS_BYTES)};
+    for (hipError_t e : allowed_too)
+      if (e != hipSuccess) return nhv_fail("few-rows gemm: %s", hipGetErrorString(e));
+    hipLaunchKernelGGL(bias ? with : without, grid, dim3(64 * TW), p.lds, s, (const bf16_t*)x, (const bf16_t*)w, (const bf16_t*)bias, (TOut*)y, M, N, K, p.rows, p.height,
+                       p.groups, f);
   }
   return 0;
 }
