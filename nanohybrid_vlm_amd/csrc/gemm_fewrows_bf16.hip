@@ -621,7 +621,7 @@ __device__ __forceinline__ void lds_barrier() {
 // down, which ask for two steps at a time and wait for the residual before the weights: 1,024 outputs of 2,048 and 3,072 columns
 // added to a residual at 1 row 6.4 -> 4.9 us and 8.5 -> 6.3, at 16 rows 8.0 -> 6.0 and 11.1 -> 8.0; 4,096 of 4,096 at 8 rows
 // 12.4 -> 10.4; 6,144 of 4,096 13.7 -> 12.2 and 15.4 -> 13.0 at 1 and 8; gated 9,728 of 2,560 26.3 -> 23.3, 3,072 of 1,024 at
-// 16 rows 9.9 -> 6.8, with biases 6,144 of 2,048 at 5 rows 16.9 -> 14.6.
+// 16 rows 9.9 -> 6.8, with biases 6,144 of 2,048 at 5 rows 16.9 -> 13.8.
 constexpr int TW = 16;                       // waves
 
 // x into LDS, [M][K + 8] (the 16 bytes between rows spread the rows over the banks): a wave's load brings 64 consecutive
