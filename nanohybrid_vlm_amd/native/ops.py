@@ -531,14 +531,19 @@ class NativeBackend:
         covered = batch.max_context_len
         if self.planned_context and self.covered_context:
             covered = min(covered, self.covered_context)
-        # A block of eight waves takes 256 keys in the time of 32. One split where the blocks fill the chip anyway (24 to 128
-        # requests of 8 key/value heads: no split faster) or where its rounds are over before a merge would be (one request of
+        # A block of eight waves takes 256 keys in the time of 32. One split where the blocks fill the chip anyway (24 to 32 and
+        # 56 to 128 requests of 8 key/value heads: no split faster) or where its rounds are over before a merge would be (one request of
         # 16 heads, 150 keys: 6.2 us, two splits of 128 8.3; eight of 300 keys 8.4 against 9.9; one of 1,000 14.4 against
         # 9.4). Else one block a compute unit, splits of at least 128 keys and not many more than 32 of them, which is what
         # the merge takes at once (8 x 2,050 keys: 21.3 us with splits of 512, 23.7 with 384 or 256; 8 x 4,000: 31.5 with
         # 1,024, 36.6 with 256; 1 x 9,000: 15.4 with 384, 19.5 with 256).
+        # A little over one block a unit is the exception: most units would wait for the few that have two. Three splits there, two
+        # up to 416 blocks (8 heads, all of 2,176 keys: 40 requests 75 us against 88, 48 requests 85 against 92; of 100 to 2,000
+        # keys, where the longest go first, 42.2 against 40.9 and 52 against 44).
         blocks = T * Hkv * -(-(Hq // Hkv) // 16)            # (a block takes up to 16 heads of a key/value head)
-        if blocks >= 192 or span <= 448:
+        if 256 < blocks <= 416 and span > 448:
+            split_len = 128 * -(-span // (128 * (3 if blocks <= 352 else 2)))
+        elif blocks >= 192 or span <= 448:
             split_len = -(-covered // 32) * 32
         else:
             split_len = max(128, 128 * round(max(span * blocks / 256, covered / 36) / 128))
