@@ -634,7 +634,10 @@ __device__ __forceinline__ void ask_x(const bf16_t* __restrict__ x, bf16_t* x_s,
       __builtin_amdgcn_global_load_lds((global_ptr)(x + (size_t)m * K + (part * 64 + lane) * 8), (lds_ptr)(x_s + m * (K + 8) + part * 512), 16, 0, 0);
   }
 }
-// The wait for x alone, when YOUNGER loads have been asked for since (a fence would wait for all).
+// The wait for x alone, when YOUNGER loads have been asked for since (a fence would wait for all). It holds only while exactly
+// these loads, the weights' first ones, stand between x's and the wait, so the two kernels' w is no __restrict__ pointer: loads
+// through one may legally cross an asm that clobbers memory, loads of memory that the asm may have written may not, neither this
+// one nor the one in front of the first of them. (A test counts the loads in what the compiler makes of each kernel.)
 template <int YOUNGER>
 __device__ __forceinline__ void wait_for_x() {
   __builtin_amdgcn_sched_barrier(0);
@@ -679,10 +682,11 @@ __device__ __forceinline__ void add_waves(const Fusion& f, const floatx4 (*red)[
 // One tile a block. XLDS: x is brought to LDS, its loads before the first weights', and the wait before the first product is
 // for x alone; without, x comes from memory step by step beside w.
 template <int AHEAD, bool GLU, bool XLDS, bool FUSED, typename TOut>
-__global__ __launch_bounds__(64 * TW) void gemm_fewrows_tile_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ w,
+__global__ __launch_bounds__(64 * TW) void gemm_fewrows_tile_kernel(const bf16_t* __restrict__ x, const bf16_t* w,
                                                                     const bf16_t* __restrict__ bias, TOut* __restrict__ y, int M, int N, int K,
                                                                     int rows, int groups, const Fusion f) {
   constexpr int NA = GLU ? 2 : 1;
+  asm volatile("" ::"s"(w));               // (fetched with the other arguments, not where it is first used)
   extern __shared__ __attribute__((aligned(16))) unsigned char lds_raw[];
   floatx4(*red)[NA][64] = reinterpret_cast<floatx4(*)[NA][64]>(lds_raw);       // [TW][NA][64]
   bf16_t* x_s = reinterpret_cast<bf16_t*>(lds_raw + TW * NA * sizeof(floatx4) * 64);
@@ -783,9 +787,10 @@ __global__ __launch_bounds__(64 * TW) void gemm_fewrows_tile_kernel(const bf16_t
 // finished, whose biases lie in LDS from the start (asked for tile by tile they would be waited for behind the weights). (After the last one each lane asks for the matrix's first bytes instead: with a branch there the compiler
 // waits for all loads before it uses one.)
 template <int AHEAD, bool GLU, bool FUSED, bool BIASED, typename TOut>
-__global__ __launch_bounds__(64 * TW) void gemm_fewrows_walk_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ w,
+__global__ __launch_bounds__(64 * TW) void gemm_fewrows_walk_kernel(const bf16_t* __restrict__ x, const bf16_t* w,
                                                                     const bf16_t* __restrict__ bias, TOut* __restrict__ y, int M, int N, int K, int rows, int height, int groups, const Fusion f) {
   constexpr int NA = GLU ? 2 : 1;
+  asm volatile("" ::"s"(w));               // (fetched with the other arguments, not where it is first used)
   extern __shared__ __attribute__((aligned(16))) unsigned char lds_raw[];
   floatx4(*red)[NA][64] = reinterpret_cast<floatx4(*)[NA][64]>(lds_raw);       // [2 TW][NA][64]: one tile's and the next one's
   bf16_t* x_s = reinterpret_cast<bf16_t*>(lds_raw + 2 * TW * NA * sizeof(floatx4) * 64);

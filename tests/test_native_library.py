@@ -4,6 +4,8 @@ What is checked here is how it fails and when it builds again: there is no other
 missing compiler or a source that does not compile has to say so, at once and by name.
 """
 import os
+import re
+import subprocess
 
 import pytest
 
@@ -57,3 +59,33 @@ def test_built_once_and_again_when_a_source_or_a_header_changes(sandbox):
     lib = library.load_library("probe", ["good.hip"])
     assert lib.answer() == 43                       # host code only: nothing here touches a GPU
     assert library.load_library("probe", ["good.hip"]) is lib
+
+
+def test_the_wait_for_x_has_the_loads_behind_it_that_it_counts(tmp_path):
+    """The few-rows products wait for their rows of x by the number of loads asked for since (``wait_for_x``). The weights'
+    pointer must be one whose loads cannot legally leave their place (no ``__restrict__``), and in what the compiler makes of each
+    kernel so many loads must stand between the last one of x and the wait."""
+    source = os.path.join(library.CSRC, "gemm_fewrows_bf16.hip")
+    text = open(source).read()
+    for kernel in ("gemm_fewrows_tile_kernel", "gemm_fewrows_walk_kernel"):
+        arguments = re.search(r"void %s\((.*?)\{" % kernel, text, re.S)[1]
+        assert re.search(r"const bf16_t\s*\*\s*w\b", arguments), arguments
+    out = tmp_path / "fewrows.s"
+    subprocess.run([library._hipcc(), *[f for f in library.HIPCC_FLAGS if f != "-fPIC"], "-I", library.CSRC, "--cuda-device-only", "-S",
+                    source, "-o", str(out)], check=True, capture_output=True)
+    listing, seen = out.read_text(), 0
+    name = re.compile(r"^(\S*gemm_fewrows_(tile|walk)_kernelILi(\d+)ELb([01])ELb([01])\S*):", re.M)
+    for m in name.finditer(listing):
+        if m[2] == "tile" and m[5] == "0":
+            continue                                     # (x does not lie in LDS: nothing to wait for)
+        body = listing[m.end():listing.index(".Lfunc_end", m.end())].split("\n")
+        ops = [" ".join(line.split(";")[0].split()) for line in body]
+        last = max(i for i, op in enumerate(ops) if "global_load_lds" in op)
+        barrier = next(i for i in range(last, len(ops)) if ops[i].startswith("s_barrier"))
+        between = ops[last + 1:barrier]
+        waits = [int(n) for op in between for n in re.findall(r"vmcnt\((\d+)\)", op)]
+        loads = sum(op.startswith("global_load") for op in between)
+        assert waits == [int(m[3]) * (2 if m[4] == "1" else 1)] and loads >= waits[0], (m[1], waits, loads)
+        assert not any(op.startswith(("scratch", "buffer", "flat", "global_store")) for op in between), m[1]
+        seen += 1
+    assert seen >= 50, seen
