@@ -210,7 +210,9 @@ __global__ __launch_bounds__(64 * WAVES) void attention_float32_kernel(FloatAtte
     __syncthreads();
     for (int p = 0; p < WAVES && round + p * KEYS <= tile_hi; ++p) {
       const float m = stats[(p * ROWS + my_row) * 2], l = stats[(p * ROWS + my_row) * 2 + 1];
-      if (m == -INFINITY) continue;                      // this row reads no key of the block
+      // a block of which this row reads no key, or none with a weight. (The maximum alone does not say that: fmaxf passes over a
+      // score that is no number, and where all are such the sum of the weights tells.)
+      if (m == -INFINITY && l == 0.f) continue;
       const float top = fmaxf(M, m), old = expf(M - top), now = expf(m - top);
       L = L * old + l * now;
       M = top;

@@ -539,6 +539,29 @@ def test_float32_attention_of_whole_tiles(ops, Hq, Hkv, D, E, page, reach, cap, 
     assert not torch.isfinite(spoilt[hit.cuda()]).any()
     torch.testing.assert_close(spoilt[~hit.cuda()], out[~hit.cuda()], rtol=1e-5, atol=1e-5)
 
+@pytest.mark.parametrize("sink", [None, 0.3])
+@pytest.mark.parametrize("dtype,D", [(torch.float32, 64), (torch.float32, 192), (torch.float32, 20)])
+def test_attention_hides_no_score_that_is_no_number(ops, dtype, D, sink):
+    """A key or a query that is no number: what reads it is no number either, also where it is the only one of its block of keys
+    (33, 65 and 257 keys) or where a sink would stand in for the rest; everything else keeps its bits."""
+    lens, q_lens = [33, 65, 257, 1, 40, 300], [33, 1, 2, 1, 7, 60]
+    q, kc, vc, batch, bt, *_ = _paged_setup(dtype, lens, q_lens, 4, 2, D, 16, seed=63)
+    options = {} if sink is None else {"sink": sink}
+    clean = ops.paged_attention(q, kc, vc, batch, bt, D ** -0.5, **options)
+    assert torch.isfinite(clean).all()
+    bad = kc.clone()
+    for r, n in enumerate(lens):
+        bad[bt[r, (n - 1) // 16], (n - 1) % 16, 1, D // 2] = float("nan")       # the last key, read by the last token's heads 2 and 3
+    out = ops.paged_attention(q, bad, vc, batch, bt, D ** -0.5, **options)
+    hit = torch.zeros(q.shape[:2], dtype=torch.bool, device="cuda")
+    hit[batch.cu_seqlens_q[1:].long() - 1, 2:] = True
+    assert torch.isnan(out[hit]).all() and torch.equal(out[~hit], clean[~hit])
+    spoilt, hit = q.clone(), torch.zeros_like(hit)
+    for t in (0, 32, 33, 34, 36, 44, 80):
+        spoilt[t, 3, 0], hit[t, 3] = float("nan"), True
+    out = ops.paged_attention(spoilt, kc, vc, batch, bt, D ** -0.5, **options)
+    assert torch.isnan(out[hit]).all() and torch.equal(out[~hit], clean[~hit])
+
 
 @pytest.mark.parametrize("Hq,Hkv,D,page,window", [
     (4, 2, 16, 4, None), (6, 1, 32, 8, None), (5, 5, 48, 7, None), (3, 1, 80, 16, 9), (8, 2, 128, 64, None),
