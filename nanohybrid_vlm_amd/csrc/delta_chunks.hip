@@ -6,7 +6,11 @@
 // so with U the chunk's u, A = beta A' strictly below the diagonal and (I + A) solved forwards for every column:
 //   W = (I + A)^-1 beta E k,   V' = (I + A)^-1 beta v,   U = V' - W S_0,   O = E q S_0 + B U = R S_0 + B V',
 //   S_16 = E_16 S_0 + K^T U,   K_j = k_j 2^(l_16 - l_j).
-// Only differences of logarithms that are never positive are raised: a strong decay gives zeros, not overflows.
+// Only differences of logarithms that are never positive are raised: a strong decay gives zeros, not overflows. A sum of
+// logarithms is kept as a float and what its additions rounded off, and a token's logarithm is no lower than -256 (whose power
+// is 0 all the same): the difference of two sums is then as exact as a sum over the tokens between them, whatever decays came
+// before, and never inf - inf. (One float alone: after three tokens of -300 a state off by 3e-5 of its largest entry, and NaN
+// after an infinite one. Token by token and with both parts 1e-7.)
 // Two kernels:
 //  - nhv_delta_chunks_prepare: all chunks at once, a block per (chunk, head, request), from the projection's rows to W, R - B W,
 //    K, V', B and the chunk's decay: convolutions, SiLU, unit vectors, decays, products and the solution without a trip to
@@ -29,6 +33,7 @@ typedef __attribute__((__vector_size__(4 * sizeof(float)))) float floatx4;
 __device__ __forceinline__ float exp2_of(float x) { return __builtin_amdgcn_exp2f(x); }   // (x <= 0; tiny results may become 0)
 __device__ __forceinline__ float silu_of(float z) { return z / (1.0f + expf(-z)); }
 __device__ __forceinline__ float softplus_of(float z) { return z > 20.f ? z : log1pf(expf(z)); }
+#define NHV_LOWEST_LOG (-256.f)
 
 struct DeltaIn {
   const void* proj;                          // [T, ld]: q (G D) | k (G D) | v (H E) | beta (H)
@@ -95,6 +100,7 @@ __global__ __launch_bounds__(256, 4) void delta_chunks_prepare_kernel(const Delt
   extern __shared__ __attribute__((aligned(16))) float lds[];
   __shared__ __attribute__((aligned(16))) float A[NHV_CHUNK][NHV_CHUNK], B[NHV_CHUNK][NHV_CHUNK];
   __shared__ float beta[NHV_CHUNK];
+  __shared__ float2 last[256];               // a channel's sum over the chunk
   const int h = blockIdx.x, req = blockIdx.z;
   const int first = in.cu[req], i0 = blockIdx.y * NHV_CHUNK, t0 = first + i0, end = in.cu[req + 1];
   if (t0 >= end) return;                     // (the same for the whole block)
@@ -104,7 +110,7 @@ __global__ __launch_bounds__(256, 4) void delta_chunks_prepare_kernel(const Delt
   const int tid = threadIdx.x, LD = Dp + 4;  // (rows of an odd number of fours)
   float* qs = lds;
   float* ks = qs + NHV_CHUNK * LD;
-  float* ls = ks + NHV_CHUNK * LD;
+  float2* ls = reinterpret_cast<float2*>(ks + NHV_CHUNK * LD);       // the sums of logarithms and what they are short of
   const float* mine = in.kept + (size_t)in.state_slots[req] * C * (in.n_taps - 1);
 
   // queries and keys, a channel a thread; the decays' logarithms; beta
@@ -118,18 +124,25 @@ __global__ __launch_bounds__(256, 4) void delta_chunks_prepare_kernel(const Delt
 #pragma unroll
     for (int t = 0; t < NHV_CHUNK; ++t) to_row[t * LD] = y[t];
   }
-  const float rate = -NHV_LOG2E * expf(in.a_log[h]);
+  const float rate = expf(in.a_log[h]);
   for (int x = tid; x < NHV_CHUNK * Dp; x += 256) {
     const int t = x / Dp, d = x % Dp, at = h * Dd + (Dd == 1 ? 0 : d);
-    ls[t * LD + d] = t < n && d < D ? rate * softplus_of(in.a_lin[(size_t)(t0 + t) * in.a_ld + at] + in.dt_bias[at]) : 0.f;
+    const float l = t < n && d < D ? -NHV_LOG2E * (rate * softplus_of(in.a_lin[(size_t)(t0 + t) * in.a_ld + at] + in.dt_bias[at])) : 0.f;
+    ls[t * LD + d].x = l < NHV_LOWEST_LOG ? NHV_LOWEST_LOG : l;      // (what is no number stays none)
   }
   if (tid < NHV_CHUNK)
     beta[tid] = tid < n ? 1.0f / (1.0f + expf(-to_f32(((const TI*)in.proj)[(size_t)(t0 + tid) * in.ld + C + h]))) : 0.f;
   __syncthreads();
   for (int d = tid; d < Dp; d += 256) {
-    float sum = 0.f;
+    float sum = 0.f, rest = 0.f;
 #pragma unroll
-    for (int t = 0; t < NHV_CHUNK; ++t) ls[t * LD + d] = sum += ls[t * LD + d];
+    for (int t = 0; t < NHV_CHUNK; ++t) {
+      const float l = ls[t * LD + d].x, next = sum + l, part = next - sum;
+      rest += (sum - (next - part)) + (l - part);        // (what the addition rounded off, exactly)
+      sum = next;
+      ls[t * LD + d] = make_float2(sum, rest);
+    }
+    last[d] = make_float2(sum, rest);        // (a row beyond the request's end adds 0)
   }
   {                                          // unit length (the sum of squares plus 1e-6 under the root), q also times D^(-1/2)
     const int t = (tid >> 3) & 15;
@@ -152,7 +165,8 @@ __global__ __launch_bounds__(256, 4) void delta_chunks_prepare_kernel(const Delt
     int t = (int)((1.0f + sqrtf(1.0f + 8.0f * (float)p)) * 0.5f);
     t = t * (t - 1) / 2 > p ? t - 1 : ((t + 1) * t / 2 <= p ? t + 1 : t);
     const int j = p - t * (t - 1) / 2, d0 = (tid & 1) * 4;
-    const float *qt = qs + t * LD, *kt = ks + t * LD, *kj = ks + j * LD, *lt = ls + t * LD, *lj = ls + j * LD;
+    const float *qt = qs + t * LD, *kt = ks + t * LD, *kj = ks + j * LD;
+    const float2 *lt = ls + t * LD, *lj = ls + j * LD;
     floatx4 kk = {0.f, 0.f, 0.f, 0.f}, qk = {0.f, 0.f, 0.f, 0.f};
     if (Dd == 1) {
       for (int d = d0; d < Dp; d += 8) {
@@ -160,15 +174,19 @@ __global__ __launch_bounds__(256, 4) void delta_chunks_prepare_kernel(const Delt
         kk += *reinterpret_cast<const floatx4*>(kt + d) * x;
         qk += *reinterpret_cast<const floatx4*>(qt + d) * x;
       }
-      const float e = exp2_of(lt[0] - lj[0]);
+      const float e = exp2_of((lt[0].x - lj[0].x) + (lt[0].y - lj[0].y));
       kk *= e;
       qk *= e;
     } else {
 #pragma unroll 2
       for (int d = d0; d < Dp; d += 8) {
-        floatx4 x = *reinterpret_cast<const floatx4*>(lt + d) - *reinterpret_cast<const floatx4*>(lj + d);
+        floatx4 x;
 #pragma unroll
-        for (int i = 0; i < 4; ++i) x[i] = exp2_of(x[i]);
+        for (int i = 0; i < 4; i += 2) {
+          const floatx4 l = *reinterpret_cast<const floatx4*>(lt + d + i) - *reinterpret_cast<const floatx4*>(lj + d + i);
+          x[i] = exp2_of(l[0] + l[1]);
+          x[i + 1] = exp2_of(l[2] + l[3]);
+        }
         x *= *reinterpret_cast<const floatx4*>(kj + d);
         kk += *reinterpret_cast<const floatx4*>(kt + d) * x;
         qk += *reinterpret_cast<const floatx4*>(qt + d) * x;
@@ -189,13 +207,23 @@ __global__ __launch_bounds__(256, 4) void delta_chunks_prepare_kernel(const Delt
     B[t][t] = (qk[0] + qk[1]) + (qk[2] + qk[3]);
   }
   __syncthreads();
+  // E_t q_t, E_t k_t and, in the sums' place, k_t 2^(l_16 - l_t) (rows beyond n are zeros)
+  for (int x = tid; x < NHV_CHUNK * Dp; x += 256) {
+    const int d = x % Dp, at = x / Dp * LD + d;
+    const float2 l = ls[at];
+    const float e = exp2_of(l.x + l.y), k = ks[at];
+    qs[at] *= e;
+    ks[at] = e * k;
+    ls[at].x = k * exp2_of((last[d].x - l.x) + (last[d].y - l.y));
+  }
+  __syncthreads();
   // a column a thread: W's Dp, then V''s E
   for (int c = tid; c < Dp + E; c += 256) {
     const bool key = c < Dp;
     float x[NHV_CHUNK];
     if (key) {
 #pragma unroll
-      for (int t = 0; t < NHV_CHUNK; ++t) x[t] = exp2_of(ls[t * LD + c]) * ks[t * LD + c];
+      for (int t = 0; t < NHV_CHUNK; ++t) x[t] = ks[t * LD + c];
     } else {
       convolved<TI, TAPS>(in, 2 * G * D + h * E + c - Dp, first, i0, pos0, mine, n, x);
     }
@@ -210,24 +238,23 @@ __global__ __launch_bounds__(256, 4) void delta_chunks_prepare_kernel(const Delt
       float* w = to.w + place * NHV_CHUNK * Dp + c;
       float* r = to.r + place * NHV_CHUNK * Dp + c;
       float* k = to.k + (place * Dp + c) * NHV_CHUNK;
-      const float last = ls[(n - 1) * LD + c];
 #pragma unroll
       for (int t = 0; t < NHV_CHUNK; ++t) {
         asm volatile("" ::: "memory");
         w[t * Dp] = x[t];
-        float y = exp2_of(ls[t * LD + c]) * qs[t * LD + c];
+        float y = qs[t * LD + c];
 #pragma unroll
         for (int j = 0; j <= t; ++j) y = fmaf(-B[t][j], x[j], y);
         r[t * Dp] = y;
       }
 #pragma unroll
       for (int t = 0; t < NHV_CHUNK; t += 4) {
-        floatx4 kk;                          // (rows beyond n are zeros, and their logarithms the last one's)
+        floatx4 kk;
 #pragma unroll
-        for (int j = 0; j < 4; ++j) kk[j] = ks[(t + j) * LD + c] * exp2_of(last - ls[(t + j) * LD + c]);
+        for (int j = 0; j < 4; ++j) kk[j] = ls[(t + j) * LD + c].x;
         *reinterpret_cast<floatx4*>(k + t) = kk;
       }
-      to.decay[place * Dp + c] = exp2_of(last);
+      to.decay[place * Dp + c] = exp2_of(last[c].x + last[c].y);
     } else {
       float* v = to.v + (place * E + c - Dp) * NHV_CHUNK;
 #pragma unroll
@@ -242,8 +269,8 @@ extern "C" int nhv_delta_chunks_prepare(const void* proj, int proj_dtype, long l
                                         const void* cu, const void* state_slots, void* w, void* r, void* k, void* v, void* b,
                                         void* decay, int B, int H, int G, int D, int E, int decay_dim, int max_q_len, void* stream) {
   NHV_REQUIRE(B > 0 && H > 0 && G > 0 && D > 0 && E > 0 && H % G == 0, "delta_chunks: bad sizes B=%d H=%d G=%d D=%d E=%d", B, H, G, D, E);
-  NHV_REQUIRE(D <= 256 && B <= 65535 && max_q_len > 0 && max_q_len <= 65535 * NHV_CHUNK, "delta_chunks: D=%d (up to 256), %d requests, portions of %d",
-              D, B, max_q_len);
+  NHV_REQUIRE(D <= 256 && E <= 1024 && B <= 65535 && max_q_len > 0 && max_q_len <= 65535 * NHV_CHUNK,
+              "delta_chunks: D=%d (up to 256), E=%d (up to 1024), %d requests, portions of %d", D, E, B, max_q_len);
   NHV_REQUIRE(decay_dim == D || decay_dim == 1, "delta_chunks: %d decays a head (one, or one per key channel: %d)", decay_dim, D);
   NHV_REQUIRE(n_taps >= 1 && n_taps <= NHV_MAX_TAPS, "delta_chunks: %d taps (1 to %d are taken)", n_taps, NHV_MAX_TAPS);
   NHV_REQUIRE(ld >= 2ll * G * D + (long long)H * E + H && a_ld >= (long long)H * decay_dim, "delta_chunks: rows of %lld and %lld entries", ld, a_ld);
@@ -251,10 +278,16 @@ extern "C" int nhv_delta_chunks_prepare(const void* proj, int proj_dtype, long l
                       (const float*)a_log, (const int*)positions, (const int*)cu, (const int*)state_slots, H, G, D, E, decay_dim};
   const DeltaChunks to = {(float*)w, (float*)r, (float*)k, (float*)v, (float*)b, (float*)decay};
   const int Dp = (D + 15) & ~15;
-  const size_t lds = 3 * (size_t)NHV_CHUNK * (Dp + 4) * sizeof(float);   // (50 KB at most)
+  const size_t lds = 4 * (size_t)NHV_CHUNK * (Dp + 4) * sizeof(float);   // (67 KB at most)
   const dim3 grid(H, (max_q_len + NHV_CHUNK - 1) / NHV_CHUNK, B);
   hipStream_t s = (hipStream_t)stream;
-#define LAUNCH(TI, TAPS) hipLaunchKernelGGL((delta_chunks_prepare_kernel<TI, TAPS>), grid, dim3(256), lds, s, in, to, Dp)
+#define LAUNCH(TI, TAPS)                                                                                                          \
+  do {                                       /* (more than 64 KB of LDS is to be allowed once per kernel) */                        \
+    static const hipError_t allowed = hipFuncSetAttribute((const void*)delta_chunks_prepare_kernel<TI, TAPS>,                        \
+                                                          hipFuncAttributeMaxDynamicSharedMemorySize, 4 * NHV_CHUNK * 260 * 4);      \
+    if (allowed != hipSuccess) return nhv_fail("delta_chunks: %zu bytes of LDS are refused: %s", lds, hipGetErrorString(allowed));   \
+    hipLaunchKernelGGL((delta_chunks_prepare_kernel<TI, TAPS>), grid, dim3(256), lds, s, in, to, Dp);                               \
+  } while (0)
   if (proj_dtype == NHV_F32) {
     if (n_taps == 4) LAUNCH(float, 4);
     else LAUNCH(float, 0);

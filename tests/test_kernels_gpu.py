@@ -1162,3 +1162,49 @@ def test_delta_rule_sixteen_tokens_at_a_time(ops, H, G, D, E, taps, per_head, pa
         want = (plain.unit_rms(torch.stack(want), 1e-5) * norm * torch.sigmoid(gates[i].double()).view(n, H, E)).reshape(n, H * E)
         torch.testing.assert_close(torch.cat(got[i]).double(), want, rtol=1e-2, atol=2e-3)
     assert state[0].isnan().all()                          # a slot that no request holds is left alone
+
+
+def _delta_rule_once(ops, proj, a_lin, gates, tap, dt_bias, a_log, norm, H, G, D, E, per_head):
+    """One portion of one request from the start: (result in bfloat16, state)."""
+    from nanohybrid_vlm_amd.native.ops import AttentionBatch
+    n = len(proj)
+    ints = lambda *v: torch.tensor(v, dtype=torch.int32).cuda()
+    batch = AttentionBatch(num_tokens=n, num_requests=1, token_req=torch.zeros(n, dtype=torch.int32).cuda(), positions=ints(*range(n)),
+                           cu_seqlens_q=ints(0, n), context_lens=ints(n), max_q_len=n, max_context_len=n)
+    kept, state = torch.zeros(1, 2 * G * D + H * E, tap.shape[1] - 1).cuda(), torch.zeros(1, H, E, D).cuda()
+    y = ops.gated_delta_rule(proj.cuda(), a_lin.cuda(), gates.cuda(), tap.cuda(), dt_bias.cuda(), a_log.cuda(), norm.cuda(), 1e-5, kept, state,
+                             batch, ints(0), H, G, D, E, torch.bfloat16, decay_per_head=per_head)
+    return y.cpu(), state[0].cpu()
+
+
+@pytest.mark.parametrize("per_head", [False, True])
+@pytest.mark.parametrize("rate,strong", [(0.6, 1.0), (4.0, 60.0), (16.0, 300.0), (0.6, float("inf")), (3e38, 5.0), (16.0, 3.0)])
+@pytest.mark.parametrize("D", [64, 256])
+def test_delta_rule_after_strong_decays(ops, D, rate, strong, per_head):
+    """Weak decays after strong and infinite ones, within sixteen tokens: the state is as far from float64 as sixteen products of decays
+    rounded to 2^-24 each (1e-6 of its largest entry; token by token 1e-7), not as the rounding of a sum of logarithms that a
+    strong decay has made large, and a decay of zero leaves zeros."""
+    import plain_pevazen as plain
+    g = torch.Generator().manual_seed(73)
+    H, G, E, n, taps = 2, 1, 32, 41, 4
+    C, Dd = 2 * G * D + H * E, 1 if per_head else D
+    proj, gates = torch.randn(n, C + H, generator=g), torch.randn(n, H * E, generator=g)
+    a_lin = torch.randn(n, H * Dd, generator=g) - (0.0 if rate < 1 else 8.0 if rate < 100 else 200.0)
+    for t in (2, 3, 4, 20, 37):
+        a_lin[t] = strong
+    tap, dt_bias, norm = 0.6 * torch.randn(C, taps, generator=g), 0.1 * torch.randn(H * Dd, generator=g), torch.ones(E)
+    a_log = torch.full((H,), rate).log()
+    y, state = _delta_rule_once(ops, proj, a_lin, gates, tap, dt_bias, a_log, norm, H, G, D, E, per_head)
+    act = plain.silu(plain.causal_taps(proj[:, :C].double(), tap.double()))
+    unit = lambda t: t / torch.sqrt(t.pow(2).sum(-1, keepdim=True) + 1e-6)
+    k = unit(act[:, G * D:2 * G * D].view(n, G, D)).repeat_interleave(H // G, dim=1)
+    v, beta = act[:, 2 * G * D:].view(n, H, E), torch.sigmoid(proj[:, C:].double())
+    z = (a_lin + dt_bias).double()
+    decay = torch.exp(-a_log.double().exp()[None, :, None] * torch.logaddexp(z, torch.zeros_like(z)).view(n, H, Dd)).expand(n, H, D)
+    S = torch.zeros(H, D, E, dtype=torch.float64)
+    for t in range(n):
+        S = decay[t][..., None] * S
+        S = S + k[t][..., None] * (beta[t][:, None] * (v[t] - torch.einsum("hde,hd->he", S, k[t])))[:, None]
+    off = (state.transpose(1, 2).double() - S).abs().max() / S.abs().max()
+    assert off < 1e-6, off
+    assert torch.isfinite(y).all()
