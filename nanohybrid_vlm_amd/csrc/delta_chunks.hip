@@ -13,7 +13,8 @@
 // after an infinite one. Token by token and with both parts 1e-7.)
 // Two kernels:
 //  - nhv_delta_chunks_prepare: all chunks at once, a block per (chunk, head, request), from the projection's rows to W, R - B W,
-//    K, V', B and the chunk's decay: convolutions, SiLU, unit vectors, decays, products and the solution without a trip to
+//    K, V', B V' and the chunk's decay (a token's sum of B V' takes the tokens up to it and no others: as a product of whole
+//    matrices an infinite value would come back to the tokens before it as 0 times infinity): convolutions, SiLU, unit vectors, decays, products and the solution without a trip to
 //    memory between them (the rows are read once and a fifth over; the separate kernel that wrote q, k, v, beta and decays
 //    took 101 us for 2,201 tokens of 16 heads of 128);
 //  - nhv_delta_chunks: a request's chunks in order, as float matrix products (v_mfma_f32_16x16x4_f32).
@@ -52,7 +53,7 @@ struct DeltaChunks {                         // per (place, head); a chunk's pla
   float *w, *r;                              // [16][Dp]
   float *k;                                  // [Dp][16]
   float *v;                                  // [E][16]
-  float *b;                                  // [16][16], zeros above the diagonal
+  float *o;                                  // [E][16]: B V'
   float *decay;                              // [Dp]
 };
 
@@ -198,7 +199,6 @@ __global__ __launch_bounds__(256, 4) void delta_chunks_prepare_kernel(const Delt
     if ((tid & 1) == 0) {
       A[t][j] = beta[t] * a;
       B[t][j] = b;
-      B[j][t] = 0.f;
     }
   } else {
     const int t = tid - 240;
@@ -257,16 +257,28 @@ __global__ __launch_bounds__(256, 4) void delta_chunks_prepare_kernel(const Delt
       to.decay[place * Dp + c] = exp2_of(last[c].x + last[c].y);
     } else {
       float* v = to.v + (place * E + c - Dp) * NHV_CHUNK;
+      float* o = to.o + (place * E + c - Dp) * NHV_CHUNK;
+#pragma unroll
+      for (int t = 0; t < NHV_CHUNK; t += 4) {
+        floatx4 y;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          asm volatile("" ::: "memory");
+          y[i] = 0.f;
+#pragma unroll
+          for (int j = 0; j <= t + i; ++j) y[i] = fmaf(B[t + i][j], x[j], y[i]);
+        }
+        *reinterpret_cast<floatx4*>(o + t) = y;
+      }
 #pragma unroll
       for (int t = 0; t < NHV_CHUNK; t += 4) *reinterpret_cast<floatx4*>(v + t) = floatx4{x[t], x[t + 1], x[t + 2], x[t + 3]};
     }
   }
-  to.b[place * 256 + tid] = B[tid >> 4][tid & 15];
 }
 
 extern "C" int nhv_delta_chunks_prepare(const void* proj, int proj_dtype, long long ld, const void* taps, int n_taps, const void* kept,
                                         const void* a_lin, long long a_ld, const void* dt_bias, const void* a_log, const void* positions,
-                                        const void* cu, const void* state_slots, void* w, void* r, void* k, void* v, void* b,
+                                        const void* cu, const void* state_slots, void* w, void* r, void* k, void* v, void* o,
                                         void* decay, int B, int H, int G, int D, int E, int decay_dim, int max_q_len, void* stream) {
   NHV_REQUIRE(B > 0 && H > 0 && G > 0 && D > 0 && E > 0 && H % G == 0, "delta_chunks: bad sizes B=%d H=%d G=%d D=%d E=%d", B, H, G, D, E);
   NHV_REQUIRE(D <= 256 && E <= 1024 && B <= 65535 && max_q_len > 0 && max_q_len <= 65535 * NHV_CHUNK,
@@ -276,7 +288,7 @@ extern "C" int nhv_delta_chunks_prepare(const void* proj, int proj_dtype, long l
   NHV_REQUIRE(ld >= 2ll * G * D + (long long)H * E + H && a_ld >= (long long)H * decay_dim, "delta_chunks: rows of %lld and %lld entries", ld, a_ld);
   const DeltaIn in = {proj, ld, (const float*)taps, n_taps, (const float*)kept, (const float*)a_lin, a_ld, (const float*)dt_bias,
                       (const float*)a_log, (const int*)positions, (const int*)cu, (const int*)state_slots, H, G, D, E, decay_dim};
-  const DeltaChunks to = {(float*)w, (float*)r, (float*)k, (float*)v, (float*)b, (float*)decay};
+  const DeltaChunks to = {(float*)w, (float*)r, (float*)k, (float*)v, (float*)o, (float*)decay};
   const int Dp = (D + 15) & ~15;
   const size_t lds = 4 * (size_t)NHV_CHUNK * (Dp + 4) * sizeof(float);   // (67 KB at most)
   const dim3 grid(H, (max_q_len + NHV_CHUNK - 1) / NHV_CHUNK, B);
@@ -306,13 +318,14 @@ extern "C" int nhv_delta_chunks_prepare(const void* proj, int proj_dtype, long l
 // A block owns 16 columns of S (value channels) of one head of one request; its four waves share D in tiles of 16 rows, TPW
 // tiles a wave, which stay in registers as the result of the matrix cores' products (lane l holds S[16 tile + 4 (l / 16) + i,
 // column l % 16]) and are the right-hand operand of W S and R S as they stand. The waves' shares of W S meet in LDS, one
-// barrier a chunk; every wave adds them up in the waves' order, and what it has then, U, lies in its registers as K^T U and
-// B U need it. The shares of O are added up and written a chunk later, behind that chunk's barrier. What a chunk needs is
+// barrier a chunk; every wave adds them up in the waves' order, and what it has then, U, lies in its registers as K^T U needs
+// it. The shares of O, which begin with a quarter of B V' each, are added up and written a chunk
+// later, behind that chunk's barrier. What a chunk needs is
 // asked for AHEAD chunks before it is used. EVEN: every wave has TPW tiles.
 template <int TPW>
 struct DeltaOperands {
   floatx4 w[TPW], r[TPW], g[TPW], kk[TPW], v;
-  float b;
+  float o;                                   // of token 4 grp + wave
 };
 
 template <int TPW, bool EVEN>
@@ -342,7 +355,7 @@ __global__ __launch_bounds__(256, TPW <= 2 ? 2 : 1) void delta_chunks_kernel(con
   const int chunks = (end - first + NHV_CHUNK - 1) / NHV_CHUNK;
   const size_t place0 = (size_t)(first / NHV_CHUNK) + req;
   const int r_at = col * Dp + tile0 * 16 + grp * 4, k_at = (tile0 * 16 + col) * NHV_CHUNK + grp * 4, g_at = tile0 * 16 + grp * 4;
-  const int b_at = col * 16 + grp * 4 + wave, v_at = e_mine * NHV_CHUNK + grp * 4;
+  const int v_at = e_mine * NHV_CHUNK + grp * 4;
   const int spare = (EVEN ? 0 : tiles) - 1;  // (a wave without a tile reads the last one's and leaves it unused)
   DeltaOperands<TPW> ops[AHEAD];
   auto ask = [&](DeltaOperands<TPW>& x, int c) {
@@ -360,7 +373,7 @@ __global__ __launch_bounds__(256, TPW <= 2 ? 2 : 1) void delta_chunks_kernel(con
       x.kk[i] = *reinterpret_cast<const floatx4*>(kb + (k_at + (i - back) * 16 * NHV_CHUNK));
     }
     x.v = *reinterpret_cast<const floatx4*>(from.v + place * NHV_CHUNK * E + v_at);
-    x.b = from.b[place * 256 + b_at];
+    x.o = from.o[place * NHV_CHUNK * E + v_at + wave];
   };
   const int o_at = (tid >> 4) * H * E + (tid & 15);
   auto emit = [&](int c) {                   // the waves' shares of chunk c added up and written
@@ -372,7 +385,7 @@ __global__ __launch_bounds__(256, TPW <= 2 ? 2 : 1) void delta_chunks_kernel(con
     if (t < end && e < E) ob[o_at] = sum;
   };
   auto step = [&](DeltaOperands<TPW>& x, int c) {
-    floatx4 p = {0.f, 0.f, 0.f, 0.f}, p2 = p, o = p, o2 = p;
+    floatx4 p = {0.f, 0.f, 0.f, 0.f}, p2 = p, o2 = p;
 #pragma unroll
     for (int i = 0; i < TPW; ++i) {
       if (!EVEN && tile0 + i >= tiles) continue;      // (the same for the whole wave)
@@ -382,7 +395,8 @@ __global__ __launch_bounds__(256, TPW <= 2 ? 2 : 1) void delta_chunks_kernel(con
       p2 = __builtin_amdgcn_mfma_f32_16x16x4f32(x.w[i][3], S[i][3], p2, 0, 0, 0);
     }
     *reinterpret_cast<floatx4*>(&share[c & 1][wave][lane * 4]) = p + p2;
-    // (while the shares meet)
+    // (while the shares meet; R holds - B W already: what is left of B U is B V')
+    floatx4 o = {wave == 0 ? x.o : 0.f, wave == 1 ? x.o : 0.f, wave == 2 ? x.o : 0.f, wave == 3 ? x.o : 0.f};
 #pragma unroll
     for (int i = 0; i < TPW; ++i) {
       if (!EVEN && tile0 + i >= tiles) continue;
@@ -408,9 +422,6 @@ __global__ __launch_bounds__(256, TPW <= 2 ? 2 : 1) void delta_chunks_kernel(con
 #pragma unroll
       for (int i = 0; i < TPW; ++i)
         if (EVEN || tile0 + i < tiles) S[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(x.kk[i][j], u[j], S[i], 0, 0, 0);
-    // R holds - B W already: what is left of B U is B V', this wave's share the tokens 4 grp + wave
-    const float v_mine = wave == 0 ? x.v[0] : wave == 1 ? x.v[1] : wave == 2 ? x.v[2] : x.v[3];
-    o2 = __builtin_amdgcn_mfma_f32_16x16x4f32(x.b, v_mine, o2, 0, 0, 0);
     ask(x, c + AHEAD);
     if (c > 0) emit(c - 1);                  // (while the products are under way; written behind the last barrier but one)
 #pragma unroll
@@ -437,12 +448,12 @@ __global__ __launch_bounds__(256, TPW <= 2 ? 2 : 1) void delta_chunks_kernel(con
     }
 }
 
-extern "C" int nhv_delta_chunks(const void* w, const void* r, const void* k, const void* v, const void* b, const void* decay, void* state,
+extern "C" int nhv_delta_chunks(const void* w, const void* r, const void* k, const void* v, const void* o, const void* decay, void* state,
                                 void* out, const void* positions, const void* cu, const void* state_slots, int B, int H, int D, int E,
                                 void* stream) {
   NHV_REQUIRE(B > 0 && H > 0 && D > 0 && E > 0 && D <= 256 && B <= 65535 && (E + 15) / 16 <= 65535, "delta_chunks: bad sizes B=%d H=%d D=%d E=%d",
               B, H, D, E);
-  const DeltaChunks from = {(float*)w, (float*)r, (float*)k, (float*)v, (float*)b, (float*)decay};
+  const DeltaChunks from = {(float*)w, (float*)r, (float*)k, (float*)v, (float*)o, (float*)decay};
   const int Dp = (D + 15) & ~15, tiles = Dp / 16, tpw = (tiles + 3) / 4;
   const dim3 grid(H, (E + 15) / 16, B);
   hipStream_t s = (hipStream_t)stream;

@@ -313,14 +313,14 @@ class NativeBackend:
         w = torch.empty((places, H, C, Dp), dtype=torch.float32, device=proj.device)
         r, k = torch.empty_like(w), torch.empty_like(w)
         v = torch.empty((places, H, E, C), dtype=torch.float32, device=proj.device)
-        b = torch.empty((places, H, C, C), dtype=torch.float32, device=proj.device)
+        o = torch.empty_like(v)
         decay = torch.empty((places, H, Dp), dtype=torch.float32, device=proj.device)
         LL = ctypes.c_longlong
         self._call("nhv_delta_chunks_prepare", _ptr(proj), dtype_code(proj), LL(proj.shape[1]), _ptr(taps), taps.shape[1], _ptr(kept),
                    ctypes.c_void_p(a_lin.data_ptr() + 4 * a_col), LL(a_lin.shape[1]), _ptr(dt_bias), _ptr(a_log), _ptr(batch.positions),
-                   _ptr(batch.cu_seqlens_q), _ptr(state_slots), _ptr(w), _ptr(r), _ptr(k), _ptr(v), _ptr(b), _ptr(decay), B, H, G, D, E,
+                   _ptr(batch.cu_seqlens_q), _ptr(state_slots), _ptr(w), _ptr(r), _ptr(k), _ptr(v), _ptr(o), _ptr(decay), B, H, G, D, E,
                    decay_dim, longest, _stream())
-        self._call("nhv_delta_chunks", _ptr(w), _ptr(r), _ptr(k), _ptr(v), _ptr(b), _ptr(decay), _ptr(state), _ptr(out),
+        self._call("nhv_delta_chunks", _ptr(w), _ptr(r), _ptr(k), _ptr(v), _ptr(o), _ptr(decay), _ptr(state), _ptr(out),
                    _ptr(batch.positions), _ptr(batch.cu_seqlens_q), _ptr(state_slots), B, H, D, E, _stream())
 
     def gated_head_norm(self, o, gate, w, y, eps, gate_col=0, gate_act=0):

@@ -1208,3 +1208,28 @@ def test_delta_rule_after_strong_decays(ops, D, rate, strong, per_head):
     off = (state.transpose(1, 2).double() - S).abs().max() / S.abs().max()
     assert off < 1e-6, off
     assert torch.isfinite(y).all()
+
+
+@pytest.mark.parametrize("per_head", [False, True])
+@pytest.mark.parametrize("D,E", [(64, 32), (20, 5), (112, 128)])
+def test_delta_rule_lets_no_token_reach_the_ones_before_it(ops, D, E, per_head):
+    """A value, a key or a decay that is infinite or no number: the tokens before it, also those of the same sixteen, and the
+    heads that do not read it keep their bits."""
+    g = torch.Generator().manual_seed(79)
+    H, G, n, taps = 2, 2, 53, 3
+    C, Dd = 2 * G * D + H * E, 1 if per_head else D
+    proj, gates, a_lin = torch.randn(n, C + H, generator=g), torch.randn(n, H * E, generator=g), torch.randn(n, H * Dd, generator=g)
+    rest = (gates, 0.6 * torch.randn(C, taps, generator=g), torch.zeros(H * Dd), torch.zeros(H), torch.ones(E), H, G, D, E, per_head)
+    clean, state = _delta_rule_once(ops, proj, a_lin, *rest)
+    assert torch.isfinite(clean).all() and torch.isfinite(state).all()
+    for t, column, value in ((22, 2 * G * D + 1, float("inf")), (37, G * D, float("nan")), (31, 0, float("nan")), (40, C + 0, float("nan")),
+                             (9, None, float("nan"))):
+        p, a = proj.clone(), a_lin.clone()
+        if column is None:
+            a[t, 0] = value
+        else:
+            p[t, column] = value
+        out, left = _delta_rule_once(ops, p, a, *rest)
+        assert torch.equal(out[:t], clean[:t]), (t, column)
+        assert torch.equal(out[:, E:], clean[:, E:]) and torch.equal(left[1], state[1]), (t, column)
+        assert not torch.isfinite(out[t, :E]).all(), (t, column)
