@@ -1673,7 +1673,8 @@ class WKV:
 
 FEW_TOKENS = 4                # up to so many tokens a request, a recurrence is one kernel from projections to gated read-out
 RECURRENCE_KEY_DIM = 256      # the largest key head that the recurrences take
-DELTA_CHUNK_TOKENS = 16       # from portions of so many tokens on, the delta rule takes sixteen tokens at a time
+DELTA_CHUNK_TOKENS = 16       # from portions of so many tokens on, the delta rule takes sixteen tokens at a time,
+DELTA_CHUNK_WORK = 92         # and from so many on, the step's tokens and the longest portion's together
 
 
 def token_shift(h: torch.Tensor, mu: torch.Tensor, kept: torch.Tensor, batch: AttentionBatch, state_slots: torch.Tensor) -> torch.Tensor:
@@ -2111,8 +2112,12 @@ def gated_delta_rule(proj: torch.Tensor, a_lin: torch.Tensor | None, gate_lin: t
     b = backend()
     act = {"gate_act": 1} if gate_activation == "silu" else {}
     # A run in 32 bits takes its tokens one by one whatever the portions, so that its results do not depend on how a prompt is
-    # cut; otherwise portions go sixteen tokens at a time (the sums within sixteen tokens are ordered differently).
-    if y.dtype != torch.float32 and batch.max_q_len >= DELTA_CHUNK_TOKENS and D <= RECURRENCE_KEY_DIM and hasattr(b, "delta_chunks"):
+    # cut; otherwise portions go sixteen tokens at a time (the sums within sixteen tokens are ordered differently), unless there are
+    # so few tokens that two kernels more cost more than the shorter chain saves. 16 heads of 128, a layer, token by token and by
+    # sixteen: one portion of 20 tokens 29 us and 37, of 40 36 and 39, of 48 40 and 39, of 64 47 and 39; two of 32 38 and 38, four of
+    # 16 35 and 39, of 32 49 and 42; 40 beside 16 decoded 67 and 70, beside 32 105 and 99; 16 beside 63 decoded 173 and 150.
+    if (y.dtype != torch.float32 and batch.max_q_len >= DELTA_CHUNK_TOKENS and T + batch.max_q_len >= DELTA_CHUNK_WORK
+            and D <= RECURRENCE_KEY_DIM and hasattr(b, "delta_chunks")):
         b.delta_chunks(proj, taps, kept, proj if packed else a_lin, C + H if packed else 0, dt_bias, a_log, state, o, batch, state_slots,
                        H, G, D, E, Dd)
         b.conv_state_update(proj, kept, n, batch, state_slots, C)

@@ -1104,6 +1104,33 @@ def test_attention_kernels_at_random_sizes(ops, Hq, Hkv, D, page, window, seed):
                                **tol(torch.bfloat16))
 
 
+@pytest.fixture
+def sixteen_at_a_time(ops, monkeypatch):
+    """The delta rule takes sixteen tokens at a time also where there are few tokens in all."""
+    monkeypatch.setattr(ops, "DELTA_CHUNK_WORK", 0)
+
+
+def test_delta_rule_of_few_tokens_goes_token_by_token(ops, monkeypatch):
+    """Which kernels a step's portions take, and that both ways give the same state."""
+    backend, taken = ops.backend(), []
+    chunks = backend.delta_chunks
+    monkeypatch.setattr(backend, "delta_chunks", lambda *a: (taken.append(1), chunks(*a))[1])
+    g = torch.Generator().manual_seed(83)
+    H, G, D, E = 2, 1, 32, 16
+    args = lambda n: (torch.randn(n, 2 * G * D + H * E + H, generator=g), torch.randn(n, H * D, generator=g), torch.randn(n, H * E, generator=g),
+                      torch.randn(2 * G * D + H * E, 4, generator=g), torch.zeros(H * D), torch.zeros(H), torch.ones(E), H, G, D, E, False)
+    for n in (15, 16, 45, 46, 200):
+        del taken[:]
+        inputs = args(n)
+        state = _delta_rule_once(ops, *inputs)[1]
+        assert len(taken) == (n >= 46), n
+        with monkeypatch.context() as m:
+            m.setattr(ops, "DELTA_CHUNK_WORK", 0 if n < 46 else 10 ** 9)
+            torch.testing.assert_close(_delta_rule_once(ops, *inputs)[1], state, rtol=1e-5, atol=2e-6)
+            assert len(taken) == (n >= 16), n
+
+
+@pytest.mark.usefixtures("sixteen_at_a_time")
 @pytest.mark.parametrize("H,G,D,E,taps,per_head,packed,lengths", [
     (2, 1, 16, 16, 4, False, False, [16, 17]), (3, 3, 20, 5, 1, False, False, [40, 1, 31]), (2, 2, 128, 128, 4, False, False, [100]),
     (4, 2, 72, 40, 5, True, True, [15, 33, 2]), (1, 1, 200, 24, 4, False, False, [64, 3]), (2, 1, 256, 100, 3, True, True, [19]),
@@ -1177,6 +1204,7 @@ def _delta_rule_once(ops, proj, a_lin, gates, tap, dt_bias, a_log, norm, H, G, D
     return y.cpu(), state[0].cpu()
 
 
+@pytest.mark.usefixtures("sixteen_at_a_time")
 @pytest.mark.parametrize("per_head", [False, True])
 @pytest.mark.parametrize("rate,strong", [(0.6, 1.0), (4.0, 60.0), (16.0, 300.0), (0.6, float("inf")), (3e38, 5.0), (16.0, 3.0)])
 @pytest.mark.parametrize("D", [64, 256])
@@ -1210,6 +1238,7 @@ def test_delta_rule_after_strong_decays(ops, D, rate, strong, per_head):
     assert torch.isfinite(y).all()
 
 
+@pytest.mark.usefixtures("sixteen_at_a_time")
 @pytest.mark.parametrize("per_head", [False, True])
 @pytest.mark.parametrize("D,E", [(64, 32), (20, 5), (112, 128)])
 def test_delta_rule_lets_no_token_reach_the_ones_before_it(ops, D, E, per_head):
