@@ -168,8 +168,8 @@ __global__ __launch_bounds__(64 * WAVES) void decode_attention_kernel(
 
   bf16x8 ka[KT][DSTEPS], vv[PASSES];
   // All keys and values of a round are asked for before anything is computed (16 KB a wave at head size 128). A key that the
-  // split does not hold is taken for the nearest that it does: its score is masked, so its weight is 0, and no load hangs on
-  // a condition.
+  // split does not hold is taken for the nearest that it does, so that no load hangs on a condition: its score is masked, and
+  // its value is 0 by the time it is used (an infinite one would make its weight of 0 a NaN).
   auto ask = [&](int kb) {
     int base[KT];                                         // where the page of each 16 keys begins, if they lie in one page
     if (page_shift >= 4) {
@@ -202,6 +202,13 @@ __global__ __launch_bounds__(64 * WAVES) void decode_attention_kernel(
       s4[kt] = floatx4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
       for (int s = 0; s < DSTEPS; ++s) s4[kt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ka[kt][s], qb[s], s4[kt], 0, 0, 0);
+    }
+    if (kb < first || kb + RK - 1 > last) {            // (the same for the whole wave)
+#pragma unroll
+      for (int ps = 0; ps < PASSES; ++ps) {
+        const int key = kb + ksub * PASSES + ps;
+        if (key < first || key > last) vv[ps] = zero8();
+      }
     }
     // ---- values into LDS, transposed: row d, columns = keys of the round (the tile is this wave's own, and a wave's
     // accesses to LDS are done in their order)

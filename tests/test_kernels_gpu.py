@@ -585,6 +585,25 @@ def test_decode_attention_bfloat16(ops, Hq, Hkv, D, page, window):
     torch.testing.assert_close(one.float(), out[9:10].float(), rtol=1e-2, atol=1e-2)
 
 
+@pytest.mark.parametrize("Hq,Hkv,D,page,window", [(4, 2, 64, 16, None), (8, 1, 128, 64, 40), (2, 2, 256, 32, None), (3, 1, 48, 7, 700)])
+def test_decode_attention_over_infinite_values(ops, Hq, Hkv, D, page, window):
+    """The last key's value, and the first one's that a window leaves, hold an infinity each: the entry is infinite for the heads
+    that read it, whatever keys beside it in its round are masked, and no other entry changes a bit."""
+    lens = [1, 2, 15, 31, 32, 33, 65, 257, 300, 500, 1000, 1025]
+    q, kc, vc, batch, bt, *_ = _paged_setup(torch.bfloat16, lens, [1] * len(lens), Hq, Hkv, D, page, seed=87, scale=0.4)
+    scale, bad = D ** -0.5, vc.clone()
+    clean = ops.paged_attention(q, kc, vc, batch, bt, scale, window)
+    for r, n in enumerate(lens):
+        lo = max(0, n - window) if window else 0
+        bad[bt[r, (n - 1) // page], (n - 1) % page, Hkv - 1, 3] = float("inf")
+        bad[bt[r, lo // page], lo % page, Hkv - 1, D - 1] = float("-inf")
+    out = ops.paged_attention(q, kc, bad, batch, bt, scale, window)
+    mine = slice(Hq // Hkv * (Hkv - 1), Hq)
+    assert (out[:, mine, 3] == float("inf")).all() and (out[:, mine, D - 1] == float("-inf")).all()
+    out[:, mine, 3], out[:, mine, D - 1] = clean[:, mine, 3], clean[:, mine, D - 1]
+    assert torch.equal(out, clean)
+
+
 @pytest.mark.parametrize("Hq,Hkv,D,page,window", [(8, 2, 128, 256, None), (6, 1, 48, 16, None), (4, 4, 64, 64, 3000)])
 def test_decode_attention_of_few_tokens_over_many_splits(ops, Hq, Hkv, D, page, window):
     """One or two requests of thousands of keys: more than 32 splits of 64 keys, which four waves merge."""
