@@ -488,7 +488,8 @@ __global__ __launch_bounds__(64 * W) void merge_splits_at_once_kernel(const floa
   for (int p = 0; p < MPIECES; ++p) acc[p] = make_float4(0.f, 0.f, 0.f, 0.f);
 #pragma unroll
   for (int i = 0; i < NL; ++i) {
-    const bool reached = mls[i].x != -INFINITY;
+    // (a split all of whose scores are no numbers has a maximum of -inf too, and a sum that is none)
+    const bool reached = mls[i].x != -INFINITY || mls[i].y != 0.f;
     const float wgt = reached ? exp2f(mls[i].x - m_ref) : 0.f;
     l += reached ? mls[i].y * wgt : 0.f;
 #pragma unroll

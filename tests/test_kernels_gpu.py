@@ -721,6 +721,34 @@ def test_merge_of_splits_in_all_its_forms(ops, D, split_len, n_splits, window):
     torch.testing.assert_close(out.double().cpu(), ref, **tol(torch.bfloat16))
 
 
+@pytest.mark.parametrize("D,split_len,n_splits", [(128, 64, 1), (128, 64, 5), (128, 64, 20), (64, 64, 100), (128, 64, 140), (256, 32, 3)])
+@pytest.mark.parametrize("sink", [None, 0.3])
+def test_merge_of_splits_hides_no_score_that_is_no_number(ops, D, split_len, n_splits, sink):
+    """A key that is no number and the only one of its split, in every form of the merge, also beside a sink: the result of what
+    reads it is no number; the other heads keep their bits."""
+    import ctypes
+    from nanohybrid_vlm_amd.native.ops import _ptr, _stream
+    Hq, Hkv, page = 4, 2, 32
+    lens = [n_splits * split_len] + [s * split_len + 1 for s in range(1, n_splits, 3)] + [1, 2]
+    q, kc, vc, batch, bt, *_ = _paged_setup(torch.bfloat16, lens, [1] * len(lens), Hq, Hkv, D, page, seed=64)
+    T, backend = len(lens), ops.backend()
+
+    def call(keys):
+        out = torch.full((T, Hq, D), 7.0, dtype=torch.bfloat16, device="cuda")
+        part_o, part_ml = torch.zeros(T, Hq, n_splits, D, device="cuda"), torch.zeros(T, Hq, n_splits, 2, device="cuda")
+        backend._call("nhv_decode_attention_bf16_more", _ptr(q), _ptr(keys), _ptr(vc), _ptr(out), _ptr(part_o), _ptr(part_ml),
+                      _ptr(batch.token_req), _ptr(batch.positions), _ptr(bt), bt.shape[1], T, Hq, Hkv, page, ctypes.c_float(D ** -0.5), 0,
+                      split_len, n_splits, ctypes.c_float(0.0), int(sink is not None), ctypes.c_float(sink or 0.0), None, None, None,
+                      ctypes.c_longlong(0), _stream(), lib=backend.attention_lib(D))
+        return out
+
+    clean, bad = call(kc), kc.clone()
+    for r, n in enumerate(lens):
+        bad[bt[r, (n - 1) // page], (n - 1) % page, 1, 5] = float("nan")
+    out = call(bad)
+    assert torch.isfinite(clean).all() and torch.equal(out[:, :2], clean[:, :2]) and torch.isnan(out[:, 2:]).all()
+
+
 def test_merge_of_splits_of_many_tokens(ops):
     """More than 1,024 (token, head) pairs with more splits than the at-once kernels take: the looping kernel with
     one wave."""
