@@ -3,7 +3,7 @@
 //
 // A block works on (token, key/value head, up to 16 of the query heads that share it, split of
 // the keys), its waves on rounds of 32 keys in turn. The query heads are the 16 columns of the MFMA tiles (more than 16 heads on one
-// key/value head, as over a cached latent, are several waves that read the same keys):
+// key/value head, as over a cached latent, are several blocks that read the same keys):
 //   S^T[key, head]  = K[key, :] . Q[head, :]        K rows straight from the cache (v_mfma_f32_16x16x32_bf16)
 //   running maximum per head in float (two shuffles), sums kept per lane
 //   O^T[d, head]   += V^T[d, key] . P^T[key, head]   V^T from the wave's own LDS tile, P in registers
@@ -74,7 +74,7 @@ __device__ __forceinline__ int slot_of(const int* bt, int key, int page_size, in
 // for before this one is computed: more than 256 registers, one wave a SIMD, and 2 to 10 % more time.)
 constexpr int WAVES = D <= 128 ? 8 : 4;
 constexpr int TURN = D <= 64 ? 2 : 1;                       // rounds a wave takes before the next wave's: 16 KB and more of keys and values
-constexpr int MOST_SORTED = 64;                             // up to so many tokens the longest contexts are taken first
+constexpr int MOST_SORTED = 64;                             // up to so many tokens a split's longest contexts are taken first
 constexpr int OPITCH = D + 4;                               // floats a head in the waves' meeting place, which lies where a wave's V^T tile was
 constexpr int MEET = 16 * OPITCH * 4 + 16 * 2 * 4;          // bytes: 16 heads' sums, maxima and sums of weights
 constexpr int TILE = D * VPITCH * 2 > MEET ? D * VPITCH * 2 : MEET;
@@ -104,48 +104,56 @@ __global__ __launch_bounds__(64 * WAVES) void decode_attention_kernel(
   // 32 and 64 requests (116 against 111 us at 64) than one whose blocks go over all heads
   int t = blockIdx.y;
   const int split = blockIdx.z;
-  // One split and contexts of different lengths: the blocks that start first take the longest (after 100 to 2,000 keys: 64
-  // requests 68.7 -> 62.7 us, 40 requests 52.5 -> 43.6; for 128 what it costs is what it saves). Every block finds its token
-  // by counting, each wave against its share of the tokens (against all of them in one thread a token: 65 us).
-  if (n_splits == 1 && gridDim.y >= 16 && gridDim.y <= MOST_SORTED) {
-    static_assert(sizeof(int) * (2 * MOST_SORTED + 1) <= sizeof(tiles_s), "the tokens' numbers of keys do not fit the tiles");
+  int pos, req;
+  // Contexts of different lengths: of a split's blocks those that start first take the most keys (64 requests after 100 to 2,000
+  // keys, one split: 68.7 -> 62.7 us; after 100 to 8,000, splits of 2,048: 225 -> 209; 48 after 100 to 16,000 329 -> 317; for 128
+  // requests what it costs is what it saves). Every block finds its token by counting, each wave against its share of the tokens
+  // (against all of them in one thread a token: 65 us for the first of these).
+  if (gridDim.y >= 16 && gridDim.y <= MOST_SORTED) {
+    static_assert(MOST_SORTED <= 64 && sizeof(int) * (2 * MOST_SORTED + 1) <= sizeof(tiles_s), "a wave and the tiles hold the tokens' numbers of keys");
     int *keys_s = reinterpret_cast<int*>(tiles_s), *place_s = keys_s + MOST_SORTED, *chosen = place_s + MOST_SORTED;
-    const int T = gridDim.y, tid = threadIdx.x;
-    for (int i = tid; i < MOST_SORTED; i += 64 * WAVES) {
-      const int p = positions[min(i, T - 1)];
-      keys_s[i] = i < T ? p - nhv_first_key(p, window) : -1;
-      place_s[i] = 0;
-    }
-    __syncthreads();
-    const int share = (T + 4 * WAVES - 1) / (4 * WAVES) * 4, j0 = wave * share;
-    for (int i = lane; i < T; i += 64) {
-      const int keys = keys_s[i];
-      int before = 0;
-      for (int j = j0; j < min(j0 + share, T); j += 4) {
-        const int4 other = *reinterpret_cast<const int4*>(&keys_s[j]);
-        before += (other.x > keys || (other.x == keys && j < i)) + (other.y > keys || (other.y == keys && j + 1 < i)) +
-                  (other.z > keys || (other.z == keys && j + 2 < i)) + (other.w > keys || (other.w == keys && j + 3 < i));
+    const int T = gridDim.y, p = positions[min(lane, T - 1)], r = token_req[min(lane, T - 1)];
+    const int mine = lane < T ? min(p, (split + 1) * split_len - 1) - max(nhv_first_key(p, window), split * split_len) + 1 : 0;
+    if (t >= __popcll(__ballot(mine > 0))) return;     // (fewer tokens have keys here: the same for the whole block)
+    const int one = __shfl(mine, 0, 64);
+    if (__ballot(lane < T && mine != one)) {           // (equal ones are taken as they come: 1.6 us less for 64 requests after 2,048 keys)
+      if (wave == 0) {
+        keys_s[lane] = lane < T ? mine : -0x7fffffff;
+        place_s[lane] = 0;
       }
-      if (before) atomicAdd(&place_s[i], before);
+      __syncthreads();
+      const int share = (T + 4 * WAVES - 1) / (4 * WAVES) * 4, j0 = wave * share;
+      if (lane < T) {
+        int before = 0;
+        for (int j = j0; j < min(j0 + share, T); j += 4) {
+          const int4 other = *reinterpret_cast<const int4*>(&keys_s[j]);
+          before += (other.x > mine || (other.x == mine && j < lane)) + (other.y > mine || (other.y == mine && j + 1 < lane)) +
+                    (other.z > mine || (other.z == mine && j + 2 < lane)) + (other.w > mine || (other.w == mine && j + 3 < lane));
+        }
+        if (before) atomicAdd(&place_s[lane], before);
+      }
+      __syncthreads();
+      if (wave == 0 && lane < T && place_s[lane] == t) *chosen = lane;
+      __syncthreads();
+      t = *chosen;
+      __syncthreads();
     }
-    __syncthreads();
-    for (int i = tid; i < T; i += 64 * WAVES)
-      if (place_s[i] == t) *chosen = i;
-    __syncthreads();
-    t = *chosen;
-    __syncthreads();
+    pos = __shfl(p, t, 64);
+    req = __shfl(r, t, 64);
+  } else {
+    pos = positions[t];
+    req = token_req[t];
   }
   const int group = (int)((blockIdx.x + blockIdx.y + blockIdx.z) % gridDim.x);
   const int per_kv = (int)gridDim.x / Hkv;         // groups of up to 16 query heads on one key/value head
   const int kvh = group / per_kv;
   const int head0 = kvh * (Hq / Hkv) + (group % per_kv) * 16;                  // this block's query heads: head0 + (0 .. G - 1)
   const int G = min(16, Hq / Hkv - (group % per_kv) * 16);
-  const int pos = positions[t];
   const int lo = nhv_first_key(pos, window);
   const int first = max(lo, split * split_len);
   const int last = min(pos, (split + 1) * split_len - 1);
   if (first > last) return;              // this split holds no visible key; the merge knows from pos and lo
-  const int* bt = block_tables + (size_t)token_req[t] * max_blocks;
+  const int* bt = block_tables + (size_t)req * max_blocks;
   const int col = lane & 15, grp = lane >> 4;
 
   // Q^T operand: lane holds 8 entries of head `col`

@@ -101,6 +101,42 @@ def _gate_args(gate):
     return ctypes.c_void_p(t.data_ptr() + col * t.element_size()), ctypes.c_longlong(t.shape[1])
 
 
+MOST_KEYS_A_SPLIT = 2048
+
+
+def decode_split_length(blocks: int, span: int, covered: int, window: int) -> int:
+    """Keys a split of the decode attention. ``blocks``: blocks a split (a block takes up to 16 heads of a key/value head of one
+    token); ``span``: the most keys that a token reads now; ``covered``: the longest context that the launch can meet; ``window``:
+    0 for none, a chunk as a negative one. (What is measured here: 8 key/value heads of 128, 4 query heads each, in a recorded
+    graph, which covers contexts half as long again as the longest.)"""
+    # A block of eight waves takes 256 keys in the time of 32. One split where the blocks fill the chip anyway (all of 2,176
+    # keys: 24 requests 45.9 us, with splits of 1,024 53.6; 32 requests 57 and 64; 64 requests 110 and 123) or where its rounds are
+    # over before a merge would be (one request of 16 heads, 150 keys: 6.2 us, two splits of 128 8.3; eight of 300 keys 8.4 against
+    # 9.9; one of 1,000 14.4 against 9.4). Else one block a compute unit, splits of at least 128 keys and not many more than 32
+    # of them, which is what the merge takes at once (8 x 2,050 keys: 21 us with splits of 512, 24 with 256; 1 x 32,000: 32.4
+    # with 1,280, 38.8 with 384).
+    # One split ends where one long context alone could be what the step lasts, 14 us for each 1,000 keys (24 requests of 200 keys
+    # and one of 32,000: 53 us with splits of 2,048, 449 with one split; 63 of 1,000 and one of 8,192 91 and 137), although equal ones
+    # lose a little by it (64 x 8,192: 400 and 393; 64 x 4,096 204 and 198, which many blocks are spared). What one split costs
+    # below that: 31 requests of 200 keys and one of 2,700 45 us, with splits of 768 27.
+    # A little over one block a unit is the exception: most units would wait for the few that have two. Three splits there, two
+    # up to 416 blocks (all of 2,176 keys: 40 requests 81 us, with one split 92; 48 requests 91 and 95; of 100 to 2,000 keys
+    # 43 and 42, 52 and 46).
+    most = min(covered, abs(window) + 64) if window else covered       # keys that a token can come to read
+    if span <= 448 or (blocks >= 192 and most <= (4096 if blocks <= 256 else 6144) and (blocks > 416 or blocks <= 256 or window)):
+        return -(-covered // 32) * 32
+    if 256 < blocks <= 416 and not window:
+        split_len = 128 * -(-span // (128 * (3 if blocks <= 352 else 2)))
+    else:
+        split_len = max(128, 128 * round(max(span * blocks / 256, most / 36) / 128))
+    split_len = min(split_len, MOST_KEYS_A_SPLIT)
+    if window and most <= MOST_KEYS_A_SPLIT:
+        # a window lies in few of its context's splits, the others are empty blocks (8 requests with a window of 1,024 after 32,000
+        # keys: 21.3 us with splits of 768, 24.7 with 384; one request 11.2 with 128, 17 with 1,024)
+        split_len = max(split_len, 128 * -(-covered * blocks // (128 * 4096)))
+    return split_len
+
+
 class NativeBackend:
     """ctypes calls into the HIP library."""
 
@@ -531,25 +567,12 @@ class NativeBackend:
         covered = batch.max_context_len
         if self.planned_context and self.covered_context:
             covered = min(covered, self.covered_context)
-        # A block of eight waves takes 256 keys in the time of 32. One split where the blocks fill the chip anyway (24 to 32 and
-        # 56 to 128 requests of 8 key/value heads: no split faster) or where its rounds are over before a merge would be (one request of
-        # 16 heads, 150 keys: 6.2 us, two splits of 128 8.3; eight of 300 keys 8.4 against 9.9; one of 1,000 14.4 against
-        # 9.4). Else one block a compute unit, splits of at least 128 keys and not many more than 32 of them, which is what
-        # the merge takes at once (8 x 2,050 keys: 21.3 us with splits of 512, 23.7 with 384 or 256; 8 x 4,000: 31.5 with
-        # 1,024, 36.6 with 256; 1 x 9,000: 15.4 with 384, 19.5 with 256).
-        # A little over one block a unit is the exception: most units would wait for the few that have two. Three splits there, two
-        # up to 416 blocks (8 heads, all of 2,176 keys: 40 requests 75 us against 88, 48 requests 85 against 92; of 100 to 2,000
-        # keys, where the longest go first, 42.2 against 40.9 and 52 against 44).
-        blocks = T * Hkv * -(-(Hq // Hkv) // 16)            # (a block takes up to 16 heads of a key/value head)
-        if 256 < blocks <= 416 and span > 448:
-            split_len = 128 * -(-span // (128 * (3 if blocks <= 352 else 2)))
-        elif blocks >= 192 or span <= 448:
-            split_len = -(-covered // 32) * 32
-        else:
-            split_len = max(128, 128 * round(max(span * blocks / 256, covered / 36) / 128))
+        split_len = decode_split_length(T * Hkv * -(-(Hq // Hkv) // 16), span, covered, window)
         n_splits = -(-covered // split_len)
-        part_o = torch.empty((T, Hq, n_splits, D), dtype=torch.float32, device=q.device)
-        part_ml = torch.empty((T, Hq, n_splits, 2), dtype=torch.float32, device=q.device)
+        part_o = part_ml = None                             # (one split: the kernel writes the result itself)
+        if n_splits > 1:
+            part_o = torch.empty((T, Hq, n_splits, D), dtype=torch.float32, device=q.device)
+            part_ml = torch.empty((T, Hq, n_splits, 2), dtype=torch.float32, device=q.device)
         self._call("nhv_decode_attention_bf16" + ("_more" if more else ""), _ptr(q), _ptr(k_cache), _ptr(v_cache), _ptr(out),
                    _ptr(part_o), _ptr(part_ml), _ptr(batch.token_req), _ptr(batch.positions), _ptr(block_tables),
                    block_tables.shape[1], T, Hq, Hkv, page_size, ctypes.c_float(scale), window, split_len, n_splits,

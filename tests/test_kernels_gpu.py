@@ -606,7 +606,7 @@ def test_decode_attention_over_infinite_values(ops, Hq, Hkv, D, page, window):
 
 @pytest.mark.parametrize("Hq,Hkv,D,page,window", [(8, 2, 128, 256, None), (6, 1, 48, 16, None), (4, 4, 64, 64, 3000)])
 def test_decode_attention_of_few_tokens_over_many_splits(ops, Hq, Hkv, D, page, window):
-    """One or two requests of thousands of keys: more than 32 splits of 64 keys, which four waves merge."""
+    """One or two requests of thousands of keys: the splits that the engine chooses, which four waves merge."""
     for lens in ([5000], [4097, 2100]):
         q_lens = [1] * len(lens)
         scale = D ** -0.5
@@ -749,6 +749,71 @@ def test_merge_of_splits_hides_no_score_that_is_no_number(ops, D, split_len, n_s
     assert torch.isfinite(clean).all() and torch.equal(out[:, :2], clean[:, :2]) and torch.isnan(out[:, 2:]).all()
 
 
+def _decode_in_splits(ops, q, kc, vc, batch, bt, scale, window, split_len, n_splits, cap=0.0, sink=None, sinks=None, slopes=None, gate=None):
+    """The decode kernel with the splits named; the buffers of the splits' results are full of NaN beforehand."""
+    import ctypes
+    from nanohybrid_vlm_amd.native.ops import _gate_args, _ptr, _stream
+    T, Hq, D = q.shape
+    out = torch.full((T, Hq, D), float("nan"), dtype=torch.bfloat16, device="cuda")
+    part_o = torch.full((T, Hq, n_splits, D), float("nan"), device="cuda")
+    part_ml = torch.full((T, Hq, n_splits, 2), float("nan"), device="cuda")
+    ops.backend()._call("nhv_decode_attention_bf16_more", _ptr(q), _ptr(kc), _ptr(vc), _ptr(out), _ptr(part_o), _ptr(part_ml), _ptr(batch.token_req),
+                        _ptr(batch.positions), _ptr(bt), bt.shape[1], T, Hq, kc.shape[2], kc.shape[1], ctypes.c_float(scale), window, split_len, n_splits,
+                        ctypes.c_float(cap), int(sink is not None), ctypes.c_float(sink or 0.0), _ptr(sinks), _ptr(slopes), *_gate_args(gate), _stream(),
+                        lib=ops.backend().attention_lib(D))
+    return out
+
+
+@pytest.mark.parametrize("options", ["cap", "sink", "sinks", "slopes", "gate", "cap sinks gate", "slopes sink gate", "cap slopes"])
+@pytest.mark.parametrize("D,split_len,n_splits,window", [(64, 640, 1, 0), (128, 128, 5, 0), (64, 64, 20, 900), (128, 64, 100, 0), (128, 64, 140, 0)])
+def test_options_of_decoded_tokens_over_splits(ops, options, D, split_len, n_splits, window):
+    """What a layer may ask for besides, where one block writes the result and in every form of the merge."""
+    Hq, Hkv = 6, 2
+    longest = n_splits * split_len
+    lens = [longest, 1, split_len, min(longest, split_len + 1), longest // 2 + 3]
+    q, kc, vc, batch, bt, ks, vs, qs = _paged_setup(torch.bfloat16, lens, [1] * len(lens), Hq, Hkv, D, 64, seed=65, scale=1.2)
+    given, scale, T = set(options.split()), D ** -0.5, len(lens)
+    rows = rnd(T, Hq + 3, dtype=torch.bfloat16, seed=66)
+    args = {"cap": 3.0, "sink": 0.7, "sinks": rnd(Hq, seed=67), "slopes": rnd(Hq, seed=68).abs() * 0.02, "gate": (rows, 2)}
+    args = {name: value for name, value in args.items() if name in given}
+    out = _decode_in_splits(ops, q, kc, vc, batch, bt, scale, window, split_len, n_splits, **args)
+    heads = torch.arange(Hq) // (Hq // Hkv)
+    for t, n in enumerate(lens):
+        keys = torch.arange(max(0, n - window) if window else 0, n)
+        s = torch.einsum("hd,khd->hk", qs[t][0].double(), ks[t].double()[keys][:, heads]) * scale
+        if "cap" in given:
+            s = 3.0 * torch.tanh(s / 3.0)
+        if "slopes" in given:
+            s = s - args["slopes"].double().cpu()[:, None] * (n - 1 - keys)[None]
+        more = torch.full((Hq, 1), 0.7, dtype=torch.float64) if "sink" in given else args["sinks"].double().cpu()[:, None] if "sinks" in given else None
+        p = torch.softmax(s if more is None else torch.cat([s, more], dim=1), dim=1)[:, :len(keys)]
+        want = torch.einsum("hk,khd->hd", p, vs[t].double()[keys][:, heads])
+        if "gate" in given:
+            want = want * torch.sigmoid(rows[t, 2:2 + Hq].double().cpu())[:, None]
+        torch.testing.assert_close(out[t].double().cpu(), want, **tol(torch.bfloat16))
+
+
+@pytest.mark.parametrize("T,D,split_len,n_splits,window", [(16, 64, 128, 5, 0), (17, 256, 64, 4, 0), (33, 128, 32, 9, 70), (63, 64, 96, 3, -50), (64, 128, 64, 6, 0),
+                                                           (64, 48, 224, 2, 0), (65, 64, 96, 3, 0), (15, 64, 96, 3, 0)])
+def test_decoded_tokens_in_any_order_over_splits(ops, T, D, split_len, n_splits, window):
+    """Of each split's blocks the ones with the most keys come first, from 16 to 64 tokens, and tokens without a key there have none:
+    every (token, split) is done once, in whatever order the contexts come, and a token's bits are those it has alone."""
+    g = torch.Generator().manual_seed(85)
+    longest = split_len * n_splits
+    lens = [longest, 1, split_len, split_len + 1, longest - 1] + torch.randint(1, longest + 1, (T - 5,), generator=g).tolist()
+    lens = [lens[i] for i in torch.randperm(T, generator=g).tolist()]
+    scale = D ** -0.5
+    q, kc, vc, batch, bt, ks, vs, qs = _paged_setup(torch.bfloat16, lens, [1] * T, 2, 1, D, 16, seed=86)
+    out = _decode_in_splits(ops, q, kc, vc, batch, bt, scale, window, split_len, n_splits)
+    if window >= 0:
+        torch.testing.assert_close(out.double().cpu(), _attention_reference(qs, ks, vs, lens, [1] * T, scale, window), **tol(torch.bfloat16))
+    for t in range(0, T, 5):
+        alone = type(batch)(1, 1, torch.zeros(1, dtype=torch.int32).cuda(), batch.positions[t:t + 1].contiguous(), torch.tensor([0, 1], dtype=torch.int32).cuda(),
+                            batch.context_lens[t:t + 1].contiguous(), 1, lens[t])
+        one = _decode_in_splits(ops, q[t:t + 1].contiguous(), kc, vc, alone, bt[t:t + 1].contiguous(), scale, window, split_len, n_splits)
+        assert torch.equal(one[0], out[t]), t
+
+
 def test_merge_of_splits_of_many_tokens(ops):
     """More than 1,024 (token, head) pairs with more splits than the at-once kernels take: the looping kernel with
     one wave."""
@@ -816,7 +881,7 @@ def test_prefill_attention_scores_that_outgrow_their_reference(ops, far):
 
 @pytest.mark.parametrize("window", [None, 5000])
 def test_attention_over_32768_keys(ops, window):
-    """Both bfloat16 attention kernels at 32,768 keys on pages of 256 (128 pages a request, hundreds of splits to
+    """Both bfloat16 attention kernels at 32,768 keys on pages of 256 (128 pages a request, the engine's splits to
     merge, block tables past what a block keeps in LDS at smaller pages), against the float64 computation: a single
     token at the end of 32,768 keys beside one after 9,001; and portions of 130 and 64 tokens that end at 32,768
     and 20,000 keys. In every request one early key is made to stand out for one head's queries, so that a key lost

@@ -89,3 +89,20 @@ def test_the_wait_for_x_has_the_loads_behind_it_that_it_counts(tmp_path):
         assert not any(op.startswith(("scratch", "buffer", "flat", "global_store")) for op in between), m[1]
         seen += 1
     assert seen >= 50, seen
+
+
+@pytest.mark.parametrize("blocks", [1, 8, 64, 184, 192, 200, 256, 264, 320, 352, 360, 416, 424, 512, 1024, 4096])
+def test_no_block_of_the_decode_attention_takes_a_long_context_alone(blocks):
+    """However long the longest context and however many blocks there are: the splits cover it, and no block's chain of keys is longer
+    than 2,048, or 6,144 where the whole context is one split. A window's tokens are split by what they read."""
+    from nanohybrid_vlm_amd.native.ops import decode_split_length
+    for covered in (1, 31, 300, 448, 449, 672, 1000, 2048, 3072, 4096, 4097, 6144, 6145, 12288, 48000, 196608, 1000000):
+        for span in {covered, max(1, covered * 2 // 3)}:
+            for window in (0, 100, 1024, -1024, 8192):
+                seen = min(span, abs(window) + 64) if window else span
+                split = decode_split_length(blocks, seen, covered, window)
+                n = -(-covered // split)
+                assert split > 0 and split % 32 == 0 and n <= 65535
+                read = min(covered, abs(window) + 64) if window else covered
+                assert min(split, read) <= (2048 if n > 1 else 6144), (covered, span, window, split)
+    assert decode_split_length(8, 1088, 48000, 1024) <= 256        # (one token of 8 key/value heads deep in a context)
