@@ -890,11 +890,17 @@ static TilesPlan tiles_plan(bool glu, bool squares, bool biased, int M, int N, i
   const size_t sums = (size_t)(tiles > 1 ? 2 : 1) * TW * (glu ? 2 : 1) * 64 * sizeof(floatx4), x_bytes = (size_t)M * (K + 8) * 2;
   const size_t biases = tiles > 1 && biased ? ((glu ? 2 : 1) * p.rows + 16) * sizeof(float) : 0;
   p.x_in_lds = sums + x_bytes + biases <= LDS_BYTES;
-  // The kernels below it is where a product of several tiles a block has a residual (or more biases than threads), and where x does not fit into LDS,
+  // The kernels below it is where a product of several tiles a block has more biases than threads, and where x does not fit into LDS,
   // but for up to 8 rows on the whole chip (4,096 outputs of 12,288 columns at 8 rows 25.2 against 26.8 us; 3,584 of 18,944 on
   // 224 units, where x beside w is too much for a unit, 36.4 against 33.9; 4,096 of 12,288 at 16 rows 31.4 against 30.7).
-  if (tiles > 1 && (squares || biases > (64 * TW + 16) * sizeof(float))) return p;
+  if (tiles > 1 && biases > (64 * TW + 16) * sizeof(float)) return p;
   if (!p.x_in_lds && (glu || tiles > 1 || M > 8 || N <= 240 * p.rows)) return p;
+  // With a residual and more than 4,096 outputs a unit has a block or two. These kernels are the faster ones then too (5,120 outputs of 5,120
+  // columns at 1 and 8 rows 17.3 against 19.8 us and 21.1 against 24.3; 5,120 of 17,408 at 4 rows 49.9 against 54.7; 8,192 of
+  // 28,672 at 1 row 91.7 against 93.8), except where x does not fit into LDS (5,120 of 17,408 at 8 rows 65.0 against 58.6; of 25,600
+  // 95.2 against 79.5; the only ones slower below it: 12,288 at 6 rows, 42.5 against 44.5) and for one row of many columns
+  // that some units take twice (5,120 of 20,480 57.4 against 56.7, of 22,528 62.3 against 58.4, of 25,600 72.2 against 66.2).
+  if (squares && N > 256 * p.rows && (!p.x_in_lds || (M == 1 && K > 20480 && N < 512 * p.rows))) return p;
   p.lds = sums + (p.x_in_lds ? x_bytes + biases : 0);
   const int steps = ((K + 31) / 32 + 15) / 16;
   int slots = 1 << 30;

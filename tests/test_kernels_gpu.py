@@ -232,6 +232,8 @@ def test_few_rows_linear_bfloat16_in_all_its_variants(ops, M, N, K):
     (1, 4100, 264), (7, 6144, 3584), (16, 8200, 2560), (4, 9732, 1544), (3, 20484, 72),
     # x beside w, and just not (LDS)
     (8, 4096, 12288), (6, 3076, 16392), (4, 4092, 18440),
+    # a residual of more than 256 tiles: x beside w in LDS and not, and one row of many columns
+    (4, 5136, 4104), (8, 4112, 17416), (1, 4100, 20488),
 ])
 def test_tiles_of_few_rows_products(ops, M, N, K):
     """Plain, activated, gated, with rows that lack their scales and added to a residual (bounds: float32 sums of K products of
