@@ -250,9 +250,12 @@ class NativeBackend:
                               _ptr(out), _ptr(batch.cu_seqlens_q), _ptr(batch.context_lens), _ptr(block_tables),
                               block_tables.shape[1], batch.num_requests, batch.max_q_len, Hq, Hkv, page_size,
                               ctypes.c_float(scale), window, *more, _stream(), lib=self.attention_lib(D))
-        # 32 bits: by the head sizes alone, so that one model's positions are always computed by one kernel
+        # 32 bits: by the head sizes, so that one model's positions are always computed by one kernel (it sums keys in blocks of 32,
+        # the other one in blocks of 64). Rows that begin off 16 bytes are copied; caches that do, or more than 65,535
+        # requests or key heads, are the other kernel's.
         if (q.dtype == torch.float32 and D % 16 == 0 and D <= 256 and E % 64 == 0 and E <= 256 and batch.num_requests <= 65535
-                and Hkv <= 65535 and all(t.data_ptr() % 16 == 0 for t in (q, k_cache, v_cache))):
+                and Hkv <= 65535 and k_cache.data_ptr() % 16 == 0 and v_cache.data_ptr() % 16 == 0):
+            q = q if q.data_ptr() % 16 == 0 else q.clone()
             return self._call("nhv_attention_float32", _ptr(q), _ptr(k_cache), _ptr(v_cache), _ptr(out), _ptr(batch.positions),
                               _ptr(batch.cu_seqlens_q), _ptr(block_tables), block_tables.shape[1], batch.num_requests, batch.max_q_len,
                               Hq, Hkv, D, E, page_size, ctypes.c_float(scale), 0 if chunk else window, chunk, *options, _stream())

@@ -565,6 +565,16 @@ def test_attention_hides_no_score_that_is_no_number(ops, dtype, D, sink):
     assert torch.isnan(out[hit]).all() and torch.equal(out[~hit], clean[~hit])
 
 
+def test_float32_attention_of_rows_that_begin_anywhere(ops):
+    """Queries that begin 4, 8 and 12 bytes off a boundary of 16: the bits of those that begin on one."""
+    lens, q_lens = [33, 257, 70], [33, 1, 20]
+    q, kc, vc, batch, bt, *_ = _paged_setup(torch.float32, lens, q_lens, 4, 2, 64, 16, seed=88)
+    want = ops.paged_attention(q, kc, vc, batch, bt, 0.125)
+    for off in (1, 2, 3):
+        rows = torch.empty(q.numel() + off, device="cuda")[off:].view_as(q).copy_(q)
+        assert rows.data_ptr() % 16 == 4 * off and torch.equal(ops.paged_attention(rows, kc, vc, batch, bt, 0.125), want)
+
+
 @pytest.mark.parametrize("Hq,Hkv,D,page,window", [
     (4, 2, 16, 4, None), (6, 1, 32, 8, None), (5, 5, 48, 7, None), (3, 1, 80, 16, 9), (8, 2, 128, 64, None),
     (32, 8, 128, 256, None), (16, 1, 64, 5, 70), (7, 7, 112, 3, None), (2, 1, 256, 32, None), (12, 2, 96, 16, 300),
