@@ -112,23 +112,23 @@ def decode_split_length(blocks: int, span: int, covered: int, window: int) -> in
     # A block of eight waves takes 256 keys in the time of 32. One split where the blocks fill the chip anyway (all of 2,176
     # keys: 24 requests 45.9 us, with splits of 1,024 53.6; 32 requests 57 and 64; 64 requests 110 and 123) or where its rounds are
     # over before a merge would be (one request of 16 heads, 150 keys: 6.2 us, two splits of 128 8.3; eight of 300 keys 8.4 against
-    # 9.9; one of 1,000 14.4 against 9.4). Else one block a compute unit, splits of at least 128 keys and not many more than 32
-    # of them, which is what the merge takes at once (8 x 2,050 keys: 21 us with splits of 512, 24 with 256; 1 x 32,000: 32.4
-    # with 1,280, 38.8 with 384).
+    # 9.9; one of 1,000 14.4 against 9.4). Else at most about one block a compute unit, in splits of a multiple of 128 keys, rounded
+    # up (steps of 12 layers, all of 2,176 keys: 12 requests 1,684 us with splits of 896, 1,766 with 768; 4 requests 1,438 with 384, 1,474
+    # with 256; 2 requests 1,386 with 256, 1,413 with 128; 8 requests 1,576 with 640, 1,600 with 512), and not many more than 32 of them,
+    # which is what the merge takes at once (1 x 32,000: 32.4 us with 1,280, 38.8 with 384).
     # One split ends where one long context alone could be what the step lasts, 14 us for each 1,000 keys (24 requests of 200 keys
     # and one of 32,000: 53 us with splits of 2,048, 449 with one split; 63 of 1,000 and one of 8,192 91 and 137), although equal ones
     # lose a little by it (64 x 8,192: 400 and 393; 64 x 4,096 204 and 198, which many blocks are spared). What one split costs
     # below that: 31 requests of 200 keys and one of 2,700 45 us, with splits of 768 27.
     # A little over one block a unit is the exception: most units would wait for the few that have two. Three splits there, two
-    # up to 416 blocks (all of 2,176 keys: 40 requests 81 us, with one split 92; 48 requests 91 and 95; of 100 to 2,000 keys
-    # 43 and 42, 52 and 46).
+    # up to 416 blocks (all of 2,176 keys, the same steps: 40 requests 2,775 us, with one split 2,806; 48 requests 2,785 and 2,852).
     most = min(covered, abs(window) + 64) if window else covered       # keys that a token can come to read
     if span <= 448 or (blocks >= 192 and most <= (4096 if blocks <= 256 else 6144) and (blocks > 416 or blocks <= 256 or window)):
         return -(-covered // 32) * 32
     if 256 < blocks <= 416 and not window:
         split_len = 128 * -(-span // (128 * (3 if blocks <= 352 else 2)))
     else:
-        split_len = max(128, 128 * round(max(span * blocks / 256, most / 36) / 128))
+        split_len = 128 * -(-max(span * blocks, most * 256 // 36) // (128 * 256))
     split_len = min(split_len, MOST_KEYS_A_SPLIT)
     if window and most <= MOST_KEYS_A_SPLIT:
         # a window lies in few of its context's splits, the others are empty blocks (8 requests with a window of 1,024 after 32,000

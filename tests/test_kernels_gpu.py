@@ -643,11 +643,13 @@ def test_decode_attention_of_many_tokens_with_one_split(ops, T, Hq, Hkv, D, page
     torch.testing.assert_close(out.double().cpu(), ref, **tol(torch.bfloat16))
 
 
-@pytest.mark.parametrize("T", [33, 44, 45, 52, 53])
-def test_decode_attention_of_a_little_over_one_block_a_unit(ops, T):
+@pytest.mark.parametrize("T,n_splits", [(32, 1), (33, 3), (44, 3), (45, 2), (52, 2), (53, 1)])
+def test_decode_attention_of_a_little_over_one_block_a_unit(ops, T, n_splits):
     """257 to 416 blocks: three splits, two, and one on either side, of contexts that end in any of them."""
+    from nanohybrid_vlm_amd.native.ops import decode_split_length
+    assert -(-700 // decode_split_length(T * 8, 700, 700, 0)) == n_splits
     g = torch.Generator().manual_seed(83)
-    lens = [500, 1] + torch.randint(2, 500, (T - 2,), generator=g).tolist()
+    lens = [700, 1] + torch.randint(2, 700, (T - 2,), generator=g).tolist()
     q, kc, vc, batch, bt, ks, vs, qs = _paged_setup(torch.bfloat16, lens, [1] * T, 8, 8, 64, 16, seed=84)
     out = ops.paged_attention(q, kc, vc, batch, bt, 0.125, None)
     torch.testing.assert_close(out.double().cpu(), _attention_reference(qs, ks, vs, lens, [1] * T, 0.125, None), **tol(torch.bfloat16))
