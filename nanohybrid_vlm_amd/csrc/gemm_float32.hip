@@ -1,31 +1,38 @@
-// y[M, N] = x[M, K] . w[N, K]^T (+ bias[N]) in float on the float matrix cores (v_mfma_f32_16x16x4_f32: every product and
-// sum in 32 bits).
+// y[M, N] = x[M, K] . w[N, K]^T (+ bias[N]) in float, on the bfloat16 matrix cores without losing any of the 32 bits.
 //
-// A row's result does not depend on how many rows there are: K is cut into 8 segments by K alone (a multiple of 16 long), a
-// segment is summed in blocks of 16 k, four matrix instructions a block (instruction j takes k = 4 g + j, g = 0..3), and the
-// segments are added in rising order. Which tile an output lies in changes nothing of that, so the tile may be chosen by
-// the shape.
+// A float is the sum of three bfloat16 numbers, exactly: what rounding to 8 bits gives, what that leaves rounded to 8 bits, and
+// the rest (nhv_split_float.h). A product of two floats is then nine products of 8 bits by 8, each exact in float; six of them
+// are summed. The three left out (middle x rest, rest x middle, rest x rest) are at most 2^-25 of the product together, half of
+// what rounding one float product may cost. One v_mfma_f32_16x16x32_bf16 sums 32 products in 16 clocks where the float
+// instruction sums 4 in 32: six of them take 96 clocks for what took 256. The products of the largest parts and the five small ones
+// have an accumulator each, which meet at a segment's end.
+// Off from 64 bits, 2-norm over 2-norm, normal entries, K = 64, 1024, 2048, 3072, 6144: 4.8e-8, 8.6e-8, 1.06e-7, 1.23e-7, 1.69e-7
+// (float matrix instructions: 8.4e-8, 2.11e-7, 2.93e-7, 3.56e-7, 5.0e-7).
 //
-// Two kernels. Up to some tens of rows, or few columns: a block is 8 waves and owns 16 RT rows by 16 CT columns, wave s sums
-// segment s, and LDS adds the segments up. Both operands come straight from memory in the instructions' own layout (a lane:
-// 16 bytes of one row), each row of x and w read once per block and by one wave only, so there is nothing for LDS to share;
-// all loads of a stage of U blocks are asked for one stage ahead. Few rows are bound by the read of w (one row: 1024 x 151,936
-// 113 us, 5.5 TB/s; 1024 x 4096 5.4 us) and, where the matrix is small, by the way there and back. Many rows: a block is 4
-// waves that share their operands through LDS, see below; bound by the matrix cores and the last round of blocks (2,048 x
-// 1024 . 4096: 160 us, 107 TFLOP/s; 517 rows 57 us). The kernel before this one (64 x 64 tiles, no matrix cores) took 197 us
-// for one row and 248 for 517 on the mean of the 0.6B shape's layers.
+// A row's result does not depend on how many rows there are: K is cut into 8 segments by K alone (a multiple of 32 long), a
+// segment is summed in blocks of 32 k, and the segments are added in rising order. Which tile an output lies in changes
+// nothing of that, so the tile may be chosen by the shape.
+//
+// The parts of an infinity are infinity and no numbers, and a number close to the largest float rounds up to infinity. So an
+// output that comes out infinite or as no number is summed once more by plain float multiply-adds, segment by segment: that
+// is what it is then. (Such inputs make every output of their row or column such a one.)
+//
+// Two kernels. Few rows, or few columns: a block is 8 waves and owns 16 RT rows by 16 CT columns, wave s sums segment s, and
+// LDS adds the segments up. Both operands come straight from memory (a lane: 16 bytes of each half of a row's 128); all loads
+// of a stage of U blocks of 32 k are asked for one stage ahead. What bounds it is what a compute unit takes in: a tile's time
+// grows by 5.6 us a 3,072 k with every 16 rows of x or w that it reads (35 GB/s), whatever their product. Many rows: a block is
+// 4 waves that share their operands' parts through LDS, see below.
 // The blocks of one column tile follow each other on one XCD, whose L2 then reads those rows of w once.
 #include "nhv_common.h"
-
-typedef float f32x4 __attribute__((ext_vector_type(4)));
+#include "nhv_split_float.h"
 
 #define SEGMENTS 8
 
-__host__ __device__ static inline int segment_length(int K) { return ((K + SEGMENTS - 1) / SEGMENTS + 15) & ~15; }
+__host__ __device__ static inline int segment_length(int K) { return ((K + SEGMENTS - 1) / SEGMENTS + 31) & ~31; }
 
 // four entries of a row from column k on. WIDE: rows of a multiple of four entries on 16-byte boundaries; beyond K the row's
 // last four (the caller puts zeros in their place), so that no load hangs on a condition: with conditions the compiler
-// waits for all loads under way, and a stage is no longer asked for ahead (47 us in place of 13 for 40 x 3072 . 1024).
+// waits for all loads under way, and a stage is no longer asked for ahead.
 template <bool WIDE>
 __device__ __forceinline__ f32x4 four_of(const float* __restrict__ row, int k, int K) {
   if (WIDE) return *reinterpret_cast<const f32x4*>(row + min(k, K - 4));
@@ -37,6 +44,20 @@ __device__ __forceinline__ f32x4 four_of(const float* __restrict__ row, int k, i
   }
   return v;
 }
+
+// the same output by plain float multiply-adds (see above)
+__device__ __attribute__((noinline)) float plain_product(const float* __restrict__ x, const float* __restrict__ w, int K) {
+  const int length = segment_length(K);
+  float total = 0.f;
+  for (int begin = 0; begin < K; begin += length) {
+    float v = 0.f;
+    for (int k = begin; k < min(K, begin + length); ++k) v = fmaf(x[k], w[k], v);
+    total = begin ? total + v : v;
+  }
+  return total;
+}
+
+__device__ __forceinline__ bool finite(float v) { return fabsf(v) < INFINITY; }
 
 template <int RT, int CT, int U, bool WIDE>
 __global__ __launch_bounds__(64 * SEGMENTS) void gemm_float32_kernel(const float* __restrict__ x, const float* __restrict__ w,
@@ -58,67 +79,86 @@ __global__ __launch_bounds__(64 * SEGMENTS) void gemm_float32_kernel(const float
 #pragma unroll
     for (int c = 0; c < CT; ++c) acc[r][c] = f32x4{0.f, 0.f, 0.f, 0.f};
   if (begin < end) {
+    f32x4 low[RT][CT];
+#pragma unroll
+    for (int r = 0; r < RT; ++r)
+#pragma unroll
+      for (int c = 0; c < CT; ++c) low[r][c] = f32x4{0.f, 0.f, 0.f, 0.f};
     const float *xp[RT], *wp[CT];                        // (rows beyond the last are the last one: their results are dropped)
 #pragma unroll
     for (int r = 0; r < RT; ++r) xp[r] = x + (size_t)min(m0 + 16 * r + r16, M - 1) * K;
 #pragma unroll
     for (int c = 0; c < CT; ++c) wp[c] = w + (size_t)min(n0 + 16 * c + r16, N - 1) * K;
-    f32x4 a[2][U][RT], b[2][U][CT];
+    f32x4 a[2][U][RT][2], b[2][U][CT][2];
     auto ask = [&](int buf, int k0) {
 #pragma unroll
       for (int u = 0; u < U; ++u) {
 #pragma unroll
-        for (int c = 0; c < CT; ++c) b[buf][u][c] = four_of<WIDE>(wp[c], k0 + 16 * u + 4 * g, K);
+        for (int c = 0; c < CT; ++c)
 #pragma unroll
-        for (int r = 0; r < RT; ++r) a[buf][u][r] = four_of<WIDE>(xp[r], k0 + 16 * u + 4 * g, K);
+          for (int h = 0; h < 2; ++h) b[buf][u][c][h] = four_of<WIDE>(wp[c], k0 + 32 * u + 4 * g + 16 * h, K);
+#pragma unroll
+        for (int r = 0; r < RT; ++r)
+#pragma unroll
+          for (int h = 0; h < 2; ++h) a[buf][u][r][h] = four_of<WIDE>(xp[r], k0 + 32 * u + 4 * g + 16 * h, K);
       }
     };
-    auto sum = [&](int buf) {
+    auto sum = [&](int buf, int u) {
+      SplitFloats8 xs[RT], ws[CT];
 #pragma unroll
-      for (int u = 0; u < U; ++u)
+      for (int c = 0; c < CT; ++c) ws[c] = split_floats(b[buf][u][c][0], b[buf][u][c][1]);
 #pragma unroll
-        for (int j = 0; j < 4; ++j)
+      for (int r = 0; r < RT; ++r) xs[r] = split_floats(a[buf][u][r][0], a[buf][u][r][1]);
 #pragma unroll
-          for (int r = 0; r < RT; ++r)
+      for (int step = 0; step < 6; ++step)
 #pragma unroll
-            for (int c = 0; c < CT; ++c)
-              acc[r][c] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[buf][u][r][j], b[buf][u][c][j], acc[r][c], 0, 0, 0);
+        for (int r = 0; r < RT; ++r)
+#pragma unroll
+          for (int c = 0; c < CT; ++c) split_product(step, xs[r], ws[c], acc[r][c], low[r][c]);
     };
-    // the last stage: what lies beyond the segment counts as zeros (which change no sum)
+    // the last stage: what lies beyond the segment is left out, or counts as zeros
     auto sum_last = [&](int buf, int k0) {
-      if (k0 + 16 * U > end) {
 #pragma unroll
-        for (int u = 0; u < U; ++u) {
-          const bool in = k0 + 16 * u + 4 * g < end;      // (WIDE: end is a multiple of four)
-          if (WIDE || k0 + 16 * u >= end) {
+      for (int u = 0; u < U; ++u) {
+        if (k0 + 32 * u >= end) break;
+        if (WIDE && k0 + 32 * u + 32 > end) {
+#pragma unroll
+          for (int h = 0; h < 2; ++h) {
+            const bool in = k0 + 32 * u + 4 * g + 16 * h < end;      // (end is a multiple of four)
 #pragma unroll
             for (int c = 0; c < CT; ++c)
-              if (!in) b[buf][u][c] = f32x4{0.f, 0.f, 0.f, 0.f};
+              if (!in) b[buf][u][c][h] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
             for (int r = 0; r < RT; ++r)
-              if (!in) a[buf][u][r] = f32x4{0.f, 0.f, 0.f, 0.f};
+              if (!in) a[buf][u][r][h] = f32x4{0.f, 0.f, 0.f, 0.f};
           }
         }
+        sum(buf, u);
       }
-      sum(buf);
     };
     ask(0, begin);
     for (int k0 = begin;;) {
-      if (k0 + 16 * U >= end) {
+      if (k0 + 32 * U >= end) {
         sum_last(0, k0);
         break;
       }
-      ask(1, k0 + 16 * U);
-      sum(0);
-      k0 += 16 * U;
-      if (k0 + 16 * U >= end) {
+      ask(1, k0 + 32 * U);
+#pragma unroll
+      for (int u = 0; u < U; ++u) sum(0, u);
+      k0 += 32 * U;
+      if (k0 + 32 * U >= end) {
         sum_last(1, k0);
         break;
       }
-      ask(0, k0 + 16 * U);
-      sum(1);
-      k0 += 16 * U;
+      ask(0, k0 + 32 * U);
+#pragma unroll
+      for (int u = 0; u < U; ++u) sum(1, u);
+      k0 += 32 * U;
     }
+#pragma unroll
+    for (int r = 0; r < RT; ++r)
+#pragma unroll
+      for (int c = 0; c < CT; ++c) acc[r][c] += low[r][c];
   }
 #pragma unroll
   for (int r = 0; r < RT; ++r) {
@@ -127,14 +167,17 @@ __global__ __launch_bounds__(64 * SEGMENTS) void gemm_float32_kernel(const float
 #pragma unroll
     for (int c = 0; c < CT; ++c) *reinterpret_cast<f32x4*>(&part[s][(c * 64 + lane) * 4]) = acc[r][c];
     __syncthreads();
-    for (int i = threadIdx.x; i < CT * 256; i += 64 * SEGMENTS) {
+    for (int i = threadIdx.x; i < 256 * CT; i += 64 * SEGMENTS) {
       // (lane 16 g + n of a tile holds rows 4 g .. 4 g + 3 of column n)
-      const int c = i % (CT * 16), row = i / (CT * 16);
+      const int c = i % (16 * CT), row = i / (16 * CT);
       const int at = ((c >> 4) * 64 + (row >> 2) * 16 + (c & 15)) * 4 + (row & 3);
       float v = part[0][at];
       for (int p = 1; p < active; ++p) v += part[p][at];
       const int m = m0 + 16 * r + row, n = n0 + c;
-      if (m < M && n < N) y[(size_t)m * N + n] = bias ? v + bias[n] : v;
+      if (m < M && n < N) {
+        if (!finite(v)) v = plain_product(x + (size_t)m * K, w + (size_t)n * K, K);
+        y[(size_t)m * N + n] = bias ? v + bias[n] : v;
+      }
     }
   }
 }
@@ -150,23 +193,28 @@ static void launch(const float* x, const float* w, const float* bias, float* y, 
 }
 
 // ---------------------------------------------------------------- many rows
-// 4 waves, 2 x 2, a wave RT x CT tiles of 16 x 16; both operands through LDS in pieces of 32 k, two buffers, the next
-// piece under way in registers while this one is summed. A wave takes every segment in turn and adds it to the total: the
-// same sums in the same order as above.
+// 4 waves, 2 x 2, a wave RT x CT tiles of 16 x 16; the parts of both operands through LDS in pieces of 32 k, two buffers, two
+// pieces under way in registers: an entry is taken apart once a block. A wave takes every segment in turn and adds it to the
+// total: the same sums in the same order as above. What bounds it: matrix and vector instructions (24 and 56 of them a piece
+// and wave of the large tile) add up more than they overlap, within a wave and between two of a SIMD; so three blocks a
+// compute unit, which is why LDS rows have no padding and only two pieces are under way (two blocks, with 80-byte rows and
+// four pieces: 517 x 4096 . 1024 in 58 us in place of 45). 2 x 2 tiles a wave: 1,500 x 12,288 . 2048 in 538 us (140 TFLOP/s;
+// float matrix instructions 672).
 #define PIECE 32
+#define AHEAD 2
 template <int RT, int CT, bool WIDE>
-__global__ __launch_bounds__(256) void gemm_float32_tiles_kernel(const float* __restrict__ x, const float* __restrict__ w,
+__global__ __launch_bounds__(256, RT * CT > 2 ? 3 : 4) void gemm_float32_tiles_kernel(const float* __restrict__ x, const float* __restrict__ w,
                                                                  const float* __restrict__ bias, float* __restrict__ y, int M, int N,
                                                                  int K, int m_tiles, int n_tiles) {
-  constexpr int BM = 32 * RT, BN = 32 * CT, STRIDE = PIECE + 4, LOADS = (BM + BN) * PIECE / 4 / 256;
-  __shared__ __attribute__((aligned(16))) float rows[2][(BM + BN) * STRIDE];
+  constexpr int BM = 32 * RT, BN = 32 * CT, LOADS = (BM + BN) * PIECE / 4 / 256, PLANE = (BM + BN) * PIECE;
+  __shared__ __attribute__((aligned(16))) bf16_t rows[2][3 * PLANE];
   const int total_tiles = m_tiles * n_tiles, share = (total_tiles + 7) >> 3;
   const int tile = (blockIdx.x & 7) * share + (blockIdx.x >> 3);
   if (tile >= total_tiles) return;
   const int m0 = (tile % m_tiles) * BM, n0 = (tile / m_tiles) * BN;
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, r16 = lane & 15, g = lane >> 4;
   const int mw = (wave >> 1) * 16 * RT, nw = (wave & 1) * 16 * CT;
-  const int length = segment_length(K);
+  const int length = segment_length(K), at = (g ^ (r16 >> 2)) << 3;
   // what this thread brings of a piece: 16 bytes of rows x (first BM) and w
   const float* src[LOADS];
   const int col = (threadIdx.x & 7) * 4;
@@ -175,74 +223,95 @@ __global__ __launch_bounds__(256) void gemm_float32_tiles_kernel(const float* __
     const int r = (threadIdx.x >> 3) + 32 * i;
     src[i] = r < BM ? x + (size_t)min(m0 + r, M - 1) * K : w + (size_t)min(n0 + r - BM, N - 1) * K;
   }
-  f32x4 hold[LOADS];
-  auto ask = [&](int k0) {
+  // where they go: lane group g of a product takes k = 4 g .. and 16 + 4 g .., 16 bytes together, whose place in the row's 64
+  // turns with the row so that 16 rows lie in different banks
+  const int r8 = threadIdx.x >> 3, to_row = r8 * PIECE + (((threadIdx.x & 3) ^ (r8 >> 2 & 3)) << 3) + ((threadIdx.x >> 2 & 1) << 2);
+  f32x4 hold[AHEAD][LOADS];
+  auto ask = [&](int i_hold, int k0) {
 #pragma unroll
-    for (int i = 0; i < LOADS; ++i) hold[i] = four_of<WIDE>(src[i], k0 + col, K);
+    for (int i = 0; i < LOADS; ++i) hold[i_hold][i] = four_of<WIDE>(src[i], k0 + col, K);
   };
-  auto put = [&](int buf, int k0) {
+  auto put = [&](int buf, int i_hold, int k0) {
+    if (WIDE && k0 + PIECE > K) {                        // (the same for the whole grid)
+      asm volatile("");                                  // a real branch: not a selection in every piece
+      if (k0 + col >= K)
+#pragma unroll
+        for (int i = 0; i < LOADS; ++i) hold[i_hold][i] = f32x4{0.f, 0.f, 0.f, 0.f};
+    }
 #pragma unroll
     for (int i = 0; i < LOADS; ++i) {
-      if (WIDE && k0 + col >= K) hold[i] = f32x4{0.f, 0.f, 0.f, 0.f};
-      *reinterpret_cast<f32x4*>(&rows[buf][((threadIdx.x >> 3) + 32 * i) * STRIDE + col]) = hold[i];
+      const SplitFloats4 p = split_floats(hold[i_hold][i]);
+      bf16_t* to = &rows[buf][32 * i * PIECE + to_row];
+      *reinterpret_cast<bf16x4*>(to) = p.high;
+      *reinterpret_cast<bf16x4*>(to + PLANE) = p.middle;
+      *reinterpret_cast<bf16x4*>(to + 2 * PLANE) = p.rest;
     }
   };
-  f32x4 acc[RT][CT], total[RT][CT];
+  f32x4 acc[RT][CT], low[RT][CT], total[RT][CT];
 #pragma unroll
   for (int r = 0; r < RT; ++r)
 #pragma unroll
     for (int c = 0; c < CT; ++c) {
-      acc[r][c] = f32x4{0.f, 0.f, 0.f, 0.f};
+      acc[r][c] = low[r][c] = f32x4{0.f, 0.f, 0.f, 0.f};
       total[r][c] = f32x4{-0.f, -0.f, -0.f, -0.f};
     }
+  auto close = [&] {                                     // a segment's end
+#pragma unroll
+    for (int r = 0; r < RT; ++r)
+#pragma unroll
+      for (int c = 0; c < CT; ++c) {
+        total[r][c] += acc[r][c] + low[r][c];
+        acc[r][c] = low[r][c] = f32x4{0.f, 0.f, 0.f, 0.f};
+      }
+  };
   int left = length;                                     // of the segment
-  ask(0);
-  put(0, 0);
+#pragma unroll
+  for (int d = 0; d < AHEAD; ++d) ask(d, d * PIECE);
+  put(0, 0, 0);
+  ask(0, AHEAD * PIECE);
   __syncthreads();
-  int buf = 0;
-  for (int k0 = 0; k0 < K; k0 += PIECE) {
-    ask(k0 + PIECE);
+  for (int k0 = 0; k0 < K; k0 += AHEAD * PIECE) {
 #pragma unroll
-    for (int h = 0; h < PIECE; h += 16) {
-      f32x4 a[RT], b[CT];
+    for (int d = 0; d < AHEAD; ++d) {                    // (piece d lies in buffer d)
+      const int k = k0 + d * PIECE, buf = d;
+      if (k >= K) break;
+      SplitFloats8 a[RT], b[CT];
 #pragma unroll
-      for (int r = 0; r < RT; ++r) a[r] = *reinterpret_cast<const f32x4*>(&rows[buf][(mw + 16 * r + r16) * STRIDE + h + 4 * g]);
+      for (int r = 0; r < RT; ++r) a[r] = split_at<PLANE>(&rows[buf][(mw + 16 * r + r16) * PIECE + at]);
 #pragma unroll
-      for (int c = 0; c < CT; ++c) b[c] = *reinterpret_cast<const f32x4*>(&rows[buf][(BM + nw + 16 * c + r16) * STRIDE + h + 4 * g]);
+      for (int c = 0; c < CT; ++c) b[c] = split_at<PLANE>(&rows[buf][(BM + nw + 16 * c + r16) * PIECE + at]);
 #pragma unroll
-      for (int j = 0; j < 4; ++j)
+      for (int step = 0; step < 6; ++step)
 #pragma unroll
         for (int r = 0; r < RT; ++r)
 #pragma unroll
-          for (int c = 0; c < CT; ++c) acc[r][c] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[r][j], b[c][j], acc[r][c], 0, 0, 0);
-      left -= 16;
+          for (int c = 0; c < CT; ++c) split_product(step, a[r], b[c], acc[r][c], low[r][c]);
+      left -= PIECE;
       if (left == 0) {
         left = length;
-#pragma unroll
-        for (int r = 0; r < RT; ++r)
-#pragma unroll
-          for (int c = 0; c < CT; ++c) {
-            total[r][c] += acc[r][c];
-            acc[r][c] = f32x4{0.f, 0.f, 0.f, 0.f};
-          }
+        asm volatile("");                                // (a real branch)
+        close();
       }
+      put(buf ^ 1, d ^ 1, k + PIECE);
+      ask(d ^ 1, k + (1 + AHEAD) * PIECE);
+      __syncthreads();
     }
-    put(buf ^ 1, k0 + PIECE);
-    __syncthreads();
-    buf ^= 1;
   }
-  const bool rest = (K + 15) / 16 * 16 % length != 0;    // (the last segment is shorter and not added yet)
+  if (left != length) close();                           // (the last segment is shorter and not added yet)
 #pragma unroll
   for (int r = 0; r < RT; ++r)
 #pragma unroll
     for (int c = 0; c < CT; ++c) {
-      if (rest) total[r][c] += acc[r][c];
       const int n = n0 + nw + 16 * c + r16;
       const float add = bias && n < N ? bias[n] : 0.f;
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         const int m = m0 + mw + 16 * r + 4 * g + i;
-        if (m < M && n < N) y[(size_t)m * N + n] = bias ? total[r][c][i] + add : total[r][c][i];
+        if (m < M && n < N) {
+          float v = total[r][c][i];
+          if (!finite(v)) v = plain_product(x + (size_t)m * K, w + (size_t)n * K, K);
+          y[(size_t)m * N + n] = bias ? v + add : v;
+        }
       }
     }
 }
@@ -263,17 +332,29 @@ extern "C" int nhv_gemm_float32(const void* x, const void* w, const void* bias, 
   hipStream_t s = (hipStream_t)stream;
   const float *xf = (const float*)x, *wf = (const float*)w, *bf = (const float*)bias;
   float* yf = (float*)y;
-  // Blocks that a tile of m rows and n columns gives. The largest tile that still fills the chip is the fastest (per output it
-  // reads the least); the lines lie where the times of the 0.6B and 1.7B shapes' products cross (1 to 2,048 rows, every tile
-  // timed): e.g. 517 x 1024 . 4096 64.5 us with 64 x 64 tiles (576 blocks), 57.5 with 32 x 64; 260 x 6144 . 2048 164 us with
-  // 32 x 64 (288 blocks), 138 with 8 waves on 32 x 32; 40 x 3072 . 1024 25 us with 32 x 32, 19 with 32 x 16, 14 with 16 x 16.
+  // Every tile's time in units of what a compute unit needs for 16 rows of an operand, from the times of all tiles at 1 to 1,500
+  // rows of the 0.6B and 1.7B shapes' products. Tiles of 8 waves: rounds of 256 blocks times 16-row operands; the tiles through
+  // LDS: a floor (one block's chain of pieces) and what a block a compute unit adds. E.g. 17 x 6144 . 1024: 32 x 32 10.1 us,
+  // 16 x 32 14.0, 16 x 16 13.9 (float matrix instructions 12.6); 130 x 2048 . 2048: 48 x 32 22.1 us, 32 x 32 33.3 (33.2); 517 x
+  // 1024 . 3072: 32 x 32 through LDS 58.9, 48 x 32 60.0, 64 x 64 66.6 (71); 517 x 4096 . 1024: 64 x 64 45, 32 x 32 through LDS 56
+  // (57). Up to 16 rows LDS has nothing to share and is left out (6 x 151,936 . 1024: 116 us with 16 x 32, 135 through LDS; 137).
   auto blocks = [&](long long m, long long n) { return ((M + m - 1) / m) * ((N + n - 1) / n); };
-  if (M <= 16) launch<1, 1, 4>(xf, wf, bf, yf, M, N, K, s);
-  else if (blocks(64, 64) >= 640) launch_tiles<2, 2>(xf, wf, bf, yf, M, N, K, s);
-  else if (blocks(32, 64) >= 400) launch_tiles<1, 2>(xf, wf, bf, yf, M, N, K, s);
-  else if (blocks(32, 32) >= 150) launch<2, 2, 2>(xf, wf, bf, yf, M, N, K, s);
-  else if (blocks(32, 16) >= 150) launch<2, 1, 4>(xf, wf, bf, yf, M, N, K, s);
-  else launch<1, 1, 4>(xf, wf, bf, yf, M, N, K, s);
+  auto rounds = [&](int rt, int ct) { return (double)((blocks(16 * rt, 16 * ct) + 255) / 256 * (rt + ct)); };
+  const double none = 1e300;
+  const double cost[6] = {rounds(1, 1), rounds(1, 2), M > 16 ? rounds(2, 2) : none, M > 32 ? rounds(3, 2) : none,
+                          M > 16 ? fmax(9.0, 1.5 + 2.9 / 256 * blocks(32, 32)) : none,
+                          M > 16 ? fmax(11.5, 4.5 + 7.7 / 256 * blocks(64, 64)) : none};
+  int best = 0;
+  for (int i = 1; i < 6; ++i)
+    if (cost[i] < cost[best]) best = i;
+  switch (best) {
+    case 0: launch<1, 1, 2>(xf, wf, bf, yf, M, N, K, s); break;
+    case 1: launch<1, 2, 1>(xf, wf, bf, yf, M, N, K, s); break;
+    case 2: launch<2, 2, 1>(xf, wf, bf, yf, M, N, K, s); break;
+    case 3: launch<3, 2, 1>(xf, wf, bf, yf, M, N, K, s); break;
+    case 4: launch_tiles<1, 1>(xf, wf, bf, yf, M, N, K, s); break;
+    default: launch_tiles<2, 2>(xf, wf, bf, yf, M, N, K, s);
+  }
   NHV_LAUNCH_CHECK("gemm_float32");
   return 0;
 }

@@ -1,0 +1,67 @@
+// Products of floats on the bfloat16 matrix cores: a float as the sum of three bfloat16 numbers.
+//
+// high = x rounded to 8 bits, middle = (x - high) rounded, rest = x - high - middle. Both differences are exact (a float has 24
+// bits; each part takes 8 and its sign one more), and so is the rest's conversion: high + middle + rest = x, bit for bit, as
+// long as the rest is no denormal (|x| above about 2^-109; below that what is lost is under 2^-133).
+#pragma once
+#include "nhv_common.h"
+
+typedef float f32x2 __attribute__((ext_vector_type(2)));
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef bf16_t bf16x2 __attribute__((ext_vector_type(2)));
+typedef bf16_t bf16x4 __attribute__((ext_vector_type(4)));
+typedef bf16_t bf16x8 __attribute__((ext_vector_type(8)));
+
+struct SplitFloats4 { bf16x4 high, middle, rest; };
+struct SplitFloats8 { bf16x8 high, middle, rest; };
+
+// (a, b) rounded to bfloat16, and what that leaves of them in their place. The dot product with (-1, 0) is one instruction where
+// a widening and a subtraction are two; it is exact, since its result is. (The two pairs come from scalar registers that the
+// compiler does not see through: it would write the first as the inline constant -1.0, which the instruction reads as another
+// pair, and every first entry's parts came out wrong.)
+__device__ __forceinline__ bf16x2 take_high(float& a, float& b) {
+  uint32_t first = 0x0000bf80u, second = 0xbf800000u;
+  asm("" : "+s"(first));
+  asm("" : "+s"(second));
+  const bf16x2 high = __builtin_convertvector((f32x2{a, b}), bf16x2);
+  a = __builtin_amdgcn_fdot2_f32_bf16(high, __builtin_bit_cast(bf16x2, first), a, false);
+  b = __builtin_amdgcn_fdot2_f32_bf16(high, __builtin_bit_cast(bf16x2, second), b, false);
+  return high;
+}
+
+__device__ __forceinline__ SplitFloats4 split_floats(f32x4 v) {
+  SplitFloats4 p;
+#pragma unroll
+  for (int i = 0; i < 4; i += 2) {
+    float a = v[i], b = v[i + 1];
+    const bf16x2 high = take_high(a, b), middle = take_high(a, b), rest = __builtin_convertvector((f32x2{a, b}), bf16x2);
+    p.high[i] = high[0], p.high[i + 1] = high[1];
+    p.middle[i] = middle[0], p.middle[i + 1] = middle[1];
+    p.rest[i] = rest[0], p.rest[i + 1] = rest[1];
+  }
+  return p;
+}
+
+__device__ __forceinline__ SplitFloats8 split_floats(f32x4 v0, f32x4 v1) {
+  const SplitFloats4 p = split_floats(v0), q = split_floats(v1);
+  return {__builtin_shufflevector(p.high, q.high, 0, 1, 2, 3, 4, 5, 6, 7),
+          __builtin_shufflevector(p.middle, q.middle, 0, 1, 2, 3, 4, 5, 6, 7),
+          __builtin_shufflevector(p.rest, q.rest, 0, 1, 2, 3, 4, 5, 6, 7)};
+}
+
+// eight entries whose parts lie PLANE entries apart (in LDS)
+template <int PLANE>
+__device__ __forceinline__ SplitFloats8 split_at(const bf16_t* p) {
+  return {*reinterpret_cast<const bf16x8*>(p), *reinterpret_cast<const bf16x8*>(p + PLANE),
+          *reinterpret_cast<const bf16x8*>(p + 2 * PLANE)};
+}
+
+// One of the six products of a block of 32 k: the one of the high parts goes to `high`, the five small ones to `low`.
+__device__ __forceinline__ void split_product(int step, const SplitFloats8& a, const SplitFloats8& b, f32x4& high, f32x4& low) {
+  if (step == 0) low = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a.middle, b.middle, low, 0, 0, 0);
+  if (step == 1) low = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a.rest, b.high, low, 0, 0, 0);
+  if (step == 2) low = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a.high, b.rest, low, 0, 0, 0);
+  if (step == 3) low = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a.middle, b.high, low, 0, 0, 0);
+  if (step == 4) low = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a.high, b.middle, low, 0, 0, 0);
+  if (step == 5) high = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a.high, b.high, high, 0, 0, 0);
+}

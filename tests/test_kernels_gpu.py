@@ -304,6 +304,35 @@ def test_float32_linear_in_all_its_tiles(ops, N, K):
         last = y
 
 
+@pytest.mark.parametrize("M,N,K", [(1, 16, 33), (6, 40, 300), (30, 600, 1024), (70, 4096, 64), (130, 9000, 96)])
+def test_float32_linear_at_the_ends_of_its_range(ops, M, N, K):
+    """Infinities, no numbers, numbers that round up to infinity in 8 bits and numbers whose parts are tiny: in their own rows and
+    columns what float multiply-adds give, everywhere else what the product without them gives, bit for bit."""
+    x, w = rnd(M, K, seed=61), rnd(N, K, seed=62)
+    clean = ops.linear(x, w)
+    odd, columns = [0] if M == 1 else [0, M // 2, M - 1], [0, 3, N // 2, N - 1]
+    top = 3.4e38                                             # (rounds to infinity in 8 bits)
+    x[odd[0], K // 3] = top
+    if M > 1:
+        x[odd[1], 0], x[odd[2], K - 1] = float("inf"), float("nan")
+    w[columns[0], K // 2], w[columns[1], 1], w[columns[2], K - 1] = float("-inf"), float("nan"), top
+    w[columns[3]] *= 1e-30
+    y = ops.linear(x, w)
+    rows, cols = [i for i in range(M) if i not in odd], [i for i in range(N) if i not in columns]
+    assert torch.equal(y[rows][:, cols], clean[rows][:, cols])
+    want = x.double().cpu() @ w.double().cpu().T
+    want = torch.where(want.abs() > 3.4028235e38, torch.sign(want) * math.inf, want)
+    got = y.double().cpu()
+    sure = (want.abs() < 3.3e38) | ~torch.isfinite(want) | (want.abs() > 3.5e38)
+    for row, column in ((odd[0], columns[2]), (odd[0], columns[0]), (odd[len(odd) // 2], columns[2])):
+        sure[row, column] = False                            # a term that overflows beside an infinite or another large one
+    assert torch.equal(torch.isnan(got)[sure], torch.isnan(want)[sure]) and torch.equal(torch.isinf(got)[sure], torch.isinf(want)[sure])
+    near = sure & torch.isfinite(want)
+    # K roundings of the sum of the terms' sizes at most
+    size = x.double().cpu().abs() @ w.double().cpu().abs().T
+    assert ((got - want).abs()[near] <= (K * 2.0 ** -24 * size)[near]).all()
+
+
 def test_linear_rows_do_not_depend_on_the_batch_in_float32(ops):
     x = rnd(70, 200, seed=7)
     w = rnd(150, 200, seed=8)
