@@ -2,18 +2,20 @@
 // for key heads of a multiple of 16 entries and value heads of 64, 128, 192 or 256; masks and options are those of
 // attention_generic.hip, which takes the other sizes.
 //
-// Keys are taken in blocks of 32 aligned to absolute positions. Each block's maximum, sum and weighted values are computed by
-// themselves and merged in rising order, masked keys count as nothing, so a position's result depends neither on the batch
-// nor on the portion, nor on which wave took a block.
+// Keys are taken in blocks of 32 aligned to absolute positions, of which wave w of a block's 8 takes numbers w, w + 8, ... in
+// turn, with a running maximum, sum and weighted values of its own; the 8 waves' results are merged in their order. Masked
+// keys count as nothing and a row's numbers hang on its own keys alone, so a position's result depends neither on the batch nor
+// on the portion.
 //
-// A block of 8 waves owns 16 rows, a row being (token, one of the query heads that read one key/value head), of one request:
-// 8 tokens of a prompt where two heads share a key head, or one decoded token. The waves take the blocks of keys in turn;
-// after each round of eight blocks the results meet in LDS and are merged. Scores come as S^T = K Q^T, whose layout is
-// that of the second product's right operand (O^T = V^T P^T), so the weights never leave their registers.
-// What bounds it: the chain of rounds of a row tile, half of it matrix instructions, the rest exponentials and the merge, which
-// a block's barrier keeps from overlapping (next round's loads asked for before the merge: no faster). 16 heads on 8 key heads
-// of 128: a prompt of 517 tokens 55 us (four waves with blocks of 64 keys and conditional loads 63), six tokens after 100
-// 9 us (29), eight after 3,000 132 us.
+// A block owns 16 rows, a row being (token, one of the query heads that read one key/value head), of one request: 8 tokens of
+// a prompt where two heads share a key head, or one decoded token. Scores come as S^T = K Q^T, whose layout is that of the
+// second product's right operand (O^T = V^T P^T), so the weights never leave their registers; neither do the sums: the waves
+// meet in LDS once, at the end (before, after every eight blocks of keys, with a barrier on either side). What bounds it: a
+// wave's blocks are 128 matrix instructions of 32 clocks each and two waves share a SIMD; registers allow one block a compute
+// unit. 16 heads on 8 key heads of 128, us, before and now: a prompt of 517 tokens 54.6, 41.1; 500 tokens after 1,500 179, 117;
+// six tokens after 100 9.1, 8.4; one after 300 18.1, 14.6; eight after 3,000 132, 89. Not faster: a block's keys all asked for
+// at once and the next block's before the values are worked on (44.8, 119, 8.9, 16.4, 89), four waves a block (39.2, 114, 8.6,
+// 16.8, 130).
 #include "nhv_common.h"
 #include <math.h>
 
@@ -40,9 +42,11 @@ struct FloatAttention {
   long long gate_ld;
 };
 
+template <int CHUNKS>                                    // of 64 value entries
 __global__ __launch_bounds__(64 * WAVES) void attention_float32_kernel(FloatAttention a) {
   extern __shared__ __attribute__((aligned(16))) float shared[];
-  const int D = a.D, E = a.E, group = a.Hq / a.Hkv;
+  constexpr int E = 64 * CHUNKS;
+  const int D = a.D, group = a.Hq / a.Hkv;
   float* qs = shared;                                    // [ROWS][D + 4]
   float* part = qs + ROWS * (D + 4);                     // [WAVES][ROWS][E + 4]
   float* stats = part + WAVES * ROWS * (E + 4);          // [WAVES][ROWS][2]: maximum and sum
@@ -74,170 +78,196 @@ __global__ __launch_bounds__(64 * WAVES) void attention_float32_kernel(FloatAtte
       v = *reinterpret_cast<const f32x4*>(a.q + ((size_t)(first + (row0 + r) / group) * a.Hq + kvh * group + (row0 + r) % group) * D + d);
     *reinterpret_cast<f32x4*>(&qs[r * (D + 4) + d]) = v;
   }
+
+  // of row r16: the maximum, this lane's share of the sum (lanes r16, 16 + r16, ... together have all) and values so far
+  float M = -INFINITY, L = 0.f;
+  f32x4 o[CHUNKS][4];
+#pragma unroll
+  for (int h = 0; h < CHUNKS; ++h)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) o[h][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+  __syncthreads();                                       // (the queries are in LDS)
+  // (the first block of this wave's from the tile's first key on)
+  const int from = (tile_lo / KEYS + ((wave - tile_lo / KEYS) & (WAVES - 1))) * KEYS;
+  for (int kb = from; kb <= tile_hi; kb += KEYS * WAVES) {
+    // lane l's own key of the block, and where it lies. A key that no row reads is taken for the tile's last: its score is
+    // masked, and every load is without a condition (with one the compiler waits for all that are under way).
+    const int mine = kb + lane % KEYS, own = mine >= tile_lo && mine <= tile_hi ? mine : tile_hi;
+    const int slot = table[own / a.page_size] * a.page_size + own % a.page_size;
+    f32x4 s[TILES], kf[2][2][TILES], vf[TILES][4];
+    const float *kr[TILES], *vr[TILES][4];
+#pragma unroll
+    for (int t = 0; t < TILES; ++t) {
+      kr[t] = a.k + ((size_t)__shfl(slot, 16 * t + r16, NHV_WAVE) * a.Hkv + kvh) * D + 4 * g;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) vr[t][i] = a.v + ((size_t)__shfl(slot, 16 * t + 4 * g + i, NHV_WAVE) * a.Hkv + kvh) * E + 4 * r16;
+      s[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+    }
+    // keys two blocks of 16 entries ahead (the last one again where there are no two); the first 64 value entries at once
+    auto ask = [&](int buf, int d) {
+#pragma unroll
+      for (int u = 0; u < 2; ++u)
+#pragma unroll
+        for (int t = 0; t < TILES; ++t) kf[buf][u][t] = *reinterpret_cast<const f32x4*>(kr[t] + min(d + 16 * u, D - 16));
+    };
+    auto score = [&](int buf, int d, int u) {
+      const f32x4 qf = *reinterpret_cast<const f32x4*>(&qs[r16 * (D + 4) + d + 16 * u + 4 * g]);
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+#pragma unroll
+        for (int t = 0; t < TILES; ++t) s[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[buf][u][t][j], qf[j], s[t], 0, 0, 0);
+    };
+    ask(0, 0);
+#pragma unroll
+    for (int t = 0; t < TILES; ++t)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) vf[t][i] = *reinterpret_cast<const f32x4*>(vr[t][i]);
+    int d = 0;
+    for (; d + 64 <= D; d += 64) {
+      ask(1, d + 32);
+      score(0, d, 0);
+      score(0, d, 1);
+      ask(0, d + 64);
+      score(1, d + 32, 0);
+      score(1, d + 32, 1);
+    }
+    if (d < D) {                                       // 16, 32 or 48 entries more
+      ask(1, d + 32);
+      score(0, d, 0);
+      if (d + 16 < D) score(0, d, 1);
+      if (d + 32 < D) score(1, d + 32, 0);
+    }
+    // s[t][i]: key kb + 16 t + 4 g + i against row r16
+    float m = -INFINITY;
+#pragma unroll
+    for (int t = 0; t < TILES; ++t)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int key = kb + 16 * t + 4 * g + i;
+        float z = s[t][i] * a.scale;
+        if (a.cap > 0.f) z = a.cap * tanhf(z / a.cap);
+        if (a.slopes) z = fmaf(-slope, (float)(pos - key), z);
+        s[t][i] = key >= lo && key <= pos ? z : -INFINITY;
+        m = fmaxf(m, s[t][i]);
+      }
+    m = fmaxf(m, __shfl_xor(m, 16, NHV_WAVE));
+    m = fmaxf(m, __shfl_xor(m, 32, NHV_WAVE));
+    m = fmaxf(m, M);
+    const float base = m == -INFINITY ? 0.f : m;       // (no visible key so far: every weight is 0)
+    const float old = expf(M - base);
+    M = m;
+    L *= old;
+#pragma unroll
+    for (int t = 0; t < TILES; ++t)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        s[t][i] = expf(s[t][i] - base);
+        L += s[t][i];
+      }
+    // value entry 64 h + 4 r + j is row r of matrix tile j: one load of 16 bytes a key feeds four tiles. The next chunk is
+    // asked for as this one is used up.
+#pragma unroll
+    for (int h = 0; h < CHUNKS; ++h) {
+      f32x4 now[4];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) now[j] = f32x4{0.f, 0.f, 0.f, 0.f};
+      float odd = 0.f;                                 // not a number as soon as some value is infinite or none
+#pragma unroll
+      for (int t = 0; t < TILES; ++t)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+#pragma unroll
+          for (int j = 0; j < 4; ++j) {
+            odd = fmaf(vf[t][i][j], 0.f, odd);
+            now[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(vf[t][i][j], s[t][i], now[j], 0, 0, 0);
+          }
+          if (h + 1 < CHUNKS) vf[t][i] = *reinterpret_cast<const f32x4*>(vr[t][i] + 64 * (h + 1));
+        }
+      // now[j][i]: row r16, entry 64 h + 16 g + 4 i + j
+      if (__any(odd != 0.f)) {
+        // a value that is no finite number: it must not reach the rows that do not read it (0 times it is not 0)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) now[j] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int t = 0; t < TILES; ++t)
+#pragma unroll
+          for (int i = 0; i < 4; ++i)
+            for (int gk = 0; gk < 4; ++gk) {
+              const int at = __shfl(slot, 16 * t + 4 * gk + i, NHV_WAVE);
+              const float p = __shfl(s[t][i], 16 * gk + r16, NHV_WAVE);
+              if (p != 0.f) {
+                const float* row_v = a.v + ((size_t)at * a.Hkv + kvh) * E + 64 * h + 16 * g;
+#pragma unroll
+                for (int ii = 0; ii < 4; ++ii)
+#pragma unroll
+                  for (int j = 0; j < 4; ++j) now[j][ii] = fmaf(p, row_v[4 * ii + j], now[j][ii]);
+              }
+            }
+      }
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) o[h][j][i] = fmaf(o[h][j][i], old, now[j][i]);
+    }
+  }
+  L += __shfl_xor(L, 16, NHV_WAVE);
+  L += __shfl_xor(L, 32, NHV_WAVE);
+  if (g == 0) {
+    stats[(wave * ROWS + r16) * 2] = M;
+    stats[(wave * ROWS + r16) * 2 + 1] = L;
+  }
+  if (from <= tile_hi) {
+#pragma unroll
+    for (int h = 0; h < CHUNKS; ++h)
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        *reinterpret_cast<f32x4*>(&part[(wave * ROWS + r16) * (E + 4) + 64 * h + 16 * g + 4 * i]) = f32x4{o[h][0][i], o[h][1][i], o[h][2][i], o[h][3][i]};
+  }
   __syncthreads();
 
   // what a thread merges: 32 threads a row, entries c + 32 i
   const int my_row = threadIdx.x / (4 * WAVES), c = threadIdx.x % (4 * WAVES);
-  float M = -INFINITY, L = 0.f, total[MAX_E / (4 * WAVES)];
+  if (row0 + my_row >= rows) return;
+  float top = -INFINITY, sum = 0.f, total[2 * CHUNKS];
 #pragma unroll
-  for (int i = 0; i < MAX_E / (4 * WAVES); ++i) total[i] = 0.f;
-
-  for (int round = tile_lo / KEYS * KEYS; round <= tile_hi; round += KEYS * WAVES) {
-    const int kb = round + wave * KEYS;
-    if (kb <= tile_hi) {
-      // lane l's own key of the block, and where it lies. A key that no row reads is taken for the tile's last: its score is
-      // masked, and every load is without a condition (with one the compiler waits for all that are under way).
-      const int mine = kb + lane % KEYS, own = mine >= tile_lo && mine <= tile_hi ? mine : tile_hi;
-      const int slot = table[own / a.page_size] * a.page_size + own % a.page_size;
-      f32x4 s[TILES], kf[2][2][TILES], vf[TILES][4];
-      const float *kr[TILES], *vr[TILES][4];
+  for (int p = 0; p < WAVES; ++p) top = fmaxf(top, stats[(p * ROWS + my_row) * 2]);
 #pragma unroll
-      for (int t = 0; t < TILES; ++t) {
-        kr[t] = a.k + ((size_t)__shfl(slot, 16 * t + r16, NHV_WAVE) * a.Hkv + kvh) * D + 4 * g;
+  for (int i = 0; i < 2 * CHUNKS; ++i) total[i] = 0.f;
 #pragma unroll
-        for (int i = 0; i < 4; ++i) vr[t][i] = a.v + ((size_t)__shfl(slot, 16 * t + 4 * g + i, NHV_WAVE) * a.Hkv + kvh) * E + 4 * r16;
-        s[t] = f32x4{0.f, 0.f, 0.f, 0.f};
-      }
-      // keys two blocks of 16 entries ahead (the last one again where there are no two); the first 64 value entries at once
-      auto ask = [&](int buf, int d) {
+  for (int p = 0; p < WAVES; ++p) {
+    const float m = stats[(p * ROWS + my_row) * 2], l = stats[(p * ROWS + my_row) * 2 + 1];
+    // a wave of whose keys this row reads none, or none with a weight. (The maximum alone does not say that: fmaxf passes over a
+    // score that is no number, and where all are such the sum of the weights tells.)
+    if (m == -INFINITY && l == 0.f) continue;
+    const float now = m == -INFINITY ? l : expf(m - top);  // (a sum that is no number makes all of the row none)
+    sum += l * now;
 #pragma unroll
-        for (int u = 0; u < 2; ++u)
-#pragma unroll
-          for (int t = 0; t < TILES; ++t) kf[buf][u][t] = *reinterpret_cast<const f32x4*>(kr[t] + min(d + 16 * u, D - 16));
-      };
-      auto score = [&](int buf, int d, int u) {
-        const f32x4 qf = *reinterpret_cast<const f32x4*>(&qs[r16 * (D + 4) + d + 16 * u + 4 * g]);
-#pragma unroll
-        for (int j = 0; j < 4; ++j)
-#pragma unroll
-          for (int t = 0; t < TILES; ++t) s[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[buf][u][t][j], qf[j], s[t], 0, 0, 0);
-      };
-      ask(0, 0);
-#pragma unroll
-      for (int t = 0; t < TILES; ++t)
-#pragma unroll
-        for (int i = 0; i < 4; ++i) vf[t][i] = *reinterpret_cast<const f32x4*>(vr[t][i]);
-      int d = 0;
-      for (; d + 64 <= D; d += 64) {
-        ask(1, d + 32);
-        score(0, d, 0);
-        score(0, d, 1);
-        ask(0, d + 64);
-        score(1, d + 32, 0);
-        score(1, d + 32, 1);
-      }
-      if (d < D) {                                       // 16, 32 or 48 entries more
-        ask(1, d + 32);
-        score(0, d, 0);
-        if (d + 16 < D) score(0, d, 1);
-        if (d + 32 < D) score(1, d + 32, 0);
-      }
-      // s[t][i]: key kb + 16 t + 4 g + i against row r16
-      float m = -INFINITY;
-#pragma unroll
-      for (int t = 0; t < TILES; ++t)
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const int key = kb + 16 * t + 4 * g + i;
-          float z = s[t][i] * a.scale;
-          if (a.cap > 0.f) z = a.cap * tanhf(z / a.cap);
-          if (a.slopes) z = fmaf(-slope, (float)(pos - key), z);
-          s[t][i] = key >= lo && key <= pos ? z : -INFINITY;
-          m = fmaxf(m, s[t][i]);
-        }
-      m = fmaxf(m, __shfl_xor(m, 16, NHV_WAVE));
-      m = fmaxf(m, __shfl_xor(m, 32, NHV_WAVE));
-      const float base = m == -INFINITY ? 0.f : m;       // (no visible key: every weight is 0)
-      float l = 0.f;
-#pragma unroll
-      for (int t = 0; t < TILES; ++t)
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          s[t][i] = expf(s[t][i] - base);
-          l += s[t][i];
-        }
-      l += __shfl_xor(l, 16, NHV_WAVE);
-      l += __shfl_xor(l, 32, NHV_WAVE);
-      if (g == 0) {
-        stats[(wave * ROWS + r16) * 2] = m;
-        stats[(wave * ROWS + r16) * 2 + 1] = l;
-      }
-      // value entry h + 4 r + j of a chunk of 64 is row r of matrix tile j: one load of 16 bytes a key feeds four tiles. The next
-      // chunk is asked for as this one is used up.
-      for (int h = 0; h < E; h += 64) {
-        const int next = min(h + 64, E - 64);
-        f32x4 o[4];
-#pragma unroll
-        for (int j = 0; j < 4; ++j) o[j] = f32x4{0.f, 0.f, 0.f, 0.f};
-        float odd = 0.f;                                 // not a number as soon as some value is infinite or none
-#pragma unroll
-        for (int t = 0; t < TILES; ++t)
-#pragma unroll
-          for (int i = 0; i < 4; ++i) {
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-              odd = fmaf(vf[t][i][j], 0.f, odd);
-              o[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(vf[t][i][j], s[t][i], o[j], 0, 0, 0);
-            }
-            vf[t][i] = *reinterpret_cast<const f32x4*>(vr[t][i] + next);
-          }
-        // o[j][i]: row r16, entry h + 16 g + 4 i + j
-        if (__any(odd != 0.f)) {
-          // a value that is no finite number: it must not reach the rows that do not read it (0 times it is not 0)
-#pragma unroll
-          for (int j = 0; j < 4; ++j) o[j] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-          for (int t = 0; t < TILES; ++t)
-#pragma unroll
-            for (int i = 0; i < 4; ++i)
-              for (int gk = 0; gk < 4; ++gk) {
-                const int at = __shfl(slot, 16 * t + 4 * gk + i, NHV_WAVE);
-                const float p = __shfl(s[t][i], 16 * gk + r16, NHV_WAVE);
-                if (p != 0.f) {
-                  const float* row_v = a.v + ((size_t)at * a.Hkv + kvh) * E + h + 16 * g;
-#pragma unroll
-                  for (int ii = 0; ii < 4; ++ii)
-#pragma unroll
-                    for (int j = 0; j < 4; ++j) o[j][ii] = fmaf(p, row_v[4 * ii + j], o[j][ii]);
-                }
-              }
-        }
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-          *reinterpret_cast<f32x4*>(&part[(wave * ROWS + r16) * (E + 4) + h + 16 * g + 4 * i]) = f32x4{o[0][i], o[1][i], o[2][i], o[3][i]};
-      }
-    }
-    __syncthreads();
-    for (int p = 0; p < WAVES && round + p * KEYS <= tile_hi; ++p) {
-      const float m = stats[(p * ROWS + my_row) * 2], l = stats[(p * ROWS + my_row) * 2 + 1];
-      // a block of which this row reads no key, or none with a weight. (The maximum alone does not say that: fmaxf passes over a
-      // score that is no number, and where all are such the sum of the weights tells.)
-      if (m == -INFINITY && l == 0.f) continue;
-      const float top = fmaxf(M, m), old = expf(M - top), now = expf(m - top);
-      L = L * old + l * now;
-      M = top;
-#pragma unroll
-      for (int i = 0; i < MAX_E / (4 * WAVES); ++i)
-        if (4 * WAVES * i < E) total[i] = total[i] * old + part[(p * ROWS + my_row) * (E + 4) + c + 4 * WAVES * i] * now;
-    }
-    __syncthreads();
+    for (int i = 0; i < 2 * CHUNKS; ++i) total[i] = fmaf(part[(p * ROWS + my_row) * (E + 4) + c + 32 * i], now, total[i]);
   }
 
-  if (row0 + my_row >= rows) return;
   const int t = first + (row0 + my_row) / group, h = kvh * group + (row0 + my_row) % group;
   float after = 1.f;
   if (a.has_sink || a.sinks) {                           // one more term of the denominator, without a value
     const float z = a.sinks ? a.sinks[h] : a.sink;
-    const float top = fmaxf(M, z);
-    after = expf(M - top);
-    L = L * after + expf(z - top);
+    const float most = fmaxf(top, z);
+    after = expf(top - most);
+    sum = sum * after + expf(z - most);
   }
-  float inv = after / L;
+  float inv = after / sum;
   if (a.gate) inv /= 1.0f + expf(-a.gate[(size_t)t * a.gate_ld + h]);
-  float* o = a.out + ((size_t)t * a.Hq + h) * E;
+  float* out = a.out + ((size_t)t * a.Hq + h) * E;
 #pragma unroll
-  for (int i = 0; i < MAX_E / (4 * WAVES); ++i)
-    if (4 * WAVES * i < E) o[c + 4 * WAVES * i] = total[i] * inv;
+  for (int i = 0; i < 2 * CHUNKS; ++i) out[c + 32 * i] = total[i] * inv;
+}
+
+template <int CHUNKS>
+static int launch(const FloatAttention& a, dim3 grid, size_t lds, hipStream_t s) {
+  static const hipError_t allowed = hipFuncSetAttribute((const void*)attention_float32_kernel<CHUNKS>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                                        (int)((ROWS * (MAX_D + 4) + WAVES * ROWS * (64 * CHUNKS + 4) + WAVES * ROWS * 2) * sizeof(float)));
+  if (allowed != hipSuccess) return nhv_fail("attention: %zu bytes of LDS are refused: %s", lds, hipGetErrorString(allowed));
+  hipLaunchKernelGGL(attention_float32_kernel<CHUNKS>, grid, dim3(64 * WAVES), lds, s, a);
+  NHV_LAUNCH_CHECK("attention_float32");
+  return 0;
 }
 
 extern "C" int nhv_attention_float32(const void* q, const void* k_cache, const void* v_cache, void* out, const void* positions,
@@ -257,10 +287,10 @@ extern "C" int nhv_attention_float32(const void* q, const void* k_cache, const v
                             (const int*)cu_seqlens_q, (const int*)block_tables, max_blocks, Hq, Hkv, D, E, page_size, scale, window, chunk,
                             cap, has_sink, sink, (const float*)sinks, (const float*)slopes, (const float*)gate, gate_ld};
   const size_t lds = (ROWS * (D + 4) + WAVES * ROWS * (E + 4) + WAVES * ROWS * 2) * sizeof(float);
-  static const hipError_t allowed = hipFuncSetAttribute((const void*)attention_float32_kernel, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                                        (int)((ROWS * (MAX_D + 4) + WAVES * ROWS * (MAX_E + 4) + WAVES * ROWS * 2) * sizeof(float)));
-  if (allowed != hipSuccess) return nhv_fail("attention: %zu bytes of LDS are refused: %s", lds, hipGetErrorString(allowed));
-  hipLaunchKernelGGL(attention_float32_kernel, dim3((unsigned)tiles, Hkv, B), dim3(64 * WAVES), lds, (hipStream_t)stream, a);
-  NHV_LAUNCH_CHECK("attention_float32");
-  return 0;
+  switch (E / 64) {
+    case 1: return launch<1>(a, dim3((unsigned)tiles, Hkv, B), lds, (hipStream_t)stream);
+    case 2: return launch<2>(a, dim3((unsigned)tiles, Hkv, B), lds, (hipStream_t)stream);
+    case 3: return launch<3>(a, dim3((unsigned)tiles, Hkv, B), lds, (hipStream_t)stream);
+    default: return launch<4>(a, dim3((unsigned)tiles, Hkv, B), lds, (hipStream_t)stream);
+  }
 }
