@@ -1,4 +1,4 @@
-// y[M, N] = x[M, K] . w[N, K]^T (+ bias[N]) in float, on the bfloat16 matrix cores without losing any of the 32 bits.
+// y[M, N] = x[M, K] . w[N, K]^T (+ bias[N]) in float, or a gate of two such products (w[2 N, K]: N gate rows, then N up rows), on the bfloat16 matrix cores without losing any of the 32 bits.
 //
 // A float is the sum of three bfloat16 numbers, exactly: what rounding to 8 bits gives, what that leaves rounded to 8 bits, and
 // the rest (nhv_split_float.h). A product of two floats is then nine products of 8 bits by 8, each exact in float; six of them
@@ -23,7 +23,10 @@
 // grows by 5.6 us a 3,072 k with every 16 rows of x or w that it reads (35 GB/s), whatever their product. Many rows: a block is
 // 4 waves that share their operands' parts through LDS, see below.
 // The blocks of one column tile follow each other on one XCD, whose L2 then reads those rows of w once.
+// A gated product takes tiles of gate rows and of their up rows in turn (two a wave), and a lane that has finished both writes
+// the gate of them: what a kernel of its own made of the packed rows before (6 rows of 3,072: 4.1 us, 517: 5.5).
 #include "nhv_common.h"
+#include "nhv_gates.h"
 #include "nhv_split_float.h"
 
 #define SEGMENTS 8
@@ -59,15 +62,17 @@ __device__ __attribute__((noinline)) float plain_product(const float* __restrict
 
 __device__ __forceinline__ bool finite(float v) { return fabsf(v) < INFINITY; }
 
-template <int RT, int CT, int U, bool WIDE>
+template <int RT, int CT, int U, bool GATED, bool WIDE>
 __global__ __launch_bounds__(64 * SEGMENTS) void gemm_float32_kernel(const float* __restrict__ x, const float* __restrict__ w,
                                                                      const float* __restrict__ bias, float* __restrict__ y,
-                                                                     int M, int N, int K, int m_tiles, int n_tiles) {
+                                                                     int M, int N, int K, int m_tiles, int n_tiles, NhvGate gate) {
+  static_assert(!GATED || CT == 2, "a gate tile and its up tile");
+  constexpr int COLS = GATED ? 16 : 16 * CT;             // outputs of a row
   __shared__ __attribute__((aligned(16))) float part[SEGMENTS][CT * 256];
   const int total = m_tiles * n_tiles, share = (total + 7) >> 3;
   const int tile = (blockIdx.x & 7) * share + (blockIdx.x >> 3);        // (consecutive blocks go round the 8 XCDs)
   if (tile >= total) return;
-  const int m0 = (tile % m_tiles) * 16 * RT, n0 = (tile / m_tiles) * 16 * CT;
+  const int m0 = (tile % m_tiles) * 16 * RT, n0 = (tile / m_tiles) * COLS;
   const int s = threadIdx.x >> 6, lane = threadIdx.x & 63, r16 = lane & 15, g = lane >> 4;
   const int length = segment_length(K);
   const int begin = s * length, end = min(K, begin + length);
@@ -88,7 +93,7 @@ __global__ __launch_bounds__(64 * SEGMENTS) void gemm_float32_kernel(const float
 #pragma unroll
     for (int r = 0; r < RT; ++r) xp[r] = x + (size_t)min(m0 + 16 * r + r16, M - 1) * K;
 #pragma unroll
-    for (int c = 0; c < CT; ++c) wp[c] = w + (size_t)min(n0 + 16 * c + r16, N - 1) * K;
+    for (int c = 0; c < CT; ++c) wp[c] = w + (GATED ? (size_t)c * N + min(n0 + r16, N - 1) : (size_t)min(n0 + 16 * c + r16, N - 1)) * K;
     f32x4 a[2][U][RT][2], b[2][U][CT][2];
     auto ask = [&](int buf, int k0) {
 #pragma unroll
@@ -167,29 +172,37 @@ __global__ __launch_bounds__(64 * SEGMENTS) void gemm_float32_kernel(const float
 #pragma unroll
     for (int c = 0; c < CT; ++c) *reinterpret_cast<f32x4*>(&part[s][(c * 64 + lane) * 4]) = acc[r][c];
     __syncthreads();
-    for (int i = threadIdx.x; i < 256 * CT; i += 64 * SEGMENTS) {
+    for (int i = threadIdx.x; i < 16 * COLS; i += 64 * SEGMENTS) {
       // (lane 16 g + n of a tile holds rows 4 g .. 4 g + 3 of column n)
-      const int c = i % (16 * CT), row = i / (16 * CT);
-      const int at = ((c >> 4) * 64 + (row >> 2) * 16 + (c & 15)) * 4 + (row & 3);
-      float v = part[0][at];
-      for (int p = 1; p < active; ++p) v += part[p][at];
-      const int m = m0 + 16 * r + row, n = n0 + c;
+      const int c = i % COLS, row = i / COLS, m = m0 + 16 * r + row, n = n0 + c;
+      float v[GATED ? 2 : 1];
+#pragma unroll
+      for (int both = 0; both < (GATED ? 2 : 1); ++both) {
+        const int at = (((c >> 4) + both) * 64 + (row >> 2) * 16 + (c & 15)) * 4 + (row & 3);
+        v[both] = part[0][at];
+        for (int p = 1; p < active; ++p) v[both] += part[p][at];
+      }
       if (m < M && n < N) {
-        if (!finite(v)) v = plain_product(x + (size_t)m * K, w + (size_t)n * K, K);
-        y[(size_t)m * N + n] = bias ? v + bias[n] : v;
+#pragma unroll
+        for (int both = 0; both < (GATED ? 2 : 1); ++both) {
+          if (!finite(v[both])) v[both] = plain_product(x + (size_t)m * K, w + ((size_t)both * N + n) * K, K);
+          if (bias) v[both] += bias[both * N + n];
+        }
+        y[(size_t)m * N + n] = GATED ? nhv_gated(v[0], v[GATED], gate) : v[0];
       }
     }
   }
 }
 
-template <int RT, int CT, int U>
-static void launch(const float* x, const float* w, const float* bias, float* y, int M, int N, int K, hipStream_t s) {
-  const int m_tiles = (M + 16 * RT - 1) / (16 * RT), n_tiles = (N + 16 * CT - 1) / (16 * CT);
+template <int RT, int CT, int U, bool GATED>
+static void launch(const float* x, const float* w, const float* bias, float* y, int M, int N, int K, const NhvGate& gate, hipStream_t s) {
+  constexpr int COLS = GATED ? 16 : 16 * CT;
+  const int m_tiles = (M + 16 * RT - 1) / (16 * RT), n_tiles = (N + COLS - 1) / COLS;
   const dim3 grid(8u * (unsigned)(((long long)m_tiles * n_tiles + 7) / 8)), block(64 * SEGMENTS);
   if (K % 4 == 0 && (uintptr_t)x % 16 == 0 && (uintptr_t)w % 16 == 0)
-    hipLaunchKernelGGL((gemm_float32_kernel<RT, CT, U, true>), grid, block, 0, s, x, w, bias, y, M, N, K, m_tiles, n_tiles);
+    hipLaunchKernelGGL((gemm_float32_kernel<RT, CT, U, GATED, true>), grid, block, 0, s, x, w, bias, y, M, N, K, m_tiles, n_tiles, gate);
   else
-    hipLaunchKernelGGL((gemm_float32_kernel<RT, CT, U, false>), grid, block, 0, s, x, w, bias, y, M, N, K, m_tiles, n_tiles);
+    hipLaunchKernelGGL((gemm_float32_kernel<RT, CT, U, GATED, false>), grid, block, 0, s, x, w, bias, y, M, N, K, m_tiles, n_tiles, gate);
 }
 
 // ---------------------------------------------------------------- many rows
@@ -202,16 +215,17 @@ static void launch(const float* x, const float* w, const float* bias, float* y, 
 // float matrix instructions 672).
 #define PIECE 32
 #define AHEAD 2
-template <int RT, int CT, bool WIDE>
+template <int RT, int CT, bool GATED, bool WIDE>
 __global__ __launch_bounds__(256, RT * CT > 2 ? 3 : 4) void gemm_float32_tiles_kernel(const float* __restrict__ x, const float* __restrict__ w,
                                                                  const float* __restrict__ bias, float* __restrict__ y, int M, int N,
-                                                                 int K, int m_tiles, int n_tiles) {
+                                                                 int K, int m_tiles, int n_tiles, NhvGate gate) {
+  static_assert(!GATED || CT == 2, "a gate tile and its up tile");
   constexpr int BM = 32 * RT, BN = 32 * CT, LOADS = (BM + BN) * PIECE / 4 / 256, PLANE = (BM + BN) * PIECE;
   __shared__ __attribute__((aligned(16))) bf16_t rows[2][3 * PLANE];
   const int total_tiles = m_tiles * n_tiles, share = (total_tiles + 7) >> 3;
   const int tile = (blockIdx.x & 7) * share + (blockIdx.x >> 3);
   if (tile >= total_tiles) return;
-  const int m0 = (tile % m_tiles) * BM, n0 = (tile / m_tiles) * BN;
+  const int m0 = (tile % m_tiles) * BM, n0 = (tile / m_tiles) * (GATED ? BN / 2 : BN);
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, r16 = lane & 15, g = lane >> 4;
   const int mw = (wave >> 1) * 16 * RT, nw = (wave & 1) * 16 * CT;
   const int length = segment_length(K), at = (g ^ (r16 >> 2)) << 3;
@@ -221,7 +235,9 @@ __global__ __launch_bounds__(256, RT * CT > 2 ? 3 : 4) void gemm_float32_tiles_k
 #pragma unroll
   for (int i = 0; i < LOADS; ++i) {
     const int r = (threadIdx.x >> 3) + 32 * i;
-    src[i] = r < BM ? x + (size_t)min(m0 + r, M - 1) * K : w + (size_t)min(n0 + r - BM, N - 1) * K;
+    // (gated: 16 gate rows and their 16 up rows in turn)
+    const int n = GATED ? n0 + ((r - BM) >> 5) * 16 + (r & 15) : n0 + r - BM, up = GATED ? (r >> 4) & 1 : 0;
+    src[i] = r < BM ? x + (size_t)min(m0 + r, M - 1) * K : w + ((size_t)up * N + min(n, N - 1)) * K;
   }
   // where they go: lane group g of a product takes k = 4 g .. and 16 + 4 g .., 16 bytes together, whose place in the row's 64
   // turns with the row so that 16 rows lie in different banks
@@ -301,29 +317,34 @@ __global__ __launch_bounds__(256, RT * CT > 2 ? 3 : 4) void gemm_float32_tiles_k
 #pragma unroll
   for (int r = 0; r < RT; ++r)
 #pragma unroll
-    for (int c = 0; c < CT; ++c) {
-      const int n = n0 + nw + 16 * c + r16;
-      const float add = bias && n < N ? bias[n] : 0.f;
+    for (int c = 0; c < CT; c += GATED ? 2 : 1) {
+      const int n = n0 + (GATED ? nw / 2 : nw + 16 * c) + r16;
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         const int m = m0 + mw + 16 * r + 4 * g + i;
         if (m < M && n < N) {
-          float v = total[r][c][i];
-          if (!finite(v)) v = plain_product(x + (size_t)m * K, w + (size_t)n * K, K);
-          y[(size_t)m * N + n] = bias ? v + add : v;
+          float v[GATED ? 2 : 1];
+#pragma unroll
+          for (int both = 0; both < (GATED ? 2 : 1); ++both) {
+            v[both] = total[r][c + both][i];
+            if (!finite(v[both])) v[both] = plain_product(x + (size_t)m * K, w + ((size_t)both * N + n) * K, K);
+            if (bias) v[both] += bias[both * N + n];
+          }
+          y[(size_t)m * N + n] = GATED ? nhv_gated(v[0], v[GATED], gate) : v[0];
         }
       }
     }
 }
 
-template <int RT, int CT>
-static void launch_tiles(const float* x, const float* w, const float* bias, float* y, int M, int N, int K, hipStream_t s) {
-  const int m_tiles = (M + 32 * RT - 1) / (32 * RT), n_tiles = (N + 32 * CT - 1) / (32 * CT);
+template <int RT, int CT, bool GATED>
+static void launch_tiles(const float* x, const float* w, const float* bias, float* y, int M, int N, int K, const NhvGate& gate, hipStream_t s) {
+  constexpr int COLS = GATED ? 16 * CT : 32 * CT;
+  const int m_tiles = (M + 32 * RT - 1) / (32 * RT), n_tiles = (N + COLS - 1) / COLS;
   const dim3 grid(8u * (unsigned)(((long long)m_tiles * n_tiles + 7) / 8)), block(256);
   if (K % 4 == 0 && (uintptr_t)x % 16 == 0 && (uintptr_t)w % 16 == 0)
-    hipLaunchKernelGGL((gemm_float32_tiles_kernel<RT, CT, true>), grid, block, 0, s, x, w, bias, y, M, N, K, m_tiles, n_tiles);
+    hipLaunchKernelGGL((gemm_float32_tiles_kernel<RT, CT, GATED, true>), grid, block, 0, s, x, w, bias, y, M, N, K, m_tiles, n_tiles, gate);
   else
-    hipLaunchKernelGGL((gemm_float32_tiles_kernel<RT, CT, false>), grid, block, 0, s, x, w, bias, y, M, N, K, m_tiles, n_tiles);
+    hipLaunchKernelGGL((gemm_float32_tiles_kernel<RT, CT, GATED, false>), grid, block, 0, s, x, w, bias, y, M, N, K, m_tiles, n_tiles, gate);
 }
 
 extern "C" int nhv_gemm_float32(const void* x, const void* w, const void* bias, void* y, int M, int N, int K, void* stream) {
@@ -348,13 +369,44 @@ extern "C" int nhv_gemm_float32(const void* x, const void* w, const void* bias, 
   for (int i = 1; i < 6; ++i)
     if (cost[i] < cost[best]) best = i;
   switch (best) {
-    case 0: launch<1, 1, 2>(xf, wf, bf, yf, M, N, K, s); break;
-    case 1: launch<1, 2, 1>(xf, wf, bf, yf, M, N, K, s); break;
-    case 2: launch<2, 2, 1>(xf, wf, bf, yf, M, N, K, s); break;
-    case 3: launch<3, 2, 1>(xf, wf, bf, yf, M, N, K, s); break;
-    case 4: launch_tiles<1, 1>(xf, wf, bf, yf, M, N, K, s); break;
-    default: launch_tiles<2, 2>(xf, wf, bf, yf, M, N, K, s);
+    case 0: launch<1, 1, 2, false>(xf, wf, bf, yf, M, N, K, {}, s); break;
+    case 1: launch<1, 2, 1, false>(xf, wf, bf, yf, M, N, K, {}, s); break;
+    case 2: launch<2, 2, 1, false>(xf, wf, bf, yf, M, N, K, {}, s); break;
+    case 3: launch<3, 2, 1, false>(xf, wf, bf, yf, M, N, K, {}, s); break;
+    case 4: launch_tiles<1, 1, false>(xf, wf, bf, yf, M, N, K, {}, s); break;
+    default: launch_tiles<2, 2, false>(xf, wf, bf, yf, M, N, K, {}, s);
   }
   NHV_LAUNCH_CHECK("gemm_float32");
+  return 0;
+}
+
+extern "C" int nhv_gemm_float32_gated(const void* x, const void* w, const void* bias, void* y, int M, int N, int K, int act, float limit,
+                                      float alpha, float offset, void* stream) {
+  NHV_REQUIRE(M > 0 && N > 0 && K > 0, "gated gemm: bad sizes M=%d N=%d K=%d", M, N, K);
+  NHV_REQUIRE(K < (1 << 30) && N < (1 << 30) && (((long long)M + 15) / 16) * (((long long)N + 15) / 16) < (1ll << 30),
+              "gated gemm: too many rows (%d) for %d columns", M, N);
+  NHV_REQUIRE(act >= 0 && act <= 2, "gated gemm: unknown gate %d", act);
+  hipStream_t s = (hipStream_t)stream;
+  const NhvGate gate = {act, limit, alpha, offset};
+  const float *xf = (const float*)x, *wf = (const float*)w, *bf = (const float*)bias;
+  float* yf = (float*)y;
+  // as above, a column counting for two rows of w; through LDS only tiles with a pair a wave
+  auto blocks = [&](long long m, long long n) { return ((M + m - 1) / m) * ((N + n - 1) / n); };
+  auto rounds = [&](int rt) { return (double)((blocks(16 * rt, 16) + 255) / 256 * (rt + 2)); };
+  const double none = 1e300;
+  const double cost[5] = {rounds(1), M > 16 ? rounds(2) : none, M > 32 ? rounds(3) : none,
+                          M > 16 ? fmax(9.5, 3.0 + 4.9 / 256 * blocks(32, 32)) : none,
+                          M > 16 ? fmax(11.5, 4.5 + 7.7 / 256 * blocks(64, 32)) : none};
+  int best = 0;
+  for (int i = 1; i < 5; ++i)
+    if (cost[i] < cost[best]) best = i;
+  switch (best) {
+    case 0: launch<1, 2, 1, true>(xf, wf, bf, yf, M, N, K, gate, s); break;
+    case 1: launch<2, 2, 1, true>(xf, wf, bf, yf, M, N, K, gate, s); break;
+    case 2: launch<3, 2, 1, true>(xf, wf, bf, yf, M, N, K, gate, s); break;
+    case 3: launch_tiles<1, 2, true>(xf, wf, bf, yf, M, N, K, gate, s); break;
+    default: launch_tiles<2, 2, true>(xf, wf, bf, yf, M, N, K, gate, s);
+  }
+  NHV_LAUNCH_CHECK("gemm_float32_gated");
   return 0;
 }

@@ -886,8 +886,11 @@ class NativeBackend:
 
     def gated_linear(self, x, w, out, gate=None, bias=None) -> bool:
         """A gate (a ``Gate``; None: SiLU) of x Wg^T and x Wu^T (+ bias) in one kernel, if this batch is one for the
-        few-rows kernel; else False. (SiLU without bias may also be one for the kernel of up to 64 rows.)"""
+        few-rows kernel; else False. (SiLU without bias may also be one for the kernel of up to 64 rows; in float32 every batch is.)"""
         M, K = x.shape
+        if x.dtype == torch.float32:
+            self._call("nhv_gemm_float32_gated", _ptr(x), _ptr(w), _ptr(bias), _ptr(out), M, out.shape[1], K, *(gate or Gate()).args(), _stream())
+            return True
         if bias is not None or (gate is not None and gate.act != 0):
             if x.dtype == torch.bfloat16 and K % 8 == 0 and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0 and M <= self.few_rows:
                 self._call("nhv_gemm_fewrows_gated_bf16", _ptr(x), _ptr(w), _ptr(bias), _ptr(out), M, out.shape[1], K,

@@ -333,6 +333,21 @@ def test_float32_linear_at_the_ends_of_its_range(ops, M, N, K):
     assert ((got - want).abs()[near] <= (K * 2.0 ** -24 * size)[near]).all()
 
 
+@pytest.mark.parametrize("N,K", [(1, 7), (40, 516), (520, 1024), (3072, 64), (9000, 36)])
+def test_float32_gated_linear_in_all_its_tiles(ops, N, K):
+    """A gate of two products in one kernel: the bits of the packed product and the gate's own kernel, for every tile that the
+    sizes can choose, with and without biases, and with an infinite row."""
+    x, w, b = rnd(300, K, seed=64), rnd(2 * N, K, seed=65), rnd(2 * N, seed=66)
+    for M in (300, 130, 70, 40, 17, 16, 3):
+        rows = x[300 - M:].contiguous()
+        if M == 40:
+            rows[M // 2, K // 2] = float("inf")
+        for gate, bias in (("silu", None), (ops.Gate(2, 3.0, 1.702, 1.0), b)):
+            packed = ops.linear(rows, w)
+            got, want = ops.gated_linear(rows, w, gate, bias), ops.act_mul(packed, gate, bias)
+            assert torch.equal(got.isnan(), want.isnan()) and torch.equal(got.nan_to_num(1.5, 2.5, 3.5), want.nan_to_num(1.5, 2.5, 3.5)), (M, gate)
+
+
 def test_linear_rows_do_not_depend_on_the_batch_in_float32(ops):
     x = rnd(70, 200, seed=7)
     w = rnd(150, 200, seed=8)
