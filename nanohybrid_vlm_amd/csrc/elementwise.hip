@@ -102,6 +102,117 @@ __device__ __forceinline__ void store8f<float>(float* p, const float* in) {
   *reinterpret_cast<float4*>(p + 4) = make_float4(in[4], in[5], in[6], in[7]);
 }
 
+// Eight entries of a product that comes as float parts (gemm_lines_bf16.hip), `stride` entries apart, added in their order; all
+// parts are asked for before the first is used.
+template <int SPLITS>
+__device__ __forceinline__ void add_parts8(const float* p, size_t stride, float* out) {
+  float part[SPLITS][8];
+#pragma unroll
+  for (int s = 0; s < SPLITS; ++s) load8f<float>(p + s * stride, part[s]);
+#pragma unroll
+  for (int e = 0; e < 8; ++e) {
+    out[e] = part[0][e];
+#pragma unroll
+    for (int s = 1; s < SPLITS; ++s) out[e] += part[s][e];
+  }
+}
+__device__ __forceinline__ void add_parts8(const float* p, size_t stride, int splits, float* out) {
+  if (splits == 8) add_parts8<8>(p, stride, out);
+  else if (splits == 4) add_parts8<4>(p, stride, out);
+  else if (splits == 2) add_parts8<2>(p, stride, out);
+  else add_parts8<1>(p, stride, out);
+}
+
+// residual += the product whose parts these are (not rounded in between); y = the norm of the sum: what rmsnorm does with mode 1.
+// Four parts cost it nothing that can be seen: 64 rows of 4,096 entries 4.8 us, of a bfloat16 product 5.1.
+template <typename W, typename R, int MAXC>
+__global__ __launch_bounds__(1024) void add_parts_norm_kernel(const float* __restrict__ parts, int splits, R* __restrict__ residual,
+                                                              const W* __restrict__ w, bf16_t* __restrict__ y, int H, float eps, int rounds_between) {
+  __shared__ float scratch[16];
+  const size_t base = (size_t)blockIdx.x * H, stride = (size_t)gridDim.x * H;
+  const int nch = H / 8;
+  float v[MAXC][8], wv[MAXC][8];
+  float ss = 0.f;
+#pragma unroll
+  for (int c = 0; c < MAXC; ++c) {
+    const int ch = threadIdx.x + c * blockDim.x;
+    if (ch < nch) {
+      float r8[8];
+      load8f<R>(residual + base + ch * 8, r8);
+      load8f<W>(w + ch * 8, wv[c]);
+      add_parts8(parts + base + ch * 8, stride, splits, v[c]);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) v[c][e] += r8[e];
+    } else {
+#pragma unroll
+      for (int e = 0; e < 8; ++e) v[c][e] = 0.f;
+    }
+  }
+#pragma unroll
+  for (int c = 0; c < MAXC; ++c) {
+    const int ch = threadIdx.x + c * blockDim.x;
+    if (ch < nch) store8f<R>(residual + base + ch * 8, v[c]);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) ss += v[c][e] * v[c][e];
+  }
+  const float total = block_sum(ss, scratch);
+  const float r = 1.0f / sqrtf(total / (float)H + eps);
+#pragma unroll
+  for (int c = 0; c < MAXC; ++c) {
+    const int ch = threadIdx.x + c * blockDim.x;
+    if (ch < nch) {
+      float o[8];
+#pragma unroll
+      for (int e = 0; e < 8; ++e) o[e] = (rounds_between ? (float)(bf16_t)(v[c][e] * r) : v[c][e] * r) * wv[c][e];
+      store8f<bf16_t>(y + base + ch * 8, o);
+    }
+  }
+}
+
+extern "C" int nhv_add_parts_norm(const void* parts, int splits, void* residual, int residual_dtype, const void* w, void* y, int T, int H, float eps,
+                                  int rounds_between, int w_dtype, void* stream) {
+  NHV_REQUIRE(T > 0 && H > 0 && H % 8 == 0 && H <= 16384, "add_parts_norm: bad sizes T=%d H=%d", T, H);
+  NHV_REQUIRE(splits == 1 || splits == 2 || splits == 4 || splits == 8, "add_parts_norm: %d parts", splits);
+  NHV_REQUIRE((((uintptr_t)parts | (uintptr_t)residual | (uintptr_t)w | (uintptr_t)y) & 15) == 0, "add_parts_norm: rows off 16-byte boundaries");
+  hipStream_t s = (hipStream_t)stream;
+  const int nch = H / 8, threads = nch <= 1024 ? (nch + 63) / 64 * 64 : 1024;
+#define LAUNCH(WW, RR)                                                                                                                     \
+  do {                                                                                                                                     \
+    if (nch <= 1024)                                                                                                                       \
+      hipLaunchKernelGGL((add_parts_norm_kernel<WW, RR, 1>), dim3(T), dim3(threads), 0, s, (const float*)parts, splits, (RR*)residual,      \
+                         (const WW*)w, (bf16_t*)y, H, eps, rounds_between);                                                                \
+    else                                                                                                                                   \
+      hipLaunchKernelGGL((add_parts_norm_kernel<WW, RR, 2>), dim3(T), dim3(threads), 0, s, (const float*)parts, splits, (RR*)residual,      \
+                         (const WW*)w, (bf16_t*)y, H, eps, rounds_between);                                                                \
+  } while (0)
+  if (w_dtype == NHV_BF16 && residual_dtype == NHV_F32) LAUNCH(bf16_t, float);
+  else if (w_dtype == NHV_F32 && residual_dtype == NHV_F32) LAUNCH(float, float);
+  else if (w_dtype == NHV_BF16 && residual_dtype == NHV_BF16) LAUNCH(bf16_t, bf16_t);
+  else if (w_dtype == NHV_F32 && residual_dtype == NHV_BF16) LAUNCH(float, bf16_t);
+  else return nhv_fail("add_parts_norm: unsupported dtypes w=%d residual=%d", w_dtype, residual_dtype);
+#undef LAUNCH
+  NHV_LAUNCH_CHECK("add_parts_norm");
+  return 0;
+}
+
+// y = the product whose parts these are, rounded once
+__global__ void sum_parts_kernel(const float* __restrict__ parts, int splits, bf16_t* __restrict__ y, size_t n) {
+  for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x) {
+    float v = parts[i];
+    for (int s = 1; s < splits; ++s) v += parts[s * n + i];
+    y[i] = (bf16_t)v;
+  }
+}
+
+extern "C" int nhv_sum_parts(const void* parts, int splits, void* y, size_t n, void* stream) {
+  NHV_REQUIRE(n > 0 && splits > 0, "sum_parts: %d parts of %zu entries", splits, n);
+  const size_t blocks = (n + 255) / 256;
+  hipLaunchKernelGGL(sum_parts_kernel, dim3((unsigned)(blocks < 4096 ? blocks : 4096)), dim3(256), 0, (hipStream_t)stream, (const float*)parts, splits,
+                     (bf16_t*)y, n);
+  NHV_LAUNCH_CHECK("sum_parts");
+  return 0;
+}
+
 template <typename T, typename W, typename R, int MAXC>
 __global__ __launch_bounds__(1024) void rmsnorm_vec_kernel(const T* __restrict__ x, R* __restrict__ residual, int residual_mode,
                                                            const W* __restrict__ w, T* __restrict__ y, int H, float eps, int rounds_between) {
@@ -381,10 +492,11 @@ __global__ void qk_rope_write_kernel(const T* __restrict__ qkv, const T* __restr
 
 // The same for head sizes that are a power of two (and full or no rotation): CH = D / 8 lanes own a head, eight
 // consecutive entries each; the norm's sum and the rotation's partner (entry d +- D/2) come by lane shuffles, nothing
-// goes through LDS, and a wave works on 64 / CH heads at once.
-template <typename T, typename W, int CH>
+// goes through LDS, and a wave works on 64 / CH heads at once. PARTS: the projection comes as `splits` float parts,
+// `part_stride` entries apart, whose sums are not rounded before the norm (64 rows of the 8B shape: 4.8 us with and without).
+template <typename T, typename W, int CH, bool PARTS>
 __global__ __launch_bounds__(256) void qk_rope_write_vec_kernel(
-    const T* __restrict__ qkv, const T* __restrict__ bias, const W* __restrict__ q_norm_w, const W* __restrict__ k_norm_w,
+    const void* __restrict__ qkv, int splits, size_t part_stride, const T* __restrict__ bias, const W* __restrict__ q_norm_w, const W* __restrict__ k_norm_w,
     float eps, const float* __restrict__ cos_sin, int rot, const int* __restrict__ positions,
     const int* __restrict__ slot_mapping, T* __restrict__ q_out, T* __restrict__ k_cache, T* __restrict__ v_cache, int Hq,
     int Hkv, int heads_per_token, long long n_items) {
@@ -400,7 +512,9 @@ __global__ __launch_bounds__(256) void qk_rope_write_vec_kernel(
   // everything that does not hang on another load is asked for before anything is looked at (a key's or value's
   // slot used to be waited for before its entries were asked for, one trip to memory after the other)
   float v[8];
-  load8f<T>(qkv + (size_t)t * width + (size_t)h * D + c * 8, v);
+  const size_t at = (size_t)t * width + (size_t)h * D + c * 8;
+  if (PARTS) add_parts8((const float*)qkv + at, part_stride, splits, v);
+  else load8f<T>((const T*)qkv + at, v);
   const int pos = rot > 0 ? positions[t] : 0;
   int slot = -1;
   if (!is_q) {
@@ -454,7 +568,9 @@ __global__ __launch_bounds__(256) void qk_rope_write_vec_kernel(
   store8f<T>(dst + c * 8, o);
 }
 
-extern "C" int nhv_qk_rope_write(const void* qkv, const void* bias, const void* q_norm_w, const void* k_norm_w, float eps,
+// splits > 0: qkv is that many float parts [splits][T][width] of a bfloat16 projection (1, 2, 4 or 8; head sizes that are a power of two, 16 to
+// 512, full rotation or none)
+extern "C" int nhv_qk_rope_write(const void* qkv, int splits, const void* bias, const void* q_norm_w, const void* k_norm_w, float eps,
                                  const void* cos_sin, int rot, int max_pos, const void* positions, const void* pair_axes,
                                  const void* slot_mapping, void* q_out, void* k_cache, void* v_cache, int T, int Hq,
                                  int Hkv, int D, int write_kv, int dtype, int w_dtype, void* stream) {
@@ -464,6 +580,7 @@ extern "C" int nhv_qk_rope_write(const void* qkv, const void* bias, const void* 
   NHV_REQUIRE(D <= 4096, "qk_rope_write: head size %d is beyond this kernel's limit of 4096", D);
   NHV_REQUIRE((q_norm_w == nullptr) == (k_norm_w == nullptr), "qk_rope_write: q and k norm weights come together");
   NHV_REQUIRE(!write_kv || (slot_mapping && k_cache && v_cache), "qk_rope_write: cache write without cache");
+  NHV_REQUIRE(splits == 0 || splits == 1 || splits == 2 || splits == 4 || splits == 8, "qk_rope_write: %d parts", splits);
   const int heads = write_kv ? Hq + 2 * Hkv : Hq;
   const size_t lds = (size_t)D * sizeof(float);
   hipStream_t s = (hipStream_t)stream;
@@ -477,29 +594,34 @@ extern "C" int nhv_qk_rope_write(const void* qkv, const void* bias, const void* 
     const long long n_items = (long long)T * heads;
     const long long vblocks = (n_items * ch + 255) / 256;
     NHV_REQUIRE(vblocks <= 0x7fffffff, "qk_rope_write: too many tokens");
-#define VLAUNCH(TT, WW, CHN)                                                                                         \
-  hipLaunchKernelGGL((qk_rope_write_vec_kernel<TT, WW, CHN>), dim3((unsigned)vblocks), dim3(256), 0, s, (const TT*)qkv, \
+    const size_t part_stride = (size_t)T * (Hq + 2 * Hkv) * D;
+#define VLAUNCH(TT, WW, CHN, PARTS)                                                                                  \
+  hipLaunchKernelGGL((qk_rope_write_vec_kernel<TT, WW, CHN, PARTS>), dim3((unsigned)vblocks), dim3(256), 0, s, qkv, splits, part_stride, \
                      (const TT*)bias, (const WW*)q_norm_w, (const WW*)k_norm_w, eps, (const float*)cos_sin, rot,     \
                      (const int*)positions, (const int*)slot_mapping, (TT*)q_out, (TT*)k_cache, (TT*)v_cache, Hq, Hkv, \
                      heads, n_items)
-#define VBY_CH(TT, WW)                      \
-  switch (ch) {                             \
-    case 2: VLAUNCH(TT, WW, 2); break;      \
-    case 4: VLAUNCH(TT, WW, 4); break;      \
-    case 8: VLAUNCH(TT, WW, 8); break;      \
-    case 16: VLAUNCH(TT, WW, 16); break;    \
-    case 32: VLAUNCH(TT, WW, 32); break;    \
-    default: VLAUNCH(TT, WW, 64); break;    \
+#define VBY_CH(TT, WW, PARTS)                      \
+  switch (ch) {                                    \
+    case 2: VLAUNCH(TT, WW, 2, PARTS); break;      \
+    case 4: VLAUNCH(TT, WW, 4, PARTS); break;      \
+    case 8: VLAUNCH(TT, WW, 8, PARTS); break;      \
+    case 16: VLAUNCH(TT, WW, 16, PARTS); break;    \
+    case 32: VLAUNCH(TT, WW, 32, PARTS); break;    \
+    default: VLAUNCH(TT, WW, 64, PARTS); break;    \
   }
-    if (dtype == NHV_F32 && w_dtype == NHV_F32) { VBY_CH(float, float) }
-    else if (dtype == NHV_BF16 && w_dtype == NHV_BF16) { VBY_CH(bf16_t, bf16_t) }
-    else if (dtype == NHV_BF16 && w_dtype == NHV_F32) { VBY_CH(bf16_t, float) }
+    if (splits > 0 && dtype == NHV_BF16 && w_dtype == NHV_BF16) { VBY_CH(bf16_t, bf16_t, true) }
+    else if (splits > 0 && dtype == NHV_BF16 && w_dtype == NHV_F32) { VBY_CH(bf16_t, float, true) }
+    else if (splits > 0) return nhv_fail("qk_rope_write: parts of dtype %d", dtype);
+    else if (dtype == NHV_F32 && w_dtype == NHV_F32) { VBY_CH(float, float, false) }
+    else if (dtype == NHV_BF16 && w_dtype == NHV_BF16) { VBY_CH(bf16_t, bf16_t, false) }
+    else if (dtype == NHV_BF16 && w_dtype == NHV_F32) { VBY_CH(bf16_t, float, false) }
     else return nhv_fail("qk_rope_write: unsupported dtypes x=%d w=%d", dtype, w_dtype);
 #undef VBY_CH
 #undef VLAUNCH
     NHV_LAUNCH_CHECK("qk_rope_write");
     return 0;
   }
+  NHV_REQUIRE(splits == 0, "qk_rope_write: parts with head size %d, rotary size %d%s", D, rot, aligned ? "" : ", rows off 16-byte boundaries");
 #define LAUNCH(TT, WW)                                                                                              \
   hipLaunchKernelGGL((qk_rope_write_kernel<TT, WW>), dim3((unsigned)((size_t)T * heads)), dim3(NHV_WAVE), lds, s,  \
                      (const TT*)qkv, (const TT*)bias, (const WW*)q_norm_w, (const WW*)k_norm_w, eps,               \

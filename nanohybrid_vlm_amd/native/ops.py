@@ -18,7 +18,7 @@ import torch
 
 from . import library
 
-CORE_SOURCES = ["error.hip", "elementwise.hip", "gemm_generic.hip", "gemm_float32.hip", "gemm_skinny_bf16.hip", "gemm_fewrows_bf16.hip",
+CORE_SOURCES = ["error.hip", "elementwise.hip", "gemm_generic.hip", "gemm_float32.hip", "gemm_skinny_bf16.hip", "gemm_fewrows_bf16.hip", "gemm_lines_bf16.hip",
                 "attention_generic.hip", "attention_float32.hip", "sampling.hip", "measure.hip", "stream_mixing.hip", "delta_rule.hip", "delta_chunks.hip", "parallel_block.hip", "latent_attention.hip",
                 "routed_experts.hip", "hyper_streams.hip", "head_outputs.hip", "sandwich_norms.hip", "linear_recurrence.hip"]
 BLAS_SOURCES = ["error.hip", "gemm_library.hip"]                                                   # the vendor's matrix library, algorithm by number
@@ -214,14 +214,23 @@ class NativeBackend:
         self._call("nhv_gather_rows", _ptr(x), _ptr(rows), _ptr(out), out.shape[0], x.shape[1], x.shape[0],
                    dtype_code(x), _stream())
 
+    def add_parts_norm(self, parts, residual, w, y, eps, rounds_between=True):
+        S, T, H = parts.shape
+        self._call("nhv_add_parts_norm", _ptr(parts), S, _ptr(residual), dtype_code(residual), _ptr(w), _ptr(y), T, H, ctypes.c_float(eps),
+                   int(rounds_between), dtype_code(w), _stream())
+
+    def sum_parts(self, parts, out):
+        self._call("nhv_sum_parts", _ptr(parts), parts.shape[0], _ptr(out), ctypes.c_size_t(out.numel()), _stream())
+
     def qk_rope_write(self, qkv, bias, q_norm_w, k_norm_w, eps, cos_sin, rot, positions, slot_mapping,
                       q_out, k_cache, v_cache, Hq, Hkv, D, write_kv, pair_axes=None):
-        wd = dtype_code(q_norm_w) if q_norm_w is not None else dtype_code(qkv)
-        self._call("nhv_qk_rope_write", _ptr(qkv), _ptr(bias), _ptr(q_norm_w), _ptr(k_norm_w), ctypes.c_float(eps),
+        """``qkv``: [tokens, width], or the float parts of such a projection [parts, tokens, width]."""
+        wd = dtype_code(q_norm_w) if q_norm_w is not None else dtype_code(q_out)
+        self._call("nhv_qk_rope_write", _ptr(qkv), qkv.shape[0] if qkv.dim() == 3 else 0, _ptr(bias), _ptr(q_norm_w), _ptr(k_norm_w), ctypes.c_float(eps),
                    _ptr(cos_sin), rot, 0 if cos_sin is None else cos_sin.shape[0], _ptr(positions), _ptr(pair_axes),
                    _ptr(slot_mapping),
-                   _ptr(q_out), _ptr(k_cache), _ptr(v_cache), qkv.shape[0], Hq, Hkv, D, int(write_kv),
-                   dtype_code(qkv), wd, _stream())
+                   _ptr(q_out), _ptr(k_cache), _ptr(v_cache), q_out.shape[0], Hq, Hkv, D, int(write_kv),
+                   dtype_code(q_out), wd, _stream())
 
     def paged_attention(self, q, k_cache, v_cache, out, batch: AttentionBatch, block_tables, scale, window, chunk=0,
                         cap=0.0, sink=None, slopes=None, gate=None):
@@ -812,6 +821,25 @@ class NativeBackend:
         self._call("nhv_gemm_generic", _ptr(x), _ptr(w), _ptr(bias), _ptr(out), M, N, K, dtype_code(x),
                    dtype_code(out), _stream())
 
+    def _by_lines(self, x, w, N: int, gated: bool) -> int:
+        """How many parts the kernels for 17 to 128 rows make of this product (1: a gated one's rows); 0: they do not do it. They are
+        faster than the best of the library's algorithms for every shape they take, so nothing is measured; a table
+        that names an algorithm for the shape is followed as it stands."""
+        M, K = x.shape
+        if not (self.few_rows < M <= 128 and x.dtype == torch.bfloat16 and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0):
+            return 0
+        how = self.chosen.get((M, w.shape[0], K, False, False))
+        return 0 if how is not None and how >= 0 else self.lib.nhv_gemm_lines_splits(M, N, K, int(gated))
+
+    def linear_parts(self, x, w):
+        """x W^T as float parts [parts, rows, out] whose sum it is, or None where another way is the faster one."""
+        splits = self._by_lines(x, w, w.shape[0], False)
+        if not splits:
+            return None
+        parts = torch.empty((splits, x.shape[0], w.shape[0]), dtype=torch.float32, device=x.device)
+        self._call("nhv_gemm_lines_bf16", _ptr(x), _ptr(w), _ptr(None), _ptr(parts), x.shape[0], w.shape[0], x.shape[1], 0, *Gate().args(), _stream())
+        return parts
+
     norm_kernel_ms = 0.003        # what a norm's own kernel costs in a decoding step, about
 
     def _measured(self, x, w, gated: bool):
@@ -886,10 +914,13 @@ class NativeBackend:
 
     def gated_linear(self, x, w, out, gate=None, bias=None) -> bool:
         """A gate (a ``Gate``; None: SiLU) of x Wg^T and x Wu^T (+ bias) in one kernel, if this batch is one for the
-        few-rows kernel; else False. (SiLU without bias may also be one for the kernel of up to 64 rows; in float32 every batch is.)"""
+        few-rows kernel or the one for up to 96 rows; else False. (SiLU without bias may also be one for the kernel of up to 64 rows; in float32 every batch is.)"""
         M, K = x.shape
         if x.dtype == torch.float32:
             self._call("nhv_gemm_float32_gated", _ptr(x), _ptr(w), _ptr(bias), _ptr(out), M, out.shape[1], K, *(gate or Gate()).args(), _stream())
+            return True
+        if self._by_lines(x, w, out.shape[1], True):
+            self._call("nhv_gemm_lines_bf16", _ptr(x), _ptr(w), _ptr(bias), _ptr(out), M, out.shape[1], K, 1, *(gate or Gate()).args(), _stream())
             return True
         if bias is not None or (gate is not None and gate.act != 0):
             if x.dtype == torch.bfloat16 and K % 8 == 0 and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0 and M <= self.few_rows:
@@ -1072,9 +1103,33 @@ class Normed:
         return out
 
 
+@dataclass
+class Parts:
+    """What ``linear`` returns where the product's kernel has cut the inner dimension over blocks and the caller has said that it
+    takes that: float32 parts [parts, rows, out] whose sum is the product. A norm that adds to a residual stream and the
+    kernel that turns queries and keys add the parts up themselves, unrounded; ``tensor()`` is the product, rounded, for any
+    other reader (one small kernel)."""
+
+    parts: torch.Tensor
+    dtype: torch.dtype            # the rows' element type
+
+    @property
+    def shape(self):
+        return self.parts.shape[1:]
+
+    @property
+    def device(self):
+        return self.parts.device
+
+    def tensor(self) -> torch.Tensor:
+        out = torch.empty(self.shape, dtype=self.dtype, device=self.device)
+        backend().sum_parts(self.parts, out)
+        return out
+
+
 def dense(x):
     """``x`` as a tensor, whatever work was left undone in it."""
-    if isinstance(x, Normed):
+    if isinstance(x, (Normed, Parts)):
         return x.tensor()
     if isinstance(x, Summed):
         raise KernelError("a sum that was made for a norm (ops.Summed) goes through that norm, not anywhere else")
@@ -1135,7 +1190,19 @@ def rmsnorm(x: torch.Tensor, w: torch.Tensor, eps: float, residual: torch.Tensor
     ``start_residual=True``: returns (norm of x, the residual that later norms add to): a new float32 tensor holding
     x, or, with ``residual_float32=False``, x itself (which later calls then add to in place).
     ``rounds_between``: the normed row is rounded to x's element type, then multiplied with the weight and rounded
-    again; False: it is rounded once, at the end."""
+    again; False: it is rounded once, at the end.
+    ``x`` may be ``Parts`` (with ``residual``)."""
+    if isinstance(x, Parts):
+        if residual is None or x.shape[1] % 8 or w.data_ptr() % 16 or residual.data_ptr() % 16:
+            return rmsnorm(x.tensor(), w, eps, residual, start_residual, residual_float32, rounds_between)
+        _need(not start_residual, "rmsnorm: a residual is either started or added to")
+        _dense(w, "rmsnorm: weight", (x.shape[1],))
+        _need(w.dtype == x.dtype or w.dtype == torch.float32, lambda: f"rmsnorm: weight of {w.dtype} with activations of {x.dtype}")
+        _dense(residual, "rmsnorm: residual", tuple(x.shape))
+        _need(residual.dtype == x.dtype or residual.dtype == torch.float32, lambda: f"rmsnorm: residual of {residual.dtype} with rows of {x.dtype}")
+        y = torch.empty(x.shape, dtype=x.dtype, device=x.device)
+        backend().add_parts_norm(x.parts, residual, w, y, float(eps), **({} if rounds_between else {"rounds_between": False}))
+        return y
     _need(x.dim() == 2, "rmsnorm: x must be [tokens, width]")
     _dense(x, "rmsnorm: x")
     _dense(w, "rmsnorm: weight", (x.shape[1],))
@@ -1187,11 +1254,19 @@ def qk_rope_write(qkv, bias, q_norm_w, k_norm_w, eps, cos_sin, positions, slot_m
     """Splits the packed projection, norms and turns q and k, stores k and v in the
     paged cache and returns q as [tokens, heads, head_dim].
     ``positions``: [tokens], or [axes, tokens] with ``pair_axes`` [rotary size / 2] (int32): the axis whose
-    coordinate turns each pair (without ``pair_axes`` every pair turns by the first axis)."""
+    coordinate turns each pair (without ``pair_axes`` every pair turns by the first axis).
+    ``qkv`` may be ``Parts``."""
     T = qkv.shape[0]
     width = (num_heads + 2 * num_kv_heads) * head_dim
-    _dense(qkv, "qk_rope_write: qkv", (T, width))
-    dtype_code(qkv)
+    split = qkv if isinstance(qkv, Parts) else None
+    if split is not None:
+        whole = 16 <= head_dim <= 512 and head_dim & (head_dim - 1) == 0 and (cos_sin is None or cos_sin.shape[1] == head_dim) and pair_axes is None
+        starts = [t.data_ptr() for t in (bias, q_norm_w, k_norm_w, cos_sin, k_cache if write_kv else None, v_cache if write_kv else None) if t is not None]
+        if not whole or any(p % 16 for p in starts):         # (the kernel that takes parts asks for whole heads in 16 bytes a lane)
+            qkv, split = qkv.tensor(), None
+    _dense(qkv if split is None else split.parts, "qk_rope_write: qkv", (T, width) if split is None else (split.parts.shape[0], T, width))
+    if split is None:
+        dtype_code(qkv)
     if bias is not None:
         _dense(bias, "qk_rope_write: bias", (width,), qkv.dtype)
     for name, w in (("q_norm", q_norm_w), ("k_norm", k_norm_w)):
@@ -1224,7 +1299,7 @@ def qk_rope_write(qkv, bias, q_norm_w, k_norm_w, eps, cos_sin, positions, slot_m
         _dense(k_cache, "qk_rope_write: k_cache", dtype=qkv.dtype)
         _dense(v_cache, "qk_rope_write: v_cache", tuple(k_cache.shape), qkv.dtype)
     q_out = torch.empty((T, num_heads, head_dim), dtype=qkv.dtype, device=qkv.device)
-    backend().qk_rope_write(qkv, bias, q_norm_w, k_norm_w, float(eps), cos_sin, rot, positions,
+    backend().qk_rope_write(qkv if split is None else split.parts, bias, q_norm_w, k_norm_w, float(eps), cos_sin, rot, positions,
                             slot_mapping if write_kv else None, q_out, k_cache if write_kv else None,
                             v_cache if write_kv else None, num_heads, num_kv_heads, head_dim, write_kv,
                             **({} if pair_axes is None else {"pair_axes": pair_axes}))
@@ -1290,13 +1365,15 @@ def paged_attention(q, k_cache, v_cache, batch: AttentionBatch, block_tables, sc
     return out
 
 
-def linear(x, w: torch.Tensor, bias: torch.Tensor | None = None, out_dtype=None, add_to: AddTo | None = None):
+def linear(x, w: torch.Tensor, bias: torch.Tensor | None = None, out_dtype=None, add_to: AddTo | None = None, parts: bool = False):
     """x[M, K] . w[N, K]^T (+ bias), accumulated in float. ``out_dtype`` may be
     float32 for bfloat16 inputs (the logits).
     ``x`` may be a ``Normed``: where the product's kernel can, it scales the rows itself.
     ``add_to``: the residual stream [M, N] that the caller is about to add the result to, and the norm that follows.
     Where the product's kernel can, it makes the addition itself (in float; the stream is rewritten) and a ``Summed``
-    is returned, which that norm takes; otherwise the plain result is returned and the stream is left alone."""
+    is returned, which that norm takes; otherwise the plain result is returned and the stream is left alone, for some sizes
+    as ``Parts``, which that norm takes too.
+    ``parts``: the caller takes ``Parts`` whatever it does with the result."""
     normed = x if isinstance(x, Normed) else None
     if normed is not None:
         x = normed.summed.weighted
@@ -1325,6 +1402,11 @@ def linear(x, w: torch.Tensor, bias: torch.Tensor | None = None, out_dtype=None,
         backend().fused_linear(x, w, bias, None, row_scales=scales, residual=residual, sum_out=weighted, ss_out=squares,
                                next_w=add_to.norm_weight)
         return Summed(weighted, squares, residual, add_to.norm_weight, add_to.eps)
+    if (parts or add_to is not None) and normed is None and bias is None and out_dtype == x.dtype:
+        make = getattr(backend(), "linear_parts", None)
+        made = None if make is None else make(x, w)
+        if made is not None:
+            return Parts(made, x.dtype)
     out = torch.empty((M, N), dtype=out_dtype, device=x.device)
     if normed is not None:
         backend().fused_linear(x, w, bias, out, row_scales=scales)

@@ -72,7 +72,7 @@ class GQAAttention(Part):
 
     def forward(self, x, step, cache: CacheView, add_to=None):
         tables = step.groups[cache.group]
-        qkv = ops.linear(x, self.qkv_weight)
+        qkv = ops.linear(x, self.qkv_weight, parts=True)
         # an encoding over several position axes says which axis turns each pair; others turn by the first axis
         pair_axes = self.position.pair_axes() if hasattr(self.position, "pair_axes") else None
         q = ops.qk_rope_write(

@@ -223,7 +223,8 @@ class DecoderModel(Part):
         if step.num_logit_rows == 0:
             return None
         # only the wanted rows go through the last norm and the head (nanovllm/layers/embed_head.py:56-61)
-        if isinstance(hidden, ops.Summed):    # the last product has added itself to the residual stream already
+        if isinstance(hidden, (ops.Summed, ops.Parts)):    # the last product has added itself to the residual stream already, or leaves
+            # its parts to the norm
             hidden, _ = self.final_norm.forward_add(hidden, residual)
             return ops.gather_rows(hidden, step.logit_rows)
         hidden = ops.gather_rows(hidden, step.logit_rows)

@@ -1201,6 +1201,69 @@ def test_library_products_refuse_what_they_cannot_do(ops):
 # The kernels choose waves, loads in flight, tiles a block and split lengths from the sizes by rules; these cases walk
 # over the rules' borders at sizes nobody picked by hand.
 
+@pytest.mark.parametrize("M,N,K", [
+    # one and two tiles past 16 rows, every number of row tiles up to 8, the last one cut off; outputs that end inside a tile, a
+    # chunk and two chunks of columns, chunks that do not divide by the parts
+    (17, 64, 256), (32, 1000, 384), (33, 4096, 4096), (49, 6144, 2560), (64, 4096, 12288), (79, 2560, 1152), (80, 1033, 3072), (96, 333, 9728),
+    (97, 512, 512), (112, 2048, 6144), (128, 1024, 3072),
+])
+def test_products_by_lines(ops, M, N, K):
+    """As float parts and as a gate of two products, with biases and without (float sums of K products of size K^-1/2)."""
+    x = rnd(M, K, dtype=torch.bfloat16, seed=81)
+    w = rnd(2 * N, K, dtype=torch.bfloat16, seed=82, scale=K ** -0.5)
+    b = rnd(2 * N, dtype=torch.bfloat16, seed=83)
+    both = x.double() @ w.double().T
+    wn = w[:N].contiguous()
+    got = ops.linear(x, wn, parts=True)
+    assert isinstance(got, ops.Parts) and got.shape == (M, N)
+    torch.testing.assert_close(got.parts.double().sum(0), both[:, :N], rtol=1e-4, atol=2e-4)
+    assert torch.equal(got.parts, ops.linear(x, wn, parts=True).parts)
+    total = got.parts[0].clone()
+    for part in got.parts[1:]:
+        total += part
+    assert torch.equal(ops.dense(got), total.bfloat16())
+    if M <= 80:
+        out = torch.full((M, N), float("nan"), dtype=torch.bfloat16, device="cuda")
+        assert ops.backend().gated_linear(x, w, out)
+        torch.testing.assert_close(out.double(), torch.nn.functional.silu(both[:, :N]) * both[:, N:], **tol(torch.bfloat16))
+        gate = ops.Gate(2, 1.5, 1.702, 1.0)
+        g, u = (both + b.double()).split(N, dim=1)
+        g, u = g.clamp(max=1.5), u.clamp(-1.5, 1.5)
+        torch.testing.assert_close(ops.gated_linear(x, w, gate, b).double(), g * torch.sigmoid(1.702 * g) * (u + 1), **tol(torch.bfloat16))
+
+
+@pytest.mark.parametrize("splits", [1, 2, 4, 8])
+def test_parts_of_a_product_through_the_norm_and_the_rotation(ops, splits):
+    """Parts whose sum is a bfloat16 number give the bits that this number gives: the norm that adds to the residual stream (in
+    both types, for widths in one piece and in two) and the kernel that turns queries and keys."""
+    def parts_of(t):
+        share = t.float() / splits                           # (a power of two: exact)
+        return ops.Parts(share.expand(splits, *t.shape).contiguous(), torch.bfloat16)
+
+    for width in (8, 520, 4096, 9216):
+        x = rnd(5, width, dtype=torch.bfloat16, seed=84)
+        for res_dtype in DTYPES:
+            for w_dtype in DTYPES:
+                w, r = rnd(width, dtype=w_dtype, seed=85) + 1, rnd(5, width, dtype=res_dtype, seed=86)
+                r2 = r.clone()
+                want = ops.rmsnorm(x, w, 1e-6, residual=r)
+                assert torch.equal(ops.rmsnorm(parts_of(x), w, 1e-6, residual=r2), want) and torch.equal(r, r2)
+    T, Hq, Hkv = 7, 6, 2
+    for D in (16, 64, 128, 512, 48):                         # (48: no power of two, the parts are summed first)
+        qkv, bias = rnd(T, (Hq + 2 * Hkv) * D, dtype=torch.bfloat16, seed=87), rnd((Hq + 2 * Hkv) * D, dtype=torch.bfloat16, seed=88)
+        nq, nk = rnd(D, dtype=torch.bfloat16, seed=89) + 1, rnd(D, dtype=torch.bfloat16, seed=90) + 1
+        table = rnd(40, D, seed=91)
+        positions = torch.arange(3, 3 + T, dtype=torch.int32, device="cuda")
+        slots = torch.tensor([4, -1, 0, 9, 10, 3, 7], dtype=torch.int32, device="cuda")
+        for norms, b in (((nq, nk), None), ((None, None), bias)):
+            results = []
+            for rows in (qkv, parts_of(qkv)):
+                k, v = (torch.zeros(3, 4, Hkv, D, dtype=torch.bfloat16, device="cuda") for _ in range(2))
+                q = ops.qk_rope_write(rows, b, *norms, 1e-6, table, positions, slots, k, v, Hq, Hkv, D)
+                results.append((q, k, v))
+            assert all(torch.equal(a, c) for a, c in zip(*results)), D
+
+
 def _random_product_sizes(seed, count, max_rows):
     import random
     rnd_ = random.Random(seed)
