@@ -26,6 +26,7 @@
 // won: the fences cost more than the balance gains.)
 #include "nhv_common.h"
 #include "nhv_gemm_fusion.h"
+#include "nhv_lines.h"
 
 namespace fewrows {
 
@@ -938,6 +939,138 @@ static int launch_tiles(const TilesPlan& p, hipStream_t s, const void* x, const 
   return 0;
 }
 
+// The kernel for rows of w that fill the chip in tiles of 16 (see lines_plan): w and x through LDS in chunks of 256 columns, a row's
+// 512 bytes in one piece, in a ring of NB chunks; a block is 8 waves, each with 32 of a chunk's columns, and a chunk costs one
+// barrier. The kernels above and below bring 16 rows of 64 bytes a load, of which a compute unit takes in 17 to 20 GB/s; pieces of
+// 512 bytes come at the memory's own rate. Their places are turned by the row, so that 16 rows lie in different banks. NT tiles of w a
+// block (gated: one and its partner). us at 1, 8 and 16 rows, before and now: 6,144 outputs of 4,096 columns 12.6, 13.7, 17.7 and 11.7,
+// 12.1, 12.6; 4,096 of 4,096 10.2, 10.6, 11.8 and 8.4, 8.6, 8.9; gated 12,288 of 4,096 42.8, 43.3, 48.6 and 36.3, 35.9, 36.5 (a kernel that only
+// reads: 32.5); 4,096 of 12,288 23.0, 28.2, 31.0 and 19.7, 20.2, 22.1; 151,936 of 4,096 204, 216, 270 and 196, 198, 201 (201);
+// gated 9,728 of 2,560 25.5, 26.0, 26.3 and 22.5, 22.9, 23.6.
+template <int NT, int NB, bool GATED, typename TOut>
+__global__ __launch_bounds__(512) void gemm_fewrows_lines_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ w, const bf16_t* __restrict__ bias,
+                                                                 TOut* __restrict__ y, int M, int N, int K, const Fusion f) {
+  constexpr int OUT = GATED ? 1 : NT, BOTH = GATED ? 2 : 1, CHUNK = 256, LOADS = NT + 1, STAGE = (NT + 1) * 16 * CHUNK;
+  // (a name of its own: an array of this alignment under the others' name would cost the kernels around their last 1,024 bytes)
+  extern __shared__ __attribute__((aligned(1024))) bf16_t line_ring[];
+  const bf16_t* ring = line_ring;
+  __shared__ float r_s[16];
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, r16 = lane & 15, g = lane >> 4;
+  const int n0 = blockIdx.x * 16 * OUT, chunks = K / CHUNK;
+  // what the thread that finishes output (row, n) needs beside the sums, asked for before the weights
+  const int row = (threadIdx.x >> 4) & 15, tile = threadIdx.x >> 8, n = n0 + 16 * tile + (threadIdx.x & 15);
+  const bool mine = tile < OUT && row < M && n < N;
+  float share[SCALE_ROWS<8>][SCALE_SHARES];
+  ask_row_scales<8>(f, share, M, wave, lane);
+  float res = 0.f, next_w = 1.f, add[2] = {0.f, 0.f};
+  if (mine) {
+    if (f.residual) res = f.residual_f32 ? ((const float*)f.residual)[(size_t)row * N + n] : (float)((const bf16_t*)f.residual)[(size_t)row * N + n];
+    if (f.next_w) next_w = f.next_w_f32 ? ((const float*)f.next_w)[n] : (float)((const bf16_t*)f.next_w)[n];
+    if (bias) {
+      add[0] = (float)bias[n];
+      if (GATED) add[1] = (float)bias[N + n];
+    }
+  }
+  // what this lane brings of a chunk: 16 bytes of row 2 wave + lane / 32 of every tile, the last tile x's. Rows beyond the matrices are their last
+  // ones (their results are dropped).
+  const bf16_t* src[LOADS];
+  const int my_row = 2 * wave + (lane >> 5), piece = (lane & 31) ^ my_row;
+#pragma unroll
+  for (int t = 0; t < LOADS; ++t)
+    src[t] = (t < NT ? w + ((size_t)(GATED ? t * N : 0) + min(n0 + (GATED ? 0 : 16 * t) + my_row, N - 1)) * K : x + (size_t)min(my_row, M - 1) * K) + piece * 8;
+  const uint32_t ring_at = nhv_lds_address(ring) + wave * 1024;
+  const int first = nhv_first_chunk(blockIdx.x, chunks, K);
+  auto ask = [&](int buf, int c) {
+    const size_t k = (size_t)nhv_chunk(first, c, chunks) * CHUNK;
+#pragma unroll
+    for (int t = 0; t < LOADS; ++t) {
+      if (t < NT) nhv_load_to_lds<true>(ring_at + (buf * STAGE + t * 16 * CHUNK) * 2, src[t] + k);
+      else nhv_load_to_lds<false>(ring_at + (buf * STAGE + t * 16 * CHUNK) * 2, src[t] + k);
+    }
+  };
+  floatx4 acc[NT];
+#pragma unroll
+  for (int t = 0; t < NT; ++t) acc[t] = floatx4{0.f, 0.f, 0.f, 0.f};
+  const int at = r16 * CHUNK + (((wave * 4 + g) ^ r16) << 3);
+#pragma unroll
+  for (int i = 0; i < NB - 1; ++i) ask(i, i);
+  int buf = 0;
+  for (int c = 0; c < chunks; ++c) {
+    nhv_wait_and_meet<(NB - 2) * LOADS>();                            // chunk c is there, chunk c - 1 has been read
+    ask(buf == 0 ? NB - 1 : buf - 1, c + NB - 1);
+    const bf16_t* now = ring + buf * STAGE + at;
+    const bf16x8 b = *reinterpret_cast<const bf16x8*>(now + NT * 16 * CHUNK);
+#pragma unroll
+    for (int t = 0; t < NT; ++t) acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b, *reinterpret_cast<const bf16x8*>(now + t * 16 * CHUNK), acc[t], 0, 0, 0);
+    buf = buf == NB - 1 ? 0 : buf + 1;
+  }
+  nhv_wait_and_meet<0>();                                             // (the ring becomes room for the sums)
+  float* part = reinterpret_cast<float*>(line_ring);                    // [tile][wave][256]
+#pragma unroll
+  for (int t = 0; t < NT; ++t) *reinterpret_cast<floatx4*>(&part[(t * 8 + wave) * 256 + lane * 4]) = acc[t];
+  set_row_scales<8>(f, share, r_s, M, K, wave, lane);
+  __syncthreads();
+  if (tile >= OUT) return;                                            // (whole waves)
+  // (lane 16 g + c of a tile holds rows 4 g .. 4 g + 3 of column c; the waves' sums in their order)
+  float v[BOTH];
+#pragma unroll
+  for (int both = 0; both < BOTH; ++both) {
+    const float* from = &part[(GATED ? both : tile) * 2048 + (row >> 2) * 64 + (threadIdx.x & 15) * 4 + (row & 3)];
+    v[both] = 0.f;
+#pragma unroll
+    for (int wv = 0; wv < 8; ++wv) v[both] += from[wv * 256];
+    if (f.ss_in) v[both] *= r_s[row];                                 // (r_s of rows beyond M is not set, nor used below)
+    v[both] += add[both];
+  }
+  float out = GATED ? nhv_gated(v[0], v[BOTH - 1], f.gate) : f.plain_act ? nhv_plain_act(v[0], f.plain_act) : v[0];
+  if (GATED || f.residual == nullptr) {
+    if (mine) y[(size_t)row * N + n] = (TOut)out;
+    return;
+  }
+  out += res;                                                         // (see emit_tile)
+  if (mine) {
+    if (f.residual_f32) ((float*)f.residual)[(size_t)row * N + n] = out;
+    else ((bf16_t*)f.residual)[(size_t)row * N + n] = (bf16_t)out;
+    f.sum_out[(size_t)row * N + n] = (bf16_t)(out * next_w);
+  }
+  float sq = mine ? out * out : 0.f;
+#pragma unroll
+  for (int o = 1; o < 16; o <<= 1) sq += __shfl_xor(sq, o, 64);
+  const int tiles = (N + 15) / 16, my_tile = blockIdx.x * OUT + tile;
+  if ((threadIdx.x & 15) == 0 && row < M && my_tile < tiles) f.ss_out[(size_t)row * tiles + my_tile] = sq;
+}
+
+// Where the rows of w are enough for it, by what was measured at 1, 4, 8, 12 and 16 rows (us before and with it): not for 4,096 outputs
+// of 1,024 columns (4.2, 4.9 at 1 row) or a gated 3,072 of 1,024 (5.5, 5.7); with fewer than 4,096 outputs a tile of 16 leaves units idle,
+// which the smaller tiles above do not, until there are so many rows that these are slower: 2,560 of 9,728 14.6, 15.1 at 1 row,
+// 15.5, 15.7 at 4, 18.8, 15.8 at 8; 2,048 of 6,144 9.9, 11.1 at 8 and 14.3, 11.5 at 12; 2,048 of 2,048 never.
+static bool lines_plan(bool glu, int M, int N, int K) {
+  if (K % 256 != 0 || K < 2048) return false;
+  if (glu) return N >= 4096;
+  return N >= 4096 || (N >= 2560 && M >= 8) || (N >= 2048 && K >= 4096 && M >= 12);
+}
+
+template <int NT, int NB, bool GATED, typename TOut>
+static int launch_lines_as(hipStream_t s, const void* x, const void* w, const void* bias, void* y, int M, int N, int K, const Fusion& f) {
+  constexpr int OUT = GATED ? 16 : 16 * NT, ring = NB * (NT + 1) * 16 * 512, sums = NT * 8192, lds = ring > sums ? ring : sums;
+  auto kernel = gemm_fewrows_lines_kernel<NT, NB, GATED, TOut>;
+  // more than 64 KB of dynamic LDS has to be allowed once per kernel (and per process)
+  static const hipError_t allowed = hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+  if (allowed != hipSuccess) return nhv_fail("few-rows gemm: %s", hipGetErrorString(allowed));
+  hipLaunchKernelGGL(kernel, dim3((N + OUT - 1) / OUT), dim3(512), lds, s, (const bf16_t*)x, (const bf16_t*)w, (const bf16_t*)bias, (TOut*)y, M, N, K, f);
+  return 0;
+}
+// One block a compute unit: four chunks in the ring; several: three.
+template <bool GATED, typename TOut>
+static int launch_lines(hipStream_t s, const void* x, const void* w, const void* bias, void* y, int M, int N, int K, const Fusion& f) {
+  if constexpr (GATED) {
+    return N <= 256 * 16 ? launch_lines_as<2, 4, true, TOut>(s, x, w, bias, y, M, N, K, f) : launch_lines_as<2, 3, true, TOut>(s, x, w, bias, y, M, N, K, f);
+  } else {
+    if (N <= 256 * 16) return launch_lines_as<1, 4, false, TOut>(s, x, w, bias, y, M, N, K, f);
+    return N <= 256 * 32 ? launch_lines_as<2, 4, false, TOut>(s, x, w, bias, y, M, N, K, f) : launch_lines_as<2, 3, false, TOut>(s, x, w, bias, y, M, N, K, f);
+  }
+}
+
 // The resident kernel's shape: waves, loads in flight and blocks per compute unit, from the best variants measured
 // (same shapes as below), and in how many pieces x comes; waves == 0 when this kernel is not the one to take.
 struct ResidentPlan {
@@ -1115,6 +1248,10 @@ int nhv_gemm_fewrows_launch(bool glu, const void* x, const void* w, const void* 
     return 0;
   }
   if (fused && out_dtype != NHV_BF16) return nhv_fail("few-rows gemm: a product that takes over its neighbours' work gives bfloat16");
+  if (lines_plan(glu, M, N, K) && !(glu && out_dtype != NHV_BF16)) {
+    if (glu) return launch_lines<true, bf16_t>(s, x, w, bias, y, M, N, K, f);
+    return out_dtype == NHV_BF16 ? launch_lines<false, bf16_t>(s, x, w, bias, y, M, N, K, f) : launch_lines<false, float>(s, x, w, bias, y, M, N, K, f);
+  }
   const TilesPlan tp = tiles_plan(glu, f.residual != nullptr, bias != nullptr, M, N, K);
   const bool on_16 = (((uintptr_t)y | (uintptr_t)bias | (uintptr_t)f.residual | (uintptr_t)f.sum_out | (uintptr_t)f.next_w) & 15) == 0;
 #define NHV_TILES_CASE(AHEAD_, GLU_, XLDS_)                                                                            \

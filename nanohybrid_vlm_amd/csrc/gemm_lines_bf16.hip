@@ -10,16 +10,16 @@
 // elementwise.hip). Parts are [splits][M][N], in rising order of K.
 // Bank conflicts: a row's piece p of 16 bytes lies at place p ^ (row & 15), which costs nothing, since a lane chooses what it brings.
 // us, and what the vendor's library takes by its best algorithm (with the gate's own kernel for gated products), cold weights: 64
-// rows, 8B shape: qkv 15.5, 18.0; o 11.5, 13.9; gated 45.8, 50.6; down 25.9, 33.3; 79 rows, 4B shape: 13.7, 15.2; 11.1, 12.8; 30.7,
-// 32.1; 18.7, 24.8; 32 rows, 0.6B shape: 4.5, 5.7; 3.9, 5.6; 6.4, 8.7; 4.3, 6.4.
+// rows, 8B shape: qkv 15.5, 18.1; o 11.5, 14.0; gated 41.0, 50.0; down 25.6, 33.1; 79 rows, 4B shape: 13.5, 15.1; 10.8, 12.8; 31.1,
+// 32.1; 18.1, 24.8; 32 rows, 0.6B shape: 4.5, 5.7; 3.9, 5.6; 6.4, 8.7; 4.3, 6.4.
 #include "nhv_common.h"
 #include "nhv_gates.h"
+#include "nhv_lines.h"
 
 namespace lines {
 
 typedef bf16_t bf16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
-typedef __attribute__((address_space(3))) void* lds_ptr;
 
 constexpr int CHUNK = 128, PIECES = CHUNK / 8, ROWS_A_LOAD = 64 / PIECES;        // columns; 16-byte pieces and rows a wave's load
 
@@ -46,18 +46,15 @@ __global__ __launch_bounds__(512) void gemm_lines_kernel(const bf16_t* __restric
                                    : x + (size_t)min(row - 16 * NT, M - 1) * K;
     src[i] = from + ((lane % PIECES) ^ (row & 15)) * 8;
   }
-  const uint32_t ring_at = (uint32_t)(uintptr_t)(lds_ptr)ring;
-  // (written as instructions: of the builtin's loads the compiler keeps account, and waits for all of them before it reads any
-  // of the ring. w is read once, x by every block: w passes the caches by.)
+  const uint32_t ring_at = nhv_lds_address(ring);
+  const int first = c1 - c0 < 16 ? 0 : nhv_first_chunk(blockIdx.x, c1 - c0, K);       // (short splits lie apart already: 11.5 us against 12.0)
   auto ask = [&](int buf, int c) {
-    const size_t k = (size_t)min(c, chunks - 1) * CHUNK;             // (behind the last chunk: it again)
+    const size_t k = (size_t)(c0 + nhv_chunk(first, c - c0, c1 - c0)) * CHUNK;
 #pragma unroll
     for (int i = 0; i < LOADS; ++i) {
-      const uint32_t to = __builtin_amdgcn_readfirstlane(ring_at + buf * stage_bytes(MT, NT) + (i * 8 + wave) * 1024);
-      if (GATED && (i + 1) * 8 * ROWS_A_LOAD <= 16 * NT)
-        asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off nt" ::"s"(to), "v"(src[i] + k) : "memory");
-      else
-        asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(to), "v"(src[i] + k) : "memory");
+      const uint32_t to = ring_at + buf * stage_bytes(MT, NT) + (i * 8 + wave) * 1024;
+      if (GATED && (i + 1) * 8 * ROWS_A_LOAD <= 16 * NT) nhv_load_to_lds<true>(to, src[i] + k);
+      else nhv_load_to_lds<false>(to, src[i] + k);
     }
   };
   f32x4 acc[MINE][MT];
@@ -72,9 +69,7 @@ __global__ __launch_bounds__(512) void gemm_lines_kernel(const bf16_t* __restric
   for (int c = c0; c < c1; ++c) {
     // this wave's loads of chunk c have arrived; behind the barrier everyone's have, and everyone has read chunk c - 1, whose
     // place the next load takes
-    __builtin_amdgcn_sched_barrier(0);
-    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"((NB - 2) * LOADS) : "memory");
-    __builtin_amdgcn_sched_barrier(0);
+    nhv_wait_and_meet<(NB - 2) * LOADS>();
     ask(buf == 0 ? NB - 1 : buf - 1, c + NB - 1);
     const bf16_t* now = ring + buf * (ROWS * CHUNK) + at;
     bf16x8 a[MINE], b[MT];
@@ -88,7 +83,7 @@ __global__ __launch_bounds__(512) void gemm_lines_kernel(const bf16_t* __restric
       for (int m = 0; m < MT; ++m) acc[t][m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b[m], a[t], acc[t][m], 0, 0, 0);
     buf = buf == NB - 1 ? 0 : buf + 1;
   }
-  asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");      // (the ring becomes room for the sums)
+  nhv_wait_and_meet<0>();                                            // (the ring becomes room for the sums)
   // the sums of the four waves that share a tile's columns, in their order
   float* part = reinterpret_cast<float*>(ring);                      // [gate, up][MT][4][256]
 #pragma unroll

@@ -234,6 +234,9 @@ def test_few_rows_linear_bfloat16_in_all_its_variants(ops, M, N, K):
     (8, 4096, 12288), (6, 3076, 16392), (4, 4092, 18440),
     # a residual of more than 256 tiles: x beside w in LDS and not, and one row of many columns
     (4, 5136, 4104), (8, 4112, 17416), (1, 4100, 20488),
+    # chunks of whole lines: one tile a block and two, ends inside a tile, as few chunks as the ring has places and fewer, the
+    # fewest outputs at every bound of rows
+    (1, 4096, 2048), (3, 4100, 2816), (16, 6148, 3072), (5, 8196, 2048), (8, 2560, 2304), (12, 2048, 4352), (16, 16388, 2304),
 ])
 def test_tiles_of_few_rows_products(ops, M, N, K):
     """Plain, activated, gated, with rows that lack their scales and added to a residual (bounds: float32 sums of K products of
