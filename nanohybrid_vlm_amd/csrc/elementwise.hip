@@ -496,10 +496,10 @@ __global__ void qk_rope_write_kernel(const T* __restrict__ qkv, const T* __restr
 // `part_stride` entries apart, whose sums are not rounded before the norm (64 rows of the 8B shape: 4.8 us with and without).
 template <typename T, typename W, int CH, bool PARTS>
 __global__ __launch_bounds__(256) void qk_rope_write_vec_kernel(
-    const void* __restrict__ qkv, int splits, size_t part_stride, const T* __restrict__ bias, const W* __restrict__ q_norm_w, const W* __restrict__ k_norm_w,
+    const void* __restrict__ qkv, const T* __restrict__ bias, const W* __restrict__ q_norm_w, const W* __restrict__ k_norm_w,
     float eps, const float* __restrict__ cos_sin, int rot, const int* __restrict__ positions,
     const int* __restrict__ slot_mapping, T* __restrict__ q_out, T* __restrict__ k_cache, T* __restrict__ v_cache, int Hq,
-    int Hkv, int heads_per_token, long long n_items) {
+    int Hkv, int heads_per_token, long long n_items, int splits, size_t part_stride) {
   constexpr int D = CH * 8;
   const long long gid = (long long)blockIdx.x * 256 + threadIdx.x;
   const long long item = gid / CH;
@@ -596,10 +596,10 @@ extern "C" int nhv_qk_rope_write(const void* qkv, int splits, const void* bias, 
     NHV_REQUIRE(vblocks <= 0x7fffffff, "qk_rope_write: too many tokens");
     const size_t part_stride = (size_t)T * (Hq + 2 * Hkv) * D;
 #define VLAUNCH(TT, WW, CHN, PARTS)                                                                                  \
-  hipLaunchKernelGGL((qk_rope_write_vec_kernel<TT, WW, CHN, PARTS>), dim3((unsigned)vblocks), dim3(256), 0, s, qkv, splits, part_stride, \
+  hipLaunchKernelGGL((qk_rope_write_vec_kernel<TT, WW, CHN, PARTS>), dim3((unsigned)vblocks), dim3(256), 0, s, qkv, \
                      (const TT*)bias, (const WW*)q_norm_w, (const WW*)k_norm_w, eps, (const float*)cos_sin, rot,     \
                      (const int*)positions, (const int*)slot_mapping, (TT*)q_out, (TT*)k_cache, (TT*)v_cache, Hq, Hkv, \
-                     heads, n_items)
+                     heads, n_items, splits, part_stride)
 #define VBY_CH(TT, WW, PARTS)                      \
   switch (ch) {                                    \
     case 2: VLAUNCH(TT, WW, 2, PARTS); break;      \

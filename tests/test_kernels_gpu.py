@@ -1235,6 +1235,15 @@ def test_products_by_lines(ops, M, N, K):
         torch.testing.assert_close(ops.gated_linear(x, w, gate, b).double(), g * torch.sigmoid(1.702 * g) * (u + 1), **tol(torch.bfloat16))
 
 
+@pytest.mark.parametrize("M,band,last,K", [(1, 1024, 32, 2048), (16, 2048, 5, 2304), (7, 1056, 1100, 2048)])
+def test_products_in_bands_by_lines(ops, M, band, last, K):
+    """Five sets of rows against a matrix's bands, where the kernel by lines takes them (float sums of K products of size K^-1/2)."""
+    x = rnd(5, M, K, dtype=torch.bfloat16, seed=92)
+    w = rnd(4 * band + last, K, dtype=torch.bfloat16, seed=93, scale=K ** -0.5)
+    want = torch.cat([x[i].double() @ w[i * band:(4 * band + last if i == 4 else (i + 1) * band)].double().T for i in range(5)], dim=1)
+    torch.testing.assert_close(torch.cat(list(ops.banded_linear(x, w, band)), dim=1).double(), want, **tol(torch.bfloat16))
+
+
 @pytest.mark.parametrize("splits", [1, 2, 4, 8])
 def test_parts_of_a_product_through_the_norm_and_the_rotation(ops, splits):
     """Parts whose sum is a bfloat16 number give the bits that this number gives: the norm that adds to the residual stream (in
