@@ -124,12 +124,11 @@ struct Plan {
 static Plan plan(int M, int N, int K, bool gated) {
   Plan best = {0, 0, 0};
   // (gated products of 128 rows 62.7 us at the 8B shape, the library's product and the gate's kernel 54; of 96 rows 44.5 against 47.5
-  // there, 33.2 against 32.1 at the 4B shape, whose 203 blocks leave units idle. Of 128 rows wide products are slower too, 6,144 of
-  // 4,096 21.9 against 21.4, narrow ones not: 4,096 of 12,288 34 against 44.)
+  // there, and inside a step of the 4B shape 31.0 against 34.6. Of 128 rows wide products are slower too, 6,144 of 4,096 21.9
+  // against 21.4, narrow ones not: 4,096 of 12,288 34 against 44.)
   if (M < 17 || M > (gated ? 96 : 128) || (M > 96 && N > K) || K % CHUNK || N < 64) return best;
   const int tiles = (M + 15) / 16, mt = tiles == 7 ? 8 : tiles;
   double least = 1e300;
-  bool idle = false;
   for (int nt : {2, 3, 4, 6}) {
     if (gated && nt == 3) continue;
     for (int splits : {1, 2, 4, 8}) {
@@ -139,10 +138,9 @@ static Plan plan(int M, int N, int K, bool gated) {
       const double taken_in = (double)rounds * (mt + nt) * 32 * ((K / CHUNK + splits - 1) / splits * CHUNK) / 32e3;
       const double of_w = 2.0 * (gated ? 2 : 1) * N * K / 5.3e6;
       const double time = (taken_in > of_w ? taken_in : of_w) + (gated ? 0.0 : 8.0 * splits * M * N / 3.5e6 + 4.0 * splits * N / 40e3);
-      if (time < least) least = time, best = {mt, nt, splits}, idle = blocks < rounds * 230;
+      if (time < least) least = time, best = {mt, nt, splits};
     }
   }
-  if (gated && M > 80 && idle) return {0, 0, 0};
   return best;
 }
 

@@ -1225,7 +1225,7 @@ def test_products_by_lines(ops, M, N, K):
     for part in got.parts[1:]:
         total += part
     assert torch.equal(ops.dense(got), total.bfloat16())
-    if M <= 80:
+    if M <= 96:
         out = torch.full((M, N), float("nan"), dtype=torch.bfloat16, device="cuda")
         assert ops.backend().gated_linear(x, w, out)
         torch.testing.assert_close(out.double(), torch.nn.functional.silu(both[:, :N]) * both[:, N:], **tol(torch.bfloat16))
