@@ -564,7 +564,7 @@ class ModelRunner:
         return arrays, meta
 
     def _context(self, dev: list[torch.Tensor], meta: dict, logit_rows: torch.Tensor | None, num_logit_rows: int,
-                 max_context_len: int) -> StepContext:
+                 max_context_len: int, every_row: bool = False) -> StepContext:
         d_ids, d_pos, d_req, d_cu, d_ctx, d_slots = dev[:6]
         num_groups = len(self.cache.groups)
         groups = [GroupTables(slot_mapping=dev[6 + 2 * gi], block_tables=dev[7 + 2 * gi]) for gi in range(num_groups)]
@@ -575,7 +575,7 @@ class ModelRunner:
                                    max_context_len=max_context_len)
         return StepContext(num_tokens=meta["T"], num_requests=meta["B"], input_ids=d_ids, positions=positions,
                            token_positions=positions[0], attention=attention, groups=groups, state_slots=d_slots, logit_rows=logit_rows,
-                           num_logit_rows=num_logit_rows,
+                           num_logit_rows=num_logit_rows, every_row=every_row,
                            host={k: meta[k] for k in ("starts", "new_lens", "q_lens", "state_slots")})
 
     def build_context(self, entries: list[StepEntry]) -> tuple[StepContext, list[int]]:
@@ -789,7 +789,7 @@ class ModelRunner:
         """The graph of a step of single tokens for ``bucket`` requests."""
         index, dev = self._index_buffer(arrays)
         all_rows = torch.arange(bucket, dtype=torch.int32, device=self.device)
-        ctx = self._context(dev, meta, all_rows, bucket, max_context_len=width * self.page_size)
+        ctx = self._context(dev, meta, all_rows, bucket, max_context_len=width * self.page_size, every_row=True)
         # the graph's launches are fixed: kernels that split the keys plan for this step's longest context, and their
         # splits (and the splits' results) cover contexts of up to half as much again; the block tables are made for
         # max_model_len. The graph serves contexts from half of ``planned`` to ``covered`` and is replaced beyond.

@@ -31,5 +31,6 @@ class StepContext:
     state_slots: torch.Tensor      # [B] int32: each request's row in the state pools
     logit_rows: torch.Tensor | None  # [n] int32: the tokens whose logits are wanted
     num_logit_rows: int = 0
+    every_row: bool = False        # ``logit_rows`` is every token in its order: nothing has to be gathered
     host: dict = field(default_factory=dict)   # the same facts as Python lists, for parts that work on the host
     scratch: dict = field(default_factory=dict)   # device buffers that parts of one step share (made by the first that needs them)

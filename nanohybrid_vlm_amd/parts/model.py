@@ -223,15 +223,15 @@ class DecoderModel(Part):
         if step.num_logit_rows == 0:
             return None
         # only the wanted rows go through the last norm and the head (nanovllm/layers/embed_head.py:56-61)
+        wanted = (lambda rows: rows) if step.every_row else (lambda rows: ops.gather_rows(rows, step.logit_rows))
         if isinstance(hidden, (ops.Summed, ops.Parts)):    # the last product has added itself to the residual stream already, or leaves
             # its parts to the norm
             hidden, _ = self.final_norm.forward_add(hidden, residual)
-            return ops.gather_rows(hidden, step.logit_rows)
-        hidden = ops.gather_rows(hidden, step.logit_rows)
+            return wanted(hidden)
+        hidden = wanted(hidden)
         if residual is None:                  # the last block has made its additions itself
             return self.final_norm.forward(hidden)
-        residual = ops.gather_rows(residual, step.logit_rows)
-        hidden, _ = self.final_norm.forward_add(hidden, residual)
+        hidden, _ = self.final_norm.forward_add(hidden, wanted(residual))
         return hidden
 
     def logits(self, hidden: torch.Tensor) -> torch.Tensor:
