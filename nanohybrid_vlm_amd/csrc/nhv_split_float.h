@@ -1,8 +1,11 @@
-// Products of floats on the bfloat16 matrix cores: a float as the sum of three bfloat16 numbers.
+// Products of floats on the bfloat16 matrix cores: 2^16 times a float as the sum of three bfloat16 numbers.
 //
-// high = x rounded to 8 bits, middle = (x - high) rounded, rest = x - high - middle. Both differences are exact (a float has 24
-// bits; each part takes 8 and its sign one more), and so is the rest's conversion: high + middle + rest = x, bit for bit, as
-// long as the rest is no denormal (|x| above about 2^-109; below that what is lost is under 2^-133).
+// high = 2^16 x rounded to 8 bits, middle = (2^16 x - high) rounded, rest = 2^16 x - high - middle. Both differences are exact (a
+// float has 24 bits; each part takes 8 and its sign one more), and so is the rest's conversion: high + middle + rest = 2^16 x, bit
+// for bit. That holds for every float, denormals too: floats end at 2^-149, the bfloat16 denormals (which the instructions used
+// here keep) at 2^-133, and the factor brings the one to the other. (Without it the parts of x below 2^-109 lost what lies under
+// 2^-133: products of entries near 1e-34 were off by 2.8e-7, near 1e-36 by 2.7e-5.) At the other end 2^16 x is infinite from
+// 2^112 on, as is a sum of products from 2^96 on.
 #pragma once
 #include "nhv_common.h"
 
@@ -11,6 +14,9 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef bf16_t bf16x2 __attribute__((ext_vector_type(2)));
 typedef bf16_t bf16x4 __attribute__((ext_vector_type(4)));
 typedef bf16_t bf16x8 __attribute__((ext_vector_type(8)));
+
+constexpr float SPLIT_SCALE = 0x1p16f;                   // of an operand
+constexpr float SPLIT_UNSCALE = 0x1p-32f;                // of a sum of products
 
 struct SplitFloats4 { bf16x4 high, middle, rest; };
 struct SplitFloats8 { bf16x8 high, middle, rest; };
@@ -33,7 +39,7 @@ __device__ __forceinline__ SplitFloats4 split_floats(f32x4 v) {
   SplitFloats4 p;
 #pragma unroll
   for (int i = 0; i < 4; i += 2) {
-    float a = v[i], b = v[i + 1];
+    float a = v[i] * SPLIT_SCALE, b = v[i + 1] * SPLIT_SCALE;
     const bf16x2 high = take_high(a, b), middle = take_high(a, b), rest = __builtin_convertvector((f32x2{a, b}), bf16x2);
     p.high[i] = high[0], p.high[i + 1] = high[1];
     p.middle[i] = middle[0], p.middle[i + 1] = middle[1];

@@ -336,6 +336,34 @@ def test_float32_linear_at_the_ends_of_its_range(ops, M, N, K):
     assert ((got - want).abs()[near] <= (K * 2.0 ** -24 * size)[near]).all()
 
 
+@pytest.mark.parametrize("M,N,K", [(1, 16, 32), (6, 512, 96), (70, 300, 64), (130, 2000, 36)])
+@pytest.mark.parametrize("of_x,of_w", [(1e-34, 1.0), (1e-36, 1.0), (1.0, 1e-37), (1e-40, 1.0), (1e-36, 1e36), (1e-38, 1e20), (1e-19, 1e-19), (1e-21, 1e-20)])
+def test_float32_linear_of_tiny_entries(ops, M, N, K, of_x, of_w):
+    """Operands down to the denormals, one of them and both, lose none of their bits (bound: an output's roundings, six an inner
+    block of 32 and a few at the ends, of the sum of its terms' sizes, and the last place of a denormal), and the same gated."""
+    x, w = rnd(M, K, seed=111) * of_x, rnd(2 * N, K, seed=112) * of_w
+    want = x.double().cpu() @ w.double().cpu().T
+    size = x.double().cpu().abs() @ w.double().cpu().abs().T
+    bound = (6 * -(-K // 32) + 10) * 2.0 ** -24 * size + 2.0 ** -149
+    assert ((ops.linear(x, w).double().cpu() - want).abs() <= bound).all()
+    if 1e-2 < of_x * of_w < 1e2:
+        g, u = want.split(N, dim=1)
+        got = ops.gated_linear(x, w).double().cpu()
+        # (SiLU's slope is at most 1.1, its own float arithmetic a few roundings)
+        slack = 1.1 * bound[:, :N] * u.abs() + torch.nn.functional.silu(g).abs() * bound[:, N:] + 2.0 ** -21 * (g * u).abs() + 2.0 ** -60
+        assert ((got - torch.nn.functional.silu(g) * u).abs() <= slack).all()
+
+
+def test_float32_linear_of_entries_whose_smallest_parts_are_largest(ops):
+    """1 + 2^-8 - 2^-17, whose products lose most by the part products that are not made (2^-24 of a term), and its negative."""
+    a = 1 + 2.0 ** -8 - 2.0 ** -17
+    for M, N, K in ((1, 16, 32), (5, 40, 256), (70, 300, 1024)):
+        x, w = torch.full((M, K), a, device="cuda"), torch.full((N, K), a, device="cuda")
+        w[N // 2:] *= -1
+        want = x.double().cpu() @ w.double().cpu().T
+        assert ((ops.linear(x, w).double().cpu() - want).abs() <= (6 * -(-K // 32) + 10) * 2.0 ** -24 * want.abs()).all()
+
+
 @pytest.mark.parametrize("N,K", [(1, 7), (40, 516), (520, 1024), (3072, 64), (9000, 36)])
 def test_float32_gated_linear_in_all_its_tiles(ops, N, K):
     """A gate of two products in one kernel: the bits of the packed product and the gate's own kernel, for every tile that the
