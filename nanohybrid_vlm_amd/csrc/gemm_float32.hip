@@ -17,8 +17,8 @@
 // What the factors 2^16 cost: one multiplication an entry taken apart, 3 % of a prompt of 517 tokens (0.6B shape), 1 % of decoding.
 //
 // The parts of an infinity are infinity and no numbers, and so are those of a number beyond 2^112. So an output that comes out
-// infinite (sums beyond 2^96 do) or as no number is summed once more by plain float multiply-adds, segment by segment: that
-// is what it is then. (Such inputs make every output of their row or column such a one.)
+// infinite (sums beyond 2^96 do) or as no number is summed once more by plain float multiply-adds: that is what it is then.
+// (Such inputs make every output of their row or column such a one.)
 //
 // Two kernels. Few rows, or few columns: a block is 8 waves and owns 16 RT rows by 16 CT columns, wave s sums segment s, and
 // LDS adds the segments up. Both operands come straight from memory (a lane: 16 bytes of each half of a row's 128); all loads
@@ -51,19 +51,43 @@ __device__ __forceinline__ f32x4 four_of(const float* __restrict__ row, int k, i
   return v;
 }
 
-// the same output by plain float multiply-adds (see above)
-__device__ __attribute__((noinline)) float plain_product(const float* __restrict__ x, const float* __restrict__ w, int K) {
-  const int length = segment_length(K);
-  float total = 0.f;
-  for (int begin = 0; begin < K; begin += length) {
-    float v = 0.f;
-    for (int k = begin; k < min(K, begin + length); ++k) v = fmaf(x[k], w[k], v);
-    total = begin ? total + v : v;
-  }
-  return total;
-}
-
 __device__ __forceinline__ bool finite(float v) { return fabsf(v) < INFINITY; }
+
+// Outputs (m, n), one a lane, of which the ``odd`` ones are made once more by plain float multiply-adds (see above): the wave takes one
+// after the other, lane l the columns l, l + 64, ..., and stops where a lane's sum is no number. A row of x or of w with an entry that is no
+// number settles all of the wave's outputs of that row. The order hangs on K alone. us, without such outputs, with one entry
+// of x that is no number, with one column of sums beyond 2^96, with nothing but infinities, with nothing but sums beyond 2^96: 517 x 4096 . 1024
+// 57, 64, 89, 720, 1730; 6 x 1024 . 3072 18, 20, 29, 51, 225 (by one lane an output: 204 and 230 with one such entry, 5,600 and 283 with infinities).
+__device__ __attribute__((noinline)) float plain_products(const float* __restrict__ x, const float* __restrict__ w, int K, float v, int m, int n, bool odd) {
+  const int lane = threadIdx.x & 63;
+  for (unsigned long long left = __ballot(odd); left;) {
+    const int from = __ffsll(left) - 1, row = __shfl(m, from, NHV_WAVE), column = __shfl(n, from, NHV_WAVE);
+    const float *xr = x + (size_t)row * K, *wr = w + (size_t)column * K;
+    float sum = 0.f;
+    bool x_none = false, w_none = false;
+    for (int k0 = lane; k0 - lane < K; k0 += 4 * 64) {
+      float a[4], b[4];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const int k = min(k0 + 64 * j, K - 1);
+        a[j] = xr[k], b[j] = wr[k];
+      }
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        x_none |= a[j] != a[j], w_none |= b[j] != b[j];
+        if (k0 + 64 * j < K) sum = fmaf(a[j], b[j], sum);
+      }
+      if (__any(sum != sum)) break;
+    }
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) sum += __shfl_xor(sum, o, NHV_WAVE);
+    x_none = __any(x_none), w_none = __any(w_none);
+    const bool settled = lane == from || (x_none && m == row) || (w_none && n == column);
+    if (odd && settled) v = sum;
+    left &= ~__ballot(settled);
+  }
+  return v;
+}
 
 template <int RT, int CT, int U, bool GATED, bool WIDE>
 __global__ __launch_bounds__(64 * SEGMENTS) void gemm_float32_kernel(const float* __restrict__ x, const float* __restrict__ w,
@@ -185,11 +209,17 @@ __global__ __launch_bounds__(64 * SEGMENTS) void gemm_float32_kernel(const float
         v[both] = part[0][at];
         for (int p = 1; p < active; ++p) v[both] += part[p][at];
       }
-      if (m < M && n < N) {
+      const bool in = m < M && n < N;
 #pragma unroll
-        for (int both = 0; both < (GATED ? 2 : 1); ++both) {
-          v[both] = finite(v[both]) ? v[both] * SPLIT_UNSCALE : plain_product(x + (size_t)m * K, w + ((size_t)both * N + n) * K, K);
-          if (bias) v[both] += bias[both * N + n];
+      for (int both = 0; both < (GATED ? 2 : 1); ++both) {
+        const bool odd = in && !finite(v[both]);
+        v[both] *= SPLIT_UNSCALE;
+        if (__any(odd)) v[both] = plain_products(x, w, K, v[both], m, both * N + n, odd);
+      }
+      if (in) {
+        if (bias) {
+#pragma unroll
+          for (int both = 0; both < (GATED ? 2 : 1); ++both) v[both] += bias[both * N + n];
         }
         y[(size_t)m * N + n] = GATED ? nhv_gated(v[0], v[GATED], gate) : v[0];
       }
@@ -325,13 +355,18 @@ __global__ __launch_bounds__(256, RT * CT > 2 ? 3 : 4) void gemm_float32_tiles_k
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         const int m = m0 + mw + 16 * r + 4 * g + i;
-        if (m < M && n < N) {
-          float v[GATED ? 2 : 1];
+        const bool in = m < M && n < N;
+        float v[GATED ? 2 : 1];
 #pragma unroll
-          for (int both = 0; both < (GATED ? 2 : 1); ++both) {
-            v[both] = total[r][c + both][i];
-            v[both] = finite(v[both]) ? v[both] * SPLIT_UNSCALE : plain_product(x + (size_t)m * K, w + ((size_t)both * N + n) * K, K);
-            if (bias) v[both] += bias[both * N + n];
+        for (int both = 0; both < (GATED ? 2 : 1); ++both) {
+          const bool odd = in && !finite(total[r][c + both][i]);
+          v[both] = total[r][c + both][i] * SPLIT_UNSCALE;
+          if (__any(odd)) v[both] = plain_products(x, w, K, v[both], m, both * N + n, odd);
+        }
+        if (in) {
+          if (bias) {
+#pragma unroll
+            for (int both = 0; both < (GATED ? 2 : 1); ++both) v[both] += bias[both * N + n];
           }
           y[(size_t)m * N + n] = GATED ? nhv_gated(v[0], v[GATED], gate) : v[0];
         }

@@ -364,6 +364,49 @@ def test_float32_linear_of_entries_whose_smallest_parts_are_largest(ops):
         assert ((ops.linear(x, w).double().cpu() - want).abs() <= (6 * -(-K // 32) + 10) * 2.0 ** -24 * want.abs()).all()
 
 
+@pytest.mark.parametrize("M,N,K", [(1, 40, 33), (7, 300, 1000), (40, 600, 260), (150, 4100, 70)])
+def test_float32_linear_of_sums_that_the_parts_cannot_hold(ops, M, N, K):
+    """Sums beyond 2^96, rows and columns with several infinities or entries that are no numbers side by side, and entries beyond 2^112:
+    what float64 gives (bound: K roundings of the sum of the terms' sizes), plain and gated, in every row and column."""
+    x, w = rnd(M, K, seed=115), rnd(2 * N, K, seed=116)
+    x[::3] *= 1e15
+    w[::2] *= 1e16
+    w[1::4] *= 1e20
+    if M > 6:
+        x[2, K // 2], x[3, 1], x[3, K - 1], x[5] = float("nan"), float("inf"), float("-inf"), 2e34
+    w[3, K - 1], w[6, 0], w[7, 5], w[11] = float("nan"), float("inf"), float("inf"), -3e35
+    want = x.double().cpu() @ w.double().cpu().T
+    size = x.double().cpu().abs().nan_to_num(0, 0, 0) @ w.double().cpu().abs().nan_to_num(0, 0, 0).T
+    got = ops.linear(x, w).double().cpu()
+    sure = torch.isnan(want) | (size < 3e38)                 # (terms or sums on the way beyond the largest float: either way)
+    assert torch.equal(torch.isnan(got)[sure], torch.isnan(want)[sure]) and torch.equal(torch.isposinf(got)[sure], torch.isposinf(want)[sure])
+    near = torch.isfinite(want) & sure
+    assert near.any() and ((got - want).abs()[near] <= (K * 2.0 ** -24 * size + 2.0 ** -149)[near]).all()
+    gated, packed = ops.gated_linear(x, w), ops.act_mul(ops.linear(x, w), "silu")
+    assert torch.equal(gated.isnan(), packed.isnan()) and torch.equal(gated.nan_to_num(1.5, 2.5, 3.5), packed.nan_to_num(1.5, 2.5, 3.5))
+
+
+@pytest.mark.parametrize("M,N,K", [(1, 151936, 1024), (6, 1024, 3072), (517, 4096, 1024)])
+def test_a_row_that_is_no_number_does_not_hold_up_a_float32_product(ops, M, N, K):
+    """Twice the product's time and 20 us at most (each output of such a row by one thread took 3 to 14 times as long)."""
+    x, w = rnd(M, K, seed=117), rnd(N, K, seed=118)
+
+    def shortest():
+        times = []
+        for _ in range(12):
+            start, end = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            start.record()
+            ops.linear(x, w)
+            end.record()
+            end.synchronize()
+            times.append(start.elapsed_time(end))
+        return min(times)
+
+    clean = shortest()
+    x[M // 2, K // 3] = float("nan")
+    assert shortest() <= 2 * clean + 0.02
+
+
 @pytest.mark.parametrize("N,K", [(1, 7), (40, 516), (520, 1024), (3072, 64), (9000, 36)])
 def test_float32_gated_linear_in_all_its_tiles(ops, N, K):
     """A gate of two products in one kernel: the bits of the packed product and the gate's own kernel, for every tile that the
