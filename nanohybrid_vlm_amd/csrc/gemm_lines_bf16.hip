@@ -116,13 +116,15 @@ __global__ __launch_bounds__(512) void gemm_lines_kernel(const bf16_t* __restric
 
 struct Plan {
   int mt, nt, splits;                                                // mt == 0: not for these kernels
+  long long blocks;
+  double taken_in;                                                   // us that a compute unit's share takes to come in
 };
 
 // The tile and the splits that take the least time by what was measured (17 to 128 rows of the 0.6B to 8B shapes' products): a
 // launch's ends, what a compute unit takes in at 32 GB/s or the whole chip of w at 5.3 TB/s, whichever is longer, the parts' way
 // to memory and back at 3.5 TB/s, and what a norm's block, which has a whole row to read, takes longer for them.
 static Plan plan(int M, int N, int K, bool gated) {
-  Plan best = {0, 0, 0};
+  Plan best = {0, 0, 0, 0, 0.0};
   // (gated products of 128 rows 62.7 us at the 8B shape, the library's product and the gate's kernel 54; of 96 rows 44.5 against 47.5
   // there, and inside a step of the 4B shape 31.0 against 34.6. Of 128 rows wide products are slower too, 6,144 of 4,096 21.9
   // against 21.4, narrow ones not: 4,096 of 12,288 34 against 44.)
@@ -138,10 +140,27 @@ static Plan plan(int M, int N, int K, bool gated) {
       const double taken_in = (double)rounds * (mt + nt) * 32 * ((K / CHUNK + splits - 1) / splits * CHUNK) / 32e3;
       const double of_w = 2.0 * (gated ? 2 : 1) * N * K / 5.3e6;
       const double time = (taken_in > of_w ? taken_in : of_w) + (gated ? 0.0 : 8.0 * splits * M * N / 3.5e6 + 4.0 * splits * N / 40e3);
-      if (time < least) least = time, best = {mt, nt, splits};
+      if (time < least) least = time, best = {mt, nt, splits, blocks, taken_in};
     }
   }
   return best;
+}
+
+// Where these kernels are the faster way: by 17, 32, 48, 64, 79, 96, 112 and 128 rows of 259 products, the 0.6B to 32B shapes and random
+// ones of 64 to 36,864 outputs and 256 to 28,672 columns, each beside the fastest of the library's algorithms (gated: and the gate's
+// kernel; plain: both with the norm that follows), cold weights; time by lines over the library's in brackets.
+// Gated: one round of blocks. Where a second one begins the units that have none wait (17,408 outputs of 5,120 columns 1.08 to 1.27,
+// 25,600 of 5,120 1.04 to 1.46, 13,824 of 5,120 from 48 rows on 1.07 to 1.17); where less than 144 blocks walk over many columns the others
+// are idle from the start, K being whole (2,048 of 16,384 1.19 to 1.47, 960 of 9,856 up to 1.3, 1,024 of 4,096 1.2), unless the walk
+// is a short one. 425 of the 726 are taken, 0.77 on average, the worst 1.04.
+// Plain: up to 12,288 outputs (16,384 of 16,384 up to 1.22, 20,480 of 5,120 up to 1.10), two rounds of blocks (13,840 of 15,744 in eight parts up
+// to 1.38, 8,192 of 28,672 at 112 rows 1.19), of more than 96 rows up to 8,192 outputs (10,256 of 14,464 1.06), and of more than 64 not the
+// smallest products (376 of 384 up to 1.12, a microsecond). 890 of the 1,028 are taken, 0.75 on average, the
+// worst 1.08 (112 rows of 300 outputs, 1.3 us). Sizes drawn after the rules were set, 827 measurements with these: gated 0.75, worst 1.09 (0.8 us),
+// plain 0.76, worst 1.07.
+static bool pays(const Plan& p, int M, int N, int K, bool gated) {
+  if (gated) return p.blocks <= 256 && K <= 12288 && (p.blocks >= 144 || p.taken_in <= 10.0);
+  return p.blocks <= 512 && N <= 12288 && K <= 32768 && (M <= 96 || N <= 8192) && (M <= 64 || (long long)N * K >= 1 << 18);
 }
 
 template <int MT, int NT, bool GATED>
@@ -175,8 +194,11 @@ static int launch_rows(const Plan& p, bool gated, const void* x, const void* w, 
 
 }  // namespace lines
 
-// How many parts these kernels make of a product (1: a gated one's finished rows); 0: it is not for them.
-extern "C" int nhv_gemm_lines_splits(int M, int N, int K, int gated) { return lines::plan(M, N, K, gated != 0).splits; }
+// How many parts these kernels make of a product (1: a gated one's finished rows); ``whenever`` 0: 0 where another way is the faster one.
+extern "C" int nhv_gemm_lines_splits(int M, int N, int K, int gated, int whenever) {
+  const lines::Plan p = lines::plan(M, N, K, gated != 0);
+  return p.mt > 0 && (whenever || lines::pays(p, M, N, K, gated != 0)) ? p.splits : 0;
+}
 
 // gated: y[M, N] in bfloat16; else y[splits][M][N] in float, whose sum over the splits is the product.
 extern "C" int nhv_gemm_lines_bf16(const void* x, const void* w, const void* bias, void* y, int M, int N, int K, int gated, int act, float limit,

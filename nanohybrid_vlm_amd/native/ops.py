@@ -822,14 +822,14 @@ class NativeBackend:
                    dtype_code(out), _stream())
 
     def _by_lines(self, x, w, N: int, gated: bool) -> int:
-        """How many parts the kernels for 17 to 128 rows make of this product (1: a gated one's rows); 0: they do not do it. They are
-        faster than the best of the library's algorithms for every shape they take, so nothing is measured; a table
+        """How many parts the kernels for 17 to 128 rows make of this product (1: a gated one's rows); 0: another way is the faster one
+        (by what was measured over sizes, gemm_lines_bf16.hip), and how the product is done is ``linear``'s matter. A table
         that names an algorithm for the shape is followed as it stands."""
         M, K = x.shape
         if not (self.few_rows < M <= 128 and x.dtype == torch.bfloat16 and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0):
             return 0
         how = self.chosen.get((M, w.shape[0], K, False, False))
-        return 0 if how is not None and how >= 0 else self.lib.nhv_gemm_lines_splits(M, N, K, int(gated))
+        return 0 if how is not None and how >= 0 else self.lib.nhv_gemm_lines_splits(M, N, K, int(gated), int(self.own_kernels_only))
 
     def linear_parts(self, x, w):
         """x W^T as float parts [parts, rows, out] whose sum it is, or None where another way is the faster one."""

@@ -1296,14 +1296,33 @@ def test_products_by_lines(ops, M, N, K):
     for part in got.parts[1:]:
         total += part
     assert torch.equal(ops.dense(got), total.bfloat16())
-    if M <= 96:
+    if M <= 96:                                              # (also where the library's way is the faster one)
         out = torch.full((M, N), float("nan"), dtype=torch.bfloat16, device="cuda")
-        assert ops.backend().gated_linear(x, w, out)
+        by_lines = ops.backend().lib.nhv_gemm_lines_bf16
+        assert by_lines(ops._ptr(x), ops._ptr(w), ops._ptr(None), ops._ptr(out), M, N, K, 1, *ops.Gate().args(), ops._stream()) == 0
         torch.testing.assert_close(out.double(), torch.nn.functional.silu(both[:, :N]) * both[:, N:], **tol(torch.bfloat16))
         gate = ops.Gate(2, 1.5, 1.702, 1.0)
         g, u = (both + b.double()).split(N, dim=1)
         g, u = g.clamp(max=1.5), u.clamp(-1.5, 1.5)
-        torch.testing.assert_close(ops.gated_linear(x, w, gate, b).double(), g * torch.sigmoid(1.702 * g) * (u + 1), **tol(torch.bfloat16))
+        assert by_lines(ops._ptr(x), ops._ptr(w), ops._ptr(b), ops._ptr(out), M, N, K, 1, *gate.args(), ops._stream()) == 0
+        torch.testing.assert_close(out.double(), g * torch.sigmoid(1.702 * g) * (u + 1), **tol(torch.bfloat16))
+
+
+@pytest.mark.parametrize("M,N,K,parts,gated", [
+    # the 0.6B to 8B shapes' products; gated ones of one round of blocks and of two, of few blocks over few columns and many
+    (17, 4096, 1024, True, True), (96, 3072, 1024, True, True), (64, 4096, 12288, True, True), (64, 12288, 4096, True, True),
+    (32, 17408, 5120, False, False), (96, 13824, 5120, False, False), (64, 25600, 1024, False, False), (79, 1024, 4096, True, False),
+    (48, 512, 1024, True, True), (17, 2040, 9344, True, False),
+    # more outputs than the plain ones are taken for, more blocks, more rows, the smallest
+    (32, 12296, 1024, False, False), (96, 8832, 28672, False, False), (112, 8704, 9216, False, False), (112, 5120, 17408, True, False),
+    (79, 376, 384, False, True), (64, 376, 384, True, True),
+])
+def test_which_products_go_by_lines(ops, M, N, K, parts, gated):
+    """As parts and as a gate, where that was measured to be the faster way; elsewhere rows that the library (or torch) makes."""
+    x, w = (torch.zeros(r, K, dtype=torch.bfloat16, device="cuda") for r in (M, 2 * N))
+    assert isinstance(ops.linear(x, w[:N], parts=True), ops.Parts) == parts
+    out = torch.empty(M, N, dtype=torch.bfloat16, device="cuda")
+    assert ops.backend().gated_linear(x, w, out) == gated
 
 
 @pytest.mark.parametrize("M,band,last,K", [(1, 1024, 32, 2048), (16, 2048, 5, 2304), (7, 1056, 1100, 2048)])
