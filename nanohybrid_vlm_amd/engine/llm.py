@@ -199,7 +199,7 @@ class LLM:
 
     def gemm_choices(self) -> dict:
         """How each shape of matrix product that this engine's table holds is done ("M,N,K,float result,gated" ->
-        -1 own kernel, -2 the rule, or a library algorithm's number)."""
+        -1 own kernel, -2 the rule, or a library algorithm's number; gated 2: a product that its reader takes as parts)."""
         from ..native import ops
         backend = ops.backend()
         if not hasattr(backend, "choices_table"):

@@ -29,6 +29,8 @@ ATTENTION_HEAD_DIMS_BUILT_AHEAD = [16, 32, 48, 64, 80, 96, 112, 128, 256]
 F32, BF16 = 0, 1
 # a measured choice for a matrix product: the own kernel, or what the rule gives (0, 1, ...: that algorithm of the library's list)
 OWN, RULE = -1, -2
+# in the place of "gated" in a product's key: its result may come as ``Parts``
+AS_PARTS = 2
 _DTYPE_CODE = {torch.float32: F32, torch.bfloat16: BF16}
 
 
@@ -161,7 +163,7 @@ class NativeBackend:
         self.lib = library.load_library("nhv_core", CORE_SOURCES)
         self.lib.nhv_last_error.restype = ctypes.c_char_p
         self._attention_libs: dict[int, ctypes.CDLL] = {}
-        # (M, N, K, float result, gated) of a product -> OWN, RULE or a library algorithm, measured. ``chosen`` is the
+        # (M, N, K, float result, gated or AS_PARTS) of a product -> OWN, RULE or a library algorithm, measured. ``chosen`` is the
         # table in force: the process-wide one that engines share by default (a shape is timed once per process), or
         # the table of the engine that runs now (see ``use_choices``)
         self.shared_chosen: dict[tuple, int] = {}
@@ -751,7 +753,7 @@ class NativeBackend:
     # -- the table of choices, so that a process can run by what another one measured --
     def choices_table(self, chosen: dict | None = None) -> dict[str, int]:
         """A table of choices (default: the one in force), by shape: "M,N,K,float result,gated" -> -1 (own kernel),
-        -2 (the rule: ``torch.mm``) or the number of a library algorithm."""
+        -2 (the rule: ``torch.mm``) or the number of a library algorithm. gated 2: a product that its reader takes as parts."""
         chosen = self.chosen if chosen is None else chosen
         return {",".join(str(int(v)) for v in key): how for key, how in sorted(chosen.items())}
 
@@ -770,7 +772,7 @@ class NativeBackend:
                 _, count = self._library_plan(M, N, K, bool(f) and not bool(g))
                 if how >= count:
                     raise KernelError(f"choice {how} for the product '{text}': the library names {count} algorithms for this shape")
-            out[(M, N, K, bool(f), bool(g))] = how
+            out[(M, N, K, bool(f), g if g == AS_PARTS else bool(g))] = how
         return out
 
     def use_choices(self, table: dict | None, measuring: bool) -> None:
@@ -823,13 +825,24 @@ class NativeBackend:
 
     def _by_lines(self, x, w, N: int, gated: bool) -> int:
         """How many parts the kernels for 17 to 128 rows make of this product (1: a gated one's rows); 0: another way is the faster one
-        (by what was measured over sizes, gemm_lines_bf16.hip), and how the product is done is ``linear``'s matter. A table
-        that names an algorithm for the shape is followed as it stands."""
+        (by what was measured over sizes, gemm_lines_bf16.hip), and how the product is done is ``linear``'s matter. It hangs on the
+        shape, not on what was measured for others before. Only a table read from a file (nothing is measured then) may say
+        otherwise: it names how the gated product, or the one that may come as parts, is done, or, if it lacks that, a library
+        algorithm for the shape."""
         M, K = x.shape
         if not (self.few_rows < M <= 128 and x.dtype == torch.bfloat16 and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0):
             return 0
-        how = self.chosen.get((M, w.shape[0], K, False, False))
-        return 0 if how is not None and how >= 0 else self.lib.nhv_gemm_lines_splits(M, N, K, int(gated), int(self.own_kernels_only))
+        splits = self.lib.nhv_gemm_lines_splits(M, N, K, int(gated), int(self.own_kernels_only))
+        if not splits or self.own_kernels_only:
+            return splits
+        key = (M, w.shape[0], K, False, True if gated else AS_PARTS)
+        if self.measuring_allowed:
+            self.chosen[key] = OWN                           # (a process that reads this table does it the same way)
+            return splits
+        how = self.chosen.get(key)
+        if how is None:
+            how = self.chosen.get((M, w.shape[0], K, False, False))
+        return 0 if how is not None and how >= 0 else splits
 
     def linear_parts(self, x, w):
         """x W^T as float parts [parts, rows, out] whose sum it is, or None where another way is the faster one."""

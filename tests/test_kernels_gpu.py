@@ -1325,6 +1325,36 @@ def test_which_products_go_by_lines(ops, M, N, K, parts, gated):
     assert ops.backend().gated_linear(x, w, out) == gated
 
 
+def test_what_goes_by_lines_hangs_on_the_shape_and_on_a_table_that_is_read(ops):
+    """A library algorithm measured for the same shape's rows changes nothing; a table from a file that names one is followed, unless it
+    says that the own kernel made the product where its reader took parts, or the gate."""
+    backend = ops.backend()
+    M, N, K = 40, 2048, 1024
+    x, w = rnd(M, K, dtype=torch.bfloat16, seed=121), rnd(2 * N, K, dtype=torch.bfloat16, seed=122, scale=K ** -0.5)
+    out = torch.empty(M, N, dtype=torch.bfloat16, device="cuda")
+
+    def ways():
+        return isinstance(ops.linear(x, w[:N], parts=True), ops.Parts), backend.gated_linear(x, w, out)
+
+    saved, allowed, chosen = dict(backend.shared_chosen), backend.measuring_allowed, backend.chosen
+    try:
+        backend.shared_chosen.clear()
+        backend.use_choices(None, True)
+        assert ways() == (True, True)
+        written = backend.choices_table()
+        assert written == {f"{M},{N},{K},0,2": -1, f"{M},{2 * N},{K},0,1": -1}
+        algorithms = {f"{M},{N},{K},0,0": 0, f"{M},{2 * N},{K},0,0": 0}
+        backend.shared_chosen.update(backend.parse_choices(algorithms))        # (as if measured for a plain product)
+        assert ways() == (True, True)
+        for table, want in (({}, (True, True)), (algorithms, (False, False)), ({**algorithms, **written}, (True, True))):
+            backend.use_choices(backend.parse_choices(table), False)
+            assert ways() == want and backend.choices_table() == table
+    finally:
+        backend.shared_chosen.clear()
+        backend.shared_chosen.update(saved)
+        backend.chosen, backend.measuring_allowed = chosen, allowed
+
+
 @pytest.mark.parametrize("M,band,last,K", [(1, 1024, 32, 2048), (16, 2048, 5, 2304), (7, 1056, 1100, 2048)])
 def test_products_in_bands_by_lines(ops, M, band, last, K):
     """Five sets of rows against a matrix's bands, where the kernel by lines takes them (float sums of K products of size K^-1/2)."""
