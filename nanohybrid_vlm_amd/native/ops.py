@@ -1195,6 +1195,11 @@ def soft_cap_(logits: torch.Tensor, cap: float) -> torch.Tensor:
     return logits
 
 
+def norm_takes_parts(width: int, w: torch.Tensor, residual: torch.Tensor) -> bool:
+    """Whether ``rmsnorm`` adds a product's parts to the residual stream itself: rows of whole 16 bytes on 16-byte boundaries."""
+    return width % 8 == 0 and w.data_ptr() % 16 == 0 and residual.data_ptr() % 16 == 0
+
+
 def rmsnorm(x: torch.Tensor, w: torch.Tensor, eps: float, residual: torch.Tensor | None = None,
             start_residual: bool = False, residual_float32: bool = True, rounds_between: bool = True):
     """``rmsnorm(x, w, eps)``: the norm of x.
@@ -1206,7 +1211,7 @@ def rmsnorm(x: torch.Tensor, w: torch.Tensor, eps: float, residual: torch.Tensor
     again; False: it is rounded once, at the end.
     ``x`` may be ``Parts`` (with ``residual``)."""
     if isinstance(x, Parts):
-        if residual is None or x.shape[1] % 8 or w.data_ptr() % 16 or residual.data_ptr() % 16:
+        if residual is None or not norm_takes_parts(x.shape[1], w, residual):
             return rmsnorm(x.tensor(), w, eps, residual, start_residual, residual_float32, rounds_between)
         _need(not start_residual, "rmsnorm: a residual is either started or added to")
         _dense(w, "rmsnorm: weight", (x.shape[1],))
@@ -1261,6 +1266,13 @@ def gather_rows(x: torch.Tensor, rows: torch.Tensor) -> torch.Tensor:
     return out
 
 
+def rotation_takes_parts(head_dim: int, cos_sin, pair_axes, *others) -> bool:
+    """Whether ``qk_rope_write`` adds up a projection's parts itself: its kernel for that takes whole heads of a power of two entries, turned whole
+    or not at all, in 16 bytes a lane. ``others``: the tensors that it reads or writes beside the rotation table."""
+    whole = 16 <= head_dim <= 512 and head_dim & (head_dim - 1) == 0 and (cos_sin is None or cos_sin.shape[1] == head_dim) and pair_axes is None
+    return whole and all(t is None or t.data_ptr() % 16 == 0 for t in (cos_sin, *others))
+
+
 def qk_rope_write(qkv, bias, q_norm_w, k_norm_w, eps, cos_sin, positions, slot_mapping, k_cache, v_cache,
                   num_heads: int, num_kv_heads: int, head_dim: int, write_kv: bool = True,
                   pair_axes: torch.Tensor | None = None) -> torch.Tensor:
@@ -1272,11 +1284,8 @@ def qk_rope_write(qkv, bias, q_norm_w, k_norm_w, eps, cos_sin, positions, slot_m
     T = qkv.shape[0]
     width = (num_heads + 2 * num_kv_heads) * head_dim
     split = qkv if isinstance(qkv, Parts) else None
-    if split is not None:
-        whole = 16 <= head_dim <= 512 and head_dim & (head_dim - 1) == 0 and (cos_sin is None or cos_sin.shape[1] == head_dim) and pair_axes is None
-        starts = [t.data_ptr() for t in (bias, q_norm_w, k_norm_w, cos_sin, k_cache if write_kv else None, v_cache if write_kv else None) if t is not None]
-        if not whole or any(p % 16 for p in starts):         # (the kernel that takes parts asks for whole heads in 16 bytes a lane)
-            qkv, split = qkv.tensor(), None
+    if split is not None and not rotation_takes_parts(head_dim, cos_sin, pair_axes, bias, q_norm_w, k_norm_w, *((k_cache, v_cache) if write_kv else ())):
+        qkv, split = qkv.tensor(), None
     _dense(qkv if split is None else split.parts, "qk_rope_write: qkv", (T, width) if split is None else (split.parts.shape[0], T, width))
     if split is None:
         dtype_code(qkv)
@@ -1386,7 +1395,7 @@ def linear(x, w: torch.Tensor, bias: torch.Tensor | None = None, out_dtype=None,
     Where the product's kernel can, it makes the addition itself (in float; the stream is rewritten) and a ``Summed``
     is returned, which that norm takes; otherwise the plain result is returned and the stream is left alone, for some sizes
     as ``Parts``, which that norm takes too.
-    ``parts``: the caller takes ``Parts`` whatever it does with the result."""
+    ``parts``: the caller's next step adds parts up itself (a reader that does not costs one kernel more)."""
     normed = x if isinstance(x, Normed) else None
     if normed is not None:
         x = normed.summed.weighted
@@ -1415,7 +1424,7 @@ def linear(x, w: torch.Tensor, bias: torch.Tensor | None = None, out_dtype=None,
         backend().fused_linear(x, w, bias, None, row_scales=scales, residual=residual, sum_out=weighted, ss_out=squares,
                                next_w=add_to.norm_weight)
         return Summed(weighted, squares, residual, add_to.norm_weight, add_to.eps)
-    if (parts or add_to is not None) and normed is None and bias is None and out_dtype == x.dtype:
+    if (parts or (add_to is not None and norm_takes_parts(N, add_to.norm_weight, add_to.residual))) and normed is None and bias is None and out_dtype == x.dtype:
         make = getattr(backend(), "linear_parts", None)
         made = None if make is None else make(x, w)
         if made is not None:

@@ -244,3 +244,28 @@ def test_builtin_parts_alone(dtype):
     rope = RotaryEmbedding(rotary_dim=24, max_position=50, base=500.0)
     ang = plain.rope_angles(torch.arange(50), 24, 500.0)
     torch.testing.assert_close(rope.rotation_table(), torch.cat((ang.cos(), ang.sin()), -1))
+
+
+@pytest.mark.parametrize("name,asked", [("A", {128, 64}), ("C", {80})])
+def test_products_come_as_parts_where_their_reader_adds_them_up(model_folders, emulated_kernels, name, asked):
+    """A head size that is no power of two (C: 48; its projection of 720 outputs) has a rotation kernel that reads rows: parts would be added
+    up by a kernel between. The output projection and the down projection (64 and 80 outputs) go to a norm."""
+    from nanohybrid_vlm_amd.engine.runner import ModelRunner, StepEntry
+    from nanohybrid_vlm_amd.native import ops
+    widths = set()
+    ops.backend().linear_parts = lambda x, w: widths.add(w.shape[0])
+    runner = ModelRunner(model_folders[name], dtype="float32", device="cpu", page_size=4, num_pages=16)
+    runner.step([StepEntry("r", list(range(20)), [19])])
+    assert widths == asked
+
+
+def test_a_norm_of_odd_width_is_not_given_parts(emulated_kernels):
+    """Rows that do not begin on 16 bytes, and a residual stream or a weight that does not."""
+    from nanohybrid_vlm_amd.native import ops
+    asked = []
+    ops.backend().linear_parts = lambda x, w: asked.append(w.shape[0])
+    for width, off, weight_off, want in ((24, 0, 0, True), (20, 0, 0, False), (24, 1, 0, False), (24, 0, 1, False)):
+        x, w = torch.randn(3, 8), torch.randn(width, 8)
+        residual, weight = torch.zeros(3 * width + 1)[off:off + 3 * width].view(3, width), torch.ones(width + 1)[weight_off:weight_off + width]
+        ops.linear(x, w, add_to=ops.AddTo(residual, weight, 1e-6))
+        assert (asked == [width]) == want and asked.clear() is None
