@@ -1077,6 +1077,7 @@ class AddTo:
     norm_weight: torch.Tensor
     eps: float
     reader: tuple | None = None
+    takes_parts: bool = False     # the norm, and whoever hands the result on to it, know ``Parts``
 
 
 @dataclass
@@ -1394,7 +1395,7 @@ def linear(x, w: torch.Tensor, bias: torch.Tensor | None = None, out_dtype=None,
     ``add_to``: the residual stream [M, N] that the caller is about to add the result to, and the norm that follows.
     Where the product's kernel can, it makes the addition itself (in float; the stream is rewritten) and a ``Summed``
     is returned, which that norm takes; otherwise the plain result is returned and the stream is left alone, for some sizes
-    as ``Parts``, which that norm takes too.
+    as ``Parts`` if ``add_to`` says that the norm takes those too.
     ``parts``: the caller's next step adds parts up itself (a reader that does not costs one kernel more)."""
     normed = x if isinstance(x, Normed) else None
     if normed is not None:
@@ -1424,7 +1425,9 @@ def linear(x, w: torch.Tensor, bias: torch.Tensor | None = None, out_dtype=None,
         backend().fused_linear(x, w, bias, None, row_scales=scales, residual=residual, sum_out=weighted, ss_out=squares,
                                next_w=add_to.norm_weight)
         return Summed(weighted, squares, residual, add_to.norm_weight, add_to.eps)
-    if (parts or (add_to is not None and norm_takes_parts(N, add_to.norm_weight, add_to.residual))) and normed is None and bias is None and out_dtype == x.dtype:
+    if add_to is not None and add_to.takes_parts:
+        parts = parts or norm_takes_parts(N, add_to.norm_weight, add_to.residual)
+    if parts and normed is None and bias is None and out_dtype == x.dtype:
         make = getattr(backend(), "linear_parts", None)
         made = None if make is None else make(x, w)
         if made is not None:

@@ -41,12 +41,18 @@ class PreNormBlock(Part):
         already): this block's first norm has to know what that is. A block that says so takes ``next_norm=``."""
         return getattr(self.mixer_norm, "takes_summed", False)
 
+    @property
+    def takes_parts(self) -> bool:
+        """Whether ``hidden`` may come as an ``ops.Parts`` (the block before has left its last product's parts to be added up)."""
+        return getattr(self.mixer_norm, "takes_parts", False)
+
     def forward(self, hidden, residual, step, cache, next_norm=None, next_reader=None):
         """``next_norm``: the norm that takes this block's result next (the next block's first norm, or the model's
-        last), if it takes an ``ops.Summed`` in place of ``hidden``; ``next_reader``: the part that reads that norm."""
+        last), if it takes an ``ops.Summed`` in place of ``hidden`` (and an ``ops.Parts``, if it says ``takes_parts``); ``next_reader``:
+        the part that reads that norm."""
         # A mixer or feed-forward that says ``adds_to_residual`` takes ``add_to=`` (the residual stream and the norm
         # that follows, ``ops.AddTo``) and may let its last product make the addition (it then returns an
-        # ``ops.Summed``); one that says ``takes_deferred_norm`` may get an ``ops.Normed`` as its input, whose rows
+        # ``ops.Summed``) or leave its parts to the norm (an ``ops.Parts``, where the norm says ``takes_parts``); one that says ``takes_deferred_norm`` may get an ``ops.Normed`` as its input, whose rows
         # its first product scales. Parts that say neither get tensors and return tensors.
         mixer, ff = self.mixer, self.feed_forward
         if residual is None:
@@ -71,8 +77,10 @@ def _add_to(part, norm, residual, reader) -> dict:
     """The argument that lets ``part`` make the addition that ``norm`` would make, if both are made for that.
     ``reader``: the part that reads ``norm`` (it counts only if it takes the norm with its scaling left to do)."""
     if norm is not None and getattr(part, "adds_to_residual", False) and getattr(norm, "takes_summed", False):
-        return {"add_to": norm.add_to(residual, reader if getattr(reader, "takes_deferred_norm", False) else None)}
+        more = {"takes_parts": True} if getattr(norm, "takes_parts", False) else {}
+        return {"add_to": norm.add_to(residual, reader if getattr(reader, "takes_deferred_norm", False) else None, **more)}
     return {}
+
 
 
 @BLOCKS.register("parallel_depth_mix")

@@ -16,6 +16,7 @@ from dataclasses import replace
 
 from .base import (BLOCKS, EMBEDDINGS, FEED_FORWARDS, MIXERS, NORMS, POSITION_ENCODINGS, CacheView, CombinedNeed, PagedKVNeed, ParamSpec,
                    Part, StateNeed)
+from .norms import WithoutParts
 
 
 @dataclass
@@ -215,7 +216,8 @@ class DecoderModel(Part):
                 else:
                     nxt = self.layers[order[i + 1].layer]
                     if getattr(nxt, "takes_summed", False):
-                        more["next_norm"], more["next_reader"] = nxt.mixer_norm, nxt.mixer
+                        norm = nxt.mixer_norm
+                        more["next_norm"], more["next_reader"] = norm if getattr(nxt, "takes_parts", False) else WithoutParts(norm), nxt.mixer
             elif getattr(layer, "norms_ahead", False) and i + 1 < len(order):
                 # a block that can norm what it hands on for the block that follows: that block's (one) norm
                 more["next_norm"] = getattr(self.layers[order[i + 1].layer], "norm", None)

@@ -13,6 +13,7 @@ class RMSNorm(Part):
     and carried on (layernorm.py:28-40)."""
 
     takes_summed = True           # ``forward_add`` takes an ``ops.Summed`` (a sum that a product has made already)
+    takes_parts = True            # ... and an ``ops.Parts`` (a product whose parts are still to be added up)
     defers_to_products = True     # ``forward_add(..., deferred=True)`` may return an ``ops.Normed``
 
     def __init__(self, size: int, eps: float, residual_float32: bool = True, rounds_between: bool = True):
@@ -39,18 +40,19 @@ class RMSNorm(Part):
     def forward(self, x) -> torch.Tensor:
         return ops.rmsnorm(ops.dense(x), self.weight, self.eps, rounds_between=self.rounds_between)
 
-    def add_to(self, residual: torch.Tensor, reader=None) -> ops.AddTo:
+    def add_to(self, residual: torch.Tensor, reader=None, takes_parts: bool = False) -> ops.AddTo:
         """What the part before this norm is handed so that its last product can make the addition to ``residual``
         and this norm's product with its weight (``forward_add`` then gets an ``ops.Summed``). ``reader``: the part
-        that reads this norm, if it says what its first product is (``first_product()``)."""
+        that reads this norm, if it says what its first product is (``first_product()``). ``takes_parts``: whoever hands the
+        product's result on to this norm does so with an ``ops.Parts`` as well."""
         first = getattr(reader, "first_product", None)
-        return ops.AddTo(residual, self.weight, self.eps, first() if first is not None else None)
+        return ops.AddTo(residual, self.weight, self.eps, first() if first is not None else None, takes_parts)
 
     def forward_add(self, x, residual: torch.Tensor, deferred: bool = False):
         """Returns (norm(x + residual), x + residual); ``residual`` is updated in place. ``x`` may be the
         ``ops.Summed`` that a product made from this norm's ``add_to``: the sum is in ``residual`` already, and what
-        is left of the norm is the scaling of the rows. ``deferred``: the caller's next step is a product, which
-        scales its rows itself; it then gets an ``ops.Normed`` in place of a tensor."""
+        is left of the norm is the scaling of the rows; or an ``ops.Parts``, whose parts are added up here. ``deferred``: the caller's
+        next step is a product, which scales its rows itself; it then gets an ``ops.Normed`` in place of a tensor."""
         if isinstance(x, ops.Summed):
             if x.norm_weight is not self.weight or x.residual is not residual:
                 raise ValueError("a sum that a product made for another norm, or into another residual stream")
@@ -58,6 +60,18 @@ class RMSNorm(Part):
             return (normed if deferred else normed.tensor()), residual
         y = ops.rmsnorm(x, self.weight, self.eps, residual=residual, rounds_between=self.rounds_between)
         return y, residual
+
+
+class WithoutParts:
+    """A norm as it is named to the block before one that takes an ``ops.Summed`` and does not know ``ops.Parts``."""
+
+    takes_parts = False
+
+    def __init__(self, norm):
+        self.norm = norm
+
+    def __getattr__(self, name):
+        return getattr(self.norm, name)
 
 
 @NORMS.register("scalar_rmsnorm")

@@ -267,5 +267,32 @@ def test_a_norm_of_odd_width_is_not_given_parts(emulated_kernels):
     for width, off, weight_off, want in ((24, 0, 0, True), (20, 0, 0, False), (24, 1, 0, False), (24, 0, 1, False)):
         x, w = torch.randn(3, 8), torch.randn(width, 8)
         residual, weight = torch.zeros(3 * width + 1)[off:off + 3 * width].view(3, width), torch.ones(width + 1)[weight_off:weight_off + width]
-        ops.linear(x, w, add_to=ops.AddTo(residual, weight, 1e-6))
+        ops.linear(x, w, add_to=ops.AddTo(residual, weight, 1e-6, takes_parts=True))
         assert (asked == [width]) == want and asked.clear() is None
+
+
+def test_parts_go_only_to_norms_and_blocks_that_say_so(model_folders, emulated_kernels):
+    """A block or a norm from outside that knows ``ops.Summed`` alone gets no ``ops.Parts``: its predecessor's product gives rows."""
+    from nanohybrid_vlm_amd.engine.runner import ModelRunner, StepEntry
+    from nanohybrid_vlm_amd.native import ops
+    from nanohybrid_vlm_amd.parts.blocks import PreNormBlock
+    from nanohybrid_vlm_amd.parts.norms import RMSNorm
+    asked = []
+    ops.backend().linear_parts = lambda x, w: asked.append(tuple(w.shape))
+    runner = ModelRunner(model_folders["A"], dtype="float32", device="cpu", page_size=4, num_pages=16)
+
+    def added():
+        asked.clear()
+        logits = runner.step([StepEntry(len(runs), list(range(20)), [19])])
+        runs.append(logits)
+        return [shape for shape in asked if shape[0] == 64]
+
+    runs, out, down = [], (64, 64), (64, 128)
+    assert added() == [out, down] * 2
+    layer = runner.model.layers[1]
+    layer.__class__ = type("Outside", (PreNormBlock,), {"takes_parts": False})
+    assert added() == [out, out, down]
+    layer.feed_forward_norm.__class__ = type("OutsideNorm", (RMSNorm,), {"takes_parts": False, "add_to": lambda self, residual, reader=None: (
+        RMSNorm.add_to(self, residual, reader))})
+    assert added() == [out, down]
+    assert all(torch.equal(r, runs[0]) for r in runs)
