@@ -980,7 +980,14 @@ __global__ __launch_bounds__(512) void gemm_fewrows_lines_kernel(const bf16_t* _
   for (int t = 0; t < LOADS; ++t)
     src[t] = (t < NT ? w + ((size_t)(GATED ? t * N : 0) + min(n0 + (GATED ? 0 : 16 * t) + my_row, N - 1)) * K : x + (size_t)min(my_row, M - 1) * K) + piece * 8;
   const uint32_t ring_at = nhv_lds_address(ring) + wave * 1024;
-  const int first = nhv_first_chunk(blockIdx.x, chunks, K);
+  // Float results are logits, and equal rows of w (unused tokens' embeddings) have to give equal ones, or rounding would choose
+  // between them: there the sums do not begin where the block does. The columns are STRETCHES stretches, a block begins with one
+  // of them, and each is summed by itself and added to the others in their order. us at 1 and 16 rows without the turning, with
+  // it, with it and two, four and eight stretches: 151,936 outputs of 4,096 columns 246 and 252, 187 and 192, 196 and 199, 187
+  // and 191, 198 and 205; 151,936 of 2,048 120 and 128, 97 and 113, 98 and 115, 97 and 114, 132 and 140 (an eighth is one chunk).
+  constexpr int STRETCHES = sizeof(TOut) == 4 ? 4 : 1;
+  const bool stretches = STRETCHES > 1 && K % 2048 == 0;
+  const int length = stretches ? chunks / STRETCHES : chunks + 1, place = nhv_first_chunk(blockIdx.x, chunks, K), first = stretches ? place / length * length : place;
   auto ask = [&](int buf, int c) {
     const size_t k = (size_t)nhv_chunk(first, c, chunks) * CHUNK;
 #pragma unroll
@@ -989,21 +996,45 @@ __global__ __launch_bounds__(512) void gemm_fewrows_lines_kernel(const bf16_t* _
       else nhv_load_to_lds<false>(ring_at + (buf * STAGE + t * 16 * CHUNK) * 2, src[t] + k);
     }
   };
-  floatx4 acc[NT];
+  floatx4 acc[NT], done[STRETCHES][NT];
 #pragma unroll
-  for (int t = 0; t < NT; ++t) acc[t] = floatx4{0.f, 0.f, 0.f, 0.f};
+  for (int t = 0; t < NT; ++t) {
+    acc[t] = floatx4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int i = 0; i < STRETCHES; ++i) done[i][t] = acc[t];
+  }
   const int at = r16 * CHUNK + (((wave * 4 + g) ^ r16) << 3);
 #pragma unroll
   for (int i = 0; i < NB - 1; ++i) ask(i, i);
-  int buf = 0;
+  int buf = 0, now = first / length, left = length;
   for (int c = 0; c < chunks; ++c) {
     nhv_wait_and_meet<(NB - 2) * LOADS>();                            // chunk c is there, chunk c - 1 has been read
     ask(buf == 0 ? NB - 1 : buf - 1, c + NB - 1);
-    const bf16_t* now = ring + buf * STAGE + at;
-    const bf16x8 b = *reinterpret_cast<const bf16x8*>(now + NT * 16 * CHUNK);
+    const bf16_t* from = ring + buf * STAGE + at;
+    const bf16x8 b = *reinterpret_cast<const bf16x8*>(from + NT * 16 * CHUNK);
 #pragma unroll
-    for (int t = 0; t < NT; ++t) acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b, *reinterpret_cast<const bf16x8*>(now + t * 16 * CHUNK), acc[t], 0, 0, 0);
+    for (int t = 0; t < NT; ++t) acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b, *reinterpret_cast<const bf16x8*>(from + t * 16 * CHUNK), acc[t], 0, 0, 0);
     buf = buf == NB - 1 ? 0 : buf + 1;
+    if (STRETCHES > 1 && --left == 0) {                               // (the same for the whole block)
+#pragma unroll
+      for (int i = 0; i < STRETCHES; ++i)
+        if (i == now) {
+#pragma unroll
+          for (int t = 0; t < NT; ++t) done[i][t] = acc[t];
+        }
+#pragma unroll
+      for (int t = 0; t < NT; ++t) acc[t] = floatx4{0.f, 0.f, 0.f, 0.f};
+      now = now == STRETCHES - 1 ? 0 : now + 1;
+      left = length;
+    }
+  }
+  if (stretches) {
+#pragma unroll
+    for (int t = 0; t < NT; ++t) {
+      acc[t] = done[0][t];
+#pragma unroll
+      for (int i = 1; i < STRETCHES; ++i) acc[t] += done[i][t];
+    }
   }
   nhv_wait_and_meet<0>();                                             // (the ring becomes room for the sums)
   float* part = reinterpret_cast<float*>(line_ring);                    // [tile][wave][256]

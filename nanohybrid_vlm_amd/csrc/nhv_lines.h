@@ -31,6 +31,8 @@ __device__ __forceinline__ void nhv_wait_and_meet() {
 // 37.8 with it; 6,144 of 4,096 at 1 to 16 rows 12.3 to 15.7 us, by where x happens to lie, and 11.7 to 12.6.
 // (Rows of other lengths lie apart already, and the turning costs what it changes in what the caches hold: gated 9,728 of 2,560 at 1
 // row 21.8 us without, 22.5 with it.)
+// The order of an output's sum then hangs on the block that makes it: equal rows of w give results that differ by rounding. Logits,
+// between which a choice is made, are summed so that they do not (gemm_fewrows_bf16.hip).
 __device__ __forceinline__ int nhv_first_chunk(int block, int chunks, int K) {
   if (K % 2048) return 0;
   return (block / 8 + block % 8 * chunks / 8) % chunks;              // (blocks go to the 8 XCDs in turn)

@@ -1396,6 +1396,20 @@ def test_parts_of_a_product_through_the_norm_and_the_rotation(ops, splits):
             assert all(torch.equal(a, c) for a, c in zip(*results)), D
 
 
+@pytest.mark.parametrize("N,K", [(5000, 2048), (9000, 4096), (4112, 6144), (4100, 2304), (700, 1024), (2600, 2560)])
+def test_equal_rows_of_a_head_give_equal_logits(ops, N, K):
+    """Whichever block makes them: between equal rows the first is chosen, not one that rounding favours. In float32 from bfloat16, few
+    rows, against float64 (float sums of K products of size K^-1/2)."""
+    w = rnd(N, K, dtype=torch.bfloat16, seed=131, scale=K ** -0.5)
+    equal = sorted({3, 16, 40, N // 3, N // 2, N - 17, N - 1})
+    w[equal] = w[3].clone()
+    for M in (1, 5, 8, 12, 16):
+        x = rnd(M, K, dtype=torch.bfloat16, seed=132 + M)
+        y = ops.linear(x, w, out_dtype=torch.float32)
+        assert torch.equal(y[:, equal], y[:, [3]].expand(M, len(equal)))
+        torch.testing.assert_close(y.double(), x.double() @ w.double().T, rtol=1e-4, atol=2e-4)
+
+
 def _random_product_sizes(seed, count, max_rows):
     import random
     rnd_ = random.Random(seed)
