@@ -1076,9 +1076,16 @@ __global__ __launch_bounds__(512) void gemm_fewrows_lines_kernel(const bf16_t* _
 // of 1,024 columns (4.2, 4.9 at 1 row) or a gated 3,072 of 1,024 (5.5, 5.7); with fewer than 4,096 outputs a tile of 16 leaves units idle,
 // which the smaller tiles above do not, until there are so many rows that these are slower: 2,560 of 9,728 14.6, 15.1 at 1 row,
 // 15.5, 15.7 at 4, 18.8, 15.8 at 8; 2,048 of 6,144 9.9, 11.1 at 8 and 14.3, 11.5 at 12; 2,048 of 2,048 never.
-static bool lines_plan(bool glu, int M, int N, int K) {
+// ``even``: the tiles above would take the product, which give every unit the same rows of w (no residual, whose squares go out by tiles of
+// 16, and no bands). They stay the faster ones where the blocks of 32 outputs are a round and a bit (time by lines over theirs, K = 2,048
+// to 12,288, at 1 to 8 rows: 8,448 outputs 1.07 to 1.18, 9,216 1.07 to 1.17, 10,240 1.00 to 1.11 and at K = 2,048 0.95, 11,264 0.96 to 1.07, 12,288 0.88 to
+// 1.04; 16 rows: K = 3,072 1.05 to 1.15, from 4,096 on 0.62 to 0.88), and with rows 16 KB apart on some of the units (K = 8,192: 4,224
+// to 6,144 outputs 1.06 to 1.22 at 1 to 4 rows, 0.81 to 0.99 at 8; 7,168 outputs 0.80 to 0.87), as long as all of x fits beside w.
+static bool lines_plan(bool glu, bool even, int M, int N, int K) {
   if (K % 256 != 0 || K < 2048) return false;
   if (glu) return N >= 4096;
+  if (even && N > 8192 && N <= (K > 2048 ? 11264 : 9216) && (long long)M * K <= 57344) return false;
+  if (even && N > 4096 && N < 7168 && K % 8192 == 0 && (long long)M * K <= 32768) return false;
   return N >= 4096 || (N >= 2560 && M >= 8) || (N >= 2048 && K >= 4096 && M >= 12);
 }
 
@@ -1276,7 +1283,7 @@ int nhv_gemm_fewrows_launch(bool glu, const void* x, const void* w, const void* 
     if (glu || fused || f.band_rows % 16 != 0) return nhv_fail("few-rows gemm: bands of %d rows (multiples of 16, no gate, no fusion)", f.band_rows);
     // (8,224 outputs of 2,048 columns at 16 rows in five bands, in a trace: 14.9 us by the kernel that takes x
     // from memory, 11.9 by lines)
-    if (f.band_rows % 32 == 0 && lines_plan(false, M, N, K))
+    if (f.band_rows % 32 == 0 && lines_plan(false, false, M, N, K))
       return out_dtype == NHV_BF16 ? launch_lines<false, bf16_t>(s, x, w, bias, y, M, N, K, f) : launch_lines<false, float>(s, x, w, bias, y, M, N, K, f);
     const Plan p = plan(false, M, N, K);
     if (f.band_rows % 32 == 0 && p.nt == 2) launch<2, 8, 2, false>(s, x, w, bias, y, M, N, K, out_dtype, false, f);
@@ -1284,7 +1291,7 @@ int nhv_gemm_fewrows_launch(bool glu, const void* x, const void* w, const void* 
     return 0;
   }
   if (fused && out_dtype != NHV_BF16) return nhv_fail("few-rows gemm: a product that takes over its neighbours' work gives bfloat16");
-  if (lines_plan(glu, M, N, K) && !(glu && out_dtype != NHV_BF16)) {
+  if (lines_plan(glu, f.residual == nullptr, M, N, K) && !(glu && out_dtype != NHV_BF16)) {
     if (glu) return launch_lines<true, bf16_t>(s, x, w, bias, y, M, N, K, f);
     return out_dtype == NHV_BF16 ? launch_lines<false, bf16_t>(s, x, w, bias, y, M, N, K, f) : launch_lines<false, float>(s, x, w, bias, y, M, N, K, f);
   }

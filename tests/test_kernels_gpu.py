@@ -237,6 +237,8 @@ def test_few_rows_linear_bfloat16_in_all_its_variants(ops, M, N, K):
     # chunks of whole lines: one tile a block and two, ends inside a tile, as few chunks as the ring has places and fewer, the
     # fewest outputs at every bound of rows
     (1, 4096, 2048), (3, 4100, 2816), (16, 6148, 3072), (5, 8196, 2048), (8, 2560, 2304), (12, 2048, 4352), (16, 16388, 2304),
+    # a round of blocks and a bit: by lines with a residual only, and where x is too large or K small; K of 8,192
+    (8, 8448, 2304), (16, 9220, 3072), (16, 11264, 4096), (2, 10000, 2048), (4, 5120, 8192), (5, 4100, 8192),
 ])
 def test_tiles_of_few_rows_products(ops, M, N, K):
     """Plain, activated, gated, with rows that lack their scales and added to a residual (bounds: float32 sums of K products of
