@@ -385,37 +385,72 @@ static void launch_tiles(const float* x, const float* w, const float* bias, floa
     hipLaunchKernelGGL((gemm_float32_tiles_kernel<RT, CT, GATED, false>), grid, block, 0, s, x, w, bias, y, M, N, K, m_tiles, n_tiles, gate);
 }
 
+// Every tile's time in units of what a compute unit needs for 16 rows of an operand, from the times of all tiles at 1 to 1,500
+// rows of the 0.6B and 1.7B shapes' products. Tiles of 8 waves: rounds of 256 blocks times 16-row operands; the tiles through
+// LDS: a floor (one block's chain of pieces) and what a block a compute unit adds. E.g. 17 x 6144 . 1024: 32 x 32 10.1 us,
+// 16 x 32 14.0, 16 x 16 13.9 (float matrix instructions 12.6); 130 x 2048 . 2048: 48 x 32 22.1 us, 32 x 32 33.3 (33.2); 517 x
+// 1024 . 3072: 32 x 32 through LDS 58.9, 48 x 32 60.0, 64 x 64 66.6 (71); 517 x 4096 . 1024: 64 x 64 45, 32 x 32 through LDS 56
+// (57). Up to 16 rows LDS has nothing to share and is left out (6 x 151,936 . 1024: 116 us with 16 x 32, 135 through LDS; 137).
+// 32 x 16, whose second 16 rows are few different ones at 17 rows and 16 at 32: 17 x 4096 . 4096 24.2 us, 16 x 32 27.4 (24.3); 32 rows 29.2 and 28.1.
+struct Choice {
+  int tile;
+  double cost;
+};
+static Choice plain_tile(long long M, long long N) {
+  auto blocks = [&](long long m, long long n) { return ((M + m - 1) / m) * ((N + n - 1) / n); };
+  auto rounds = [&](int rt, int ct) { return (double)((blocks(16 * rt, 16 * ct) + 255) / 256 * (rt + ct)); };
+  const double none = 1e300;
+  const double cost[7] = {rounds(1, 1), rounds(1, 2), M > 16 ? rounds(2, 2) : none, M > 32 ? rounds(3, 2) : none,
+                          M > 16 ? fmax(9.0, 1.5 + 2.9 / 256 * blocks(32, 32)) : none,
+                          M > 16 ? fmax(11.5, 4.5 + 7.7 / 256 * blocks(64, 64)) : none,
+                          M > 16 && M <= 32 ? rounds(2, 1) / 3 * (2.05 + 0.035 * M) : none};
+  Choice best = {0, cost[0]};
+  for (int i = 1; i < 7; ++i)
+    if (cost[i] < best.cost) best = {i, cost[i]};
+  return best;
+}
+// a gate of two products: a column counting for two rows of w; through LDS only tiles with a pair a wave
+static Choice gated_tile(long long M, long long N) {
+  auto blocks = [&](long long m, long long n) { return ((M + m - 1) / m) * ((N + n - 1) / n); };
+  auto rounds = [&](int rt) { return (double)((blocks(16 * rt, 16) + 255) / 256 * (rt + 2)); };
+  const double none = 1e300;
+  const double cost[5] = {rounds(1), M > 16 ? rounds(2) : none, M > 32 ? rounds(3) : none,
+                          M > 16 ? fmax(9.5, 3.0 + 4.9 / 256 * blocks(32, 32)) : none,
+                          M > 16 ? fmax(11.5, 4.5 + 7.7 / 256 * blocks(64, 32)) : none};
+  Choice best = {0, cost[0]};
+  for (int i = 1; i < 5; ++i)
+    if (cost[i] < best.cost) best = {i, cost[i]};
+  return best;
+}
+
 extern "C" int nhv_gemm_float32(const void* x, const void* w, const void* bias, void* y, int M, int N, int K, void* stream) {
   NHV_REQUIRE(M > 0 && N > 0 && K > 0, "gemm: bad sizes M=%d N=%d K=%d", M, N, K);
   NHV_REQUIRE(K < (1 << 30) && (((long long)M + 15) / 16) * (((long long)N + 15) / 16) < (1ll << 30), "gemm: too many rows (%d) for %d columns", M, N);
   hipStream_t s = (hipStream_t)stream;
   const float *xf = (const float*)x, *wf = (const float*)w, *bf = (const float*)bias;
   float* yf = (float*)y;
-  // Every tile's time in units of what a compute unit needs for 16 rows of an operand, from the times of all tiles at 1 to 1,500
-  // rows of the 0.6B and 1.7B shapes' products. Tiles of 8 waves: rounds of 256 blocks times 16-row operands; the tiles through
-  // LDS: a floor (one block's chain of pieces) and what a block a compute unit adds. E.g. 17 x 6144 . 1024: 32 x 32 10.1 us,
-  // 16 x 32 14.0, 16 x 16 13.9 (float matrix instructions 12.6); 130 x 2048 . 2048: 48 x 32 22.1 us, 32 x 32 33.3 (33.2); 517 x
-  // 1024 . 3072: 32 x 32 through LDS 58.9, 48 x 32 60.0, 64 x 64 66.6 (71); 517 x 4096 . 1024: 64 x 64 45, 32 x 32 through LDS 56
-  // (57). Up to 16 rows LDS has nothing to share and is left out (6 x 151,936 . 1024: 116 us with 16 x 32, 135 through LDS; 137).
-  auto blocks = [&](long long m, long long n) { return ((M + m - 1) / m) * ((N + n - 1) / n); };
-  auto rounds = [&](int rt, int ct) { return (double)((blocks(16 * rt, 16 * ct) + 255) / 256 * (rt + ct)); };
-  const double none = 1e300;
-  const double cost[6] = {rounds(1, 1), rounds(1, 2), M > 16 ? rounds(2, 2) : none, M > 32 ? rounds(3, 2) : none,
-                          M > 16 ? fmax(9.0, 1.5 + 2.9 / 256 * blocks(32, 32)) : none,
-                          M > 16 ? fmax(11.5, 4.5 + 7.7 / 256 * blocks(64, 64)) : none};
-  int best = 0;
-  for (int i = 1; i < 6; ++i)
-    if (cost[i] < cost[best]) best = i;
-  switch (best) {
+  switch (plain_tile(M, N).tile) {
     case 0: launch<1, 1, 2, false>(xf, wf, bf, yf, M, N, K, {}, s); break;
     case 1: launch<1, 2, 1, false>(xf, wf, bf, yf, M, N, K, {}, s); break;
     case 2: launch<2, 2, 1, false>(xf, wf, bf, yf, M, N, K, {}, s); break;
     case 3: launch<3, 2, 1, false>(xf, wf, bf, yf, M, N, K, {}, s); break;
     case 4: launch_tiles<1, 1, false>(xf, wf, bf, yf, M, N, K, {}, s); break;
-    default: launch_tiles<2, 2, false>(xf, wf, bf, yf, M, N, K, {}, s);
+    case 5: launch_tiles<2, 2, false>(xf, wf, bf, yf, M, N, K, {}, s); break;
+    default: launch<2, 1, 2, false>(xf, wf, bf, yf, M, N, K, {}, s);
   }
   NHV_LAUNCH_CHECK("gemm_float32");
   return 0;
+}
+
+// Whether the gate is best made in the product's kernel (1), or of the packed product's rows by a kernel of its own (0). A block takes both
+// rows of w of an output, so a gated product of few outputs has half the packed one's blocks and as many more units idle: us at 1 and
+// 17 rows, here and packed (before this kernel was there): 512 of 8,192 columns 38.1, 47.3 and 25.8, 35.8 (25.4, 35.5); 1,024 of 3,072 18.6,
+// 21.8 and 15.0, 19.0 (14.2, 18.5); 2,048 of 6,144 32.8, 38.6 and 25.4, 40.8 (24.9, 36.7); 2,560 of 9,728 48.2, 62.8 and 50.8, 64.6 (59.1, 80.5);
+// 3,072 of 1,024 10.8, 13.4 and 12.5, 15.1 (13.0, 16.4). A unit of the costs above takes 5.6 us a 3,072 columns, five times that where rows come
+// entry by entry (1,000 of 1,001 at 1 row 20.8 and 13.4), the gate's kernel 2 and more (in a recorded step 4).
+extern "C" int nhv_gemm_float32_gated_pays(const void* x, const void* w, int M, int N, int K) {
+  const bool wide = K % 4 == 0 && (uintptr_t)x % 16 == 0 && (uintptr_t)w % 16 == 0;
+  return (gated_tile(M, N).cost - plain_tile(M, 2ll * N).cost) * (wide ? 5.6 : 28.0) * K / 3072 <= 2.0;
 }
 
 extern "C" int nhv_gemm_float32_gated(const void* x, const void* w, const void* bias, void* y, int M, int N, int K, int act, float limit,
@@ -428,17 +463,7 @@ extern "C" int nhv_gemm_float32_gated(const void* x, const void* w, const void* 
   const NhvGate gate = {act, limit, alpha, offset};
   const float *xf = (const float*)x, *wf = (const float*)w, *bf = (const float*)bias;
   float* yf = (float*)y;
-  // as above, a column counting for two rows of w; through LDS only tiles with a pair a wave
-  auto blocks = [&](long long m, long long n) { return ((M + m - 1) / m) * ((N + n - 1) / n); };
-  auto rounds = [&](int rt) { return (double)((blocks(16 * rt, 16) + 255) / 256 * (rt + 2)); };
-  const double none = 1e300;
-  const double cost[5] = {rounds(1), M > 16 ? rounds(2) : none, M > 32 ? rounds(3) : none,
-                          M > 16 ? fmax(9.5, 3.0 + 4.9 / 256 * blocks(32, 32)) : none,
-                          M > 16 ? fmax(11.5, 4.5 + 7.7 / 256 * blocks(64, 32)) : none};
-  int best = 0;
-  for (int i = 1; i < 5; ++i)
-    if (cost[i] < cost[best]) best = i;
-  switch (best) {
+  switch (gated_tile(M, N).tile) {
     case 0: launch<1, 2, 1, true>(xf, wf, bf, yf, M, N, K, gate, s); break;
     case 1: launch<2, 2, 1, true>(xf, wf, bf, yf, M, N, K, gate, s); break;
     case 2: launch<3, 2, 1, true>(xf, wf, bf, yf, M, N, K, gate, s); break;

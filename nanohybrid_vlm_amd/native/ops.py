@@ -927,9 +927,12 @@ class NativeBackend:
 
     def gated_linear(self, x, w, out, gate=None, bias=None) -> bool:
         """A gate (a ``Gate``; None: SiLU) of x Wg^T and x Wu^T (+ bias) in one kernel, if this batch is one for the
-        few-rows kernel or the one for up to 96 rows; else False. (SiLU without bias may also be one for the kernel of up to 64 rows; in float32 every batch is.)"""
+        few-rows kernel or the one for up to 96 rows; else False. (SiLU without bias may also be one for the kernel of up to 64 rows; in
+        float32 most batches are.)"""
         M, K = x.shape
         if x.dtype == torch.float32:
+            if not self.lib.nhv_gemm_float32_gated_pays(_ptr(x), _ptr(w), M, out.shape[1], K):
+                return False
             self._call("nhv_gemm_float32_gated", _ptr(x), _ptr(w), _ptr(bias), _ptr(out), M, out.shape[1], K, *(gate or Gate()).args(), _stream())
             return True
         if self._by_lines(x, w, out.shape[1], True):

@@ -294,7 +294,7 @@ def test_gated_linear(ops, M, I, K):
             backend.own_kernels_only = False
 
 
-@pytest.mark.parametrize("N,K", [(1, 1), (17, 130), (48, 16), (130, 20), (65, 516), (300, 2064), (16400, 36), (24000, 7)])
+@pytest.mark.parametrize("N,K", [(1, 1), (17, 130), (48, 16), (130, 20), (65, 516), (300, 2064), (16400, 36), (24000, 7), (2500, 68), (2100, 331)])
 def test_float32_linear_in_all_its_tiles(ops, N, K):
     """Every tile that the number of rows and columns can choose, K below and beyond eight blocks of 16, ends inside a block of
     16, rows off 16-byte boundaries: against float64 (a sum of K products of size 1 is off by K^(1/2) roundings of its own size,
@@ -422,6 +422,22 @@ def test_float32_gated_linear_in_all_its_tiles(ops, N, K):
             packed = ops.linear(rows, w)
             got, want = ops.gated_linear(rows, w, gate, bias), ops.act_mul(packed, gate, bias)
             assert torch.equal(got.isnan(), want.isnan()) and torch.equal(got.nan_to_num(1.5, 2.5, 3.5), want.nan_to_num(1.5, 2.5, 3.5)), (M, gate)
+
+
+@pytest.mark.parametrize("M,N,K,fused", [
+    (1, 3072, 1024, True), (6, 2560, 2560, True), (300, 512, 4096, True), (16, 512, 512, True), (70, 1000, 1001, True),
+    (1, 512, 8192, False), (17, 1024, 3072, False), (16, 2048, 2048, False), (1, 1000, 1001, False),
+])
+def test_which_float32_gates_are_made_in_the_products_kernel(ops, M, N, K, fused):
+    """Not where the packed product's blocks are twice as many and the chip is not full: the same bits either way."""
+    x, w = rnd(M, K, seed=67), rnd(2 * N, K, seed=68)
+    out = torch.full((M, N), float("nan"), device="cuda")
+    assert ops.backend().gated_linear(x, w, out) == fused
+    want = ops.act_mul(ops.linear(x, w), "silu")
+    assert torch.equal(ops.gated_linear(x, w), want)
+    by_product = ops.backend().lib.nhv_gemm_float32_gated
+    assert by_product(ops._ptr(x), ops._ptr(w), ops._ptr(None), ops._ptr(out), M, N, K, *ops.Gate().args(), ops._stream()) == 0
+    assert torch.equal(out, want)
 
 
 def test_linear_rows_do_not_depend_on_the_batch_in_float32(ops):
