@@ -209,10 +209,12 @@ def test_skinny_linear_bfloat16(ops, M, N, K):
     # every way the kernel for up to 16 rows cuts the work: one or two tiles of 16 outputs per block, 4 or 8 waves
     (1, 6144, 264), (2, 5000, 4096), (5, 7168, 72), (8, 6100, 1032), (12, 5120, 520), (16, 151936, 64), (9, 10240, 40),
     (16, 16, 8), (3, 17, 25608),
-    # x too large for LDS at once, up to 256 tiles: it comes in pieces
-    (16, 4000, 12296), (7, 272, 12288), (11, 4096, 25600),
+    # x too large for LDS at once, up to 256 tiles: it comes in pieces (K off 256: the others go by lines)
+    (16, 4000, 12296), (7, 272, 12288), (11, 4096, 25608),
     # x too large for LDS at once and more than 256 tiles: two pieces, every tile walked over twice
-    (16, 7168, 5120), (10, 5136, 8200), (5, 4112, 17408),
+    (16, 7168, 5128), (10, 5136, 8200), (5, 4112, 17416),
+    # K a multiple of 256: by lines
+    (11, 4096, 25600), (16, 7168, 5120), (5, 4112, 17408),
 ])
 def test_few_rows_linear_bfloat16_in_all_its_variants(ops, M, N, K):
     x = rnd(M, K, dtype=torch.bfloat16, seed=34)
@@ -1298,6 +1300,8 @@ def test_library_products_refuse_what_they_cannot_do(ops):
     # chunk and two chunks of columns, chunks that do not divide by the parts
     (17, 64, 256), (32, 1000, 384), (33, 4096, 4096), (49, 6144, 2560), (64, 4096, 12288), (79, 2560, 1152), (80, 1033, 3072), (96, 333, 9728),
     (97, 512, 512), (112, 2048, 6144), (128, 1024, 3072),
+    # wider than the 8B shape
+    (31, 5120, 17408), (64, 10240, 5120),
 ])
 def test_products_by_lines(ops, M, N, K):
     """As float parts and as a gate of two products, with biases and without (float sums of K products of size K^-1/2)."""
@@ -1373,6 +1377,32 @@ def test_what_goes_by_lines_hangs_on_the_shape_and_on_a_table_that_is_read(ops):
         backend.chosen, backend.measuring_allowed = chosen, allowed
 
 
+@pytest.mark.parametrize("M,N,K", [(3, 4096, 2048), (16, 4100, 2304), (17, 2048, 1024), (40, 3000, 1280), (90, 4096, 2048)])
+def test_products_by_lines_keep_rows_and_columns_apart(ops, M, N, K):
+    """Rows of x and of w that are infinite or no numbers: their own rows and columns are what float64 says of them, all others the same bits as
+    without them, as rows, parts and a gate."""
+    x, w = rnd(M, K, dtype=torch.bfloat16, seed=141), rnd(2 * N, K, dtype=torch.bfloat16, seed=142, scale=K ** -0.5)
+
+    def results():
+        made = [ops.linear(x, w[:N]), ops.gated_linear(x, w)]
+        if M <= 16:
+            return made + [ops.linear(x, w[:N], out_dtype=torch.float32)]
+        return made + list(ops.linear(x, w[:N], parts=True).parts)
+
+    clean = [r.clone() for r in results()]
+    x[0, K // 2], x[M - 1, 7] = float("nan"), float("inf")
+    w[5, K - 1], w[N - 1, 0], w[N + 9, 3] = float("-inf"), float("nan"), float("inf")
+    rows = [i for i in range(M) if i not in (0, M - 1)]
+    columns = [j for j in range(N) if j not in (5, N - 1, 9)]
+    want = x.double() @ w[:N].double().T
+    got = results()
+    for before, now in zip(clean, got):
+        assert torch.equal(now[rows][:, columns], before[rows][:, columns])
+    for odd in [got[0]] + ([got[2]] if M <= 16 else [sum(got[2:])]):
+        odd = odd.double()
+        assert torch.equal(odd.isnan(), want.isnan()) and torch.equal(odd.isposinf(), want.isposinf()) and torch.equal(odd.isneginf(), want.isneginf())
+
+
 @pytest.mark.parametrize("M,band,last,K", [(1, 1024, 32, 2048), (16, 2048, 5, 2304), (7, 1056, 1100, 2048)])
 def test_products_in_bands_by_lines(ops, M, band, last, K):
     """Five sets of rows against a matrix's bands, where the kernel by lines takes them (float sums of K products of size K^-1/2)."""
@@ -1398,6 +1428,13 @@ def test_parts_of_a_product_through_the_norm_and_the_rotation(ops, splits):
                 r2 = r.clone()
                 want = ops.rmsnorm(x, w, 1e-6, residual=r)
                 assert torch.equal(ops.rmsnorm(parts_of(x), w, 1e-6, residual=r2), want) and torch.equal(r, r2)
+    # a width that is no multiple of 8, a residual and a weight off 16 bytes: the parts are summed first
+    for width, off, w_off in ((20, 0, 0), (520, 1, 0), (520, 0, 1)):
+        x, space, w_space = rnd(5, width, dtype=torch.bfloat16, seed=84), rnd(5 * width + 1, seed=86), rnd(width + 1, seed=85)
+        w, r = w_space[w_off:w_off + width], space[off:off + 5 * width].view(5, width)
+        r2 = space.clone()[off:off + 5 * width].view(5, width)
+        want = ops.rmsnorm(x, w, 1e-6, residual=r)
+        assert torch.equal(ops.rmsnorm(parts_of(x), w, 1e-6, residual=r2), want) and torch.equal(r, r2)
     T, Hq, Hkv = 7, 6, 2
     for D in (16, 64, 128, 512, 48):                         # (48: no power of two, the parts are summed first)
         qkv, bias = rnd(T, (Hq + 2 * Hkv) * D, dtype=torch.bfloat16, seed=87), rnd((Hq + 2 * Hkv) * D, dtype=torch.bfloat16, seed=88)
