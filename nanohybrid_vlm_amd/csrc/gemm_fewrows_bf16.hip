@@ -8,16 +8,18 @@
 // The waves' sums meet in LDS and are added in the order of the waves, so the result does not depend
 // on timing. Rows of x beyond M and columns beyond K read as zero.
 //
-// Most products take one of two kernels in whose tiles nothing waits (tiles_plan() below). For the others: where all rows of
-// x fit into LDS beside the sums (M (K + 8) 2 bytes of the 160 KB) a second kernel is used
-// instead: a block copies x into LDS once (straight from memory, global_load_lds) and then walks over
-// tiles of w, tile after tile, one or two blocks per compute unit for the whole matrix. The rows of x
-// then cross from L2 to a compute unit once per call instead of once per tile: 5 to 25 % less time at
-// every size measured, most where N is large (the head: 266 to 221 us at 8 rows). Where x does not
-// fit at once and w has at most 256 tiles, a third kernel gives every block one tile and takes x through
-// LDS in pieces (the 8B down projection from 7 rows on: 2 to 6 % less time, 12 % with 2,048 outputs). With more
-// tiles than that, and x fitting in two pieces, a fourth kernel walks over all of a block's tiles once for each
-// piece and keeps the tiles' sums in LDS between the two (16 rows of 5,120 columns: 13 % less time for gate_up).
+// Rows of a multiple of 256 columns and 2,048 and more, with outputs enough to fill the chip in tiles of 16, take a kernel that brings w and
+// x through LDS by lines of 512 bytes (gemm_fewrows_lines_kernel, lines_plan() below): nearly all layer shapes and heads from the
+// 1.7B widths on. Most of the others take one of two kernels in whose tiles nothing waits (tiles_plan() below). What neither takes:
+// where all rows of x fit into LDS beside the sums (M (K + 8) 2 bytes of the 160 KB) a block copies x into LDS once (straight from
+// memory, global_load_lds) and then walks over tiles of w, tile after tile, one or two blocks per compute unit for the whole matrix.
+// The rows of x then cross from L2 to a compute unit once per call instead of once per tile: 5 to 25 % less time than by the kernel
+// described above at every size measured, most where N is large. Where x does not fit at once and w has at most 256 tiles, a further
+// kernel gives every block one tile and takes x through LDS in pieces (4,096 outputs of 12,288 columns from 7 rows on: 2 to 6 % less time,
+// 12 % with 2,048 outputs). With more tiles than that, and x fitting in two pieces, another one walks over all of a block's tiles once for
+// each piece and keeps the tiles' sums in LDS between the two (16 rows of 5,120 columns: 13 % less time for gate_up). (Sizes that are quoted
+// here and at those kernels were measured before the kernel by lines was there, which takes those of 256 columns' multiples now; the
+// rules hold for the others.)
 //
 // How many tiles a block takes, how many waves share K and how many loads a wave keeps in flight is
 // chosen per call from M, N and K (plan() below): blocks that spread evenly over the compute units
@@ -891,6 +893,7 @@ static TilesPlan tiles_plan(bool glu, bool squares, bool biased, int M, int N, i
   const size_t sums = (size_t)(tiles > 1 ? 2 : 1) * TW * (glu ? 2 : 1) * 64 * sizeof(floatx4), x_bytes = (size_t)M * (K + 8) * 2;
   const size_t biases = tiles > 1 && biased ? ((glu ? 2 : 1) * p.rows + 16) * sizeof(float) : 0;
   p.x_in_lds = sums + x_bytes + biases <= LDS_BYTES;
+  // (Of the sizes quoted here, those of a multiple of 256 columns go by lines now, but for what lines_plan() leaves.)
   // The kernels below it is where a product of several tiles a block has more biases than threads, and where x does not fit into LDS,
   // but for up to 8 rows on the whole chip (4,096 outputs of 12,288 columns at 8 rows 25.2 against 26.8 us; 3,584 of 18,944 on
   // 224 units, where x beside w is too much for a unit, 36.4 against 33.9; 4,096 of 12,288 at 16 rows 31.4 against 30.7).

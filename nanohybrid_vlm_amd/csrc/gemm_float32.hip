@@ -1,4 +1,5 @@
-// y[M, N] = x[M, K] . w[N, K]^T (+ bias[N]) in float, or a gate of two such products (w[2 N, K]: N gate rows, then N up rows), on the bfloat16 matrix cores without losing any of the 32 bits.
+// y[M, N] = x[M, K] . w[N, K]^T (+ bias[N]) in float, or a gate of two such products (w[2 N, K]: N gate rows, then N up rows), on the
+// bfloat16 matrix cores, to float's precision.
 //
 // A float (times 2^16) is the sum of three bfloat16 numbers, exactly: what rounding to 8 bits gives, what that leaves rounded to
 // 8 bits, and the rest (nhv_split_float.h). A product of two floats is then nine products of 8 bits by 8, each exact in float; six
@@ -241,10 +242,10 @@ static void launch(const float* x, const float* w, const float* bias, float* y, 
 // ---------------------------------------------------------------- many rows
 // 4 waves, 2 x 2, a wave RT x CT tiles of 16 x 16; the parts of both operands through LDS in pieces of 32 k, two buffers, two
 // pieces under way in registers: an entry is taken apart once a block. A wave takes every segment in turn and adds it to the
-// total: the same sums in the same order as above. What bounds it: matrix and vector instructions (24 and 56 of them a piece
+// total: the same sums in the same order as above. What bounds it: matrix and vector instructions (24 and 72 of them a piece
 // and wave of the large tile) add up more than they overlap, within a wave and between two of a SIMD; so three blocks a
 // compute unit, which is why LDS rows have no padding and only two pieces are under way (two blocks, with 80-byte rows and
-// four pieces: 517 x 4096 . 1024 in 58 us in place of 45). 2 x 2 tiles a wave: 1,500 x 12,288 . 2048 in 538 us (140 TFLOP/s;
+// four pieces: 517 x 4096 . 1024 in 58 us in place of 45, before the factors 2^16). 2 x 2 tiles a wave: 1,500 x 12,288 . 2048 in 564 us (134 TFLOP/s;
 // float matrix instructions 672).
 #define PIECE 32
 #define AHEAD 2
