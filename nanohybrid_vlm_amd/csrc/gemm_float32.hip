@@ -21,11 +21,12 @@
 // infinite (sums beyond 2^96 do) or as no number is summed once more by plain float multiply-adds: that is what it is then.
 // (Such inputs make every output of their row or column such a one.)
 //
-// Two kernels. Few rows, or few columns: a block is 8 waves and owns 16 RT rows by 16 CT columns, wave s sums segment s, and
+// Three kernels. Few rows, or few columns: a block is 8 waves and owns 16 RT rows by 16 CT columns, wave s sums segment s, and
 // LDS adds the segments up. Both operands come straight from memory (a lane: 16 bytes of each half of a row's 128); all loads
 // of a stage of U blocks of 32 k are asked for one stage ahead. What bounds it is what a compute unit takes in: a tile's time
 // grows by 5.6 us a 3,072 k with every 16 rows of x or w that it reads (35 GB/s), whatever their product. Many rows: a block is
-// 4 waves that share their operands' parts through LDS, see below.
+// 4 waves that share their operands' parts through LDS, 32 or 64 rows of x a block, see below. And where a product has few outputs and its
+// reader adds parts up (a norm does), the segments go to blocks of their own and the sums over segments are left to that reader.
 // The blocks of one column tile follow each other on one XCD, whose L2 then reads those rows of w once.
 // A gated product takes tiles of gate rows and of their up rows in turn (two a wave), and a lane that has finished both writes
 // the gate of them: what a kernel of its own made of the packed rows before (6 rows of 3,072: 4.1 us, 517: 5.5).
@@ -36,6 +37,7 @@
 #define SEGMENTS 8
 
 __host__ __device__ static inline int segment_length(int K) { return ((K + SEGMENTS - 1) / SEGMENTS + 31) & ~31; }
+__host__ __device__ static inline int segments(int K) { return (K + segment_length(K) - 1) / segment_length(K); }
 
 // four entries of a row from column k on. WIDE: rows of a multiple of four entries on 16-byte boundaries; beyond K the row's
 // last four (the caller puts zeros in their place), so that no load hangs on a condition: with conditions the compiler
@@ -90,21 +92,22 @@ __device__ __attribute__((noinline)) float plain_products(const float* __restric
   return v;
 }
 
-template <int RT, int CT, int U, bool GATED, bool WIDE>
-__global__ __launch_bounds__(64 * SEGMENTS) void gemm_float32_kernel(const float* __restrict__ x, const float* __restrict__ w,
+// PARTS: two waves a block, each with a segment of its own, whose sums are the result (times 2^32, [segment][M][N]).
+template <int RT, int CT, int U, bool GATED, bool PARTS, bool WIDE>
+__global__ __launch_bounds__(PARTS ? 128 : 64 * SEGMENTS) void gemm_float32_kernel(const float* __restrict__ x, const float* __restrict__ w,
                                                                      const float* __restrict__ bias, float* __restrict__ y,
                                                                      int M, int N, int K, int m_tiles, int n_tiles, NhvGate gate) {
   static_assert(!GATED || CT == 2, "a gate tile and its up tile");
   constexpr int COLS = GATED ? 16 : 16 * CT;             // outputs of a row
-  __shared__ __attribute__((aligned(16))) float part[SEGMENTS][CT * 256];
+  __shared__ __attribute__((aligned(16))) float part[PARTS ? 1 : SEGMENTS][PARTS ? 1 : CT * 256];
   const int total = m_tiles * n_tiles, share = (total + 7) >> 3;
   const int tile = (blockIdx.x & 7) * share + (blockIdx.x >> 3);        // (consecutive blocks go round the 8 XCDs)
   if (tile >= total) return;
   const int m0 = (tile % m_tiles) * 16 * RT, n0 = (tile / m_tiles) * COLS;
-  const int s = threadIdx.x >> 6, lane = threadIdx.x & 63, r16 = lane & 15, g = lane >> 4;
+  const int s = (threadIdx.x >> 6) + (PARTS ? 2 * blockIdx.y : 0), lane = threadIdx.x & 63, r16 = lane & 15, g = lane >> 4;
   const int length = segment_length(K);
   const int begin = s * length, end = min(K, begin + length);
-  const int active = (K + length - 1) / length;
+  const int active = segments(K);
 
   f32x4 acc[RT][CT];
 #pragma unroll
@@ -193,6 +196,19 @@ __global__ __launch_bounds__(64 * SEGMENTS) void gemm_float32_kernel(const float
 #pragma unroll
       for (int c = 0; c < CT; ++c) acc[r][c] += low[r][c];
   }
+  if (PARTS) {
+    if (begin < end)
+#pragma unroll
+      for (int r = 0; r < RT; ++r)
+#pragma unroll
+        for (int c = 0; c < CT; ++c)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            const int m = m0 + 16 * r + 4 * g + i, n = n0 + 16 * c + r16;
+            if (m < M && n < N) y[((size_t)s * M + m) * N + n] = acc[r][c][i];
+          }
+    return;
+  }
 #pragma unroll
   for (int r = 0; r < RT; ++r) {
     if (m0 + 16 * r >= M) break;                         // (the same for the whole block)
@@ -228,29 +244,26 @@ __global__ __launch_bounds__(64 * SEGMENTS) void gemm_float32_kernel(const float
   }
 }
 
-template <int RT, int CT, int U, bool GATED>
+template <int RT, int CT, int U, bool GATED, bool PARTS = false>
 static void launch(const float* x, const float* w, const float* bias, float* y, int M, int N, int K, const NhvGate& gate, hipStream_t s) {
   constexpr int COLS = GATED ? 16 : 16 * CT;
   const int m_tiles = (M + 16 * RT - 1) / (16 * RT), n_tiles = (N + COLS - 1) / COLS;
-  const dim3 grid(8u * (unsigned)(((long long)m_tiles * n_tiles + 7) / 8)), block(64 * SEGMENTS);
-  if (K % 4 == 0 && (uintptr_t)x % 16 == 0 && (uintptr_t)w % 16 == 0)
-    hipLaunchKernelGGL((gemm_float32_kernel<RT, CT, U, GATED, true>), grid, block, 0, s, x, w, bias, y, M, N, K, m_tiles, n_tiles, gate);
+  const dim3 grid(8u * (unsigned)(((long long)m_tiles * n_tiles + 7) / 8), PARTS ? (segments(K) + 1) / 2 : 1), block(PARTS ? 128 : 64 * SEGMENTS);
+  if (PARTS || (K % 4 == 0 && (uintptr_t)x % 16 == 0 && (uintptr_t)w % 16 == 0))
+    hipLaunchKernelGGL((gemm_float32_kernel<RT, CT, U, GATED, PARTS, true>), grid, block, 0, s, x, w, bias, y, M, N, K, m_tiles, n_tiles, gate);
   else
-    hipLaunchKernelGGL((gemm_float32_kernel<RT, CT, U, GATED, false>), grid, block, 0, s, x, w, bias, y, M, N, K, m_tiles, n_tiles, gate);
+    hipLaunchKernelGGL((gemm_float32_kernel<RT, CT, U, GATED, false, false>), grid, block, 0, s, x, w, bias, y, M, N, K, m_tiles, n_tiles, gate);
 }
 
 // ---------------------------------------------------------------- many rows
 // 4 waves, 2 x 2, a wave RT x CT tiles of 16 x 16; the parts of both operands through LDS in pieces of 32 k, two buffers, two
 // pieces under way in registers: an entry is taken apart once a block. A wave takes every segment in turn and adds it to the
-// total: the same sums in the same order as above. What bounds it: matrix and vector instructions (24 and 72 of them a piece
-// and wave of the large tile) add up more than they overlap, within a wave and between two of a SIMD; so three blocks a
-// compute unit, which is why LDS rows have no padding and only two pieces are under way (two blocks, with 80-byte rows and
-// four pieces: 517 x 4096 . 1024 in 58 us in place of 45, before the factors 2^16). 2 x 2 tiles a wave: 1,500 x 12,288 . 2048 in 564 us (134 TFLOP/s;
-// float matrix instructions 672).
+// total: the same sums in the same order as above. What bounds it is a block's chain of pieces (0.4 us each at 32 x 32); for the middling
+// numbers of rows and outputs whose larger tiles would leave units idle.
 #define PIECE 32
 #define AHEAD 2
 template <int RT, int CT, bool GATED, bool WIDE>
-__global__ __launch_bounds__(256, RT * CT > 2 ? 3 : 4) void gemm_float32_tiles_kernel(const float* __restrict__ x, const float* __restrict__ w,
+__global__ __launch_bounds__(256, 4) void gemm_float32_tiles_kernel(const float* __restrict__ x, const float* __restrict__ w,
                                                                  const float* __restrict__ bias, float* __restrict__ y, int M, int N,
                                                                  int K, int m_tiles, int n_tiles, NhvGate gate) {
   static_assert(!GATED || CT == 2, "a gate tile and its up tile");
@@ -386,27 +399,210 @@ static void launch_tiles(const float* x, const float* w, const float* bias, floa
     hipLaunchKernelGGL((gemm_float32_tiles_kernel<RT, CT, GATED, false>), grid, block, 0, s, x, w, bias, y, M, N, K, m_tiles, n_tiles, gate);
 }
 
+// The same with 32 x 32 outputs a matrix instruction, CT of them a wave: 64 rows by 64 CT columns a block. A 32x32x16 instruction leaves
+// vector instructions three quarters of its 32 clocks, a 16x16x32 one next to nothing of its 16 (two waves of a SIMD, ns for two matrix
+// and twelve vector instructions: 31 where 27 and 22 apart; 39 for as many products of the smaller kind). Two of them in a
+// row sum eight k after eight k as one of the other kind does: the same bits.
+// PARTS: a block sums one segment, whose sums are the result (times 2^32, [segment][M][N]): K over blocks where there are few outputs.
+// What bounds it: a piece takes a block 0.8 us (24 matrix instructions a wave are 0.37, its 190 others as much), and two blocks on
+// a unit hardly less each. Rows of LDS turn by their number / 4: 16-byte reads go in quarters of lanes 0-3, 12-15, 20-23, 24-27 and
+// the like (by / 2: 8 % slower). Asked for LDS one piece ahead, with two barriers or a third buffer, it was no faster.
+// us, tiles of 64 x 64 of 16x16x32 instructions in brackets: 517 x 4096 . 1024 47 (53), gated 517 x 3072 . 1024 56 (67), 300 x 6144 . 2048 106 (140),
+// 1,500 x 12,288 . 2048 454 (550).
+// WHOLE: K a multiple of 32, rows on 16-byte boundaries.
+template <int CT, bool GATED, bool PARTS, bool WHOLE>
+__global__ __launch_bounds__(256, CT == 2 ? 2 : 3) void gemm_float32_blocks_kernel(const float* __restrict__ x, const float* __restrict__ w,
+                                                                                   const float* __restrict__ bias, float* __restrict__ y, int M, int N,
+                                                                                   int K, int m_tiles, int n_tiles, NhvGate gate) {
+  static_assert(!GATED || (CT == 2 && !PARTS), "a gate tile and its up tile");
+  static_assert(!PARTS || WHOLE, "parts of whole pieces");
+  constexpr int BM = 64, BN = 64 * CT, LOADS = (BM + BN) / 64, PLANE = (BM + BN) * PIECE, OUT = GATED ? BN / 2 : BN, TOTALS = PARTS ? 1 : CT;
+  __shared__ __attribute__((aligned(16))) bf16_t rows[2][3 * PLANE];
+  const int total_tiles = m_tiles * n_tiles, share = (total_tiles + 7) >> 3;
+  const int tile = (blockIdx.x & 7) * share + (blockIdx.x >> 3);
+  if (tile >= total_tiles) return;
+  const int m0 = (tile % m_tiles) * BM, n0 = (tile / m_tiles) * OUT;
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, r32 = lane & 31, half = lane >> 5;
+  const int mw = (wave >> 1) * 32, nw = (wave & 1) * 32 * CT;
+  const int length = segment_length(K), begin = PARTS ? blockIdx.y * length : 0, end = PARTS ? min(K, begin + length) : K;
+  // what this thread brings of a piece: 16 bytes of each half of the 128 of rows row, row + 64, ...: an address that the wave shares, and
+  // an offset of less than 2^32
+  const int col = (threadIdx.x & 3) * 4, row = threadIdx.x >> 2;
+  const float* base[LOADS];
+  uint32_t offset[LOADS];
+#pragma unroll
+  for (int i = 0; i < LOADS; ++i) {
+    // (gated: 32 gate rows and their 32 up rows in turn)
+    const int b = row + 64 * (i - 1), n = GATED ? n0 + (b >> 6) * 32 + (b & 31) : n0 + b;
+    const int up = GATED ? __builtin_amdgcn_readfirstlane((b >> 5) & 1) : 0;
+    base[i] = i == 0 ? x + (size_t)m0 * K : w + ((size_t)up * N + n0) * K;
+    offset[i] = (uint32_t)(i == 0 ? min(row, M - 1 - m0) : min(n, N - 1) - n0) * (uint32_t)K;
+  }
+  const int to_row = row * PIECE + (((threadIdx.x & 3) ^ (row >> 2 & 3)) << 3);
+  f32x4 hold[AHEAD][LOADS][2];
+  auto ask = [&](int i_hold, int k0) {
+    const int at = WHOLE ? min(k0, K - PIECE) : k0;        // (beyond the last piece it again, into registers that nobody reads)
+#pragma unroll
+    for (int i = 0; i < LOADS; ++i)
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+        hold[i_hold][i][h] = WHOLE ? *reinterpret_cast<const f32x4*>(base[i] + at + (offset[i] + col + 16 * h)) : four_of<false>(base[i] + offset[i], at + col + 16 * h, K);
+  };
+  auto put = [&](int buf, int i_hold, int i) {
+    const SplitFloats8 p = split_floats(hold[i_hold][i][0], hold[i_hold][i][1]);
+    bf16_t* to = &rows[buf][64 * i * PIECE + to_row];
+    *reinterpret_cast<bf16x8*>(to) = p.high;
+    *reinterpret_cast<bf16x8*>(to + PLANE) = p.middle;
+    *reinterpret_cast<bf16x8*>(to + 2 * PLANE) = p.rest;
+  };
+  f32x16 acc[CT], low[CT], total[TOTALS];
+#pragma unroll
+  for (int c = 0; c < CT; ++c)
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      acc[c][i] = low[c][i] = 0.f;
+      if (!PARTS) total[c % TOTALS][i] = -0.f;
+    }
+  auto close = [&] {                                     // a segment's end
+#pragma unroll
+    for (int c = 0; c < CT; ++c) {
+      total[c % TOTALS] += acc[c] + low[c];
+#pragma unroll
+      for (int i = 0; i < 16; ++i) acc[c][i] = low[c][i] = 0.f;
+    }
+  };
+  // (a lane holds rows 8 (i / 4) + 4 half + i % 4 of column r32 of a tile)
+  auto row_of = [&](int i) { return m0 + mw + 8 * (i >> 2) + 4 * half + (i & 3); };
+  int left = length;                                     // of the segment
+#pragma unroll
+  for (int d = 0; d < AHEAD; ++d) ask(d, begin + d * PIECE);
+#pragma unroll
+  for (int i = 0; i < LOADS; ++i) put(0, 0, i);
+  ask(0, begin + AHEAD * PIECE);
+  __syncthreads();
+  int a_at[2], b_at[2];                                  // of 16 k: lane groups' 8 k are pieces 2 s and 2 s + 1
+#pragma unroll
+  for (int s = 0; s < 2; ++s) {
+    a_at[s] = (mw + r32) * PIECE + (((2 * s + half) ^ (r32 >> 2 & 3)) << 3);
+    b_at[s] = (BM + nw + r32) * PIECE + (((2 * s + half) ^ (r32 >> 2 & 3)) << 3);
+  }
+  for (int k0 = begin; k0 < end; k0 += AHEAD * PIECE) {
+#pragma unroll
+    for (int d = 0; d < AHEAD; ++d) {                    // (piece d lies in buffer d)
+      const int k = k0 + d * PIECE, buf = d;
+      if (k >= end) break;
+      // the parts in the order in which the products need them
+      SplitFloats8 a[2], b[2][CT];
+      auto part = [&](int at, int plane) { return *reinterpret_cast<const bf16x8*>(&rows[buf][at + plane * PLANE]); };
+#pragma unroll
+      for (int s = 0; s < 2; ++s) a[s].middle = part(a_at[s], 1);
+#pragma unroll
+      for (int s = 0; s < 2; ++s)
+#pragma unroll
+        for (int c = 0; c < CT; ++c) b[s][c].middle = part(b_at[s] + 32 * c * PIECE, 1);
+#pragma unroll
+      for (int s = 0; s < 2; ++s) a[s].rest = part(a_at[s], 2);
+#pragma unroll
+      for (int s = 0; s < 2; ++s)
+#pragma unroll
+        for (int c = 0; c < CT; ++c) b[s][c].high = part(b_at[s] + 32 * c * PIECE, 0);
+#pragma unroll
+      for (int s = 0; s < 2; ++s) a[s].high = part(a_at[s], 0);
+#pragma unroll
+      for (int s = 0; s < 2; ++s)
+#pragma unroll
+        for (int c = 0; c < CT; ++c) b[s][c].rest = part(b_at[s] + 32 * c * PIECE, 2);
+#pragma unroll
+      for (int step = 0; step < 6; ++step) {
+#pragma unroll
+        for (int s = 0; s < 2; ++s)
+#pragma unroll
+          for (int c = 0; c < CT; ++c) split_product(step, a[s], b[s][c], acc[c], low[c]);
+        if (step < LOADS) put(buf ^ 1, d ^ 1, step);
+      }
+      ask(d ^ 1, k + (1 + AHEAD) * PIECE);
+      left -= PIECE;
+      if (!PARTS && left == 0) {
+        left = length;
+        asm volatile("");                                // (a real branch)
+        close();
+      }
+      __syncthreads();
+    }
+  }
+  if (PARTS) {
+#pragma unroll
+    for (int c = 0; c < CT; ++c) {
+      const int n = n0 + nw + 32 * c + r32;
+#pragma unroll
+      for (int i = 0; i < 16; ++i) {
+        const int m = row_of(i);
+        if (m < M && n < N) y[((size_t)blockIdx.y * M + m) * N + n] = acc[c][i] + low[c][i];
+      }
+    }
+    return;
+  }
+  if (left != length) close();                           // (the last segment is shorter and not added yet)
+#pragma unroll
+  for (int c = 0; c < CT; c += GATED ? 2 : 1) {
+    const int n = n0 + (GATED ? nw / 2 : nw + 32 * c) + r32;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      const int m = row_of(i);
+      const bool in = m < M && n < N;
+      float v[GATED ? 2 : 1];
+#pragma unroll
+      for (int both = 0; both < (GATED ? 2 : 1); ++both) {
+        const float t = total[(c + both) % TOTALS][i];
+        const bool odd = in && !finite(t);
+        v[both] = t * SPLIT_UNSCALE;
+        if (__any(odd)) v[both] = plain_products(x, w, K, v[both], m, both * N + n, odd);
+      }
+      if (in) {
+        if (bias) {
+#pragma unroll
+          for (int both = 0; both < (GATED ? 2 : 1); ++both) v[both] += bias[both * N + n];
+        }
+        y[(size_t)m * N + n] = GATED ? nhv_gated(v[0], v[GATED], gate) : v[0];
+      }
+    }
+  }
+}
+
+template <int CT, bool GATED, bool PARTS = false>
+static void launch_blocks(const float* x, const float* w, const float* bias, float* y, int M, int N, int K, const NhvGate& gate, hipStream_t s) {
+  constexpr int COLS = GATED ? 32 * CT : 64 * CT;
+  const int m_tiles = (M + 63) / 64, n_tiles = (N + COLS - 1) / COLS;
+  const dim3 grid(8u * (unsigned)(((long long)m_tiles * n_tiles + 7) / 8), PARTS ? segments(K) : 1), block(256);
+  if (PARTS || (K % PIECE == 0 && K < (1 << 22) && (uintptr_t)x % 16 == 0 && (uintptr_t)w % 16 == 0))
+    hipLaunchKernelGGL((gemm_float32_blocks_kernel<CT, GATED, PARTS, true>), grid, block, 0, s, x, w, bias, y, M, N, K, m_tiles, n_tiles, gate);
+  else
+    hipLaunchKernelGGL((gemm_float32_blocks_kernel<CT, GATED, false, false>), grid, block, 0, s, x, w, bias, y, M, N, K, m_tiles, n_tiles, gate);
+}
+
 // Every tile's time in units of what a compute unit needs for 16 rows of an operand, from the times of all tiles at 1 to 1,500
 // rows of the 0.6B and 1.7B shapes' products. Tiles of 8 waves: rounds of 256 blocks times 16-row operands; the tiles through
-// LDS: a floor (one block's chain of pieces) and what a block a compute unit adds. E.g. 17 x 6144 . 1024: 32 x 32 10.1 us,
-// 16 x 32 14.0, 16 x 16 13.9 (float matrix instructions 12.6); 130 x 2048 . 2048: 48 x 32 22.1 us, 32 x 32 33.3 (33.2); 517 x
-// 1024 . 3072: 32 x 32 through LDS 58.9, 48 x 32 60.0, 64 x 64 66.6 (71); 517 x 4096 . 1024: 64 x 64 45, 32 x 32 through LDS 56
-// (57). Up to 16 rows LDS has nothing to share and is left out (6 x 151,936 . 1024: 116 us with 16 x 32, 135 through LDS; 137).
-// 32 x 16, whose second 16 rows are few different ones at 17 rows and 16 at 32: 17 x 4096 . 4096 24.2 us, 16 x 32 27.4 (24.3); 32 rows 29.2 and 28.1.
+// LDS: a floor (one block's chain of pieces) and what a block a compute unit adds (64 x 128: whole rounds). E.g. 17 x 6144 . 1024: 32 x 32 10.1 us,
+// 16 x 32 14.0, 16 x 16 13.9; 130 x 2048 . 2048: 48 x 32 21.9 us, 32 x 32 33.7, 64 x 64 42.4; 517 x 4096 . 1024: 64 x 64 46, 64 x 128 50, 32 x 32
+// through LDS 56; 1,500 x 4096 . 1024: 98, 90 and 147. Up to 16 rows LDS has nothing to share and is left out (6 x 151,936 . 1024: 116 us with 16 x 32,
+// 135 through LDS).
+// 32 x 16, whose second 16 rows are few different ones at 17 rows and 16 at 32: 17 x 4096 . 4096 24.2 us, 16 x 32 27.4; 32 rows 29.2 and 28.1.
 struct Choice {
   int tile;
   double cost;
 };
+static double wide_tiles(long long blocks) { return fmax(15.2, 13.3 * (blocks <= 2048 ? (double)((blocks + 255) / 256) : blocks / 256.0) - 1.5); }
 static Choice plain_tile(long long M, long long N) {
   auto blocks = [&](long long m, long long n) { return ((M + m - 1) / m) * ((N + n - 1) / n); };
   auto rounds = [&](int rt, int ct) { return (double)((blocks(16 * rt, 16 * ct) + 255) / 256 * (rt + ct)); };
   const double none = 1e300;
-  const double cost[7] = {rounds(1, 1), rounds(1, 2), M > 16 ? rounds(2, 2) : none, M > 32 ? rounds(3, 2) : none,
+  const double cost[8] = {rounds(1, 1), rounds(1, 2), M > 16 ? rounds(2, 2) : none, M > 32 ? rounds(3, 2) : none,
                           M > 16 ? fmax(9.0, 1.5 + 2.9 / 256 * blocks(32, 32)) : none,
-                          M > 16 ? fmax(11.5, 4.5 + 7.7 / 256 * blocks(64, 64)) : none,
-                          M > 16 && M <= 32 ? rounds(2, 1) / 3 * (2.05 + 0.035 * M) : none};
+                          M > 16 ? fmax(11.5, 6.0 + 7.7 / 256 * blocks(64, 64)) : none,
+                          M > 16 && M <= 32 ? rounds(2, 1) / 3 * (2.05 + 0.035 * M) : none,
+                          M > 16 ? wide_tiles(blocks(64, 128)) : none};
   Choice best = {0, cost[0]};
-  for (int i = 1; i < 7; ++i)
+  for (int i = 1; i < 8; ++i)
     if (cost[i] < best.cost) best = {i, cost[i]};
   return best;
 }
@@ -417,7 +613,7 @@ static Choice gated_tile(long long M, long long N) {
   const double none = 1e300;
   const double cost[5] = {rounds(1), M > 16 ? rounds(2) : none, M > 32 ? rounds(3) : none,
                           M > 16 ? fmax(9.5, 3.0 + 4.9 / 256 * blocks(32, 32)) : none,
-                          M > 16 ? fmax(11.5, 4.5 + 7.7 / 256 * blocks(64, 32)) : none};
+                          M > 16 ? wide_tiles(blocks(64, 64)) : none};
   Choice best = {0, cost[0]};
   for (int i = 1; i < 5; ++i)
     if (cost[i] < best.cost) best = {i, cost[i]};
@@ -436,10 +632,145 @@ extern "C" int nhv_gemm_float32(const void* x, const void* w, const void* bias, 
     case 2: launch<2, 2, 1, false>(xf, wf, bf, yf, M, N, K, {}, s); break;
     case 3: launch<3, 2, 1, false>(xf, wf, bf, yf, M, N, K, {}, s); break;
     case 4: launch_tiles<1, 1, false>(xf, wf, bf, yf, M, N, K, {}, s); break;
-    case 5: launch_tiles<2, 2, false>(xf, wf, bf, yf, M, N, K, {}, s); break;
+    case 5: launch_blocks<1, false>(xf, wf, bf, yf, M, N, K, {}, s); break;
+    case 7: launch_blocks<2, false>(xf, wf, bf, yf, M, N, K, {}, s); break;
     default: launch<2, 1, 2, false>(xf, wf, bf, yf, M, N, K, {}, s);
   }
   NHV_LAUNCH_CHECK("gemm_float32");
+  return 0;
+}
+
+// ---------------------------------------------------------------- parts that their reader adds up
+// How many parts (the segments of K) a product is best left in for a reader that adds them up; 0: it is best finished here. us, cold
+// weights, finished and in parts: 6 rows, 1024 . 2048 8.7, 6.5, 1024 . 3072 11.6, 7.0, 2048 . 6144 19.2, 15.0, but 4096 . 2048 8.9, 9.6; 65 rows, 1024 . 3072 18.8,
+// 11.4; 130 rows, 1024 . 3072 24.5, 14.7, 2048 . 6144 56.7, 37, 4096 . 2048 41.6, 28.4; 517 rows, 1024 . 2048 43, 24.4, 1024 . 3072 61.6, 33, 2048 . 6144 156, 101.
+// The reader then takes in 8 entries for one, at 4 TB/s (517 x 2048 7 us), which 517 x 4096 . 2048 (87 and 77) and 1,500 x 2048 . 2048 (98 and 97) lose by.
+extern "C" int nhv_gemm_float32_parts_count(const void* x, const void* w, int M, int N, int K) {
+  const bool whole = M > 0 && N > 0 && K % PIECE == 0 && K >= 512 && K < (1 << 22) && (uintptr_t)x % 16 == 0 && (uintptr_t)w % 16 == 0;
+  return whole && (M <= 16 ? N <= 2560 : (long long)M * N <= 1200000) ? segments(K) : 0;
+}
+
+// y[segments][M][N], times 2^32. Up to 16 rows two waves a block, each with all of a segment under way (one with half of it: 8.1 us where 7.0
+// are kept at 1024 . 3072); else tiles of 64 x 64, or of 64 x 128, which read x half as often, where few tiles of rows leave w the larger part of
+// what is read (130 x 4096 . 2048 32.2 and 28.4 us, 517 x 1024 . 3072 33 and 38).
+extern "C" int nhv_gemm_float32_parts(const void* x, const void* w, void* y, int M, int N, int K, void* stream) {
+  NHV_REQUIRE(M > 0 && N > 0 && K > 0 && K % PIECE == 0 && K < (1 << 22), "gemm in parts: bad sizes M=%d N=%d K=%d (a multiple of %d)", M, N, K, PIECE);
+  NHV_REQUIRE((((uintptr_t)x | (uintptr_t)w) & 15) == 0, "gemm in parts: rows off 16-byte boundaries");
+  NHV_REQUIRE((((long long)M + 15) / 16) * (((long long)N + 15) / 16) < (1ll << 27), "gemm in parts: too many rows (%d) for %d columns", M, N);
+  hipStream_t s = (hipStream_t)stream;
+  const float *xf = (const float*)x, *wf = (const float*)w;
+  float* yf = (float*)y;
+  const long long tiles = (((long long)M + 63) / 64) * (((long long)N + 63) / 64);
+  if (M <= 16) launch<1, 1, 4, false, true>(xf, wf, nullptr, yf, M, N, K, {}, s);
+  else if (tiles * segments(K) > 3000 || (M > 64 && M <= 192 && N >= 2048)) launch_blocks<2, false, true>(xf, wf, nullptr, yf, M, N, K, {}, s);
+  else launch_blocks<1, false, true>(xf, wf, nullptr, yf, M, N, K, {}, s);
+  NHV_LAUNCH_CHECK("gemm_float32_parts");
+  return 0;
+}
+
+// Eight neighbouring outputs of row m from their parts: the finished product's bits. The whole wave comes here; `in`: the lane has outputs.
+__device__ __forceinline__ void finish_parts8(const float* __restrict__ parts, int count, size_t stride, const float* __restrict__ x,
+                                              const float* __restrict__ w, int K, int m, int n, size_t at, bool in, float* v) {
+  f32x4 part[SEGMENTS][2];
+#pragma unroll
+  for (int p = 0; p < SEGMENTS; ++p)                       // (all are asked for before the first is used; those beyond the last are it again)
+#pragma unroll
+    for (int h = 0; h < 2; ++h) part[p][h] = *reinterpret_cast<const f32x4*>(parts + (in ? min(p, count - 1) * stride + at : 0) + 4 * h);
+#pragma unroll
+  for (int e = 0; e < 8; ++e) {
+    float sum = part[0][e >> 2][e & 3];
+#pragma unroll
+    for (int p = 1; p < SEGMENTS; ++p)
+      if (p < count) sum += part[p][e >> 2][e & 3];
+    const bool odd = in && !finite(sum);
+    v[e] = sum * SPLIT_UNSCALE;
+    if (__any(odd)) v[e] = plain_products(x, w, K, v[e], m, n + e, odd);
+  }
+}
+
+// residual += the product whose parts these are; y = the norm of the sum: what rmsnorm does with mode 1, bit for bit.
+// 6 rows of 1,024 in 8 parts take 4.8 us in a recorded step, of the finished product 4.6; 517 rows 8.6 and 5.1.
+template <int MAXC>
+__global__ __launch_bounds__(1024) void add_parts_norm_float32_kernel(const float* __restrict__ parts, int count, const float* __restrict__ x,
+                                                                      const float* __restrict__ xw, int K, float* __restrict__ residual,
+                                                                      const float* __restrict__ w, float* __restrict__ y, int H, float eps) {
+  __shared__ float scratch[16];
+  const size_t base = (size_t)blockIdx.x * H, stride = (size_t)gridDim.x * H;
+  const int nch = H / 8;
+  float v[MAXC][8];
+  float ss = 0.f;
+#pragma unroll
+  for (int c = 0; c < MAXC; ++c) {
+    const int ch = threadIdx.x + c * blockDim.x;
+    const bool in = ch < nch;
+    f32x4 r[2];
+#pragma unroll
+    for (int h = 0; h < 2; ++h) r[h] = *reinterpret_cast<const f32x4*>(residual + base + (in ? ch * 8 : 0) + 4 * h);
+    finish_parts8(parts, count, stride, x, xw, K, blockIdx.x, ch * 8, base + ch * 8, in, v[c]);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) v[c][e] = in ? v[c][e] + r[e >> 2][e & 3] : 0.f;
+  }
+#pragma unroll
+  for (int c = 0; c < MAXC; ++c) {
+    const int ch = threadIdx.x + c * blockDim.x;
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+      if (ch < nch) *reinterpret_cast<f32x4*>(residual + base + ch * 8 + 4 * h) = f32x4{v[c][4 * h], v[c][4 * h + 1], v[c][4 * h + 2], v[c][4 * h + 3]};
+#pragma unroll
+    for (int e = 0; e < 8; ++e) ss += v[c][e] * v[c][e];
+  }
+  const float total = block_sum(ss, scratch);
+  const float r = 1.0f / sqrtf(total / (float)H + eps);
+#pragma unroll
+  for (int c = 0; c < MAXC; ++c) {
+    const int ch = threadIdx.x + c * blockDim.x;
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+      if (ch < nch) {
+        const f32x4 g = *reinterpret_cast<const f32x4*>(w + ch * 8 + 4 * h);
+        *reinterpret_cast<f32x4*>(y + base + ch * 8 + 4 * h) =
+            f32x4{v[c][4 * h] * r * g[0], v[c][4 * h + 1] * r * g[1], v[c][4 * h + 2] * r * g[2], v[c][4 * h + 3] * r * g[3]};
+      }
+  }
+}
+
+// x[T, K] and xw[H, K]: the product's operands, from which outputs that are not finite are made once more
+extern "C" int nhv_add_parts_norm_float32(const void* parts, int count, const void* x, const void* xw, int K, void* residual, const void* w, void* y,
+                                          int T, int H, float eps, void* stream) {
+  NHV_REQUIRE(T > 0 && H > 0 && H % 8 == 0 && H <= 16384 && K > 0, "add_parts_norm: bad sizes T=%d H=%d K=%d", T, H, K);
+  NHV_REQUIRE(count == segments(K), "add_parts_norm: %d parts of a product over %d", count, K);
+  NHV_REQUIRE((((uintptr_t)parts | (uintptr_t)residual | (uintptr_t)w | (uintptr_t)y) & 15) == 0, "add_parts_norm: rows off 16-byte boundaries");
+  const int nch = H / 8, threads = nch <= 1024 ? (nch + 63) / 64 * 64 : 1024;
+  auto kernel = nch <= 1024 ? add_parts_norm_float32_kernel<1> : add_parts_norm_float32_kernel<2>;
+  hipLaunchKernelGGL(kernel, dim3(T), dim3(threads), 0, (hipStream_t)stream, (const float*)parts, count, (const float*)x, (const float*)xw, K,
+                     (float*)residual, (const float*)w, (float*)y, H, eps);
+  NHV_LAUNCH_CHECK("add_parts_norm_float32");
+  return 0;
+}
+
+// y[M, N] = the product whose parts these are, one output a lane, a row's lanes in whole waves
+__global__ __launch_bounds__(256) void sum_parts_float32_kernel(const float* __restrict__ parts, int count, const float* __restrict__ x,
+                                                                const float* __restrict__ w, int K, float* __restrict__ y, int M, int N) {
+  const int n = blockIdx.y * 256 + threadIdx.x;
+  for (int m = blockIdx.x; m < M; m += gridDim.x) {
+    const bool in = n < N;
+    float v = 0.f;
+    if (in) {
+      v = parts[(size_t)m * N + n];
+      for (int p = 1; p < count; ++p) v += parts[((size_t)p * M + m) * N + n];
+    }
+    const bool odd = in && !finite(v);
+    v *= SPLIT_UNSCALE;
+    if (__any(odd)) v = plain_products(x, w, K, v, m, n, odd);
+    if (in) y[(size_t)m * N + n] = v;
+  }
+}
+
+extern "C" int nhv_sum_parts_float32(const void* parts, int count, const void* x, const void* w, int K, void* y, int M, int N, void* stream) {
+  NHV_REQUIRE(M > 0 && N > 0 && N < (1 << 23) && K > 0 && count == segments(K), "sum_parts: %d parts of a product M=%d N=%d K=%d", count, M, N, K);
+  hipLaunchKernelGGL(sum_parts_float32_kernel, dim3(M < 4096 ? M : 4096, (N + 255) / 256), dim3(256), 0, (hipStream_t)stream, (const float*)parts, count,
+                     (const float*)x, (const float*)w, K, (float*)y, M, N);
+  NHV_LAUNCH_CHECK("sum_parts_float32");
   return 0;
 }
 
@@ -469,7 +800,7 @@ extern "C" int nhv_gemm_float32_gated(const void* x, const void* w, const void* 
     case 1: launch<2, 2, 1, true>(xf, wf, bf, yf, M, N, K, gate, s); break;
     case 2: launch<3, 2, 1, true>(xf, wf, bf, yf, M, N, K, gate, s); break;
     case 3: launch_tiles<1, 2, true>(xf, wf, bf, yf, M, N, K, gate, s); break;
-    default: launch_tiles<2, 2, true>(xf, wf, bf, yf, M, N, K, gate, s);
+    default: launch_blocks<2, true>(xf, wf, bf, yf, M, N, K, gate, s);
   }
   NHV_LAUNCH_CHECK("gemm_float32_gated");
   return 0;

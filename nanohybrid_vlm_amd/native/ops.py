@@ -221,6 +221,15 @@ class NativeBackend:
         self._call("nhv_add_parts_norm", _ptr(parts), S, _ptr(residual), dtype_code(residual), _ptr(w), _ptr(y), T, H, ctypes.c_float(eps),
                    int(rounds_between), dtype_code(w), _stream())
 
+    def add_parts_norm_float32(self, parts, operands, residual, w, y, eps):
+        (S, T, H), (x, xw) = parts.shape, operands
+        self._call("nhv_add_parts_norm_float32", _ptr(parts), S, _ptr(x), _ptr(xw), x.shape[1], _ptr(residual), _ptr(w), _ptr(y), T, H,
+                   ctypes.c_float(eps), _stream())
+
+    def sum_parts_float32(self, parts, operands, out):
+        (S, M, N), (x, w) = parts.shape, operands
+        self._call("nhv_sum_parts_float32", _ptr(parts), S, _ptr(x), _ptr(w), x.shape[1], _ptr(out), M, N, _stream())
+
     def sum_parts(self, parts, out):
         self._call("nhv_sum_parts", _ptr(parts), parts.shape[0], _ptr(out), ctypes.c_size_t(out.numel()), _stream())
 
@@ -853,6 +862,15 @@ class NativeBackend:
         self._call("nhv_gemm_lines_bf16", _ptr(x), _ptr(w), _ptr(None), _ptr(parts), x.shape[0], w.shape[0], x.shape[1], 0, *Gate().args(), _stream())
         return parts
 
+    def float32_parts(self, x, w):
+        """2^32 times x W^T of floats as parts [parts, rows, out], or None where the finished product is the faster way."""
+        count = self.lib.nhv_gemm_float32_parts_count(_ptr(x), _ptr(w), x.shape[0], w.shape[0], x.shape[1])
+        if not count:
+            return None
+        parts = torch.empty((count, x.shape[0], w.shape[0]), dtype=torch.float32, device=x.device)
+        self._call("nhv_gemm_float32_parts", _ptr(x), _ptr(w), _ptr(parts), x.shape[0], w.shape[0], x.shape[1], _stream())
+        return parts
+
     norm_kernel_ms = 0.003        # what a norm's own kernel costs in a decoding step, about
 
     def _measured(self, x, w, gated: bool):
@@ -1129,6 +1147,7 @@ class Parts:
 
     parts: torch.Tensor
     dtype: torch.dtype            # the rows' element type
+    operands: tuple | None = None # of a float32 product: (x, w). Its parts are 2^32 times it, and what their sum cannot hold is made anew
 
     @property
     def shape(self):
@@ -1140,7 +1159,10 @@ class Parts:
 
     def tensor(self) -> torch.Tensor:
         out = torch.empty(self.shape, dtype=self.dtype, device=self.device)
-        backend().sum_parts(self.parts, out)
+        if self.operands is not None:
+            backend().sum_parts_float32(self.parts, self.operands, out)
+        else:
+            backend().sum_parts(self.parts, out)
         return out
 
 
@@ -1223,6 +1245,9 @@ def rmsnorm(x: torch.Tensor, w: torch.Tensor, eps: float, residual: torch.Tensor
         _dense(residual, "rmsnorm: residual", tuple(x.shape))
         _need(residual.dtype == x.dtype or residual.dtype == torch.float32, lambda: f"rmsnorm: residual of {residual.dtype} with rows of {x.dtype}")
         y = torch.empty(x.shape, dtype=x.dtype, device=x.device)
+        if x.operands is not None:
+            backend().add_parts_norm_float32(x.parts, x.operands, residual, w, y, float(eps))     # (float32 throughout: nothing is rounded in between)
+            return y
         backend().add_parts_norm(x.parts, residual, w, y, float(eps), **({} if rounds_between else {"rounds_between": False}))
         return y
     _need(x.dim() == 2, "rmsnorm: x must be [tokens, width]")
@@ -1288,7 +1313,7 @@ def qk_rope_write(qkv, bias, q_norm_w, k_norm_w, eps, cos_sin, positions, slot_m
     T = qkv.shape[0]
     width = (num_heads + 2 * num_kv_heads) * head_dim
     split = qkv if isinstance(qkv, Parts) else None
-    if split is not None and not rotation_takes_parts(head_dim, cos_sin, pair_axes, bias, q_norm_w, k_norm_w, *((k_cache, v_cache) if write_kv else ())):
+    if split is not None and (split.operands is not None or not rotation_takes_parts(head_dim, cos_sin, pair_axes, bias, q_norm_w, k_norm_w, *((k_cache, v_cache) if write_kv else ()))):
         qkv, split = qkv.tensor(), None
     _dense(qkv if split is None else split.parts, "qk_rope_write: qkv", (T, width) if split is None else (split.parts.shape[0], T, width))
     if split is None:
@@ -1428,13 +1453,16 @@ def linear(x, w: torch.Tensor, bias: torch.Tensor | None = None, out_dtype=None,
         backend().fused_linear(x, w, bias, None, row_scales=scales, residual=residual, sum_out=weighted, ss_out=squares,
                                next_w=add_to.norm_weight)
         return Summed(weighted, squares, residual, add_to.norm_weight, add_to.eps)
-    if add_to is not None and add_to.takes_parts:
-        parts = parts or norm_takes_parts(N, add_to.norm_weight, add_to.residual)
-    if parts and normed is None and bias is None and out_dtype == x.dtype:
+    for_norm = add_to is not None and add_to.takes_parts and norm_takes_parts(N, add_to.norm_weight, add_to.residual)
+    if (parts or for_norm) and normed is None and bias is None and out_dtype == x.dtype:
         make = getattr(backend(), "linear_parts", None)
         made = None if make is None else make(x, w)
         if made is not None:
             return Parts(made, x.dtype)
+        make = getattr(backend(), "float32_parts", None) if for_norm and x.dtype == torch.float32 else None      # (no other reader adds up these)
+        made = None if make is None else make(x, w)
+        if made is not None:
+            return Parts(made, x.dtype, (x, w))
     out = torch.empty((M, N), dtype=out_dtype, device=x.device)
     if normed is not None:
         backend().fused_linear(x, w, bias, out, row_scales=scales)

@@ -311,6 +311,51 @@ def test_float32_linear_in_all_its_tiles(ops, N, K):
         last = y
 
 
+@pytest.mark.parametrize("M,N,K", [(1090, 4100, 64), (1090, 4100, 70), (577, 4130, 256), (577, 4130, 33), (321, 4096, 1000)])
+def test_float32_linear_in_tiles_of_64_rows(ops, M, N, K):
+    """Tiles of 64 x 64 and 64 x 128, whole pieces of 32 columns and not, plain and gated: the rows that few rows alone give, bit for bit."""
+    x, w, b = rnd(M, K, seed=121), rnd(2 * N, K, seed=122), rnd(2 * N, seed=123)
+    y, g = ops.linear(x, w[:N], b[:N]), ops.gated_linear(x, w, "silu", b)
+    for rows in (slice(0, 16), slice(M - 5, M), slice(60, 70)):
+        some = x[rows].contiguous()
+        assert torch.equal(y[rows], ops.linear(some, w[:N], b[:N]))
+        assert torch.equal(g[rows], ops.act_mul(ops.linear(some, w), "silu", b))
+
+
+@pytest.mark.parametrize("M,N,K", [(1, 64, 512), (6, 1024, 3072), (16, 2560, 544), (17, 72, 1024), (65, 1000, 2080), (150, 2056, 512), (517, 1024, 768)])
+def test_float32_parts_through_the_norm(ops, M, N, K):
+    """The norm that adds up a product's parts gives the bits of the norm that takes the finished product, and leaves the same sums in the
+    residual; so does the kernel that only adds them up. With sums beyond 2^96 and entries that are no numbers as well."""
+    norm_w = 1 + 0.1 * rnd(N, seed=133)
+    for odd in (False, True):
+        x, w, r = rnd(M, K, seed=131), rnd(N, K, seed=132), rnd(M, N, seed=134)
+        if odd:
+            x[M // 2] *= 1e16
+            w[N // 3] *= 1e16
+            w[5, K - 1], x[0, K // 2] = float("inf"), float("nan") if M > 1 else 1.0
+        rows = ops.linear(x, w)
+        want_r = r.clone()
+        want = ops.rmsnorm(rows, norm_w, 1e-6, residual=want_r)
+        made = ops.linear(x, w, add_to=ops.AddTo(r, norm_w, 1e-6, None, takes_parts=True))
+        assert isinstance(made, ops.Parts) and made.shape == (M, N)
+        same = lambda a, b: torch.equal(a.isnan(), b.isnan()) and torch.equal(a.nan_to_num(1.5, 2.5, 3.5), b.nan_to_num(1.5, 2.5, 3.5))
+        assert same(made.tensor(), rows)
+        got = ops.rmsnorm(made, norm_w, 1e-6, residual=r)
+        assert same(got, want) and same(r, want_r)
+
+
+def test_which_float32_products_come_in_parts(ops):
+    """For the norm that adds to the residual alone, few outputs, whole pieces of 32 columns on 16-byte boundaries."""
+    def parts(M, N, K, off=0, takes=True):
+        x, w = rnd(M * K + off, seed=1)[off:].view(M, K), rnd(N, K, seed=2)
+        return isinstance(ops.linear(x, w, add_to=ops.AddTo(rnd(M, N, seed=3), rnd(N, seed=4), 1e-6, None, takes_parts=takes)), ops.Parts)
+
+    assert parts(6, 1024, 2048) and parts(16, 2560, 1024) and parts(517, 2048, 512)
+    assert not parts(6, 4096, 2048) and not parts(1500, 2048, 512) and not parts(6, 1024, 500) and not parts(6, 1024, 256)
+    assert not parts(6, 1024, 2048, off=1) and not parts(6, 1024, 2048, takes=False)
+    assert not isinstance(ops.linear(rnd(6, 1024, seed=1), rnd(1024, 1024, seed=2), parts=True), ops.Parts)
+
+
 @pytest.mark.parametrize("M,N,K", [(1, 16, 33), (6, 40, 300), (30, 600, 1024), (70, 4096, 64), (130, 9000, 96)])
 def test_float32_linear_at_the_ends_of_its_range(ops, M, N, K):
     """Infinities, no numbers, numbers that round up to infinity in 8 bits and numbers whose parts are tiny: in their own rows and
