@@ -29,6 +29,7 @@
 #include "nhv_common.h"
 #include "nhv_gemm_fusion.h"
 #include "nhv_lines.h"
+#include <type_traits>
 
 namespace fewrows {
 
@@ -877,17 +878,20 @@ __global__ __launch_bounds__(64 * TW) void gemm_fewrows_walk_kernel(const bf16_t
 
 constexpr size_t LDS_BYTES = 160 * 1024 - 64;      // (64 bytes are the rows' scales, which every kernel keeps beside)
 // How the kernels above are launched; ahead == 0 where they are not the ones to take.
+static int even_rows(int N) { return 4 * ((N + 4 * 256 - 1) / (4 * 256)); }
 struct TilesPlan {
   int ahead;
   bool x_in_lds;
   int rows, height, groups;                                 // rows of w a block and a tile
   size_t lds;
 };
-static TilesPlan tiles_plan(bool glu, bool squares, bool biased, int M, int N, int K) {
+// square_rows: outputs whose squares go out together, which are then a block's (0: no residual).
+static TilesPlan tiles_plan(bool glu, int square_rows, bool biased, int M, int N, int K) {
+  const bool squares = square_rows > 0;
   TilesPlan p = {};
   if (N % 4 || (size_t)N * K * sizeof(bf16_t) >> 32) return p;       // (four outputs a store; places in w are 32 bits)
-  // as many rows a block as give each of the 256 compute units the same (sums of squares go out by tiles of 16)
-  p.rows = squares ? 16 : 4 * ((N + 4 * 256 - 1) / (4 * 256));
+  // as many rows a block as give each of the 256 compute units the same
+  p.rows = squares ? square_rows : even_rows(N);
   const int tiles = (p.rows + 15) / 16;
   p.height = 4 * ((p.rows + 4 * tiles - 1) / (4 * tiles));
   const size_t sums = (size_t)(tiles > 1 ? 2 : 1) * TW * (glu ? 2 : 1) * 64 * sizeof(floatx4), x_bytes = (size_t)M * (K + 8) * 2;
@@ -950,7 +954,10 @@ static int launch_tiles(const TilesPlan& p, hipStream_t s, const void* x, const 
 // 12.1, 12.6; 4,096 of 4,096 10.2, 10.6, 11.8 and 8.4, 8.6, 8.9; gated 12,288 of 4,096 42.8, 43.3, 48.6 and 36.3, 35.9, 36.5 (a kernel that only
 // reads: 32.5); 4,096 of 12,288 23.0, 28.2, 31.0 and 19.7, 20.2, 22.1; 151,936 of 4,096 204, 216, 270 and 196, 198, 201 (201);
 // gated 9,728 of 2,560 25.5, 26.0, 26.3 and 22.5, 22.9, 23.6.
-template <int NT, int NB, bool GATED, typename TOut>
+// SKIPS: up to 8 rows, whose waves without rows of x bring none (in their place the others bring the last one: 2,560 outputs of 4,096 columns at 1 and
+// 4 rows 7.5 and 7.6 us, with it 6.9 and 7.1; 2,560 of 9,728 15.2 and 15.3, 14.0 and 14.7; 3,584 of 18,944 25.9 and 26.1, 24.9 and 25.6). Not for
+// gated products (12,288 of 4,096 at 1 and 8 rows 33.7 and 33.1 us, with it 35.5 and 34.2) nor for float results, whose stretches are summed apart.
+template <int NT, int NB, bool GATED, typename TOut, bool SKIPS>
 __global__ __launch_bounds__(512) void gemm_fewrows_lines_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ w, const bf16_t* __restrict__ bias,
                                                                  TOut* __restrict__ y, int M, int N, int K, const Fusion f) {
   constexpr int OUT = GATED ? 1 : NT, BOTH = GATED ? 2 : 1, CHUNK = 256, LOADS = NT + 1, STAGE = (NT + 1) * 16 * CHUNK;
@@ -991,10 +998,10 @@ __global__ __launch_bounds__(512) void gemm_fewrows_lines_kernel(const bf16_t* _
   constexpr int STRETCHES = sizeof(TOut) == 4 ? 4 : 1;
   const bool stretches = STRETCHES > 1 && K % 2048 == 0;
   const int length = stretches ? chunks / STRETCHES : chunks + 1, place = nhv_first_chunk(blockIdx.x, chunks, K), first = stretches ? place / length * length : place;
-  auto ask = [&](int buf, int c) {
+  auto ask = [&](auto brings_x, int buf, int c) {
     const size_t k = (size_t)nhv_chunk(first, c, chunks) * CHUNK;
 #pragma unroll
-    for (int t = 0; t < LOADS; ++t) {
+    for (int t = 0; t < (decltype(brings_x)::value ? LOADS : NT); ++t) {
       if (t < NT) nhv_load_to_lds<true>(ring_at + (buf * STAGE + t * 16 * CHUNK) * 2, src[t] + k);
       else nhv_load_to_lds<false>(ring_at + (buf * STAGE + t * 16 * CHUNK) * 2, src[t] + k);
     }
@@ -1007,29 +1014,49 @@ __global__ __launch_bounds__(512) void gemm_fewrows_lines_kernel(const bf16_t* _
     for (int i = 0; i < STRETCHES; ++i) done[i][t] = acc[t];
   }
   const int at = r16 * CHUNK + (((wave * 4 + g) ^ r16) << 3);
+  if constexpr (!SKIPS) {
 #pragma unroll
-  for (int i = 0; i < NB - 1; ++i) ask(i, i);
-  int buf = 0, now = first / length, left = length;
-  for (int c = 0; c < chunks; ++c) {
-    nhv_wait_and_meet<(NB - 2) * LOADS>();                            // chunk c is there, chunk c - 1 has been read
-    ask(buf == 0 ? NB - 1 : buf - 1, c + NB - 1);
-    const bf16_t* from = ring + buf * STAGE + at;
-    const bf16x8 b = *reinterpret_cast<const bf16x8*>(from + NT * 16 * CHUNK);
+    for (int i = 0; i < NB - 1; ++i) ask(std::true_type{}, i, i);
+    int buf = 0, now = first / length, left = length;
+    for (int c = 0; c < chunks; ++c) {
+      nhv_wait_and_meet<(NB - 2) * LOADS>();                            // chunk c is there, chunk c - 1 has been read
+      ask(std::true_type{}, buf == 0 ? NB - 1 : buf - 1, c + NB - 1);
+      const bf16_t* from = ring + buf * STAGE + at;
+      const bf16x8 b = *reinterpret_cast<const bf16x8*>(from + NT * 16 * CHUNK);
 #pragma unroll
-    for (int t = 0; t < NT; ++t) acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b, *reinterpret_cast<const bf16x8*>(from + t * 16 * CHUNK), acc[t], 0, 0, 0);
-    buf = buf == NB - 1 ? 0 : buf + 1;
-    if (STRETCHES > 1 && --left == 0) {                               // (the same for the whole block)
+      for (int t = 0; t < NT; ++t) acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b, *reinterpret_cast<const bf16x8*>(from + t * 16 * CHUNK), acc[t], 0, 0, 0);
+      buf = buf == NB - 1 ? 0 : buf + 1;
+      if (STRETCHES > 1 && --left == 0) {                               // (the same for the whole block)
 #pragma unroll
-      for (int i = 0; i < STRETCHES; ++i)
-        if (i == now) {
+        for (int i = 0; i < STRETCHES; ++i)
+          if (i == now) {
 #pragma unroll
-          for (int t = 0; t < NT; ++t) done[i][t] = acc[t];
-        }
+            for (int t = 0; t < NT; ++t) done[i][t] = acc[t];
+          }
 #pragma unroll
-      for (int t = 0; t < NT; ++t) acc[t] = floatx4{0.f, 0.f, 0.f, 0.f};
-      now = now == STRETCHES - 1 ? 0 : now + 1;
-      left = length;
+        for (int t = 0; t < NT; ++t) acc[t] = floatx4{0.f, 0.f, 0.f, 0.f};
+        now = now == STRETCHES - 1 ? 0 : now + 1;
+        left = length;
+      }
     }
+  } else {
+    // a wave whose rows of x are not there brings none (what lies in LDS in their place comes into rows whose results are dropped)
+    auto walk = [&](auto brings_x) {
+#pragma unroll
+      for (int i = 0; i < NB - 1; ++i) ask(brings_x, i, i);
+      int buf = 0;
+      for (int c = 0; c < chunks; ++c) {
+        nhv_wait_and_meet<(NB - 2) * (decltype(brings_x)::value ? LOADS : NT)>();
+        ask(brings_x, buf == 0 ? NB - 1 : buf - 1, c + NB - 1);
+        const bf16_t* from = ring + buf * STAGE + at;
+        const bf16x8 b = *reinterpret_cast<const bf16x8*>(from + NT * 16 * CHUNK);
+#pragma unroll
+        for (int t = 0; t < NT; ++t) acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b, *reinterpret_cast<const bf16x8*>(from + t * 16 * CHUNK), acc[t], 0, 0, 0);
+        buf = buf == NB - 1 ? 0 : buf + 1;
+      }
+    };
+    if (2 * wave < M) walk(std::true_type{});
+    else walk(std::false_type{});
   }
   if (stretches) {
 #pragma unroll
@@ -1076,9 +1103,10 @@ __global__ __launch_bounds__(512) void gemm_fewrows_lines_kernel(const bf16_t* _
 }
 
 // Where the rows of w are enough for it, by what was measured at 1, 4, 8, 12 and 16 rows (us before and with it): not for 4,096 outputs
-// of 1,024 columns (4.2, 4.9 at 1 row) or a gated 3,072 of 1,024 (5.5, 5.7); with fewer than 4,096 outputs a tile of 16 leaves units idle,
-// which the smaller tiles above do not, until there are so many rows that these are slower: 2,560 of 9,728 14.6, 15.1 at 1 row,
-// 15.5, 15.7 at 4, 18.8, 15.8 at 8; 2,048 of 6,144 9.9, 11.1 at 8 and 14.3, 11.5 at 12; 2,048 of 2,048 never.
+// of 1,024 columns (4.2, 4.9 at 1 row) or a gated 3,072 of 1,024 (5.5, 5.7); with fewer than 2,560 outputs a tile of 16 leaves units idle,
+// which the smaller tiles above do not, until there are so many rows that these are slower: 2,560 of 4,096 7.7, 6.9 at 1 row and 7.8, 7.1 at 4;
+// 2,560 of 9,728 14.6, 14.0 and 15.3, 14.7; 3,584 of 3,584 8.5, 7.6 and 8.7, 7.8; 3,072 of 8,192 12.9, 12.0 and 13.6, 12.2; 2,048 of 6,144 8.3, 11
+// at 1 and 9.5, 11.1 at 8, but 14.3, 11.5 at 12; 2,048 of 2,048 never.
 // ``even``: the tiles above would take the product, which give every unit the same rows of w (no residual, whose squares go out by tiles of
 // 16, and no bands). They stay the faster ones where the blocks of 32 outputs are a round and a bit (time by lines over theirs, K = 2,048
 // to 12,288, at 1 to 8 rows: 8,448 outputs 1.07 to 1.18, 9,216 1.07 to 1.17, 10,240 1.00 to 1.11 and at K = 2,048 0.95, 11,264 0.96 to 1.07, 12,288 0.88 to
@@ -1089,13 +1117,13 @@ static bool lines_plan(bool glu, bool even, int M, int N, int K) {
   if (glu) return N >= 4096;
   if (even && N > 8192 && N <= (K > 2048 ? 11264 : 9216) && (long long)M * K <= 57344) return false;
   if (even && N > 4096 && N < 7168 && K % 8192 == 0 && (long long)M * K <= 32768) return false;
-  return N >= 4096 || (N >= 2560 && M >= 8) || (N >= 2048 && K >= 4096 && M >= 12);
+  return N >= 2560 || (N >= 2048 && K >= 4096 && M >= 12);
 }
 
-template <int NT, int NB, bool GATED, typename TOut>
+template <int NT, int NB, bool GATED, typename TOut, bool SKIPS>
 static int launch_lines_as(hipStream_t s, const void* x, const void* w, const void* bias, void* y, int M, int N, int K, const Fusion& f) {
   constexpr int OUT = GATED ? 16 : 16 * NT, ring = NB * (NT + 1) * 16 * 512, sums = NT * 8192, lds = ring > sums ? ring : sums;
-  auto kernel = gemm_fewrows_lines_kernel<NT, NB, GATED, TOut>;
+  auto kernel = gemm_fewrows_lines_kernel<NT, NB, GATED, TOut, SKIPS>;
   // more than 64 KB of dynamic LDS has to be allowed once per kernel (and per process)
   static const hipError_t allowed = hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
   if (allowed != hipSuccess) return nhv_fail("few-rows gemm: %s", hipGetErrorString(allowed));
@@ -1103,14 +1131,22 @@ static int launch_lines_as(hipStream_t s, const void* x, const void* w, const vo
   return 0;
 }
 // One block a compute unit: four chunks in the ring; several: three.
+template <bool GATED, bool SKIPS, typename TOut>
+static int launch_lines_of(hipStream_t s, const void* x, const void* w, const void* bias, void* y, int M, int N, int K, const Fusion& f) {
+  if constexpr (GATED) {
+    return N <= 256 * 16 ? launch_lines_as<2, 4, true, TOut, false>(s, x, w, bias, y, M, N, K, f)
+                         : launch_lines_as<2, 3, true, TOut, false>(s, x, w, bias, y, M, N, K, f);
+  } else {
+    if (N <= 256 * 16) return launch_lines_as<1, 4, false, TOut, SKIPS>(s, x, w, bias, y, M, N, K, f);
+    return N <= 256 * 32 ? launch_lines_as<2, 4, false, TOut, SKIPS>(s, x, w, bias, y, M, N, K, f) : launch_lines_as<2, 3, false, TOut, SKIPS>(s, x, w, bias, y, M, N, K, f);
+  }
+}
 template <bool GATED, typename TOut>
 static int launch_lines(hipStream_t s, const void* x, const void* w, const void* bias, void* y, int M, int N, int K, const Fusion& f) {
-  if constexpr (GATED) {
-    return N <= 256 * 16 ? launch_lines_as<2, 4, true, TOut>(s, x, w, bias, y, M, N, K, f) : launch_lines_as<2, 3, true, TOut>(s, x, w, bias, y, M, N, K, f);
-  } else {
-    if (N <= 256 * 16) return launch_lines_as<1, 4, false, TOut>(s, x, w, bias, y, M, N, K, f);
-    return N <= 256 * 32 ? launch_lines_as<2, 4, false, TOut>(s, x, w, bias, y, M, N, K, f) : launch_lines_as<2, 3, false, TOut>(s, x, w, bias, y, M, N, K, f);
+  if constexpr (!GATED && sizeof(TOut) == 2) {
+    if (M <= 8) return launch_lines_of<false, true, TOut>(s, x, w, bias, y, M, N, K, f);
   }
+  return launch_lines_of<GATED, false, TOut>(s, x, w, bias, y, M, N, K, f);
 }
 
 // The resident kernel's shape: waves, loads in flight and blocks per compute unit, from the best variants measured
@@ -1274,6 +1310,18 @@ static void launch(hipStream_t s, const void* x, const void* w, const void* bias
 
 }  // namespace fewrows
 
+// Outputs whose squares a product that is added to the residual stream best sends out together: those of a block. With tiles of 16 the
+// products of fewer than 4,096 outputs leave units idle, as many as a quarter of the chip has for 1,024 of them. (`aligned`: biases, residual
+// and norm weights on 16-byte boundaries.) us at 1, 4, 8 and 16 rows by 16 and by
+// even blocks: 1,024 of 2,048 4.9, 5.3, 5.5, 5.8 and 4.3, 4.6, 4.7, 5.1; 1,024 of 3,072 5.8, 6.4, 6.6, 7.2 and 4.8, 5.2, 5.6, 6.1; 2,048 of
+// 2,048 5.4, 5.9, 6.0, 6.5 and 5.1, 5.3, 5.6, 6.0; 2,048 of 6,144 11.5, 11.1, 12.0 (10.8 by lines) and 8.5, 9.0, 10.0. The reader then
+// adds up 256 shares a row where it added 64. (Of fewer than 1,024 columns a block is over before that matters.)
+extern "C" int nhv_gemm_fewrows_square_rows(int M, int N, int K, int biased, int aligned) {
+  using namespace fewrows;
+  if (!aligned || K < 1024 || N >= 4096 || even_rows(N) >= 16 || lines_plan(false, false, M, N, K)) return 16;
+  return tiles_plan(false, even_rows(N), biased != 0, M, N, K).ahead ? even_rows(N) : 16;
+}
+
 // The caller has checked sizes, alignment and types (1 <= M <= 16, K a multiple of 8). Returns 0, or 1 with the
 // error message set.
 int nhv_gemm_fewrows_launch(bool glu, const void* x, const void* w, const void* bias, void* y, int M, int N, int K,
@@ -1294,11 +1342,11 @@ int nhv_gemm_fewrows_launch(bool glu, const void* x, const void* w, const void* 
     return 0;
   }
   if (fused && out_dtype != NHV_BF16) return nhv_fail("few-rows gemm: a product that takes over its neighbours' work gives bfloat16");
-  if (lines_plan(glu, f.residual == nullptr, M, N, K) && !(glu && out_dtype != NHV_BF16)) {
+  if (lines_plan(glu, f.residual == nullptr, M, N, K) && !(glu && out_dtype != NHV_BF16) && !(f.residual && f.square_rows != 16)) {
     if (glu) return launch_lines<true, bf16_t>(s, x, w, bias, y, M, N, K, f);
     return out_dtype == NHV_BF16 ? launch_lines<false, bf16_t>(s, x, w, bias, y, M, N, K, f) : launch_lines<false, float>(s, x, w, bias, y, M, N, K, f);
   }
-  const TilesPlan tp = tiles_plan(glu, f.residual != nullptr, bias != nullptr, M, N, K);
+  const TilesPlan tp = tiles_plan(glu, f.residual ? f.square_rows : 0, bias != nullptr, M, N, K);
   const bool on_16 = (((uintptr_t)y | (uintptr_t)bias | (uintptr_t)f.residual | (uintptr_t)f.sum_out | (uintptr_t)f.next_w) & 15) == 0;
 #define NHV_TILES_CASE(AHEAD_, GLU_, XLDS_)                                                                            \
   if (tp.ahead == AHEAD_ && glu == GLU_ && tp.x_in_lds == XLDS_ && on_16)                                             \
@@ -1311,6 +1359,7 @@ int nhv_gemm_fewrows_launch(bool glu, const void* x, const void* w, const void* 
   NHV_TILES_CASE(2, false, false) NHV_TILES_CASE(3, false, false) NHV_TILES_CASE(4, false, false) NHV_TILES_CASE(5, false, false)
   NHV_TILES_CASE(6, false, false)
 #undef NHV_TILES_CASE
+  if (f.residual && f.square_rows != 16) return nhv_fail("few-rows gemm: squares by %d outputs of M=%d N=%d K=%d", f.square_rows, M, N, K);
   const ResidentPlan rp = resident_plan(glu, M, N, K);
 #define NHV_RESIDENT_CASE(WV_, UN_, GLU_, PIECES_)                                                                     \
   if (rp.waves == WV_ && rp.unroll == UN_ && glu == GLU_ && (rp.nchunks > 1) == PIECES_)                              \

@@ -242,10 +242,12 @@ extern "C" int nhv_gemm_fewrows_banded_bf16(const void* x, const void* w, void* 
 // [M, tiles_in] (the tiles' shares of the row's sum of squares over its K entries) and eps; without: r = 1.
 // With residual: the product is not stored; it is added to residual [M, N] (float or bfloat16, rewritten), the sum
 // times next_w [N] (if given), rounded, goes to sum_out [M, N] (bfloat16) and the tiles' shares of its rows' sums of
-// squares to ss_out [M, (N + 15) / 16]; y is then not touched (may be null). Not with glu.
+// squares to ss_out [M, tiles_out], where a tile is 16 outputs, or as many as nhv_gemm_fewrows_square_rows() says; y is then not touched (may
+// be null). Not with glu.
+extern "C" int nhv_gemm_fewrows_square_rows(int M, int N, int K, int biased, int aligned);
 extern "C" int nhv_gemm_fewrows_fused_bf16(const void* x, const void* ss_in, int tiles_in, float eps, const void* w,
                                            const void* bias, void* y, int M, int N, int K, int out_dtype, int glu,
-                                           void* residual, int residual_dtype, void* sum_out, void* ss_out,
+                                           void* residual, int residual_dtype, void* sum_out, void* ss_out, int tiles_out,
                                            const void* next_w, int next_w_dtype, int act, float limit, float alpha,
                                            float offset, void* stream) {
   if (sk_check("fused few-rows gemm", x, w, M, N, K, out_dtype)) return 1;
@@ -268,6 +270,10 @@ extern "C" int nhv_gemm_fewrows_fused_bf16(const void* x, const void* ss_in, int
     f.residual_f32 = residual_dtype == NHV_F32;
     f.sum_out = (bf16_t*)sum_out;
     f.ss_out = (float*)ss_out;
+    const int rows = nhv_gemm_fewrows_square_rows(M, N, K, bias != nullptr, (((uintptr_t)bias | (uintptr_t)residual | (uintptr_t)next_w) & 15) == 0);
+    NHV_REQUIRE(tiles_out == (N + 15) / 16 || tiles_out == (N + rows - 1) / rows, "fused few-rows gemm: squares of %d tiles, not %d or %d", tiles_out,
+                (N + 15) / 16, (N + rows - 1) / rows);
+    f.square_rows = tiles_out == (N + 15) / 16 ? 16 : rows;
     f.next_w = next_w;
     f.next_w_f32 = next_w_dtype == NHV_F32;
   } else {

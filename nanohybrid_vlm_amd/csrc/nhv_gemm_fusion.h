@@ -1,7 +1,7 @@
 // What a few-rows matrix product may take over from the kernels around it (all null: a plain product).
 //
 // After the product: its result is added to the residual stream in the product's own kernel. The kernel reads
-// and rewrites `residual`; every tile of 16 outputs leaves its share of each row's sum of squares in
+// and rewrites `residual`; every tile of `square_rows` outputs leaves its share of each row's sum of squares in
 // `ss_out[row][tile]` (added up in a fixed order by whoever norms the rows); and `sum_out` gets the sum times the
 // weight of the norm that follows (`next_w`, by column), rounded to bfloat16: the norm's product with its weight is
 // done here, its scaling of the rows is left to the reader.
@@ -17,6 +17,7 @@ struct NhvGemmFusion {
   int residual_f32;
   bf16_t* sum_out;       // [M, N]: (residual + product) * next_w, rounded
   float* ss_out;         // [M, tiles of N]
+  int square_rows;       // outputs of a tile: 16, or what nhv_gemm_fewrows_square_rows() says
   const void* next_w;    // [N] float or bfloat16; null: the sum goes out as it is
   int next_w_f32;
   const float* ss_in;    // [M, tiles_in]

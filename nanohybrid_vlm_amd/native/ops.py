@@ -937,7 +937,12 @@ class NativeBackend:
         self._call("nhv_gemm_fewrows_fused_bf16", _ptr(x), _ptr(ss), 0 if ss is None else ss.shape[1], ctypes.c_float(eps),
                    _ptr(w), _ptr(bias), _ptr(out), M, N, K, BF16 if out is None else dtype_code(out), int(gated),
                    _ptr(residual), F32 if residual is None else dtype_code(residual), _ptr(sum_out), _ptr(ss_out),
-                   _ptr(next_w), F32 if next_w is None else dtype_code(next_w), *(gate or Gate()).args(), _stream())
+                   0 if ss_out is None else ss_out.shape[1], _ptr(next_w), F32 if next_w is None else dtype_code(next_w), *(gate or Gate()).args(), _stream())
+
+    def square_tiles(self, x, w, bias, residual, next_w) -> int:
+        """Tiles of a product that is added to the residual stream, each with its share of the rows' sums of squares."""
+        aligned = all(t is None or t.data_ptr() % 16 == 0 for t in (bias, residual, next_w))
+        return -(-w.shape[0] // self.lib.nhv_gemm_fewrows_square_rows(x.shape[0], w.shape[0], w.shape[1], int(bias is not None), int(aligned)))
 
     def scale_rows(self, x, squares, eps, out):
         self._call("nhv_scale_rows", _ptr(x), _ptr(squares), squares.shape[1], ctypes.c_float(eps), _ptr(out), x.shape[0],
@@ -1449,7 +1454,9 @@ def linear(x, w: torch.Tensor, bias: torch.Tensor | None = None, out_dtype=None,
         _dense(add_to.norm_weight, "linear: the next norm's weight", (N,))
         dtype_code(add_to.norm_weight)
         weighted = torch.empty((M, N), dtype=x.dtype, device=x.device)
-        squares = torch.empty((M, (N + 15) // 16), dtype=torch.float32, device=x.device)
+        tiles = getattr(backend(), "square_tiles", None)
+        tiles = (N + 15) // 16 if tiles is None else tiles(x, w, bias, residual, add_to.norm_weight)
+        squares = torch.empty((M, tiles), dtype=torch.float32, device=x.device)
         backend().fused_linear(x, w, bias, None, row_scales=scales, residual=residual, sum_out=weighted, ss_out=squares,
                                next_w=add_to.norm_weight)
         return Summed(weighted, squares, residual, add_to.norm_weight, add_to.eps)

@@ -277,6 +277,42 @@ def test_tiles_of_few_rows_products(ops, M, N, K):
         torch.testing.assert_close(left.double(), tiles, rtol=1e-3, atol=1e-3)
 
 
+@pytest.mark.parametrize("M,N,K,rows", [(1, 1024, 1024, 4), (16, 1024, 3072, 4), (5, 40, 1032, 4), (3, 1028, 1080, 8), (16, 2040, 2048, 8), (9, 2052, 1096, 12),
+                                        (2, 2556, 2056, 12), (7, 3084, 1048, 16), (4, 2560, 2048, 16), (8, 2564, 2304, 16), (1, 1024, 1016, 16)])
+def test_sums_of_squares_by_the_blocks_outputs(ops, M, N, K, rows):
+    """A product that is added to the residual stream leaves its blocks' shares of the rows' sums of squares, of fewer than 16 outputs where these
+    give every unit a block; the norm and the product that read them (bounds: float32 sums of K products of size K^-1/2, one rounding to 8 bits)."""
+    x, w = rnd(M, K, dtype=torch.bfloat16, seed=81), rnd(N, K, dtype=torch.bfloat16, seed=82, scale=K ** -0.5)
+    w2 = rnd(64, N, dtype=torch.bfloat16, seed=85, scale=N ** -0.5) if N % 8 == 0 else None
+    for dtype in DTYPES:
+        residual, next_w = rnd(M, N, dtype=dtype, seed=83), rnd(N, dtype=torch.float32, seed=84, scale=0.1) + 1
+        want = residual.double() + x.double() @ w.double().T
+        summed = ops.linear(x, w, add_to=ops.AddTo(residual, next_w, 1e-6))
+        assert isinstance(summed, ops.Summed) and summed.squares.shape == (M, -(-N // rows))
+        torch.testing.assert_close(residual.double(), want, **(dict(rtol=1e-4, atol=2e-4) if dtype == torch.float32 else tol(dtype)))
+        torch.testing.assert_close(summed.weighted.double(), want * next_w.double(), **tol(torch.bfloat16))
+        tiles = torch.nn.functional.pad(want, (0, -N % rows)).view(M, -1, rows).pow(2).sum(-1)
+        torch.testing.assert_close(summed.squares.double(), tiles, rtol=1e-3, atol=1e-3)
+        scale = torch.rsqrt(want.pow(2).mean(-1, keepdim=True) + 1e-6)
+        torch.testing.assert_close(ops.Normed(summed).tensor().double(), want * next_w.double() * scale, **tol(torch.bfloat16))
+        if w2 is not None:
+            torch.testing.assert_close(ops.linear(ops.Normed(summed), w2).double(), summed.weighted.double() @ w2.double().T * scale, **tol(torch.bfloat16))
+
+
+@pytest.mark.parametrize("M", [1, 2, 3, 7, 8, 9])
+@pytest.mark.parametrize("N,K", [(2560, 2048), (4100, 2304), (9000, 2560)])
+def test_few_rows_by_lines_whose_other_rows_are_not_there(ops, M, N, K):
+    """Up to 8 rows only the waves that have some bring x: against float64, and where more rows take the same tiles, the bits that these give."""
+    x, w = rnd(16, K, dtype=torch.bfloat16, seed=86), rnd(N, K, dtype=torch.bfloat16, seed=87, scale=K ** -0.5)
+    b = ops.backend()
+    rows, more = torch.empty(M, N, dtype=torch.bfloat16, device="cuda"), torch.empty(16, N, dtype=torch.bfloat16, device="cuda")
+    b.fused_linear(x[:M].contiguous(), w, None, rows)
+    b.fused_linear(x, w, None, more)
+    torch.testing.assert_close(rows.double(), x[:M].double() @ w.double().T, **tol(torch.bfloat16))
+    if M < 9 and N == 2560:
+        assert torch.equal(rows, more[:M])
+
+
 @pytest.mark.parametrize("M,I,K", [(1, 112, 80), (5, 1001, 96), (16, 12288, 4096), (17, 160, 96), (64, 300, 1024),
                                    (4, 17408, 136), (16, 25600, 72), (13, 25000, 264), (16, 9000, 5120), (15, 520, 5384)])
 def test_gated_linear(ops, M, I, K):
