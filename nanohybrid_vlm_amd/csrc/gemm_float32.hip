@@ -689,7 +689,7 @@ __device__ __forceinline__ void finish_parts8(const float* __restrict__ parts, i
 }
 
 // residual += the product whose parts these are; y = the norm of the sum: what rmsnorm does with mode 1, bit for bit.
-// 6 rows of 1,024 in 8 parts take 4.8 us in a recorded step, of the finished product 4.6; 517 rows 8.6 and 5.1.
+// 6 rows of 1,024 take 4.5 us in a recorded step, of the finished product 4.6; 517 rows 6.4 and 5.1.
 template <int MAXC>
 __global__ __launch_bounds__(1024) void add_parts_norm_float32_kernel(const float* __restrict__ parts, int count, const float* __restrict__ x,
                                                                       const float* __restrict__ xw, int K, float* __restrict__ residual,

@@ -438,6 +438,88 @@ __global__ __launch_bounds__(256) void split_write_vec_kernel(const T* __restric
   }
 }
 
+// The same where heads are turned by halves, not normed, and every part of a head is whole pieces of eight entries: a block
+// takes one token, and a thread one piece of eight pairs (or, past the rotation, of eight entries) of one of its heads
+// (blockIdx.y over what 512 threads do not cover). A wave to a head spent its time on being launched and on angles: 72,448
+// blocks of one wave, each with a sincosf for every pair of every head, though a token's heads share them. Here they are
+// taken once into LDS while the entries are on their way, and these come and go in 16 bytes. us at 2,264 tokens in bfloat16,
+// before and now: 16 + 8 + 8 heads of 128, all turned, 24.2, 9.7; the first 64 of queries and keys turned 24.2, 11.8 (of
+// 16 query heads alone 16.0, 7.1). A copy of the 37 MB that move takes 6 to 7.
+template <typename T>
+__global__ __launch_bounds__(512) void rotary_split_write_pieces_kernel(
+    const T* __restrict__ qkv, const T* __restrict__ bias, const float* __restrict__ qk_freqs, int qk_half,
+    const float* __restrict__ v_freqs, int v_half, const int* __restrict__ positions, const int* __restrict__ slot_mapping,
+    T* __restrict__ q_out, T* __restrict__ k_cache, T* __restrict__ v_cache, int Hq, int Hkv, int D, int E, int pieces_qk,
+    int pieces_v, int ld, int v_from_k, int heads, const SplitMore more) {
+  extern __shared__ float angles[];            // cos and sin of the token's angles: qk_half each, then v_half each
+  struct alignas(sizeof(T) * 8) Pack { T e[8]; };
+  const int t = blockIdx.x, pos = positions[t];
+  const int turned_heads = min(heads, Hq + Hkv), turned = turned_heads * pieces_qk;
+  const int item = blockIdx.y * blockDim.x + threadIdx.x;
+  const bool of_v = item >= turned;
+  const int rest = of_v ? item - turned : item, pieces = of_v ? pieces_v : pieces_qk;
+  const int g = rest / pieces, i = (rest - g * pieces) * 8;    // head, of the value heads from the first one on
+  const bool is_q = !of_v && g < Hq;
+  int slot = 0;
+  if (!is_q) slot = heads > Hq ? slot_mapping[t] : -1;
+  const bool mine = !(of_v && g >= heads - turned_heads) && slot >= 0;   // (a row without a slot stores nothing: padding)
+  const int half = of_v ? v_half : qk_half;
+  const int col = !of_v ? g * D : v_from_k ? (Hq + g) * D : (Hq + Hkv) * D + g * E;
+  const T* src = qkv + (size_t)t * ld + col;
+  float u[8], v[8];
+  auto values = [&](int at, float* x) {        // as in the kernel above: the sum with the bias is rounded to the rows' type
+    split_load8(src + at, x);
+    if (bias) {
+      float b[8];
+      split_load8(bias + col + at, b);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) x[e] = to_f32(from_f32<T>(x[e] + b[e]));
+    }
+    if (of_v && more.v_first) {
+      float o[8];
+      split_load8(reinterpret_cast<const T*>(more.v_first) + (size_t)t * more.v_first_ld + g * E + at, o);
+      const float lam = *more.v_lam;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) x[e] = (1.0f - lam) * x[e] + lam * o[e];
+    }
+  };
+  if (mine) {                                  // (on their way while the angles are taken)
+    values(i + half, v);
+    if (i < half) values(i, u);
+  }
+  const float p = (float)pos;
+  for (int m = threadIdx.x; m < qk_half + v_half; m += blockDim.x) {
+    const bool other = m >= qk_half;
+    const int n = other ? m - qk_half : m;
+    float sn, cs;
+    sincosf(p * (other ? v_freqs[n] : qk_freqs[n]), &sn, &cs);
+    float* at = angles + (other ? 2 * qk_half : 0);
+    at[n] = cs;
+    at[(other ? v_half : qk_half) + n] = sn;
+  }
+  __syncthreads();
+  if (!mine) return;
+  const float factor = is_q ? query_temperature(pos, more) : 1.0f;
+  T* dst = is_q    ? q_out + ((size_t)t * Hq + g) * D
+           : !of_v ? k_cache + ((size_t)slot * Hkv + (g - Hq)) * D
+                   : v_cache + ((size_t)slot * Hkv + g) * E;
+  Pack out;
+  if (i < half) {
+    const float *cs = angles + (of_v ? 2 * qk_half : 0) + i, *sn = cs + half;
+    Pack first;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      first.e[e] = from_f32<T>((u[e] * cs[e] - v[e] * sn[e]) * factor);
+      out.e[e] = from_f32<T>((v[e] * cs[e] + u[e] * sn[e]) * factor);
+    }
+    *reinterpret_cast<Pack*>(dst + i) = first;
+  } else {
+#pragma unroll
+    for (int e = 0; e < 8; ++e) out.e[e] = from_f32<T>(v[e] * factor);
+  }
+  *reinterpret_cast<Pack*>(dst + i + half) = out;
+}
+
 extern "C" int nhv_rotary_split_write(const void* qkv, const void* bias, const void* qk_freqs, int rot, const void* v_freqs,
                                       const void* positions, const void* slot_mapping, void* q_out, void* k_cache,
                                       void* v_cache, int T, int Hq, int Hkv, int D, int E, int with_kv, int more_columns,
@@ -475,6 +557,28 @@ extern "C" int nhv_rotary_split_write(const void* qkv, const void* bias, const v
       hipLaunchKernelGGL(split_write_vec_kernel<bf16_t>, grid, dim3(256), 0, s, (const bf16_t*)qkv, (const int*)positions,
                          (const int*)slot_mapping, (bf16_t*)q_out, (bf16_t*)k_cache, (bf16_t*)v_cache, nq, nk, nv, ld, T, more);
     NHV_LAUNCH_CHECK("split_write_vec");
+    return 0;
+  }
+  // pieces of eight pairs: the halves and what follows them are whole pieces, at addresses that 8 entries may be read from
+  const int qk_half = rot / 2, v_half = with_kv && v_freqs ? E / 2 : 0;
+  const int pieces_qk = (D - qk_half) / 8, pieces_v = (E - v_half) / 8;
+  const long long items = (long long)(with_kv ? Hq + Hkv : Hq) * pieces_qk + (with_kv ? (long long)Hkv * pieces_v : 0);
+  const size_t angles = 2 * (size_t)(qk_half + v_half) * sizeof(float);
+  if (!unit && !interleaved && maps == 1 && qk_half % 8 == 0 && v_half % 8 == 0 && D % 8 == 0 && E % 8 == 0 && ld % 8 == 0 &&
+      v_first_ld % 8 == 0 && (starts | (uintptr_t)bias) % (8 * item) == 0 && items < 65535 * 512ll && angles <= 64 * 1024 &&
+      (dtype == NHV_F32 || dtype == NHV_BF16)) {
+    const long long per_token = (items + 511) / 512, threads = ((items + per_token - 1) / per_token + 63) / 64 * 64;
+    const dim3 grid((unsigned)T, (unsigned)per_token);
+    hipStream_t s = (hipStream_t)stream;
+#define LAUNCH(TT)                                                                                                       \
+  hipLaunchKernelGGL(rotary_split_write_pieces_kernel<TT>, grid, dim3((unsigned)threads), angles, s, (const TT*)qkv, (const TT*)bias, \
+                     (const float*)qk_freqs, qk_half, (const float*)v_freqs, v_half, (const int*)positions,              \
+                     (const int*)slot_mapping, (TT*)q_out, (TT*)k_cache, (TT*)v_cache, Hq, Hkv, D, E, pieces_qk,         \
+                     pieces_v, ld, v_from_k, heads, more)
+    if (dtype == NHV_F32) LAUNCH(float);
+    else LAUNCH(bf16_t);
+#undef LAUNCH
+    NHV_LAUNCH_CHECK("rotary_split_write_pieces");
     return 0;
   }
   const size_t lds = unit ? (size_t)D * sizeof(float) : 0;
@@ -692,10 +796,60 @@ __global__ void turn_back_kernel(T* __restrict__ x, const float* __restrict__ fr
   }
 }
 
+// The same in pieces of eight pairs (E / 2 a multiple of eight, rows at addresses that 8 entries may be read from): a block
+// takes one token and its angles once, a thread one piece of one head (blockIdx.y over what 512 do not cover). us at 2,264 tokens of 16 heads of 128 in
+// bfloat16: 5.7, by a block of one wave to a head, with a sincosf for every pair, 10.3.
+template <typename T>
+__global__ __launch_bounds__(512) void turn_back_pieces_kernel(T* __restrict__ x, const float* __restrict__ freqs,
+                                                               const int* __restrict__ positions, int H, int E) {
+  extern __shared__ float angles[];            // cos | sin, E / 2 each
+  struct alignas(sizeof(T) * 8) Pack { T e[8]; };
+  const int t = blockIdx.x, half = E / 2, pieces = half / 8;
+  const int item = blockIdx.y * blockDim.x + threadIdx.x, head = item / pieces, i = (item - head * pieces) * 8;
+  T* row = x + ((size_t)t * H + head) * E;
+  float u[8], v[8];
+  if (head < H) {                              // (on their way while the angles are taken)
+    split_load8(row + i, u);
+    split_load8(row + i + half, v);
+  }
+  const float p = (float)positions[t];
+  for (int m = threadIdx.x; m < half; m += blockDim.x) {
+    float sn, cs;
+    sincosf(p * freqs[m], &sn, &cs);
+    angles[m] = cs;
+    angles[half + m] = sn;
+  }
+  __syncthreads();
+  if (head >= H) return;
+  const float *cs = angles + i, *sn = angles + half + i;
+  Pack a, b;
+#pragma unroll
+  for (int e = 0; e < 8; ++e) {
+    a.e[e] = from_f32<T>(u[e] * cs[e] + v[e] * sn[e]);
+    b.e[e] = from_f32<T>(v[e] * cs[e] - u[e] * sn[e]);
+  }
+  *reinterpret_cast<Pack*>(row + i) = a;
+  *reinterpret_cast<Pack*>(row + i + half) = b;
+}
+
 extern "C" int nhv_turn_back(void* x, const void* freqs, const void* positions, int T, int H, int E, int dtype, void* stream) {
   NHV_REQUIRE(T > 0 && H > 0 && E > 0 && E % 2 == 0, "turn_back: bad sizes T=%d H=%d E=%d", T, H, E);
   NHV_REQUIRE((long long)T * H < (1ll << 31), "turn_back: too many tokens");
   hipStream_t s = (hipStream_t)stream;
+  const size_t angles = (size_t)E * sizeof(float), item = dtype == NHV_F32 ? 4 : 2;
+  if (E % 16 == 0 && (uintptr_t)x % (8 * item) == 0 && (long long)H * (E / 16) < 65535 * 512ll && angles <= 64 * 1024 &&
+      (dtype == NHV_F32 || dtype == NHV_BF16)) {
+    const int pieces = H * (E / 16), per_token = (pieces + 511) / 512;
+    const dim3 grid((unsigned)T, (unsigned)per_token), block((unsigned)(((pieces + per_token - 1) / per_token + 63) / 64 * 64));
+    if (dtype == NHV_F32)
+      hipLaunchKernelGGL(turn_back_pieces_kernel<float>, grid, block, angles, s, (float*)x, (const float*)freqs,
+                         (const int*)positions, H, E);
+    else
+      hipLaunchKernelGGL(turn_back_pieces_kernel<bf16_t>, grid, block, angles, s, (bf16_t*)x, (const float*)freqs,
+                         (const int*)positions, H, E);
+    NHV_LAUNCH_CHECK("turn_back_pieces");
+    return 0;
+  }
   if (dtype == NHV_F32)
     hipLaunchKernelGGL(turn_back_kernel<float>, dim3((unsigned)((size_t)T * H)), dim3(NHV_WAVE), 0, s, (float*)x,
                        (const float*)freqs, (const int*)positions, H, E);

@@ -1777,3 +1777,50 @@ def test_delta_rule_lets_no_token_reach_the_ones_before_it(ops, D, E, per_head):
         assert torch.equal(out[:t], clean[:t]), (t, column)
         assert torch.equal(out[:, E:], clean[:, E:]) and torch.equal(left[1], state[1]), (t, column)
         assert not torch.isfinite(out[t, :E]).all(), (t, column)
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("T,Hq,Hkv,D,E,rot,of_values,more", [(1, 1, 1, 16, 8, 16, None, ()), (70, 5, 2, 24, 40, 16, None, ("bias",)),
+                                                             (3, 16, 8, 128, 128, 128, "turned", ()),
+                                                             (37, 33, 11, 128, 64, 48, "mixed", ("temperature",)),
+                                                             (9, 6, 3, 64, 64, 64, "keys", ("bias", "columns")),
+                                                             (5, 7, 3, 32, 16, 0, "turned", ("bias",)),
+                                                             (40, 12, 4, 80, 48, 80, "none", ("columns",))])
+def test_heads_turned_in_pieces_of_eight_pairs(ops, dtype, T, Hq, Hkv, D, E, rot, of_values, more):
+    """Against the kernel of one wave to a head, which takes the same rows where they start one entry off a piece: the same
+    expressions of the same angles, whose products a compiler may contract one way or the other (half a float's last place,
+    which can become one of bfloat16's). Rows without a slot store nothing; so the caches keep what they held."""
+    kv = of_values != "none"
+    width = Hq * D + (Hkv * D + (0 if of_values == "keys" else Hkv * E) if kv else 0) + (8 if "columns" in more else 0)
+    bias = rnd(width - (8 if "columns" in more else 0), dtype=dtype, seed=91) if "bias" in more else None
+    rows = rnd(T * width, dtype=dtype, seed=92)
+    off = torch.cat((rows[:1], rows))[1:].view(T, width)
+    rows = rows.view(T, width)
+    assert rows.data_ptr() % 16 == 0 and off.data_ptr() % 16 != 0
+    freqs = None if rot == 0 else torch.rand(rot // 2, device="cuda")
+    v_freqs = torch.rand(E // 2, device="cuda") if of_values == "turned" else None
+    positions = torch.randint(0, 20000, (T,), dtype=torch.int32, device="cuda")
+    slots = torch.randperm(T + 3, device="cuda")[:T].int()
+    slots[T // 2 + 1:T // 2 + 3] = -1
+    options = {"temperature": (0.1, 100.0)} if "temperature" in more else {}
+    if of_values == "mixed":
+        options["mix"] = ((rnd(T, Hkv * E + 16, dtype=dtype, seed=93), 8), torch.tensor([0.3], device="cuda"))
+    got = []
+    for x in (rows, off):
+        k_cache, v_cache = (torch.full((T + 3, 1, Hkv, n), 7.0, dtype=dtype, device="cuda") for n in (D, E))
+        q = ops.rotary_split_write(x, bias, freqs, v_freqs, positions, slots if kv else None, k_cache if kv else None,
+                                   v_cache if kv else None, Hq, Hkv, D, E, with_kv=kv,
+                                   more_columns=8 if "columns" in more else 0, values_from_keys=of_values == "keys", **options)
+        got.append((q, k_cache, v_cache))
+    for a, b in zip(*got):
+        torch.testing.assert_close(a, b, rtol=2.0 ** -7 if dtype == torch.bfloat16 else 0.0, atol=2.0 ** -20)
+    if kv and T > 1:
+        empty = torch.ones(T + 3, dtype=torch.bool, device="cuda")
+        empty[slots[slots >= 0].long()] = False
+        assert (got[0][1][empty] == 7).all() and (got[0][2][empty] == 7).all() and empty.sum() >= 4
+    if E % 16 == 0:
+        o = rnd(T * Hq * E, dtype=dtype, seed=94)
+        o_off = torch.cat((o[:1], o))[1:].view(T, Hq, E)
+        f = torch.rand(E // 2, device="cuda")
+        a, b = ops.turn_back_(o.view(T, Hq, E), f, positions), ops.turn_back_(o_off, f, positions)
+        torch.testing.assert_close(a, b, rtol=2.0 ** -7 if dtype == torch.bfloat16 else 0.0, atol=2.0 ** -20)
