@@ -12,10 +12,17 @@
 // second product's right operand (O^T = V^T P^T), so the weights never leave their registers; neither do the sums: the waves
 // meet in LDS once, at the end (before, after every eight blocks of keys, with a barrier on either side). What bounds it: a
 // wave's blocks are 128 matrix instructions of 32 clocks each and two waves share a SIMD; registers allow one block a compute
-// unit. 16 heads on 8 key heads of 128, us, before and now: a prompt of 517 tokens 54.6, 41.1; 500 tokens after 1,500 179, 117;
-// six tokens after 100 9.1, 8.4; one after 300 18.1, 14.6; eight after 3,000 132, 89. Not faster: a block's keys all asked for
-// at once and the next block's before the values are worked on (44.8, 119, 8.9, 16.4, 89), four waves a block (39.2, 114, 8.6,
-// 16.8, 130).
+// unit. 16 heads on 8 key heads of 128, us, before and now: a prompt of 517 tokens 54.6, 41.6; 500 tokens after 1,500 179, 122.
+// Not faster there: a block's keys all asked for at once and the next block's before the values are worked on (44.8, 119), four
+// waves a block (39.2, 114).
+//
+// AT_ONCE, where a request's rows are one tile (a decoded token, a portion of up to 16 rows) and heads are 64 or 128 entries for
+// keys and values: what a few blocks of keys take is the way to them, four trips to memory for a wave's 32 keys after three
+// for the positions and the table. So a block is asked for as a whole, keys and values, the first one while the
+// queries are on their way and, where keys begin with the request's, at a place looked up before the positions are known; the
+// next one's keys follow this one's scores. The sums and their order are the same, so are the bits. us where keys come from
+// memory, the other order first: six tokens after 100 10.5, 8.5; one after 300 16.1, 15.0; eight after 3,000 112, 90; 64 after
+// 500 59, 54; two after 200, 32 heads of 64 on 2, 9.0, 8.1. Where they lie in the L2: 8.1, 7.6; 14.4, 14.5; 90, 78.
 #include "nhv_common.h"
 #include <math.h>
 
@@ -42,19 +49,30 @@ struct FloatAttention {
   long long gate_ld;
 };
 
-template <int CHUNKS>                                    // of 64 value entries
+template <int CHUNKS, bool AT_ONCE>                      // of 64 value entries
 __global__ __launch_bounds__(64 * WAVES) void attention_float32_kernel(FloatAttention a) {
   extern __shared__ __attribute__((aligned(16))) float shared[];
-  constexpr int E = 64 * CHUNKS;
-  const int D = a.D, group = a.Hq / a.Hkv;
+  constexpr int E = 64 * CHUNKS, UNITS = AT_ONCE ? E / 16 : 4;   // (blocks of 16 key entries that have registers)
+  const int D = AT_ONCE ? E : a.D, group = a.Hq / a.Hkv;
   float* qs = shared;                                    // [ROWS][D + 4]
   float* part = qs + ROWS * (D + 4);                     // [WAVES][ROWS][E + 4]
   float* stats = part + WAVES * ROWS * (E + 4);          // [WAVES][ROWS][2]: maximum and sum
   const int kvh = blockIdx.y, req = blockIdx.z;
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, r16 = lane & 15, g = lane >> 4;
+  const int* table = a.block_tables + (size_t)req * a.max_blocks;
+  // where this lane's key of the wave's first block lies if the keys that are read begin with the request's
+  int page = 0;
+  if constexpr (AT_ONCE) page = table[min((wave * KEYS + lane % KEYS) / a.page_size, a.max_blocks - 1)];
   const int first = a.cu[req], rows = (a.cu[req + 1] - first) * group;
   const int row0 = (gridDim.x - 1 - blockIdx.x) * ROWS;  // (the tiles with the longest chains of keys first)
   if (row0 >= rows) return;                              // (the same for the whole block)
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, r16 = lane & 15, g = lane >> 4;
+
+  f32x4 mine_q = {0.f, 0.f, 0.f, 0.f};                   // (AT_ONCE: what this thread brings of the queries)
+  const int q_row = (int)threadIdx.x * 4 / D, q_at = (int)threadIdx.x * 4 % D;
+  auto query = [&](int r, int d) {
+    return *reinterpret_cast<const f32x4*>(a.q + ((size_t)(first + (row0 + r) / group) * a.Hq + kvh * group + (row0 + r) % group) * D + d);
+  };
+  if (AT_ONCE && q_row < ROWS && row0 + q_row < rows) mine_q = query(q_row, q_at);
 
   // this lane's row: what it may read
   const int row = row0 + r16;
@@ -69,14 +87,48 @@ __global__ __launch_bounds__(64 * WAVES) void attention_float32_kernel(FloatAtte
     tile_hi = max(tile_hi, __shfl_xor(tile_hi, o, NHV_WAVE));
   }
   const float slope = a.slopes && live ? a.slopes[head] : 0.f;
-  const int* table = a.block_tables + (size_t)req * a.max_blocks;
 
-  for (int i = threadIdx.x * 4; i < ROWS * D; i += 64 * WAVES * 4) {
-    const int r = i / D, d = i % D;
-    f32x4 v = {0.f, 0.f, 0.f, 0.f};
-    if (row0 + r < rows)
-      v = *reinterpret_cast<const f32x4*>(a.q + ((size_t)(first + (row0 + r) / group) * a.Hq + kvh * group + (row0 + r) % group) * D + d);
-    *reinterpret_cast<f32x4*>(&qs[r * (D + 4) + d]) = v;
+  // lane l's own key of a block from kb on, and where it lies. A key that no row reads is taken for the tile's last: its score
+  // is masked, and every load is without a condition (with one the compiler waits for all that are under way).
+  auto slot_in = [&](int kb) {
+    const int mine = kb + lane % KEYS, own = mine >= tile_lo && mine <= tile_hi ? mine : tile_hi;
+    return table[own / a.page_size] * a.page_size + own % a.page_size;
+  };
+  // (the first block of this wave's from the tile's first key on)
+  const int from = (tile_lo / KEYS + ((wave - tile_lo / KEYS) & (WAVES - 1))) * KEYS;
+  int slot = 0;
+  f32x4 kf[UNITS][TILES];
+  const float* kr[TILES];
+  auto keys_at = [&]() {
+#pragma unroll
+    for (int t = 0; t < TILES; ++t) kr[t] = a.k + ((size_t)__shfl(slot, 16 * t + r16, NHV_WAVE) * a.Hkv + kvh) * D + 4 * g;
+  };
+  auto ask = [&](int unit, int d) {                      // (the last 16 entries again where there are no more)
+#pragma unroll
+    for (int t = 0; t < TILES; ++t) kf[unit][t] = *reinterpret_cast<const f32x4*>(kr[t] + (AT_ONCE ? d : min(d, D - 16)));
+  };
+  if constexpr (AT_ONCE) {
+    if (from <= tile_hi) {
+      if (tile_lo == 0) {
+        // (a key that no row reads is taken for the block's first here, whose page is known too)
+        const int mine = from + lane % KEYS, own = mine <= tile_hi ? mine : from;
+        const int first_page = __shfl(page, 0, NHV_WAVE);
+        slot = (mine <= tile_hi ? page : first_page) * a.page_size + own % a.page_size;
+      } else {
+        slot = slot_in(from);
+      }
+      keys_at();
+#pragma unroll
+      for (int u = 0; u < UNITS; ++u) ask(u, 16 * u);
+    }
+    if (q_row < ROWS) *reinterpret_cast<f32x4*>(&qs[q_row * (D + 4) + q_at]) = mine_q;
+  } else {
+    for (int i = threadIdx.x * 4; i < ROWS * D; i += 64 * WAVES * 4) {
+      const int r = i / D, d = i % D;
+      f32x4 v = {0.f, 0.f, 0.f, 0.f};
+      if (row0 + r < rows) v = query(r, d);
+      *reinterpret_cast<f32x4*>(&qs[r * (D + 4) + d]) = v;
+    }
   }
 
   // of row r16: the maximum, this lane's share of the sum (lanes r16, 16 + r16, ... together have all) and values so far
@@ -87,55 +139,72 @@ __global__ __launch_bounds__(64 * WAVES) void attention_float32_kernel(FloatAtte
 #pragma unroll
     for (int j = 0; j < 4; ++j) o[h][j] = f32x4{0.f, 0.f, 0.f, 0.f};
   __syncthreads();                                       // (the queries are in LDS)
-  // (the first block of this wave's from the tile's first key on)
-  const int from = (tile_lo / KEYS + ((wave - tile_lo / KEYS) & (WAVES - 1))) * KEYS;
   for (int kb = from; kb <= tile_hi; kb += KEYS * WAVES) {
-    // lane l's own key of the block, and where it lies. A key that no row reads is taken for the tile's last: its score is
-    // masked, and every load is without a condition (with one the compiler waits for all that are under way).
-    const int mine = kb + lane % KEYS, own = mine >= tile_lo && mine <= tile_hi ? mine : tile_hi;
-    const int slot = table[own / a.page_size] * a.page_size + own % a.page_size;
-    f32x4 s[TILES], kf[2][2][TILES], vf[TILES][4];
-    const float *kr[TILES], *vr[TILES][4];
+    const int next = kb + KEYS * WAVES;
+    int next_slot = 0;
+    if constexpr (!AT_ONCE) {
+      slot = slot_in(kb);
+      keys_at();
+    }
+    f32x4 s[TILES], vf[AT_ONCE ? CHUNKS : 1][TILES][4];
+    const float* vr[TILES][4];
 #pragma unroll
     for (int t = 0; t < TILES; ++t) {
-      kr[t] = a.k + ((size_t)__shfl(slot, 16 * t + r16, NHV_WAVE) * a.Hkv + kvh) * D + 4 * g;
 #pragma unroll
       for (int i = 0; i < 4; ++i) vr[t][i] = a.v + ((size_t)__shfl(slot, 16 * t + 4 * g + i, NHV_WAVE) * a.Hkv + kvh) * E + 4 * r16;
       s[t] = f32x4{0.f, 0.f, 0.f, 0.f};
     }
-    // keys two blocks of 16 entries ahead (the last one again where there are no two); the first 64 value entries at once
-    auto ask = [&](int buf, int d) {
+    auto values = [&](int h) {
 #pragma unroll
-      for (int u = 0; u < 2; ++u)
+      for (int t = 0; t < TILES; ++t)
 #pragma unroll
-        for (int t = 0; t < TILES; ++t) kf[buf][u][t] = *reinterpret_cast<const f32x4*>(kr[t] + min(d + 16 * u, D - 16));
+        for (int i = 0; i < 4; ++i) vf[AT_ONCE ? h : 0][t][i] = *reinterpret_cast<const f32x4*>(vr[t][i] + 64 * h);
     };
-    auto score = [&](int buf, int d, int u) {
-      const f32x4 qf = *reinterpret_cast<const f32x4*>(&qs[r16 * (D + 4) + d + 16 * u + 4 * g]);
+    auto score = [&](int unit, int d) {
+      const f32x4 qf = *reinterpret_cast<const f32x4*>(&qs[r16 * (D + 4) + d + 4 * g]);
 #pragma unroll
       for (int j = 0; j < 4; ++j)
 #pragma unroll
-        for (int t = 0; t < TILES; ++t) s[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[buf][u][t][j], qf[j], s[t], 0, 0, 0);
+        for (int t = 0; t < TILES; ++t) s[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[unit][t][j], qf[j], s[t], 0, 0, 0);
     };
-    ask(0, 0);
+    const int held = slot;                               // (where this block's keys lie)
+    if constexpr (AT_ONCE) {
+      // all of the block is under way before the first product; the next block's keys follow behind this one's scores
+      next_slot = slot_in(next);                         // (before the values: it is waited for with the keys)
+      __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-    for (int t = 0; t < TILES; ++t)
+      for (int h = 0; h < CHUNKS; ++h) values(h);
 #pragma unroll
-      for (int i = 0; i < 4; ++i) vf[t][i] = *reinterpret_cast<const f32x4*>(vr[t][i]);
-    int d = 0;
-    for (; d + 64 <= D; d += 64) {
-      ask(1, d + 32);
-      score(0, d, 0);
-      score(0, d, 1);
-      ask(0, d + 64);
-      score(1, d + 32, 0);
-      score(1, d + 32, 1);
-    }
-    if (d < D) {                                       // 16, 32 or 48 entries more
-      ask(1, d + 32);
-      score(0, d, 0);
-      if (d + 16 < D) score(0, d, 1);
-      if (d + 32 < D) score(1, d + 32, 0);
+      for (int u = 0; u < UNITS; ++u) score(u, 16 * u);
+      if (next <= tile_hi) {
+        slot = next_slot;
+        keys_at();
+#pragma unroll
+        for (int u = 0; u < UNITS; ++u) ask(u, 16 * u);
+      }
+    } else {
+      // keys two blocks of 16 entries ahead; the first 64 value entries at once
+      ask(0, 0);
+      ask(1, 16);
+      values(0);
+      int d = 0;
+      for (; d + 64 <= D; d += 64) {
+        ask(2, d + 32);
+        ask(3, d + 48);
+        score(0, d);
+        score(1, d + 16);
+        ask(0, d + 64);
+        ask(1, d + 80);
+        score(2, d + 32);
+        score(3, d + 48);
+      }
+      if (d < D) {                                       // 16, 32 or 48 entries more
+        ask(2, d + 32);
+        ask(3, d + 48);
+        score(0, d);
+        if (d + 16 < D) score(1, d + 16);
+        if (d + 32 < D) score(2, d + 32);
+      }
     }
     // s[t][i]: key kb + 16 t + 4 g + i against row r16
     float m = -INFINITY;
@@ -178,10 +247,10 @@ __global__ __launch_bounds__(64 * WAVES) void attention_float32_kernel(FloatAtte
         for (int i = 0; i < 4; ++i) {
 #pragma unroll
           for (int j = 0; j < 4; ++j) {
-            odd = fmaf(vf[t][i][j], 0.f, odd);
-            now[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(vf[t][i][j], s[t][i], now[j], 0, 0, 0);
+            odd = fmaf(vf[AT_ONCE ? h : 0][t][i][j], 0.f, odd);
+            now[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(vf[AT_ONCE ? h : 0][t][i][j], s[t][i], now[j], 0, 0, 0);
           }
-          if (h + 1 < CHUNKS) vf[t][i] = *reinterpret_cast<const f32x4*>(vr[t][i] + 64 * (h + 1));
+          if (!AT_ONCE && h + 1 < CHUNKS) vf[0][t][i] = *reinterpret_cast<const f32x4*>(vr[t][i] + 64 * (h + 1));
         }
       // now[j][i]: row r16, entry 64 h + 16 g + 4 i + j
       if (__any(odd != 0.f)) {
@@ -193,7 +262,7 @@ __global__ __launch_bounds__(64 * WAVES) void attention_float32_kernel(FloatAtte
 #pragma unroll
           for (int i = 0; i < 4; ++i)
             for (int gk = 0; gk < 4; ++gk) {
-              const int at = __shfl(slot, 16 * t + 4 * gk + i, NHV_WAVE);
+              const int at = __shfl(held, 16 * t + 4 * gk + i, NHV_WAVE);
               const float p = __shfl(s[t][i], 16 * gk + r16, NHV_WAVE);
               if (p != 0.f) {
                 const float* row_v = a.v + ((size_t)at * a.Hkv + kvh) * E + 64 * h + 16 * g;
@@ -260,12 +329,12 @@ __global__ __launch_bounds__(64 * WAVES) void attention_float32_kernel(FloatAtte
   for (int i = 0; i < 2 * CHUNKS; ++i) out[c + 32 * i] = total[i] * inv;
 }
 
-template <int CHUNKS>
+template <int CHUNKS, bool AT_ONCE = false>
 static int launch(const FloatAttention& a, dim3 grid, size_t lds, hipStream_t s) {
-  static const hipError_t allowed = hipFuncSetAttribute((const void*)attention_float32_kernel<CHUNKS>, hipFuncAttributeMaxDynamicSharedMemorySize,
+  static const hipError_t allowed = hipFuncSetAttribute((const void*)attention_float32_kernel<CHUNKS, AT_ONCE>, hipFuncAttributeMaxDynamicSharedMemorySize,
                                                         (int)((ROWS * (MAX_D + 4) + WAVES * ROWS * (64 * CHUNKS + 4) + WAVES * ROWS * 2) * sizeof(float)));
   if (allowed != hipSuccess) return nhv_fail("attention: %zu bytes of LDS are refused: %s", lds, hipGetErrorString(allowed));
-  hipLaunchKernelGGL(attention_float32_kernel<CHUNKS>, grid, dim3(64 * WAVES), lds, s, a);
+  hipLaunchKernelGGL((attention_float32_kernel<CHUNKS, AT_ONCE>), grid, dim3(64 * WAVES), lds, s, a);
   NHV_LAUNCH_CHECK("attention_float32");
   return 0;
 }
@@ -287,6 +356,9 @@ extern "C" int nhv_attention_float32(const void* q, const void* k_cache, const v
                             (const int*)cu_seqlens_q, (const int*)block_tables, max_blocks, Hq, Hkv, D, E, page_size, scale, window, chunk,
                             cap, has_sink, sink, (const float*)sinks, (const float*)slopes, (const float*)gate, gate_ld};
   const size_t lds = (ROWS * (D + 4) + WAVES * ROWS * (E + 4) + WAVES * ROWS * 2) * sizeof(float);
+  // (sizes whose registers and addresses are known when this is compiled: with any D up to 128 two tokens of 64 after 200 took 9.9)
+  if (tiles == 1 && D == E && E == 64) return launch<1, true>(a, dim3(1, Hkv, B), lds, (hipStream_t)stream);
+  if (tiles == 1 && D == E && E == 128) return launch<2, true>(a, dim3(1, Hkv, B), lds, (hipStream_t)stream);
   switch (E / 64) {
     case 1: return launch<1>(a, dim3((unsigned)tiles, Hkv, B), lds, (hipStream_t)stream);
     case 2: return launch<2>(a, dim3((unsigned)tiles, Hkv, B), lds, (hipStream_t)stream);

@@ -784,6 +784,31 @@ def test_attention_hides_no_score_that_is_no_number(ops, dtype, D, sink):
     assert torch.isnan(out[hit]).all() and torch.equal(out[~hit], clean[~hit])
 
 
+@pytest.mark.parametrize("Hq,Hkv,D,page,reach", [(16, 8, 128, 16, {}), (16, 8, 128, 256, {"window": 70}), (4, 4, 64, 7, {}),
+                                                 (16, 1, 64, 5, {"chunk": 50}), (6, 2, 128, 8, {"window": 33, "softcap": 3.0})])
+def test_float32_attention_of_one_tile_of_rows(ops, Hq, Hkv, D, page, reach):
+    """Where 16 rows hold a request's portion, a block of keys is asked for at once, the first one before it is known which of its
+    keys are read: the bits of the same tokens among longer portions, also beside keys and values that are no numbers and pages
+    that no request holds (-1 in the table)."""
+    import dataclasses
+    lens = [1, 31, 32, 33, 64, 255, 256, 257, 300, 530, 40]
+    q_lens = [1, 1, 2, 1, 1, 1, 1, 1, 1, 1, 40]
+    q, kc, vc, batch, bt, *_ = _paged_setup(torch.float32, lens, q_lens, Hq, Hkv, D, page, seed=95)
+    vc[bt[8, 3 // page], 3 % page, 0, 1] = float("inf")
+    vc[bt[9, 500 // page], 500 % page, Hkv - 1, 2] = float("nan")
+    kc[bt[7, 256 // page], 256 % page, 0, 3] = float("nan")
+    together = ops.paged_attention(q, kc, vc, batch, bt, D ** -0.5, **reach)
+    n = len(lens) - 1
+    few = dataclasses.replace(batch, num_tokens=n + 1, num_requests=n, token_req=batch.token_req[:n + 1], positions=batch.positions[:n + 1],
+                              cu_seqlens_q=batch.cu_seqlens_q[:n + 1], context_lens=batch.context_lens[:n], max_q_len=2, max_context_len=530)
+    if 2 * (Hq // Hkv) > 16:                   # (only single tokens are one tile)
+        few = dataclasses.replace(few, num_tokens=2, num_requests=2, token_req=batch.token_req[:2], positions=batch.positions[:2],
+                                  cu_seqlens_q=batch.cu_seqlens_q[:3], context_lens=batch.context_lens[:2], max_q_len=1, max_context_len=31)
+        n = 1
+    alone = ops.paged_attention(q[:few.num_tokens].contiguous(), kc, vc, few, bt[:few.num_requests].contiguous(), D ** -0.5, **reach)
+    assert torch.equal(alone.view(torch.int32), together[:few.num_tokens].view(torch.int32))
+
+
 def test_float32_attention_of_rows_that_begin_anywhere(ops):
     """Queries that begin 4, 8 and 12 bytes off a boundary of 16: the bits of those that begin on one."""
     lens, q_lens = [33, 257, 70], [33, 1, 20]
