@@ -25,6 +25,7 @@
 // without values would) and a gate per (token, head) whose sigmoid multiplies the head's result (in the merge, with the
 // division by the sum).
 #include "nhv_common.h"
+#include "nhv_head_pieces.h"
 #include "nhv_no_alloc.h"
 #include <math.h>
 #include <mutex>
@@ -86,13 +87,31 @@ struct Finish {                                             // what follows the 
   long long gate_ld;
 };
 
-template <bool CAPPED, bool BIASED>
+// ROTATED: the queries and the token's own key and value come as their projection left them, and a block norms and turns what
+// it needs of them itself while its first keys and values are on their way: its query heads (again in every split), and in the
+// split with the token's position also the key and the value, which it stores and takes from LDS in place of what it read. One token
+// after 150 keys at the 0.6B shape: 3.1 us of a launch for it and 7.6 for the attention, 28 times a step of 942; 907 with this.
+struct Rotated {
+  const void* qkv;                                          // [tokens, (Hq + 2 Hkv) D], or that many float parts of it
+  int splits;
+  size_t part_stride;
+  const bf16_t* bias;
+  const void *q_norm, *k_norm;
+  int float_norms;
+  float eps;
+  const float* cos_sin;                                     // null: nothing is turned
+  const int *positions, *slots;
+};
+constexpr bool CAN_ROTATE = D >= 32 && D <= 128 && (D & (D - 1)) == 0;
+static_assert(!CAN_ROTATE || (18 * CHUNKS <= 64 * WAVES && 16 * (D + 8) * 2 <= TILE && 2 * CHUNKS <= D), "a block's threads and tiles hold 16 queries, a key and a value");
+
+template <bool CAPPED, bool BIASED, bool ROTATED = false>
 __global__ __launch_bounds__(64 * WAVES) void decode_attention_kernel(
     const bf16_t* __restrict__ q, const bf16_t* __restrict__ k_cache, const bf16_t* __restrict__ v_cache,
     float* __restrict__ part_o, float* __restrict__ part_ml, bf16_t* __restrict__ out, const int* __restrict__ token_req,
     const int* __restrict__ positions, const int* __restrict__ block_tables, int max_blocks, int Hq, int Hkv,
     int page_size, int page_shift, float scale_log2e, int window, int split_len, int n_splits, float cap_l2, float tanh_k,
-    const float* __restrict__ slopes, const Finish finish) {
+    const float* __restrict__ slopes, const Finish finish, const Rotated rotated) {
   __shared__ __attribute__((aligned(16))) char tiles_s[WAVES][TILE];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   bf16_t* vt_s = reinterpret_cast<bf16_t*>(tiles_s[wave]);
@@ -158,10 +177,12 @@ __global__ __launch_bounds__(64 * WAVES) void decode_attention_kernel(
 
   // Q^T operand: lane holds 8 entries of head `col`
   bf16x8 qb[DSTEPS];
+  if constexpr (!ROTATED) {
 #pragma unroll
-  for (int s = 0; s < DSTEPS; ++s) {
-    const int d = s * 32 + grp * 8;
-    qb[s] = (col < G && d < D) ? load8(q + ((size_t)t * Hq + head0 + col) * D + d) : zero8();
+    for (int s = 0; s < DSTEPS; ++s) {
+      const int d = s * 32 + grp * 8;
+      qb[s] = (col < G && d < D) ? load8(q + ((size_t)t * Hq + head0 + col) * D + d) : zero8();
+    }
   }
 
   const float slope_l2 = BIASED && col < G ? slopes[head0 + col] * 1.4426950408889634f : 0.f;
@@ -306,9 +327,73 @@ __global__ __launch_bounds__(64 * WAVES) void decode_attention_kernel(
       }
     }
   };
-  for (int turn = first / RK * RK + wave * RK * TURN; turn <= last; turn += RK * TURN * WAVES)
+  const int start = first / RK * RK + wave * RK * TURN;
+  const int holder = (pos / RK - first / RK) / TURN % WAVES;   // the wave whose rounds hold the token's own key
+  bool own = false;                                       // (what is read at the token's position is what it stores)
+  if constexpr (ROTATED) {
+    if (start <= last) ask(start);
+    const int slot = last == pos ? rotated.slots[t] : -1;
+    own = slot >= 0 && slot == slot_of(bt, pos, page_size, page_shift);
+    bf16_t* const q_s = reinterpret_cast<bf16_t*>(tiles_s[(holder + 1) % WAVES]);
+    const int item = threadIdx.x / CHUNKS, c = threadIdx.x % CHUNKS;
+    if (item < G + (slot >= 0 ? 2 : 0)) {                  // (the lanes of a head together)
+      const bool is_q = item < G, is_v = item == G + 1;
+      const int h = is_q ? head0 + item : Hq + (is_v ? Hkv : 0) + kvh;
+      const size_t at = ((size_t)t * (Hq + 2 * Hkv) + h) * D + c * 8;
+      float v[8], y[8], cs[8], sn[8];
+      if (rotated.splits) add_parts8((const float*)rotated.qkv + at, rotated.part_stride, rotated.splits, v);
+      else load8f<bf16_t>((const bf16_t*)rotated.qkv + at, v);
+      const bool turns = rotated.cos_sin != nullptr;
+      if (turns) {
+        const float* row = rotated.cos_sin + (size_t)rotated.positions[t] * D + c % (CHUNKS / 2) * 8;
+        load8f<float>(row, cs);
+        load8f<float>(row + D / 2, sn);
+      }
+      if (rotated.bias) {
+        float b[8];
+        load8f<bf16_t>(rotated.bias + (size_t)h * D + c * 8, b);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) v[e] = to_f32(from_f32<bf16_t>(v[e] + b[e]));
+      }
+      const void* norm = is_q ? rotated.q_norm : rotated.k_norm;
+      if (is_v) {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) y[e] = v[e];
+      } else if (rotated.float_norms) {
+        normed_and_turned<bf16_t, float, CHUNKS>(v, (const float*)norm, rotated.eps, turns, cs, sn, c, y);
+      } else {
+        normed_and_turned<bf16_t, bf16_t, CHUNKS>(v, (const bf16_t*)norm, rotated.eps, turns, cs, sn, c, y);
+      }
+      if (is_q) {
+        store8f<bf16_t>(q_s + item * (D + 8) + c * 8, y);
+      } else {
+        // (where the rows of the holder's tile have no columns of values: nothing else is written there before the waves meet)
+        store8f<bf16_t>(reinterpret_cast<bf16_t*>(tiles_s[holder]) + ((is_v ? CHUNKS : 0) + c) * VPITCH + RK, y);
+        // (through the pointer that the loads go by, so that the two are known to meet)
+        if (group % per_kv == 0) store8f<bf16_t>(const_cast<bf16_t*>(is_v ? v_cache : k_cache) + ((size_t)slot * Hkv + kvh) * D + c * 8, y);
+      }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int s = 0; s < DSTEPS; ++s) qb[s] = col < G ? load8(q_s + col * (D + 8) + s * 32 + grp * 8) : zero8();
+    __syncthreads();                                      // (the tile is its wave's again)
+  }
+  for (int turn = start; turn <= last; turn += RK * TURN * WAVES)
     for (int kb = turn; kb <= min(last, turn + RK * (TURN - 1)); kb += RK) {
-      ask(kb);
+      if (!ROTATED || kb != start) ask(kb);
+      if (ROTATED && own && kb <= pos && pos < kb + RK) {
+#pragma unroll
+        for (int kt = 0; kt < KT; ++kt)
+#pragma unroll
+          for (int s = 0; s < DSTEPS; ++s) {
+            const bf16x8 k = load8(vt_s + (s * 4 + grp) * VPITCH + RK);
+            if (kb + kt * 16 + col == pos) ka[kt][s] = k;
+          }
+        const bf16x8 v = load8(vt_s + (CHUNKS + chunk_at / 8) * VPITCH + RK);
+#pragma unroll
+        for (int ps = 0; ps < PASSES; ++ps)
+          if (kb + ksub * PASSES + ps == pos) vv[ps] = v;
+      }
       round(kb);
     }
   // ---- the waves meet: a wave's sums lie where its values lay
@@ -567,21 +652,24 @@ static int launch_decode_attention(const void* q, const void* k_cache, const voi
                                    const void* block_tables, int max_blocks, int T, int Hq, int Hkv, int page_size,
                                    float scale, int window, int split_len, int n_splits, hipStream_t s, float cap = 0.f,
                                    int has_sink = 0, float sink = 0.f, const void* sinks = nullptr, const void* slopes = nullptr,
-                                   const void* gate = nullptr, long long gate_ld = 0) {
+                                   const void* gate = nullptr, long long gate_ld = 0, const Rotated* rotated = nullptr) {
   int page_shift = -1;
   for (int b = 0; b < 31; ++b)
     if (page_size == (1 << b)) page_shift = b;
   dim3 grid(Hkv * ((Hq / Hkv + 15) / 16), T, n_splits);
   const float log2e = 1.4426950408889634f;
-#define NHV_DECODE_LAUNCH(CAPPED_, BIASED_)                                                                           \
-  hipLaunchKernelGGL((decode_attention_kernel<CAPPED_, BIASED_>), grid, dim3(64 * WAVES), 0, s, (const bf16_t*)q, (const bf16_t*)k_cache, \
+#define NHV_DECODE_LAUNCH(...)                                                                                        \
+  hipLaunchKernelGGL((decode_attention_kernel<__VA_ARGS__>), grid, dim3(64 * WAVES), 0, s, (const bf16_t*)q, (const bf16_t*)k_cache, \
                      (const bf16_t*)v_cache, part_o, part_ml, (bf16_t*)out, (const int*)token_req,                    \
                      (const int*)positions, (const int*)block_tables, max_blocks, Hq, Hkv, page_size, page_shift,     \
                      scale * log2e, window, split_len, n_splits, cap * log2e, cap > 0.f ? 2.0f * log2e * scale / cap : 0.f, \
-                     (const float*)slopes, finish)
+                     (const float*)slopes, finish, rotated ? *rotated : Rotated{})
   const float sink_l2 = has_sink ? sink * log2e : -INFINITY;
   const Finish finish = {sink_l2, (const float*)sinks, (const bf16_t*)gate, gate_ld};
-  if (cap > 0.f && slopes) NHV_DECODE_LAUNCH(true, true);
+  if (rotated) {
+    if constexpr (CAN_ROTATE) NHV_DECODE_LAUNCH(false, false, true);
+    else return nhv_fail("decode attention: heads of %d entries are not turned here", D);
+  } else if (cap > 0.f && slopes) NHV_DECODE_LAUNCH(true, true);
   else if (cap > 0.f) NHV_DECODE_LAUNCH(true, false);
   else if (slopes) NHV_DECODE_LAUNCH(false, true);
   else NHV_DECODE_LAUNCH(false, false);
@@ -631,6 +719,32 @@ extern "C" int nhv_decode_attention_bf16(const void* q, const void* k_cache, con
   return launch_decode_attention(q, k_cache, v_cache, out, (float*)part_o, (float*)part_ml, token_req, positions,
                                  block_tables, max_blocks, T, Hq, Hkv, page_size, scale, window, split_len, n_splits,
                                  (hipStream_t)stream);
+}
+
+// The same with queries and the tokens' own keys and values as their projection left them: ``qkv`` [T, (Hq + 2 Hkv) D] in
+// bfloat16, or (splits > 0) that many float parts of it; the kernel adds the bias (null: none), divides every head of queries and
+// keys by its root mean square and multiplies by its weight (null: not), turns it by the halves' angles of its position (cos_sin
+// [positions, D]; null: not) and stores keys and values at slot_mapping[t] (negative: nowhere). Every token is of another request
+// and reads no slot that another one of the call stores to.
+extern "C" int nhv_decode_attention_rotated_bf16(const void* qkv, int splits, const void* bias, const void* q_norm_w, const void* k_norm_w,
+                                                 int w_dtype, float eps, const void* cos_sin, const void* rotation_positions,
+                                                 const void* slot_mapping, void* k_cache, void* v_cache, void* out, void* part_o,
+                                                 void* part_ml, const void* token_req, const void* positions, const void* block_tables,
+                                                 int max_blocks, int T, int Hq, int Hkv, int page_size, float scale, int window,
+                                                 int split_len, int n_splits, void* stream) {
+  if (check_decode_attention(max_blocks, T, Hq, Hkv, page_size, window, split_len, n_splits)) return 1;
+  NHV_REQUIRE(splits == 0 || splits == 1 || splits == 2 || splits == 4 || splits == 8, "decode attention: %d parts", splits);
+  NHV_REQUIRE((q_norm_w == nullptr) == (k_norm_w == nullptr) && (!q_norm_w || w_dtype == NHV_F32 || w_dtype == NHV_BF16),
+              "decode attention: q and k norm weights come together, in float or bfloat16");
+  NHV_REQUIRE(slot_mapping && k_cache && v_cache && (!cos_sin || rotation_positions), "decode attention: keys and values without a place");
+  const uintptr_t starts = (uintptr_t)qkv | (uintptr_t)bias | (uintptr_t)q_norm_w | (uintptr_t)k_norm_w | (uintptr_t)cos_sin |
+                           (uintptr_t)k_cache | (uintptr_t)v_cache;
+  NHV_REQUIRE(starts % 16 == 0, "decode attention: rows off 16-byte boundaries");
+  const Rotated rotated = {qkv, splits, (size_t)T * (Hq + 2 * Hkv) * D, (const bf16_t*)bias, q_norm_w, k_norm_w, w_dtype == NHV_F32, eps,
+                           (const float*)cos_sin, (const int*)rotation_positions, (const int*)slot_mapping};
+  return launch_decode_attention(nullptr, k_cache, v_cache, out, (float*)part_o, (float*)part_ml, token_req, positions, block_tables,
+                                 max_blocks, T, Hq, Hkv, page_size, scale, window, split_len, n_splits, (hipStream_t)stream, 0.f, 0, 0.f,
+                                 nullptr, nullptr, nullptr, 0, &rotated);
 }
 
 // The same with a cap on the scores (0: none), one more term exp(sink) in the denominator (has_sink: sink; sinks: one

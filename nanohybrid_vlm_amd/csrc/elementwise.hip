@@ -3,6 +3,7 @@
 // (float, bfloat16); statistics, angles and sums are float.
 #include "nhv_common.h"
 #include "nhv_gates.h"
+#include "nhv_head_pieces.h"
 
 // ---------------------------------------------------------------- embedding
 // scale: the row is multiplied by it in float and rounded once (1: the row is copied as it is)
@@ -64,64 +65,8 @@ __global__ void rmsnorm_kernel(const T* __restrict__ x, R* __restrict__ residual
   }
 }
 
-// The same for widths that are a multiple of 8: every thread owns up to MAXC pieces of 8 consecutive entries,
-// asks for all of them (rows, residual and weight) before it uses any, and keeps the sums in registers.
-template <typename V>
-__device__ __forceinline__ void load8f(const V* p, float* out) {
-#pragma unroll
-  for (int e = 0; e < 8; ++e) out[e] = to_f32(p[e]);
-}
-template <>
-__device__ __forceinline__ void load8f<bf16_t>(const bf16_t* p, float* out) {
-  typedef __attribute__((__vector_size__(8 * sizeof(__bf16)))) __bf16 v8;
-  const v8 v = *reinterpret_cast<const v8*>(p);
-#pragma unroll
-  for (int e = 0; e < 8; ++e) out[e] = (float)v[e];
-}
-template <>
-__device__ __forceinline__ void load8f<float>(const float* p, float* out) {
-  const float4 a = *reinterpret_cast<const float4*>(p), b = *reinterpret_cast<const float4*>(p + 4);
-  out[0] = a.x; out[1] = a.y; out[2] = a.z; out[3] = a.w; out[4] = b.x; out[5] = b.y; out[6] = b.z; out[7] = b.w;
-}
-template <typename V>
-__device__ __forceinline__ void store8f(V* p, const float* in) {
-#pragma unroll
-  for (int e = 0; e < 8; ++e) p[e] = from_f32<V>(in[e]);
-}
-template <>
-__device__ __forceinline__ void store8f<bf16_t>(bf16_t* p, const float* in) {
-  typedef __attribute__((__vector_size__(8 * sizeof(__bf16)))) __bf16 v8;
-  v8 v;
-#pragma unroll
-  for (int e = 0; e < 8; ++e) v[e] = (__bf16)in[e];
-  *reinterpret_cast<v8*>(p) = v;
-}
-template <>
-__device__ __forceinline__ void store8f<float>(float* p, const float* in) {
-  *reinterpret_cast<float4*>(p) = make_float4(in[0], in[1], in[2], in[3]);
-  *reinterpret_cast<float4*>(p + 4) = make_float4(in[4], in[5], in[6], in[7]);
-}
-
-// Eight entries of a product that comes as float parts (gemm_lines_bf16.hip), `stride` entries apart, added in their order; all
-// parts are asked for before the first is used.
-template <int SPLITS>
-__device__ __forceinline__ void add_parts8(const float* p, size_t stride, float* out) {
-  float part[SPLITS][8];
-#pragma unroll
-  for (int s = 0; s < SPLITS; ++s) load8f<float>(p + s * stride, part[s]);
-#pragma unroll
-  for (int e = 0; e < 8; ++e) {
-    out[e] = part[0][e];
-#pragma unroll
-    for (int s = 1; s < SPLITS; ++s) out[e] += part[s][e];
-  }
-}
-__device__ __forceinline__ void add_parts8(const float* p, size_t stride, int splits, float* out) {
-  if (splits == 8) add_parts8<8>(p, stride, out);
-  else if (splits == 4) add_parts8<4>(p, stride, out);
-  else if (splits == 2) add_parts8<2>(p, stride, out);
-  else add_parts8<1>(p, stride, out);
-}
+// Widths that are a multiple of 8: every thread owns up to MAXC pieces of 8 consecutive entries, asks for all of them
+// (rows, residual and weight) before it uses any, and keeps the sums in registers.
 
 // residual += the product whose parts these are (not rounded in between); y = the norm of the sum: what rmsnorm does with mode 1.
 // Four parts cost it nothing that can be seen: 64 rows of 4,096 entries 4.8 us, of a bfloat16 product 5.1.
@@ -539,31 +484,8 @@ __global__ __launch_bounds__(256) void qk_rope_write_vec_kernel(
     store8f<T>(v_cache + ((size_t)slot * Hkv + (h - Hq - Hkv)) * D + c * 8, v);
     return;
   }
-  const W* nw = is_q ? q_norm_w : k_norm_w;
-  if (nw) {
-    float ss = 0.f;
-#pragma unroll
-    for (int e = 0; e < 8; ++e) ss += v[e] * v[e];
-#pragma unroll
-    for (int off = 1; off < CH; off <<= 1) ss += __shfl_xor(ss, off, NHV_WAVE);
-    const float r = 1.0f / sqrtf(ss / (float)D + eps);
-    float wv[8];
-    load8f<W>(nw + c * 8, wv);
-#pragma unroll
-    for (int e = 0; e < 8; ++e) v[e] = to_f32(from_f32<T>(to_f32(from_f32<T>(v[e] * r)) * wv[e]));
-  }
   float o[8];
-  if (rot > 0) {
-    const bool first_half = c < HALF_LANES;
-#pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      const float partner = __shfl_xor(v[e], HALF_LANES, NHV_WAVE);
-      o[e] = first_half ? v[e] * cs[e] - partner * sn[e] : v[e] * cs[e] + partner * sn[e];
-    }
-  } else {
-#pragma unroll
-    for (int e = 0; e < 8; ++e) o[e] = v[e];
-  }
+  normed_and_turned<T, W, CH>(v, is_q ? q_norm_w : k_norm_w, eps, rot > 0, cs, sn, c, o);
   T* dst = is_q ? q_out + ((size_t)t * Hq + h) * D : k_cache + ((size_t)slot * Hkv + (h - Hq)) * D;
   store8f<T>(dst + c * 8, o);
 }

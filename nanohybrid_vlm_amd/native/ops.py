@@ -580,6 +580,14 @@ class NativeBackend:
         scores, a further term in the denominator and a gate per head, for the entry point that takes them."""
         T, Hq, D = q.shape
         _, page_size, Hkv, _ = k_cache.shape
+        part_o, part_ml, split_len, n_splits = self._decode_splits(T, Hq, Hkv, D, batch, window, q.device)
+        self._call("nhv_decode_attention_bf16" + ("_more" if more else ""), _ptr(q), _ptr(k_cache), _ptr(v_cache), _ptr(out),
+                   _ptr(part_o), _ptr(part_ml), _ptr(batch.token_req), _ptr(batch.positions), _ptr(block_tables),
+                   block_tables.shape[1], T, Hq, Hkv, page_size, ctypes.c_float(scale), window, split_len, n_splits,
+                   *more, _stream(), lib=self.attention_lib(D))
+
+    def _decode_splits(self, T, Hq, Hkv, D, batch, window, device):
+        """(partial sums, maxima and sums of weights, keys a split, splits) of a launch over single tokens."""
         # inside a graph the lengths are only bounded (by max_model_len): the recorder says what to plan for
         span = min(self.planned_context, batch.max_context_len) if self.planned_context else batch.max_context_len
         if window:                                   # (a chunk comes as a negative window)
@@ -594,12 +602,21 @@ class NativeBackend:
         n_splits = -(-covered // split_len)
         part_o = part_ml = None                             # (one split: the kernel writes the result itself)
         if n_splits > 1:
-            part_o = torch.empty((T, Hq, n_splits, D), dtype=torch.float32, device=q.device)
-            part_ml = torch.empty((T, Hq, n_splits, 2), dtype=torch.float32, device=q.device)
-        self._call("nhv_decode_attention_bf16" + ("_more" if more else ""), _ptr(q), _ptr(k_cache), _ptr(v_cache), _ptr(out),
-                   _ptr(part_o), _ptr(part_ml), _ptr(batch.token_req), _ptr(batch.positions), _ptr(block_tables),
-                   block_tables.shape[1], T, Hq, Hkv, page_size, ctypes.c_float(scale), window, split_len, n_splits,
-                   *more, _stream(), lib=self.attention_lib(D))
+            part_o = torch.empty((T, Hq, n_splits, D), dtype=torch.float32, device=device)
+            part_ml = torch.empty((T, Hq, n_splits, 2), dtype=torch.float32, device=device)
+        return part_o, part_ml, split_len, n_splits
+
+    def decode_attention_rotated(self, qkv, bias, q_norm_w, k_norm_w, eps, cos_sin, rotation_positions, slot_mapping, k_cache, v_cache,
+                                 out, batch, block_tables, scale, window):
+        """``qk_rope_write`` and the attention of single tokens in one launch (the splits' merge aside)."""
+        T, Hq, D = out.shape
+        _, page_size, Hkv, _ = k_cache.shape
+        part_o, part_ml, split_len, n_splits = self._decode_splits(T, Hq, Hkv, D, batch, window, out.device)
+        self._call("nhv_decode_attention_rotated_bf16", _ptr(qkv), qkv.shape[0] if qkv.dim() == 3 else 0, _ptr(bias), _ptr(q_norm_w),
+                   _ptr(k_norm_w), BF16 if q_norm_w is None else dtype_code(q_norm_w), ctypes.c_float(eps), _ptr(cos_sin),
+                   _ptr(rotation_positions), _ptr(slot_mapping), _ptr(k_cache), _ptr(v_cache), _ptr(out), _ptr(part_o), _ptr(part_ml),
+                   _ptr(batch.token_req), _ptr(batch.positions), _ptr(block_tables), block_tables.shape[1], T, Hq, Hkv, page_size,
+                   ctypes.c_float(scale), window, split_len, n_splits, _stream(), lib=self.attention_lib(D))
 
     # -- matrix products of few rows: own kernel or one of the library's algorithms, by measurement --
     def blas_lib(self) -> ctypes.CDLL:
@@ -1307,14 +1324,17 @@ def rotation_takes_parts(head_dim: int, cos_sin, pair_axes, *others) -> bool:
     return whole and all(t is None or t.data_ptr() % 16 == 0 for t in (cos_sin, *others))
 
 
-def qk_rope_write(qkv, bias, q_norm_w, k_norm_w, eps, cos_sin, positions, slot_mapping, k_cache, v_cache,
-                  num_heads: int, num_kv_heads: int, head_dim: int, write_kv: bool = True,
-                  pair_axes: torch.Tensor | None = None) -> torch.Tensor:
-    """Splits the packed projection, norms and turns q and k, stores k and v in the
-    paged cache and returns q as [tokens, heads, head_dim].
-    ``positions``: [tokens], or [axes, tokens] with ``pair_axes`` [rotary size / 2] (int32): the axis whose
-    coordinate turns each pair (without ``pair_axes`` every pair turns by the first axis).
-    ``qkv`` may be ``Parts``."""
+# Up to so many blocks (tokens times groups of query heads) queries and keys are turned in the attention's own launch. A block is alone on
+# its compute unit, and what it does before its first keys have come is hidden behind them; beyond a block a unit it adds up to what
+# the launch saved. us a step, two launches and one: 14 layers of the 0.6B shape, 1 request after 4,000 keys 575, 543, 16 after 30 to
+# 300 624, 603, 32 after 500 766, 741, 40 after 300 868, 867, 64 after 50 to 700 963, 971, 128 1,577, 1,633; 6 layers of the 8B shape,
+# 4 after 97 to 900 756, 742, 16 after 2,000 936, 924, 32 after 100 to 4,000 1,275, 1,267, 96 after 97 to 1,500 1,546, 1,557.
+ROTATED_BLOCKS = 256
+
+
+def _rotation_rows(qkv, bias, q_norm_w, k_norm_w, cos_sin, positions, slot_mapping, k_cache, v_cache, num_heads, num_kv_heads, head_dim,
+                   write_kv, pair_axes):
+    """What ``qk_rope_write`` checks. Returns (the projection's rows, or its parts where the kernel adds them up; the rotary size)."""
     T = qkv.shape[0]
     width = (num_heads + 2 * num_kv_heads) * head_dim
     split = qkv if isinstance(qkv, Parts) else None
@@ -1354,12 +1374,46 @@ def qk_rope_write(qkv, bias, q_norm_w, k_norm_w, eps, cos_sin, positions, slot_m
               lambda: f"qk_rope_write: cache shape {tuple(k_cache.shape)} does not fit {num_kv_heads} heads of {head_dim}")
         _dense(k_cache, "qk_rope_write: k_cache", dtype=qkv.dtype)
         _dense(v_cache, "qk_rope_write: v_cache", tuple(k_cache.shape), qkv.dtype)
-    q_out = torch.empty((T, num_heads, head_dim), dtype=qkv.dtype, device=qkv.device)
-    backend().qk_rope_write(qkv if split is None else split.parts, bias, q_norm_w, k_norm_w, float(eps), cos_sin, rot, positions,
+    return (qkv if split is None else split.parts), rot
+
+
+def qk_rope_write(qkv, bias, q_norm_w, k_norm_w, eps, cos_sin, positions, slot_mapping, k_cache, v_cache,
+                  num_heads: int, num_kv_heads: int, head_dim: int, write_kv: bool = True,
+                  pair_axes: torch.Tensor | None = None) -> torch.Tensor:
+    """Splits the packed projection, norms and turns q and k, stores k and v in the
+    paged cache and returns q as [tokens, heads, head_dim].
+    ``positions``: [tokens], or [axes, tokens] with ``pair_axes`` [rotary size / 2] (int32): the axis whose
+    coordinate turns each pair (without ``pair_axes`` every pair turns by the first axis).
+    ``qkv`` may be ``Parts``."""
+    rows, rot = _rotation_rows(qkv, bias, q_norm_w, k_norm_w, cos_sin, positions, slot_mapping, k_cache, v_cache, num_heads, num_kv_heads,
+                               head_dim, write_kv, pair_axes)
+    q_out = torch.empty((qkv.shape[0], num_heads, head_dim), dtype=qkv.dtype, device=rows.device)
+    backend().qk_rope_write(rows, bias, q_norm_w, k_norm_w, float(eps), cos_sin, rot, positions,
                             slot_mapping if write_kv else None, q_out, k_cache if write_kv else None,
                             v_cache if write_kv else None, num_heads, num_kv_heads, head_dim, write_kv,
                             **({} if pair_axes is None else {"pair_axes": pair_axes}))
     return q_out
+
+
+def _check_paged(T, Hq, D, dtype, k_cache, v_cache, batch: AttentionBatch, block_tables):
+    """That tokens, caches, batch and block tables fit each other."""
+    _need(k_cache.dim() == 4 and k_cache.shape[3] == D, lambda: f"attention: cache shape {tuple(k_cache.shape)} with head size {D}")
+    _dense(k_cache, "attention: k_cache", dtype=dtype)
+    _need(v_cache.dim() == 4 and tuple(v_cache.shape[:3]) == tuple(k_cache.shape[:3]),
+          lambda: f"attention: value cache {tuple(v_cache.shape)} beside key cache {tuple(k_cache.shape)}")
+    _dense(v_cache, "attention: v_cache", dtype=dtype)
+    Hkv = k_cache.shape[2]
+    _need(Hq % Hkv == 0, lambda: f"attention: {Hq} query heads are not a multiple of {Hkv} key heads")
+    _need(T == batch.num_tokens, lambda: f"attention: {T} tokens but the batch has {batch.num_tokens}")
+    _dense(batch.token_req, "attention: token_req", (T,), torch.int32)
+    _dense(batch.positions, "attention: positions", (T,), torch.int32)
+    _need(block_tables.dim() == 2 and block_tables.shape[0] == batch.num_requests,
+          lambda: f"attention: block tables {tuple(block_tables.shape)} for {batch.num_requests} requests")
+    _dense(block_tables, "attention: block_tables", dtype=torch.int32)
+    page_size = k_cache.shape[1]
+    _need(block_tables.shape[1] * page_size >= batch.max_context_len,
+          lambda: f"attention: block tables of {block_tables.shape[1]} pages of {page_size} are too short for "
+          f"{batch.max_context_len} keys")
 
 
 def paged_attention(q, k_cache, v_cache, batch: AttentionBatch, block_tables, scale: float,
@@ -1376,25 +1430,9 @@ def paged_attention(q, k_cache, v_cache, batch: AttentionBatch, block_tables, sc
     T, Hq, D = q.shape
     _dense(q, "attention: q")
     dtype_code(q)
-    _need(k_cache.dim() == 4 and k_cache.shape[3] == D, lambda: f"attention: cache shape {tuple(k_cache.shape)} with head size {D}")
-    _dense(k_cache, "attention: k_cache", dtype=q.dtype)
-    _need(v_cache.dim() == 4 and tuple(v_cache.shape[:3]) == tuple(k_cache.shape[:3]),
-          lambda: f"attention: value cache {tuple(v_cache.shape)} beside key cache {tuple(k_cache.shape)}")
-    _dense(v_cache, "attention: v_cache", dtype=q.dtype)
     _need(not (window and chunk), "attention: a window or a chunk, not both")
     _need(chunk is None or chunk > 0, lambda: f"attention: chunk {chunk}")
-    Hkv = k_cache.shape[2]
-    _need(Hq % Hkv == 0, lambda: f"attention: {Hq} query heads are not a multiple of {Hkv} key heads")
-    _need(T == batch.num_tokens, lambda: f"attention: {T} tokens but the batch has {batch.num_tokens}")
-    _dense(batch.token_req, "attention: token_req", (T,), torch.int32)
-    _dense(batch.positions, "attention: positions", (T,), torch.int32)
-    _need(block_tables.dim() == 2 and block_tables.shape[0] == batch.num_requests,
-          lambda: f"attention: block tables {tuple(block_tables.shape)} for {batch.num_requests} requests")
-    _dense(block_tables, "attention: block_tables", dtype=torch.int32)
-    page_size = k_cache.shape[1]
-    _need(block_tables.shape[1] * page_size >= batch.max_context_len,
-          lambda: f"attention: block tables of {block_tables.shape[1]} pages of {page_size} are too short for "
-          f"{batch.max_context_len} keys")
+    _check_paged(T, Hq, D, q.dtype, k_cache, v_cache, batch, block_tables)
     out = torch.empty((T, Hq, v_cache.shape[3]), dtype=q.dtype, device=q.device)
     more = {}
     if softcap is not None:
@@ -1419,6 +1457,34 @@ def paged_attention(q, k_cache, v_cache, batch: AttentionBatch, block_tables, sc
     else:
         backend().paged_attention(q, k_cache, v_cache, out, batch, block_tables, float(scale), int(window or 0), **more)
     return out
+
+
+def rotated_attention(qkv, bias, q_norm_w, k_norm_w, eps, cos_sin, positions, slot_mapping, k_cache, v_cache, num_heads: int,
+                      num_kv_heads: int, head_dim: int, batch: AttentionBatch, block_tables, scale: float, window: int | None = None,
+                      write_kv: bool = True, pair_axes: torch.Tensor | None = None) -> torch.Tensor:
+    """``qk_rope_write`` and ``paged_attention`` of what it returns; in one launch where every request brings one token.
+
+    One launch: bfloat16, heads of 32, 64 or 128 turned whole or not at all, rows, weights and caches on 16 bytes, no more than
+    ``ROTATED_BLOCKS`` blocks, and only where keys and values are stored: a token's key is then stored by the block that reads it,
+    so no other token of the call may read its slot, which holds for tokens of different requests (pages are known to others
+    only once they have been committed)."""
+    T = qkv.shape[0]
+    make = getattr(backend(), "decode_attention_rotated", None)
+    if (make is not None and batch.max_q_len == 1 and write_kv and pair_axes is None and positions.dim() == 1
+            and 0 < T * num_kv_heads * -(-num_heads // num_kv_heads // 16) <= ROTATED_BLOCKS
+            and qkv.dtype == torch.bfloat16 and head_dim in (32, 64, 128)
+            and rotation_takes_parts(head_dim, cos_sin, pair_axes, bias, q_norm_w, k_norm_w, k_cache, v_cache)):
+        rows, _ = _rotation_rows(qkv, bias, q_norm_w, k_norm_w, cos_sin, positions, slot_mapping, k_cache, v_cache, num_heads,
+                                 num_kv_heads, head_dim, True, None)
+        if rows.data_ptr() % 16 == 0:
+            _check_paged(T, num_heads, head_dim, qkv.dtype, k_cache, v_cache, batch, block_tables)
+            out = torch.empty((T, num_heads, head_dim), dtype=qkv.dtype, device=rows.device)
+            make(rows, bias, q_norm_w, k_norm_w, float(eps), cos_sin, positions, slot_mapping, k_cache, v_cache, out, batch, block_tables,
+                 float(scale), int(window or 0))
+            return out
+    q = qk_rope_write(qkv, bias, q_norm_w, k_norm_w, eps, cos_sin, positions, slot_mapping, k_cache, v_cache, num_heads, num_kv_heads,
+                      head_dim, write_kv=write_kv, pair_axes=pair_axes)
+    return paged_attention(q, k_cache, v_cache, batch, block_tables, scale, window)
 
 
 def linear(x, w: torch.Tensor, bias: torch.Tensor | None = None, out_dtype=None, add_to: AddTo | None = None, parts: bool = False):

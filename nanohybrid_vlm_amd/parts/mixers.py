@@ -77,13 +77,12 @@ class GQAAttention(Part):
         table = self.position.rotation_table()
         qkv = ops.linear(x, self.qkv_weight, parts=ops.rotation_takes_parts(
             self.head_dim, table, pair_axes, self.qkv_bias_t, self.q_norm_weight, self.k_norm_weight, cache.k, cache.v))
-        q = ops.qk_rope_write(
+        o = ops.rotated_attention(
             qkv, self.qkv_bias_t, self.q_norm_weight, self.k_norm_weight,
             self.qk_norm_eps if self.qk_norm_eps is not None else 0.0,
             table, step.token_positions if pair_axes is None else step.positions,
-            tables.slot_mapping, cache.k, cache.v, self.num_heads, self.num_kv_heads, self.head_dim,
-            write_kv=cache.writes, pair_axes=pair_axes)
-        o = ops.paged_attention(q, cache.k, cache.v, step.attention, tables.block_tables, self.scale, self.window)
+            tables.slot_mapping, cache.k, cache.v, self.num_heads, self.num_kv_heads, self.head_dim, step.attention,
+            tables.block_tables, self.scale, self.window, write_kv=cache.writes, pair_axes=pair_axes)
         return ops.linear(o.view(o.shape[0], self.num_heads * self.head_dim), self.o_weight, add_to=add_to)
 
 

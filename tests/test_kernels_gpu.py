@@ -1849,3 +1849,44 @@ def test_heads_turned_in_pieces_of_eight_pairs(ops, dtype, T, Hq, Hkv, D, E, rot
         f = torch.rand(E // 2, device="cuda")
         a, b = ops.turn_back_(o.view(T, Hq, E), f, positions), ops.turn_back_(o_off, f, positions)
         torch.testing.assert_close(a, b, rtol=2.0 ** -7 if dtype == torch.bfloat16 else 0.0, atol=2.0 ** -20)
+
+
+@pytest.mark.parametrize("Hq,Hkv,D,page,window,norm,bias,parts", [
+    (16, 8, 128, 16, None, "float", False, 0), (6, 2, 64, 5, 70, None, True, 4), (20, 1, 32, 7, None, "rows", True, 0),
+    (32, 2, 128, 256, 300, "rows", False, 8), (4, 4, 64, 64, None, "turn nothing", False, 0),
+])
+@pytest.mark.parametrize("lens", [[150], [1, 2, 31, 32, 33, 64, 65, 300, 17], [40, 3, 2000, 500, 501] * 4, [300] * 40])
+def test_single_tokens_turned_stored_and_read_in_one_launch(ops, monkeypatch, Hq, Hkv, D, page, window, norm, bias, parts, lens):
+    """Against the two launches, bit for bit: what is read, and the whole cache afterwards (keys and values that are stored, rows
+    without a slot, a slot that is not where the token's position lies); also beside values that are no numbers and over
+    several splits."""
+    T = len(lens)
+    _, k, v, batch, bt, *_ = _paged_setup(torch.bfloat16, lens, [1] * T, Hq, Hkv, D, page, seed=96)
+    width = (Hq + 2 * Hkv) * D
+    rows = rnd(T, width, dtype=torch.bfloat16, seed=97)
+    if parts:
+        rows = ops.Parts(rnd(parts, T, width, seed=98), torch.bfloat16)
+    b = rnd(width, dtype=torch.bfloat16, seed=99) if bias else None
+    norms = (None, None) if norm in (None, "turn nothing") else tuple(
+        rnd(D, dtype=torch.float32 if norm == "float" else torch.bfloat16, seed=i) + 1 for i in (100, 101))
+    table = None if norm == "turn nothing" else rnd(max(lens), D, seed=102)
+    t = torch.arange(T, device="cuda")
+    pos = batch.positions.long()
+    slots = (bt[t, pos // page] * page + pos % page).int()
+    spare = k.shape[0]
+    k, v = (torch.cat((c, c[:1])) for c in (k, v))            # (a page that no request holds)
+    if T > 4:
+        slots[1], slots[3] = -1, spare * page + page - 1
+        k[bt[1, (lens[1] - 1) // page], (lens[1] - 1) % page] = 0.5
+        v[bt[1, (lens[1] - 1) // page], (lens[1] - 1) % page] = 0.25
+        v[bt[4, 0], 0, 0, 1] = float("inf")
+    k[bt[t, pos // page].long()[2:3], (pos % page)[2:3]] = float("nan")          # (what a token's own place held before is not read)
+    arguments = (rows, b, *norms, 1e-6, table, batch.positions, slots)
+    k1, v1, k2, v2 = k.clone(), v.clone(), k.clone(), v.clone()
+    q = ops.qk_rope_write(*arguments, k1, v1, Hq, Hkv, D)
+    want = ops.paged_attention(q, k1, v1, batch, bt, D ** -0.5, window)
+    monkeypatch.setattr(ops, "ROTATED_BLOCKS", 1 << 20)
+    monkeypatch.setattr(ops, "qk_rope_write", None)
+    got = ops.rotated_attention(*arguments, k2, v2, Hq, Hkv, D, batch, bt, D ** -0.5, window)
+    for a, c in ((got, want), (k2, k1), (v2, v1)):
+        assert torch.equal(a.view(torch.int16), c.view(torch.int16))
