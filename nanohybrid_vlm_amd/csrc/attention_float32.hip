@@ -24,6 +24,7 @@
 // memory, the other order first: six tokens after 100 10.5, 8.5; one after 300 16.1, 15.0; eight after 3,000 112, 90; 64 after
 // 500 59, 54; two after 200, 32 heads of 64 on 2, 9.0, 8.1. Where they lie in the L2: 8.1, 7.6; 14.4, 14.5; 90, 78.
 #include "nhv_common.h"
+#include "nhv_head_pieces.h"
 #include <math.h>
 
 typedef float f32x4 __attribute__((ext_vector_type(4)));
@@ -49,14 +50,26 @@ struct FloatAttention {
   long long gate_ld;
 };
 
-template <int CHUNKS, bool AT_ONCE>                      // of 64 value entries
-__global__ __launch_bounds__(64 * WAVES) void attention_float32_kernel(FloatAttention a) {
+// ROTATED (one token a request): queries and the token's own key and value come as their projection left them; a block norms and
+// turns its heads while its first keys are on their way, stores the key and the value, and takes these from LDS. us a step of 14
+// layers of the 0.6B shape, two launches and one: 1 request after 100 keys 762, 751, after 2,000 1,475, 1,472, 6 after 50 to 150
+// 827, 811, 32 after 300 1,207, 1,190.
+struct FloatRotated {
+  const float *qkv, *bias, *q_norm, *k_norm;
+  float eps;
+  const float* cos_sin;                                  // null: nothing is turned
+  const int *positions, *slots;
+};
+
+template <int CHUNKS, bool AT_ONCE, bool ROTATED>        // of 64 value entries
+__global__ __launch_bounds__(64 * WAVES) void attention_float32_kernel(FloatAttention a, FloatRotated from_rows) {
   extern __shared__ __attribute__((aligned(16))) float shared[];
   constexpr int E = 64 * CHUNKS, UNITS = AT_ONCE ? E / 16 : 4;   // (blocks of 16 key entries that have registers)
   const int D = AT_ONCE ? E : a.D, group = a.Hq / a.Hkv;
   float* qs = shared;                                    // [ROWS][D + 4]
   float* part = qs + ROWS * (D + 4);                     // [WAVES][ROWS][E + 4]
   float* stats = part + WAVES * ROWS * (E + 4);          // [WAVES][ROWS][2]: maximum and sum
+  float *own_k = stats + WAVES * ROWS * 2, *own_v = own_k + E;           // ROTATED: the token's own key and value
   const int kvh = blockIdx.y, req = blockIdx.z;
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, r16 = lane & 15, g = lane >> 4;
   const int* table = a.block_tables + (size_t)req * a.max_blocks;
@@ -72,7 +85,18 @@ __global__ __launch_bounds__(64 * WAVES) void attention_float32_kernel(FloatAtte
   auto query = [&](int r, int d) {
     return *reinterpret_cast<const f32x4*>(a.q + ((size_t)(first + (row0 + r) / group) * a.Hq + kvh * group + (row0 + r) % group) * D + d);
   };
-  if (AT_ONCE && q_row < ROWS && row0 + q_row < rows) mine_q = query(q_row, q_at);
+  if (AT_ONCE && !ROTATED && q_row < ROWS && row0 + q_row < rows) mine_q = query(q_row, q_at);
+  // (ROTATED: threads take eight entries of a head, heads the group's queries, then the key and the value)
+  constexpr int LANES = E / 8;
+  const int item = threadIdx.x / LANES, lane8 = threadIdx.x % LANES;
+  const bool of_v = item == group + 1, mine_item = ROTATED && item < group + 2;
+  float piece[8];
+  const int item_head = item < group ? kvh * group + item : a.Hq + (of_v ? a.Hkv : 0) + kvh;
+  int store_at = -1;
+  if constexpr (ROTATED) {
+    if (mine_item) load8f<float>(from_rows.qkv + ((size_t)first * (a.Hq + 2 * a.Hkv) + item_head) * D + lane8 * 8, piece);
+    store_at = from_rows.slots[first];
+  }
 
   // this lane's row: what it may read
   const int row = row0 + r16;
@@ -91,7 +115,9 @@ __global__ __launch_bounds__(64 * WAVES) void attention_float32_kernel(FloatAtte
   // lane l's own key of a block from kb on, and where it lies. A key that no row reads is taken for the tile's last: its score
   // is masked, and every load is without a condition (with one the compiler waits for all that are under way).
   auto slot_in = [&](int kb) {
-    const int mine = kb + lane % KEYS, own = mine >= tile_lo && mine <= tile_hi ? mine : tile_hi;
+    const int mine = kb + lane % KEYS;
+    // (ROTATED: the tile's last key may be under way to its place, so a key before the first is taken for the first)
+    const int own = ROTATED ? min(max(mine, tile_lo), tile_hi) : mine >= tile_lo && mine <= tile_hi ? mine : tile_hi;
     return table[own / a.page_size] * a.page_size + own % a.page_size;
   };
   // (the first block of this wave's from the tile's first key on)
@@ -121,7 +147,37 @@ __global__ __launch_bounds__(64 * WAVES) void attention_float32_kernel(FloatAtte
 #pragma unroll
       for (int u = 0; u < UNITS; ++u) ask(u, 16 * u);
     }
-    if (q_row < ROWS) *reinterpret_cast<f32x4*>(&qs[q_row * (D + 4) + q_at]) = mine_q;
+    if constexpr (ROTATED) {
+      if (mine_item) {
+        float y[8], cs[8], sn[8];
+        const bool turns = from_rows.cos_sin != nullptr && !of_v;
+        if (turns) {
+          const float* row = from_rows.cos_sin + (size_t)from_rows.positions[first] * D + lane8 % (LANES / 2) * 8;
+          load8f<float>(row, cs);
+          load8f<float>(row + D / 2, sn);
+        }
+        if (from_rows.bias) {
+          float b[8];
+          load8f<float>(from_rows.bias + (size_t)item_head * D + lane8 * 8, b);
+#pragma unroll
+          for (int e = 0; e < 8; ++e) piece[e] += b[e];
+        }
+        if (of_v) {
+#pragma unroll
+          for (int e = 0; e < 8; ++e) y[e] = piece[e];
+        } else {
+          normed_and_turned<float, float, LANES>(piece, item < group ? from_rows.q_norm : from_rows.k_norm, from_rows.eps, turns, cs, sn, lane8, y);
+        }
+        store8f<float>(item < group ? qs + item * (D + 4) + lane8 * 8 : (of_v ? own_v : own_k) + lane8 * 8, y);
+        if (item >= group && store_at >= 0)
+          store8f<float>(const_cast<float*>(of_v ? a.v : a.k) + ((size_t)store_at * a.Hkv + kvh) * D + lane8 * 8, y);
+      } else if (item < ROWS + 2) {                      // (rows of the tile that no head has)
+        float y[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+        store8f<float>(qs + (item - 2) * (D + 4) + lane8 * 8, y);
+      }
+    } else if (q_row < ROWS) {
+      *reinterpret_cast<f32x4*>(&qs[q_row * (D + 4) + q_at]) = mine_q;
+    }
   } else {
     for (int i = threadIdx.x * 4; i < ROWS * D; i += 64 * WAVES * 4) {
       const int r = i / D, d = i % D;
@@ -138,6 +194,9 @@ __global__ __launch_bounds__(64 * WAVES) void attention_float32_kernel(FloatAtte
   for (int h = 0; h < CHUNKS; ++h)
 #pragma unroll
     for (int j = 0; j < 4; ++j) o[h][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+  // what is read at the token's position is what it stores
+  bool own = false;
+  if constexpr (ROTATED) own = store_at >= 0 && store_at == table[tile_hi / a.page_size] * a.page_size + tile_hi % a.page_size;
   __syncthreads();                                       // (the queries are in LDS)
   for (int kb = from; kb <= tile_hi; kb += KEYS * WAVES) {
     const int next = kb + KEYS * WAVES;
@@ -167,15 +226,35 @@ __global__ __launch_bounds__(64 * WAVES) void attention_float32_kernel(FloatAtte
 #pragma unroll
         for (int t = 0; t < TILES; ++t) s[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[unit][t][j], qf[j], s[t], 0, 0, 0);
     };
-    const int held = slot;                               // (where this block's keys lie)
     if constexpr (AT_ONCE) {
       // all of the block is under way before the first product; the next block's keys follow behind this one's scores
       next_slot = slot_in(next);                         // (before the values: it is waited for with the keys)
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
       for (int h = 0; h < CHUNKS; ++h) values(h);
+      const bool newest = ROTATED && own && kb + KEYS > tile_hi;          // (keys beyond the last stand for it here, too)
+      if (newest)
+#pragma unroll
+        for (int u = 0; u < UNITS; ++u) {
+          const f32x4 k = *reinterpret_cast<const f32x4*>(&own_k[16 * u + 4 * g]);
+#pragma unroll
+          for (int t = 0; t < TILES; ++t)
+            if (kb + 16 * t + r16 >= tile_hi) kf[u][t] = k;
+          __builtin_amdgcn_sched_barrier(0);             // (one piece at a time: registers)
+        }
 #pragma unroll
       for (int u = 0; u < UNITS; ++u) score(u, 16 * u);
+      if (newest)
+#pragma unroll
+        for (int h = 0; h < CHUNKS; ++h) {
+          const f32x4 v = *reinterpret_cast<const f32x4*>(&own_v[64 * h + 4 * r16]);
+#pragma unroll
+          for (int t = 0; t < TILES; ++t)
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+              if (kb + 16 * t + 4 * g + i >= tile_hi) vf[h][t][i] = v;
+          __builtin_amdgcn_sched_barrier(0);
+        }
       if (next <= tile_hi) {
         slot = next_slot;
         keys_at();
@@ -262,14 +341,24 @@ __global__ __launch_bounds__(64 * WAVES) void attention_float32_kernel(FloatAtte
 #pragma unroll
           for (int i = 0; i < 4; ++i)
             for (int gk = 0; gk < 4; ++gk) {
-              const int at = __shfl(held, 16 * t + 4 * gk + i, NHV_WAVE);
               const float p = __shfl(s[t][i], 16 * gk + r16, NHV_WAVE);
-              if (p != 0.f) {
-                const float* row_v = a.v + ((size_t)at * a.Hkv + kvh) * E + 64 * h + 16 * g;
+              if constexpr (AT_ONCE) {                   // (the lanes of group gk hold the key's entries)
 #pragma unroll
                 for (int ii = 0; ii < 4; ++ii)
 #pragma unroll
-                  for (int j = 0; j < 4; ++j) now[j][ii] = fmaf(p, row_v[4 * ii + j], now[j][ii]);
+                  for (int j = 0; j < 4; ++j) {
+                    const float value = __shfl(vf[h][t][i][j], 16 * gk + 4 * g + ii, NHV_WAVE);
+                    if (p != 0.f) now[j][ii] = fmaf(p, value, now[j][ii]);
+                  }
+              } else {
+                const int at = __shfl(slot, 16 * t + 4 * gk + i, NHV_WAVE);
+                if (p != 0.f) {
+                  const float* row_v = a.v + ((size_t)at * a.Hkv + kvh) * E + 64 * h + 16 * g;
+#pragma unroll
+                  for (int ii = 0; ii < 4; ++ii)
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) now[j][ii] = fmaf(p, row_v[4 * ii + j], now[j][ii]);
+                }
               }
             }
       }
@@ -329,12 +418,12 @@ __global__ __launch_bounds__(64 * WAVES) void attention_float32_kernel(FloatAtte
   for (int i = 0; i < 2 * CHUNKS; ++i) out[c + 32 * i] = total[i] * inv;
 }
 
-template <int CHUNKS, bool AT_ONCE = false>
-static int launch(const FloatAttention& a, dim3 grid, size_t lds, hipStream_t s) {
-  static const hipError_t allowed = hipFuncSetAttribute((const void*)attention_float32_kernel<CHUNKS, AT_ONCE>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                                        (int)((ROWS * (MAX_D + 4) + WAVES * ROWS * (64 * CHUNKS + 4) + WAVES * ROWS * 2) * sizeof(float)));
+template <int CHUNKS, bool AT_ONCE = false, bool ROTATED = false>
+static int launch(const FloatAttention& a, dim3 grid, size_t lds, hipStream_t s, const FloatRotated& from_rows = {}) {
+  static const hipError_t allowed = hipFuncSetAttribute((const void*)attention_float32_kernel<CHUNKS, AT_ONCE, ROTATED>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                                        (int)((ROWS * (MAX_D + 4) + WAVES * ROWS * (64 * CHUNKS + 4) + WAVES * ROWS * 2 + 128 * CHUNKS) * sizeof(float)));
   if (allowed != hipSuccess) return nhv_fail("attention: %zu bytes of LDS are refused: %s", lds, hipGetErrorString(allowed));
-  hipLaunchKernelGGL((attention_float32_kernel<CHUNKS, AT_ONCE>), grid, dim3(64 * WAVES), lds, s, a);
+  hipLaunchKernelGGL((attention_float32_kernel<CHUNKS, AT_ONCE, ROTATED>), grid, dim3(64 * WAVES), lds, s, a, from_rows);
   NHV_LAUNCH_CHECK("attention_float32");
   return 0;
 }
@@ -365,4 +454,34 @@ extern "C" int nhv_attention_float32(const void* q, const void* k_cache, const v
     case 3: return launch<3>(a, dim3((unsigned)tiles, Hkv, B), lds, (hipStream_t)stream);
     default: return launch<4>(a, dim3((unsigned)tiles, Hkv, B), lds, (hipStream_t)stream);
   }
+}
+
+// One token a request (max_q_len 1), heads of 64 or 128 entries, up to 16 query heads a key head: the same with queries, keys and
+// values as their projection left them, ``qkv`` [T, (Hq + 2 Hkv) D]: the kernel adds the bias (null: none), divides every head of
+// queries and keys by its root mean square and multiplies by its weight (null: not), turns it by its position's angles (cos_sin
+// [positions, D]; null: not) and stores keys and values at slot_mapping[t] (negative: nowhere). Every token is of another request
+// and reads no slot that another one of the call stores to.
+extern "C" int nhv_attention_float32_rotated(const void* qkv, const void* bias, const void* q_norm_w, const void* k_norm_w, float eps,
+                                             const void* cos_sin, const void* rotation_positions, const void* slot_mapping, void* k_cache,
+                                             void* v_cache, void* out, const void* positions, const void* cu_seqlens_q,
+                                             const void* block_tables, int max_blocks, int B, int Hq, int Hkv, int D, int page_size,
+                                             float scale, int window, void* stream) {
+  NHV_REQUIRE(B > 0 && B <= 65535 && Hq > 0 && Hkv > 0 && Hkv <= 65535 && page_size > 0 && max_blocks > 0,
+              "attention: bad sizes B=%d Hq=%d Hkv=%d page=%d blocks=%d", B, Hq, Hkv, page_size, max_blocks);
+  NHV_REQUIRE(Hq % Hkv == 0 && Hq / Hkv <= ROWS && (D == 64 || D == 128) && window >= 0,
+              "attention: %d query heads of %d on %d key heads are not turned here", Hq, D, Hkv);
+  NHV_REQUIRE((q_norm_w == nullptr) == (k_norm_w == nullptr), "attention: q and k norm weights come together");
+  NHV_REQUIRE(slot_mapping && k_cache && v_cache && (!cos_sin || rotation_positions), "attention: keys and values without a place");
+  const uintptr_t starts = (uintptr_t)qkv | (uintptr_t)bias | (uintptr_t)q_norm_w | (uintptr_t)k_norm_w | (uintptr_t)cos_sin |
+                           (uintptr_t)k_cache | (uintptr_t)v_cache;
+  NHV_REQUIRE(starts % 16 == 0, "attention: rows off 16-byte boundaries");
+  FloatAttention a = {};
+  a.k = (const float*)k_cache, a.v = (const float*)v_cache, a.out = (float*)out;
+  a.positions = (const int*)positions, a.cu = (const int*)cu_seqlens_q, a.block_tables = (const int*)block_tables;
+  a.max_blocks = max_blocks, a.Hq = Hq, a.Hkv = Hkv, a.D = D, a.E = D, a.page_size = page_size, a.scale = scale, a.window = window;
+  const FloatRotated from_rows = {(const float*)qkv, (const float*)bias, (const float*)q_norm_w, (const float*)k_norm_w, eps,
+                                  (const float*)cos_sin, (const int*)rotation_positions, (const int*)slot_mapping};
+  const size_t lds = (ROWS * (D + 4) + WAVES * ROWS * (D + 4) + WAVES * ROWS * 2 + 2 * D) * sizeof(float);
+  const dim3 grid(1, Hkv, B);
+  return D == 64 ? launch<1, true, true>(a, grid, lds, (hipStream_t)stream, from_rows) : launch<2, true, true>(a, grid, lds, (hipStream_t)stream, from_rows);
 }

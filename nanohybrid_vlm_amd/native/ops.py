@@ -618,6 +618,15 @@ class NativeBackend:
                    _ptr(batch.token_req), _ptr(batch.positions), _ptr(block_tables), block_tables.shape[1], T, Hq, Hkv, page_size,
                    ctypes.c_float(scale), window, split_len, n_splits, _stream(), lib=self.attention_lib(D))
 
+    def attention_float32_rotated(self, qkv, bias, q_norm_w, k_norm_w, eps, cos_sin, rotation_positions, slot_mapping, k_cache, v_cache,
+                                  out, batch, block_tables, scale, window):
+        """The same in 32 bits."""
+        _, Hq, D = out.shape
+        self._call("nhv_attention_float32_rotated", _ptr(qkv), _ptr(bias), _ptr(q_norm_w), _ptr(k_norm_w), ctypes.c_float(eps), _ptr(cos_sin),
+                   _ptr(rotation_positions), _ptr(slot_mapping), _ptr(k_cache), _ptr(v_cache), _ptr(out), _ptr(batch.positions),
+                   _ptr(batch.cu_seqlens_q), _ptr(block_tables), block_tables.shape[1], batch.num_requests, Hq, k_cache.shape[2], D,
+                   k_cache.shape[1], ctypes.c_float(scale), window, _stream())
+
     # -- matrix products of few rows: own kernel or one of the library's algorithms, by measurement --
     def blas_lib(self) -> ctypes.CDLL:
         """The wrapper of the vendor's matrix library, loaded when a product is first given to it."""
@@ -1464,15 +1473,17 @@ def rotated_attention(qkv, bias, q_norm_w, k_norm_w, eps, cos_sin, positions, sl
                       write_kv: bool = True, pair_axes: torch.Tensor | None = None) -> torch.Tensor:
     """``qk_rope_write`` and ``paged_attention`` of what it returns; in one launch where every request brings one token.
 
-    One launch: bfloat16, heads of 32, 64 or 128 turned whole or not at all, rows, weights and caches on 16 bytes, no more than
-    ``ROTATED_BLOCKS`` blocks, and only where keys and values are stored: a token's key is then stored by the block that reads it,
+    One launch: heads of 32 (bfloat16 alone), 64 or 128 turned whole or not at all, in 32 bits up to 16 of them on a key head, rows,
+    weights and caches on 16 bytes, no more than ``ROTATED_BLOCKS`` blocks, and only where keys and values are stored: a token's key is then stored by the block that reads it,
     so no other token of the call may read its slot, which holds for tokens of different requests (pages are known to others
     only once they have been committed)."""
     T = qkv.shape[0]
-    make = getattr(backend(), "decode_attention_rotated", None)
+    float32 = qkv.dtype == torch.float32
+    make = getattr(backend(), "attention_float32_rotated" if float32 else "decode_attention_rotated", None)
+    group = num_heads // num_kv_heads
     if (make is not None and batch.max_q_len == 1 and write_kv and pair_axes is None and positions.dim() == 1
-            and 0 < T * num_kv_heads * -(-num_heads // num_kv_heads // 16) <= ROTATED_BLOCKS
-            and qkv.dtype == torch.bfloat16 and head_dim in (32, 64, 128)
+            and 0 < T * num_kv_heads * -(-group // 16) <= ROTATED_BLOCKS
+            and (head_dim in (64, 128) and group <= 16 if float32 else qkv.dtype == torch.bfloat16 and head_dim in (32, 64, 128))
             and rotation_takes_parts(head_dim, cos_sin, pair_axes, bias, q_norm_w, k_norm_w, k_cache, v_cache)):
         rows, _ = _rotation_rows(qkv, bias, q_norm_w, k_norm_w, cos_sin, positions, slot_mapping, k_cache, v_cache, num_heads,
                                  num_kv_heads, head_dim, True, None)

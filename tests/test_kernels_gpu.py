@@ -1854,22 +1854,24 @@ def test_heads_turned_in_pieces_of_eight_pairs(ops, dtype, T, Hq, Hkv, D, E, rot
 @pytest.mark.parametrize("Hq,Hkv,D,page,window,norm,bias,parts", [
     (16, 8, 128, 16, None, "float", False, 0), (6, 2, 64, 5, 70, None, True, 4), (20, 1, 32, 7, None, "rows", True, 0),
     (32, 2, 128, 256, 300, "rows", False, 8), (4, 4, 64, 64, None, "turn nothing", False, 0),
+    (16, 8, 128, 16, None, "in 32 bits", False, 0), (6, 2, 64, 5, 70, "in 32 bits", True, 0), (16, 1, 128, 256, 33, "in 32 bits", True, 0),
+    (4, 4, 64, 7, None, "in 32 bits, turn nothing", False, 0),
 ])
 @pytest.mark.parametrize("lens", [[150], [1, 2, 31, 32, 33, 64, 65, 300, 17], [40, 3, 2000, 500, 501] * 4, [300] * 40])
 def test_single_tokens_turned_stored_and_read_in_one_launch(ops, monkeypatch, Hq, Hkv, D, page, window, norm, bias, parts, lens):
     """Against the two launches, bit for bit: what is read, and the whole cache afterwards (keys and values that are stored, rows
     without a slot, a slot that is not where the token's position lies); also beside values that are no numbers and over
     several splits."""
-    T = len(lens)
-    _, k, v, batch, bt, *_ = _paged_setup(torch.bfloat16, lens, [1] * T, Hq, Hkv, D, page, seed=96)
+    T, dtype = len(lens), torch.float32 if norm and "32" in norm else torch.bfloat16
+    _, k, v, batch, bt, *_ = _paged_setup(dtype, lens, [1] * T, Hq, Hkv, D, page, seed=96)
     width = (Hq + 2 * Hkv) * D
-    rows = rnd(T, width, dtype=torch.bfloat16, seed=97)
+    rows = rnd(T, width, dtype=dtype, seed=97)
     if parts:
         rows = ops.Parts(rnd(parts, T, width, seed=98), torch.bfloat16)
-    b = rnd(width, dtype=torch.bfloat16, seed=99) if bias else None
-    norms = (None, None) if norm in (None, "turn nothing") else tuple(
-        rnd(D, dtype=torch.float32 if norm == "float" else torch.bfloat16, seed=i) + 1 for i in (100, 101))
-    table = None if norm == "turn nothing" else rnd(max(lens), D, seed=102)
+    b = rnd(width, dtype=dtype, seed=99) if bias else None
+    norms = (None, None) if norm is None or "nothing" in norm else tuple(
+        rnd(D, dtype=torch.float32 if norm == "float" else dtype, seed=i) + 1 for i in (100, 101))
+    table = None if norm and "nothing" in norm else rnd(max(lens), D, seed=102)
     t = torch.arange(T, device="cuda")
     pos = batch.positions.long()
     slots = (bt[t, pos // page] * page + pos % page).int()
@@ -1889,4 +1891,4 @@ def test_single_tokens_turned_stored_and_read_in_one_launch(ops, monkeypatch, Hq
     monkeypatch.setattr(ops, "qk_rope_write", None)
     got = ops.rotated_attention(*arguments, k2, v2, Hq, Hkv, D, batch, bt, D ** -0.5, window)
     for a, c in ((got, want), (k2, k1), (v2, v1)):
-        assert torch.equal(a.view(torch.int16), c.view(torch.int16))
+        assert torch.equal(a.view(torch.uint8), c.view(torch.uint8))
