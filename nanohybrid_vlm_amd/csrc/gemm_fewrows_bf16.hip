@@ -957,20 +957,22 @@ static int launch_tiles(const TilesPlan& p, hipStream_t s, const void* x, const 
 // SKIPS: up to 8 rows, whose waves without rows of x bring none (in their place the others bring the last one: 2,560 outputs of 4,096 columns at 1 and
 // 4 rows 7.5 and 7.6 us, with it 6.9 and 7.1; 2,560 of 9,728 15.2 and 15.3, 14.0 and 14.7; 3,584 of 18,944 25.9 and 26.1, 24.9 and 25.6). Not for
 // gated products (12,288 of 4,096 at 1 and 8 rows 33.7 and 33.1 us, with it 35.5 and 34.2) nor for float results, whose stretches are summed apart.
-template <int NT, int NB, bool GATED, typename TOut, bool SKIPS>
+// HALF: 8 rows of w a block, where 16 leave units idle: the lower half of the waves brings them, all of them bring x.
+template <int NT, int NB, bool GATED, typename TOut, bool SKIPS, bool HALF>
 __global__ __launch_bounds__(512) void gemm_fewrows_lines_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ w, const bf16_t* __restrict__ bias,
                                                                  TOut* __restrict__ y, int M, int N, int K, const Fusion f) {
-  constexpr int OUT = GATED ? 1 : NT, BOTH = GATED ? 2 : 1, CHUNK = 256, LOADS = NT + 1, STAGE = (NT + 1) * 16 * CHUNK;
+  constexpr int OUT = GATED ? 1 : NT, BOTH = GATED ? 2 : 1, CHUNK = 256, LOADS = NT + 1, STAGE = (NT + 1) * 16 * CHUNK, ROWS_W = HALF ? 8 : 16;
+  static_assert(!HALF || (NT == 1 && !GATED && !SKIPS), "half tiles are a block's only ones");
   // (a name of its own: an array of this alignment under the others' name would cost the kernels around their last 1,024 bytes)
   extern __shared__ __attribute__((aligned(1024))) bf16_t line_ring[];
   const bf16_t* ring = line_ring;
   __shared__ float r_s[16];
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, r16 = lane & 15, g = lane >> 4;
-  const int n0 = blockIdx.x * 16 * OUT, chunks = K / CHUNK;
+  const int n0 = blockIdx.x * ROWS_W * OUT, chunks = K / CHUNK;
   if (f.band_rows) x += (size_t)min(n0 / f.band_rows, f.bands - 1) * M * K;      // (a block's tiles lie in one band)
   // what the thread that finishes output (row, n) needs beside the sums, asked for before the weights
   const int row = (threadIdx.x >> 4) & 15, tile = threadIdx.x >> 8, n = n0 + 16 * tile + (threadIdx.x & 15);
-  const bool mine = tile < OUT && row < M && n < N;
+  const bool mine = tile < OUT && row < M && n < N && (int)(threadIdx.x & 15) < ROWS_W;
   float share[SCALE_ROWS<8>][SCALE_SHARES];
   ask_row_scales<8>(f, share, M, wave, lane);
   float res = 0.f, next_w = 1.f, add[2] = {0.f, 0.f};
@@ -998,10 +1000,10 @@ __global__ __launch_bounds__(512) void gemm_fewrows_lines_kernel(const bf16_t* _
   constexpr int STRETCHES = sizeof(TOut) == 4 ? 4 : 1;
   const bool stretches = STRETCHES > 1 && K % 2048 == 0;
   const int length = stretches ? chunks / STRETCHES : chunks + 1, place = nhv_first_chunk(blockIdx.x, chunks, K), first = stretches ? place / length * length : place;
-  auto ask = [&](auto brings_x, int buf, int c) {
+  auto ask = [&](auto brings_w, auto brings_x, int buf, int c) {
     const size_t k = (size_t)nhv_chunk(first, c, chunks) * CHUNK;
 #pragma unroll
-    for (int t = 0; t < (decltype(brings_x)::value ? LOADS : NT); ++t) {
+    for (int t = decltype(brings_w)::value ? 0 : NT; t < (decltype(brings_x)::value ? LOADS : NT); ++t) {
       if (t < NT) nhv_load_to_lds<true>(ring_at + (buf * STAGE + t * 16 * CHUNK) * 2, src[t] + k);
       else nhv_load_to_lds<false>(ring_at + (buf * STAGE + t * 16 * CHUNK) * 2, src[t] + k);
     }
@@ -1014,13 +1016,13 @@ __global__ __launch_bounds__(512) void gemm_fewrows_lines_kernel(const bf16_t* _
     for (int i = 0; i < STRETCHES; ++i) done[i][t] = acc[t];
   }
   const int at = r16 * CHUNK + (((wave * 4 + g) ^ r16) << 3);
-  if constexpr (!SKIPS) {
+  if constexpr (!SKIPS && !HALF) {
 #pragma unroll
-    for (int i = 0; i < NB - 1; ++i) ask(std::true_type{}, i, i);
+    for (int i = 0; i < NB - 1; ++i) ask(std::true_type{}, std::true_type{}, i, i);
     int buf = 0, now = first / length, left = length;
     for (int c = 0; c < chunks; ++c) {
       nhv_wait_and_meet<(NB - 2) * LOADS>();                            // chunk c is there, chunk c - 1 has been read
-      ask(std::true_type{}, buf == 0 ? NB - 1 : buf - 1, c + NB - 1);
+      ask(std::true_type{}, std::true_type{}, buf == 0 ? NB - 1 : buf - 1, c + NB - 1);
       const bf16_t* from = ring + buf * STAGE + at;
       const bf16x8 b = *reinterpret_cast<const bf16x8*>(from + NT * 16 * CHUNK);
 #pragma unroll
@@ -1040,14 +1042,15 @@ __global__ __launch_bounds__(512) void gemm_fewrows_lines_kernel(const bf16_t* _
       }
     }
   } else {
-    // a wave whose rows of x are not there brings none (what lies in LDS in their place comes into rows whose results are dropped)
-    auto walk = [&](auto brings_x) {
+    // a wave whose rows of x (HALF: of w) are not there brings none (what lies in LDS in their place comes into rows or columns whose
+    // results are dropped)
+    auto walk = [&](auto brings_w, auto brings_x) {
 #pragma unroll
-      for (int i = 0; i < NB - 1; ++i) ask(brings_x, i, i);
+      for (int i = 0; i < NB - 1; ++i) ask(brings_w, brings_x, i, i);
       int buf = 0;
       for (int c = 0; c < chunks; ++c) {
-        nhv_wait_and_meet<(NB - 2) * (decltype(brings_x)::value ? LOADS : NT)>();
-        ask(brings_x, buf == 0 ? NB - 1 : buf - 1, c + NB - 1);
+        nhv_wait_and_meet<(NB - 2) * ((decltype(brings_w)::value ? NT : 0) + (decltype(brings_x)::value ? 1 : 0))>();
+        ask(brings_w, brings_x, buf == 0 ? NB - 1 : buf - 1, c + NB - 1);
         const bf16_t* from = ring + buf * STAGE + at;
         const bf16x8 b = *reinterpret_cast<const bf16x8*>(from + NT * 16 * CHUNK);
 #pragma unroll
@@ -1055,8 +1058,9 @@ __global__ __launch_bounds__(512) void gemm_fewrows_lines_kernel(const bf16_t* _
         buf = buf == NB - 1 ? 0 : buf + 1;
       }
     };
-    if (2 * wave < M) walk(std::true_type{});
-    else walk(std::false_type{});
+    if (HALF ? wave < 4 : 2 * wave < M) walk(std::true_type{}, std::true_type{});
+    else if constexpr (HALF) walk(std::false_type{}, std::true_type{});
+    else walk(std::true_type{}, std::false_type{});
   }
   if (stretches) {
 #pragma unroll
@@ -1112,18 +1116,23 @@ __global__ __launch_bounds__(512) void gemm_fewrows_lines_kernel(const bf16_t* _
 // to 12,288, at 1 to 8 rows: 8,448 outputs 1.07 to 1.18, 9,216 1.07 to 1.17, 10,240 1.00 to 1.11 and at K = 2,048 0.95, 11,264 0.96 to 1.07, 12,288 0.88 to
 // 1.04; 16 rows: K = 3,072 1.05 to 1.15, from 4,096 on 0.62 to 0.88), and with rows 16 KB apart on some of the units (K = 8,192: 4,224
 // to 6,144 outputs 1.06 to 1.22 at 1 to 4 rows, 0.81 to 0.99 at 8; 7,168 outputs 0.80 to 0.87), as long as all of x fits beside w.
-static bool lines_plan(bool glu, bool even, int M, int N, int K) {
+// ``half``: a bfloat16 result without residual, which 8 rows of w a block can make. us by the tiles above (M = 12 and more, 2,048 outputs: by
+// lines of 16 rows) and by those, of 2,048 outputs: of 2,048 columns at 4, 8 and 16 rows 5.2, 5.1, 5.7 and 4.8, 4.8, 5.0; of 6,144 9.0,
+// 9.9, 11.2 and 9.9, 9.9, 9.0 to 10.0; of 12,288 14.7, 18.7, 19.3 and 16.8, 16.7, 17.2 (10 rows 22.1, 16.6); 1,536 of 8,960 11.5, 12.5, 21.1 and 11.9, 11.8,
+// 11.3; 1,280 of 5,120 7.6, 8.2, 14.0 and 7.5, 7.4, 7.5; 1,040 of 2,048 4.7, 4.7, 5.0 and 4.5, 4.5, 4.6 (1 row 4.2, 4.5).
+static bool lines_plan(bool glu, bool even, bool half, int M, int N, int K) {
   if (K % 256 != 0 || K < 2048) return false;
   if (glu) return N >= 4096;
   if (even && N > 8192 && N <= (K > 2048 ? 11264 : 9216) && (long long)M * K <= 57344) return false;
   if (even && N > 4096 && N < 7168 && K % 8192 == 0 && (long long)M * K <= 32768) return false;
+  if (half && N > 1024 && N <= 2048 && (M >= 8 || (M >= 4 && K <= 5120))) return true;
   return N >= 2560 || (N >= 2048 && K >= 4096 && M >= 12);
 }
 
-template <int NT, int NB, bool GATED, typename TOut, bool SKIPS>
+template <int NT, int NB, bool GATED, typename TOut, bool SKIPS, bool HALF = false>
 static int launch_lines_as(hipStream_t s, const void* x, const void* w, const void* bias, void* y, int M, int N, int K, const Fusion& f) {
-  constexpr int OUT = GATED ? 16 : 16 * NT, ring = NB * (NT + 1) * 16 * 512, sums = NT * 8192, lds = ring > sums ? ring : sums;
-  auto kernel = gemm_fewrows_lines_kernel<NT, NB, GATED, TOut, SKIPS>;
+  constexpr int OUT = HALF ? 8 : GATED ? 16 : 16 * NT, ring = NB * (NT + 1) * 16 * 512, sums = NT * 8192, lds = ring > sums ? ring : sums;
+  auto kernel = gemm_fewrows_lines_kernel<NT, NB, GATED, TOut, SKIPS, HALF>;
   // more than 64 KB of dynamic LDS has to be allowed once per kernel (and per process)
   static const hipError_t allowed = hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
   if (allowed != hipSuccess) return nhv_fail("few-rows gemm: %s", hipGetErrorString(allowed));
@@ -1144,6 +1153,7 @@ static int launch_lines_of(hipStream_t s, const void* x, const void* w, const vo
 template <bool GATED, typename TOut>
 static int launch_lines(hipStream_t s, const void* x, const void* w, const void* bias, void* y, int M, int N, int K, const Fusion& f) {
   if constexpr (!GATED && sizeof(TOut) == 2) {
+    if (N <= 128 * 16 && !f.residual) return launch_lines_as<1, 4, false, TOut, false, true>(s, x, w, bias, y, M, N, K, f);
     if (M <= 8) return launch_lines_of<false, true, TOut>(s, x, w, bias, y, M, N, K, f);
   }
   return launch_lines_of<GATED, false, TOut>(s, x, w, bias, y, M, N, K, f);
@@ -1318,7 +1328,7 @@ static void launch(hipStream_t s, const void* x, const void* w, const void* bias
 // adds up 256 shares a row where it added 64. (Of fewer than 1,024 columns a block is over before that matters.)
 extern "C" int nhv_gemm_fewrows_square_rows(int M, int N, int K, int biased, int aligned) {
   using namespace fewrows;
-  if (!aligned || K < 1024 || N >= 4096 || even_rows(N) >= 16 || lines_plan(false, false, M, N, K)) return 16;
+  if (!aligned || K < 1024 || N >= 4096 || even_rows(N) >= 16 || lines_plan(false, false, false, M, N, K)) return 16;
   return tiles_plan(false, even_rows(N), biased != 0, M, N, K).ahead ? even_rows(N) : 16;
 }
 
@@ -1334,7 +1344,7 @@ int nhv_gemm_fewrows_launch(bool glu, const void* x, const void* w, const void* 
     if (glu || fused || f.band_rows % 16 != 0) return nhv_fail("few-rows gemm: bands of %d rows (multiples of 16, no gate, no fusion)", f.band_rows);
     // (8,224 outputs of 2,048 columns at 16 rows in five bands, in a trace: 14.9 us by the kernel that takes x
     // from memory, 11.9 by lines)
-    if (f.band_rows % 32 == 0 && lines_plan(false, false, M, N, K))
+    if (f.band_rows % 32 == 0 && lines_plan(false, false, false, M, N, K))
       return out_dtype == NHV_BF16 ? launch_lines<false, bf16_t>(s, x, w, bias, y, M, N, K, f) : launch_lines<false, float>(s, x, w, bias, y, M, N, K, f);
     const Plan p = plan(false, M, N, K);
     if (f.band_rows % 32 == 0 && p.nt == 2) launch<2, 8, 2, false>(s, x, w, bias, y, M, N, K, out_dtype, false, f);
@@ -1342,7 +1352,7 @@ int nhv_gemm_fewrows_launch(bool glu, const void* x, const void* w, const void* 
     return 0;
   }
   if (fused && out_dtype != NHV_BF16) return nhv_fail("few-rows gemm: a product that takes over its neighbours' work gives bfloat16");
-  if (lines_plan(glu, f.residual == nullptr, M, N, K) && !(glu && out_dtype != NHV_BF16) && !(f.residual && f.square_rows != 16)) {
+  if (lines_plan(glu, f.residual == nullptr, f.residual == nullptr && out_dtype == NHV_BF16, M, N, K) && !(glu && out_dtype != NHV_BF16) && !(f.residual && f.square_rows != 16)) {
     if (glu) return launch_lines<true, bf16_t>(s, x, w, bias, y, M, N, K, f);
     return out_dtype == NHV_BF16 ? launch_lines<false, bf16_t>(s, x, w, bias, y, M, N, K, f) : launch_lines<false, float>(s, x, w, bias, y, M, N, K, f);
   }

@@ -313,6 +313,23 @@ def test_few_rows_by_lines_whose_other_rows_are_not_there(ops, M, N, K):
         assert torch.equal(rows, more[:M])
 
 
+@pytest.mark.parametrize("M", [4, 7, 8, 11, 16])
+@pytest.mark.parametrize("N,K", [(1025, 2048), (1532, 4352), (2044, 5120), (2048, 6144)])
+def test_few_rows_by_lines_of_eight_rows_of_weights(ops, M, N, K):
+    """Blocks of 8 outputs, whose other columns are not there: against float64, with a bias; values that are no numbers in a row of x or
+    of w reach their outputs alone."""
+    x, w = rnd(M, K, dtype=torch.bfloat16, seed=108), rnd(N, K, dtype=torch.bfloat16, seed=109, scale=K ** -0.5)
+    bias = rnd(N, dtype=torch.bfloat16, seed=110)
+    want = x.double() @ w.double().T
+    torch.testing.assert_close(ops.linear(x, w).double(), want, **tol(torch.bfloat16))
+    torch.testing.assert_close(ops.linear(x, w, bias).double(), want + bias.double(), **tol(torch.bfloat16))
+    x[1, 3], w[9, 5], w[N - 1, 7] = float("nan"), float("inf"), float("nan")
+    out, hit = ops.linear(x, w), torch.zeros(M, N, dtype=torch.bool, device="cuda")
+    hit[1], hit[:, 9], hit[:, N - 1] = True, True, True
+    assert not torch.isfinite(out[hit]).any()
+    torch.testing.assert_close(out[~hit].double(), want[~hit], **tol(torch.bfloat16))
+
+
 @pytest.mark.parametrize("M,I,K", [(1, 112, 80), (5, 1001, 96), (16, 12288, 4096), (17, 160, 96), (64, 300, 1024),
                                    (4, 17408, 136), (16, 25600, 72), (13, 25000, 264), (16, 9000, 5120), (15, 520, 5384)])
 def test_gated_linear(ops, M, I, K):
