@@ -29,6 +29,7 @@
 #include "nhv_no_alloc.h"
 #include <math.h>
 #include <mutex>
+#include <type_traits>
 
 #ifndef NHV_HEAD_DIM
 #error "compile with -DNHV_HEAD_DIM=<head size>"
@@ -102,6 +103,7 @@ struct Rotated {
   const float* cos_sin;                                     // null: nothing is turned
   const int *positions, *slots;
 };
+struct AsTheyAre {};
 constexpr bool CAN_ROTATE = D >= 32 && D <= 128 && (D & (D - 1)) == 0;
 static_assert(!CAN_ROTATE || (18 * CHUNKS <= 64 * WAVES && 16 * (D + 8) * 2 <= TILE && 2 * CHUNKS <= D), "a block's threads and tiles hold 16 queries, a key and a value");
 
@@ -111,7 +113,7 @@ __global__ __launch_bounds__(64 * WAVES) void decode_attention_kernel(
     float* __restrict__ part_o, float* __restrict__ part_ml, bf16_t* __restrict__ out, const int* __restrict__ token_req,
     const int* __restrict__ positions, const int* __restrict__ block_tables, int max_blocks, int Hq, int Hkv,
     int page_size, int page_shift, float scale_log2e, int window, int split_len, int n_splits, float cap_l2, float tanh_k,
-    const float* __restrict__ slopes, const Finish finish, const Rotated rotated) {
+    const float* __restrict__ slopes, const Finish finish, const std::conditional_t<ROTATED, Rotated, AsTheyAre> rotated) {
   __shared__ __attribute__((aligned(16))) char tiles_s[WAVES][TILE];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   bf16_t* vt_s = reinterpret_cast<bf16_t*>(tiles_s[wave]);
@@ -356,13 +358,15 @@ __global__ __launch_bounds__(64 * WAVES) void decode_attention_kernel(
         for (int e = 0; e < 8; ++e) v[e] = to_f32(from_f32<bf16_t>(v[e] + b[e]));
       }
       const void* norm = is_q ? rotated.q_norm : rotated.k_norm;
-      if (is_v) {
+      if (norm && !is_v) {
+        if (rotated.float_norms) normed_head<bf16_t, float, CHUNKS>(v, (const float*)norm, rotated.eps, c);
+        else normed_head<bf16_t, bf16_t, CHUNKS>(v, (const bf16_t*)norm, rotated.eps, c);
+      }
+      if (turns && !is_v) {
+        turned_head<CHUNKS>(v, cs, sn, c, y);
+      } else {
 #pragma unroll
         for (int e = 0; e < 8; ++e) y[e] = v[e];
-      } else if (rotated.float_norms) {
-        normed_and_turned<bf16_t, float, CHUNKS>(v, (const float*)norm, rotated.eps, turns, cs, sn, c, y);
-      } else {
-        normed_and_turned<bf16_t, bf16_t, CHUNKS>(v, (const bf16_t*)norm, rotated.eps, turns, cs, sn, c, y);
       }
       if (is_q) {
         store8f<bf16_t>(q_s + item * (D + 8) + c * 8, y);
@@ -658,21 +662,21 @@ static int launch_decode_attention(const void* q, const void* k_cache, const voi
     if (page_size == (1 << b)) page_shift = b;
   dim3 grid(Hkv * ((Hq / Hkv + 15) / 16), T, n_splits);
   const float log2e = 1.4426950408889634f;
-#define NHV_DECODE_LAUNCH(...)                                                                                        \
+#define NHV_DECODE_LAUNCH(ROTATED_, ...)                                                                              \
   hipLaunchKernelGGL((decode_attention_kernel<__VA_ARGS__>), grid, dim3(64 * WAVES), 0, s, (const bf16_t*)q, (const bf16_t*)k_cache, \
                      (const bf16_t*)v_cache, part_o, part_ml, (bf16_t*)out, (const int*)token_req,                    \
                      (const int*)positions, (const int*)block_tables, max_blocks, Hq, Hkv, page_size, page_shift,     \
                      scale * log2e, window, split_len, n_splits, cap * log2e, cap > 0.f ? 2.0f * log2e * scale / cap : 0.f, \
-                     (const float*)slopes, finish, rotated ? *rotated : Rotated{})
+                     (const float*)slopes, finish, ROTATED_)
   const float sink_l2 = has_sink ? sink * log2e : -INFINITY;
   const Finish finish = {sink_l2, (const float*)sinks, (const bf16_t*)gate, gate_ld};
   if (rotated) {
-    if constexpr (CAN_ROTATE) NHV_DECODE_LAUNCH(false, false, true);
+    if constexpr (CAN_ROTATE) NHV_DECODE_LAUNCH(*rotated, false, false, true);
     else return nhv_fail("decode attention: heads of %d entries are not turned here", D);
-  } else if (cap > 0.f && slopes) NHV_DECODE_LAUNCH(true, true);
-  else if (cap > 0.f) NHV_DECODE_LAUNCH(true, false);
-  else if (slopes) NHV_DECODE_LAUNCH(false, true);
-  else NHV_DECODE_LAUNCH(false, false);
+  } else if (cap > 0.f && slopes) NHV_DECODE_LAUNCH(AsTheyAre{}, true, true);
+  else if (cap > 0.f) NHV_DECODE_LAUNCH(AsTheyAre{}, true, false);
+  else if (slopes) NHV_DECODE_LAUNCH(AsTheyAre{}, false, true);
+  else NHV_DECODE_LAUNCH(AsTheyAre{}, false, false);
 #undef NHV_DECODE_LAUNCH
   NHV_LAUNCH_CHECK("decode_attention");
   if (n_splits == 1) return 0;

@@ -162,11 +162,13 @@ __global__ __launch_bounds__(64 * WAVES) void attention_float32_kernel(FloatAtte
 #pragma unroll
           for (int e = 0; e < 8; ++e) piece[e] += b[e];
         }
-        if (of_v) {
+        const float* norm = item < group ? from_rows.q_norm : from_rows.k_norm;
+        if (norm && !of_v) normed_head<float, float, LANES>(piece, norm, from_rows.eps, lane8);
+        if (turns) {
+          turned_head<LANES>(piece, cs, sn, lane8, y);
+        } else {
 #pragma unroll
           for (int e = 0; e < 8; ++e) y[e] = piece[e];
-        } else {
-          normed_and_turned<float, float, LANES>(piece, item < group ? from_rows.q_norm : from_rows.k_norm, from_rows.eps, turns, cs, sn, lane8, y);
         }
         store8f<float>(item < group ? qs + item * (D + 4) + lane8 * 8 : (of_v ? own_v : own_k) + lane8 * 8, y);
         if (item >= group && store_at >= 0)

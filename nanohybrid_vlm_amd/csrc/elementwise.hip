@@ -484,8 +484,15 @@ __global__ __launch_bounds__(256) void qk_rope_write_vec_kernel(
     store8f<T>(v_cache + ((size_t)slot * Hkv + (h - Hq - Hkv)) * D + c * 8, v);
     return;
   }
+  const W* nw = is_q ? q_norm_w : k_norm_w;
+  if (nw) normed_head<T, W, CH>(v, nw, eps, c);
   float o[8];
-  normed_and_turned<T, W, CH>(v, is_q ? q_norm_w : k_norm_w, eps, rot > 0, cs, sn, c, o);
+  if (rot > 0) {
+    turned_head<CH>(v, cs, sn, c, o);
+  } else {
+#pragma unroll
+    for (int e = 0; e < 8; ++e) o[e] = v[e];
+  }
   T* dst = is_q ? q_out + ((size_t)t * Hq + h) * D : k_cache + ((size_t)slot * Hkv + (h - Hq)) * D;
   store8f<T>(dst + c * 8, o);
 }

@@ -1110,7 +1110,7 @@ __global__ __launch_bounds__(512) void gemm_fewrows_lines_kernel(const bf16_t* _
 // of 1,024 columns (4.2, 4.9 at 1 row) or a gated 3,072 of 1,024 (5.5, 5.7); with fewer than 2,560 outputs a tile of 16 leaves units idle,
 // which the smaller tiles above do not, until there are so many rows that these are slower: 2,560 of 4,096 7.7, 6.9 at 1 row and 7.8, 7.1 at 4;
 // 2,560 of 9,728 14.6, 14.0 and 15.3, 14.7; 3,584 of 3,584 8.5, 7.6 and 8.7, 7.8; 3,072 of 8,192 12.9, 12.0 and 13.6, 12.2; 2,048 of 6,144 8.3, 11
-// at 1 and 9.5, 11.1 at 8, but 14.3, 11.5 at 12; 2,048 of 2,048 never.
+// at 1 and 9.5, 11.1 at 8, but 14.3, 11.5 at 12; 2,048 of 2,048 never (all by blocks of 16 outputs).
 // ``even``: the tiles above would take the product, which give every unit the same rows of w (no residual, whose squares go out by tiles of
 // 16, and no bands). They stay the faster ones where the blocks of 32 outputs are a round and a bit (time by lines over theirs, K = 2,048
 // to 12,288, at 1 to 8 rows: 8,448 outputs 1.07 to 1.18, 9,216 1.07 to 1.17, 10,240 1.00 to 1.11 and at K = 2,048 0.95, 11,264 0.96 to 1.07, 12,288 0.88 to

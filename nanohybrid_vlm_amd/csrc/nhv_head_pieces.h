@@ -59,34 +59,32 @@ __device__ __forceinline__ void add_parts8(const float* p, size_t stride, int sp
   else add_parts8<1>(p, stride, out);
 }
 
-// A head of 8 CH entries in CH lanes, lane c of it with v = entries 8 c ...: divided by its root mean square and multiplied by its
-// weight (nw; none: null), each rounded, then turned by halves (cs, sn: the cosines and sines of entries 8 c ... modulo the half).
-// The norm's sum and the rotation's partner come by shuffles: the lanes of a head come here together.
+// A head of 8 CH entries in CH lanes, lane c of it with v = entries 8 c ...: the norm's sum and the rotation's partner come by shuffles, so the
+// lanes of a head come here together.
+// Divided by its root mean square and multiplied by its weight, each rounded.
 template <typename T, typename W, int CH>
-__device__ __forceinline__ void normed_and_turned(float* v, const W* nw, float eps, bool turns, const float* cs, const float* sn, int c,
-                                                  float* o) {
-  constexpr int D = CH * 8, HALF_LANES = CH / 2 > 0 ? CH / 2 : 1;
-  if (nw) {
-    float ss = 0.f;
+__device__ __forceinline__ void normed_head(float* v, const W* nw, float eps, int c) {
+  constexpr int D = CH * 8;
+  float ss = 0.f;
 #pragma unroll
-    for (int e = 0; e < 8; ++e) ss += v[e] * v[e];
+  for (int e = 0; e < 8; ++e) ss += v[e] * v[e];
 #pragma unroll
-    for (int off = 1; off < CH; off <<= 1) ss += __shfl_xor(ss, off, NHV_WAVE);
-    const float r = 1.0f / sqrtf(ss / (float)D + eps);
-    float wv[8];
-    load8f<W>(nw + c * 8, wv);
+  for (int off = 1; off < CH; off <<= 1) ss += __shfl_xor(ss, off, NHV_WAVE);
+  const float r = 1.0f / sqrtf(ss / (float)D + eps);
+  float wv[8];
+  load8f<W>(nw + c * 8, wv);
 #pragma unroll
-    for (int e = 0; e < 8; ++e) v[e] = to_f32(from_f32<T>(to_f32(from_f32<T>(v[e] * r)) * wv[e]));
-  }
-  if (turns) {
-    const bool first_half = c < HALF_LANES;
+  for (int e = 0; e < 8; ++e) v[e] = to_f32(from_f32<T>(to_f32(from_f32<T>(v[e] * r)) * wv[e]));
+}
+
+// Turned by halves: cs, sn are the cosines and sines of entries 8 c ... modulo the half.
+template <int CH>
+__device__ __forceinline__ void turned_head(const float* v, const float* cs, const float* sn, int c, float* o) {
+  constexpr int HALF_LANES = CH / 2 > 0 ? CH / 2 : 1;
+  const bool first_half = c < HALF_LANES;
 #pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      const float partner = __shfl_xor(v[e], HALF_LANES, NHV_WAVE);
-      o[e] = first_half ? v[e] * cs[e] - partner * sn[e] : v[e] * cs[e] + partner * sn[e];
-    }
-  } else {
-#pragma unroll
-    for (int e = 0; e < 8; ++e) o[e] = v[e];
+  for (int e = 0; e < 8; ++e) {
+    const float partner = __shfl_xor(v[e], HALF_LANES, NHV_WAVE);
+    o[e] = first_half ? v[e] * cs[e] - partner * sn[e] : v[e] * cs[e] + partner * sn[e];
   }
 }
