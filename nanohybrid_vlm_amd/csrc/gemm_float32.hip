@@ -251,19 +251,21 @@ static void launch(const float* x, const float* w, const float* bias, float* y, 
   const dim3 grid(8u * (unsigned)(((long long)m_tiles * n_tiles + 7) / 8), PARTS ? (segments(K) + 1) / 2 : 1), block(PARTS ? 128 : 64 * SEGMENTS);
   if (PARTS || (K % 4 == 0 && (uintptr_t)x % 16 == 0 && (uintptr_t)w % 16 == 0))
     hipLaunchKernelGGL((gemm_float32_kernel<RT, CT, U, GATED, PARTS, true>), grid, block, 0, s, x, w, bias, y, M, N, K, m_tiles, n_tiles, gate);
-  else
+  else if constexpr (!PARTS)
     hipLaunchKernelGGL((gemm_float32_kernel<RT, CT, U, GATED, false, false>), grid, block, 0, s, x, w, bias, y, M, N, K, m_tiles, n_tiles, gate);
 }
 
 // ---------------------------------------------------------------- many rows
 // 4 waves, 2 x 2, a wave RT x CT tiles of 16 x 16; the parts of both operands through LDS in pieces of 32 k, two buffers, two
 // pieces under way in registers: an entry is taken apart once a block. A wave takes every segment in turn and adds it to the
-// total: the same sums in the same order as above. What bounds it is a block's chain of pieces (0.4 us each at 32 x 32); for the middling
-// numbers of rows and outputs whose larger tiles would leave units idle.
+// total: the same sums in the same order as above. What bounds it is a block's chain of pieces (0.4 us each at 32 x 32). 32 x 32: for the
+// middling numbers of rows and outputs whose larger tiles would leave units idle. 64 x 64: for more of them in rows that are not whole pieces of
+// 32 columns on 16-byte boundaries, which the kernel below does not take: made to, it took 1,024 x 3072 . 1001 in 140 us and 517 x
+// 4096 . 1176 in 55 (gated 104) where this one takes 85 and 56 (95).
 #define PIECE 32
 #define AHEAD 2
 template <int RT, int CT, bool GATED, bool WIDE>
-__global__ __launch_bounds__(256, 4) void gemm_float32_tiles_kernel(const float* __restrict__ x, const float* __restrict__ w,
+__global__ __launch_bounds__(256, RT * CT > 2 ? 3 : 4) void gemm_float32_tiles_kernel(const float* __restrict__ x, const float* __restrict__ w,
                                                                  const float* __restrict__ bias, float* __restrict__ y, int M, int N,
                                                                  int K, int m_tiles, int n_tiles, NhvGate gate) {
   static_assert(!GATED || CT == 2, "a gate tile and its up tile");
@@ -409,13 +411,12 @@ static void launch_tiles(const float* x, const float* w, const float* bias, floa
 // the like (by / 2: 8 % slower). Asked for LDS one piece ahead, with two barriers or a third buffer, it was no faster.
 // us, tiles of 64 x 64 of 16x16x32 instructions in brackets: 517 x 4096 . 1024 47 (53), gated 517 x 3072 . 1024 56 (67), 300 x 6144 . 2048 106 (140),
 // 1,500 x 12,288 . 2048 454 (550).
-// WHOLE: K a multiple of 32, rows on 16-byte boundaries.
-template <int CT, bool GATED, bool PARTS, bool WHOLE>
+// Rows are whole pieces of 32 columns on 16-byte boundaries (whole_pieces).
+template <int CT, bool GATED, bool PARTS>
 __global__ __launch_bounds__(256, CT == 2 ? 2 : 3) void gemm_float32_blocks_kernel(const float* __restrict__ x, const float* __restrict__ w,
                                                                                    const float* __restrict__ bias, float* __restrict__ y, int M, int N,
                                                                                    int K, int m_tiles, int n_tiles, NhvGate gate) {
   static_assert(!GATED || (CT == 2 && !PARTS), "a gate tile and its up tile");
-  static_assert(!PARTS || WHOLE, "parts of whole pieces");
   constexpr int BM = 64, BN = 64 * CT, LOADS = (BM + BN) / 64, PLANE = (BM + BN) * PIECE, OUT = GATED ? BN / 2 : BN, TOTALS = PARTS ? 1 : CT;
   __shared__ __attribute__((aligned(16))) bf16_t rows[2][3 * PLANE];
   const int total_tiles = m_tiles * n_tiles, share = (total_tiles + 7) >> 3;
@@ -426,7 +427,7 @@ __global__ __launch_bounds__(256, CT == 2 ? 2 : 3) void gemm_float32_blocks_kern
   const int mw = (wave >> 1) * 32, nw = (wave & 1) * 32 * CT;
   const int length = segment_length(K), begin = PARTS ? blockIdx.y * length : 0, end = PARTS ? min(K, begin + length) : K;
   // what this thread brings of a piece: 16 bytes of each half of the 128 of rows row, row + 64, ...: an address that the wave shares, and
-  // an offset of less than 2^32
+  // an offset (of less than 128 rows of less than 2^22 entries: 32 bits)
   const int col = (threadIdx.x & 3) * 4, row = threadIdx.x >> 2;
   const float* base[LOADS];
   uint32_t offset[LOADS];
@@ -441,12 +442,11 @@ __global__ __launch_bounds__(256, CT == 2 ? 2 : 3) void gemm_float32_blocks_kern
   const int to_row = row * PIECE + (((threadIdx.x & 3) ^ (row >> 2 & 3)) << 3);
   f32x4 hold[AHEAD][LOADS][2];
   auto ask = [&](int i_hold, int k0) {
-    const int at = WHOLE ? min(k0, K - PIECE) : k0;        // (beyond the last piece it again, into registers that nobody reads)
+    const int at = min(k0, K - PIECE);                     // (beyond the last piece it again, into registers that nobody reads)
 #pragma unroll
     for (int i = 0; i < LOADS; ++i)
 #pragma unroll
-      for (int h = 0; h < 2; ++h)
-        hold[i_hold][i][h] = WHOLE ? *reinterpret_cast<const f32x4*>(base[i] + at + (offset[i] + col + 16 * h)) : four_of<false>(base[i] + offset[i], at + col + 16 * h, K);
+      for (int h = 0; h < 2; ++h) hold[i_hold][i][h] = *reinterpret_cast<const f32x4*>(base[i] + at + (offset[i] + col + 16 * h));
   };
   auto put = [&](int buf, int i_hold, int i) {
     const SplitFloats8 p = split_floats(hold[i_hold][i][0], hold[i_hold][i][1]);
@@ -574,10 +574,11 @@ static void launch_blocks(const float* x, const float* w, const float* bias, flo
   constexpr int COLS = GATED ? 32 * CT : 64 * CT;
   const int m_tiles = (M + 63) / 64, n_tiles = (N + COLS - 1) / COLS;
   const dim3 grid(8u * (unsigned)(((long long)m_tiles * n_tiles + 7) / 8), PARTS ? segments(K) : 1), block(256);
-  if (PARTS || (K % PIECE == 0 && K < (1 << 22) && (uintptr_t)x % 16 == 0 && (uintptr_t)w % 16 == 0))
-    hipLaunchKernelGGL((gemm_float32_blocks_kernel<CT, GATED, PARTS, true>), grid, block, 0, s, x, w, bias, y, M, N, K, m_tiles, n_tiles, gate);
-  else
-    hipLaunchKernelGGL((gemm_float32_blocks_kernel<CT, GATED, false, false>), grid, block, 0, s, x, w, bias, y, M, N, K, m_tiles, n_tiles, gate);
+  hipLaunchKernelGGL((gemm_float32_blocks_kernel<CT, GATED, PARTS>), grid, block, 0, s, x, w, bias, y, M, N, K, m_tiles, n_tiles, gate);
+}
+
+static bool whole_pieces(const void* x, const void* w, int K) {
+  return K % PIECE == 0 && K < (1 << 22) && (((uintptr_t)x | (uintptr_t)w) & 15) == 0;
 }
 
 // Every tile's time in units of what a compute unit needs for 16 rows of an operand, from the times of all tiles at 1 to 1,500
@@ -585,35 +586,35 @@ static void launch_blocks(const float* x, const float* w, const float* bias, flo
 // LDS: a floor (one block's chain of pieces) and what a block a compute unit adds (64 x 128: whole rounds). E.g. 17 x 6144 . 1024: 32 x 32 10.1 us,
 // 16 x 32 14.0, 16 x 16 13.9; 130 x 2048 . 2048: 48 x 32 21.9 us, 32 x 32 33.7, 64 x 64 42.4; 517 x 4096 . 1024: 64 x 64 46, 64 x 128 50, 32 x 32
 // through LDS 56; 1,500 x 4096 . 1024: 98, 90 and 147. Up to 16 rows LDS has nothing to share and is left out (6 x 151,936 . 1024: 116 us with 16 x 32,
-// 135 through LDS).
+// 135 through LDS). Not whole pieces: 64 x 64 of 16x16x32 instructions in place of both.
 // 32 x 16, whose second 16 rows are few different ones at 17 rows and 16 at 32: 17 x 4096 . 4096 24.2 us, 16 x 32 27.4; 32 rows 29.2 and 28.1.
 struct Choice {
   int tile;
   double cost;
 };
 static double wide_tiles(long long blocks) { return fmax(15.2, 13.3 * (blocks <= 2048 ? (double)((blocks + 255) / 256) : blocks / 256.0) - 1.5); }
-static Choice plain_tile(long long M, long long N) {
+static Choice plain_tile(long long M, long long N, bool whole) {
   auto blocks = [&](long long m, long long n) { return ((M + m - 1) / m) * ((N + n - 1) / n); };
   auto rounds = [&](int rt, int ct) { return (double)((blocks(16 * rt, 16 * ct) + 255) / 256 * (rt + ct)); };
   const double none = 1e300;
   const double cost[8] = {rounds(1, 1), rounds(1, 2), M > 16 ? rounds(2, 2) : none, M > 32 ? rounds(3, 2) : none,
                           M > 16 ? fmax(9.0, 1.5 + 2.9 / 256 * blocks(32, 32)) : none,
-                          M > 16 ? fmax(11.5, 6.0 + 7.7 / 256 * blocks(64, 64)) : none,
+                          M > 16 ? fmax(11.5, (whole ? 6.0 : 4.5) + 7.7 / 256 * blocks(64, 64)) : none,
                           M > 16 && M <= 32 ? rounds(2, 1) / 3 * (2.05 + 0.035 * M) : none,
-                          M > 16 ? wide_tiles(blocks(64, 128)) : none};
+                          M > 16 && whole ? wide_tiles(blocks(64, 128)) : none};
   Choice best = {0, cost[0]};
   for (int i = 1; i < 8; ++i)
     if (cost[i] < best.cost) best = {i, cost[i]};
   return best;
 }
 // a gate of two products: a column counting for two rows of w; through LDS only tiles with a pair a wave
-static Choice gated_tile(long long M, long long N) {
+static Choice gated_tile(long long M, long long N, bool whole) {
   auto blocks = [&](long long m, long long n) { return ((M + m - 1) / m) * ((N + n - 1) / n); };
   auto rounds = [&](int rt) { return (double)((blocks(16 * rt, 16) + 255) / 256 * (rt + 2)); };
   const double none = 1e300;
   const double cost[5] = {rounds(1), M > 16 ? rounds(2) : none, M > 32 ? rounds(3) : none,
                           M > 16 ? fmax(9.5, 3.0 + 4.9 / 256 * blocks(32, 32)) : none,
-                          M > 16 ? wide_tiles(blocks(64, 64)) : none};
+                          M <= 16 ? none : whole ? wide_tiles(blocks(64, 64)) : fmax(11.5, 4.5 + 7.7 / 256 * blocks(64, 32))};
   Choice best = {0, cost[0]};
   for (int i = 1; i < 5; ++i)
     if (cost[i] < best.cost) best = {i, cost[i]};
@@ -626,13 +627,17 @@ extern "C" int nhv_gemm_float32(const void* x, const void* w, const void* bias, 
   hipStream_t s = (hipStream_t)stream;
   const float *xf = (const float*)x, *wf = (const float*)w, *bf = (const float*)bias;
   float* yf = (float*)y;
-  switch (plain_tile(M, N).tile) {
+  const bool whole = whole_pieces(x, w, K);
+  switch (plain_tile(M, N, whole).tile) {
     case 0: launch<1, 1, 2, false>(xf, wf, bf, yf, M, N, K, {}, s); break;
     case 1: launch<1, 2, 1, false>(xf, wf, bf, yf, M, N, K, {}, s); break;
     case 2: launch<2, 2, 1, false>(xf, wf, bf, yf, M, N, K, {}, s); break;
     case 3: launch<3, 2, 1, false>(xf, wf, bf, yf, M, N, K, {}, s); break;
     case 4: launch_tiles<1, 1, false>(xf, wf, bf, yf, M, N, K, {}, s); break;
-    case 5: launch_blocks<1, false>(xf, wf, bf, yf, M, N, K, {}, s); break;
+    case 5:
+      if (whole) launch_blocks<1, false>(xf, wf, bf, yf, M, N, K, {}, s);
+      else launch_tiles<2, 2, false>(xf, wf, bf, yf, M, N, K, {}, s);
+      break;
     case 7: launch_blocks<2, false>(xf, wf, bf, yf, M, N, K, {}, s); break;
     default: launch<2, 1, 2, false>(xf, wf, bf, yf, M, N, K, {}, s);
   }
@@ -646,7 +651,7 @@ extern "C" int nhv_gemm_float32(const void* x, const void* w, const void* bias, 
 // 11.4; 130 rows, 1024 . 3072 24.5, 14.7, 2048 . 6144 56.7, 37, 4096 . 2048 41.6, 28.4; 517 rows, 1024 . 2048 43, 24.4, 1024 . 3072 61.6, 33, 2048 . 6144 156, 101.
 // The reader then takes in 8 entries for one, at 4 TB/s (517 x 2048 7 us), which 517 x 4096 . 2048 (87 and 77) and 1,500 x 2048 . 2048 (98 and 97) lose by.
 extern "C" int nhv_gemm_float32_parts_count(const void* x, const void* w, int M, int N, int K) {
-  const bool whole = M > 0 && N > 0 && K % PIECE == 0 && K >= 512 && K < (1 << 22) && (uintptr_t)x % 16 == 0 && (uintptr_t)w % 16 == 0;
+  const bool whole = M > 0 && N > 0 && K >= 512 && whole_pieces(x, w, K);
   return whole && (M <= 16 ? N <= 2560 : (long long)M * N <= 1200000) ? segments(K) : 0;
 }
 
@@ -782,7 +787,8 @@ extern "C" int nhv_sum_parts_float32(const void* parts, int count, const void* x
 // entry by entry (1,000 of 1,001 at 1 row 20.8 and 13.4), the gate's kernel 2 and more (in a recorded step 4).
 extern "C" int nhv_gemm_float32_gated_pays(const void* x, const void* w, int M, int N, int K) {
   const bool wide = K % 4 == 0 && (uintptr_t)x % 16 == 0 && (uintptr_t)w % 16 == 0;
-  return (gated_tile(M, N).cost - plain_tile(M, 2ll * N).cost) * (wide ? 5.6 : 28.0) * K / 3072 <= 2.0;
+  const bool whole = whole_pieces(x, w, K);
+  return (gated_tile(M, N, whole).cost - plain_tile(M, 2ll * N, whole).cost) * (wide ? 5.6 : 28.0) * K / 3072 <= 2.0;
 }
 
 extern "C" int nhv_gemm_float32_gated(const void* x, const void* w, const void* bias, void* y, int M, int N, int K, int act, float limit,
@@ -795,12 +801,15 @@ extern "C" int nhv_gemm_float32_gated(const void* x, const void* w, const void* 
   const NhvGate gate = {act, limit, alpha, offset};
   const float *xf = (const float*)x, *wf = (const float*)w, *bf = (const float*)bias;
   float* yf = (float*)y;
-  switch (gated_tile(M, N).tile) {
+  const bool whole = whole_pieces(x, w, K);
+  switch (gated_tile(M, N, whole).tile) {
     case 0: launch<1, 2, 1, true>(xf, wf, bf, yf, M, N, K, gate, s); break;
     case 1: launch<2, 2, 1, true>(xf, wf, bf, yf, M, N, K, gate, s); break;
     case 2: launch<3, 2, 1, true>(xf, wf, bf, yf, M, N, K, gate, s); break;
     case 3: launch_tiles<1, 2, true>(xf, wf, bf, yf, M, N, K, gate, s); break;
-    default: launch_blocks<2, true>(xf, wf, bf, yf, M, N, K, gate, s);
+    default:
+      if (whole) launch_blocks<2, true>(xf, wf, bf, yf, M, N, K, gate, s);
+      else launch_tiles<2, 2, true>(xf, wf, bf, yf, M, N, K, gate, s);
   }
   NHV_LAUNCH_CHECK("gemm_float32_gated");
   return 0;
