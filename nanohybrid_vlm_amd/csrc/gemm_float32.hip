@@ -142,9 +142,9 @@ __global__ __launch_bounds__(PARTS ? 128 : 64 * SEGMENTS) void gemm_float32_kern
     auto sum = [&](int buf, int u) {
       SplitFloats8 xs[RT], ws[CT];
 #pragma unroll
-      for (int c = 0; c < CT; ++c) ws[c] = split_floats(b[buf][u][c][0], b[buf][u][c][1]);
+      for (int c = 0; c < CT; ++c) ws[c] = split_floats<true>(b[buf][u][c][0], b[buf][u][c][1]);
 #pragma unroll
-      for (int r = 0; r < RT; ++r) xs[r] = split_floats(a[buf][u][r][0], a[buf][u][r][1]);
+      for (int r = 0; r < RT; ++r) xs[r] = split_floats<true>(a[buf][u][r][0], a[buf][u][r][1]);
 #pragma unroll
       for (int step = 0; step < 6; ++step)
 #pragma unroll
@@ -305,7 +305,7 @@ __global__ __launch_bounds__(256, RT * CT > 2 ? 3 : 4) void gemm_float32_tiles_k
     }
 #pragma unroll
     for (int i = 0; i < LOADS; ++i) {
-      const SplitFloats4 p = split_floats(hold[i_hold][i]);
+      const SplitFloats4 p = split_floats<true>(hold[i_hold][i]);
       bf16_t* to = &rows[buf][32 * i * PIECE + to_row];
       *reinterpret_cast<bf16x4*>(to) = p.high;
       *reinterpret_cast<bf16x4*>(to + PLANE) = p.middle;
@@ -449,7 +449,7 @@ __global__ __launch_bounds__(256, CT == 2 ? 2 : 3) void gemm_float32_blocks_kern
       for (int h = 0; h < 2; ++h) hold[i_hold][i][h] = *reinterpret_cast<const f32x4*>(base[i] + at + (offset[i] + col + 16 * h));
   };
   auto put = [&](int buf, int i_hold, int i) {
-    const SplitFloats8 p = split_floats(hold[i_hold][i][0], hold[i_hold][i][1]);
+    const SplitFloats8 p = split_floats<false>(hold[i_hold][i][0], hold[i_hold][i][1]);
     bf16_t* to = &rows[buf][64 * i * PIECE + to_row];
     *reinterpret_cast<bf16x8*>(to) = p.high;
     *reinterpret_cast<bf16x8*>(to + PLANE) = p.middle;

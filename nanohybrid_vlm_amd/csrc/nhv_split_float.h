@@ -22,23 +22,37 @@ constexpr float SPLIT_UNSCALE = 0x1p-32f;                // of a sum of products
 struct SplitFloats4 { bf16x4 high, middle, rest; };
 struct SplitFloats8 { bf16x8 high, middle, rest; };
 
-// (a, b) rounded to bfloat16, and what that leaves of them in their place. (A dot product with (-1, 0) is one instruction where
-// the widening and the subtraction are two, but it does not run beside matrix instructions, which these do: 1,500 x 12,288 . 2048
-// 488 us with dot products, 468 without.)
+// (a, b) rounded to bfloat16, and what that leaves of them in their place, exactly either way.
+// DOTS: by a dot product with (-1, 0), one instruction where the widening and the subtraction are two. (The two pairs come from scalar
+// registers that the compiler does not see through: it would write the first as the inline constant -1.0, which the instruction reads
+// as another pair, and every first entry's parts came out wrong.) It does not run beside matrix instructions, which the two do where
+// these leave room: 32x32x16 ones (1,500 x 12,288 . 2048 454 us, with dots 20 more), not the 16x16x32 ones of the other kernels
+// (6 x 2048 . 2048 9.4 us without dots, 8.7 with; 1 x 2048 . 6144 18.8, 17.6; 20 x 3072 . 1001, whose loads the compiler then leaves in
+// scratch memory, 46 and 16).
+template <bool DOTS>
 __device__ __forceinline__ bf16x2 take_high(float& a, float& b) {
   const bf16x2 high = __builtin_convertvector((f32x2{a, b}), bf16x2);
-  const uint32_t bits = __builtin_bit_cast(uint32_t, high);
-  a -= __builtin_bit_cast(float, bits << 16);
-  b -= __builtin_bit_cast(float, bits & 0xffff0000u);
+  if constexpr (DOTS) {
+    uint32_t first = 0x0000bf80u, second = 0xbf800000u;
+    asm("" : "+s"(first));
+    asm("" : "+s"(second));
+    a = __builtin_amdgcn_fdot2_f32_bf16(high, __builtin_bit_cast(bf16x2, first), a, false);
+    b = __builtin_amdgcn_fdot2_f32_bf16(high, __builtin_bit_cast(bf16x2, second), b, false);
+  } else {
+    const uint32_t bits = __builtin_bit_cast(uint32_t, high);
+    a -= __builtin_bit_cast(float, bits << 16);
+    b -= __builtin_bit_cast(float, bits & 0xffff0000u);
+  }
   return high;
 }
 
+template <bool DOTS>
 __device__ __forceinline__ SplitFloats4 split_floats(f32x4 v) {
   SplitFloats4 p;
 #pragma unroll
   for (int i = 0; i < 4; i += 2) {
     float a = v[i] * SPLIT_SCALE, b = v[i + 1] * SPLIT_SCALE;
-    const bf16x2 high = take_high(a, b), middle = take_high(a, b), rest = __builtin_convertvector((f32x2{a, b}), bf16x2);
+    const bf16x2 high = take_high<DOTS>(a, b), middle = take_high<DOTS>(a, b), rest = __builtin_convertvector((f32x2{a, b}), bf16x2);
     p.high[i] = high[0], p.high[i + 1] = high[1];
     p.middle[i] = middle[0], p.middle[i + 1] = middle[1];
     p.rest[i] = rest[0], p.rest[i + 1] = rest[1];
@@ -46,8 +60,9 @@ __device__ __forceinline__ SplitFloats4 split_floats(f32x4 v) {
   return p;
 }
 
+template <bool DOTS>
 __device__ __forceinline__ SplitFloats8 split_floats(f32x4 v0, f32x4 v1) {
-  const SplitFloats4 p = split_floats(v0), q = split_floats(v1);
+  const SplitFloats4 p = split_floats<DOTS>(v0), q = split_floats<DOTS>(v1);
   return {__builtin_shufflevector(p.high, q.high, 0, 1, 2, 3, 4, 5, 6, 7),
           __builtin_shufflevector(p.middle, q.middle, 0, 1, 2, 3, 4, 5, 6, 7),
           __builtin_shufflevector(p.rest, q.rest, 0, 1, 2, 3, 4, 5, 6, 7)};
