@@ -592,6 +592,12 @@ struct Choice {
   int tile;
   double cost;
 };
+// 64 x 64 of whole pieces: one block a unit, two, three; beyond, what a block adds (1,000 x 1024 . 3072 62 us, 32 x 32 through LDS 76; 256 x 4096 .
+// 4096 83 and 102; 130 x 6144 . 2048 58 and 53; 700 x 2048 . 2048 59, 64 x 128 55).
+static double square_tiles(long long blocks) {
+  const double a_unit = blocks / 256.0;
+  return a_unit <= 1 ? 11.2 : a_unit <= 2 ? 12.0 + 2.75 * a_unit : a_unit <= 3 ? 13.5 + 3.8 * a_unit : 1.8 + 7.7 * a_unit;
+}
 static double wide_tiles(long long blocks) { return fmax(15.2, 13.3 * (blocks <= 2048 ? (double)((blocks + 255) / 256) : blocks / 256.0) - 1.5); }
 static Choice plain_tile(long long M, long long N, bool whole) {
   auto blocks = [&](long long m, long long n) { return ((M + m - 1) / m) * ((N + n - 1) / n); };
@@ -599,7 +605,7 @@ static Choice plain_tile(long long M, long long N, bool whole) {
   const double none = 1e300;
   const double cost[8] = {rounds(1, 1), rounds(1, 2), M > 16 ? rounds(2, 2) : none, M > 32 ? rounds(3, 2) : none,
                           M > 16 ? fmax(9.0, 1.5 + 2.9 / 256 * blocks(32, 32)) : none,
-                          M > 16 ? fmax(11.5, (whole ? 6.0 : 4.5) + 7.7 / 256 * blocks(64, 64)) : none,
+                          M <= 16 ? none : whole ? square_tiles(blocks(64, 64)) : fmax(11.5, 4.5 + 7.7 / 256 * blocks(64, 64)),
                           M > 16 && M <= 32 ? rounds(2, 1) / 3 * (2.05 + 0.035 * M) : none,
                           M > 16 && whole ? wide_tiles(blocks(64, 128)) : none};
   Choice best = {0, cost[0]};
