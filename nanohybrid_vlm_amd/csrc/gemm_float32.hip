@@ -652,13 +652,18 @@ extern "C" int nhv_gemm_float32(const void* x, const void* w, const void* bias, 
 }
 
 // ---------------------------------------------------------------- parts that their reader adds up
-// How many parts (the segments of K) a product is best left in for a reader that adds them up; 0: it is best finished here. us, cold
-// weights, finished and in parts: 6 rows, 1024 . 2048 8.7, 6.5, 1024 . 3072 11.6, 7.0, 2048 . 6144 19.2, 15.0, but 4096 . 2048 8.9, 9.6; 65 rows, 1024 . 3072 18.8,
-// 11.4; 130 rows, 1024 . 3072 24.5, 14.7, 2048 . 6144 56.7, 37, 4096 . 2048 41.6, 28.4; 517 rows, 1024 . 2048 43, 24.4, 1024 . 3072 61.6, 33, 2048 . 6144 156, 101.
-// The reader then takes in 8 entries for one, at 4 TB/s (517 x 2048 7 us), which 517 x 4096 . 2048 (87 and 77) and 1,500 x 2048 . 2048 (98 and 97) lose by.
+// How many parts (the segments of K) a product is best left in for a reader that adds them up; 0: it is best finished here. What K over more
+// blocks saves grows with K and is little where outputs alone make blocks enough; what it costs are the parts' way to memory and
+// back, 8 entries for one at 4 TB/s. us of the product (cold weights) and the norm behind it, finished and in parts: 6 rows, 1024 . 2048 11.5, 8.9, 1024
+// . 3072 13.9, 9.5, 2048 . 6144 23.2, 19.6, but 2560 . 1024 9.2, 9.9, 1536 . 512 7.4, 7.9, 4096 . 2048 13.7, 15.8; 17 rows, 2560 . 4096 24.3, 23.3, 4096 . 12288 60.6,
+// 59.5, but 4096 . 4096 25.2, 28.0; 40 rows, 5120 . 5120 54.9, 42.4, but 8192 . 8192 89, 104; 130 rows, 1024 . 3072 28.0, 20.0, 2048 . 6144 61, 45, but 2048 . 512
+// 12.8, 16.0; 517 rows, 1024 . 2048 46.5, 31.4, 2048 . 6144 192, 122, but 2048 . 512 27.8, 31.3; 1,000 rows, 1024 . 2048 51.9, 47.5, but 1024 . 512 22.2, 28.6
+// and 1024 . 1024 32.0, 34.3; 450 rows, 4096 . 2048 (in parts 9 % longer).
 extern "C" int nhv_gemm_float32_parts_count(const void* x, const void* w, int M, int N, int K) {
   const bool whole = M > 0 && N > 0 && K >= 512 && whole_pieces(x, w, K);
-  return whole && (M <= 16 ? N <= 2560 : (long long)M * N <= 1200000) ? segments(K) : 0;
+  const int most = M <= 16 ? 2560 : M <= 32 ? (K >= 2ll * N ? 4096 : 2560) : M <= 48 ? 5120 : 1200000 / M;
+  const bool pays = N <= most && (M <= 16 ? 2ll * K > N : K >= 2048 && (long long)M * N <= 1200000);
+  return whole && pays ? segments(K) : 0;
 }
 
 // y[segments][M][N], times 2^32. Up to 16 rows two waves a block, each with all of a segment under way (one with half of it: 8.1 us where 7.0
