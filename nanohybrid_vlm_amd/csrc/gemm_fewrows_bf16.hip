@@ -1106,26 +1106,35 @@ __global__ __launch_bounds__(512) void gemm_fewrows_lines_kernel(const bf16_t* _
   if ((threadIdx.x & 15) == 0 && row < M && my_tile < tiles) f.ss_out[(size_t)row * tiles + my_tile] = sq;
 }
 
+// Blocks of 8 outputs, by lines. us by the tiles above (M = 12 and more, 2,048 outputs: by lines of 16 rows) and by those, of 2,048 outputs: of 2,048
+// columns at 4, 8 and 16 rows 4.9, 4.9, 5.2 and 4.8, 4.8, 4.9; of 3,072 at 4 and 7 rows 5.9, 6.0 and 5.7, 5.7; of 4,096 6.9, 7.2 and 6.6, 6.8; of
+// 5,120 7.8, 8.1 and 7.7, 7.8; of 6,144 at 4, 8 and 16 rows 8.5, 9.3, 10.3 and 9.9, 8.7, 9.1; of 12,288 13.8, 16.9, 17.5 and 16.8, 14.7, 15.2; 1,280 of 4,096 6.2,
+// 6.7, 7.7 and 6.3, 6.4, 6.5; 1,040 of 2,560 at 4 and 6 rows 5.0, 5.1 and 5.2, 5.0. ``scaled`` (x a sum whose rows lack their norm's scales): these cost
+// such a block 0.5 us more and the tiles 0.1; 2,048 of 2,048 at 4, 8 and 16 rows 5.0, 5.2, 5.7 and 5.6, 5.6, 5.8; 1,536 of 3,072 at 4, 6 and 8 rows 6.1, 6.4, 6.5 and
+// 6.1, 6.2, 6.2; 1,280 of 3,072 at 8, 12 and 16 rows 6.1, 6.4, 6.7 and 6.2, 6.3, 6.4; 1,040 of 4,096 at 4 and 8 rows 6.6, 7.1 and 6.9, 6.9.
+static bool half_plan(bool scaled, int M, int N, int K) {
+  if (N <= 1024 || N > 2048) return false;
+  if (scaled) return (M >= 6 && K <= 5120 && (long long)N * K >= 1536 * 3072) || (K >= 3072 && M >= (K >= 4096 ? 8 : 12));
+  return M >= 8 || (M >= 4 && K <= 5120 && (M >= 6 || N >= 1280 || K <= 2048));
+}
+
 // Where the rows of w are enough for it, by what was measured at 1, 4, 8, 12 and 16 rows (us before and with it): not for 4,096 outputs
 // of 1,024 columns (4.2, 4.9 at 1 row) or a gated 3,072 of 1,024 (5.5, 5.7); with fewer than 2,560 outputs a tile of 16 leaves units idle,
 // which the smaller tiles above do not, until there are so many rows that these are slower: 2,560 of 4,096 7.7, 6.9 at 1 row and 7.8, 7.1 at 4;
 // 2,560 of 9,728 14.6, 14.0 and 15.3, 14.7; 3,584 of 3,584 8.5, 7.6 and 8.7, 7.8; 3,072 of 8,192 12.9, 12.0 and 13.6, 12.2; 2,048 of 6,144 8.3, 11
 // at 1 and 9.5, 11.1 at 8, but 14.3, 11.5 at 12; 2,048 of 2,048 never (all by blocks of 16 outputs).
-// ``even``: the tiles above would take the product, which give every unit the same rows of w (no residual, whose squares go out by tiles of
-// 16, and no bands). They stay the faster ones where the blocks of 32 outputs are a round and a bit (time by lines over theirs, K = 2,048
+// ``even``: the tiles above would take the product and give every unit the same rows of w (with a residual they do so for fewer than 4,096 outputs
+// alone, see nhv_gemm_fewrows_square_rows; with bands never). They stay the faster ones where the blocks of 32 outputs are a round and a bit (time by lines over theirs, K = 2,048
 // to 12,288, at 1 to 8 rows: 8,448 outputs 1.07 to 1.18, 9,216 1.07 to 1.17, 10,240 1.00 to 1.11 and at K = 2,048 0.95, 11,264 0.96 to 1.07, 12,288 0.88 to
 // 1.04; 16 rows: K = 3,072 1.05 to 1.15, from 4,096 on 0.62 to 0.88), and with rows 16 KB apart on some of the units (K = 8,192: 4,224
 // to 6,144 outputs 1.06 to 1.22 at 1 to 4 rows, 0.81 to 0.99 at 8; 7,168 outputs 0.80 to 0.87), as long as all of x fits beside w.
-// ``half``: a bfloat16 result without residual, which 8 rows of w a block can make. us by the tiles above (M = 12 and more, 2,048 outputs: by
-// lines of 16 rows) and by those, of 2,048 outputs: of 2,048 columns at 4, 8 and 16 rows 5.2, 5.1, 5.7 and 4.8, 4.8, 5.0; of 6,144 9.0,
-// 9.9, 11.2 and 9.9, 9.9, 9.0 to 10.0; of 12,288 14.7, 18.7, 19.3 and 16.8, 16.7, 17.2 (10 rows 22.1, 16.6); 1,536 of 8,960 11.5, 12.5, 21.1 and 11.9, 11.8,
-// 11.3; 1,280 of 5,120 7.6, 8.2, 14.0 and 7.5, 7.4, 7.5; 1,040 of 2,048 4.7, 4.7, 5.0 and 4.5, 4.5, 4.6 (1 row 4.2, 4.5).
-static bool lines_plan(bool glu, bool even, bool half, int M, int N, int K) {
+// ``half``: a bfloat16 result without residual, which 8 rows of w a block can make (half_plan).
+static bool lines_plan(bool glu, bool even, bool half, bool scaled, int M, int N, int K) {
   if (K % 256 != 0 || K < 2048) return false;
   if (glu) return N >= 4096;
   if (even && N > 8192 && N <= (K > 2048 ? 11264 : 9216) && (long long)M * K <= 57344) return false;
   if (even && N > 4096 && N < 7168 && K % 8192 == 0 && (long long)M * K <= 32768) return false;
-  if (half && N > 1024 && N <= 2048 && (M >= 8 || (M >= 4 && K <= 5120))) return true;
+  if (half && half_plan(scaled, M, N, K)) return true;
   return N >= 2560 || (N >= 2048 && K >= 4096 && M >= 12);
 }
 
@@ -1328,7 +1337,7 @@ static void launch(hipStream_t s, const void* x, const void* w, const void* bias
 // adds up 256 shares a row where it added 64. (Of fewer than 1,024 columns a block is over before that matters.)
 extern "C" int nhv_gemm_fewrows_square_rows(int M, int N, int K, int biased, int aligned) {
   using namespace fewrows;
-  if (!aligned || K < 1024 || N >= 4096 || even_rows(N) >= 16 || lines_plan(false, false, false, M, N, K)) return 16;
+  if (!aligned || K < 1024 || N >= 4096 || even_rows(N) >= 16 || lines_plan(false, false, false, false, M, N, K)) return 16;
   return tiles_plan(false, even_rows(N), biased != 0, M, N, K).ahead ? even_rows(N) : 16;
 }
 
@@ -1344,7 +1353,7 @@ int nhv_gemm_fewrows_launch(bool glu, const void* x, const void* w, const void* 
     if (glu || fused || f.band_rows % 16 != 0) return nhv_fail("few-rows gemm: bands of %d rows (multiples of 16, no gate, no fusion)", f.band_rows);
     // (8,224 outputs of 2,048 columns at 16 rows in five bands, in a trace: 14.9 us by the kernel that takes x
     // from memory, 11.9 by lines)
-    if (f.band_rows % 32 == 0 && lines_plan(false, false, false, M, N, K))
+    if (f.band_rows % 32 == 0 && lines_plan(false, false, false, false, M, N, K))
       return out_dtype == NHV_BF16 ? launch_lines<false, bf16_t>(s, x, w, bias, y, M, N, K, f) : launch_lines<false, float>(s, x, w, bias, y, M, N, K, f);
     const Plan p = plan(false, M, N, K);
     if (f.band_rows % 32 == 0 && p.nt == 2) launch<2, 8, 2, false>(s, x, w, bias, y, M, N, K, out_dtype, false, f);
@@ -1352,7 +1361,7 @@ int nhv_gemm_fewrows_launch(bool glu, const void* x, const void* w, const void* 
     return 0;
   }
   if (fused && out_dtype != NHV_BF16) return nhv_fail("few-rows gemm: a product that takes over its neighbours' work gives bfloat16");
-  if (lines_plan(glu, f.residual == nullptr, f.residual == nullptr && out_dtype == NHV_BF16, M, N, K) && !(glu && out_dtype != NHV_BF16) && !(f.residual && f.square_rows != 16)) {
+  if (lines_plan(glu, f.residual == nullptr, f.residual == nullptr && out_dtype == NHV_BF16, f.ss_in != nullptr, M, N, K) && !(glu && out_dtype != NHV_BF16) && !(f.residual && f.square_rows != 16)) {
     if (glu) return launch_lines<true, bf16_t>(s, x, w, bias, y, M, N, K, f);
     return out_dtype == NHV_BF16 ? launch_lines<false, bf16_t>(s, x, w, bias, y, M, N, K, f) : launch_lines<false, float>(s, x, w, bias, y, M, N, K, f);
   }

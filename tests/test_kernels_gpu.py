@@ -330,6 +330,17 @@ def test_few_rows_by_lines_of_eight_rows_of_weights(ops, M, N, K):
     torch.testing.assert_close(out[~hit].double(), want[~hit], **tol(torch.bfloat16))
 
 
+@pytest.mark.parametrize("M,N,K", [(4, 2048, 2048), (16, 2048, 2048), (5, 1536, 3072), (6, 1536, 3072), (11, 1040, 3072), (12, 1040, 3072), (7, 1040, 4096),
+                                   (8, 1040, 4096), (12, 1025, 6144), (6, 2044, 5120)])
+def test_products_that_scale_their_rows_on_either_side_of_the_blocks_of_eight(ops, M, N, K):
+    """A reader of a norm with 1,025 to 2,048 outputs, by tiles and by blocks of 8 outputs: against float64 (bound: one rounding to 8 bits)."""
+    x, w = rnd(M, K, dtype=torch.bfloat16, seed=151), rnd(N, K, dtype=torch.bfloat16, seed=152, scale=K ** -0.5)
+    squares = rnd(M, K // 16, seed=153).abs() + 0.1
+    scale = torch.rsqrt(squares.double().sum(-1, keepdim=True) / K + 1e-6)
+    got = ops.linear(ops.Normed(ops.Summed(x, squares, rnd(M, K, seed=154), rnd(K, dtype=torch.bfloat16, seed=155), 1e-6)), w)
+    torch.testing.assert_close(got.double(), x.double() @ w.double().T * scale, rtol=1.6e-2, atol=1.6e-2 * float(scale.max()))
+
+
 @pytest.mark.parametrize("M,I,K", [(1, 112, 80), (5, 1001, 96), (16, 12288, 4096), (17, 160, 96), (64, 300, 1024),
                                    (4, 17408, 136), (16, 25600, 72), (13, 25000, 264), (16, 9000, 5120), (15, 520, 5384)])
 def test_gated_linear(ops, M, I, K):
