@@ -1128,12 +1128,15 @@ static bool half_plan(bool scaled, int M, int N, int K) {
 // to 12,288, at 1 to 8 rows: 8,448 outputs 1.07 to 1.18, 9,216 1.07 to 1.17, 10,240 1.00 to 1.11 and at K = 2,048 0.95, 11,264 0.96 to 1.07, 12,288 0.88 to
 // 1.04; 16 rows: K = 3,072 1.05 to 1.15, from 4,096 on 0.62 to 0.88), and with rows 16 KB apart on some of the units (K = 8,192: 4,224
 // to 6,144 outputs 1.06 to 1.22 at 1 to 4 rows, 0.81 to 0.99 at 8; 7,168 outputs 0.80 to 0.87), as long as all of x fits beside w.
-// ``half``: a bfloat16 result without residual, which 8 rows of w a block can make (half_plan).
-static bool lines_plan(bool glu, bool even, bool half, bool scaled, int M, int N, int K) {
+// ``half``: a bfloat16 result without residual, which 8 rows of w a block can make (half_plan). ``floats``: a float result, whose stretches are
+// summed apart where K is a multiple of 2,048: 2,560 outputs of 4,096 columns 7.1 us by the tiles above and 7.8 at 1 row, 7.4 and 7.9 at 4, 8.0 and 7.9
+// at 8; 2,816 of 2,048 5.3 and 5.5, 5.6 and 5.6, 5.7 and 5.7; 3,072 of 6,144 9.9 and 9.8, 10.5 and 9.9, 10.3 and 10.3.
+static bool lines_plan(bool glu, bool even, bool half, bool scaled, bool floats, int M, int N, int K) {
   if (K % 256 != 0 || K < 2048) return false;
   if (glu) return N >= 4096;
   if (even && N > 8192 && N <= (K > 2048 ? 11264 : 9216) && (long long)M * K <= 57344) return false;
   if (even && N > 4096 && N < 7168 && K % 8192 == 0 && (long long)M * K <= 32768) return false;
+  if (floats && N < 3072 && M < 8 && K % 2048 == 0) return false;
   if (half && half_plan(scaled, M, N, K)) return true;
   return N >= 2560 || (N >= 2048 && K >= 4096 && M >= 12);
 }
@@ -1337,7 +1340,7 @@ static void launch(hipStream_t s, const void* x, const void* w, const void* bias
 // adds up 256 shares a row where it added 64. (Of fewer than 1,024 columns a block is over before that matters.)
 extern "C" int nhv_gemm_fewrows_square_rows(int M, int N, int K, int biased, int aligned) {
   using namespace fewrows;
-  if (!aligned || K < 1024 || N >= 4096 || even_rows(N) >= 16 || lines_plan(false, false, false, false, M, N, K)) return 16;
+  if (!aligned || K < 1024 || N >= 4096 || even_rows(N) >= 16 || lines_plan(false, false, false, false, false, M, N, K)) return 16;
   return tiles_plan(false, even_rows(N), biased != 0, M, N, K).ahead ? even_rows(N) : 16;
 }
 
@@ -1353,7 +1356,7 @@ int nhv_gemm_fewrows_launch(bool glu, const void* x, const void* w, const void* 
     if (glu || fused || f.band_rows % 16 != 0) return nhv_fail("few-rows gemm: bands of %d rows (multiples of 16, no gate, no fusion)", f.band_rows);
     // (8,224 outputs of 2,048 columns at 16 rows in five bands, in a trace: 14.9 us by the kernel that takes x
     // from memory, 11.9 by lines)
-    if (f.band_rows % 32 == 0 && lines_plan(false, false, false, false, M, N, K))
+    if (f.band_rows % 32 == 0 && lines_plan(false, false, false, false, false, M, N, K))
       return out_dtype == NHV_BF16 ? launch_lines<false, bf16_t>(s, x, w, bias, y, M, N, K, f) : launch_lines<false, float>(s, x, w, bias, y, M, N, K, f);
     const Plan p = plan(false, M, N, K);
     if (f.band_rows % 32 == 0 && p.nt == 2) launch<2, 8, 2, false>(s, x, w, bias, y, M, N, K, out_dtype, false, f);
@@ -1361,7 +1364,7 @@ int nhv_gemm_fewrows_launch(bool glu, const void* x, const void* w, const void* 
     return 0;
   }
   if (fused && out_dtype != NHV_BF16) return nhv_fail("few-rows gemm: a product that takes over its neighbours' work gives bfloat16");
-  if (lines_plan(glu, f.residual == nullptr, f.residual == nullptr && out_dtype == NHV_BF16, f.ss_in != nullptr, M, N, K) && !(glu && out_dtype != NHV_BF16) && !(f.residual && f.square_rows != 16)) {
+  if (lines_plan(glu, f.residual == nullptr, f.residual == nullptr && out_dtype == NHV_BF16, f.ss_in != nullptr, out_dtype != NHV_BF16, M, N, K) && !(glu && out_dtype != NHV_BF16) && !(f.residual && f.square_rows != 16)) {
     if (glu) return launch_lines<true, bf16_t>(s, x, w, bias, y, M, N, K, f);
     return out_dtype == NHV_BF16 ? launch_lines<false, bf16_t>(s, x, w, bias, y, M, N, K, f) : launch_lines<false, float>(s, x, w, bias, y, M, N, K, f);
   }

@@ -341,6 +341,17 @@ def test_products_that_scale_their_rows_on_either_side_of_the_blocks_of_eight(op
     torch.testing.assert_close(got.double(), x.double() @ w.double().T * scale, rtol=1.6e-2, atol=1.6e-2 * float(scale.max()))
 
 
+@pytest.mark.parametrize("M,N,K", [(1, 2560, 2048), (7, 3068, 2048), (8, 2560, 2048), (1, 3072, 2048), (3, 2816, 4096), (3, 2816, 2304)])
+def test_float_results_of_few_rows_by_tiles_and_by_lines(ops, M, N, K):
+    """On either side of where they go by lines: against float64 (bound: float sums of K products of size K^-1/2), and alike for equal rows of w."""
+    x, w = rnd(M, K, dtype=torch.bfloat16, seed=156), rnd(N, K, dtype=torch.bfloat16, seed=157, scale=K ** -0.5)
+    w[N - 1], w[N // 2] = w[1], w[1]
+    got = ops.linear(x, w, out_dtype=torch.float32)
+    torch.testing.assert_close(got.double(), x.double() @ w.double().T, rtol=1e-4, atol=2e-4)
+    if K % 2048 == 0:
+        assert torch.equal(got[:, 1], got[:, N - 1]) and torch.equal(got[:, 1], got[:, N // 2])
+
+
 @pytest.mark.parametrize("M,I,K", [(1, 112, 80), (5, 1001, 96), (16, 12288, 4096), (17, 160, 96), (64, 300, 1024),
                                    (4, 17408, 136), (16, 25600, 72), (13, 25000, 264), (16, 9000, 5120), (15, 520, 5384)])
 def test_gated_linear(ops, M, I, K):
