@@ -559,12 +559,15 @@ extern "C" int nhv_rotary_split_write(const void* qkv, const void* bias, const v
     NHV_LAUNCH_CHECK("split_write_vec");
     return 0;
   }
-  // pieces of eight pairs: the halves and what follows them are whole pieces, at addresses that 8 entries may be read from
+  // pieces of eight pairs: the halves and what follows them are whole pieces, at addresses that 8 entries may be read from. Not for few heads in
+  // all: up to six waves a unit each take theirs at once, with no waves to meet. us by a wave a head and by pieces, bfloat16, 32 heads of 128 all turned, 4
+  // tokens 2.8, 3.2, 24 2.9, 3.2, 64 3.2, 3.3, 100 3.7, 3.4; the first 64 of 128 turned 3.0, 3.2 at 24, 3.3, 3.2 at 48; 16 query heads alone 2.8, 3.0 at 64, 3.1,
+  // 3.1 at 100, 3.8, 3.2 at 256; 12 heads of 64 2.9, 3.1 at 64, 3.1, 3.1 at 100, 3.5, 3.2 at 256 (32 bits: the same to 0.1).
   const int qk_half = rot / 2, v_half = with_kv && v_freqs ? E / 2 : 0;
   const int pieces_qk = (D - qk_half) / 8, pieces_v = (E - v_half) / 8;
   const long long items = (long long)(with_kv ? Hq + Hkv : Hq) * pieces_qk + (with_kv ? (long long)Hkv * pieces_v : 0);
   const size_t angles = 2 * (size_t)(qk_half + v_half) * sizeof(float);
-  if (!unit && !interleaved && maps == 1 && qk_half % 8 == 0 && v_half % 8 == 0 && D % 8 == 0 && E % 8 == 0 && ld % 8 == 0 &&
+  if ((long long)T * heads > 6 * 256 && !unit && !interleaved && maps == 1 && qk_half % 8 == 0 && v_half % 8 == 0 && D % 8 == 0 && E % 8 == 0 && ld % 8 == 0 &&
       v_first_ld % 8 == 0 && (starts | (uintptr_t)bias) % (8 * item) == 0 && items < 65535 * 512ll && angles <= 64 * 1024 &&
       (dtype == NHV_F32 || dtype == NHV_BF16)) {
     const long long per_token = (items + 511) / 512, threads = ((items + per_token - 1) / per_token + 63) / 64 * 64;
@@ -798,7 +801,8 @@ __global__ void turn_back_kernel(T* __restrict__ x, const float* __restrict__ fr
 
 // The same in pieces of eight pairs (E / 2 a multiple of eight, rows at addresses that 8 entries may be read from): a block
 // takes one token and its angles once, a thread one piece of one head (blockIdx.y over what 512 do not cover). us at 2,264 tokens of 16 heads of 128 in
-// bfloat16: 5.7, by a block of one wave to a head, with a sincosf for every pair, 10.3.
+// bfloat16: 5.7, by a block of one wave to a head, with a sincosf for every pair, 10.3. Where these waves are eight a unit or fewer they are as fast or
+// faster: 24 tokens 2.5 us and here 2.6, 100 2.6 and 2.7, 256 3.2 and 2.8; of 8 heads of 64 256 2.7 and 2.7, 400 2.9 and 2.75.
 template <typename T>
 __global__ __launch_bounds__(512) void turn_back_pieces_kernel(T* __restrict__ x, const float* __restrict__ freqs,
                                                                const int* __restrict__ positions, int H, int E) {
@@ -837,7 +841,7 @@ extern "C" int nhv_turn_back(void* x, const void* freqs, const void* positions, 
   NHV_REQUIRE((long long)T * H < (1ll << 31), "turn_back: too many tokens");
   hipStream_t s = (hipStream_t)stream;
   const size_t angles = (size_t)E * sizeof(float), item = dtype == NHV_F32 ? 4 : 2;
-  if (E % 16 == 0 && (uintptr_t)x % (8 * item) == 0 && (long long)H * (E / 16) < 65535 * 512ll && angles <= 64 * 1024 &&
+  if ((long long)T * H > 8 * 256 && E % 16 == 0 && (uintptr_t)x % (8 * item) == 0 && (long long)H * (E / 16) < 65535 * 512ll && angles <= 64 * 1024 &&
       (dtype == NHV_F32 || dtype == NHV_BF16)) {
     const int pieces = H * (E / 16), per_token = (pieces + 511) / 512;
     const dim3 grid((unsigned)T, (unsigned)per_token), block((unsigned)(((pieces + per_token - 1) / per_token + 63) / 64 * 64));

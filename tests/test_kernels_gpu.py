@@ -1847,16 +1847,16 @@ def test_delta_rule_lets_no_token_reach_the_ones_before_it(ops, D, E, per_head):
 
 
 @pytest.mark.parametrize("dtype", DTYPES)
-@pytest.mark.parametrize("T,Hq,Hkv,D,E,rot,of_values,more", [(1, 1, 1, 16, 8, 16, None, ()), (70, 5, 2, 24, 40, 16, None, ("bias",)),
-                                                             (3, 16, 8, 128, 128, 128, "turned", ()),
-                                                             (37, 33, 11, 128, 64, 48, "mixed", ("temperature",)),
-                                                             (9, 6, 3, 64, 64, 64, "keys", ("bias", "columns")),
-                                                             (5, 7, 3, 32, 16, 0, "turned", ("bias",)),
-                                                             (40, 12, 4, 80, 48, 80, "none", ("columns",))])
+@pytest.mark.parametrize("T,Hq,Hkv,D,E,rot,of_values,more", [(1, 1, 1, 16, 8, 16, None, ()), (513, 1, 1, 16, 8, 16, None, ()), (190, 5, 2, 24, 40, 16, None, ("bias",)),
+                                                             (140, 16, 8, 128, 128, 128, "turned", ()), (48, 16, 8, 128, 128, 128, "turned", ()),
+                                                             (70, 33, 11, 128, 64, 48, "mixed", ("temperature",)),
+                                                             (360, 6, 3, 64, 64, 64, "keys", ("bias", "columns")),
+                                                             (300, 7, 3, 32, 16, 0, "turned", ("bias",)),
+                                                             (171, 12, 4, 80, 48, 80, "none", ("columns",))])
 def test_heads_turned_in_pieces_of_eight_pairs(ops, dtype, T, Hq, Hkv, D, E, rot, of_values, more):
     """Against the kernel of one wave to a head, which takes the same rows where they start one entry off a piece: the same
     expressions of the same angles, whose products a compiler may contract one way or the other (half a float's last place,
-    which can become one of bfloat16's). Rows without a slot store nothing; so the caches keep what they held."""
+    which can become one of bfloat16's); up to 1,536 heads of all tokens (2,048 that are turned back) both take that kernel. Rows without a slot store nothing; so the caches keep what they held."""
     kv = of_values != "none"
     width = Hq * D + (Hkv * D + (0 if of_values == "keys" else Hkv * E) if kv else 0) + (8 if "columns" in more else 0)
     bias = rnd(width - (8 if "columns" in more else 0), dtype=dtype, seed=91) if "bias" in more else None
