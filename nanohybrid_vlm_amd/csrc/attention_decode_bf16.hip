@@ -125,6 +125,8 @@ __global__ __launch_bounds__(64 * WAVES) void decode_attention_kernel(
   // 32 and 64 requests (116 against 111 us at 64) than one whose blocks go over all heads
   int t = blockIdx.y;
   const int split = blockIdx.z;
+  // (ROTATED: what the splits leave over belongs to the last one: a key that no block took would not be stored either)
+  const int split_end = ROTATED && split == n_splits - 1 ? max_blocks * page_size - 1 : (split + 1) * split_len - 1;
   int pos, req;
   // Contexts of different lengths: of a split's blocks those that start first take the most keys (64 requests after 100 to 2,000
   // keys, one split: 68.7 -> 62.7 us; after 100 to 8,000, splits of 2,048: 225 -> 209; 48 after 100 to 16,000 329 -> 317; for 128
@@ -134,7 +136,7 @@ __global__ __launch_bounds__(64 * WAVES) void decode_attention_kernel(
     static_assert(MOST_SORTED <= 64 && sizeof(int) * (2 * MOST_SORTED + 1) <= sizeof(tiles_s), "a wave and the tiles hold the tokens' numbers of keys");
     int *keys_s = reinterpret_cast<int*>(tiles_s), *place_s = keys_s + MOST_SORTED, *chosen = place_s + MOST_SORTED;
     const int T = gridDim.y, p = positions[min(lane, T - 1)], r = token_req[min(lane, T - 1)];
-    const int mine = lane < T ? min(p, (split + 1) * split_len - 1) - max(nhv_first_key(p, window), split * split_len) + 1 : 0;
+    const int mine = lane < T ? min(p, split_end) - max(nhv_first_key(p, window), split * split_len) + 1 : 0;
     if (t >= __popcll(__ballot(mine > 0))) return;     // (fewer tokens have keys here: the same for the whole block)
     const int one = __shfl(mine, 0, 64);
     if (__ballot(lane < T && mine != one)) {           // (equal ones are taken as they come: 1.6 us less for 64 requests after 2,048 keys)
@@ -172,7 +174,7 @@ __global__ __launch_bounds__(64 * WAVES) void decode_attention_kernel(
   const int G = min(16, Hq / Hkv - (group % per_kv) * 16);
   const int lo = nhv_first_key(pos, window);
   const int first = max(lo, split * split_len);
-  const int last = min(pos, (split + 1) * split_len - 1);
+  const int last = min(pos, split_end);
   if (first > last) return;              // this split holds no visible key; the merge knows from pos and lo
   const int* bt = block_tables + (size_t)req * max_blocks;
   const int col = lane & 15, grp = lane >> 4;
@@ -468,9 +470,9 @@ __global__ __launch_bounds__(64 * W) void merge_splits_kernel(const float* __res
   const int t = item / Hq;
   const int pos = positions[t];
   const int lo = nhv_first_key(pos, window);
-  // (the launch's splits must cover every position; one that they do not cover loses its last keys here rather
-  // than reading past the splits' results)
-  const int s0 = lo / split_len, s1 = min(pos / split_len, n_splits - 1);
+  // (the launch's splits must cover every position; one that they do not cover loses its last keys, or gets them from the last split
+  // where queries are turned in the attention's launch, and reads nothing past the splits' results)
+  const int s0 = min(lo / split_len, n_splits - 1), s1 = min(pos / split_len, n_splits - 1);
   const float* ml = part_ml + (size_t)item * n_splits * 2;
   float m = -INFINITY;
   for (int s = s0 + lane; s <= s1; s += 64) m = fmaxf(m, ml[s * 2]);
@@ -567,7 +569,7 @@ __global__ __launch_bounds__(64 * W) void merge_splits_at_once_kernel(const floa
     }
   }
   const int lo = nhv_first_key(pos, window);
-  const int s0 = lo / split_len, s1 = min(pos / split_len, n_splits - 1);
+  const int s0 = min(lo / split_len, n_splits - 1), s1 = min(pos / split_len, n_splits - 1);   // (as in the kernel above)
   float m = -INFINITY;
 #pragma unroll
   for (int i = 0; i < NL; ++i) {
@@ -729,7 +731,8 @@ extern "C" int nhv_decode_attention_bf16(const void* q, const void* k_cache, con
 // bfloat16, or (splits > 0) that many float parts of it; the kernel adds the bias (null: none), divides every head of queries and
 // keys by its root mean square and multiplies by its weight (null: not), turns it by the halves' angles of its position (cos_sin
 // [positions, D]; null: not) and stores keys and values at slot_mapping[t] (negative: nowhere). Every token is of another request
-// and reads no slot that another one of the call stores to.
+// and reads no slot that another one of the call stores to. Every token's key and value are stored whatever the splits cover: the last
+// one takes all keys that are left.
 extern "C" int nhv_decode_attention_rotated_bf16(const void* qkv, int splits, const void* bias, const void* q_norm_w, const void* k_norm_w,
                                                  int w_dtype, float eps, const void* cos_sin, const void* rotation_positions,
                                                  const void* slot_mapping, void* k_cache, void* v_cache, void* out, void* part_o,

@@ -1934,3 +1934,25 @@ def test_single_tokens_turned_stored_and_read_in_one_launch(ops, monkeypatch, Hq
     got = ops.rotated_attention(*arguments, k2, v2, Hq, Hkv, D, batch, bt, D ** -0.5, window)
     for a, c in ((got, want), (k2, k1), (v2, v1)):
         assert torch.equal(a.view(torch.uint8), c.view(torch.uint8))
+
+
+@pytest.mark.parametrize("T,window", [(3, None), (20, None), (3, 40)])
+@pytest.mark.parametrize("splits", [1, 2])
+def test_single_tokens_beyond_what_the_splits_cover_are_stored_and_read(ops, monkeypatch, T, window, splits):
+    """A launch whose splits end before the tokens' positions (as many keys a split, and splits, as are asked for here): the last split takes the
+    keys that are left, so that the token's own key and value lie in the cache afterwards. Against the two launches: the cache bit for bit, the
+    result within one rounding to 8 bits."""
+    Hq, Hkv, D, page = 8, 2, 64, 16
+    lens = [200 - 7 * i for i in range(T)]
+    _, k, v, batch, bt, *_ = _paged_setup(torch.bfloat16, lens, [1] * T, Hq, Hkv, D, page, seed=161)
+    rows, table = rnd(T, (Hq + 2 * Hkv) * D, dtype=torch.bfloat16, seed=162), rnd(256, D, seed=163)
+    t, pos = torch.arange(T, device="cuda"), batch.positions.long()
+    slots = (bt[t, pos // page] * page + pos % page).int()
+    arguments = (rows, None, None, None, 0.0, table, batch.positions, slots)
+    k1, v1, k2, v2 = k.clone(), v.clone(), k.clone(), v.clone()
+    want = ops.paged_attention(ops.qk_rope_write(*arguments, k1, v1, Hq, Hkv, D), k1, v1, batch, bt, D ** -0.5, window)
+    parts = [torch.zeros((T, Hq, splits, n), device="cuda") if splits > 1 else None for n in (D, 2)]
+    monkeypatch.setattr(ops.backend(), "_decode_splits", lambda *args: (*parts, 32, splits), raising=False)
+    got = ops.rotated_attention(*arguments, k2, v2, Hq, Hkv, D, batch, bt, D ** -0.5, window)
+    assert torch.equal(k1.view(torch.int16), k2.view(torch.int16)) and torch.equal(v1.view(torch.int16), v2.view(torch.int16))
+    torch.testing.assert_close(got, want, rtol=1.6e-2, atol=1.6e-2)
