@@ -1106,16 +1106,43 @@ __global__ __launch_bounds__(512) void gemm_fewrows_lines_kernel(const bf16_t* _
   if ((threadIdx.x & 15) == 0 && row < M && my_tile < tiles) f.ss_out[(size_t)row * tiles + my_tile] = sq;
 }
 
-// Blocks of 8 outputs, by lines. us by the tiles above (M = 12 and more, 2,048 outputs: by lines of 16 rows) and by those, of 2,048 outputs: of 2,048
-// columns at 4, 8 and 16 rows 4.9, 4.9, 5.2 and 4.8, 4.8, 4.9; of 3,072 at 4 and 7 rows 5.9, 6.0 and 5.7, 5.7; of 4,096 6.9, 7.2 and 6.6, 6.8; of
-// 5,120 7.8, 8.1 and 7.7, 7.8; of 6,144 at 4, 8 and 16 rows 8.5, 9.3, 10.3 and 9.9, 8.7, 9.1; of 12,288 13.8, 16.9, 17.5 and 16.8, 14.7, 15.2; 1,280 of 4,096 6.2,
-// 6.7, 7.7 and 6.3, 6.4, 6.5; 1,040 of 2,560 at 4 and 6 rows 5.0, 5.1 and 5.2, 5.0. ``scaled`` (x a sum whose rows lack their norm's scales): these cost
-// such a block 0.5 us more and the tiles 0.1; 2,048 of 2,048 at 4, 8 and 16 rows 5.0, 5.2, 5.7 and 5.6, 5.6, 5.8; 1,536 of 3,072 at 4, 6 and 8 rows 6.1, 6.4, 6.5 and
-// 6.1, 6.2, 6.2; 1,280 of 3,072 at 8, 12 and 16 rows 6.1, 6.4, 6.7 and 6.2, 6.3, 6.4; 1,040 of 4,096 at 4 and 8 rows 6.6, 7.1 and 6.9, 6.9.
+// What else a product is, beside its sizes.
+struct Form {
+  bool glu, residual, banded;
+  bool scaled;                                              // x is a sum whose rows lack their norm's scales
+  bool floats;                                              // a float result
+};
+
+// Blocks of 8 outputs, by lines, for a bfloat16 result of 1,025 to 2,048 outputs without residual, where the tiles above have 8 rows of w a block
+// as well: they differ by a block's fixed cost and by how x comes. Measured over nine numbers of outputs by twelve of columns (2,048 to 8,192)
+// at ten numbers of rows; time by blocks of 8 over the tiles': from 12 rows on 0.55 to 0.99 everywhere; up to 2,304 columns 0.91 to 1.01 from 4 rows on;
+// with more, from where w has 2,048 x 2,816 entries, 0.90 to 1.0 at 6 and 7 rows (below that 0.95 to 1.07: 1,536 of 3,584 1.05, 1,040 of 5,120 1.07), 0.90
+// to 1.0 at 8 (below 0.98 to 1.07 beyond 3,072 columns). At 4 and 5 rows 2,048 of 3,072 0.99 and 0.98, of 4,096 0.97 and 0.95, but 1,280 of 3,584 1.05 and
+// 1.04, 1,536 of 5,120 1.02 and 1.0. us: 2,048 of 2,048 at 4 and 16 rows 4.9, 5.2 and 4.8, 4.9; of 4,096 at 4 and 7 6.9, 7.2 and 6.6, 6.8; of 12,288 at 8 and 16 16.9,
+// 17.5 and 14.7, 15.2. ``scaled``: such a block takes 0.5 us more and the tiles 0.1: below those 2,048 x 2,816 entries 1.0 to 1.13 at 6 to 8 rows (2,048 of 2,560 1.08,
+// 1,040 of 5,120 1.13), from there on 0.95 to 1.02; at 12 and 16 rows 0.83 to 1.03 for 2,816 to 4,096 columns, up to 1.09 for others, but 0.57 to 0.71 where x
+// no longer fits beside w in the tiles' LDS (16 rows of 4,608 columns, 12 of 6,144).
 static bool half_plan(bool scaled, int M, int N, int K) {
   if (N <= 1024 || N > 2048) return false;
-  if (scaled) return (M >= 6 && K <= 5120 && (long long)N * K >= 1536 * 3072) || (K >= 3072 && M >= (K >= 4096 ? 8 : 12));
-  return M >= 8 || (M >= 4 && K <= 5120 && (M >= 6 || N >= 1280 || K <= 2048));
+  const bool many = (long long)N * K >= 2048 * 2816;
+  if (scaled) return (M >= 6 && many && (K <= 5120 || M >= 8)) || (M >= 12 && K >= 2816 && K <= 4096) || (M >= 8 && M * K >= 16 * 4608);
+  if (M >= 12 || K <= 2304 || (M >= 8 && K <= 3072)) return M >= 4;
+  if (!many || M < 4 || (K > 5120 && M < 8)) return false;
+  return M >= 6 || (K <= 4096 && N >= 1920) || (M == 5 && K >= 4096);
+}
+
+// Fewer than 8 rows and 2,560 to 4,095 outputs: where the tiles above are the faster ones all the same, of 2,048 columns above all, which are a
+// ring's two fillings. Time by lines over theirs at 1, 2, 4 and 7 rows: rows to scale, 2,560 outputs of 2,048 columns 1.09, 1.09, 1.05, 1.07, 2,816 1.06, 1.07, 1.02,
+// 1.02, 3,072 1.0, 1.03, 0.99, 0.98; 2,560 of 3,072 1.03, 1.04, 0.99, 0.96, of 2,304 0.98, 0.97, 0.96, 0.94; added to the residual stream as well, 2,560 of 2,048 1.06,
+// 1.07, 1.0, 1.0, 2,816 1.04, 1.01, 0.97, 0.96. (Neither: 2,560 of 2,048 1.04, 1.05, 0.97, 1.0, which is left by lines, 2,816 0.99, 0.99, 0.92, 0.96; the
+// addition alone never above 1.0.) In bands, whose other way is the kernel that takes x from memory: 2,560 outputs 1.08, 1.05, 1.02, 1.01, 2,816 1.04, 1.02, 0.99, 0.95,
+// 3,584 1.02, 0.98, 0.96, 0.89; of 2,304 0.88 to 0.8. Float results are summed in stretches where K is a multiple of 2,048: 2,560
+// outputs of 4,096 columns 7.1 us by the tiles and 7.8 at 1 row, 7.4 and 7.9 at 4; 3,072 of 2,048 1.02, 1.03, 0.96, 0.99, of 6,144 9.9 and 9.8, 10.5 and 9.9.
+static bool lines_lose(const Form& p, int M, int N, int K) {
+  if (p.banded) return K == 2048 && (N < 2816 || M == 1);
+  if (p.floats) return K % 2048 == 0 && N < (K == 2048 && M <= 2 ? 3200 : 3072);
+  if (p.residual) return p.scaled && K == 2048 && N < 2944 && M < 4;
+  return p.scaled && (K == 2048 ? N < 3072 : N < 2944 && M <= 2 && K > 2304 && K <= 3072);
 }
 
 // Where the rows of w are enough for it, by what was measured at 1, 4, 8, 12 and 16 rows (us before and with it): not for 4,096 outputs
@@ -1123,21 +1150,19 @@ static bool half_plan(bool scaled, int M, int N, int K) {
 // which the smaller tiles above do not, until there are so many rows that these are slower: 2,560 of 4,096 7.7, 6.9 at 1 row and 7.8, 7.1 at 4;
 // 2,560 of 9,728 14.6, 14.0 and 15.3, 14.7; 3,584 of 3,584 8.5, 7.6 and 8.7, 7.8; 3,072 of 8,192 12.9, 12.0 and 13.6, 12.2; 2,048 of 6,144 8.3, 11
 // at 1 and 9.5, 11.1 at 8, but 14.3, 11.5 at 12; 2,048 of 2,048 never (all by blocks of 16 outputs).
-// ``even``: the tiles above would take the product and give every unit the same rows of w (with a residual they do so for fewer than 4,096 outputs
+// ``even`` (in the rule): the tiles above would take the product and give every unit the same rows of w (with a residual they do so for fewer than 4,096 outputs
 // alone, see nhv_gemm_fewrows_square_rows; with bands never). They stay the faster ones where the blocks of 32 outputs are a round and a bit (time by lines over theirs, K = 2,048
 // to 12,288, at 1 to 8 rows: 8,448 outputs 1.07 to 1.18, 9,216 1.07 to 1.17, 10,240 1.00 to 1.11 and at K = 2,048 0.95, 11,264 0.96 to 1.07, 12,288 0.88 to
 // 1.04; 16 rows: K = 3,072 1.05 to 1.15, from 4,096 on 0.62 to 0.88), and with rows 16 KB apart on some of the units (K = 8,192: 4,224
 // to 6,144 outputs 1.06 to 1.22 at 1 to 4 rows, 0.81 to 0.99 at 8; 7,168 outputs 0.80 to 0.87), as long as all of x fits beside w.
-// ``half``: a bfloat16 result without residual, which 8 rows of w a block can make (half_plan). ``floats``: a float result, whose stretches are
-// summed apart where K is a multiple of 2,048: 2,560 outputs of 4,096 columns 7.1 us by the tiles above and 7.8 at 1 row, 7.4 and 7.9 at 4, 8.0 and 7.9
-// at 8; 2,816 of 2,048 5.3 and 5.5, 5.6 and 5.6, 5.7 and 5.7; 3,072 of 6,144 9.9 and 9.8, 10.5 and 9.9, 10.3 and 10.3.
-static bool lines_plan(bool glu, bool even, bool half, bool scaled, bool floats, int M, int N, int K) {
+static bool lines_plan(const Form& p, int M, int N, int K) {
   if (K % 256 != 0 || K < 2048) return false;
-  if (glu) return N >= 4096;
+  if (p.glu) return N >= 4096;
+  const bool even = !p.residual && !p.banded;
   if (even && N > 8192 && N <= (K > 2048 ? 11264 : 9216) && (long long)M * K <= 57344) return false;
   if (even && N > 4096 && N < 7168 && K % 8192 == 0 && (long long)M * K <= 32768) return false;
-  if (floats && N < 3072 && M < 8 && K % 2048 == 0) return false;
-  if (half && half_plan(scaled, M, N, K)) return true;
+  if (even && !p.floats && half_plan(p.scaled, M, N, K)) return true;
+  if (M < 8 && N < 4096 && lines_lose(p, M, N, K)) return false;
   return N >= 2560 || (N >= 2048 && K >= 4096 && M >= 12);
 }
 
@@ -1340,7 +1365,7 @@ static void launch(hipStream_t s, const void* x, const void* w, const void* bias
 // adds up 256 shares a row where it added 64. (Of fewer than 1,024 columns a block is over before that matters.)
 extern "C" int nhv_gemm_fewrows_square_rows(int M, int N, int K, int biased, int aligned) {
   using namespace fewrows;
-  if (!aligned || K < 1024 || N >= 4096 || even_rows(N) >= 16 || lines_plan(false, false, false, false, false, M, N, K)) return 16;
+  if (!aligned || K < 1024 || N >= 4096 || even_rows(N) >= 16 || lines_plan({.residual = true}, M, N, K)) return 16;
   return tiles_plan(false, even_rows(N), biased != 0, M, N, K).ahead ? even_rows(N) : 16;
 }
 
@@ -1356,7 +1381,7 @@ int nhv_gemm_fewrows_launch(bool glu, const void* x, const void* w, const void* 
     if (glu || fused || f.band_rows % 16 != 0) return nhv_fail("few-rows gemm: bands of %d rows (multiples of 16, no gate, no fusion)", f.band_rows);
     // (8,224 outputs of 2,048 columns at 16 rows in five bands, in a trace: 14.9 us by the kernel that takes x
     // from memory, 11.9 by lines)
-    if (f.band_rows % 32 == 0 && lines_plan(false, false, false, false, false, M, N, K))
+    if (f.band_rows % 32 == 0 && lines_plan({.banded = true, .floats = out_dtype != NHV_BF16}, M, N, K))
       return out_dtype == NHV_BF16 ? launch_lines<false, bf16_t>(s, x, w, bias, y, M, N, K, f) : launch_lines<false, float>(s, x, w, bias, y, M, N, K, f);
     const Plan p = plan(false, M, N, K);
     if (f.band_rows % 32 == 0 && p.nt == 2) launch<2, 8, 2, false>(s, x, w, bias, y, M, N, K, out_dtype, false, f);
@@ -1364,7 +1389,8 @@ int nhv_gemm_fewrows_launch(bool glu, const void* x, const void* w, const void* 
     return 0;
   }
   if (fused && out_dtype != NHV_BF16) return nhv_fail("few-rows gemm: a product that takes over its neighbours' work gives bfloat16");
-  if (lines_plan(glu, f.residual == nullptr, f.residual == nullptr && out_dtype == NHV_BF16, f.ss_in != nullptr, out_dtype != NHV_BF16, M, N, K) && !(glu && out_dtype != NHV_BF16) && !(f.residual && f.square_rows != 16)) {
+  const Form form = {.glu = glu, .residual = f.residual != nullptr, .scaled = f.ss_in != nullptr, .floats = out_dtype != NHV_BF16};
+  if (lines_plan(form, M, N, K) && !(glu && out_dtype != NHV_BF16) && !(f.residual && f.square_rows != 16)) {
     if (glu) return launch_lines<true, bf16_t>(s, x, w, bias, y, M, N, K, f);
     return out_dtype == NHV_BF16 ? launch_lines<false, bf16_t>(s, x, w, bias, y, M, N, K, f) : launch_lines<false, float>(s, x, w, bias, y, M, N, K, f);
   }

@@ -331,9 +331,10 @@ def test_few_rows_by_lines_of_eight_rows_of_weights(ops, M, N, K):
 
 
 @pytest.mark.parametrize("M,N,K", [(4, 2048, 2048), (16, 2048, 2048), (5, 1536, 3072), (6, 1536, 3072), (11, 1040, 3072), (12, 1040, 3072), (7, 1040, 4096),
-                                   (8, 1040, 4096), (12, 1025, 6144), (6, 2044, 5120)])
+                                   (8, 1040, 4096), (12, 1025, 6144), (6, 2044, 5120), (6, 2048, 2816), (12, 1040, 2816), (16, 1028, 4608), (15, 1028, 4608),
+                                   (1, 2560, 2048), (7, 3068, 2048), (2, 2940, 2560), (3, 2940, 2560), (7, 3072, 2048)])
 def test_products_that_scale_their_rows_on_either_side_of_the_blocks_of_eight(ops, M, N, K):
-    """A reader of a norm with 1,025 to 2,048 outputs, by tiles and by blocks of 8 outputs: against float64 (bound: one rounding to 8 bits)."""
+    """A reader of a norm, by tiles and by blocks of 8 outputs (1,025 to 2,048 outputs) or of 16: against float64 (bound: one rounding to 8 bits)."""
     x, w = rnd(M, K, dtype=torch.bfloat16, seed=151), rnd(N, K, dtype=torch.bfloat16, seed=152, scale=K ** -0.5)
     squares = rnd(M, K // 16, seed=153).abs() + 0.1
     scale = torch.rsqrt(squares.double().sum(-1, keepdim=True) / K + 1e-6)
