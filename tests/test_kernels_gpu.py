@@ -1561,6 +1561,23 @@ def test_products_in_bands_by_lines(ops, M, band, last, K):
     torch.testing.assert_close(torch.cat(list(ops.banded_linear(x, w, band)), dim=1).double(), want, **tol(torch.bfloat16))
 
 
+@pytest.mark.parametrize("M", [1, 3, 8, 12])
+@pytest.mark.parametrize("band,last,K", [(512, 512, 2048), (640, 704, 2304), (960, 250, 2304), (512, 512, 4096), (512, 544, 4096)])
+def test_products_in_bands_of_few_outputs(ops, M, band, last, K):
+    """Four sets of rows against the bands of 2,048 to 3,130 outputs, in both result types: on either side of where they go by lines (by blocks of 8
+    outputs for 12 rows of 2,048), each band's rows of a size of their own (float sums of K products of that size times K^-1/2, and one rounding)."""
+    sizes = torch.tensor([1.0, 4.0, 16.0, 64.0], device="cuda").view(4, 1, 1)
+    x = (rnd(4, M, K, seed=94) * sizes).to(torch.bfloat16)
+    w = rnd(3 * band + last, K, dtype=torch.bfloat16, seed=95, scale=K ** -0.5)
+    out = torch.empty(M, 3 * band + last, dtype=torch.bfloat16, device="cuda")
+    assert ops.backend().banded_linear(x, w, out, band)
+    for i, got in enumerate(ops.banded_linear(x, w, band)):
+        of = slice(i * band, (i + 1) * band if i < 3 else None)
+        want = x[i].double() @ w[of].double().T
+        torch.testing.assert_close(got.double(), want, rtol=1e-4, atol=2e-4 * float(sizes[i]))
+        torch.testing.assert_close(out[:, of].double(), want, rtol=8e-3, atol=2e-4 * float(sizes[i]))
+
+
 @pytest.mark.parametrize("splits", [1, 2, 4, 8])
 def test_parts_of_a_product_through_the_norm_and_the_rotation(ops, splits):
     """Parts whose sum is a bfloat16 number give the bits that this number gives: the norm that adds to the residual stream (in
