@@ -1358,7 +1358,7 @@ static void launch(hipStream_t s, const void* x, const void* w, const void* bias
 }  // namespace fewrows
 
 // Outputs whose squares a product that is added to the residual stream best sends out together: those of a block. With tiles of 16 the
-// products of fewer than 4,096 outputs leave units idle, as many as a quarter of the chip has for 1,024 of them. (`aligned`: biases, residual
+// products of fewer than 4,096 outputs leave units idle, three quarters of the chip with 1,024 of them. (`aligned`: biases, residual
 // and norm weights on 16-byte boundaries.) us at 1, 4, 8 and 16 rows by 16 and by
 // even blocks: 1,024 of 2,048 4.9, 5.3, 5.5, 5.8 and 4.3, 4.6, 4.7, 5.1; 1,024 of 3,072 5.8, 6.4, 6.6, 7.2 and 4.8, 5.2, 5.6, 6.1; 2,048 of
 // 2,048 5.4, 5.9, 6.0, 6.5 and 5.1, 5.3, 5.6, 6.0; 2,048 of 6,144 11.5, 11.1, 12.0 (10.8 by lines) and 8.5, 9.0, 10.0. The reader then

@@ -60,7 +60,7 @@ __device__ __forceinline__ bool finite(float v) { return fabsf(v) < INFINITY; }
 // after the other, lane l the columns l, l + 64, ..., and stops where a lane's sum is no number. A row of x or of w with an entry that is no
 // number settles all of the wave's outputs of that row. The order hangs on K alone. us, without such outputs, with one entry
 // of x that is no number, with one column of sums beyond 2^96, with nothing but infinities, with nothing but sums beyond 2^96: 517 x 4096 . 1024
-// 57, 64, 89, 720, 1730; 6 x 1024 . 3072 18, 20, 29, 51, 225 (by one lane an output: 204 and 230 with one such entry, 5,600 and 283 with infinities).
+// 50, 50, 87, 697, 1,706; 6 x 1024 . 3072 11, 12, 24, 44, 222 (by one lane an output: 204 and 230 with one such entry, 5,600 and 283 with infinities).
 __device__ __attribute__((noinline)) float plain_products(const float* __restrict__ x, const float* __restrict__ w, int K, float v, int m, int n, bool odd) {
   const int lane = threadIdx.x & 63;
   for (unsigned long long left = __ballot(odd); left;) {
