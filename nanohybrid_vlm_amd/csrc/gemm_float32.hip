@@ -652,23 +652,41 @@ extern "C" int nhv_gemm_float32(const void* x, const void* w, const void* bias, 
 }
 
 // ---------------------------------------------------------------- parts that their reader adds up
-// How many parts (the segments of K) a product is best left in for a reader that adds them up; 0: it is best finished here. What K over more
-// blocks saves grows with K and is little where outputs alone make blocks enough; what it costs are the parts' way to memory and
-// back, 8 entries for one at 4 TB/s. us of the product (cold weights) and the norm behind it, finished and in parts: 6 rows, 1024 . 2048 11.5, 8.9, 1024
-// . 3072 13.9, 9.5, 2048 . 6144 23.2, 19.6, but 2560 . 1024 9.2, 9.9, 1536 . 512 7.4, 7.9, 4096 . 2048 13.7, 15.8; 17 rows, 2560 . 4096 24.3, 23.3, 4096 . 12288 60.6,
-// 59.5, but 4096 . 4096 25.2, 28.0; 40 rows, 5120 . 5120 54.9, 42.4, but 8192 . 8192 89, 104; 130 rows, 1024 . 3072 28.0, 20.0, 2048 . 6144 61, 45, but 2048 . 512
-// 12.8, 16.0; 517 rows, 1024 . 2048 46.5, 31.4, 2048 . 6144 192, 122, but 2048 . 512 27.8, 31.3; 1,000 rows, 1024 . 2048 51.9, 47.5, but 1024 . 512 22.2, 28.6
-// and 1024 . 1024 32.0, 34.3; 450 rows, 4096 . 2048 (in parts 9 % longer).
+// Which tiles make the parts of more than 16 rows: 64 x 64, or 64 x 128, which read x half as often, where few tiles of rows leave w the larger part of
+// what is read (130 x 4096 . 2048 32.2 and 28.4 us, 517 x 1024 . 3072 33 and 38).
+static bool wide_parts(long long M, long long N, int K) {
+  return ((M + 63) / 64) * ((N + 63) / 64) * segments(K) > 3000 || (M > 64 && M <= 192 && N >= 2048);
+}
+
+// Whether a product is best left in parts for a norm that adds them up. What K over more blocks saves grows with K and is little where outputs alone
+// make blocks enough; what it costs are the parts' way to memory and back, 8 entries for one, and the tiles' first pieces. Measured over 4,600 sizes (cold
+// weights, product and norm; time in parts over finished). Up to 16 rows, 1 and 16: 1,024 outputs of 512 columns 0.96, 0.91, 2,048 of 512 1.09, 1.09, of 768 0.99, 0.92, of
+// 3,072 0.85, 0.79; 2,560 of 1,536 1.14, 1.14, of 2,048 0.97, 1.02, of 3,072 0.92, 0.94; 4,096 of 3,072 1.03, 1.1. More rows: 512 columns 1.0 to 1.6
+// everywhere, 2,048 and more 0.6 to 1.0 but for few rows of many outputs (17 rows, 4,096 outputs of 4,096 1.13, 5,120 of 8,192 1.04, 32 rows, 4,096 of 2,048 1.12, of 4,096 0.96, 40
+// rows, 8,192 of 2,048 1.18). In between it hangs on how the tiles fill the chip either way (1,024 columns: 256 x 1536 0.81, 257 x 1280 1.2; 1,536 columns: 256 x
+// 1536 0.68, 96 x 2304 1.14), for which both ways' times are estimated: the finished one's by its tile's cost, the parts' by a block's pieces and how many
+// blocks a unit has, both with the norm that reads them (mean error 4 and 6 %). Of those sizes 3 % are now more than 3 % slower than by the better way, the worst 16 %.
+static bool parts_pay(int M, int N, int K) {
+  if (M <= 16) return N <= (K < 768 ? 1024 : K < 3072 ? 2048 : 2560);
+  if ((long long)M * N > 1200000 || K < 768) return false;
+  if (M <= 48 && N > 2560 && (N > 5120 || K < 1280 || (M <= 32 && (long long)M * K < 28ll * N))) return false;
+  if (K >= 2048 || (K >= 1280 && N < 2304)) return true;
+  const bool wide = wide_parts(M, N, K);
+  if (wide ? K < 1024 : M <= 48 && N >= 2304) return false;
+  const Choice tile = plain_tile(M, N, true);
+  const double outputs = 1e-6 * M * N, finished = 5.2 + 5.5 / 3072 * tile.cost * K + (tile.tile == 4 ? 1.5 : 0.0) + 9.5 * outputs;
+  const int count = segments(K), pieces = segment_length(K) / PIECE, columns = wide ? 128 : 64;
+  const double a_unit = fmax(1.0, (double)((M + 63) / 64) * ((N + columns - 1) / columns) * count / 256);
+  return (wide ? 8.9 + pieces * (0.76 * a_unit + 0.15) + 2.0 * a_unit + 1.0 * count * outputs : 7.1 + pieces * (0.43 * a_unit + 0.15) + 2.25 * count * outputs) < finished;
+}
+
+// How many parts (the segments of K) that are; 0: the product is best finished here.
 extern "C" int nhv_gemm_float32_parts_count(const void* x, const void* w, int M, int N, int K) {
-  const bool whole = M > 0 && N > 0 && K >= 512 && whole_pieces(x, w, K);
-  const int most = M <= 16 ? 2560 : M <= 32 ? (K >= 2ll * N ? 4096 : 2560) : M <= 48 ? 5120 : 1200000 / M;
-  const bool pays = N <= most && (M <= 16 ? 2ll * K > N : K >= 2048 && (long long)M * N <= 1200000);
-  return whole && pays ? segments(K) : 0;
+  return M > 0 && N > 0 && K >= 512 && whole_pieces(x, w, K) && parts_pay(M, N, K) ? segments(K) : 0;
 }
 
 // y[segments][M][N], times 2^32. Up to 16 rows two waves a block, each with all of a segment under way (one with half of it: 8.1 us where 7.0
-// are kept at 1024 . 3072); else tiles of 64 x 64, or of 64 x 128, which read x half as often, where few tiles of rows leave w the larger part of
-// what is read (130 x 4096 . 2048 32.2 and 28.4 us, 517 x 1024 . 3072 33 and 38).
+// are kept at 1024 . 3072).
 extern "C" int nhv_gemm_float32_parts(const void* x, const void* w, void* y, int M, int N, int K, void* stream) {
   NHV_REQUIRE(M > 0 && N > 0 && K > 0 && K % PIECE == 0 && K < (1 << 22), "gemm in parts: bad sizes M=%d N=%d K=%d (a multiple of %d)", M, N, K, PIECE);
   NHV_REQUIRE((((uintptr_t)x | (uintptr_t)w) & 15) == 0, "gemm in parts: rows off 16-byte boundaries");
@@ -676,9 +694,8 @@ extern "C" int nhv_gemm_float32_parts(const void* x, const void* w, void* y, int
   hipStream_t s = (hipStream_t)stream;
   const float *xf = (const float*)x, *wf = (const float*)w;
   float* yf = (float*)y;
-  const long long tiles = (((long long)M + 63) / 64) * (((long long)N + 63) / 64);
   if (M <= 16) launch<1, 1, 4, false, true>(xf, wf, nullptr, yf, M, N, K, {}, s);
-  else if (tiles * segments(K) > 3000 || (M > 64 && M <= 192 && N >= 2048)) launch_blocks<2, false, true>(xf, wf, nullptr, yf, M, N, K, {}, s);
+  else if (wide_parts(M, N, K)) launch_blocks<2, false, true>(xf, wf, nullptr, yf, M, N, K, {}, s);
   else launch_blocks<1, false, true>(xf, wf, nullptr, yf, M, N, K, {}, s);
   NHV_LAUNCH_CHECK("gemm_float32_parts");
   return 0;
