@@ -807,6 +807,16 @@ extern "C" int nhv_sum_parts_float32(const void* parts, int count, const void* x
   return 0;
 }
 
+// Gates of whole pieces whose 64 x 64 tiles (64 x 128 of w) are best halved, by the kernel of 16x16x32 instructions: a block of the larger ones takes 4 us more
+// before its first product, which short rows do not make up where half of the last round's units have nothing to do. us, larger and halved: 200 x
+// 6144 of 256, 512, 1,024, 2,048 and 4,096 columns 22.4, 32.6, 53.9, 96.5, 183 and 19.7, 29.9, 50.9, 93.6, 178; 700 x 3072 34.5, 48.4, 81.9, 151, 281 and
+// 28.9, 45.7, 80.1, 151, 287; in one round, 200 x 3072 16.6, 22.4, 35.0 and 14.0, 21.4, 36.2, 256 x 2048 of
+// 768 and 1,024 25.1, 29.3 and 22.4, 27.4 (of 256 columns 32 x 32 are the faster ones with fewer halves than 1.4 a unit: 600 x 1024 13.2, halved 15.3).
+static bool halved(long long M, long long N, int K) {
+  const long long m = (M + 63) / 64, rounds = (m * ((N + 63) / 64) + 255) / 256, halves = m * ((N + 31) / 32);
+  return K <= 1024 && (rounds == 1 ? (K < 512 ? halves > 358 : halves <= 256) : rounds <= 3 && halves <= 256 * (2 * rounds - 1));
+}
+
 // Whether the gate is best made in the product's kernel (1), or of the packed product's rows by a kernel of its own (0). A block takes both
 // rows of w of an output, so a gated product of few outputs has half the packed one's blocks and as many more units idle: us at 1 and
 // 17 rows, here and packed (before this kernel was there): 512 of 8,192 columns 38.1, 47.3 and 25.8, 35.8 (25.4, 35.5); 1,024 of 3,072 18.6,
@@ -816,7 +826,10 @@ extern "C" int nhv_sum_parts_float32(const void* parts, int count, const void* x
 extern "C" int nhv_gemm_float32_gated_pays(const void* x, const void* w, int M, int N, int K) {
   const bool wide = K % 4 == 0 && (uintptr_t)x % 16 == 0 && (uintptr_t)w % 16 == 0;
   const bool whole = whole_pieces(x, w, K);
-  return (gated_tile(M, N, whole).cost - plain_tile(M, 2ll * N, whole).cost) * (wide ? 5.6 : 28.0) * K / 3072 <= 2.0;
+  const bool halves = whole && halved(M, N, K);
+  const Choice gated = gated_tile(M, N, whole && !halves);
+  if (halves && gated.tile == 4) return 1;                 // (the packed product's larger blocks cost the same 4 us more: 1,000 x 1024 of 256 15.6 here, packed 21.2)
+  return (gated.cost - plain_tile(M, 2ll * N, whole).cost) * (wide ? 5.6 : 28.0) * K / 3072 <= 2.0;
 }
 
 extern "C" int nhv_gemm_float32_gated(const void* x, const void* w, const void* bias, void* y, int M, int N, int K, int act, float limit,
@@ -829,7 +842,7 @@ extern "C" int nhv_gemm_float32_gated(const void* x, const void* w, const void* 
   const NhvGate gate = {act, limit, alpha, offset};
   const float *xf = (const float*)x, *wf = (const float*)w, *bf = (const float*)bias;
   float* yf = (float*)y;
-  const bool whole = whole_pieces(x, w, K);
+  const bool whole = whole_pieces(x, w, K) && !halved(M, N, K);
   switch (gated_tile(M, N, whole).tile) {
     case 0: launch<1, 2, 1, true>(xf, wf, bf, yf, M, N, K, gate, s); break;
     case 1: launch<2, 2, 1, true>(xf, wf, bf, yf, M, N, K, gate, s); break;

@@ -387,9 +387,10 @@ def test_float32_linear_in_all_its_tiles(ops, N, K):
         last = y
 
 
-@pytest.mark.parametrize("M,N,K", [(1090, 4100, 64), (1090, 4100, 70), (577, 4130, 256), (577, 4130, 33), (321, 4096, 1000)])
+@pytest.mark.parametrize("M,N,K", [(1090, 4100, 64), (1090, 4100, 70), (577, 4130, 256), (577, 4130, 33), (321, 4096, 1000), (190, 6150, 256), (200, 3080, 288),
+                                   (250, 2047, 768), (700, 3072, 1024)])
 def test_float32_linear_in_tiles_of_64_rows(ops, M, N, K):
-    """Tiles of 64 x 64 and 64 x 128, whole pieces of 32 columns and not, plain and gated: the rows that few rows alone give, bit for bit."""
+    """Tiles of 64 x 64 and 64 x 128, whole pieces of 32 columns and not, plain and gated (halved or not): the rows that few rows alone give, bit for bit."""
     x, w, b = rnd(M, K, seed=121), rnd(2 * N, K, seed=122), rnd(2 * N, seed=123)
     y, g = ops.linear(x, w[:N], b[:N]), ops.gated_linear(x, w, "silu", b)
     for rows in (slice(0, 16), slice(M - 5, M), slice(60, 70)):
