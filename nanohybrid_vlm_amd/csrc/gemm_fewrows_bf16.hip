@@ -1115,18 +1115,18 @@ struct Form {
 
 // Blocks of 8 outputs, by lines, for a bfloat16 result of 1,025 to 2,048 outputs without residual, where the tiles above have 8 rows of w a block
 // as well: they differ by a block's fixed cost and by how x comes. Measured over nine numbers of outputs by twelve of columns (2,048 to 8,192)
-// at ten numbers of rows; time by blocks of 8 over the tiles': from 12 rows on 0.55 to 0.99 everywhere; up to 2,304 columns 0.91 to 1.01 from 4 rows on;
-// with more, from where w has 2,048 x 2,816 entries, 0.90 to 1.0 at 6 and 7 rows (below that 0.95 to 1.07: 1,536 of 3,584 1.05, 1,040 of 5,120 1.07), 0.90
+// at ten numbers of rows; time by blocks of 8 over the tiles': from 9 rows on 0.55 to 1.0 nearly everywhere; up to 2,304 columns 0.91 to 1.01 from 4 rows on;
+// with more, from where w has 2,048 x 2,816 entries, 0.90 to 1.0 at 6 and 7 rows (below that 0.95 to 1.0 for 2,816 and 3,072 columns, up to 1.07 for others: 1,536 of 3,584 1.05, 1,040 of 5,120 1.07), 0.90
 // to 1.0 at 8 (below 0.98 to 1.07 beyond 3,072 columns). At 4 and 5 rows 2,048 of 3,072 0.99 and 0.98, of 4,096 0.97 and 0.95, but 1,280 of 3,584 1.05 and
 // 1.04, 1,536 of 5,120 1.02 and 1.0. us: 2,048 of 2,048 at 4 and 16 rows 4.9, 5.2 and 4.8, 4.9; of 4,096 at 4 and 7 6.9, 7.2 and 6.6, 6.8; of 12,288 at 8 and 16 16.9,
 // 17.5 and 14.7, 15.2. ``scaled``: such a block takes 0.5 us more and the tiles 0.1: below those 2,048 x 2,816 entries 1.0 to 1.13 at 6 to 8 rows (2,048 of 2,560 1.08,
-// 1,040 of 5,120 1.13), from there on 0.95 to 1.02; at 12 and 16 rows 0.83 to 1.03 for 2,816 to 4,096 columns, up to 1.09 for others, but 0.57 to 0.71 where x
+// 1,040 of 5,120 1.13), from there on 0.95 to 1.02; at 12 and 16 rows 0.83 to 1.03 for 2,816 to 4,096 columns (2,304: 0.96 to 1.0 and 0.92 to 0.98), up to 1.09 for others, but 0.57 to 0.71 where x
 // no longer fits beside w in the tiles' LDS (16 rows of 4,608 columns, 12 of 6,144).
 static bool half_plan(bool scaled, int M, int N, int K) {
   if (N <= 1024 || N > 2048) return false;
   const bool many = (long long)N * K >= 2048 * 2816;
-  if (scaled) return (M >= 6 && many && (K <= 5120 || M >= 8)) || (M >= 12 && K >= 2816 && K <= 4096) || (M >= 8 && M * K >= 16 * 4608);
-  if (M >= 12 || K <= 2304 || (M >= 8 && K <= 3072)) return M >= 4;
+  if (scaled) return (M >= 6 && many && (K <= 5120 || M >= 8)) || (M >= 12 && K > (M >= 14 ? 2048 : 2560) && K <= 4096) || (M >= 8 && M * K >= 16 * 4608);
+  if (M >= 9 || K <= 2304 || (M >= 8 && K <= 3072) || (M >= 6 && K > 2560 && K <= 3072)) return M >= 4;
   if (!many || M < 4 || (K > 5120 && M < 8)) return false;
   return M >= 6 || (K <= 4096 && N >= 1920) || (M == 5 && K >= 4096);
 }
@@ -1140,9 +1140,9 @@ static bool half_plan(bool scaled, int M, int N, int K) {
 // outputs of 4,096 columns 7.1 us by the tiles and 7.8 at 1 row, 7.4 and 7.9 at 4; 3,072 of 2,048 1.02, 1.03, 0.96, 0.99, of 6,144 9.9 and 9.8, 10.5 and 9.9.
 static bool lines_lose(const Form& p, int M, int N, int K) {
   if (p.banded) return K == 2048 && (N < 2816 || M == 1);
-  if (p.floats) return K % 2048 == 0 && N < (K == 2048 && M <= 2 ? 3200 : 3072);
+  if (p.floats) return K % 2048 == 0 && N < (K > 2048 ? 3072 : M <= 2 ? 3200 : 2944);
   if (p.residual) return p.scaled && K == 2048 && N < 2944 && M < 4;
-  return p.scaled && (K == 2048 ? N < 3072 : N < 2944 && M <= 2 && K > 2304 && K <= 3072);
+  return p.scaled && (K == 2048 ? N < (M < 4 ? 3072 : 2944) : N < 2944 && M <= 2 && K > 2304 && K <= 3072);
 }
 
 // Where the rows of w are enough for it, by what was measured at 1, 4, 8, 12 and 16 rows (us before and with it): not for 4,096 outputs
