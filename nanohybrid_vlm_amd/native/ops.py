@@ -18,7 +18,7 @@ import torch
 
 from . import library
 
-CORE_SOURCES = ["error.hip", "elementwise.hip", "gemm_generic.hip", "gemm_float32.hip", "gemm_skinny_bf16.hip", "gemm_fewrows_bf16.hip", "gemm_lines_bf16.hip",
+CORE_SOURCES = ["error.hip", "elementwise.hip", "gemm_generic.hip", "gemm_float32.hip", "gemm_skinny_bf16.hip", "gemm_fewrows_bf16.hip", "gemm_lines_bf16.hip", "gemm_phases_bf16.hip",
                 "attention_generic.hip", "attention_float32.hip", "sampling.hip", "measure.hip", "stream_mixing.hip", "delta_rule.hip", "delta_chunks.hip", "parallel_block.hip", "latent_attention.hip",
                 "routed_experts.hip", "hyper_streams.hip", "head_outputs.hip", "sandwich_norms.hip", "linear_recurrence.hip"]
 BLAS_SOURCES = ["error.hip", "gemm_library.hip"]                                                   # the vendor's matrix library, algorithm by number
@@ -879,6 +879,16 @@ class NativeBackend:
             how = self.chosen.get((M, w.shape[0], K, False, False))
         return 0 if how is not None and how >= 0 else splits
 
+    def _by_phases(self, x, w, out, bias, gated: bool, gate: "Gate") -> bool:
+        """A gated or activated product of many rows in one kernel, where that is the faster way (gemm_phases_bf16.hip; it hangs on the
+        shape alone); else False."""
+        (M, K), N = x.shape, out.shape[1]
+        if not (self.few_rows < M and x.dtype == out.dtype == torch.bfloat16 and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0
+                and (bias is None or bias.data_ptr() % 8 == 0) and self.lib.nhv_gemm_phases_pays(M, N, K, int(gated))):
+            return False
+        self._call("nhv_gemm_phases_bf16", _ptr(x), _ptr(w), _ptr(bias), _ptr(out), M, N, K, int(gated), *gate.args(), _stream())
+        return True
+
     def linear_parts(self, x, w):
         """x W^T as float parts [parts, rows, out] whose sum it is, or None where another way is the faster one."""
         splits = self._by_lines(x, w, w.shape[0], False)
@@ -976,7 +986,7 @@ class NativeBackend:
 
     def gated_linear(self, x, w, out, gate=None, bias=None) -> bool:
         """A gate (a ``Gate``; None: SiLU) of x Wg^T and x Wu^T (+ bias) in one kernel, if this batch is one for the
-        few-rows kernel or the one for up to 96 rows; else False. (SiLU without bias may also be one for the kernel of up to 64 rows; in
+        few-rows kernel, the one for up to 96 rows or the one for many; else False. (SiLU without bias may also be one for the kernel of up to 64 rows; in
         float32 most batches are.)"""
         M, K = x.shape
         if x.dtype == torch.float32:
@@ -986,6 +996,8 @@ class NativeBackend:
             return True
         if self._by_lines(x, w, out.shape[1], True):
             self._call("nhv_gemm_lines_bf16", _ptr(x), _ptr(w), _ptr(bias), _ptr(out), M, out.shape[1], K, 1, *(gate or Gate()).args(), _stream())
+            return True
+        if self._by_phases(x, w, out, bias, True, gate or Gate()):
             return True
         if bias is not None or (gate is not None and gate.act != 0):
             if x.dtype == torch.bfloat16 and K % 8 == 0 and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0 and M <= self.few_rows:
@@ -1006,9 +1018,11 @@ class NativeBackend:
 
     def activated_linear(self, x, w, out, act: int) -> bool:
         """act(x W^T) in one kernel, if this batch is one for the few-rows kernel and no library algorithm was found
-        faster for the shape; else False. ``act``: a value of ``PLAIN_ACTIVATIONS``."""
+        faster for the shape, or one for the kernel of many rows; else False. ``act``: a value of ``PLAIN_ACTIVATIONS``."""
         M, K = x.shape
-        if not (x.dtype == torch.bfloat16 and K % 8 == 0 and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0 and M <= self.few_rows):
+        if M > self.few_rows:
+            return self._by_phases(x, w, out, None, False, Gate(act))
+        if not (x.dtype == torch.bfloat16 and K % 8 == 0 and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0):
             return False
         if not self.own_kernels_only:
             how = self._choose(x, w, out)

@@ -372,6 +372,60 @@ def test_gated_linear(ops, M, I, K):
             backend.own_kernels_only = False
 
 
+@pytest.mark.parametrize("gated", [True, False])
+@pytest.mark.parametrize("M,N,K", [(1, 8, 128), (255, 136, 256), (256, 256, 128), (257, 1000, 384), (300, 264, 1152), (2049, 520, 256), (4400, 2200, 128), (700, 9728, 640)])
+def test_gates_and_activations_of_many_rows(ops, M, N, K, gated):
+    """Edges of the tiles of 256 x 256, two pieces of 64 columns and more, one tile a block and several, more than eight tiles of rows, every gate with and
+    without biases and every activation: against float64. A float sum of K products is off by K^(1/2) roundings of 2^-24 of its size at most,
+    which rounding the result to 8 bits (2^-9 of it) hides. Nothing behind the last row is written."""
+    b = ops.backend()
+    x = rnd(M, K, dtype=torch.bfloat16, seed=131)
+    w = rnd((2 if gated else 1) * N, K, dtype=torch.bfloat16, seed=132, scale=2 * K ** -0.5)
+    sums = x.double() @ w.double().T
+    bias = rnd(2 * N, dtype=torch.bfloat16, seed=133)
+    for act in range(3):
+        for with_bias in ((False, True) if gated else (False,)):
+            gate = ops.Gate(act, 1.5, 1.702, 1.0)
+            out = torch.full((M + 1, N), 7.0, dtype=torch.bfloat16, device="cuda")
+            b._call("nhv_gemm_phases_bf16", ops._ptr(x), ops._ptr(w), ops._ptr(bias if with_bias else None), ops._ptr(out), M, N, K, int(gated),
+                    *gate.args(), ops._stream())
+            z = sums + bias.double() if with_bias else sums
+            g = z[:, :N]
+            if gated and act == 2:
+                g = g.clamp(max=1.5)
+                want = g * torch.sigmoid(1.702 * g) * (z[:, N:].clamp(-1.5, 1.5) + 1.0)
+            else:
+                silu, gelu = g * torch.sigmoid(g), torch.nn.functional.gelu(g, approximate="tanh")
+                want = (silu, gelu, g.clamp(min=0).square())[act] * (z[:, N:] if gated else 1.0)
+            torch.testing.assert_close(out[:M].double(), want, rtol=2.0 ** -8, atol=1e-4)
+            assert bool((out[M] == 7.0).all())
+
+
+def test_many_rows_take_the_kernel_that_gates_them_where_it_pays(ops):
+    """By the share of the tiles' rounds that are outputs; a bias goes with it; a step of the same rows gives the same bits."""
+    pays = ops.backend().lib.nhv_gemm_phases_pays
+    assert [pays(*size) for size in ((2048, 12288, 4096, 1), (1866, 12288, 4096, 1), (600, 12288, 4096, 1), (97, 12288, 4096, 1), (2048, 12288, 4096 + 64, 1),
+                                     (2048, 12284, 4096, 1), (1925, 6144, 2048, 0), (1000, 6144, 2048, 0))] == [1, 1, 0, 0, 0, 0, 1, 0]
+    x, w = rnd(1300, 512, dtype=torch.bfloat16, seed=134), rnd(2 * 8192, 512, dtype=torch.bfloat16, seed=135, scale=512 ** -0.5)
+    bias = rnd(2 * 8192, dtype=torch.bfloat16, seed=136)
+    sums = x.double() @ w.double().T
+    # (against float64: gates of rounded rows are off by more, 2^-9 (|h'(g) g u| + 2 |y|), 0.1 at the largest of these)
+    bound = dict(rtol=2.0 ** -8, atol=1e-4)
+    for gate, b in (("silu", None), ("gelu_tanh", bias), (ops.Gate(2, 7.0, 1.702, 1.0), bias)):
+        assert ops.backend().gated_linear(x, w, torch.empty(1300, 8192, dtype=torch.bfloat16, device="cuda"), ops.gate_of(gate), b)
+        y = ops.gated_linear(x, w, gate, b)
+        g, u = (sums if b is None else sums + b.double()).chunk(2, dim=1)
+        if gate == "silu":
+            want = g * torch.sigmoid(g) * u
+        elif gate == "gelu_tanh":
+            want = torch.nn.functional.gelu(g, approximate="tanh") * u
+        else:
+            want = g.clamp(max=7.0) * torch.sigmoid(1.702 * g.clamp(max=7.0)) * (u.clamp(-7.0, 7.0) + 1.0)
+        torch.testing.assert_close(y.double(), want, **bound)
+        assert torch.equal(y, ops.gated_linear(x, w, gate, b))
+    torch.testing.assert_close(ops.activated_linear(x, w[:8192], "gelu_tanh").double(), torch.nn.functional.gelu(sums[:, :8192], approximate="tanh"), **bound)
+
+
 @pytest.mark.parametrize("N,K", [(1, 1), (17, 130), (48, 16), (130, 20), (65, 516), (300, 2064), (16400, 36), (24000, 7), (2500, 68), (2100, 331)])
 def test_float32_linear_in_all_its_tiles(ops, N, K):
     """Every tile that the number of rows and columns can choose, K below and beyond eight blocks of 16, ends inside a block of
