@@ -378,6 +378,17 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void p
         for (int r = 0; r < RT; ++r) o[r][dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(va, pa[r][a], o[r][dt], 0, 0, 0);
       }
     }
+    // V^T operands are read eight ahead of the one that is multiplied. (Left to itself the compiler reads two, waits for them, and multiplies: us
+    // so and now, 2,048 tokens after 14,336 502, 485; alone 59.1, 54.9; 512 after 4,000 77.9, 71.1; 901, 400 and 700 tokens 34.6, 33.1; 1 after 300,
+    // 17 after 40 and 333 after 1,000 27.2, 25.8. Two ahead 499, 58.0, 76.8; four 487, 55.9, 71.7. The same for the first product's operands: nothing.)
+    constexpr int OPERANDS = DTILES * KT / 2, AHEAD = OPERANDS < 8 ? OPERANDS : 8, DS_READ = 0x100, MATRIX = 0x8;
+    __builtin_amdgcn_sched_group_barrier(DS_READ, 2 * AHEAD, 0);
+#pragma unroll
+    for (int i = 0; i < OPERANDS - AHEAD; ++i) {
+      __builtin_amdgcn_sched_group_barrier(MATRIX, RT, 0);
+      __builtin_amdgcn_sched_group_barrier(DS_READ, 2, 0);
+    }
+    __builtin_amdgcn_sched_group_barrier(MATRIX, AHEAD * RT, 0);
   };
 
   auto run = [&](int kb, const bf16_t* k_s, const bf16_t* v_s) {
