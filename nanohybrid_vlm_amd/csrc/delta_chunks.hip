@@ -19,7 +19,12 @@
 //    took 101 us for 2,201 tokens of 16 heads of 128);
 //  - nhv_delta_chunks: a request's chunks in order, as float matrix products (v_mfma_f32_16x16x4_f32).
 // The second is a chain of chunks, and what it lasts is what a chunk waits for (two rows of dependent matrix instructions and
-// one exchange between the waves: 1.05 us a chunk), not its arithmetic; the token-by-token kernel takes 0.36 us a token.
+// one exchange between the waves: 0.82 us a chunk), not its arithmetic; the token-by-token kernel takes 0.36 us a token. Eight
+// waves a block, a tile each, wait longer for each other (99 us where four took 91).
+// us, before and now, of the preparation (which brings W and R into the second kernel's order) and of the chain (whose loads are
+// whole kilobytes, whose results are stored without a branch, and which multiplies R while the shares come back): portions of 1,500 and 764 tokens, 16 heads of
+// 128, 75, 77 and 88, 77; of 64 53, 56 and 55, 49; 8 heads of 256 on 128 108, 114 and 171, 140; 24 of 80 tokens, 16 heads of 128, 67, 69 and 69, 54; 8,000 tokens 248, 274
+// and 446, 389.
 // Portions of 1,500 and 701 tokens, 16 heads of 128, with the update of the kept inputs and the read-out's norm: 198 us where the
 // separate kernels take 638; one of 8,000 770 against 3,204. The blocks of the preparation are requests by the longest portion:
 // for 2,000 tokens beside 60 decoded ones 98 of 100 are empty, which is 16 us of 290 (a search for each place's request gave
@@ -56,7 +61,7 @@ struct DeltaIn {
 };
 
 struct DeltaChunks {                         // per (place, head); a chunk's place: cu[req] / 16 + req + its number in the request
-  float *w, *r;                              // [16][Dp]
+  float *w, *r;                              // [Dp / 16][4][16][4]: of a tile of 16 channels, four channels, their tokens
   float *k;                                  // [Dp][16]
   float *v;                                  // [E][16]
   float *o;                                  // [E][16]: B V'
@@ -241,17 +246,15 @@ __global__ __launch_bounds__(256, 4) void delta_chunks_prepare_kernel(const Delt
       for (int j = 0; j < t; ++j) x[t] = fmaf(-A[t][j], x[j], x[t]);
     }
     if (key) {
-      float* w = to.w + place * NHV_CHUNK * Dp + c;
-      float* r = to.r + place * NHV_CHUNK * Dp + c;
       float* k = to.k + (place * Dp + c) * NHV_CHUNK;
 #pragma unroll
       for (int t = 0; t < NHV_CHUNK; ++t) {
         asm volatile("" ::: "memory");
-        w[t * Dp] = x[t];
+        ks[t * LD + c] = x[t];
         float y = qs[t * LD + c];
 #pragma unroll
         for (int j = 0; j <= t; ++j) y = fmaf(-B[t][j], x[j], y);
-        r[t * Dp] = y;
+        qs[t * LD + c] = y;
       }
 #pragma unroll
       for (int t = 0; t < NHV_CHUNK; t += 4) {
@@ -279,6 +282,15 @@ __global__ __launch_bounds__(256, 4) void delta_chunks_prepare_kernel(const Delt
 #pragma unroll
       for (int t = 0; t < NHV_CHUNK; t += 4) *reinterpret_cast<floatx4*>(v + t) = floatx4{x[t], x[t + 1], x[t + 2], x[t + 3]};
     }
+  }
+  __syncthreads();
+  // W and R as the second kernel's lanes take them: a load of a tile is a kilobyte in a row (with rows of Dp entries, sixteen times
+  // 64 bytes, which come to a compute unit half as fast)
+  for (int x = tid; x < 4 * Dp; x += 256) {
+    const int at = (x & 15) * LD + (x >> 4) * 4;
+    const size_t out = place * NHV_CHUNK * Dp + 4 * x;
+    *reinterpret_cast<floatx4*>(to.w + out) = *reinterpret_cast<const floatx4*>(ks + at);
+    *reinterpret_cast<floatx4*>(to.r + out) = *reinterpret_cast<const floatx4*>(qs + at);
   }
 }
 
@@ -340,7 +352,7 @@ __global__ __launch_bounds__(256, TPW <= 2 ? 2 : 1) void delta_chunks_kernel(con
                                                            const int* __restrict__ state_slots, int H, int D, int Dp, int E) {
   constexpr int AHEAD = TPW <= 2 ? 3 : 2;
   __shared__ __attribute__((aligned(16))) float share[2][4][64 * 4];
-  __shared__ float red[2][4][NHV_CHUNK][17];
+  __shared__ __attribute__((aligned(16))) float red[2][4][64 * 4];
   const int req = blockIdx.z, h = blockIdx.x, e0 = blockIdx.y * 16;
   const int first = cu[req], end = cu[req + 1];
   if (end <= first) return;                  // (the same for the whole block)
@@ -360,35 +372,41 @@ __global__ __launch_bounds__(256, TPW <= 2 ? 2 : 1) void delta_chunks_kernel(con
     }
   const int chunks = (end - first + NHV_CHUNK - 1) / NHV_CHUNK;
   const size_t place0 = (size_t)(first / NHV_CHUNK) + req;
-  const int r_at = col * Dp + tile0 * 16 + grp * 4, k_at = (tile0 * 16 + col) * NHV_CHUNK + grp * 4, g_at = tile0 * 16 + grp * 4;
+  const int r_at = tile0 * 256 + lane * 4, k_at = (tile0 * 16 + col) * NHV_CHUNK + grp * 4, g_at = tile0 * 16 + grp * 4;
   const int v_at = e_mine * NHV_CHUNK + grp * 4;
   const int spare = (EVEN ? 0 : tiles) - 1;  // (a wave without a tile reads the last one's and leaves it unused)
   DeltaOperands<TPW> ops[AHEAD];
-  auto ask = [&](DeltaOperands<TPW>& x, int c) {
-    const size_t place = (place0 + min(c, chunks - 1)) * H + h;      // (always asked, so that the waits count the same loads on every way)
-    const float* wb = from.w + place * NHV_CHUNK * Dp;
-    const float* rb = from.r + place * NHV_CHUNK * Dp;
-    const float* kb = from.k + place * NHV_CHUNK * Dp;
-    const float* gb = from.decay + place * Dp;
+  const size_t place = place0 * H + h;
+  const float *wb = from.w + place * NHV_CHUNK * Dp, *rb = from.r + place * NHV_CHUNK * Dp, *kb = from.k + place * NHV_CHUNK * Dp;
+  const float *gb = from.decay + place * Dp, *vb = from.v + place * NHV_CHUNK * E, *ob = from.o + place * NHV_CHUNK * E;
+  int asked = 0;
+  auto ask = [&](DeltaOperands<TPW>& x) {    // (behind the last chunk: it again, so that the waits count the same loads on every way)
 #pragma unroll
     for (int i = 0; i < TPW; ++i) {
       const int back = EVEN ? 0 : max(tile0 + i - spare, 0);
-      x.w[i] = *reinterpret_cast<const floatx4*>(wb + (r_at + (i - back) * 16));
-      x.r[i] = *reinterpret_cast<const floatx4*>(rb + (r_at + (i - back) * 16));
-      x.g[i] = *reinterpret_cast<const floatx4*>(gb + (g_at + (i - back) * 16));
-      x.kk[i] = *reinterpret_cast<const floatx4*>(kb + (k_at + (i - back) * 16 * NHV_CHUNK));
+      x.w[i] = *reinterpret_cast<const floatx4*>(wb + (uint32_t)(r_at + (i - back) * 256));
+      x.r[i] = *reinterpret_cast<const floatx4*>(rb + (uint32_t)(r_at + (i - back) * 256));
+      x.g[i] = *reinterpret_cast<const floatx4*>(gb + (uint32_t)(g_at + (i - back) * 16));
+      x.kk[i] = *reinterpret_cast<const floatx4*>(kb + (uint32_t)(k_at + (i - back) * 16 * NHV_CHUNK));
     }
-    x.v = *reinterpret_cast<const floatx4*>(from.v + place * NHV_CHUNK * E + v_at);
-    x.o = from.o[place * NHV_CHUNK * E + v_at + wave];
+    x.v = *reinterpret_cast<const floatx4*>(vb + (uint32_t)v_at);
+    x.o = ob[(uint32_t)(v_at + wave)];
+    const bool more = ++asked < chunks;
+    const size_t rows = more ? (size_t)H * NHV_CHUNK * Dp : 0, columns = more ? (size_t)H * NHV_CHUNK * E : 0;
+    wb += rows, rb += rows, kb += rows, gb += more ? (size_t)H * Dp : 0, vb += columns, ob += columns;
   };
-  const int o_at = (tid >> 4) * H * E + (tid & 15);
-  auto emit = [&](int c) {                   // the waves' shares of chunk c added up and written
-    const int t = first + c * NHV_CHUNK + (tid >> 4), e = e0 + (tid & 15);
-    float sum = 0.f;
+  // wave w writes tokens 4 grp + w of a chunk, the sum of the four waves' shares. Tokens behind the request's last one and columns behind E lie
+  // behind the end of what is described here, and are not written: without a branch the products go on beside it.
+  const uint32_t o_at = column ? (uint32_t)((grp * 4 + wave) * H * E + col) * 4 : 0x80000000u;
+  auto emit = [&](const float* part, int c) {
+    const int t = first + c * NHV_CHUNK;
+    const int bytes = (min(NHV_CHUNK, end - t) * H * E - h * E - e0) * 4;
+    __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, ((part[0] + part[1]) + part[2]) + part[3]),
+                                          __builtin_amdgcn_make_buffer_rsrc(out + ((size_t)t * H + h) * E + e0, 0, bytes, 0x00020000), o_at, 0, 0);
+  };
+  auto parts = [&](int c, float* part) {
 #pragma unroll
-    for (int w = 0; w < 4; ++w) sum += red[c & 1][w][tid >> 4][tid & 15];
-    float* ob = out + ((size_t)(first + c * NHV_CHUNK) * H + h) * E + e0;
-    if (t < end && e < E) ob[o_at] = sum;
+    for (int w = 0; w < 4; ++w) part[w] = red[c & 1][w][lane * 4 + wave];
   };
   auto step = [&](DeltaOperands<TPW>& x, int c) {
     floatx4 p = {0.f, 0.f, 0.f, 0.f}, p2 = p, o2 = p;
@@ -401,7 +419,16 @@ __global__ __launch_bounds__(256, TPW <= 2 ? 2 : 1) void delta_chunks_kernel(con
       p2 = __builtin_amdgcn_mfma_f32_16x16x4f32(x.w[i][3], S[i][3], p2, 0, 0, 0);
     }
     *reinterpret_cast<floatx4*>(&share[c & 1][wave][lane * 4]) = p + p2;
-    // (while the shares meet; R holds - B W already: what is left of B U is B V')
+    // a barrier for LDS alone: __syncthreads would also wait for the loads that were asked for ahead. A buffer of shares is
+    // read right behind its barrier and written again only behind the next one.
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    floatx4 u = x.v, got[4];
+    float part[4];
+#pragma unroll
+    for (int w = 0; w < 4; ++w) got[w] = *reinterpret_cast<const floatx4*>(&share[c & 1][w][lane * 4]);
+    if (c > 0) parts(c - 1, part);
+    __builtin_amdgcn_sched_barrier(0);
+    // (while the shares come; R holds - B W already: what is left of B U is B V')
     floatx4 o = {wave == 0 ? x.o : 0.f, wave == 1 ? x.o : 0.f, wave == 2 ? x.o : 0.f, wave == 3 ? x.o : 0.f};
 #pragma unroll
     for (int i = 0; i < TPW; ++i) {
@@ -411,30 +438,21 @@ __global__ __launch_bounds__(256, TPW <= 2 ? 2 : 1) void delta_chunks_kernel(con
       o = __builtin_amdgcn_mfma_f32_16x16x4f32(x.r[i][2], S[i][2], o, 0, 0, 0);
       o2 = __builtin_amdgcn_mfma_f32_16x16x4f32(x.r[i][3], S[i][3], o2, 0, 0, 0);
     }
+    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int i = 0; i < TPW; ++i) S[i] *= x.g[i];
-    // a barrier for LDS alone: __syncthreads would also wait for the loads that were asked for ahead. A buffer of shares is
-    // read right behind its barrier and written again only behind the next one.
-    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-    floatx4 u = x.v;
-    {
-      floatx4 sum = *reinterpret_cast<const floatx4*>(&share[c & 1][0][lane * 4]);
-#pragma unroll
-      for (int w = 1; w < 4; ++w) sum += *reinterpret_cast<const floatx4*>(&share[c & 1][w][lane * 4]);
-      u -= sum;
-    }
+    u -= ((got[0] + got[1]) + got[2]) + got[3];
 #pragma unroll
     for (int j = 0; j < 4; ++j)
 #pragma unroll
       for (int i = 0; i < TPW; ++i)
         if (EVEN || tile0 + i < tiles) S[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(x.kk[i][j], u[j], S[i], 0, 0, 0);
-    ask(x, c + AHEAD);
-    if (c > 0) emit(c - 1);                  // (while the products are under way; written behind the last barrier but one)
-#pragma unroll
-    for (int j = 0; j < 4; ++j) red[c & 1][wave][grp * 4 + j][col] = o[j] + o2[j];
+    ask(x);
+    if (c > 0) emit(part, c - 1);            // (while the products are under way; written behind the last barrier but one)
+    *reinterpret_cast<floatx4*>(&red[c & 1][wave][lane * 4]) = o + o2;
   };
 #pragma unroll
-  for (int i = 0; i < AHEAD; ++i) ask(ops[i], i);
+  for (int i = 0; i < AHEAD; ++i) ask(ops[i]);
   int c = 0;
   for (; c + AHEAD <= chunks; c += AHEAD) {
 #pragma unroll
@@ -444,7 +462,9 @@ __global__ __launch_bounds__(256, TPW <= 2 ? 2 : 1) void delta_chunks_kernel(con
   for (int i = 0; i < AHEAD - 1; ++i)
     if (c + i < chunks) step(ops[i], c + i);
   __syncthreads();
-  emit(chunks - 1);
+  float part[4];
+  parts(chunks - 1, part);
+  emit(part, chunks - 1);
 #pragma unroll
   for (int i = 0; i < TPW; ++i)
 #pragma unroll
