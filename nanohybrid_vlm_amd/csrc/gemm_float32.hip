@@ -412,12 +412,20 @@ static void launch_tiles(const float* x, const float* w, const float* bias, floa
 // us, tiles of 64 x 64 of 16x16x32 instructions in brackets: 517 x 4096 . 1024 47 (53), gated 517 x 3072 . 1024 56 (67), 300 x 6144 . 2048 106 (140),
 // 1,500 x 12,288 . 2048 454 (550).
 // Rows are whole pieces of 32 columns on 16-byte boundaries (whole_pieces).
-template <int CT, bool GATED, bool PARTS>
-__global__ __launch_bounds__(256, CT == 2 ? 2 : 3) void gemm_float32_blocks_kernel(const float* __restrict__ x, const float* __restrict__ w,
+//
+// WAVES 8: 128 x 128 outputs, a wave 32 by 64. Half the loads and half the parts taken from floats a product, but what is read from LDS for
+// it is the same, and eight waves that have all met wait for it: 1,125 clocks a piece, beside which nothing ran. So the middle parts
+// of the next piece are read among this one's last products, behind a barrier that stands between its third and its fourth kind of
+// product. Taken where its rounds of blocks are half of what the smaller tiles need (big_tiles). us, 64 x 128 and 128 x 128: 517 x 3072 . 1024 gated 60, 52 (read all at
+// once 56), 416 rows 50, 45, 1,000 x 4096 . 1024 58, 52, 1,049 x 3,072 . 1024 56, 54; without the matrix instructions 46 for the 56, without loads 44, matrix
+// instructions alone 34. Three pieces under way in registers: the same; 4 waves of 64 x 64, whose accumulators move between register files, 70.
+template <int CT, bool GATED, bool PARTS, int WAVES>
+__global__ __launch_bounds__(64 * WAVES, CT == 2 ? 2 : 3) void gemm_float32_blocks_kernel(const float* __restrict__ x, const float* __restrict__ w,
                                                                                    const float* __restrict__ bias, float* __restrict__ y, int M, int N,
                                                                                    int K, int m_tiles, int n_tiles, NhvGate gate) {
   static_assert(!GATED || (CT == 2 && !PARTS), "a gate tile and its up tile");
-  constexpr int BM = 64, BN = 64 * CT, LOADS = (BM + BN) / 64, PLANE = (BM + BN) * PIECE, OUT = GATED ? BN / 2 : BN, TOTALS = PARTS ? 1 : CT;
+  static_assert(WAVES == 4 || !PARTS, "parts come from the smaller tiles");
+  constexpr int BM = 16 * WAVES, BN = 64 * CT, LOADS = (BM + BN) / BM, PLANE = (BM + BN) * PIECE, OUT = GATED ? BN / 2 : BN, TOTALS = PARTS ? 1 : CT;
   __shared__ __attribute__((aligned(16))) bf16_t rows[2][3 * PLANE];
   const int total_tiles = m_tiles * n_tiles, share = (total_tiles + 7) >> 3;
   const int tile = (blockIdx.x & 7) * share + (blockIdx.x >> 3);
@@ -426,7 +434,7 @@ __global__ __launch_bounds__(256, CT == 2 ? 2 : 3) void gemm_float32_blocks_kern
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, r32 = lane & 31, half = lane >> 5;
   const int mw = (wave >> 1) * 32, nw = (wave & 1) * 32 * CT;
   const int length = segment_length(K), begin = PARTS ? blockIdx.y * length : 0, end = PARTS ? min(K, begin + length) : K;
-  // what this thread brings of a piece: 16 bytes of each half of the 128 of rows row, row + 64, ...: an address that the wave shares, and
+  // what this thread brings of a piece: 16 bytes of each half of the 128 of rows row, row + BM, ...: an address that the wave shares, and
   // an offset (of less than 128 rows of less than 2^22 entries: 32 bits)
   const int col = (threadIdx.x & 3) * 4, row = threadIdx.x >> 2;
   const float* base[LOADS];
@@ -434,7 +442,7 @@ __global__ __launch_bounds__(256, CT == 2 ? 2 : 3) void gemm_float32_blocks_kern
 #pragma unroll
   for (int i = 0; i < LOADS; ++i) {
     // (gated: 32 gate rows and their 32 up rows in turn)
-    const int b = row + 64 * (i - 1), n = GATED ? n0 + (b >> 6) * 32 + (b & 31) : n0 + b;
+    const int b = row + BM * (i - 1), n = GATED ? n0 + (b >> 6) * 32 + (b & 31) : n0 + b;
     const int up = GATED ? __builtin_amdgcn_readfirstlane((b >> 5) & 1) : 0;
     base[i] = i == 0 ? x + (size_t)m0 * K : w + ((size_t)up * N + n0) * K;
     offset[i] = (uint32_t)(i == 0 ? min(row, M - 1 - m0) : min(n, N - 1) - n0) * (uint32_t)K;
@@ -450,7 +458,7 @@ __global__ __launch_bounds__(256, CT == 2 ? 2 : 3) void gemm_float32_blocks_kern
   };
   auto put = [&](int buf, int i_hold, int i) {
     const SplitFloats8 p = split_floats<false>(hold[i_hold][i][0], hold[i_hold][i][1]);
-    bf16_t* to = &rows[buf][64 * i * PIECE + to_row];
+    bf16_t* to = &rows[buf][BM * i * PIECE + to_row];
     *reinterpret_cast<bf16x8*>(to) = p.high;
     *reinterpret_cast<bf16x8*>(to + PLANE) = p.middle;
     *reinterpret_cast<bf16x8*>(to + 2 * PLANE) = p.rest;
@@ -486,20 +494,41 @@ __global__ __launch_bounds__(256, CT == 2 ? 2 : 3) void gemm_float32_blocks_kern
     a_at[s] = (mw + r32) * PIECE + (((2 * s + half) ^ (r32 >> 2 & 3)) << 3);
     b_at[s] = (BM + nw + r32) * PIECE + (((2 * s + half) ^ (r32 >> 2 & 3)) << 3);
   }
+  constexpr bool EARLY = WAVES == 8;                     // the middle parts are read a piece ahead
+  auto part_of = [&](int buf, int at, int plane) { return *reinterpret_cast<const bf16x8*>(&rows[buf][at + plane * PLANE]); };
+  SplitFloats8 a[2], b[2][CT];
+  bf16x8 a_next[2], b_next[2][CT];
+  auto read_middle = [&](int buf) {
+#pragma unroll
+    for (int s = 0; s < 2; ++s) {
+      a_next[s] = part_of(buf, a_at[s], 1);
+#pragma unroll
+      for (int c = 0; c < CT; ++c) b_next[s][c] = part_of(buf, b_at[s] + 32 * c * PIECE, 1);
+    }
+  };
+  if (EARLY) read_middle(0);
   for (int k0 = begin; k0 < end; k0 += AHEAD * PIECE) {
 #pragma unroll
     for (int d = 0; d < AHEAD; ++d) {                    // (piece d lies in buffer d)
       const int k = k0 + d * PIECE, buf = d;
       if (k >= end) break;
       // the parts in the order in which the products need them
-      SplitFloats8 a[2], b[2][CT];
-      auto part = [&](int at, int plane) { return *reinterpret_cast<const bf16x8*>(&rows[buf][at + plane * PLANE]); };
+      auto part = [&](int at, int plane) { return part_of(buf, at, plane); };
+      if (EARLY) {
 #pragma unroll
-      for (int s = 0; s < 2; ++s) a[s].middle = part(a_at[s], 1);
+        for (int s = 0; s < 2; ++s) {
+          a[s].middle = a_next[s];
 #pragma unroll
-      for (int s = 0; s < 2; ++s)
+          for (int c = 0; c < CT; ++c) b[s][c].middle = b_next[s][c];
+        }
+      } else {
 #pragma unroll
-        for (int c = 0; c < CT; ++c) b[s][c].middle = part(b_at[s] + 32 * c * PIECE, 1);
+        for (int s = 0; s < 2; ++s) a[s].middle = part(a_at[s], 1);
+#pragma unroll
+        for (int s = 0; s < 2; ++s)
+#pragma unroll
+          for (int c = 0; c < CT; ++c) b[s][c].middle = part(b_at[s] + 32 * c * PIECE, 1);
+      }
 #pragma unroll
       for (int s = 0; s < 2; ++s) a[s].rest = part(a_at[s], 2);
 #pragma unroll
@@ -519,15 +548,20 @@ __global__ __launch_bounds__(256, CT == 2 ? 2 : 3) void gemm_float32_blocks_kern
 #pragma unroll
           for (int c = 0; c < CT; ++c) split_product(step, a[s], b[s][c], acc[c], low[c]);
         if (step < LOADS) put(buf ^ 1, d ^ 1, step);
+        if (EARLY && step == LOADS - 1) ask(d ^ 1, k + (1 + AHEAD) * PIECE);
+        if (EARLY && step == 2) {
+          __syncthreads();
+          read_middle(buf ^ 1);
+        }
       }
-      ask(d ^ 1, k + (1 + AHEAD) * PIECE);
+      if (!EARLY) ask(d ^ 1, k + (1 + AHEAD) * PIECE);
       left -= PIECE;
       if (!PARTS && left == 0) {
         left = length;
         asm volatile("");                                // (a real branch)
         close();
       }
-      __syncthreads();
+      if (!EARLY) __syncthreads();
     }
   }
   if (PARTS) {
@@ -569,12 +603,12 @@ __global__ __launch_bounds__(256, CT == 2 ? 2 : 3) void gemm_float32_blocks_kern
   }
 }
 
-template <int CT, bool GATED, bool PARTS = false>
+template <int CT, bool GATED, bool PARTS = false, int WAVES = 4>
 static void launch_blocks(const float* x, const float* w, const float* bias, float* y, int M, int N, int K, const NhvGate& gate, hipStream_t s) {
   constexpr int COLS = GATED ? 32 * CT : 64 * CT;
-  const int m_tiles = (M + 63) / 64, n_tiles = (N + COLS - 1) / COLS;
-  const dim3 grid(8u * (unsigned)(((long long)m_tiles * n_tiles + 7) / 8), PARTS ? segments(K) : 1), block(256);
-  hipLaunchKernelGGL((gemm_float32_blocks_kernel<CT, GATED, PARTS>), grid, block, 0, s, x, w, bias, y, M, N, K, m_tiles, n_tiles, gate);
+  const int m_tiles = (M + 16 * WAVES - 1) / (16 * WAVES), n_tiles = (N + COLS - 1) / COLS;
+  const dim3 grid(8u * (unsigned)(((long long)m_tiles * n_tiles + 7) / 8), PARTS ? segments(K) : 1), block(64 * WAVES);
+  hipLaunchKernelGGL((gemm_float32_blocks_kernel<CT, GATED, PARTS, WAVES>), grid, block, 0, s, x, w, bias, y, M, N, K, m_tiles, n_tiles, gate);
 }
 
 static bool whole_pieces(const void* x, const void* w, int K) {
@@ -627,6 +661,16 @@ static Choice gated_tile(long long M, long long N, bool whole) {
   return best;
 }
 
+// Whether tiles of 128 x 128 rows of x and of w (gated: 64 outputs) are the faster ones: where tiles of 64 x 128 need twice the rounds of 256
+// blocks that these do; a first one that is hardly begun is little to save. Measured over 9,700 sizes (90 to 2,048 rows, 700 to 8,200 outputs of 256 to 4,096
+// columns; time over that of the choice without them): 1 round 0.86 and 0.88 gated, the worst 1.01 and 1.03 (from 257 smaller blocks on 1.17); 2 rounds 0.87 and 0.91,
+// 1.01; 3 0.89 and 0.91, 1.0; 4 and more 0.92, 1.08. Elsewhere 0.9 to 1.57 (2 rounds where the others need 2).
+static bool big_tiles(long long M, long long N, bool whole, bool gated) {
+  const long long columns = gated ? 64 : 128, n = (N + columns - 1) / columns, blocks = (M + 127) / 128 * n, smaller = (M + 63) / 64 * n;
+  const long long rounds = (blocks + 255) / 256;
+  return whole && M > 64 && smaller > (2 * rounds - 1) * 256 + (rounds == 1 ? 44 : 0);
+}
+
 extern "C" int nhv_gemm_float32(const void* x, const void* w, const void* bias, void* y, int M, int N, int K, void* stream) {
   NHV_REQUIRE(M > 0 && N > 0 && K > 0, "gemm: bad sizes M=%d N=%d K=%d", M, N, K);
   NHV_REQUIRE(K < (1 << 30) && (((long long)M + 15) / 16) * (((long long)N + 15) / 16) < (1ll << 30), "gemm: too many rows (%d) for %d columns", M, N);
@@ -634,7 +678,7 @@ extern "C" int nhv_gemm_float32(const void* x, const void* w, const void* bias, 
   const float *xf = (const float*)x, *wf = (const float*)w, *bf = (const float*)bias;
   float* yf = (float*)y;
   const bool whole = whole_pieces(x, w, K);
-  switch (plain_tile(M, N, whole).tile) {
+  switch (big_tiles(M, N, whole, false) ? 8 : plain_tile(M, N, whole).tile) {
     case 0: launch<1, 1, 2, false>(xf, wf, bf, yf, M, N, K, {}, s); break;
     case 1: launch<1, 2, 1, false>(xf, wf, bf, yf, M, N, K, {}, s); break;
     case 2: launch<2, 2, 1, false>(xf, wf, bf, yf, M, N, K, {}, s); break;
@@ -645,6 +689,7 @@ extern "C" int nhv_gemm_float32(const void* x, const void* w, const void* bias, 
       else launch_tiles<2, 2, false>(xf, wf, bf, yf, M, N, K, {}, s);
       break;
     case 7: launch_blocks<2, false>(xf, wf, bf, yf, M, N, K, {}, s); break;
+    case 8: launch_blocks<2, false, false, 8>(xf, wf, bf, yf, M, N, K, {}, s); break;
     default: launch<2, 1, 2, false>(xf, wf, bf, yf, M, N, K, {}, s);
   }
   NHV_LAUNCH_CHECK("gemm_float32");
@@ -826,6 +871,7 @@ static bool halved(long long M, long long N, int K) {
 extern "C" int nhv_gemm_float32_gated_pays(const void* x, const void* w, int M, int N, int K) {
   const bool wide = K % 4 == 0 && (uintptr_t)x % 16 == 0 && (uintptr_t)w % 16 == 0;
   const bool whole = whole_pieces(x, w, K);
+  if (big_tiles(M, N, whole, true)) return 1;              // (as many blocks as the packed product)
   const bool halves = whole && halved(M, N, K);
   const Choice gated = gated_tile(M, N, whole && !halves);
   if (halves && gated.tile == 4) return 1;                 // (the packed product's larger blocks cost the same 4 us more: 1,000 x 1024 of 256 15.6 here, packed 21.2)
@@ -842,12 +888,13 @@ extern "C" int nhv_gemm_float32_gated(const void* x, const void* w, const void* 
   const NhvGate gate = {act, limit, alpha, offset};
   const float *xf = (const float*)x, *wf = (const float*)w, *bf = (const float*)bias;
   float* yf = (float*)y;
-  const bool whole = whole_pieces(x, w, K) && !halved(M, N, K);
-  switch (gated_tile(M, N, whole).tile) {
+  const bool big = big_tiles(M, N, whole_pieces(x, w, K), true), whole = whole_pieces(x, w, K) && !halved(M, N, K);
+  switch (big ? 5 : gated_tile(M, N, whole).tile) {
     case 0: launch<1, 2, 1, true>(xf, wf, bf, yf, M, N, K, gate, s); break;
     case 1: launch<2, 2, 1, true>(xf, wf, bf, yf, M, N, K, gate, s); break;
     case 2: launch<3, 2, 1, true>(xf, wf, bf, yf, M, N, K, gate, s); break;
     case 3: launch_tiles<1, 2, true>(xf, wf, bf, yf, M, N, K, gate, s); break;
+    case 5: launch_blocks<2, true, false, 8>(xf, wf, bf, yf, M, N, K, gate, s); break;
     default:
       if (whole) launch_blocks<2, true>(xf, wf, bf, yf, M, N, K, gate, s);
       else launch_tiles<2, 2, true>(xf, wf, bf, yf, M, N, K, gate, s);
