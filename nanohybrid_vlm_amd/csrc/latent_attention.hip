@@ -40,6 +40,30 @@ __device__ __forceinline__ void nhv_turn_pair(const T* s, T* d, int p, int rot, 
   d[b] = from_f32<T>(v * cs + u * sn);
 }
 
+// Pairs p to p + 7 (a multiple of 8) of a part of a multiple of 16 entries, source and result 16 bytes aligned: pieces of 16
+// bytes, for which the values are those of nhv_turn_pair.
+__device__ __forceinline__ void nhv_turn_eight_pairs(const bf16_t* s, bf16_t* d, int p, int rot, int halves, int pos, const double* freqs,
+                                                     float gain) {
+  typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+  const int lo = halves ? p : 2 * p, hi = halves ? p + rot / 2 : 2 * p + 8;
+  const bf16x8 in_lo = *reinterpret_cast<const bf16x8*>(s + lo), in_hi = *reinterpret_cast<const bf16x8*>(s + hi);
+  bf16x8 out_lo, out_hi;
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    float sn, cs;
+    nhv_turn_angle<bf16_t>(pos, freqs[p + i], gain, &sn, &cs);
+    const int e = 2 * i % 8;
+    const float u = (float)(halves ? in_lo[i] : i < 4 ? in_lo[e] : in_hi[e]);
+    const float v = (float)(halves ? in_hi[i] : i < 4 ? in_lo[e + 1] : in_hi[e + 1]);
+    const __bf16 a = (__bf16)(u * cs - v * sn), b = (__bf16)(v * cs + u * sn);
+    if (halves) out_lo[i] = a, out_hi[i] = b;
+    else if (i < 4) out_lo[e] = a, out_lo[e + 1] = b;
+    else out_hi[e] = a, out_hi[e + 1] = b;
+  }
+  *reinterpret_cast<bf16x8*>(d + lo) = out_lo;
+  *reinterpret_cast<bf16x8*>(d + hi) = out_hi;
+}
+
 // a: [T, A] rows of type TA. Query latent (q_rank > 0): columns q_off .. q_off + q_rank, normed with wq into cq [T, q_rank]. Latent:
 // columns c_off .. c_off + kv_rank normed with wc, then ``rot`` columns turned; both stored at slot_mapping[t] in
 // ``cache`` (rows of ``row`` entries; entries beyond kv_rank + rot become zeros). kv_rank 0: nothing is stored.
@@ -457,135 +481,112 @@ __global__ __launch_bounds__(64 * WAVES) void head_gemm_mfma_kernel(const bf16_t
   }
 }
 
-// The same for many rows (K <= HT_MAX_K): a block owns 64 rows of one head and walks over all of its outputs, 128 at a time.
-// The rows come into LDS once, whole rows of K entries; a wave takes 32 of the 128 outputs, with the matrix rows straight
-// from memory (L2), and the results go back through LDS so that rows are written in pieces of 16 bytes side by side.
-#define HT_ROWS 64
-#define HT_COLS 128
+// The same for many rows (K <= HT_MAX_K). Bound by the bytes of x, y and the gate: a wave owns 16 rows of one head, whose
+// entries it holds as operands, and the head's matrix comes into LDS once a block (up to 64 KB at a time), as operands in
+// the order in which they are read. Two tiles of 16 outputs are 32 outputs side by side: tile t's line i is output
+// 8 (i / 4) + 4 t + i % 4, so that a lane ends up with eight outputs in a row and writes (and reads the gate) in pieces of
+// 16 bytes, with nothing but the matrix behind a barrier. 4,220 rows of 16 heads: 128 to 192 entries and 64 turned, 44 us as
+// blocks of 64 rows that walk over the outputs with the rows in LDS and the matrix from memory, 24 so; 192 to 128 with a gate
+// per entry 32 and 23 (these bytes at 5 TB/s: 12). Blocks of 4, 8 and 16 waves 27, 25 and 24.
 #define HT_MAX_K 512
-template <int U>
-__global__ __launch_bounds__(256) void head_gemm_tile_kernel(const bf16_t* __restrict__ x, long long xs_t, long long xs_h,
-                                                             const bf16_t* __restrict__ w, bf16_t* __restrict__ y,
-                                                             long long ys_t, long long ys_h, const void* __restrict__ gate,
-                                                             int gate_mode, long long gs_t, int rows, int N, int K, int rot,
-                                                             int x_rot_off, int y_rot_off, int halves,
-                                                             const double* __restrict__ freqs, float gain,
-                                                             const int* __restrict__ positions, int vec_out, int vec_gate) {
+#define HT_LDS 65536
+template <int KS, int WAVES>
+__global__ __launch_bounds__(64 * WAVES) void head_gemm_rows_kernel(const bf16_t* __restrict__ x, long long xs_t, long long xs_h,
+                                                                    const bf16_t* __restrict__ w, bf16_t* __restrict__ y,
+                                                                    long long ys_t, long long ys_h, const void* __restrict__ gate,
+                                                                    int gate_mode, long long gs_t, int rows, int N, int K, int rot,
+                                                                    int x_rot_off, int y_rot_off, int halves,
+                                                                    const double* __restrict__ freqs, float gain,
+                                                                    const int* __restrict__ positions, int vec_out, int vec_gate,
+                                                                    int vec_turn) {
   extern __shared__ __attribute__((aligned(16))) unsigned char ht_lds[];
-  const int pitch = K + 8;                               // 16 bytes more than a row: the rows spread over the banks
-  bf16_t* xs = reinterpret_cast<bf16_t*>(ht_lds);        // [64][pitch]
-  constexpr int YP = HT_COLS + 8;
-  bf16_t* ys = xs + HT_ROWS * pitch;                     // [64][YP]
-  const int h = blockIdx.x, m0 = blockIdx.y * HT_ROWS;
-  const int here = min(HT_ROWS, rows - m0);
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  hg_bf16x8* ws = reinterpret_cast<hg_bf16x8*>(ht_lds);  // [tile of 16 outputs][KS][64]
+  constexpr int PAIRS = HT_LDS / (2 * KS * 1024) / 2 * 2;  // of tiles, in LDS at a time: whole groups
+  constexpr int AT_ONCE = 8;                             // operands of the matrix on their way, a wave
+  constexpr int GROUP = 2;                               // pairs of tiles multiplied with no branch between them
+  const int h = blockIdx.x, m0 = blockIdx.y * 16 * WAVES;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int col = lane & 15, grp = lane >> 4;
-  const int pieces = K / 8;
-  for (int i = threadIdx.x; i < HT_ROWS * pieces; i += 256) {
-    const int m = i / pieces, p = i % pieces;
-    hg_bf16x8 v;
-    if (m < here) v = *reinterpret_cast<const hg_bf16x8*>(x + (size_t)(m0 + m) * xs_t + (size_t)h * xs_h + p * 8);
-    else {
-#pragma unroll
-      for (int e = 0; e < 8; ++e) v[e] = (__bf16)0.f;
-    }
-    *reinterpret_cast<hg_bf16x8*>(xs + m * pitch + p * 8) = v;
-  }
-  // the rotated part of these rows, while the rows are on their way
-  for (int i = threadIdx.x; i < here * (rot / 2); i += 256) {
-    const int t = m0 + i / (rot / 2);
-    nhv_turn_pair(x + (size_t)t * xs_t + (size_t)h * xs_h + x_rot_off, y + (size_t)t * ys_t + (size_t)h * ys_h + y_rot_off,
-                  i % (rot / 2), rot, halves, positions[t], freqs, gain);
-  }
+  const int m = m0 + wave * 16 + col;
+  const bool live = m < rows;
   hg_bf16x8 zero;
 #pragma unroll
   for (int i = 0; i < 8; ++i) zero[i] = (__bf16)0.f;
-  __syncthreads();
-  for (int c0 = 0; c0 < N; c0 += HT_COLS) {
-    const int n0 = c0 + wave * 32;
-    if (n0 < N) {                                        // the whole wave; every wave meets the barriers below
-      const bf16_t* wrow[2];
-      bool n_ok[2];
+  hg_bf16x8 b[KS];
+  const bf16_t* xr = x + (size_t)(live ? m : rows - 1) * xs_t + (size_t)h * xs_h;
 #pragma unroll
-      for (int nt = 0; nt < 2; ++nt) {
-        const int n = n0 + nt * 16 + col;
-        n_ok[nt] = n < N;
-        wrow[nt] = w + ((size_t)h * N + (n_ok[nt] ? n : 0)) * K;
+  for (int ks = 0; ks < KS; ++ks) {
+    const int k = ks * 32 + grp * 8;
+    b[ks] = k < K ? *reinterpret_cast<const hg_bf16x8*>(xr + k) : zero;
+  }
+  const int line = 8 * (col >> 2) + (col & 3);
+  const bf16_t* wh = w + (size_t)h * N * K;
+  const bf16_t* gr = reinterpret_cast<const bf16_t*>(gate) + (size_t)(live ? m : rows - 1) * gs_t + (size_t)h * N;   // (mode 2)
+  bf16_t* yr = y + (size_t)m * ys_t + (size_t)h * ys_h;
+  for (int c0 = 0; c0 < N; c0 += PAIRS * 32) {
+    const int pairs = min(PAIRS, (N - c0 + 63) / 64 * 2), pieces = pairs * 2 * KS;
+    if (c0 > 0) __syncthreads();                         // the pieces before these have been read
+    for (int f0 = wave; f0 < pieces; f0 += AT_ONCE * WAVES) {
+      hg_bf16x8 a[AT_ONCE];
+#pragma unroll
+      for (int i = 0; i < AT_ONCE; ++i) {
+        const int f = f0 + i * WAVES, tile = f / KS;
+        const int n = c0 + (tile >> 1) * 32 + (tile & 1) * 4 + line, k = (f % KS) * 32 + grp * 8;
+        a[i] = f < pieces && n < N && k < K ? *reinterpret_cast<const hg_bf16x8*>(wh + (size_t)n * K + k) : zero;
       }
-      hg_floatx4 acc[4][2];
 #pragma unroll
-      for (int mt = 0; mt < 4; ++mt)
-#pragma unroll
-        for (int nt = 0; nt < 2; ++nt) acc[mt][nt] = hg_floatx4{0.f, 0.f, 0.f, 0.f};
-      // gates of four entries at once, asked for before the products
-      hg_bf16x4 g4[4][2];
+      for (int i = 0; i < AT_ONCE; ++i)
+        if (f0 + i * WAVES < pieces) ws[(f0 + i * WAVES) * 64 + lane] = a[i];
+    }
+    if (c0 == 0) {                                       // the rotated part of these rows, while the matrix is on its way
+      const int here = min(16 * WAVES, rows - m0), items = vec_turn ? rot / 16 : rot / 2;
+      for (int i = threadIdx.x; i < here * items; i += 64 * WAVES) {
+        const int t = m0 + i / items, p = i % items;
+        const bf16_t* src = x + (size_t)t * xs_t + (size_t)h * xs_h + x_rot_off;
+        bf16_t* dst = y + (size_t)t * ys_t + (size_t)h * ys_h + y_rot_off;
+        if (vec_turn) nhv_turn_eight_pairs(src, dst, p * 8, rot, halves, positions[t], freqs, gain);
+        else nhv_turn_pair(src, dst, p, rot, halves, positions[t], freqs, gain);
+      }
+    }
+    for (int p0 = 0; p0 < pairs; p0 += GROUP) {
+      hg_bf16x4 g4[GROUP][2];
       if (vec_gate) {
 #pragma unroll
-        for (int mt = 0; mt < 4; ++mt)
+        for (int i = 0; i < GROUP; ++i)
 #pragma unroll
-          for (int nt = 0; nt < 2; ++nt) {
-            const int n = n0 + nt * 16 + grp * 4, m = m0 + min(mt * 16 + col, here - 1);
-            g4[mt][nt] = *reinterpret_cast<const hg_bf16x4*>(reinterpret_cast<const bf16_t*>(gate) + (size_t)m * gs_t + (size_t)h * N +
-                                                             (n < N ? n : 0));
+          for (int t = 0; t < 2; ++t) {
+            const int n = c0 + (p0 + i) * 32 + grp * 8 + t * 4;
+            g4[i][t] = *reinterpret_cast<const hg_bf16x4*>(gr + (n < N ? n : 0));
           }
       }
-      for (int k0 = 0; k0 < K; k0 += 32 * U) {
-        hg_bf16x8 a[U][2];
+      if (p0 == 0) __syncthreads();                      // the pieces are there
 #pragma unroll
-        for (int u = 0; u < U; ++u) {
-          const int k = k0 + u * 32 + grp * 8;
+      for (int i = 0; i < GROUP; ++i) {
+
+        hg_floatx4 acc[2] = {hg_floatx4{0.f, 0.f, 0.f, 0.f}, hg_floatx4{0.f, 0.f, 0.f, 0.f}};
 #pragma unroll
-          for (int nt = 0; nt < 2; ++nt) a[u][nt] = (n_ok[nt] && k < K) ? *reinterpret_cast<const hg_bf16x8*>(wrow[nt] + k) : zero;
+        for (int ks = 0; ks < KS; ++ks)
+#pragma unroll
+          for (int t = 0; t < 2; ++t)
+            acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ws[(((p0 + i) * 2 + t) * KS + ks) * 64 + lane], b[ks], acc[t], 0, 0, 0);
+        const int n = c0 + (p0 + i) * 32 + grp * 8;
+        hg_bf16x8 eight;
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+          float v = acc[j / 4][j % 4];
+          if (vec_gate) v *= __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(-1.4426950408889634f * (float)g4[i][j / 4][j % 4]));
+          else if (gate != nullptr && live && n + j < N) v *= nhv_head_gate_of<bf16_t>(gate, gate_mode, gs_t, m, h, N, n + j);
+          eight[j] = (__bf16)v;
         }
+        if (vec_out) {                                   // N and the rows of y are pieces of 16 bytes
+          if (live && n < N) *reinterpret_cast<hg_bf16x8*>(yr + n) = eight;
+        } else {
 #pragma unroll
-        for (int u = 0; u < U; ++u) {
-          const int k = k0 + u * 32 + grp * 8;
-#pragma unroll
-          for (int mt = 0; mt < 4; ++mt) {
-            const hg_bf16x8 b = k < K ? *reinterpret_cast<const hg_bf16x8*>(xs + (mt * 16 + col) * pitch + k) : zero;
-#pragma unroll
-            for (int nt = 0; nt < 2; ++nt) acc[mt][nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[u][nt], b, acc[mt][nt], 0, 0, 0);
-          }
+          for (int j = 0; j < 8; ++j)
+            if (live && n + j < N) yr[n + j] = (bf16_t)eight[j];
         }
-      }
-#pragma unroll
-      for (int mt = 0; mt < 4; ++mt)
-#pragma unroll
-        for (int nt = 0; nt < 2; ++nt) {
-          hg_bf16x4 four;
-          float v[4];
-#pragma unroll
-          for (int j = 0; j < 4; ++j) v[j] = acc[mt][nt][j];
-          if (vec_gate) {
-#pragma unroll
-            for (int j = 0; j < 4; ++j)
-              v[j] *= __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(-1.4426950408889634f * (float)g4[mt][nt][j]));
-          } else if (gate != nullptr && mt * 16 + col < here) {
-            const int n = n0 + nt * 16 + grp * 4;
-#pragma unroll
-            for (int j = 0; j < 4; ++j)
-              if (n + j < N) v[j] *= nhv_head_gate_of<bf16_t>(gate, gate_mode, gs_t, m0 + mt * 16 + col, h, N, n + j);
-          }
-#pragma unroll
-          for (int j = 0; j < 4; ++j) four[j] = (__bf16)v[j];
-          *reinterpret_cast<hg_bf16x4*>(ys + (mt * 16 + col) * YP + wave * 32 + nt * 16 + grp * 4) = four;
-        }
-    }
-    __syncthreads();
-    const int width = min(HT_COLS, N - c0);
-    if (vec_out) {                                       // N and the rows of y are pieces of 16 bytes
-      for (int i = threadIdx.x; i < here * (width / 8); i += 256) {
-        const int m = i / (width / 8), p = i % (width / 8);
-        *reinterpret_cast<hg_bf16x8*>(y + (size_t)(m0 + m) * ys_t + (size_t)h * ys_h + c0 + p * 8) =
-            *reinterpret_cast<const hg_bf16x8*>(ys + m * YP + p * 8);
-      }
-    } else {
-      for (int i = threadIdx.x; i < here * width; i += 256) {
-        const int m = i / width, p = i % width;
-        y[(size_t)(m0 + m) * ys_t + (size_t)h * ys_h + c0 + p] = ys[m * YP + p];
       }
     }
-    __syncthreads();
   }
 }
 
@@ -609,19 +610,34 @@ extern "C" int nhv_head_gemm_bf16(const void* x, long long xs_t, long long xs_h,
                        x_rot_off, y_rot_off, halves, (const double*)freqs, gain, (const int*)positions);                  \
   } while (0)
   if (rows > 64 && K <= HT_MAX_K) {
-    const size_t lds = (size_t)HT_ROWS * (K + 8 + HT_COLS + 8) * sizeof(bf16_t);
-    auto kernel = head_gemm_tile_kernel<4>;
-    // more than 64 KB of dynamic LDS has to be allowed once per kernel (and per process)
-    static const hipError_t allowed = hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                                          (int)(HT_ROWS * (HT_MAX_K + 8 + HT_COLS + 8) * sizeof(bf16_t)));
-    NHV_REQUIRE(allowed == hipSuccess, "head_gemm_bf16: %s", hipGetErrorString(allowed));
-    const dim3 grid(H, (rows + HT_ROWS - 1) / HT_ROWS);
-    NHV_REQUIRE(grid.y <= 65535, "head_gemm_bf16: %d rows are too many", rows);
     const int vec_out = N % 8 == 0 && ys_t % 8 == 0 && ys_h % 8 == 0 && (uintptr_t)y % 16 == 0;
     const int vec_gate = gate != nullptr && gate_mode == 2 && N % 4 == 0 && gs_t % 4 == 0 && (uintptr_t)gate % 8 == 0;
-    hipLaunchKernelGGL(kernel, grid, dim3(256), lds, s, (const bf16_t*)x, xs_t, xs_h, (const bf16_t*)w, (bf16_t*)y, ys_t, ys_h, gate,
-                       gate_mode, gs_t, rows, N, K, rot, x_rot_off, y_rot_off, halves, (const double*)freqs, gain,
-                       (const int*)positions, vec_out, vec_gate);
+    const int vec_turn = rot % 16 == 0 && x_rot_off % 8 == 0 && y_rot_off % 8 == 0 && ys_t % 8 == 0 && ys_h % 8 == 0 && (uintptr_t)y % 16 == 0;
+#define ROWS_LAUNCH(KS, WAVES)                                                                                            \
+  do {                                                                                                                    \
+    const int pairs = (N + 63) / 64 * 2, most = HT_LDS / (2 * KS * 1024) / 2 * 2;                                                     \
+    const dim3 grid(H, (rows + 16 * WAVES - 1) / (16 * WAVES));                                                           \
+    NHV_REQUIRE(grid.y <= 65535, "head_gemm_bf16: %d rows are too many", rows);                                           \
+    hipLaunchKernelGGL((head_gemm_rows_kernel<KS, WAVES>), grid, dim3(64 * WAVES),                                        \
+                       (size_t)(pairs < most ? pairs : most) * 2 * KS * 1024, s, (const bf16_t*)x, xs_t, xs_h,            \
+                       (const bf16_t*)w, (bf16_t*)y, ys_t, ys_h, gate, gate_mode, gs_t, rows, N, K, rot, x_rot_off,       \
+                       y_rot_off, halves, (const double*)freqs, gain, (const int*)positions, vec_out, vec_gate,           \
+                       vec_turn);                                                                                         \
+  } while (0)
+#define ROWS_LAUNCH_OF(KS)                                                                                                \
+  do {                                                                                                                    \
+    if (few) ROWS_LAUNCH(KS, 4);                                                                                          \
+    else ROWS_LAUNCH(KS, 16);                                                                                              \
+  } while (0)
+    // 256 rows a block share a matrix; where these are fewer than half the compute units, 64 (1,000 rows of 16 heads,
+    // 192 to 128 entries: 8.1 us with 64, 8.2 with 128; 2,500 rows, 128 to 192: 13.6 us with 256, 14.9 with 128)
+    const bool few = (long long)H * ((rows + 255) / 256) < 128;
+    if (K <= 128) ROWS_LAUNCH_OF(4);
+    else if (K <= 192) ROWS_LAUNCH_OF(6);
+    else if (K <= 256) ROWS_LAUNCH_OF(8);
+    else ROWS_LAUNCH_OF(16);
+#undef ROWS_LAUNCH_OF
+#undef ROWS_LAUNCH
   } else if (rows <= 16) {
     LAUNCH(1, 1, 1, 4);
   } else if (rows <= 64) {

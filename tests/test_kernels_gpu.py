@@ -2044,3 +2044,45 @@ def test_single_tokens_beyond_what_the_splits_cover_are_stored_and_read(ops, mon
     got = ops.rotated_attention(*arguments, k2, v2, Hq, Hkv, D, batch, bt, D ** -0.5, window)
     assert torch.equal(k1.view(torch.int16), k2.view(torch.int16)) and torch.equal(v1.view(torch.int16), v2.view(torch.int16))
     torch.testing.assert_close(got, want, rtol=1.6e-2, atol=1.6e-2)
+
+
+@pytest.mark.parametrize("H, N, K, rot, rows", [(3, 8, 8, 16, 65), (2, 130, 40, 6, 257), (16, 192, 128, 64, 2100), (16, 128, 192, 0, 2050),
+                                                (5, 330, 168, 32, 129), (2, 72, 512, 16, 191), (40, 33, 264, 0, 1030), (1, 520, 256, 64, 16500)])
+def test_a_matrix_per_head_of_many_rows(ops, H, N, K, rot, rows):
+    """Products with a matrix per head of more than 64 rows at the edges of a block's rows, of the pieces of the matrix that
+    are in LDS at a time and of the outputs that a lane writes at once, with and without gates and a turned part."""
+    g = torch.Generator(device="cuda").manual_seed(rows)
+    rand = lambda *shape: torch.randn(*shape, generator=g, device="cuda").to(torch.bfloat16)
+    pad = -(K + rot) % 8
+    x, w = rand(rows, H, K + rot + pad), rand(H, N, K)
+    pos = torch.randint(0, 5000, (rows,), generator=g, device="cuda", dtype=torch.int32)
+    want = torch.stack([x[:, h, :K].double() @ w[h].double().T for h in range(H)], dim=1)
+    # one rounding to bfloat16, and the sums' own in float
+    bound = want.abs() * 2.0 ** -8 + 2.0 ** -22 * K ** 0.5 * float(want.std())
+    for off in (0, 1):
+        for halves in ((True, False) if rot else (None,)):
+            freqs = 10000.0 ** (-2.0 * torch.arange(rot // 2, dtype=torch.float64, device="cuda") / max(rot, 1))
+            width = -(-(N + rot + off) // 8) * 8 + 8
+            out = torch.full((rows, H, width), 7.0, dtype=torch.bfloat16, device="cuda")
+            at = -(-(N + off) // 8) * 8 if off == 0 and N + rot <= width - 8 and N % 8 == 0 else N + off
+            turn = (rot, K, at, freqs, 1.0, pos, halves) if rot else None
+            ops.head_gemm(x, w.view(H * N, K), False, N, K, out=out, out_off=off, turn=turn)
+            assert bool(((out[:, :, off:off + N].double() - want).abs() <= bound).all()), (off, halves)
+            mask = torch.ones(width, dtype=torch.bool)
+            mask[off:off + N] = False
+            if rot:
+                mask[at:at + rot] = False
+                angle = (pos.double()[:, None] * freqs)[:, None]
+                t = x[:, :, K:K + rot].double()
+                u, v = (t[..., :rot // 2], t[..., rot // 2:]) if halves else (t[..., 0::2], t[..., 1::2])
+                a, b = u * angle.cos() - v * angle.sin(), v * angle.cos() + u * angle.sin()
+                turned = torch.cat((a, b), dim=-1) if halves else torch.stack((a, b), dim=-1).flatten(-2)
+                # one rounding to bfloat16; the hardware's sine and cosine to 2^-16
+                limit = turned.abs() * 2.0 ** -8 + 2.0 ** -16 * float(t.abs().max())
+                assert bool(((out[:, :, at:at + rot].double() - turned).abs() <= limit).all()), (off, halves)
+            assert bool((out[:, :, mask.to(out.device)] == 7.0).all())
+    for gate, per in ((rand(rows, H * N + 4), "per entry"), (torch.randn(rows, H + 2, generator=g, device="cuda"), "per head")):
+        for col in (0, 1):
+            got = ops.head_gemm(x, w.view(H * N, K), False, N, K, gate=(gate, col, per))
+            s = torch.sigmoid(gate.double())[:, col:col + (H * N if per == "per entry" else H)].reshape(rows, H, -1)
+            assert bool(((got.double() - want * s).abs() <= (want * s).abs() * 2.0 ** -8 + 2.0 ** -20 * K ** 0.5 * float(want.std())).all()), (per, col)
