@@ -42,6 +42,7 @@
 // and joins the row's sum at the end) and a gate per (token, head) whose sigmoid multiplies the head's result (with the
 // division by the sum).
 #include "nhv_common.h"
+#include "nhv_lines.h"
 #include <math.h>
 #include <type_traits>
 
@@ -66,6 +67,7 @@ constexpr bool CH_POW2 = (CH & (CH - 1)) == 0;
 constexpr int KSWZ = CH_POW2 ? (CH < 16 ? CH : 16) - 1 : 0;
 // and at c ^ ((k & VSWZ) << 1) in the V tile, whose transposed reads take 32 bytes of 8 keys at once
 constexpr int VSWZ = CH_POW2 && CH >= 4 ? (CH / 2 < 8 ? CH / 2 : 8) - 1 : 0;
+constexpr bool ONE_TILE = D <= 128;         // requests whose rows are one tile get a path of their own (its tiles fit into that LDS)
 constexpr int MAX_RT = D <= 128 ? 2 : 1;    // row tiles per wave (template argument RT): all of them use every key and value
                                             // that the wave reads from LDS; two need the registers of head sizes up to 128
 
@@ -89,6 +91,157 @@ template <typename P>
 __device__ __forceinline__ int slot_of(P bt, int key, int page_size, int page_shift) {
   if (page_shift >= 0) return (bt[key >> page_shift] << page_shift) + (key & (page_size - 1));
   return bt[key / page_size] * page_size + key % page_size;
+}
+
+// What a wave keeps of its rows: row tile r's row `col` is this lane's row in both products.
+template <int RT>
+struct Rows {
+  bf16x8 q[RT][DSTEPS];
+  int pos[RT], lo[RT];
+  float slope[RT];                                         // (as the unscaled scores see it)
+  float m[RT], l[RT];                                      // reference point (base 2); this lane's share of the row's sum
+  floatx4 o[RT][DTILES];                                   // o[r][dt][j]: entry dt * 16 + 4 grp + j
+};
+
+// KT sub-tiles of 16 keys from kb on against a wave's rows. key_operand(kt, s): the first product's operand, sub-tile kt, step s over the
+// head; v_s: the values as rows of D entries, pieces where VSWZ puts them.
+// MASKED: whether some key of the tile is hidden from some row of the wave. Tiles wholly inside every row's range, which are nearly all, run
+// code without the comparisons: as a run-time flag the test cost three to four instructions for every score in every tile.
+template <int RT, int KT, bool MASKED, bool CAPPED, bool BIASED, typename KeyOperand>
+__device__ __forceinline__ void attend(Rows<RT>& w, int kb, KeyOperand key_operand, const bf16_t* v_s, int col, int grp, float scale_log2e,
+                                       float cap_ratio, float tanh_k) {
+  // ---- scores of the tile's keys for this wave's rows: every K operand serves all row tiles
+  floatx4 s4[RT][KT];
+  float first_bias[RT];                                  // at this lane's first key of the tile; the others follow by steps
+#pragma unroll
+  for (int r = 0; r < RT; ++r) first_bias[r] = BIASED ? w.slope[r] * (float)(kb + grp * 4 - w.pos[r]) : 0.f;
+#pragma unroll
+  for (int kt = 0; kt < KT; ++kt) {
+#pragma unroll
+    for (int r = 0; r < RT; ++r) {
+      if (BIASED) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) s4[r][kt][j] = __builtin_fmaf(w.slope[r], (float)(kt * 16 + j), first_bias[r]);
+      } else {
+        s4[r][kt] = floatx4{0.f, 0.f, 0.f, 0.f};
+      }
+    }
+#pragma unroll
+    for (int s = 0; s < DSTEPS; ++s) {
+      const bf16x8 ka = key_operand(kt, s);
+#pragma unroll
+      for (int r = 0; r < RT; ++r) s4[r][kt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ka, w.q[r][s], s4[r][kt], 0, 0, 0);
+    }
+  }
+  if (CAPPED) {
+#pragma unroll
+    for (int r = 0; r < RT; ++r)
+#pragma unroll
+      for (int kt = 0; kt < KT; ++kt)
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+          s4[r][kt][j] = __builtin_fmaf(-2.0f * cap_ratio,
+                                        __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(s4[r][kt][j] * tanh_k)), cap_ratio);
+  }
+  bf16x8 pa[RT][KT / 2];                                 // P of keys (32 a + 4 grp + j) and (32 a + 16 + 4 grp + j)
+  float alpha[RT];
+  bool grow[RT];
+#pragma unroll
+  for (int r = 0; r < RT; ++r) {
+    // The reference point of a row's exponentials stays where it is as long as they stay far below float's range:
+    // they are taken against it at once, without the tile's maximum, and only a sum that has grown past 2^40 (or is
+    // no number: a row that has seen no key yet has no reference) sends the wave to the maximum and a new reference.
+    if (MASKED) {
+#pragma unroll
+      for (int kt = 0; kt < KT; ++kt)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          const int key = kb + kt * 16 + grp * 4 + j;
+          if (key > w.pos[r] || key < w.lo[r]) s4[r][kt][j] = -INFINITY;
+        }
+    }
+    float psum = 0.f;
+#pragma unroll
+    for (int kt = 0; kt < KT; ++kt)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const float p = __builtin_amdgcn_exp2f(__builtin_fmaf(s4[r][kt][j], scale_log2e, -w.m[r]));
+        psum += p;
+        pa[r][kt / 2][(kt % 2) * 4 + j] = (__bf16)p;
+      }
+    grow[r] = __any(!(psum < 1.0995116e12f));
+    alpha[r] = 1.0f;
+    if (grow[r]) {
+      asm volatile("" ::: "memory");
+      float m_tile = -INFINITY;
+#pragma unroll
+      for (int kt = 0; kt < KT; ++kt)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) m_tile = fmaxf(m_tile, s4[r][kt][j]);
+      m_tile *= scale_log2e;
+      m_tile = fmaxf(m_tile, __shfl_xor(m_tile, 16, 64));
+      m_tile = fmaxf(m_tile, __shfl_xor(m_tile, 32, 64));
+      const float m_new = fmaxf(w.m[r], m_tile);
+      const float m_safe = m_new == -INFINITY ? 0.f : m_new;  // a row that has still seen no key
+      alpha[r] = w.m[r] == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(w.m[r] - m_safe);
+      psum = 0.f;
+#pragma unroll
+      for (int kt = 0; kt < KT; ++kt)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          const float p = __builtin_amdgcn_exp2f(__builtin_fmaf(s4[r][kt][j], scale_log2e, -m_safe));
+          psum += p;
+          pa[r][kt / 2][(kt % 2) * 4 + j] = (__bf16)p;
+        }
+      w.l[r] = w.l[r] * alpha[r] + psum;
+      w.m[r] = m_new;
+    } else {
+      w.l[r] += psum;
+    }
+  }
+  // The outputs are rescaled only when a reference has moved: a branch of the whole wave, taken rarely. (Written
+  // as a condition inside the loop over the output tiles, the compiler made a multiply and a select of it for
+  // every output entry in every tile, 128 instructions a tile; the empty statement keeps the branch a branch.)
+#pragma unroll
+  for (int r = 0; r < RT; ++r)
+    if (grow[r]) {
+      asm volatile("" ::: "memory");
+#pragma unroll
+      for (int dt = 0; dt < DTILES; ++dt)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) w.o[r][dt][j] *= alpha[r];
+    }
+  // this lane points at key 4 grp + col / 4 of a 16-key sub-tile, entries 4 (col % 4).. of the 16-entry block dt
+  const int tr_key = grp * 4 + (col >> 2);
+  const int tr_piece = (col & 3) >> 1, tr_half = (col & 1) * 4;
+#pragma unroll
+  for (int dt = 0; dt < DTILES; ++dt) {
+#pragma unroll
+    for (int a = 0; a < KT / 2; ++a) {
+      // this lane's eight summation slots: keys 32 a + 4 grp + (0..3) and 32 a + 16 + 4 grp + (0..3), entry dt * 16 + col
+      const int k_lo = a * 32 + tr_key, k_hi = k_lo + 16;
+      const bf16_t* p_lo = v_s + k_lo * D + ((dt * 2 + tr_piece) ^ ((k_lo & VSWZ) << 1)) * 8 + tr_half;
+      const bf16_t* p_hi = v_s + k_hi * D + ((dt * 2 + tr_piece) ^ ((k_hi & VSWZ) << 1)) * 8 + tr_half;
+      const short4_t lo4 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) short4_t*)p_lo);
+      const short4_t hi4 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) short4_t*)p_hi);
+      typedef short short8_t __attribute__((ext_vector_type(8)));
+      const short8_t both = __builtin_shufflevector(lo4, hi4, 0, 1, 2, 3, 4, 5, 6, 7);
+      const bf16x8 va = __builtin_bit_cast(bf16x8, both);
+#pragma unroll
+      for (int r = 0; r < RT; ++r) w.o[r][dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(va, pa[r][a], w.o[r][dt], 0, 0, 0);
+    }
+  }
+  // V^T operands are read eight ahead of the one that is multiplied. (Left to itself the compiler reads two, waits for them, and multiplies: us
+  // so and now, 2,048 tokens after 14,336 502, 485; alone 59.1, 54.9; 512 after 4,000 77.9, 71.1; 901, 400 and 700 tokens 34.6, 33.1; 1 after 300,
+  // 17 after 40 and 333 after 1,000 27.2, 25.8. Two ahead 499, 58.0, 76.8; four 487, 55.9, 71.7. The same for the first product's operands: nothing.)
+  constexpr int OPERANDS = DTILES * KT / 2, AHEAD = OPERANDS < 8 ? OPERANDS : 8, DS_READ = 0x100, MATRIX = 0x8;
+  __builtin_amdgcn_sched_group_barrier(DS_READ, 2 * AHEAD, 0);
+#pragma unroll
+  for (int i = 0; i < OPERANDS - AHEAD; ++i) {
+    __builtin_amdgcn_sched_group_barrier(MATRIX, RT, 0);
+    __builtin_amdgcn_sched_group_barrier(DS_READ, 2, 0);
+  }
+  __builtin_amdgcn_sched_group_barrier(MATRIX, AHEAD * RT, 0);
 }
 
 // BT_IN_LDS: the request's block table (up to the block's last key) is copied into LDS first, so that the
@@ -143,6 +296,135 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void p
 
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int col = lane & 15, grp = lane >> 4;
+  const int* bt_g = block_tables + (size_t)req * max_blocks;
+  // the block table up to the block's last key goes into LDS; where the key look-ups go then: LDS copy or memory
+  auto keep_table = [&](int last_key) {
+    const int n_entries = min(BT_LDS, last_key / page_size + 1);
+    for (int i = tid; i < n_entries; i += 256) bt_s[i] = bt_g[i];
+    __syncthreads();
+  };
+  auto slot = [&](int key) {
+    return BT_IN_LDS ? slot_of((const int*)bt_s, key, page_size, page_shift) : slot_of(bt_g, key, page_size, page_shift);
+  };
+
+  // A request whose tokens and heads fill no more than one tile (one that decodes beside prompts): its rows are one tile of all of them,
+  // and the four waves share its keys, 32 at a time in turn, each with its next 32 on their way: keys as operands in registers, values in a
+  // part of LDS of its own, no barrier. The waves' sums meet at the end. Otherwise every head's few rows are a tile, all keys pass every
+  // wave one tile after the other, 1 us each, and the block is the last to end. 13 tokens after 60 to 1,700 keys beside
+  // prompts of 901, 90 and 500: 47.7 to 37.0 us (the prompts last: 56.2 to 40.0); one token after 1,700 alone 28.9 to 20.5; four after 40
+  // to 700 beside 75 new ones 14.6 to 12.4.
+  if constexpr (ONE_TILE) {
+    if (G * q_len <= 16) {                                 // the whole block
+      if (bx > 0) return;
+      // (values of its own: what both paths work out from the lane would be kept in registers that the other path needs)
+      int my_lane = threadIdx.x & 63;
+      asm volatile("" : "+v"(my_lane));
+      const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+      const int lane = my_lane, col = lane & 15, grp = lane >> 4;
+      Rows<1> rows;
+      const bool row_ok = col < G * q_len;
+      const int row_tok = row_ok ? col % q_len : 0, head = kvh * G + (row_ok ? col / q_len : 0);
+      const int key_hi = ctx - 1, key_lo = nhv_first_key(start_pos, window), max_lo = nhv_first_key(key_hi, window);
+      rows.pos[0] = start_pos + row_tok;
+      rows.lo[0] = nhv_first_key(rows.pos[0], window);
+#pragma unroll
+      for (int s = 0; s < DSTEPS; ++s) {
+        const int d = s * 32 + grp * 8;
+        rows.q[0][s] = row_ok && d < D ? *reinterpret_cast<const bf16x8*>(q + ((size_t)(q_begin + row_tok) * Hq + head) * D + d) : zero8();
+      }
+      rows.slope[0] = BIASED ? slopes[head] * slope_ratio : 0.f;
+      const float row_sink = MORE ? (sinks ? sinks[head] * LOG2E : sink_l2) : -INFINITY;
+      rows.m[0] = row_sink;
+      rows.l[0] = 0.f;
+#pragma unroll
+      for (int dt = 0; dt < DTILES; ++dt) rows.o[0][dt] = floatx4{0.f, 0.f, 0.f, 0.f};
+      if (BT_IN_LDS) keep_table(key_hi);
+
+      constexpr int KEYS = 32, STEP = 4 * KEYS;            // of a wave's tile; of the four waves' tiles
+      static_assert(2 * KEYS * D <= TILE && DTILES * 1024 + 128 <= TILE * 2, "two tiles of values, and later the sums, lie in a wave's part");
+      bf16_t* mine = wave == 0 ? k_s0 : wave == 1 ? k_s1 : wave == 2 ? v_s0 : v_s1;
+      const bool in_page = page_shift >= 0 && page_size >= KEYS;
+      auto issue_one = [&](int kb, bf16x8 (&k)[2][DSTEPS], bf16_t* v_s) {
+        // (whole tiles inside a page need one look-up)
+        const bool whole = in_page && kb >= key_lo && kb + KEYS - 1 <= key_hi;
+        const size_t first = whole ? (size_t)__builtin_amdgcn_readfirstlane(slot(kb)) : 0;
+        auto row_at = [&](int kl) {
+          const size_t at = whole ? first + kl : (size_t)slot(min(max(kb + kl, key_lo), key_hi));
+          return (at * Hkv + kvh) * D;
+        };
+#pragma unroll
+        for (int i = 0; i < CH / 2; ++i) {
+          const int u = i * 64 + lane, kl = u / CH, piece = u % CH;
+          nhv_load_to_lds<false>(nhv_lds_address(v_s) + i * 1024, v_cache + row_at(kl) + (piece ^ ((kl & VSWZ) << 1)) * 8);
+        }
+#pragma unroll
+        for (int kt = 0; kt < 2; ++kt) {
+          const bf16_t* row = k_cache + row_at(kt * 16 + col);
+#pragma unroll
+          for (int s = 0; s < DSTEPS; ++s) k[kt][s] = s * 4 + grp < CH ? *reinterpret_cast<const bf16x8*>(row + (s * 4 + grp) * 8) : zero8();
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      };
+      auto turn = [&](int kb, const bf16x8 (&k)[2][DSTEPS], const bf16_t* v_s, bf16x8 (&k_next)[2][DSTEPS], bf16_t* v_next) {
+        __builtin_amdgcn_sched_barrier(0);
+        asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");        // this tile has arrived, the one before it has been read
+        __builtin_amdgcn_s_waitcnt(0x0070);                                // (the same, for the compiler's account)
+        __builtin_amdgcn_sched_barrier(0);
+        if (kb + STEP <= key_hi) issue_one(kb + STEP, k_next, v_next);
+        auto key_operand = [&](int kt, int s) { return k[kt][s]; };
+        if (kb + KEYS - 1 > start_pos || kb < max_lo)
+          attend<1, 2, true, CAPPED, BIASED>(rows, kb, key_operand, v_s, col, grp, scale_log2e, cap_ratio, tanh_k);
+        else
+          attend<1, 2, false, CAPPED, BIASED>(rows, kb, key_operand, v_s, col, grp, scale_log2e, cap_ratio, tanh_k);
+      };
+      bf16x8 k0[2][DSTEPS], k1[2][DSTEPS];
+      int kb = key_lo / KEYS * KEYS + wave * KEYS;
+      if (kb <= key_hi) issue_one(kb, k0, mine);
+      for (; kb <= key_hi; kb += 2 * STEP) {
+        turn(kb, k0, mine, k1, mine + KEYS * D);
+        if (kb + STEP > key_hi) break;
+        turn(kb + STEP, k1, mine + KEYS * D, k0, mine);
+      }
+
+      // the four waves' sums meet: outputs, then reference points and sums of the 16 rows
+      float l = rows.l[0];
+      l += __shfl_xor(l, 16, 64);
+      l += __shfl_xor(l, 32, 64);
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");                   // (the last tile has been read)
+      floatx4* sums = reinterpret_cast<floatx4*>(mine);
+#pragma unroll
+      for (int dt = 0; dt < DTILES; ++dt) sums[dt * 64 + lane] = rows.o[0][dt];
+      if (grp == 0) reinterpret_cast<float2*>(sums + DTILES * 64)[col] = float2{rows.m[0], l};
+      __syncthreads();
+      const floatx4* all[4] = {(const floatx4*)k_s0, (const floatx4*)k_s1, (const floatx4*)v_s0, (const floatx4*)v_s1};
+      float m = -INFINITY, factor[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) m = fmaxf(m, reinterpret_cast<const float2*>(all[i] + DTILES * 64)[col].x);
+      l = MORE ? __builtin_amdgcn_exp2f(row_sink - m) : 0.f;               // (a row has seen its own key: m is a number)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const float2 ml = reinterpret_cast<const float2*>(all[i] + DTILES * 64)[col];
+        factor[i] = __builtin_amdgcn_exp2f(ml.x - m);
+        l += ml.y * factor[i];
+      }
+      float inv = 1.0f / l;
+      if (MORE && gate && row_ok) inv /= 1.0f + expf(-(float)gate[(size_t)(q_begin + row_tok) * gate_ld + head]);
+      for (int dt = wave; dt < DTILES; dt += 4) {
+        floatx4 sum{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const floatx4 part = all[i][dt * 64 + lane];
+#pragma unroll
+          for (int j = 0; j < 4; ++j) sum[j] = __builtin_fmaf(part[j], factor[i], sum[j]);
+        }
+        bf16x4 four;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) four[j] = (__bf16)(sum[j] * inv);
+        if (row_ok) *reinterpret_cast<bf16x4*>(out + ((size_t)(q_begin + row_tok) * Hq + head) * D + dt * 16 + grp * 4) = four;
+      }
+      return;
+    }
+  }
 
   // the block's key range: from the smallest lower bound to the largest position of its rows
   const int last_tile = min(first_tile + TPB - 1, n_row_tiles - 1);
@@ -153,10 +435,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void p
 
   // this wave's row tiles; this lane's row (in both products) is token tok0 + col of the tile's head
   const bool live = first_tile + wave * RT < n_row_tiles;
-  int row_pos[RT], row_lo[RT], row_tok[RT], head[RT];
+  Rows<RT> rows;
+  int row_tok[RT], head[RT];
   bool row_ok[RT];
   int wave_lo_pos = 0x7fffffff, wave_hi = -1, wave_max_lo = 0;
-  bf16x8 qb[RT][DSTEPS];
 #pragma unroll
   for (int r = 0; r < RT; ++r) {
     const int my_tile = first_tile + wave * RT + r;
@@ -165,8 +447,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void p
     const int tok0 = tile_live ? (my_tile / G) * 16 : 0;
     row_tok[r] = tok0 + col;
     row_ok[r] = tile_live && row_tok[r] < q_len;
-    row_pos[r] = tile_live ? start_pos + min(row_tok[r], q_len - 1) : -1;    // a tile beyond the portion sees no key
-    row_lo[r] = nhv_first_key(row_pos[r], window);
+    rows.pos[r] = tile_live ? start_pos + min(row_tok[r], q_len - 1) : -1;    // a tile beyond the portion sees no key
+    rows.lo[r] = nhv_first_key(rows.pos[r], window);
     if (tile_live) {
       const int hi = start_pos + min(tok0 + 15, q_len - 1);                 // beyond it the tile has nothing to do
       wave_lo_pos = min(wave_lo_pos, start_pos + tok0);                       // the tile's first row sees the fewest keys
@@ -176,37 +458,26 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void p
 #pragma unroll
     for (int s = 0; s < DSTEPS; ++s) {
       const int d = s * 32 + grp * 8;
-      qb[r][s] = (row_ok[r] && d < D)
+      rows.q[r][s] = (row_ok[r] && d < D)
                      ? *reinterpret_cast<const bf16x8*>(q + ((size_t)(q_begin + row_tok[r]) * Hq + head[r]) * D + d)
                      : zero8();
     }
   }
-  float slope[RT], row_sink[RT];                           // (the slope as the unscaled scores see it)
+  float row_sink[RT];
 #pragma unroll
   for (int r = 0; r < RT; ++r) {
-    slope[r] = BIASED ? slopes[head[r]] * slope_ratio : 0.f;
+    rows.slope[r] = BIASED ? slopes[head[r]] * slope_ratio : 0.f;
     row_sink[r] = MORE ? (sinks ? sinks[head[r]] * LOG2E : sink_l2) : -INFINITY;
   }
-  float m_run[RT], l_part[RT];                             // of row `col` (base 2); l_part is this lane's share of the row's sum
-  floatx4 o[RT][DTILES];                                   // o[r][dt][j]: entry dt * 16 + 4 grp + j of row `col`
 #pragma unroll
   for (int r = 0; r < RT; ++r) {
-    m_run[r] = row_sink[r];                                // (no sink: -inf, the first tile gives the reference)
-    l_part[r] = 0.f;
+    rows.m[r] = row_sink[r];                                // (no sink: -inf, the first tile gives the reference)
+    rows.l[r] = 0.f;
 #pragma unroll
-    for (int dt = 0; dt < DTILES; ++dt) o[r][dt] = floatx4{0.f, 0.f, 0.f, 0.f};
+    for (int dt = 0; dt < DTILES; ++dt) rows.o[r][dt] = floatx4{0.f, 0.f, 0.f, 0.f};
   }
 
-  const int* bt_g = block_tables + (size_t)req * max_blocks;
-  if (BT_IN_LDS) {
-    const int n_entries = min(BT_LDS, key_hi / page_size + 1);
-    for (int i = tid; i < n_entries; i += 256) bt_s[i] = bt_g[i];
-    __syncthreads();
-  }
-  // where the key look-ups go: LDS copy or memory
-  auto slot = [&](int key) {
-    return BT_IN_LDS ? slot_of((const int*)bt_s, key, page_size, page_shift) : slot_of(bt_g, key, page_size, page_shift);
-  };
+  if (BT_IN_LDS) keep_table(key_hi);
 
   // memory -> LDS without registers: wave w's load number i brings pieces (4 i + w) * 64 + lane of the tile.
   // With pages that are a power of two and hold whole tiles, a tile inside the block's key range lies in one page
@@ -250,145 +521,12 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void p
     }
   };
 
-  // MASKED (a type, so that each call site names a compile-time choice): whether some key of the tile is hidden from
-  // some row of the wave. Tiles wholly inside every row's range, which are nearly all, run code without the
-  // comparisons: as a run-time flag the test cost three to four instructions for every score in every tile.
   auto compute = [&](auto masked, int kb, const bf16_t* k_s, const bf16_t* v_s) {
-    constexpr bool MASKED = decltype(masked)::value;
-    // ---- scores of the tile's keys for this wave's rows: every K operand serves all row tiles
-    floatx4 s4[RT][KT];
-    float first_bias[RT];                                  // at this lane's first key of the tile; the others follow by steps
-#pragma unroll
-    for (int r = 0; r < RT; ++r) first_bias[r] = BIASED ? slope[r] * (float)(kb + grp * 4 - row_pos[r]) : 0.f;
-#pragma unroll
-    for (int kt = 0; kt < KT; ++kt) {
-#pragma unroll
-      for (int r = 0; r < RT; ++r) {
-        if (BIASED) {
-#pragma unroll
-          for (int j = 0; j < 4; ++j) s4[r][kt][j] = __builtin_fmaf(slope[r], (float)(kt * 16 + j), first_bias[r]);
-        } else {
-          s4[r][kt] = floatx4{0.f, 0.f, 0.f, 0.f};
-        }
-      }
-#pragma unroll
-      for (int s = 0; s < DSTEPS; ++s) {
-        const int piece = s * 4 + grp;
-        const bf16x8 ka = piece < CH ? *reinterpret_cast<const bf16x8*>(k_s + (kt * 16 + col) * D + (piece ^ (col & KSWZ)) * 8)
-                                     : zero8();
-#pragma unroll
-        for (int r = 0; r < RT; ++r) s4[r][kt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ka, qb[r][s], s4[r][kt], 0, 0, 0);
-      }
-    }
-    if (CAPPED) {
-#pragma unroll
-      for (int r = 0; r < RT; ++r)
-#pragma unroll
-        for (int kt = 0; kt < KT; ++kt)
-#pragma unroll
-          for (int j = 0; j < 4; ++j)
-            s4[r][kt][j] = __builtin_fmaf(-2.0f * cap_ratio,
-                                          __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(s4[r][kt][j] * tanh_k)), cap_ratio);
-    }
-    bf16x8 pa[RT][KT / 2];                                 // P of keys (32 a + 4 grp + j) and (32 a + 16 + 4 grp + j)
-    float alpha[RT];
-    bool grow[RT];
-#pragma unroll
-    for (int r = 0; r < RT; ++r) {
-      // The reference point of a row's exponentials stays where it is as long as they stay far below float's range:
-      // they are taken against it at once, without the tile's maximum, and only a sum that has grown past 2^40 (or is
-      // no number: a row that has seen no key yet has no reference) sends the wave to the maximum and a new reference.
-      if (MASKED) {
-#pragma unroll
-        for (int kt = 0; kt < KT; ++kt)
-#pragma unroll
-          for (int j = 0; j < 4; ++j) {
-            const int key = kb + kt * 16 + grp * 4 + j;
-            if (key > row_pos[r] || key < row_lo[r]) s4[r][kt][j] = -INFINITY;
-          }
-      }
-      float psum = 0.f;
-#pragma unroll
-      for (int kt = 0; kt < KT; ++kt)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          const float p = __builtin_amdgcn_exp2f(__builtin_fmaf(s4[r][kt][j], scale_log2e, -m_run[r]));
-          psum += p;
-          pa[r][kt / 2][(kt % 2) * 4 + j] = (__bf16)p;
-        }
-      grow[r] = __any(!(psum < 1.0995116e12f));
-      alpha[r] = 1.0f;
-      if (grow[r]) {
-        asm volatile("" ::: "memory");
-        float m_tile = -INFINITY;
-#pragma unroll
-        for (int kt = 0; kt < KT; ++kt)
-#pragma unroll
-          for (int j = 0; j < 4; ++j) m_tile = fmaxf(m_tile, s4[r][kt][j]);
-        m_tile *= scale_log2e;
-        m_tile = fmaxf(m_tile, __shfl_xor(m_tile, 16, 64));
-        m_tile = fmaxf(m_tile, __shfl_xor(m_tile, 32, 64));
-        const float m_new = fmaxf(m_run[r], m_tile);
-        const float m_safe = m_new == -INFINITY ? 0.f : m_new;  // a row that has still seen no key
-        alpha[r] = m_run[r] == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m_run[r] - m_safe);
-        psum = 0.f;
-#pragma unroll
-        for (int kt = 0; kt < KT; ++kt)
-#pragma unroll
-          for (int j = 0; j < 4; ++j) {
-            const float p = __builtin_amdgcn_exp2f(__builtin_fmaf(s4[r][kt][j], scale_log2e, -m_safe));
-            psum += p;
-            pa[r][kt / 2][(kt % 2) * 4 + j] = (__bf16)p;
-          }
-        l_part[r] = l_part[r] * alpha[r] + psum;
-        m_run[r] = m_new;
-      } else {
-        l_part[r] += psum;
-      }
-    }
-    // The outputs are rescaled only when a reference has moved: a branch of the whole wave, taken rarely. (Written
-    // as a condition inside the loop over the output tiles, the compiler made a multiply and a select of it for
-    // every output entry in every tile, 128 instructions a tile; the empty statement keeps the branch a branch.)
-#pragma unroll
-    for (int r = 0; r < RT; ++r)
-      if (grow[r]) {
-        asm volatile("" ::: "memory");
-#pragma unroll
-        for (int dt = 0; dt < DTILES; ++dt)
-#pragma unroll
-          for (int j = 0; j < 4; ++j) o[r][dt][j] *= alpha[r];
-      }
-    // this lane points at key 4 grp + col / 4 of a 16-key sub-tile, entries 4 (col % 4).. of the 16-entry block dt
-    const int tr_key = grp * 4 + (col >> 2);
-    const int tr_piece = (col & 3) >> 1, tr_half = (col & 1) * 4;
-#pragma unroll
-    for (int dt = 0; dt < DTILES; ++dt) {
-#pragma unroll
-      for (int a = 0; a < KT / 2; ++a) {
-        // this lane's eight summation slots: keys 32 a + 4 grp + (0..3) and 32 a + 16 + 4 grp + (0..3), entry dt * 16 + col
-        const int k_lo = a * 32 + tr_key, k_hi = k_lo + 16;
-        const bf16_t* p_lo = v_s + k_lo * D + ((dt * 2 + tr_piece) ^ ((k_lo & VSWZ) << 1)) * 8 + tr_half;
-        const bf16_t* p_hi = v_s + k_hi * D + ((dt * 2 + tr_piece) ^ ((k_hi & VSWZ) << 1)) * 8 + tr_half;
-        const short4_t lo4 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) short4_t*)p_lo);
-        const short4_t hi4 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) short4_t*)p_hi);
-        typedef short short8_t __attribute__((ext_vector_type(8)));
-        const short8_t both = __builtin_shufflevector(lo4, hi4, 0, 1, 2, 3, 4, 5, 6, 7);
-        const bf16x8 va = __builtin_bit_cast(bf16x8, both);
-#pragma unroll
-        for (int r = 0; r < RT; ++r) o[r][dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(va, pa[r][a], o[r][dt], 0, 0, 0);
-      }
-    }
-    // V^T operands are read eight ahead of the one that is multiplied. (Left to itself the compiler reads two, waits for them, and multiplies: us
-    // so and now, 2,048 tokens after 14,336 502, 485; alone 59.1, 54.9; 512 after 4,000 77.9, 71.1; 901, 400 and 700 tokens 34.6, 33.1; 1 after 300,
-    // 17 after 40 and 333 after 1,000 27.2, 25.8. Two ahead 499, 58.0, 76.8; four 487, 55.9, 71.7. The same for the first product's operands: nothing.)
-    constexpr int OPERANDS = DTILES * KT / 2, AHEAD = OPERANDS < 8 ? OPERANDS : 8, DS_READ = 0x100, MATRIX = 0x8;
-    __builtin_amdgcn_sched_group_barrier(DS_READ, 2 * AHEAD, 0);
-#pragma unroll
-    for (int i = 0; i < OPERANDS - AHEAD; ++i) {
-      __builtin_amdgcn_sched_group_barrier(MATRIX, RT, 0);
-      __builtin_amdgcn_sched_group_barrier(DS_READ, 2, 0);
-    }
-    __builtin_amdgcn_sched_group_barrier(MATRIX, AHEAD * RT, 0);
+    auto key_operand = [&](int kt, int s) {
+      const int piece = s * 4 + grp;
+      return piece < CH ? *reinterpret_cast<const bf16x8*>(k_s + (kt * 16 + col) * D + (piece ^ (col & KSWZ)) * 8) : zero8();
+    };
+    attend<RT, KT, decltype(masked)::value, CAPPED, BIASED>(rows, kb, key_operand, v_s, col, grp, scale_log2e, cap_ratio, tanh_k);
   };
 
   auto run = [&](int kb, const bf16_t* k_s, const bf16_t* v_s) {
@@ -414,11 +552,11 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void p
   if (!live) return;
 #pragma unroll
   for (int r = 0; r < RT; ++r) {
-    float l = l_part[r];
+    float l = rows.l[r];
     l += __shfl_xor(l, 16, 64);
     l += __shfl_xor(l, 32, 64);
     if (row_ok[r]) {
-      if (MORE) l += __builtin_amdgcn_exp2f(row_sink[r] - m_run[r]);      // (a row that is stored has seen its own key: m_run is a number)
+      if (MORE) l += __builtin_amdgcn_exp2f(row_sink[r] - rows.m[r]);     // (a row that is stored has seen its own key: m is a number)
       float inv = 1.0f / l;
       if (MORE && gate) inv /= 1.0f + expf(-(float)gate[(size_t)(q_begin + row_tok[r]) * gate_ld + head[r]]);
       bf16_t* dst = out + ((size_t)(q_begin + row_tok[r]) * Hq + head[r]) * D;
@@ -426,7 +564,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void p
       for (int dt = 0; dt < DTILES; ++dt) {
         bf16x4 four;
 #pragma unroll
-        for (int j = 0; j < 4; ++j) four[j] = (__bf16)(o[r][dt][j] * inv);
+        for (int j = 0; j < 4; ++j) four[j] = (__bf16)(rows.o[r][dt][j] * inv);
         *reinterpret_cast<bf16x4*>(dst + dt * 16 + grp * 4) = four;
       }
     }

@@ -1224,6 +1224,51 @@ def test_prefill_attention_bfloat16(ops, Hq, Hkv, D, page, window):
     torch.testing.assert_close(out.double().cpu(), ref, **tol(torch.bfloat16))
 
 
+@pytest.mark.parametrize("Hq,Hkv,D,page,reach,cap,sinks,slopes,gated", [
+    (32, 8, 128, 16, None, None, None, False, False), (8, 2, 128, 256, ("window", 70), None, "each", False, True),
+    (16, 1, 128, 64, ("chunk", 50), 3.0, "one", False, False), (5, 5, 48, 7, None, None, None, True, True),
+    (6, 2, 80, 32, ("window", 1), None, "each", True, False), (3, 1, 16, 8, None, 2.0, None, False, True),
+    (4, 4, 64, 48, ("chunk", 33), None, "each", True, False), (7, 1, 112, 128, ("window", 333), None, None, False, False),
+])
+def test_prefill_attention_of_one_tile_beside_prompts(ops, Hq, Hkv, D, page, reach, cap, sinks, slopes, gated):
+    """Requests whose rows are one tile, whose keys four waves share, beside a longer portion: one to four tokens, from one key
+    over the edges of a wave's 32 and the four waves' 128 on, every option, and an infinite value that only its readers see."""
+    lens = [1, 31, 32, 33, 64, 127, 128, 129, 257, 300, 1700, 385, 200]
+    q_lens = [1, 1, 2, 1, 3, 1, 1, 4, 1, 2, 1, 16, 60]
+    q, kc, vc, batch, bt, ks, vs, qs = _paged_setup(torch.bfloat16, lens, q_lens, Hq, Hkv, D, page, seed=97, scale=1.5)
+    g = torch.Generator().manual_seed(98)
+    rows = torch.randn(q.shape[0], Hq + 3, generator=g).to(torch.bfloat16)
+    slope = torch.rand(Hq, generator=g) * 0.1 if slopes else None
+    sink = {None: None, "one": 0.7, "each": torch.randn(Hq, generator=g)}[sinks]
+    options = {"softcap": cap, "slopes": None if slope is None else slope.cuda(), "sink": sink.cuda() if sinks == "each" else sink,
+               "gate": (rows.cuda(), 2) if gated else None, **({reach[0]: reach[1]} if reach else {})}
+    out = ops.paged_attention(q, kc, vc, batch, bt, D ** -0.5, **options)
+    want, at = [], 0
+    for r, (n, nq) in enumerate(zip(lens, q_lens)):
+        pos, key = torch.arange(n - nq, n)[:, None], torch.arange(n)[None]
+        ok = key <= pos
+        if reach:
+            ok &= key > pos - reach[1] if reach[0] == "window" else key // reach[1] == pos // reach[1]
+        s = torch.einsum("qhd,khd->hqk", qs[r].double(), ks[r].double().repeat_interleave(Hq // Hkv, 1)) * D ** -0.5
+        s = cap * torch.tanh(s / cap) if cap else s
+        s = s - slope.double()[:, None, None] * (pos - key) if slopes else s
+        s = s.masked_fill(~ok, float("-inf"))
+        if sinks:
+            s = torch.cat((s, torch.as_tensor(sink, dtype=torch.float64).expand(Hq)[:, None, None].expand(Hq, nq, 1)), -1)
+        o = torch.einsum("hqk,khd->qhd", torch.softmax(s, -1)[..., :n], vs[r].double().repeat_interleave(Hq // Hkv, 1))
+        want.append(o * torch.sigmoid(rows[at:at + nq, 2:2 + Hq].double())[..., None] if gated else o)
+        at += nq
+    torch.testing.assert_close(out.double().cpu(), torch.cat(want), **tol(torch.bfloat16))
+    vc[bt[10, 1690 // page], 1690 % page, Hkv - 1, D - 1] = float("inf")
+    spoilt = ops.paged_attention(q, kc, vc, batch, bt, D ** -0.5, **options)
+    row = sum(q_lens[:10])
+    reads = not reach or (1690 > 1699 - reach[1] if reach[0] == "window" else 1690 // reach[1] == 1699 // reach[1])
+    assert bool(torch.isfinite(spoilt[row, Hq - 1, D - 1])) is not reads
+    hit = torch.zeros_like(out, dtype=torch.bool)
+    hit[row, Hq - Hq // Hkv:, D - 1] = reads
+    assert torch.equal(spoilt[~hit], out[~hit])
+
+
 @pytest.mark.parametrize("far", [3, 650, 1290])
 def test_prefill_attention_scores_that_outgrow_their_reference(ops, far):
     """The prompt kernel takes a row's exponentials against a reference point that stays while they stay far below
