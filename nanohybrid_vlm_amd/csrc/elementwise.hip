@@ -22,11 +22,21 @@ __global__ void embed_kernel(const int* __restrict__ ids, const T* __restrict__ 
   }
 }
 
+template <typename T>
+__global__ void embed_vec_kernel(const int* __restrict__ ids, const T* __restrict__ table, T* __restrict__ out, int H, int V, float scale) {
+  embed_row<T, T>(ids, table, out, H, V, scale);
+}
+
 extern "C" int nhv_embed(const void* ids, const void* table, void* out, int T, int H, int V, int dtype, float scale,
                          void* stream) {
   NHV_REQUIRE(T > 0 && H > 0 && V > 0, "embed: bad sizes T=%d H=%d V=%d", T, H, V);
   hipStream_t s = (hipStream_t)stream;
-  if (dtype == NHV_F32)
+  const bool pieces = embeds_by_pieces(table, out, H);
+  if (dtype == NHV_F32 && pieces)
+    hipLaunchKernelGGL(embed_vec_kernel<float>, dim3(T), dim3(embed_threads(H)), 0, s, (const int*)ids, (const float*)table, (float*)out, H, V, scale);
+  else if (dtype == NHV_BF16 && pieces)
+    hipLaunchKernelGGL(embed_vec_kernel<bf16_t>, dim3(T), dim3(embed_threads(H)), 0, s, (const int*)ids, (const bf16_t*)table, (bf16_t*)out, H, V, scale);
+  else if (dtype == NHV_F32)
     hipLaunchKernelGGL(embed_kernel<float>, dim3(T), dim3(256), 0, s, (const int*)ids, (const float*)table, (float*)out, H, V, scale);
   else if (dtype == NHV_BF16)
     hipLaunchKernelGGL(embed_kernel<bf16_t>, dim3(T), dim3(256), 0, s, (const int*)ids, (const bf16_t*)table, (bf16_t*)out, H, V, scale);
@@ -579,10 +589,37 @@ __global__ void scale_rows_kernel(const bf16_t* __restrict__ x, const float* __r
   for (int i = threadIdx.x; i < H; i += blockDim.x) y[(size_t)m * H + i] = (bf16_t)((float)x[(size_t)m * H + i] * r);
 }
 
+// The same in pieces of eight entries, the row asked for with the squares: 8 rows of 4,096 7.5 us entry by entry, 4.7 so.
+template <int PIECES>
+__global__ __launch_bounds__(256) void scale_rows_vec_kernel(const bf16_t* __restrict__ x, const float* __restrict__ ss, int tiles, float eps,
+                                                             bf16_t* __restrict__ y, int H) {
+  __shared__ float scratch[16];
+  const int m = blockIdx.x;
+  float v[PIECES][8];
+#pragma unroll
+  for (int p = 0; p < PIECES; ++p) load8f<bf16_t>(x + (size_t)m * H + min((p * 256 + (int)threadIdx.x) * 8, H - 8), v[p]);
+  float sum = 0.f;
+  for (int t = threadIdx.x; t < tiles; t += 256) sum += ss[(size_t)m * tiles + t];
+  const float total = block_sum(sum, scratch);
+  const float r = 1.0f / sqrtf(total / (float)H + eps);
+#pragma unroll
+  for (int p = 0; p < PIECES; ++p) {
+    const int i = (p * 256 + (int)threadIdx.x) * 8;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) v[p][e] *= r;
+    if (i < H) store8f<bf16_t>(y + (size_t)m * H + i, v[p]);
+  }
+}
+
 extern "C" int nhv_scale_rows(const void* x, const void* ss, int tiles, float eps, void* y, int M, int H, void* stream) {
   NHV_REQUIRE(M > 0 && H > 0 && tiles > 0, "scale_rows: bad sizes M=%d H=%d tiles=%d", M, H, tiles);
-  hipLaunchKernelGGL(scale_rows_kernel, dim3(M), dim3(256), 0, (hipStream_t)stream, (const bf16_t*)x, (const float*)ss, tiles,
-                     eps, (bf16_t*)y, H);
+  const bool aligned = H % 8 == 0 && (((uintptr_t)x | (uintptr_t)y) & 15) == 0;
+  if (aligned && H <= 2048)
+    hipLaunchKernelGGL(scale_rows_vec_kernel<1>, dim3(M), dim3(256), 0, (hipStream_t)stream, (const bf16_t*)x, (const float*)ss, tiles, eps, (bf16_t*)y, H);
+  else if (aligned && H <= 8192)
+    hipLaunchKernelGGL(scale_rows_vec_kernel<4>, dim3(M), dim3(256), 0, (hipStream_t)stream, (const bf16_t*)x, (const float*)ss, tiles, eps, (bf16_t*)y, H);
+  else
+    hipLaunchKernelGGL(scale_rows_kernel, dim3(M), dim3(256), 0, (hipStream_t)stream, (const bf16_t*)x, (const float*)ss, tiles, eps, (bf16_t*)y, H);
   NHV_LAUNCH_CHECK("scale_rows");
   return 0;
 }

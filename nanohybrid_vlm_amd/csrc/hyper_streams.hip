@@ -15,6 +15,7 @@
 // 1,024 on); a thread owns columns i, i + threads, ...; the sum over a row's squares is taken in an order that
 // depends on the width only, so a token's result does not depend on its batch.
 #include "nhv_common.h"
+#include "nhv_head_pieces.h"
 #include <math.h>
 
 #define NHV_MAX_STREAMS 16
@@ -138,11 +139,21 @@ __global__ void embed_float_kernel(const int* __restrict__ ids, const T* __restr
   for (int i = threadIdx.x; i < W; i += blockDim.x) out[(size_t)t * W + i] = ok ? to_f32(src[i]) * scale : 0.f;
 }
 
+template <typename T>
+__global__ void embed_float_vec_kernel(const int* __restrict__ ids, const T* __restrict__ table, float* __restrict__ out, int W, int V, float scale) {
+  embed_row<T, float>(ids, table, out, W, V, scale);
+}
+
 extern "C" int nhv_embed_float(const void* ids, const void* table, void* out, int T, int W, int V, int dtype, float scale,
                                void* stream) {
   NHV_REQUIRE(T > 0 && W > 0 && V > 0, "embed_float: bad sizes T=%d W=%d V=%d", T, W, V);
   hipStream_t s = (hipStream_t)stream;
-  if (dtype == NHV_F32)
+  const bool pieces = embeds_by_pieces(table, out, W);
+  if (dtype == NHV_F32 && pieces)
+    hipLaunchKernelGGL(embed_float_vec_kernel<float>, dim3(T), dim3(embed_threads(W)), 0, s, (const int*)ids, (const float*)table, (float*)out, W, V, scale);
+  else if (dtype == NHV_BF16 && pieces)
+    hipLaunchKernelGGL(embed_float_vec_kernel<bf16_t>, dim3(T), dim3(embed_threads(W)), 0, s, (const int*)ids, (const bf16_t*)table, (float*)out, W, V, scale);
+  else if (dtype == NHV_F32)
     hipLaunchKernelGGL(embed_float_kernel<float>, dim3(T), dim3(256), 0, s, (const int*)ids, (const float*)table, (float*)out, W, V, scale);
   else if (dtype == NHV_BF16)
     hipLaunchKernelGGL(embed_float_kernel<bf16_t>, dim3(T), dim3(256), 0, s, (const int*)ids, (const bf16_t*)table, (float*)out, W, V, scale);

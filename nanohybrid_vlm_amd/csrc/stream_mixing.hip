@@ -9,6 +9,7 @@
 //    position, mixes values with another layer's, and stores keys and values at the step's slots.
 // Statistics, angles and sums are float; rows are float or bfloat16.
 #include "nhv_common.h"
+#include "nhv_head_pieces.h"
 #include "nhv_rotation.h"
 #include <math.h>
 
@@ -28,13 +29,43 @@ __global__ void scalar_rmsnorm_kernel(const TI* __restrict__ x, const float* __r
   for (int i = threadIdx.x; i < W; i += blockDim.x) y[base + i] = from_f32<TO>(to_f32(x[base + i]) * r);
 }
 
+// The same with the row in registers, in pieces of eight entries: 2,264 rows of 2,048 12.1 us from bfloat16 to
+// float and 11.2 the other way, entry by entry and read twice, 9.0 and 6.8 so.
+template <typename TI, typename TO, int PIECES>
+__global__ __launch_bounds__(256) void scalar_rmsnorm_vec_kernel(const TI* __restrict__ x, const float* __restrict__ gain, TO* __restrict__ y, int W,
+                                                                 float eps) {
+  __shared__ float scratch[16];
+  const size_t base = (size_t)blockIdx.x * W;
+  float v[PIECES][8], ss = 0.f;
+#pragma unroll
+  for (int p = 0; p < PIECES; ++p) load8f<TI>(x + base + min((p * 256 + (int)threadIdx.x) * 8, W - 8), v[p]);
+#pragma unroll
+  for (int p = 0; p < PIECES; ++p)
+    if ((p * 256 + (int)threadIdx.x) * 8 < W)
+#pragma unroll
+      for (int e = 0; e < 8; ++e) ss = fmaf(v[p][e], v[p][e], ss);
+  const float r = gain[0] / sqrtf(block_sum(ss, scratch) / (float)W + eps);
+#pragma unroll
+  for (int p = 0; p < PIECES; ++p) {
+    const int i = (p * 256 + (int)threadIdx.x) * 8;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) v[p][e] *= r;
+    if (i < W) store8f<TO>(y + base + i, v[p]);
+  }
+}
+
 extern "C" int nhv_scalar_rmsnorm(const void* x, int x_dtype, const void* gain, void* y, int y_dtype, int T, int W, float eps,
                                   void* stream) {
   NHV_REQUIRE(T > 0 && W > 0, "scalar_rmsnorm: bad sizes T=%d W=%d", T, W);
   hipStream_t s = (hipStream_t)stream;
-#define LAUNCH(TI, TO)                                                                                               \
-  hipLaunchKernelGGL((scalar_rmsnorm_kernel<TI, TO>), dim3(T), dim3(256), 0, s, (const TI*)x, (const float*)gain, (TO*)y, \
-                     W, eps)
+  const bool aligned = W % 8 == 0 && (((uintptr_t)x | (uintptr_t)y) & 15) == 0;
+#define LAUNCH(TI, TO)                                                                                                     \
+  do {                                                                                                                     \
+    auto kernel = !aligned || W > 8192 ? scalar_rmsnorm_kernel<TI, TO>                                                     \
+                  : W <= 2048          ? scalar_rmsnorm_vec_kernel<TI, TO, 1>                                              \
+                                       : scalar_rmsnorm_vec_kernel<TI, TO, 4>;                                             \
+    hipLaunchKernelGGL(kernel, dim3(T), dim3(256), 0, s, (const TI*)x, (const float*)gain, (TO*)y, W, eps);                \
+  } while (0)
   if (x_dtype == NHV_F32 && y_dtype == NHV_F32) LAUNCH(float, float);
   else if (x_dtype == NHV_F32 && y_dtype == NHV_BF16) LAUNCH(float, bf16_t);
   else if (x_dtype == NHV_BF16 && y_dtype == NHV_F32) LAUNCH(bf16_t, float);

@@ -2131,3 +2131,35 @@ def test_a_matrix_per_head_of_many_rows(ops, H, N, K, rot, rows):
             got = ops.head_gemm(x, w.view(H * N, K), False, N, K, gate=(gate, col, per))
             s = torch.sigmoid(gate.double())[:, col:col + (H * N if per == "per entry" else H)].reshape(rows, H, -1)
             assert bool(((got.double() - want * s).abs() <= (want * s).abs() * 2.0 ** -8 + 2.0 ** -20 * K ** 0.5 * float(want.std())).all()), (per, col)
+
+
+@pytest.mark.parametrize("H", [8, 24, 511, 520, 2048, 2056, 4096, 8192, 8200])
+def test_rows_in_pieces_of_eight(ops, H):
+    """Embeddings, scaled sums and norms by one number where a row is a whole number of pieces, one or several a thread, and where
+    it is not or does not begin on 16 bytes: the same as entry by entry."""
+    g = torch.Generator(device="cuda").manual_seed(H)
+    backend = ops.backend()
+    for dtype in (torch.float32, torch.bfloat16):
+        flat = torch.randn(40 * H + 1, generator=g, device="cuda").to(dtype)
+        for table in (flat[:-1].view(40, H), flat[1:].view(40, H)):
+            ids = torch.tensor([0, 39, 7, -1, 40, 12], dtype=torch.int32, device="cuda")
+            want = table[ids.long().clamp(0, 39)] * ((ids >= 0) & (ids < 40))[:, None].to(dtype)
+            for scale in (1.0, 1.75):
+                out = torch.empty(6, H, dtype=dtype, device="cuda")
+                backend.embed(ids, table, out, scale)
+                assert torch.equal(out, (want.float() * scale).to(dtype))
+                out = torch.empty(6, H, device="cuda")
+                backend.embed_float(ids, table, out, scale)
+                assert torch.equal(out, want.float() * scale)
+            gain = torch.tensor([1.3], device="cuda")
+            for to in (torch.float32, torch.bfloat16):
+                got = ops.scalar_rmsnorm(table, gain, 1e-5, to)
+                exact = table.double() * (1.3 / (table.double().square().mean(-1, keepdim=True) + 1e-5).sqrt())
+                # float sums of H squares: H^0.5 2^-24 of the mean, half of that of the root; and one rounding
+                assert bool(((got.double() - exact).abs() <= exact.abs() * (2.0 ** -8 if to == torch.bfloat16 else 2.0 ** -21)).all())
+    for tiles in (1, 128, 300):
+        x, squares = torch.randn(5, H, generator=g, device="cuda").to(torch.bfloat16), torch.rand(5, tiles, generator=g, device="cuda")
+        out = torch.empty_like(x)
+        backend.scale_rows(x, squares, 1e-5, out)
+        exact = x.double() / (squares.double().sum(-1, keepdim=True) / H + 1e-5).sqrt()
+        assert bool(((out.double() - exact).abs() <= exact.abs() * (2.0 ** -8 + 2.0 ** -20)).all())
