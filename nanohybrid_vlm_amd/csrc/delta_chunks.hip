@@ -21,10 +21,14 @@
 // The second is a chain of chunks, and what it lasts is what a chunk waits for (two rows of dependent matrix instructions and
 // one exchange between the waves: 0.82 us a chunk), not its arithmetic; the token-by-token kernel takes 0.36 us a token. Eight
 // waves a block, a tile each, wait longer for each other (99 us where four took 91).
-// us, before and now, of the preparation (which brings W and R into the second kernel's order) and of the chain (whose loads are
-// whole kilobytes, whose results are stored without a branch, and which multiplies R while the shares come back): portions of 1,500 and 764 tokens, 16 heads of
-// 128, 75, 77 and 88, 77; of 64 53, 56 and 55, 49; 8 heads of 256 on 128 108, 114 and 171, 140; 24 of 80 tokens, 16 heads of 128, 67, 69 and 69, 54; 8,000 tokens 248, 274
-// and 446, 389.
+// us of the chain, before its loads were whole kilobytes in the preparation's order, its results were stored without a branch and R was
+// multiplied while the shares come back, and now: portions of 1,500 and 764 tokens, 16 heads of 128, 88, 77; of 64 55, 49; 8 heads of 256 on
+// 128 171, 140; 24 of 80 tokens, 16 heads of 128, 69, 54; 8,000 tokens 446, 389.
+// The preparation is bound by its vector instructions (80 % of the clocks of all SIMDs). It took 4,230 a wave, of which 1,520 were the
+// decays (a division to find token and channel, log1pf, expf), 720 the inputs' SiLU and 280 moved scalar values to vector
+// registers and back; with the functions below, rows dealt to waves, and nothing worked out ahead that a wave cannot keep, half of
+// that: the same sizes 77, 60; 56, 42; 114, 81; 69, 50; 274, 175 us, 40 and 17 tokens 22, 15. Results are as far from 64 bits as before (1.7e-7 to
+// 2.8e-7 of their size, by how slowly they decay).
 // Portions of 1,500 and 701 tokens, 16 heads of 128, with the update of the kept inputs and the read-out's norm: 198 us where the
 // separate kernels take 638; one of 8,000 770 against 3,204. The blocks of the preparation are requests by the longest portion:
 // for 2,000 tokens beside 60 decoded ones 98 of 100 are empty, which is 16 us of 290 (a search for each place's request gave
@@ -34,6 +38,7 @@
 // "The WY representation for products of Householder matrices", 1987), is that of Yang, Wang, Zhang, Shen and Kim,
 // "Parallelizing Linear Transformers with the Delta Rule over Sequence Length", 2024, here with a decay a key channel.
 #include "nhv_common.h"
+#include <float.h>
 #include <math.h>
 
 typedef __attribute__((__vector_size__(4 * sizeof(float)))) float floatx4;
@@ -43,8 +48,25 @@ typedef __attribute__((__vector_size__(4 * sizeof(float)))) float floatx4;
 #define NHV_MAX_TAPS 16
 
 __device__ __forceinline__ float exp2_of(float x) { return __builtin_amdgcn_exp2f(x); }   // (x <= 0; tiny results may become 0)
-__device__ __forceinline__ float silu_of(float z) { return z / (1.0f + expf(-z)); }
-__device__ __forceinline__ float softplus_of(float z) { return z > 20.f ? z : log1pf(expf(z)); }
+// e^x for |x| up to 110, the part of x log2(e) behind the whole number in two pieces of log2(e)
+__device__ __forceinline__ float exp_of(float x) {
+  const float whole = __builtin_rintf(x * 1.44269502f);
+  return ldexpf(exp2_of(fmaf(x, 1.92596299e-8f, fmaf(x, 1.44269502f, -whole))), (int)whole);
+}
+// z / (1 + e^-z): the quotient by the reciprocal, put right by what it leaves of z (off by 3.7e-8 on average, as the division is, in half
+// the instructions)
+__device__ __forceinline__ float silu_of(float z) {
+  const float d = 1.0f + exp_of(__builtin_amdgcn_fmed3f(-z, -110.f, 110.f)), r = __builtin_amdgcn_rcpf(d), q = z * r;
+  const float y = fmaf(fmaf(-d, q, z), r, q);
+  return y == y ? y : q;                     // (an infinite d or z leaves no number)
+}
+// rate log2(1 + e^z), rate log2(e) in two pieces: max(z, 0) log2(e) and log2(w), w = 1 + e^-|z|, of which w's own rounding c is the part c / w.
+// Off by 2.5e-8 (z > 1) to 5.1e-8 (z down to -12; below, where nothing decays, 7e-8) on average; -log2(e) rate log1p(e^z) by the
+// library's functions 4.6e-8 to 5.3e-8, and 190 instructions with its addresses where this is 40.
+__device__ __forceinline__ float softplus_bits(float z, float rate, float bits, float rest) {
+  const float a = fabsf(z), u = exp_of(a > 110.f ? -110.f : -a), w = 1.0f + u, c = u - (w - 1.0f), m = fmaxf(z, 0.f);
+  return fmaf(bits, m, fmaf(rest, m, fmaf(rate, __builtin_amdgcn_logf(w), c * __builtin_amdgcn_rcpf(w) * bits)));
+}
 #define NHV_LOWEST_LOG (-256.f)
 
 struct DeltaIn {
@@ -71,6 +93,8 @@ struct DeltaChunks {                         // per (place, head); a chunk's pla
 // A channel's sixteen convolved inputs, through SiLU; zeros for tokens beyond n. TAPS 0: any number.
 template <typename TI, int TAPS>
 __device__ __forceinline__ void convolved(const DeltaIn& in, int c, int first, int i0, int pos0, const float* mine, int n, float* y) {
+  // (taken anew at each call: worked out ahead for all calls, rows' places and conditions would be kept in parts of vector registers)
+  asm volatile("" : "+s"(first), "+s"(i0), "+s"(n), "+s"(pos0));
   const TI* col = (const TI*)in.proj + (size_t)first * in.ld + c;
   const int taps = TAPS ? TAPS : in.n_taps;
   const float* tap = in.taps + (size_t)c * taps;
@@ -95,15 +119,20 @@ __device__ __forceinline__ void convolved(const DeltaIn& in, int c, int first, i
       float sum = 0.f;
 #pragma unroll
       for (int j = 0; j < TAPS; ++j) sum = fmaf(m[j], x[t + TAPS - 1 - j], sum);
-      y[t] = t < n ? silu_of(sum) : 0.f;
+      y[t] = silu_of(sum);
     }
   } else {
 #pragma unroll
     for (int t = 0; t < NHV_CHUNK; ++t) {
       float sum = 0.f;
       for (int j = 0; j < taps; ++j) sum = fmaf(tap[taps - 1 - j], input(t - j), sum);
-      y[t] = t < n ? silu_of(sum) : 0.f;
+      y[t] = silu_of(sum);
     }
+  }
+  if (n < NHV_CHUNK) {                       // (one branch, not one a token)
+    asm volatile("");
+#pragma unroll
+    for (int t = 0; t < NHV_CHUNK; ++t) y[t] = t < n ? y[t] : 0.f;
   }
 }
 
@@ -127,7 +156,7 @@ __global__ __launch_bounds__(256, 4) void delta_chunks_prepare_kernel(const Delt
 
   // queries and keys, a channel a thread; the decays' logarithms; beta
   for (int x = tid; x < 2 * Dp; x += 256) {
-    const int d = x % Dp;
+    const int d = x < Dp ? x : x - Dp;
     float* to_row = (x < Dp ? qs : ks) + d;
     float y[NHV_CHUNK];
 #pragma unroll
@@ -136,11 +165,20 @@ __global__ __launch_bounds__(256, 4) void delta_chunks_prepare_kernel(const Delt
 #pragma unroll
     for (int t = 0; t < NHV_CHUNK; ++t) to_row[t * LD] = y[t];
   }
-  const float rate = expf(in.a_log[h]);
-  for (int x = tid; x < NHV_CHUNK * Dp; x += 256) {
-    const int t = x / Dp, d = x % Dp, at = h * Dd + (Dd == 1 ? 0 : d);
-    const float l = t < n && d < D ? -NHV_LOG2E * (rate * softplus_of(in.a_lin[(size_t)(t0 + t) * in.a_ld + at] + in.dt_bias[at])) : 0.f;
-    ls[t * LD + d].x = l < NHV_LOWEST_LOG ? NHV_LOWEST_LOG : l;      // (what is no number stays none)
+  // (four rows a wave, channels on its lanes: no division, and a row's address is the wave's)
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
+  // (finite pieces, so that they leave nothing of what does not decay; what is no number stays none)
+  const float asked = expf(in.a_log[h]), rate = asked > FLT_MAX ? FLT_MAX : asked;
+  const float bits = rate > FLT_MAX / 1.5f ? FLT_MAX : rate * 1.44269502f, rest = fmaf(rate, 1.92596299e-8f, fmaf(rate, 1.44269502f, -bits));
+  for (int d = lane; d < Dp; d += 64) {
+    const int at = h * Dd + (Dd == 1 ? 0 : min(d, D - 1));
+    const float bias = in.dt_bias[at];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int t = wave + 4 * i;
+      const float l = -softplus_bits(in.a_lin[(size_t)(t0 + min(t, n - 1)) * in.a_ld + at] + bias, rate, bits, rest);
+      ls[t * LD + d].x = t < n && d < D ? (l < NHV_LOWEST_LOG ? NHV_LOWEST_LOG : l) : 0.f;      // (what is no number stays none)
+    }
   }
   if (tid < NHV_CHUNK)
     beta[tid] = tid < n ? 1.0f / (1.0f + expf(-to_f32(((const TI*)in.proj)[(size_t)(t0 + tid) * in.ld + C + h]))) : 0.f;
@@ -219,13 +257,17 @@ __global__ __launch_bounds__(256, 4) void delta_chunks_prepare_kernel(const Delt
   }
   __syncthreads();
   // E_t q_t, E_t k_t and, in the sums' place, k_t 2^(l_16 - l_t) (rows beyond n are zeros)
-  for (int x = tid; x < NHV_CHUNK * Dp; x += 256) {
-    const int d = x % Dp, at = x / Dp * LD + d;
-    const float2 l = ls[at];
-    const float e = exp2_of(l.x + l.y), k = ks[at];
-    qs[at] *= e;
-    ks[at] = e * k;
-    ls[at].x = k * exp2_of((last[d].x - l.x) + (last[d].y - l.y));
+  for (int d = lane; d < Dp; d += 64) {
+    const float2 all = last[d];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int at = (wave + 4 * i) * LD + d;
+      const float2 l = ls[at];
+      const float e = exp2_of(l.x + l.y), k = ks[at];
+      qs[at] *= e;
+      ks[at] = e * k;
+      ls[at].x = k * exp2_of((all.x - l.x) + (all.y - l.y));
+    }
   }
   __syncthreads();
   // a column a thread: W's Dp, then V''s E
