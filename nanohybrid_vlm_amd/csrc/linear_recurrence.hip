@@ -161,24 +161,34 @@ __global__ __launch_bounds__(256) void recurrence_prepare_kernel(const Recurrenc
     floatx4 acc[MAX_TILES];
 #pragma unroll
     for (int i = 0; i < MAX_TILES; ++i) acc[i] = zero;
-    const float* z = in.z + (size_t)(t0 + min(col, n - 1)) * in.z_ld;
-    for (int r0 = 0; r0 < in.rank; r0 += 16) {
-      const int r = r0 + grp * 4;
-      floatx4 x, w[MAX_TILES];
+    // (Vector instructions keep this kernel: every wave's own tanh of all of z, and a condition a load, were a quarter of them. Once a block, 64
+    // columns at a time through LDS: the sizes of the chain's figures 56, 44 us; 77, 62; 82, 65; 73, 58.)
+    constexpr int PIECE = 64, ZLD = PIECE + 4;
+    __shared__ __attribute__((aligned(16))) float zs[NHV_CHUNK * ZLD];
+    for (int r00 = 0; r00 < in.rank; r00 += PIECE) {
+      if (r00 > 0) __syncthreads();
 #pragma unroll
-      for (int j = 0; j < 4; ++j) x[j] = r + j < in.rank ? z[r + j] : 0.f;
-#pragma unroll
-      for (int i = 0; i < MAX_TILES; ++i) {
-        const int d = (wave + 4 * i) * 16 + col;
-        w[i] = (d < D && r < in.rank) ? four_of((const TW*)in.w2 + ((size_t)h * D + d) * in.rank + r, in.rank - r, whole_rank) : zero;
+      for (int i = 0; i < 4; ++i) {
+        const int t = wave + 4 * i, r = r00 + lane;
+        const float z = in.z[(size_t)(t0 + min(t, n - 1)) * in.z_ld + min(r, in.rank - 1)];
+        zs[t * ZLD + lane] = r < in.rank ? tanhf(z) : 0.f;
       }
+      __syncthreads();
+      for (int r0 = r00; r0 < min(r00 + PIECE, in.rank); r0 += 16) {
+        const int r = r0 + grp * 4;
+        floatx4 w[MAX_TILES];
 #pragma unroll
-      for (int j = 0; j < 4; ++j) x[j] = tanhf(x[j]);
+        for (int i = 0; i < MAX_TILES; ++i) {
+          const int d = (wave + 4 * i) * 16 + col;
+          w[i] = (d < D && r < in.rank) ? four_of((const TW*)in.w2 + ((size_t)h * D + d) * in.rank + r, in.rank - r, whole_rank) : zero;
+        }
+        const floatx4 x = *reinterpret_cast<const floatx4*>(&zs[col * ZLD + r - r00]);
 #pragma unroll
-      for (int i = 0; i < MAX_TILES; ++i)
-        if ((wave + 4 * i) * 16 < Dp)
+        for (int i = 0; i < MAX_TILES; ++i)
+          if ((wave + 4 * i) * 16 < Dp)
 #pragma unroll
-          for (int j = 0; j < 4; ++j) acc[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(x[j], w[i][j], acc[i], 0, 0, 0);
+            for (int j = 0; j < 4; ++j) acc[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(x[j], w[i][j], acc[i], 0, 0, 0);
+      }
     }
     // a lane holds channel d at the tokens 4 grp .. 4 grp + 3: sums along them, then over the groups before
 #pragma unroll
@@ -278,8 +288,9 @@ __global__ __launch_bounds__(256) void recurrence_prepare_kernel(const Recurrenc
     }
     a_out[place * 256 + tid] = sum;
   }
+  // R lies as the second kernel's lanes take it, [Dp / 16][4][16][4]: of a tile of 16 channels, four channels, their tokens
   for (int x = tid; x < NHV_CHUNK * fours; x += 256) {
-    const int t = x / fours, d = (x % fours) * 4;
+    const int t = x & 15, d = (x >> 4) * 4;
     floatx4 r = *reinterpret_cast<const floatx4*>(&rs[t * LD + d]);
     if (KIND == 0) {
       r *= exp2_of(l2 * (float)(t + 1));
@@ -316,16 +327,20 @@ struct ChunkOperands {
   float a;
 };
 
-// (two waves a SIMD at least: with at most 256 registers a wave the products' sums stay in ordinary registers)
-template <typename T, int TPW, bool EVEN>
-__global__ __launch_bounds__(256, 2) void recurrence_chunks_kernel(const float* __restrict__ r_in, const float* __restrict__ k_in,
+// What bounds it is the way to a chunk's operands, for which few chains wait at a time. Loads are whole kilobytes in the preparation's order, places go on by
+// additions, results are stored without a branch. us before and now, 16 heads of 128: 16 portions of 20 to 200 60, 48; 24 of 100 to 160 92, 72; 3 of 900 to 1,300 107, 90;
+// one of 3,000 137, 124.
+// AHEAD 2 leaves room for three waves a SIMD, AHEAD 3 for two (at least: with at most 256 registers a wave the products' sums stay in
+// ordinary registers); tiles of more than 32 rows a wave have room for 2 and two. Where there are more blocks than two a compute unit the third
+// counts for more, else the third chunk: 16 portions of 20 to 200 52, 48 us, 24 of 100 to 160 77, 72; 3 of 900 to 1,300 89, 91, one of 3,000 125, 130.
+template <typename T, int TPW, bool EVEN, int AHEAD>
+__global__ __launch_bounds__(256, TPW <= 2 && AHEAD == 2 ? 3 : 2) void recurrence_chunks_kernel(const float* __restrict__ r_in, const float* __restrict__ k_in,
                                                                 const float* __restrict__ a_in, const float* __restrict__ decay_in,
                                                                 const T* __restrict__ v, long long ld, float* __restrict__ state,
                                                                 float* __restrict__ out, const int* __restrict__ positions,
                                                                 const int* __restrict__ cu, const int* __restrict__ state_slots,
                                                                 int H, int D, int Dp, int E) {
-  constexpr int AHEAD = TPW <= 2 ? 3 : 2;
-  __shared__ float red[2][4][NHV_CHUNK][17];
+  __shared__ __attribute__((aligned(16))) float red[2][4][64 * 4];
   const int req = blockIdx.z, h = blockIdx.x, e0 = blockIdx.y * 16;
   const int first = cu[req], end = cu[req + 1];
   if (end <= first) return;                  // (the same for the whole block)
@@ -345,52 +360,57 @@ __global__ __launch_bounds__(256, 2) void recurrence_chunks_kernel(const float* 
   const int chunks = (end - first + NHV_CHUNK - 1) / NHV_CHUNK;
   const size_t place0 = (size_t)(first / NHV_CHUNK) + req;
   ChunkOperands<T, TPW> ops[AHEAD];
-  // what a lane reads of a chunk lies at offsets that do not change, from bases that are the same for the whole block
-  const int r_at = col * Dp + tile0 * 16 + grp * 4, k_at = (tile0 * 16 + col) * NHV_CHUNK + grp * 4, g_at = tile0 * 16 + grp * 4;
+  // what a lane reads of a chunk lies at offsets that do not change, from bases that are the same for the whole block and go on by additions
+  const int r_at = tile0 * 256 + lane * 4, k_at = (tile0 * 16 + col) * NHV_CHUNK + grp * 4, g_at = tile0 * 16 + grp * 4;
   const int a_at = col * 16 + grp * 4 + wave;
+  const size_t place = place0 * H + h;
+  const float *rb = r_in + place * NHV_CHUNK * Dp, *kb = k_in + place * NHV_CHUNK * Dp, *gb = decay_in + place * Dp, *ab = a_in + place * 256;
   const int spare = (EVEN ? 0 : tiles) - 1;  // (a wave without a tile reads the last one's and leaves it unused)
   const T* vbase = v + (size_t)first * ld + (size_t)h * E + e0;
   const int row = (int)ld, vlast = (end - first - 1) * row + (column ? col : 0);       // (a lane beyond E works on a column that it does not write)
   int v_at[4], v_mine_at = (grp * 4 + wave) * row + (column ? col : 0);
 #pragma unroll
   for (int j = 0; j < 4; ++j) v_at[j] = (grp * 4 + j) * row + (column ? col : 0);
-  auto ask = [&](ChunkOperands<T, TPW>& x, int c) {      // (in the order of the chunks)
-    c = min(c, chunks - 1);                  // (always asked, so that the loop's waits count the same loads on every way)
-    const size_t place = (place0 + c) * H + h;
-    const float* rb = r_in + place * NHV_CHUNK * Dp;
-    const float* kb = k_in + place * NHV_CHUNK * Dp;
-    const float* gb = decay_in + place * Dp;
+  int asked = 0;
+  auto ask = [&](ChunkOperands<T, TPW>& x) {             // (behind the last chunk: it again, so that the loop's waits count the same loads on every way)
 #pragma unroll
     for (int i = 0; i < TPW; ++i) {
       const int back = EVEN ? 0 : max(tile0 + i - spare, 0);
-      x.r[i] = *reinterpret_cast<const floatx4*>(rb + (r_at + (i - back) * 16));
-      x.g[i] = *reinterpret_cast<const floatx4*>(gb + (g_at + (i - back) * 16));
-      x.kk[i] = *reinterpret_cast<const floatx4*>(kb + (k_at + (i - back) * 16 * NHV_CHUNK));
+      x.r[i] = *reinterpret_cast<const floatx4*>(rb + (uint32_t)(r_at + (i - back) * 256));
+      x.g[i] = *reinterpret_cast<const floatx4*>(gb + (uint32_t)(g_at + (i - back) * 16));
+      x.kk[i] = *reinterpret_cast<const floatx4*>(kb + (uint32_t)(k_at + (i - back) * 16 * NHV_CHUNK));
     }
     // (rows beyond the request meet zeros in A and K: the request's last row stands in for them)
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
-      x.v[j] = vbase[min(v_at[j], vlast)];
+      x.v[j] = vbase[(uint32_t)min(v_at[j], vlast)];
       v_at[j] += NHV_CHUNK * row;
     }
-    x.v_mine = vbase[min(v_mine_at, vlast)];
+    x.v_mine = vbase[(uint32_t)min(v_mine_at, vlast)];
     v_mine_at += NHV_CHUNK * row;
-    x.a = a_in[place * 256 + a_at];
+    x.a = ab[(uint32_t)a_at];
+    const size_t on = ++asked < chunks ? (size_t)H : 0;
+    rb += on * NHV_CHUNK * Dp, kb += on * NHV_CHUNK * Dp, gb += on * Dp, ab += on * 256;
   };
-  const int o_at = (tid >> 4) * H * E + (tid & 15);
-  // the waves' shares of chunk c added up and written
-  auto emit = [&](int c) {
-    const int t = first + c * NHV_CHUNK + (tid >> 4), e = e0 + (tid & 15);
-    float sum = 0.f;
+  // Wave w writes tokens 4 grp + w of a chunk, the sum of the four waves' shares. Tokens behind the request's last one and columns behind E lie
+  // behind the end of what is described here, and are not written: without a branch the products go on beside it.
+  const uint32_t o_at = column ? (uint32_t)((grp * 4 + wave) * H * E + col) * 4 : 0x80000000u;
+  auto emit = [&](const float* share, int c) {
+    const int t = first + c * NHV_CHUNK;
+    const int bytes = (min(NHV_CHUNK, end - t) * H * E - h * E - e0) * 4;
+    __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, ((share[0] + share[1]) + share[2]) + share[3]),
+                                          __builtin_amdgcn_make_buffer_rsrc(out + ((size_t)t * H + h) * E + e0, 0, bytes, 0x00020000), o_at, 0, 0);
+  };
+  auto shares = [&](int c, float* share) {
 #pragma unroll
-    for (int w = 0; w < 4; ++w) sum += red[c & 1][w][tid >> 4][tid & 15];
-    float* ob = out + ((size_t)(first + c * NHV_CHUNK) * H + h) * E + e0;
-    if (t < end && e < E) ob[o_at] = sum;
+    for (int w = 0; w < 4; ++w) share[w] = red[c & 1][w][lane * 4 + wave];
   };
   auto step = [&](ChunkOperands<T, TPW>& x, int c) {
     float vv[4];
 #pragma unroll
     for (int j = 0; j < 4; ++j) vv[j] = to_f32(x.v[j]);
+    float share[4];
+    if (c > 0) shares(c - 1, share);
     floatx4 o = {0.f, 0.f, 0.f, 0.f}, o2 = {0.f, 0.f, 0.f, 0.f};
     // this wave's share of A V: the tokens 4 grp + wave
     o2 = __builtin_amdgcn_mfma_f32_16x16x4f32(x.a, to_f32(x.v_mine), o2, 0, 0, 0);
@@ -409,16 +429,16 @@ __global__ __launch_bounds__(256, 2) void recurrence_chunks_kernel(const float* 
 #pragma unroll
       for (int i = 0; i < TPW; ++i)
         if (EVEN || tile0 + i < tiles) S[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(x.kk[i][j], vv[j], S[i], 0, 0, 0);
-    ask(x, c + AHEAD);
-    if (c > 0) emit(c - 1);                  // (while the products are under way)
-#pragma unroll
-    for (int j = 0; j < 4; ++j) red[c & 1][wave][grp * 4 + j][col] = o[j] + o2[j];
+    __builtin_amdgcn_sched_barrier(0);       // (what is asked for takes the places of what was used: loads between the products would need others)
+    ask(x);
+    if (c > 0) emit(share, c - 1);           // (while the products are under way)
+    *reinterpret_cast<floatx4*>(&red[c & 1][wave][lane * 4]) = o + o2;
     // a barrier for LDS alone: __syncthreads would also wait for the loads that were asked for ahead. A buffer's sums are read
     // in the step after (below), before that step's barrier, and written again only behind it.
     asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
   };
 #pragma unroll
-  for (int i = 0; i < AHEAD; ++i) ask(ops[i], i);
+  for (int i = 0; i < AHEAD; ++i) ask(ops[i]);
   int c = 0;
   for (; c + AHEAD <= chunks; c += AHEAD) {
 #pragma unroll
@@ -427,7 +447,9 @@ __global__ __launch_bounds__(256, 2) void recurrence_chunks_kernel(const float* 
 #pragma unroll
   for (int i = 0; i < AHEAD - 1; ++i)
     if (c + i < chunks) step(ops[i], c + i);
-  emit(chunks - 1);
+  float share[4];
+  shares(chunks - 1, share);
+  emit(share, chunks - 1);
 #pragma unroll
   for (int i = 0; i < TPW; ++i)
 #pragma unroll
@@ -680,8 +702,9 @@ extern "C" int nhv_recurrence_chunks(const void* r_in, const void* k_in, const v
   const int Dp = (D + 15) / 16 * 16, tpw = (Dp / 16 + 3) / 4;
   const dim3 grid(H, (E + 15) / 16, B);
   hipStream_t s = (hipStream_t)stream;
+  const bool many = (long long)grid.x * grid.y * grid.z > 512;
 #define LAUNCH(TT, N, EVEN)                                                                                                  \
-  hipLaunchKernelGGL((recurrence_chunks_kernel<TT, N, EVEN>), grid, dim3(256), 0, s, (const float*)r_in, (const float*)k_in,    \
+  hipLaunchKernelGGL((N <= 2 && !many ? recurrence_chunks_kernel<TT, N, EVEN, N <= 2 ? 3 : 2> : recurrence_chunks_kernel<TT, N, EVEN, 2>), grid, dim3(256), 0, s, (const float*)r_in, (const float*)k_in,    \
                      (const float*)a_in, (const float*)decay_in, (const TT*)v, ld, (float*)state, (float*)out,            \
                      (const int*)positions, (const int*)cu, (const int*)state_slots, H, D, Dp, E)
   const bool even = Dp / 16 == 4 * tpw;

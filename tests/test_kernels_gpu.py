@@ -2163,3 +2163,35 @@ def test_rows_in_pieces_of_eight(ops, H):
         backend.scale_rows(x, squares, 1e-5, out)
         exact = x.double() / (squares.double().sum(-1, keepdim=True) / H + 1e-5).sqrt()
         assert bool(((out.double() - exact).abs() <= exact.abs() * (2.0 ** -8 + 2.0 ** -20)).all())
+
+
+@pytest.mark.parametrize("B, H, D, rank", [(200, 1, 40, 7), (70, 2, 64, 64), (70, 1, 128, 100), (40, 3, 80, 129), (60, 1, 160, 16), (40, 1, 256, 65)])
+def test_recurrences_of_many_requests_at_once(ops, B, H, D, rank):
+    """More chains than two a compute unit, of one to four chunks, which are asked for otherwise than few chains are: the bits that each
+    request gives alone, and zeros from states of others nowhere."""
+    g = torch.Generator(device="cuda").manual_seed(D)
+    rand = lambda *shape: torch.randn(*shape, generator=g, device="cuda")
+    lens = [1 + (17 * i) % 50 for i in range(B)]
+    cu = [0]
+    for n in lens:
+        cu.append(cu[-1] + n)
+    T, n = cu[-1], H * D
+    r, k, v, gate = (rand(T, n).to(torch.bfloat16) for _ in range(4))
+    z, w2, w0, u = 2.0 * rand(T, rank), (rand(n, rank) * rank ** -0.5).to(torch.bfloat16), rand(n) - 1.0, rand(H, D)
+    start = rand(B, H, D, D)
+    ints = lambda values: torch.tensor(values, dtype=torch.int32, device="cuda")
+
+    def run(first, last):
+        at, end = cu[first], cu[last]
+        batch = ops.AttentionBatch(num_tokens=end - at, num_requests=last - first, token_req=ints([i - first for i in range(first, last) for _ in range(lens[i])]),
+                                   positions=ints([7 + j for i in range(first, last) for j in range(lens[i])]), cu_seqlens_q=ints([c - at for c in cu[first:last + 1]]),
+                                   context_lens=ints([7 + m for m in lens[first:last]]), max_q_len=50, max_context_len=57)
+        state = start.clone()
+        y = ops.linear_recurrence(ops.WKV(z[at:end], w2, w0, u), r[at:end], k[at:end], v[at:end], gate[at:end], state, 1e-5, batch, ints(list(range(first, last))), torch.bfloat16)
+        return y, state
+
+    y, state = run(0, B)
+    assert bool(torch.isfinite(y).all()) and bool(torch.isfinite(state).all())
+    for i in range(0, B, 7):
+        alone, left = run(i, i + 1)
+        assert torch.equal(y[cu[i]:cu[i + 1]], alone) and torch.equal(state[i], left[i])
