@@ -314,7 +314,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void p
   // prompts of 901, 90 and 500: 47.7 to 37.0 us (the prompts last: 56.2 to 40.0); one token after 1,700 alone 28.9 to 20.5; four after 40
   // to 700 beside 75 new ones 14.6 to 12.4.
   if constexpr (ONE_TILE) {
-    if (G * q_len <= 16) {                                 // the whole block
+    // (Up to 256 keys are four tiles, which are no chain to speak of: there a token's sums stay in the order of the prompt's.)
+    if (G * q_len <= 16 && ctx > 256) {                    // the whole block
       if (bx > 0) return;
       // (values of its own: what both paths work out from the lane would be kept in registers that the other path needs)
       int my_lane = threadIdx.x & 63;
