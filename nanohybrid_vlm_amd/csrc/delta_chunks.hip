@@ -63,9 +63,12 @@ __device__ __forceinline__ float silu_of(float z) {
 // rate log2(1 + e^z), rate log2(e) in two pieces: max(z, 0) log2(e) and log2(w), w = 1 + e^-|z|, of which w's own rounding c is the part c / w.
 // Off by 2.5e-8 (z > 1) to 5.1e-8 (z down to -12; below, where nothing decays, 7e-8) on average; -log2(e) rate log1p(e^z) by the
 // library's functions 4.6e-8 to 5.3e-8, and 190 instructions with its addresses where this is 40.
+// Where the first part alone is beyond what counts (512; the logarithm ends at -256) it is the result: of an infinite or huge z the second, whose sign is
+// that of log2(e) rate's rounding, would be as infinite, against it.
 __device__ __forceinline__ float softplus_bits(float z, float rate, float bits, float rest) {
-  const float a = fabsf(z), u = exp_of(a > 110.f ? -110.f : -a), w = 1.0f + u, c = u - (w - 1.0f), m = fmaxf(z, 0.f);
-  return fmaf(bits, m, fmaf(rest, m, fmaf(rate, __builtin_amdgcn_logf(w), c * __builtin_amdgcn_rcpf(w) * bits)));
+  const float a = fabsf(z), u = exp_of(a > 110.f ? -110.f : -a), w = 1.0f + u, c = u - (w - 1.0f), m = fmaxf(z, 0.f), first = bits * m;
+  const float sum = fmaf(bits, m, fmaf(rest, m, fmaf(rate, __builtin_amdgcn_logf(w), c * __builtin_amdgcn_rcpf(w) * bits)));
+  return first > 512.f ? first : sum;
 }
 #define NHV_LOWEST_LOG (-256.f)
 

@@ -1955,6 +1955,37 @@ def test_delta_rule_after_strong_decays(ops, D, rate, strong, per_head):
 
 @pytest.mark.usefixtures("sixteen_at_a_time")
 @pytest.mark.parametrize("per_head", [False, True])
+@pytest.mark.parametrize("strong", [float("inf"), 3e38, 1e30, 700.0])
+def test_delta_rule_after_decays_beyond_any_number_at_many_rates(ops, strong, per_head):
+    """Infinite and huge decays at rates whose product with log2(e) is rounded up and down, a head each: what lies before them
+    is gone, what comes after is there, within sixteen roundings of 2^-24 of the largest entry."""
+    import plain_pevazen as plain
+    g = torch.Generator().manual_seed(83)
+    a_log = torch.cat((torch.linspace(-6.0, 4.0, 51), torch.tensor([20.0, 40.0, 60.0, 80.0])))
+    H, G, D, E, n, taps = len(a_log), 1, 16, 16, 37, 4
+    C, Dd = 2 * G * D + H * E, 1 if per_head else D
+    proj, gates = torch.randn(n, C + H, generator=g), torch.randn(n, H * E, generator=g)
+    a_lin = torch.randn(n, H, Dd, generator=g) - (a_log.clamp(min=0.0) + 1.0)[:, None]
+    a_lin[[2, 3, 20, 33]] = strong
+    tap, dt_bias = 0.6 * torch.randn(C, taps, generator=g), 0.1 * torch.randn(H * Dd, generator=g)
+    y, state = _delta_rule_once(ops, proj, a_lin.view(n, H * Dd), gates, tap, dt_bias, a_log, torch.ones(E), H, G, D, E, per_head)
+    act = plain.silu(plain.causal_taps(proj[:, :C].double(), tap.double()))
+    k = act[:, G * D:2 * G * D]
+    k = k / torch.sqrt(k.pow(2).sum(-1, keepdim=True) + 1e-6)
+    v, beta = act[:, 2 * G * D:].view(n, H, E), torch.sigmoid(proj[:, C:].double())
+    z = (a_lin + dt_bias.view(H, Dd)).double()
+    decay = torch.exp(-a_log.double().exp()[:, None] * torch.logaddexp(z, torch.zeros_like(z)))
+    S = torch.zeros(H, D, E, dtype=torch.float64)
+    for t in range(n):
+        S = decay[t][..., None] * S
+        S = S + k[t][:, None] * (beta[t][:, None] * (v[t] - torch.einsum("hde,d->he", S, k[t])))[:, None]
+    assert torch.isfinite(y).all() and torch.isfinite(state).all(), a_log[~torch.isfinite(state).flatten(1).all(1)]
+    off = (state.transpose(1, 2).double() - S).abs().amax((1, 2)) / S.abs().amax((1, 2))
+    assert off.max() < 1e-6, (off.max(), a_log[off.argmax()])
+
+
+@pytest.mark.usefixtures("sixteen_at_a_time")
+@pytest.mark.parametrize("per_head", [False, True])
 @pytest.mark.parametrize("D,E", [(64, 32), (20, 5), (112, 128)])
 def test_delta_rule_lets_no_token_reach_the_ones_before_it(ops, D, E, per_head):
     """A value, a key or a decay that is infinite or no number: the tokens before it, also those of the same sixteen, and the
