@@ -36,10 +36,12 @@ constexpr int TILE = 256, PIECE = 64;                    // rows of x and of w a
 constexpr int UNIT = 128 * PIECE * 2, LDS = 8 * UNIT;    // bytes of 128 rows of a piece; two pieces of both operands
 
 // 16 bytes a lane to LDS at `to` + 16 lane, from `lane_at` + `at` bytes behind the start of `rows`. What lies behind the end of `rows` is
-// not read, also where `at` alone lies behind it (zeros come to LDS: looked at with descriptors of 512 bytes and `at` up to 256 KB). (Written as an
-// instruction, see nhv_lines.h.)
+// not read, also where `at` alone lies behind it: a lane's offset is compared with what the scalar offset leaves of the size, so that
+// one is cut off at the size, which leaves nothing. (Written as an instruction, see nhv_lines.h; the one between gives m0 its wait.)
 __device__ __forceinline__ void load_to_lds(uint32_t to, uint32_t lane_at, i32x4 rows, uint32_t at) {
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds" ::"s"(to), "v"(lane_at), "s"(rows), "s"(at) : "memory", "m0");
+  uint32_t cut;
+  asm volatile("s_mov_b32 m0, %1\n\ts_min_u32 %0, %4, %5\n\tbuffer_load_dwordx4 %2, %3, %0 offen lds"
+               : "=&s"(cut) : "s"(to), "v"(lane_at), "s"(rows), "s"(at), "s"(rows[2]) : "memory", "m0", "scc");
 }
 __device__ __forceinline__ i32x4 rows_from(const bf16_t* first, long long bytes) {
   const uint64_t at = (uint64_t)first;

@@ -91,6 +91,37 @@ def test_the_wait_for_x_has_the_loads_behind_it_that_it_counts(tmp_path):
     assert seen >= 50, seen
 
 
+def test_no_scalar_offset_of_the_gates_kernel_lies_behind_its_rows(tmp_path):
+    """Of a tile that is cut off at the end, the rows behind it are kept out by the descriptor's size, with which the lane's offset is
+    compared after the scalar offset has been taken from it: that one must not be the larger. In what the compiler makes of each kernel
+    every load to LDS has a scalar offset that has just been cut off at the size in its own descriptor."""
+    source, out = os.path.join(library.CSRC, "gemm_phases_bf16.hip"), tmp_path / "phases.s"
+    subprocess.run([library._hipcc(), *[f for f in library.HIPCC_FLAGS if f != "-fPIC"], "-I", library.CSRC, "--cuda-device-only", "-S",
+                    source, "-o", str(out)], check=True, capture_output=True)
+    kernels = re.findall(r"^(\S*gemm_phases_kernel\S*):[^\n]*\n(.*?)^\.Lfunc_end", out.read_text(), re.M | re.S)
+    assert len(kernels) == 6
+    for name, body in kernels:
+        ops = [op for op in (" ".join(line.split(";")[0].split()) for line in body.split("\n")) if op]
+        copies, loads = {}, 0
+        for i, op in enumerate(ops):
+            if re.match(r"\S+:$", op):                    # (where ways meet, only what is true on both would count)
+                copies = {}
+            if move := re.match(r"s_mov_b32 (s\d+), (s\d+)$", op):
+                copies[move[1]] = copies.get(move[2], move[2])
+            elif written := re.match(r"s_\S+ s(\d+|\[\d+:\d+\]),", op):
+                first, last = (re.findall(r"\d+", written[1]) * 2)[:2] if "[" not in written[1] else re.findall(r"\d+", written[1])
+                for n in range(int(first), int(last) + 1):
+                    copies = {k: v for k, v in copies.items() if f"s{n}" not in (k, v)}
+            if op.startswith("buffer_load") and op.endswith("lds"):
+                rows, offset = re.match(r"buffer_load_dwordx4 v\d+, s\[(\d+):\d+\], (s\d+) offen lds$", op).groups()
+                cut = re.match(r"s_min_u32 (s\d+), (s\d+), (s\d+)$", ops[i - 1])
+                assert cut and cut[1] == offset, (name, ops[i - 3:i + 1])
+                size = f"s{int(rows) + 2}"
+                assert size in (cut[3], copies.get(cut[3])) or copies.get(size, size) == copies.get(cut[3], cut[3]), (name, ops[i - 3:i + 1])
+                loads += 1
+        assert loads >= 32, (name, loads)
+
+
 @pytest.mark.parametrize("blocks", [1, 8, 64, 184, 192, 200, 256, 264, 320, 352, 360, 416, 424, 512, 1024, 4096])
 def test_no_block_of_the_decode_attention_takes_a_long_context_alone(blocks):
     """However long the longest context and however many blocks there are: the splits cover it, and no block's chain of keys is longer
