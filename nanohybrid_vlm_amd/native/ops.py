@@ -788,7 +788,8 @@ class NativeBackend:
     # -- the table of choices, so that a process can run by what another one measured --
     def choices_table(self, chosen: dict | None = None) -> dict[str, int]:
         """A table of choices (default: the one in force), by shape: "M,N,K,float result,gated" -> -1 (own kernel),
-        -2 (the rule: ``torch.mm``) or the number of a library algorithm. gated 2: a product that its reader takes as parts."""
+        -2 (the rule: ``torch.mm``) or the number of a library algorithm. gated 1: the product with its gate (many rows: or its
+        activation) in one kernel; 2: a product that its reader takes as parts."""
         chosen = self.chosen if chosen is None else chosen
         return {",".join(str(int(v)) for v in key): how for key, how in sorted(chosen.items())}
 
@@ -881,11 +882,21 @@ class NativeBackend:
 
     def _by_phases(self, x, w, out, bias, gated: bool, gate: "Gate") -> bool:
         """A gated or activated product of many rows in one kernel, where that is the faster way (gemm_phases_bf16.hip; it hangs on the
-        shape alone); else False."""
+        shape, not on what was measured for others before), else False. An engine's own table, read from a file, may say otherwise: where it names
+        another way than the own kernel for the gated product or, if it lacks that, for the shape's rows."""
         (M, K), N = x.shape, out.shape[1]
         if not (self.few_rows < M and x.dtype == out.dtype == torch.bfloat16 and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0
                 and (bias is None or bias.data_ptr() % 8 == 0) and self.lib.nhv_gemm_phases_pays(M, N, K, int(gated))):
             return False
+        if not self.own_kernels_only:
+            key = (M, w.shape[0], K, False, True)
+            how = self.chosen.get(key)
+            if how is None and not (self.measuring_allowed and self.chosen is self.shared_chosen):
+                how = self.chosen.get((M, w.shape[0], K, False, False))
+            if how is not None and how != OWN:
+                return False
+            if self.measuring_allowed:
+                self.chosen[key] = OWN                       # (a process that reads this table does it the same way)
         self._call("nhv_gemm_phases_bf16", _ptr(x), _ptr(w), _ptr(bias), _ptr(out), M, N, K, int(gated), *gate.args(), _stream())
         return True
 

@@ -1641,6 +1641,46 @@ def test_what_goes_by_lines_hangs_on_the_shape_and_on_a_table_that_is_read(ops):
         backend.chosen, backend.measuring_allowed = chosen, allowed
 
 
+@pytest.mark.parametrize("how", [-2, 0])
+def test_many_rows_are_gated_the_way_that_a_table_which_is_read_names(ops, how):
+    """A gated and an activated product of many rows: a table from a file that names torch.mm or a library algorithm for the shape is followed,
+    whether or not other shapes may be timed, unless it says that the own kernel joined the gate; what was measured for the same shape's
+    plain products in this process changes nothing, also where an engine's own table comes to hold it."""
+    backend = ops.backend()
+    M, N, K = 1300, 8192, 512
+    x, w = rnd(M, K, dtype=torch.bfloat16, seed=134), rnd(2 * N, K, dtype=torch.bfloat16, seed=135, scale=K ** -0.5)
+    out = torch.empty(M, N, dtype=torch.bfloat16, device="cuda")
+
+    def ways():
+        done = backend.gated_linear(x, w, out), backend.activated_linear(x, w[:N], out, 1)
+        assert torch.equal(ops.gated_linear(x, w), ops.act_mul(ops.linear(x, w), "silu")) is not done[0]
+        return done
+
+    saved, allowed, chosen, many = dict(backend.shared_chosen), backend.measuring_allowed, backend.chosen, backend.measure_many_rows
+    try:
+        backend.measure_many_rows = False
+        backend.shared_chosen.clear()
+        backend.use_choices(None, True)
+        assert ways() == (True, True)
+        written = backend.choices_table()
+        assert written == {f"{M},{N},{K},0,1": -1, f"{M},{2 * N},{K},0,1": -1}
+        apart = {f"{M},{N},{K},0,0": how, f"{M},{2 * N},{K},0,0": how}
+        backend.shared_chosen.update(backend.parse_choices(apart))             # (as if measured for plain products)
+        assert ways() == (True, True)
+        for measuring in (False, True):
+            for table, want in (({}, True), (apart, False), ({**apart, **written}, True)):
+                backend.use_choices(backend.parse_choices(table), measuring)
+                assert ways() == (want, want) and backend.choices_table() == ({**written, **table} if measuring and want else table)
+        backend.use_choices({}, True)
+        assert ways() == (True, True)
+        backend.chosen.update(backend.parse_choices(apart))
+        assert ways() == (True, True)
+    finally:
+        backend.shared_chosen.clear()
+        backend.shared_chosen.update(saved)
+        backend.chosen, backend.measuring_allowed, backend.measure_many_rows = chosen, allowed, many
+
+
 @pytest.mark.parametrize("M,N,K", [(3, 4096, 2048), (16, 4100, 2304), (17, 2048, 1024), (40, 3000, 1280), (90, 4096, 2048)])
 def test_products_by_lines_keep_rows_and_columns_apart(ops, M, N, K):
     """Rows of x and of w that are infinite or no numbers: their own rows and columns are what float64 says of them, all others the same bits as
