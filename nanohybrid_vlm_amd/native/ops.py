@@ -886,7 +886,7 @@ class NativeBackend:
         another way than the own kernel for the gated product or, if it lacks that, for the shape's rows."""
         (M, K), N = x.shape, out.shape[1]
         if not (self.few_rows < M and x.dtype == out.dtype == torch.bfloat16 and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0
-                and (bias is None or bias.data_ptr() % 8 == 0) and self.lib.nhv_gemm_phases_pays(M, N, K, int(gated))):
+                and out.data_ptr() % 8 == 0 and (bias is None or bias.data_ptr() % 8 == 0) and self.lib.nhv_gemm_phases_pays(M, N, K, int(gated))):
             return False
         if not self.own_kernels_only:
             key = (M, w.shape[0], K, False, True)

@@ -1641,6 +1641,20 @@ def test_what_goes_by_lines_hangs_on_the_shape_and_on_a_table_that_is_read(ops):
         backend.chosen, backend.measuring_allowed = chosen, allowed
 
 
+def test_results_off_their_boundaries_are_not_the_kernel_of_many_rows_ones(ops):
+    """Rows of results that do not begin on 8 bytes: left to the product and the kernel behind it, untouched."""
+    backend = ops.backend()
+    M, N, K = 1300, 8192, 512
+    x, w = rnd(M, K, dtype=torch.bfloat16, seed=134), rnd(2 * N, K, dtype=torch.bfloat16, seed=135, scale=K ** -0.5)
+    room = torch.full((M * N + 8,), 7.0, dtype=torch.bfloat16, device="cuda")
+    for off in (1, 2, 3, 4):
+        out, taken = room[off:off + M * N].view(M, N), off == 4
+        assert backend.gated_linear(x, w, out) is taken and (taken or bool((room == 7.0).all()))
+    assert torch.equal(room[4:4 + M * N].view(M, N), ops.gated_linear(x, w)) and bool((room[:4] == 7.0).all())
+    room.fill_(7.0)
+    assert not backend.activated_linear(x, w[:N], room[1:1 + M * N].view(M, N), 1) and bool((room == 7.0).all())
+
+
 @pytest.mark.parametrize("how", [-2, 0])
 def test_many_rows_are_gated_the_way_that_a_table_which_is_read_names(ops, how):
     """A gated and an activated product of many rows: a table from a file that names torch.mm or a library algorithm for the shape is followed,
