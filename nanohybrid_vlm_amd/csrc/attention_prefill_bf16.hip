@@ -256,7 +256,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void p
     bf16_t* __restrict__ out, const int* __restrict__ cu_seqlens_q, const int* __restrict__ context_lens,
     const int* __restrict__ block_tables, int max_blocks, int Hq, int Hkv, int page_size, int page_shift,
     float scale_log2e, int window, float cap_ratio, float tanh_k, float sink_l2, const float* __restrict__ sinks,
-    const float* __restrict__ slopes, float slope_ratio, const bf16_t* __restrict__ gate, long long gate_ld) {
+    const float* __restrict__ slopes, float slope_ratio, const bf16_t* __restrict__ gate, long long gate_ld, int one_tile_from) {
   static_assert((MORE || !(BIASED || CAPPED)) && !(BIASED && CAPPED), "cap and bias are further options, one of them at most");
   constexpr float LOG2E = 1.4426950408889634f;
   constexpr int DL = SUPPORTED ? D : 16;                   // keeps the unsupported sizes compilable; they are never launched
@@ -311,11 +311,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void p
   // and the four waves share its keys, 32 at a time in turn, each with its next 32 on their way: keys as operands in registers, values in a
   // part of LDS of its own, no barrier. The waves' sums meet at the end. Otherwise every head's few rows are a tile, all keys pass every
   // wave one tile after the other, 1 us each, and the block is the last to end. 13 tokens after 60 to 1,700 keys beside
-  // prompts of 901, 90 and 500: 47.7 to 37.0 us (the prompts last: 56.2 to 40.0); one token after 1,700 alone 28.9 to 20.5; four after 40
-  // to 700 beside 75 new ones 14.6 to 12.4.
+  // prompts of 901, 90 and 500: 51.6 to 39.1 us (the prompts last: 42.5 to 36.1); 4 tokens after 1,700 beside 20 to 200 new ones 29 to 22.5; 1 after
+  // 14,000 200 to 126, after 30,000 541 to 372 (one block's chain still); four after 40 to 700 beside 75 14.4 to 12.3.
   if constexpr (ONE_TILE) {
-    // (Up to 256 keys are four tiles, which are no chain to speak of: there a token's sums stay in the order of the prompt's.)
-    if (G * q_len <= 16 && ctx > 256) {                    // the whole block
+    if (G * q_len <= 16 && ctx > one_tile_from) {          // the whole block
       if (bx > 0) return;
       // (values of its own: what both paths work out from the lane would be kept in registers that the other path needs)
       int my_lane = threadIdx.x & 63;
@@ -574,6 +573,40 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void p
 
 }  // namespace prefill
 
+// Two row tiles a wave where that still leaves two blocks for every compute unit (1,024 new tokens of 8 kv heads
+// are 256 such blocks: 41 us, and 31 us as 512 blocks of one row tile a wave; after 7,000 keys 259 and 216 us).
+static bool two_row_tiles(int B, int max_q_len, int G, int Hkv) {
+  return prefill::MAX_RT >= 2 && ((long long)G * ((max_q_len + 15) / 16) + 7) / 8 * Hkv * B >= 512;
+}
+static long long groups_of_tiles(int max_q_len, int G, bool two) {
+  const int tpb = two ? 8 : 4;
+  return ((long long)G * ((max_q_len + 15) / 16) + tpb - 1) / tpb;
+}
+
+// Beyond how many keys a request whose rows are one tile shares its keys out among the waves, where that is the faster way. Where two of
+// its blocks come to one unit it is not: loads of keys as operands touch sixteen rows at a time, of which a unit takes in less a ns (13 tokens after 1,700 keys of 32 on 8 heads
+// beside 50 new ones, 104 blocks on 64 units: 45 us, 53 so; with a unit each 39 and 32). Which units the blocks come to hangs on the empty ones between
+// them, gx to a request's. So: where the other way takes several blocks of all keys (G of 8 and more), or has two row tiles a wave and two waves
+// without any (53 and 53 where blocks meet, else 0.5 to 0.9), or where few blocks are spread over many units, heads of their own few blocks apart (G of 1: 5 tokens after 1,700 beside 500,
+// gx 8, 28.6 and 36.0). Measured over 2,500 sizes (1 to 200 tokens of heads of 64 and 128, groups of 1 to 16, after 17 to 30,000 keys beside 20 to 1,000 new ones): time over the other way's
+// 0.84 on average, the worst 1.03; taken everywhere 0.84, 1.26.
+// Up to 448 keys groups of less than 4 gain nothing (1 to 25 tokens after 280 to 400: 0.96 to 1.1), and up to 256 larger ones at most 0.7 us (1 token after
+// 128: 6.3 and 6.4; 256: 7.6 and 7.2; groups of 8 of 64 6.1 and 5.4): there a token's sums keep the portions' order, so that a short
+// request's results hang less on how it is cut up (logits of sharpened scores 0.0190 apart, with the waves' sums 0.0204). Neither is further from 64
+// bits: 0.0016 to 0.0024 of the results' size after 64 to 2,000 keys, the waves' sums up to a fifth closer at the fewest, the same at the most.
+static int one_tile_from_keys(int B, int G, int Hkv, bool two, long long gx) {
+  if (!(G >= 8 || (two && G >= 4) || ((long long)B * Hkv <= 64 && (G >= 4 || gx <= 4)))) return 0x7fffffff;
+  return G >= 4 ? 256 : 448;
+}
+
+// The same for a launch's sizes (0x7fffffff: no request does).
+extern "C" int nhv_prefill_attention_one_tile_from(int B, int max_q_len, int Hq, int Hkv) {
+  if (!prefill::ONE_TILE || B <= 0 || max_q_len <= 0 || Hkv <= 0 || Hq % Hkv) return 0x7fffffff;
+  const int G = Hq / Hkv;
+  const bool two = two_row_tiles(B, max_q_len, G, Hkv);
+  return one_tile_from_keys(B, G, Hkv, two, groups_of_tiles(max_q_len, G, two));
+}
+
 static int launch_prefill_attention(const void* q, const void* k_cache, const void* v_cache, void* out,
                                     const void* cu_seqlens_q, const void* context_lens, const void* block_tables,
                                     int max_blocks, int B, int max_q_len, int Hq, int Hkv, int page_size, float scale,
@@ -586,12 +619,9 @@ static int launch_prefill_attention(const void* q, const void* k_cache, const vo
   for (int b = 0; b < 31; ++b)
     if (page_size == (1 << b)) page_shift = b;
   const int G = Hq / Hkv;
-  const long long row_tiles = (long long)G * ((max_q_len + 15) / 16);
-  // two row tiles a wave where that still leaves two blocks for every compute unit (1,024 new tokens of 8 kv heads
-  // are 256 such blocks: 41 us, and 31 us as 512 blocks of one row tile a wave; after 7,000 keys 259 and 216 us)
-  const bool two = prefill::MAX_RT >= 2 && (row_tiles + 7) / 8 * Hkv * B >= 512;
-  const int tpb = two ? 8 : 4;
-  const long long gx = (row_tiles + tpb - 1) / tpb;
+  const bool two = two_row_tiles(B, max_q_len, G, Hkv);
+  const long long gx = groups_of_tiles(max_q_len, G, two);
+  const int one_tile_from = prefill::ONE_TILE ? one_tile_from_keys(B, G, Hkv, two, gx) : 0x7fffffff;
   NHV_REQUIRE(gx <= 0x7fffffff && Hkv <= 65535 && B <= 65535, "prefill attention: grid too large");
   const float log2e = 1.4426950408889634f;
   const bool capped = more && cap > 0.f;
@@ -601,7 +631,7 @@ static int launch_prefill_attention(const void* q, const void* k_cache, const vo
                      (const int*)cu_seqlens_q, (const int*)context_lens, (const int*)block_tables, max_blocks, Hq, Hkv, \
                      page_size, page_shift, scale * log2e, window, capped ? cap / scale : 0.f,                         \
                      capped ? 2.0f * log2e * scale / cap : 0.f, more && has_sink ? sink * log2e : -INFINITY,           \
-                     (const float*)sinks, (const float*)slopes, 1.0f / scale, (const bf16_t*)gate, gate_ld)
+                     (const float*)sinks, (const float*)slopes, 1.0f / scale, (const bf16_t*)gate, gate_ld, one_tile_from)
 #define NHV_PREFILL_LAUNCH(BT, RT_)                                      \
   do {                                                                   \
     if (slopes) NHV_PREFILL_LAUNCH_AS(BT, RT_, true, false, true);       \

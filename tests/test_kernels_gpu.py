@@ -1224,17 +1224,45 @@ def test_prefill_attention_bfloat16(ops, Hq, Hkv, D, page, window):
     torch.testing.assert_close(out.double().cpu(), ref, **tol(torch.bfloat16))
 
 
-@pytest.mark.parametrize("Hq,Hkv,D,page,reach,cap,sinks,slopes,gated", [
-    (32, 8, 128, 16, None, None, None, False, False), (8, 2, 128, 256, ("window", 70), None, "each", False, True),
-    (16, 1, 128, 64, ("chunk", 50), 3.0, "one", False, False), (5, 5, 48, 7, None, None, None, True, True),
-    (6, 2, 80, 32, ("window", 1), None, "each", True, False), (3, 1, 16, 8, None, 2.0, None, False, True),
-    (4, 4, 64, 48, ("chunk", 33), None, "each", True, False), (7, 1, 112, 128, ("window", 333), None, None, False, False),
+@pytest.mark.parametrize("B,new,Hq,Hkv,keys", [
+    # few blocks, larger groups; many, with two row tiles a wave; groups that the other way gives several blocks
+    (5, 75, 32, 8, 256), (8, 1000, 32, 8, 256), (16, 901, 32, 8, 256), (61, 100, 32, 8, 256), (61, 20, 32, 2, 256), (200, 20, 64, 4, 256),
+    # many blocks of one row tile a wave, or two of which one is without any; few of groups of one beside longer portions
+    (14, 50, 32, 8, None), (14, 100, 32, 8, None), (31, 33, 32, 8, None), (14, 75, 40, 8, None), (46, 20, 16, 8, None), (14, 500, 16, 8, None),
+    (6, 500, 8, 8, None), (6, 20, 8, 8, 448), (8, 64, 16, 8, 448), (9, 64, 16, 8, None),
 ])
-def test_prefill_attention_of_one_tile_beside_prompts(ops, Hq, Hkv, D, page, reach, cap, sinks, slopes, gated):
-    """Requests whose rows are one tile, whose keys four waves share, beside a longer portion: one to four tokens, from one key
-    over the edges of a wave's 32 and the four waves' 128 on, every option, and an infinite value that only its readers see."""
-    lens = [1, 31, 32, 33, 64, 127, 128, 129, 257, 300, 1700, 385, 200]
-    q_lens = [1, 1, 2, 1, 3, 1, 1, 4, 1, 2, 1, 16, 60]
+def test_which_short_requests_share_their_keys_out(ops, B, new, Hq, Hkv, keys):
+    """Where that was measured to be the faster way for a request of a few tokens beside portions (else another 4 to 26 % slower)."""
+    for D, most in ((128, keys), (64, keys), (256, None)):
+        assert ops.backend().attention_lib(D).nhv_prefill_attention_one_tile_from(B, new, Hq, Hkv) == (most or 2 ** 31 - 1)
+
+
+@pytest.mark.parametrize("Hq,Hkv,D,page,portion,two,reach,cap,sinks,slopes,gated", [
+    (32, 8, 128, 16, 900, True, None, None, None, False, False), (8, 2, 128, 256, 60, False, ("window", 70), None, "each", False, True),
+    (16, 1, 128, 64, 60, False, ("chunk", 50), 3.0, "one", False, False), (5, 5, 48, 7, 60, False, None, None, None, True, True),
+    (6, 2, 80, 32, 60, False, ("window", 1), None, "each", True, False), (3, 1, 16, 8, 60, False, None, 2.0, None, False, True),
+    (4, 4, 64, 48, 60, False, ("chunk", 33), None, "each", True, False), (7, 1, 112, 128, 60, False, ("window", 333), None, None, False, False),
+    # tables of more than 1,024 entries: of single tokens, of pages; and with two row tiles a wave, plain, capped and biased
+    (8, 2, 64, 1, 60, False, None, None, None, False, False), (8, 1, 64, 32, 60, False, None, None, "one", False, True),
+    (16, 4, 64, 1, 700, True, ("window", 600), None, None, True, False), (32, 4, 128, 32, 700, True, ("window", 500), 5.0, "each", False, True),
+    (12, 3, 96, 1, 900, True, None, None, None, False, False),
+])
+def test_prefill_attention_of_one_tile_beside_prompts(ops, Hq, Hkv, D, page, portion, two, reach, cap, sinks, slopes, gated):
+    """Requests whose rows are one tile, whose keys four waves share, beside a longer portion: one to four tokens, from the last length that goes
+    the portions' way over the edges of a wave's 32 and the four waves' 128 on, every option, one and two row tiles a wave, tables in LDS and in
+    memory, and an infinite value that only its readers see."""
+    G = Hq // Hkv
+    start = 256 if G >= 4 else 448
+    some = min(4, 16 // G)
+    lens = [31, start, start + 1, start + 31, start + 32, start + 33, start + 127, start + 128, start + 129, start + 300, 1700, start + 129, portion + 140]
+    q_lens = [1, 1, 1, 1, some, 1, some, 1, 1, min(2, some), 1, 16 // G, portion]
+    if G == 1:
+        lens, q_lens = lens[1:], q_lens[1:]
+    if page == 32 and G >= 8:                                # (a table of 1,026 pages)
+        lens[2] = 32 * 1024 + 40
+    assert (G * -(-portion // 16) + 7) // 8 * Hkv * len(lens) >= 512 if two else (G * -(-portion // 16) + 7) // 8 * Hkv * len(lens) < 512
+    assert ops.backend().attention_lib(D).nhv_prefill_attention_one_tile_from(len(lens), portion, Hq, Hkv) == start
+    at_1700 = lens.index(1700)
     q, kc, vc, batch, bt, ks, vs, qs = _paged_setup(torch.bfloat16, lens, q_lens, Hq, Hkv, D, page, seed=97, scale=1.5)
     g = torch.Generator().manual_seed(98)
     rows = torch.randn(q.shape[0], Hq + 3, generator=g).to(torch.bfloat16)
@@ -1259,14 +1287,33 @@ def test_prefill_attention_of_one_tile_beside_prompts(ops, Hq, Hkv, D, page, rea
         want.append(o * torch.sigmoid(rows[at:at + nq, 2:2 + Hq].double())[..., None] if gated else o)
         at += nq
     torch.testing.assert_close(out.double().cpu(), torch.cat(want), **tol(torch.bfloat16))
-    vc[bt[10, 1690 // page], 1690 % page, Hkv - 1, D - 1] = float("inf")
+    vc[bt[at_1700, 1690 // page], 1690 % page, Hkv - 1, D - 1] = float("inf")
     spoilt = ops.paged_attention(q, kc, vc, batch, bt, D ** -0.5, **options)
-    row = sum(q_lens[:10])
+    row = sum(q_lens[:at_1700])
     reads = not reach or (1690 > 1699 - reach[1] if reach[0] == "window" else 1690 // reach[1] == 1699 // reach[1])
     assert bool(torch.isfinite(spoilt[row, Hq - 1, D - 1])) is not reads
     hit = torch.zeros_like(out, dtype=torch.bool)
     hit[row, Hq - Hq // Hkv:, D - 1] = reads
     assert torch.equal(spoilt[~hit], out[~hit])
+
+
+@pytest.mark.parametrize("scale", [1.0, 3.0])
+@pytest.mark.parametrize("n", [257, 300, 1000, 2000])
+def test_a_token_is_as_exact_alone_beside_a_portion_as_inside_one(ops, n, scale):
+    """Requests' last tokens where four waves share the keys and at the end of portions, against float64 and each other: rounding the weights and the
+    result to 8 bits is 2^-9 of the result each at most, either way."""
+    Hq, Hkv, D = 32, 4, 128
+    assert ops.backend().attention_lib(D).nhv_prefill_attention_one_tile_from(7, 60, Hq, Hkv) < n
+    q, kc, vc, batch, bt, ks, vs, qs = _paged_setup(torch.bfloat16, [n] * 6 + [60], [40] * 6 + [60], Hq, Hkv, D, 64, seed=n, scale=scale)
+    inside = ops.paged_attention(q, kc, vc, batch, bt, D ** -0.5).double().cpu()
+    last = [40 * i + 39 for i in range(6)]
+    alone, _, _, batch, *_ = _paged_setup(torch.bfloat16, [n] * 6 + [60], [1] * 6 + [60], Hq, Hkv, D, 64, seed=n, scale=scale)
+    alone[:6], alone[6:] = q[last], q[240:]
+    alone = ops.paged_attention(alone, kc, vc, batch, bt, D ** -0.5).double().cpu()[:6]
+    want = _attention_reference([x[-1:] for x in qs[:6]], ks[:6], vs[:6], [n] * 6, [1] * 6, D ** -0.5, None)
+    off = lambda x, y: float((x - y).norm() / want.norm())
+    assert off(alone, want) < 2.0 ** -8 and off(inside[last], want) < 2.0 ** -8
+    assert off(alone, want) < 1.1 * off(inside[last], want) and off(alone, inside[last]) < 2.0 ** -7
 
 
 @pytest.mark.parametrize("far", [3, 650, 1290])
