@@ -67,7 +67,10 @@ constexpr bool CH_POW2 = (CH & (CH - 1)) == 0;
 constexpr int KSWZ = CH_POW2 ? (CH < 16 ? CH : 16) - 1 : 0;
 // and at c ^ ((k & VSWZ) << 1) in the V tile, whose transposed reads take 32 bytes of 8 keys at once
 constexpr int VSWZ = CH_POW2 && CH >= 4 ? (CH / 2 < 8 ? CH / 2 : 8) - 1 : 0;
-constexpr bool ONE_TILE = D <= 128;         // requests whose rows are one tile get a path of their own (its tiles fit into that LDS)
+// Requests whose rows are one tile get a path of their own (its tiles fit into that LDS). Not of heads of 80 and 96: of them three blocks share a unit, with 168
+// registers a wave, of which that path takes 200 (20 portions of 100 tokens, 16 on 4 heads of 80, 9.9 us, with two blocks 11.7; 2,000 tokens after 4,000, 24 on 8 of 96,
+// 143 and 174; with what is beyond 168 in memory the compiler also moves the portions' own).
+constexpr bool ONE_TILE = D <= 64 || (D >= 112 && D <= 128);
 constexpr int MAX_RT = D <= 128 ? 2 : 1;    // row tiles per wave (template argument RT): all of them use every key and value
                                             // that the wave reads from LDS; two need the registers of head sizes up to 128
 
@@ -250,8 +253,14 @@ __device__ __forceinline__ void attend(Rows<RT>& w, int kb, KeyOperand key_opera
 // multiplied by the scale as every score is, costs one exp2 and one reciprocal: tanh(x) = 1 - 2 / (1 + exp(2 x)), and an
 // exp2 that overflows gives the limit 1; sink_l2 = sink log2(e), or -inf for none (sinks, may be null: one per head in
 // its place); gate (may be null). BIASED: slopes per head, slope_ratio = 1 / scale.
+//
+// Blocks a compute unit, four waves each, that the compiler is to leave registers for: as many as the tiles in LDS leave room for, where the portions' way
+// has no use for more (heads of 64, one row tile a wave: 125 of 128; left at two blocks it takes 130 to 140, for the one-tile path).
+template <int RT, bool PLAIN>
+constexpr int blocks_a_unit() { return RT == 1 && D <= 64 && PLAIN ? 4 : D <= 48 && PLAIN ? 3 : 2; }
+
 template <bool BT_IN_LDS, int RT, bool MORE, bool CAPPED, bool BIASED>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void prefill_attention_kernel(
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(blocks_a_unit<RT, !CAPPED && !BIASED>()))) void prefill_attention_kernel(
     const bf16_t* __restrict__ q, const bf16_t* __restrict__ k_cache, const bf16_t* __restrict__ v_cache,
     bf16_t* __restrict__ out, const int* __restrict__ cu_seqlens_q, const int* __restrict__ context_lens,
     const int* __restrict__ block_tables, int max_blocks, int Hq, int Hkv, int page_size, int page_shift,

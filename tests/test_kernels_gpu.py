@@ -1233,19 +1233,19 @@ def test_prefill_attention_bfloat16(ops, Hq, Hkv, D, page, window):
 ])
 def test_which_short_requests_share_their_keys_out(ops, B, new, Hq, Hkv, keys):
     """Where that was measured to be the faster way for a request of a few tokens beside portions (else another 4 to 26 % slower)."""
-    for D, most in ((128, keys), (64, keys), (256, None)):
+    for D, most in ((128, keys), (64, keys), (96, None), (256, None)):
         assert ops.backend().attention_lib(D).nhv_prefill_attention_one_tile_from(B, new, Hq, Hkv) == (most or 2 ** 31 - 1)
 
 
 @pytest.mark.parametrize("Hq,Hkv,D,page,portion,two,reach,cap,sinks,slopes,gated", [
     (32, 8, 128, 16, 900, True, None, None, None, False, False), (8, 2, 128, 256, 60, False, ("window", 70), None, "each", False, True),
     (16, 1, 128, 64, 60, False, ("chunk", 50), 3.0, "one", False, False), (5, 5, 48, 7, 60, False, None, None, None, True, True),
-    (6, 2, 80, 32, 60, False, ("window", 1), None, "each", True, False), (3, 1, 16, 8, 60, False, None, 2.0, None, False, True),
+    (6, 2, 48, 32, 60, False, ("window", 1), None, "each", True, False), (3, 1, 16, 8, 60, False, None, 2.0, None, False, True),
     (4, 4, 64, 48, 60, False, ("chunk", 33), None, "each", True, False), (7, 1, 112, 128, 60, False, ("window", 333), None, None, False, False),
     # tables of more than 1,024 entries: of single tokens, of pages; and with two row tiles a wave, plain, capped and biased
     (8, 2, 64, 1, 60, False, None, None, None, False, False), (8, 1, 64, 32, 60, False, None, None, "one", False, True),
     (16, 4, 64, 1, 700, True, ("window", 600), None, None, True, False), (32, 4, 128, 32, 700, True, ("window", 500), 5.0, "each", False, True),
-    (12, 3, 96, 1, 900, True, None, None, None, False, False),
+    (12, 3, 32, 1, 900, True, None, None, None, False, False),
 ])
 def test_prefill_attention_of_one_tile_beside_prompts(ops, Hq, Hkv, D, page, portion, two, reach, cap, sinks, slopes, gated):
     """Requests whose rows are one tile, whose keys four waves share, beside a longer portion: one to four tokens, from the last length that goes

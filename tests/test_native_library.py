@@ -91,6 +91,21 @@ def test_the_wait_for_x_has_the_loads_behind_it_that_it_counts(tmp_path):
     assert seen >= 50, seen
 
 
+@pytest.mark.parametrize("D,tiles,blocks", [(48, 2, 3), (64, 1, 4), (80, 1, 3), (96, 1, 3)])
+def test_the_prompts_attention_leaves_registers_for_the_blocks_that_fit(tmp_path, D, tiles, blocks):
+    """Where LDS has room for three or four blocks of four waves a compute unit, a SIMD's 512 registers a lane have room for as many
+    waves, and nothing is kept in memory instead: heads of these sizes, so many row tiles a wave, without cap or bias."""
+    source, out = os.path.join(library.CSRC, "attention_prefill_bf16.hip"), tmp_path / "attention.s"
+    subprocess.run([library._hipcc(), *[f for f in library.HIPCC_FLAGS if f != "-fPIC"], f"-DNHV_HEAD_DIM={D}", "-I", library.CSRC,
+                    "--cuda-device-only", "-S", source, "-o", str(out)], check=True, capture_output=True)
+    text, seen = out.read_text(), 0
+    for name, registers in re.findall(r"\.set (\S*prefill_attention_kernelILb[01]ELi%dELb[01]ELb0ELb0E\S*?)\.num_vgpr, (\d+)" % tiles, text):
+        scratch = re.search(re.escape(name) + r"\.private_seg_size, (\d+)", text)
+        assert int(registers) <= 512 // blocks // 8 * 8 and scratch[1] == "0", (name, registers, scratch[1])
+        seen += 1
+    assert seen == 4
+
+
 def test_no_scalar_offset_of_the_gates_kernel_lies_behind_its_rows(tmp_path):
     """Of a tile that is cut off at the end, the rows behind it are kept out by the descriptor's size, with which the lane's offset is
     compared after the scalar offset has been taken from it: that one must not be the larger. In what the compiler makes of each kernel
