@@ -662,13 +662,21 @@ static Choice gated_tile(long long M, long long N, bool whole) {
 }
 
 // Whether tiles of 128 x 128 rows of x and of w (gated: 64 outputs) are the faster ones: where tiles of 64 x 128 need twice the rounds of 256
-// blocks that these do; a first one that is hardly begun is little to save. Measured over 9,700 sizes (90 to 2,048 rows, 700 to 8,200 outputs of 256 to 4,096
-// columns; time over that of the choice without them): 1 round 0.86 and 0.88 gated, the worst 1.01 and 1.03 (from 257 smaller blocks on 1.17); 2 rounds 0.87 and 0.91,
+// blocks that these do. Measured over 9,700 sizes (90 to 2,048 rows, 700 to 8,200 outputs of 256 to 4,096
+// columns; time over that of the choice without them): 1 round 0.86 and 0.88 gated, the worst 1.01 and 1.03; 2 rounds 0.87 and 0.91,
 // 1.01; 3 0.89 and 0.91, 1.0; 4 and more 0.92, 1.08. Elsewhere 0.9 to 1.57 (2 rounds where the others need 2).
-static bool big_tiles(long long M, long long N, bool whole, bool gated) {
+// A second round of smaller ones that is hardly begun is little to save: of 257 to 300 blocks up to 1.17. And of few columns a tile's first pieces and its
+// sums are most of its time: 192 columns 0.97, 224 0.89, but 128 1.05, the worst 1.07 (1,004 x 2,592 12.2, 13.1 us).
+constexpr int BEGUN = 44, BIG_COLUMNS = 192;
+static bool big_tiles(long long M, long long N, int K, bool whole, bool gated) {
   const long long columns = gated ? 64 : 128, n = (N + columns - 1) / columns, blocks = (M + 127) / 128 * n, smaller = (M + 63) / 64 * n;
   const long long rounds = (blocks + 255) / 256;
-  return whole && M > 64 && smaller > (2 * rounds - 1) * 256 + (rounds == 1 ? 44 : 0);
+  return whole && K >= BIG_COLUMNS && M > 64 && smaller > (2 * rounds - 1) * 256 + (rounds == 1 ? BEGUN : 0);
+}
+
+// The same for operands on 16-byte boundaries.
+extern "C" int nhv_gemm_float32_big_tiles(int M, int N, int K, int gated) {
+  return M > 0 && N > 0 && K > 0 && big_tiles(M, N, K, whole_pieces(nullptr, nullptr, K), gated != 0);
 }
 
 extern "C" int nhv_gemm_float32(const void* x, const void* w, const void* bias, void* y, int M, int N, int K, void* stream) {
@@ -678,7 +686,7 @@ extern "C" int nhv_gemm_float32(const void* x, const void* w, const void* bias, 
   const float *xf = (const float*)x, *wf = (const float*)w, *bf = (const float*)bias;
   float* yf = (float*)y;
   const bool whole = whole_pieces(x, w, K);
-  switch (big_tiles(M, N, whole, false) ? 8 : plain_tile(M, N, whole).tile) {
+  switch (big_tiles(M, N, K, whole, false) ? 8 : plain_tile(M, N, whole).tile) {
     case 0: launch<1, 1, 2, false>(xf, wf, bf, yf, M, N, K, {}, s); break;
     case 1: launch<1, 2, 1, false>(xf, wf, bf, yf, M, N, K, {}, s); break;
     case 2: launch<2, 2, 1, false>(xf, wf, bf, yf, M, N, K, {}, s); break;
@@ -871,7 +879,7 @@ static bool halved(long long M, long long N, int K) {
 extern "C" int nhv_gemm_float32_gated_pays(const void* x, const void* w, int M, int N, int K) {
   const bool wide = K % 4 == 0 && (uintptr_t)x % 16 == 0 && (uintptr_t)w % 16 == 0;
   const bool whole = whole_pieces(x, w, K);
-  if (big_tiles(M, N, whole, true)) return 1;              // (as many blocks as the packed product)
+  if (big_tiles(M, N, K, whole, true)) return 1;              // (as many blocks as the packed product)
   const bool halves = whole && halved(M, N, K);
   const Choice gated = gated_tile(M, N, whole && !halves);
   if (halves && gated.tile == 4) return 1;                 // (the packed product's larger blocks cost the same 4 us more: 1,000 x 1024 of 256 15.6 here, packed 21.2)
@@ -888,7 +896,7 @@ extern "C" int nhv_gemm_float32_gated(const void* x, const void* w, const void* 
   const NhvGate gate = {act, limit, alpha, offset};
   const float *xf = (const float*)x, *wf = (const float*)w, *bf = (const float*)bias;
   float* yf = (float*)y;
-  const bool big = big_tiles(M, N, whole_pieces(x, w, K), true), whole = whole_pieces(x, w, K) && !halved(M, N, K);
+  const bool big = big_tiles(M, N, K, whole_pieces(x, w, K), true), whole = whole_pieces(x, w, K) && !halved(M, N, K);
   switch (big ? 5 : gated_tile(M, N, whole).tile) {
     case 0: launch<1, 2, 1, true>(xf, wf, bf, yf, M, N, K, gate, s); break;
     case 1: launch<2, 2, 1, true>(xf, wf, bf, yf, M, N, K, gate, s); break;

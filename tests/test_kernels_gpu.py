@@ -441,13 +441,16 @@ def test_float32_linear_in_all_its_tiles(ops, N, K):
         last = y
 
 
-@pytest.mark.parametrize("M,N,K", [(300, 7970, 32), (300, 8000, 64), (517, 7168, 288), (517, 7100, 1024), (1000, 6267, 96), (1100, 14400, 64)])
-def test_float32_linear_in_tiles_of_128_rows(ops, M, N, K):
-    """Tiles of 128 x 128 in one round of blocks, two and four: one piece of 32 columns and more, rows and columns that end inside a tile,
-    plain and gated, an infinite row: the rows that few rows alone give, bit for bit."""
+@pytest.mark.parametrize("M,N,K,taken", [(300, 8000, 192, 1), (300, 7970, 224, 1), (417, 6144, 544, 1), (517, 6100, 288, 1), (517, 6144, 1024, 1), (577, 4130, 256, 1),
+                                         (1000, 6268, 352, 1), (1049, 3072, 1056, 1), (1100, 14400, 256, 1), (128, 20000, 256, 1),
+                                         (300, 8000, 160, 0), (517, 7168, 288, 0), (300, 8000, 1200, 0), (545, 4130, 256, 0), (150, 2000, 256, 0)])
+def test_float32_linear_in_tiles_of_128_rows(ops, M, N, K, taken):
+    """Tiles of 128 x 128 in one round of blocks, two and four, and sizes that just do not take them: segments of one piece of 32 columns and
+    of several, rows and columns that end inside a tile, plain and gated, an infinite row: the rows that few rows alone give, bit for bit."""
+    big = ops.backend().lib.nhv_gemm_float32_big_tiles
+    assert big(M, N, K, 0) == taken and big(M, N // 2, K, 1) == taken
     x, w, b = rnd(M, K, seed=141), rnd(N, K, seed=142), rnd(N, seed=143)
     x[M - 3, K // 2] = float("inf")
-    N -= N % 2
     y, g = ops.linear(x, w[:N], b[:N]), ops.gated_linear(x, w[:N], "silu", b[:N])
     for rows in (slice(0, 16), slice(M - 5, M), slice(124, 134)):
         some = x[rows].contiguous()
@@ -455,7 +458,7 @@ def test_float32_linear_in_tiles_of_128_rows(ops, M, N, K):
             assert torch.equal(got.isnan(), want.isnan()) and torch.equal(got.nan_to_num(1.5, 2.5, 3.5), want.nan_to_num(1.5, 2.5, 3.5))
 
 
-@pytest.mark.parametrize("M,N,K", [(1090, 4100, 64), (1090, 4100, 70), (577, 4130, 256), (577, 4130, 33), (321, 4096, 1000), (190, 6150, 256), (200, 3080, 288),
+@pytest.mark.parametrize("M,N,K", [(1090, 4100, 64), (1090, 4100, 70), (545, 4130, 256), (577, 4130, 33), (321, 4096, 1000), (190, 6150, 256), (200, 3080, 288),
                                    (250, 2047, 768), (700, 3072, 1024)])
 def test_float32_linear_in_tiles_of_64_rows(ops, M, N, K):
     """Tiles of 64 x 64 and 64 x 128, whole pieces of 32 columns and not, plain and gated (halved or not): the rows that few rows alone give, bit for bit."""
