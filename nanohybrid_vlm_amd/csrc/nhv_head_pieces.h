@@ -39,33 +39,66 @@ __device__ __forceinline__ void store8f<float>(float* p, const float* in) {
   *reinterpret_cast<float4*>(p + 4) = make_float4(in[4], in[5], in[6], in[7]);
 }
 
-// Row ids[t] of a table times scale, as TO, by the whole block in pieces of eight entries (H a multiple of 8, table and rows 16 bytes aligned). An
-// id out of range gives a row of zeros. One trip to memory after the id's; entry by entry, a row of 4,096 in bfloat16 takes 256 threads 16
+// E entries of a row (16 bytes of floats or of the type itself), in float
+template <int E, typename V>
+__device__ __forceinline__ void load_entries(const V* p, float* out) {
+  if constexpr (E == 8) {
+    load8f<V>(p, out);
+  } else if constexpr (sizeof(V) == 4) {
+    const float4 a = *reinterpret_cast<const float4*>(p);
+    out[0] = a.x, out[1] = a.y, out[2] = a.z, out[3] = a.w;
+  } else {
+    typedef V four __attribute__((ext_vector_type(4)));
+    const four a = *reinterpret_cast<const four*>(p);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) out[i] = (float)a[i];
+  }
+}
+template <int E, typename V>
+__device__ __forceinline__ void store_entries(V* p, const float* in) {
+  if constexpr (E == 8) store8f<V>(p, in);
+  else *reinterpret_cast<float4*>(p) = make_float4(in[0], in[1], in[2], in[3]);
+}
+
+// Row ids[t] of a table times scale, as TO, by the whole block, eight entries a thread at a time (H a multiple of 8, table and rows 16 bytes aligned), in pieces of
+// 16 bytes of the result, neighbours' side by side: what a wave stores is in a row. (Eight floats a thread side by side: 2,048 rows of 4,096 floats 12.0 us, so 10.7,
+// entry by entry 11.4.) An id out of range gives a row of zeros. One trip to memory after the id's; entry by entry, a row of 4,096 in bfloat16 takes 256 threads 16
 // trips: 8 rows 8.9 us, so 3.8, 2,048 rows 16.6 and 11.5; 16 rows of 2,048 as floats 7.3 and 3.1.
 template <typename T, typename TO>
 __device__ __forceinline__ void embed_row(const int* ids, const T* table, TO* out, int H, int V, float scale) {
+  constexpr int E = 16 / sizeof(TO), P = 8 / E;
   const int t = blockIdx.x, id = ids[t];
   const bool ok = id >= 0 && id < V;
-  for (int i = threadIdx.x * 8; i < H; i += blockDim.x * 8) {
-    const T* from = table + (size_t)(ok ? id : 0) * H + i;
-    TO* to = out + (size_t)t * H + i;
+  const T* row = table + (size_t)(ok ? id : 0) * H;
+  TO* to = out + (size_t)t * H;
+  for (int first = threadIdx.x * E; first < H; first += blockDim.x * 8) {
+    int at[P];
+#pragma unroll
+    for (int p = 0; p < P; ++p) at[p] = min(first + p * (int)blockDim.x * E, H - E);   // (behind the end: the last piece once more)
     if (std::is_same<T, TO>::value && scale == 1.0f) {   // (the bytes)
+      uint4 v[P];
 #pragma unroll
-      for (int p = 0; p < (int)sizeof(T) / 2; ++p) {
-        const uint4 v = reinterpret_cast<const uint4*>(from)[p];
-        reinterpret_cast<uint4*>(to)[p] = ok ? v : uint4{0, 0, 0, 0};
-      }
+      for (int p = 0; p < P; ++p) v[p] = *reinterpret_cast<const uint4*>(row + at[p]);
+#pragma unroll
+      for (int p = 0; p < P; ++p) *reinterpret_cast<uint4*>(to + at[p]) = ok ? v[p] : uint4{0, 0, 0, 0};
     } else {
-      float v[8];
-      load8f<T>(from, v);
+      float v[P][E];
 #pragma unroll
-      for (int e = 0; e < 8; ++e) v[e] = ok ? v[e] * scale : 0.f;
-      store8f<TO>(to, v);
+      for (int p = 0; p < P; ++p) load_entries<E, T>(row + at[p], v[p]);
+#pragma unroll
+      for (int p = 0; p < P; ++p) {
+#pragma unroll
+        for (int e = 0; e < E; ++e) v[p][e] = ok ? v[p][e] * scale : 0.f;
+        store_entries<E, TO>(to + at[p], v[p]);
+      }
     }
   }
 }
 inline bool embeds_by_pieces(const void* table, const void* out, int H) { return H % 8 == 0 && (((uintptr_t)table | (uintptr_t)out) & 15) == 0; }
-inline unsigned embed_threads(int H) { return H >= 8192 ? 1024 : (unsigned)((H / 8 + 63) / 64 * 64); }
+inline unsigned embed_threads(int H) {       // (as many trips as 1,024 threads need, all of them full)
+  const int trips = (H / 8 + 1023) / 1024;
+  return (unsigned)((H / 8 + 64 * trips - 1) / (64 * trips) * 64);
+}
 
 // Eight entries of a product that comes as float parts (gemm_lines_bf16.hip), `stride` entries apart, added in their order; all
 // parts are asked for before the first is used.
