@@ -481,14 +481,145 @@ __global__ __launch_bounds__(64 * WAVES) void head_gemm_mfma_kernel(const bf16_t
   }
 }
 
-// The same for many rows (K <= HT_MAX_K). Bound by the bytes of x, y and the gate: a wave owns 16 rows of one head, whose
-// entries it holds as operands, and the head's matrix comes into LDS once a block (up to 64 KB at a time), as operands in
+#define HT_MAX_K 512
+// The same for many rows (K <= HT_MAX_K), of any outputs: a block owns 64 rows of one head and walks over all of them, 128 at a time.
+// The rows come into LDS once, whole rows of K entries; a wave takes 32 of the 128 outputs, with the matrix rows straight
+// from memory (L2), and the results go back through LDS so that rows are written in pieces of 16 bytes side by side.
+#define HT_ROWS 64
+#define HT_COLS 128
+template <int U>
+__global__ __launch_bounds__(256) void head_gemm_tile_kernel(const bf16_t* __restrict__ x, long long xs_t, long long xs_h,
+                                                             const bf16_t* __restrict__ w, bf16_t* __restrict__ y,
+                                                             long long ys_t, long long ys_h, const void* __restrict__ gate,
+                                                             int gate_mode, long long gs_t, int rows, int N, int K, int rot,
+                                                             int x_rot_off, int y_rot_off, int halves,
+                                                             const double* __restrict__ freqs, float gain,
+                                                             const int* __restrict__ positions, int vec_out, int vec_gate) {
+  extern __shared__ __attribute__((aligned(16))) unsigned char ht_lds[];
+  const int pitch = K + 8;                               // 16 bytes more than a row: the rows spread over the banks
+  bf16_t* xs = reinterpret_cast<bf16_t*>(ht_lds);        // [64][pitch]
+  constexpr int YP = HT_COLS + 8;
+  bf16_t* ys = xs + HT_ROWS * pitch;                     // [64][YP]
+  const int h = blockIdx.x, m0 = blockIdx.y * HT_ROWS;
+  const int here = min(HT_ROWS, rows - m0);
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int col = lane & 15, grp = lane >> 4;
+  const int pieces = K / 8;
+  for (int i = threadIdx.x; i < HT_ROWS * pieces; i += 256) {
+    const int m = i / pieces, p = i % pieces;
+    hg_bf16x8 v;
+    if (m < here) v = *reinterpret_cast<const hg_bf16x8*>(x + (size_t)(m0 + m) * xs_t + (size_t)h * xs_h + p * 8);
+    else {
+#pragma unroll
+      for (int e = 0; e < 8; ++e) v[e] = (__bf16)0.f;
+    }
+    *reinterpret_cast<hg_bf16x8*>(xs + m * pitch + p * 8) = v;
+  }
+  // the rotated part of these rows, while the rows are on their way
+  for (int i = threadIdx.x; i < here * (rot / 2); i += 256) {
+    const int t = m0 + i / (rot / 2);
+    nhv_turn_pair(x + (size_t)t * xs_t + (size_t)h * xs_h + x_rot_off, y + (size_t)t * ys_t + (size_t)h * ys_h + y_rot_off,
+                  i % (rot / 2), rot, halves, positions[t], freqs, gain);
+  }
+  hg_bf16x8 zero;
+#pragma unroll
+  for (int i = 0; i < 8; ++i) zero[i] = (__bf16)0.f;
+  __syncthreads();
+  for (int c0 = 0; c0 < N; c0 += HT_COLS) {
+    const int n0 = c0 + wave * 32;
+    if (n0 < N) {                                        // the whole wave; every wave meets the barriers below
+      const bf16_t* wrow[2];
+      bool n_ok[2];
+#pragma unroll
+      for (int nt = 0; nt < 2; ++nt) {
+        const int n = n0 + nt * 16 + col;
+        n_ok[nt] = n < N;
+        wrow[nt] = w + ((size_t)h * N + (n_ok[nt] ? n : 0)) * K;
+      }
+      hg_floatx4 acc[4][2];
+#pragma unroll
+      for (int mt = 0; mt < 4; ++mt)
+#pragma unroll
+        for (int nt = 0; nt < 2; ++nt) acc[mt][nt] = hg_floatx4{0.f, 0.f, 0.f, 0.f};
+      // gates of four entries at once, asked for before the products
+      hg_bf16x4 g4[4][2];
+      if (vec_gate) {
+#pragma unroll
+        for (int mt = 0; mt < 4; ++mt)
+#pragma unroll
+          for (int nt = 0; nt < 2; ++nt) {
+            const int n = n0 + nt * 16 + grp * 4, m = m0 + min(mt * 16 + col, here - 1);
+            g4[mt][nt] = *reinterpret_cast<const hg_bf16x4*>(reinterpret_cast<const bf16_t*>(gate) + (size_t)m * gs_t + (size_t)h * N +
+                                                             (n < N ? n : 0));
+          }
+      }
+      for (int k0 = 0; k0 < K; k0 += 32 * U) {
+        hg_bf16x8 a[U][2];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+          const int k = k0 + u * 32 + grp * 8;
+#pragma unroll
+          for (int nt = 0; nt < 2; ++nt) a[u][nt] = (n_ok[nt] && k < K) ? *reinterpret_cast<const hg_bf16x8*>(wrow[nt] + k) : zero;
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+          const int k = k0 + u * 32 + grp * 8;
+#pragma unroll
+          for (int mt = 0; mt < 4; ++mt) {
+            const hg_bf16x8 b = k < K ? *reinterpret_cast<const hg_bf16x8*>(xs + (mt * 16 + col) * pitch + k) : zero;
+#pragma unroll
+            for (int nt = 0; nt < 2; ++nt) acc[mt][nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[u][nt], b, acc[mt][nt], 0, 0, 0);
+          }
+        }
+      }
+#pragma unroll
+      for (int mt = 0; mt < 4; ++mt)
+#pragma unroll
+        for (int nt = 0; nt < 2; ++nt) {
+          hg_bf16x4 four;
+          float v[4];
+#pragma unroll
+          for (int j = 0; j < 4; ++j) v[j] = acc[mt][nt][j];
+          if (vec_gate) {
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+              v[j] *= __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(-1.4426950408889634f * (float)g4[mt][nt][j]));
+          } else if (gate != nullptr && mt * 16 + col < here) {
+            const int n = n0 + nt * 16 + grp * 4;
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+              if (n + j < N) v[j] *= nhv_head_gate_of<bf16_t>(gate, gate_mode, gs_t, m0 + mt * 16 + col, h, N, n + j);
+          }
+#pragma unroll
+          for (int j = 0; j < 4; ++j) four[j] = (__bf16)v[j];
+          *reinterpret_cast<hg_bf16x4*>(ys + (mt * 16 + col) * YP + wave * 32 + nt * 16 + grp * 4) = four;
+        }
+    }
+    __syncthreads();
+    const int width = min(HT_COLS, N - c0);
+    if (vec_out) {                                       // N and the rows of y are pieces of 16 bytes
+      for (int i = threadIdx.x; i < here * (width / 8); i += 256) {
+        const int m = i / (width / 8), p = i % (width / 8);
+        *reinterpret_cast<hg_bf16x8*>(y + (size_t)(m0 + m) * ys_t + (size_t)h * ys_h + c0 + p * 8) =
+            *reinterpret_cast<const hg_bf16x8*>(ys + m * YP + p * 8);
+      }
+    } else {
+      for (int i = threadIdx.x; i < here * width; i += 256) {
+        const int m = i / width, p = i % width;
+        y[(size_t)(m0 + m) * ys_t + (size_t)h * ys_h + c0 + p] = ys[m * YP + p];
+      }
+    }
+    __syncthreads();
+  }
+}
+
+// The same where outputs are pieces of 16 bytes and the matrix nearly fills its tiles, or blocks are many (nhv_head_gemm_rows_pays). Bound by the bytes of x, y and the gate: a wave owns
+// 16 rows of one head, whose entries it holds as operands, and the head's matrix comes into LDS once a block (up to 64 KB at a time), as operands in
 // the order in which they are read. Two tiles of 16 outputs are 32 outputs side by side: tile t's line i is output
 // 8 (i / 4) + 4 t + i % 4, so that a lane ends up with eight outputs in a row and writes (and reads the gate) in pieces of
 // 16 bytes, with nothing but the matrix behind a barrier. 4,220 rows of 16 heads: 128 to 192 entries and 64 turned, 44 us as
 // blocks of 64 rows that walk over the outputs with the rows in LDS and the matrix from memory, 24 so; 192 to 128 with a gate
 // per entry 32 and 23 (these bytes at 5 TB/s: 12). Blocks of 4, 8 and 16 waves 27, 25 and 24.
-#define HT_MAX_K 512
 #define HT_LDS 65536
 template <int KS, int WAVES>
 __global__ __launch_bounds__(64 * WAVES) void head_gemm_rows_kernel(const bf16_t* __restrict__ x, long long xs_t, long long xs_h,
@@ -497,8 +628,7 @@ __global__ __launch_bounds__(64 * WAVES) void head_gemm_rows_kernel(const bf16_t
                                                                     int gate_mode, long long gs_t, int rows, int N, int K, int rot,
                                                                     int x_rot_off, int y_rot_off, int halves,
                                                                     const double* __restrict__ freqs, float gain,
-                                                                    const int* __restrict__ positions, int vec_out, int vec_gate,
-                                                                    int vec_turn) {
+                                                                    const int* __restrict__ positions, int vec_gate, int vec_turn) {
   extern __shared__ __attribute__((aligned(16))) unsigned char ht_lds[];
   hg_bf16x8* ws = reinterpret_cast<hg_bf16x8*>(ht_lds);  // [tile of 16 outputs][KS][64]
   constexpr int PAIRS = HT_LDS / (2 * KS * 1024) / 2 * 2;  // of tiles, in LDS at a time: whole groups
@@ -562,7 +692,6 @@ __global__ __launch_bounds__(64 * WAVES) void head_gemm_rows_kernel(const bf16_t
       if (p0 == 0) __syncthreads();                      // the pieces are there
 #pragma unroll
       for (int i = 0; i < GROUP; ++i) {
-
         hg_floatx4 acc[2] = {hg_floatx4{0.f, 0.f, 0.f, 0.f}, hg_floatx4{0.f, 0.f, 0.f, 0.f}};
 #pragma unroll
         for (int ks = 0; ks < KS; ++ks)
@@ -578,16 +707,21 @@ __global__ __launch_bounds__(64 * WAVES) void head_gemm_rows_kernel(const bf16_t
           else if (gate != nullptr && live && n + j < N) v *= nhv_head_gate_of<bf16_t>(gate, gate_mode, gs_t, m, h, N, n + j);
           eight[j] = (__bf16)v;
         }
-        if (vec_out) {                                   // N and the rows of y are pieces of 16 bytes
-          if (live && n < N) *reinterpret_cast<hg_bf16x8*>(yr + n) = eight;
-        } else {
-#pragma unroll
-          for (int j = 0; j < 8; ++j)
-            if (live && n + j < N) yr[n + j] = (bf16_t)eight[j];
-        }
+        if (live && n < N) *reinterpret_cast<hg_bf16x8*>(yr + n) = eight;
       }
     }
   }
+}
+
+// Whether the matrix in LDS is the faster way for outputs in pieces of 16 bytes: of many blocks of 64 rows, or where at most a sixth of its tiles' products (64 outputs
+// by 128, 192, 256 or 512 entries) are for nothing, or heads are small. Measured over 845 such sizes (1 to 128 heads of 8 to 750 outputs of 8 to 512 entries, 65 to
+// 6,000 rows; time over the other way's): blocks from 700 on 0.65 on average, fewer and full tiles 0.90, small heads 0.84, the worst 1.07 (200 rows of 64 heads, 512 outputs
+// of 512 entries 38.1, 40.6 us); others 1.07, up to 1.24 (5 heads of 368 outputs of 288 entries 19.0, 23.3). Outputs of other lengths, or that begin elsewhere, can only
+// be stored entry by entry so: 321 sizes 1.03, up to 2.05 (2,038 rows of 16 heads, 64 to 300 entries, 22 us, 44).
+extern "C" int nhv_head_gemm_rows_pays(int rows, int H, int N, int K) {
+  if (rows <= 64 || H <= 0 || N <= 0 || N % 8 || K <= 0 || K > HT_MAX_K) return 0;
+  const long long blocks = (long long)H * ((rows + 63) / 64), tiles = (N + 63) / 64 * 64ll * (K <= 128 ? 128 : K <= 192 ? 192 : K <= 256 ? 256 : 512);
+  return blocks >= 700 || 5 * tiles <= 6ll * N * K || (N <= 64 && K > 32);
 }
 
 extern "C" int nhv_head_gemm_bf16(const void* x, long long xs_t, long long xs_h, const void* w, void* y, long long ys_t,
@@ -609,20 +743,19 @@ extern "C" int nhv_head_gemm_bf16(const void* x, long long xs_t, long long xs_h,
                        (const bf16_t*)w, (bf16_t*)y, ys_t, ys_h, gate, gate_mode, gs_t, rows, N, K, n_chunks, rot,        \
                        x_rot_off, y_rot_off, halves, (const double*)freqs, gain, (const int*)positions);                  \
   } while (0)
-  if (rows > 64 && K <= HT_MAX_K) {
-    const int vec_out = N % 8 == 0 && ys_t % 8 == 0 && ys_h % 8 == 0 && (uintptr_t)y % 16 == 0;
-    const int vec_gate = gate != nullptr && gate_mode == 2 && N % 4 == 0 && gs_t % 4 == 0 && (uintptr_t)gate % 8 == 0;
-    const int vec_turn = rot % 16 == 0 && x_rot_off % 8 == 0 && y_rot_off % 8 == 0 && ys_t % 8 == 0 && ys_h % 8 == 0 && (uintptr_t)y % 16 == 0;
+  const int vec_out = N % 8 == 0 && ys_t % 8 == 0 && ys_h % 8 == 0 && (uintptr_t)y % 16 == 0;
+  const int vec_gate = gate != nullptr && gate_mode == 2 && N % 4 == 0 && gs_t % 4 == 0 && (uintptr_t)gate % 8 == 0;
+  if (vec_out && nhv_head_gemm_rows_pays(rows, H, N, K)) {
+    const int vec_turn = rot % 16 == 0 && x_rot_off % 8 == 0 && y_rot_off % 8 == 0;
 #define ROWS_LAUNCH(KS, WAVES)                                                                                            \
   do {                                                                                                                    \
-    const int pairs = (N + 63) / 64 * 2, most = HT_LDS / (2 * KS * 1024) / 2 * 2;                                                     \
+    const int pairs = (N + 63) / 64 * 2, most = HT_LDS / (2 * KS * 1024) / 2 * 2;                          \
     const dim3 grid(H, (rows + 16 * WAVES - 1) / (16 * WAVES));                                                           \
     NHV_REQUIRE(grid.y <= 65535, "head_gemm_bf16: %d rows are too many", rows);                                           \
     hipLaunchKernelGGL((head_gemm_rows_kernel<KS, WAVES>), grid, dim3(64 * WAVES),                                        \
                        (size_t)(pairs < most ? pairs : most) * 2 * KS * 1024, s, (const bf16_t*)x, xs_t, xs_h,            \
                        (const bf16_t*)w, (bf16_t*)y, ys_t, ys_h, gate, gate_mode, gs_t, rows, N, K, rot, x_rot_off,       \
-                       y_rot_off, halves, (const double*)freqs, gain, (const int*)positions, vec_out, vec_gate,           \
-                       vec_turn);                                                                                         \
+                       y_rot_off, halves, (const double*)freqs, gain, (const int*)positions, vec_gate, vec_turn);           \
   } while (0)
 #define ROWS_LAUNCH_OF(KS)                                                                                                \
   do {                                                                                                                    \
@@ -638,6 +771,18 @@ extern "C" int nhv_head_gemm_bf16(const void* x, long long xs_t, long long xs_h,
     else ROWS_LAUNCH_OF(16);
 #undef ROWS_LAUNCH_OF
 #undef ROWS_LAUNCH
+  } else if (rows > 64 && K <= HT_MAX_K) {
+    const size_t lds = (size_t)HT_ROWS * (K + 8 + HT_COLS + 8) * sizeof(bf16_t);
+    auto kernel = head_gemm_tile_kernel<4>;
+    // more than 64 KB of dynamic LDS has to be allowed once per kernel (and per process)
+    static const hipError_t allowed = hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                                          (int)(HT_ROWS * (HT_MAX_K + 8 + HT_COLS + 8) * sizeof(bf16_t)));
+    NHV_REQUIRE(allowed == hipSuccess, "head_gemm_bf16: %s", hipGetErrorString(allowed));
+    const dim3 grid(H, (rows + HT_ROWS - 1) / HT_ROWS);
+    NHV_REQUIRE(grid.y <= 65535, "head_gemm_bf16: %d rows are too many", rows);
+    hipLaunchKernelGGL(kernel, grid, dim3(256), lds, s, (const bf16_t*)x, xs_t, xs_h, (const bf16_t*)w, (bf16_t*)y, ys_t, ys_h, gate,
+                       gate_mode, gs_t, rows, N, K, rot, x_rot_off, y_rot_off, halves, (const double*)freqs, gain,
+                       (const int*)positions, vec_out, vec_gate);
   } else if (rows <= 16) {
     LAUNCH(1, 1, 1, 4);
   } else if (rows <= 64) {

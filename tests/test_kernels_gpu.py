@@ -2226,11 +2226,18 @@ def test_single_tokens_beyond_what_the_splits_cover_are_stored_and_read(ops, mon
     torch.testing.assert_close(got, want, rtol=1.6e-2, atol=1.6e-2)
 
 
-@pytest.mark.parametrize("H, N, K, rot, rows", [(3, 8, 8, 16, 65), (2, 130, 40, 6, 257), (16, 192, 128, 64, 2100), (16, 128, 192, 0, 2050),
-                                                (5, 330, 168, 32, 129), (2, 72, 512, 16, 191), (40, 33, 264, 0, 1030), (1, 520, 256, 64, 16500)])
-def test_a_matrix_per_head_of_many_rows(ops, H, N, K, rot, rows):
+@pytest.mark.parametrize("H, N, K, rot, rows, in_lds", [
+    # the matrix in LDS: full tiles, small heads, many blocks; once and in pieces, rows that end inside a block and a wave
+    (16, 192, 128, 64, 2100, 1), (16, 128, 192, 0, 2050, 1), (1, 520, 256, 64, 16500, 1), (3, 8, 40, 16, 65, 1), (5, 56, 264, 32, 129, 1), (2, 64, 512, 0, 257, 1),
+    (40, 72, 40, 16, 1170, 1), (64, 88, 512, 0, 700, 1), (128, 200, 8, 16, 330, 1), (7, 128, 480, 0, 191, 1), (2, 600, 128, 16, 66, 1),
+    # outputs over the rows in LDS
+    (3, 8, 8, 16, 65, 0), (2, 130, 40, 6, 257, 0), (5, 330, 168, 32, 129, 0), (2, 72, 512, 16, 191, 0), (40, 33, 264, 0, 1030, 0), (16, 300, 64, 0, 2038, 0),
+    (5, 368, 288, 32, 512, 0), (40, 100, 24, 6, 1200, 0)])
+def test_a_matrix_per_head_of_many_rows(ops, H, N, K, rot, rows, in_lds):
     """Products with a matrix per head of more than 64 rows at the edges of a block's rows, of the pieces of the matrix that
-    are in LDS at a time and of the outputs that a lane writes at once, with and without gates and a turned part."""
+    are in LDS at a time and of the outputs that a lane writes at once, with and without gates and a turned part; rows of results that
+    begin anywhere, of the same bits."""
+    assert ops.backend().lib.nhv_head_gemm_rows_pays(rows, H, N, K) == in_lds
     g = torch.Generator(device="cuda").manual_seed(rows)
     rand = lambda *shape: torch.randn(*shape, generator=g, device="cuda").to(torch.bfloat16)
     pad = -(K + rot) % 8
@@ -2248,6 +2255,9 @@ def test_a_matrix_per_head_of_many_rows(ops, H, N, K, rot, rows):
             turn = (rot, K, at, freqs, 1.0, pos, halves) if rot else None
             ops.head_gemm(x, w.view(H * N, K), False, N, K, out=out, out_off=off, turn=turn)
             assert bool(((out[:, :, off:off + N].double() - want).abs() <= bound).all()), (off, halves)
+            got = out[:, :, off:off + N].clone()
+            assert off == 0 or torch.equal(got, first)
+            first = got
             mask = torch.ones(width, dtype=torch.bool)
             mask[off:off + N] = False
             if rot:
