@@ -27,7 +27,7 @@
 // The preparation is bound by its vector instructions (80 % of the clocks of all SIMDs). It took 4,230 a wave, of which 1,520 were the
 // decays (a division to find token and channel, log1pf, expf), 720 the inputs' SiLU and 280 moved scalar values to vector
 // registers and back; with the functions below, rows dealt to waves, and nothing worked out ahead that a wave cannot keep, half of
-// that: the same sizes 77, 60; 56, 42; 114, 81; 69, 50; 274, 175 us, 40 and 17 tokens 22, 15. Results are as far from 64 bits as before (1.7e-7 to
+// that: the same sizes 77, 61; 56, 43; 114, 82; 69, 51; 274, 179 us, 40 and 17 tokens 22, 15. Results are as far from 64 bits as before (1.7e-7 to
 // 2.8e-7 of their size, by how slowly they decay).
 // Portions of 1,500 and 701 tokens, 16 heads of 128, with the update of the kept inputs and the read-out's norm: 198 us where the
 // separate kernels take 638; one of 8,000 770 against 3,204. The blocks of the preparation are requests by the longest portion:

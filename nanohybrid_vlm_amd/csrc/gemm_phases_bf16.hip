@@ -1,14 +1,14 @@
 // A gate of two products of many rows in bfloat16, y[M, N] = gate(x[M, K] . wg[N, K]^T + bg, x . wu^T + bu) with w = [wg; wu], or
 // one product and what its result passes, y = act(x . w^T).
 //
-// The product alone is no faster than the vendor's library's (0.96 to 1.1 of its time where tiles fill the chip); what is gained is
-// that its rows need not exist: at 2,048 rows of 12,288 gates of 4,096 columns 100 MB that are written and read again, 30 us beside 280.
-// us, the library's product and the gate's kernel before, and this one: 2,048 x 12288 of 4,096 columns 311, 284; 1,866 rows 300, 276;
+// The product alone is no faster than the vendor's library's (0.96 to 1.1 of its time where tiles fill the chip); what is gained is that its rows need not exist:
+// at 2,048 rows of 12,288 gates of 4,096 columns 100 MB that are written and read again, 30 us of 311. The library's product with the gate's
+// kernel behind it, and this one, us: 2,048 x 12288 of 4,096 columns 311, 284; 1,866 rows 300, 276;
 // 2,048 x 9728 of 2,560 214, 173; x 6144 of 2,048 104, 93; x 3072 of 1,024 37.6, 27.9; x 17408 of 5,120 618, 545; 8,192 x 12288 of 4,096
-// 1,157, 1,093; activated, 1,925 x 6144 of 2,048 57.7, 48.3.
+// 1,157, 1,093; activated, 1,925 x 6144 of 2,048 57.7, 48.3. (Gates are taken of float sums so, not of sums rounded to bfloat16.)
 //
 // A block is 8 waves, 2 x 4, and has 256 rows of x by 256 of w, a wave 128 by 64. The more both are, the less comes in for a
-// product: at this size a compute unit takes in 64 KB for 1,024 matrix instructions, 45 bytes a ns, which the L2s give. Both
+// product: at this size a compute unit takes in 64 KB for 512 matrix instructions, 45 bytes a ns, which the L2s give. Both
 // operands go through LDS in pieces of 64 columns (whole lines of the caches), two pieces of 64 KB; a piece is four units, and a
 // unit's place is loaded again as soon as every wave has read it, so that six of the eight units that fit are always under way:
 // loads arrive 1.5 pieces after they are asked for (with whole pieces, one after they are asked for, 323 us for the 284). A

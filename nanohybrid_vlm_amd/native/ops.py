@@ -997,8 +997,8 @@ class NativeBackend:
 
     def gated_linear(self, x, w, out, gate=None, bias=None) -> bool:
         """A gate (a ``Gate``; None: SiLU) of x Wg^T and x Wu^T (+ bias) in one kernel, if this batch is one for the
-        few-rows kernel, the one for up to 96 rows or the one for many; else False. (SiLU without bias may also be one for the kernel of up to 64 rows; in
-        float32 most batches are.)"""
+        few-rows kernel, the one for up to 96 rows or the one for many; else False. (SiLU without bias may also be one for the kernel of up to 64
+        rows; in float32 most batches are.)"""
         M, K = x.shape
         if x.dtype == torch.float32:
             if not self.lib.nhv_gemm_float32_gated_pays(_ptr(x), _ptr(w), M, out.shape[1], K):
@@ -1604,8 +1604,8 @@ def gate_of(activation) -> Gate:
 
 def gated_linear(x, w: torch.Tensor, activation="silu", bias: torch.Tensor | None = None) -> torch.Tensor:
     """A gate (``gate_of(activation)``) of x . w[:I]^T + bias[:I] and x . w[I:]^T + bias[I:] for a packed gate | up matrix
-    w[2 I, K]: fused into one kernel for few rows, else the matrix product followed by ``act_mul``. ``x`` may be a
-    ``Normed`` (see ``linear``)."""
+    w[2 I, K]: fused into one kernel for few rows, in float32 for most, and for many in bfloat16 where that is the faster way (the gate is then taken of
+    sums that were not rounded to bfloat16), else the matrix product followed by ``act_mul``. ``x`` may be a ``Normed`` (see ``linear``)."""
     gate = gate_of(activation)
     plain = gate.act == 0 and bias is None
     normed = x if isinstance(x, Normed) else None
@@ -2525,9 +2525,9 @@ def activation_(x: torch.Tensor, activation: str) -> torch.Tensor:
 
 
 def activated_linear(x: torch.Tensor, w: torch.Tensor, activation: str) -> torch.Tensor:
-    """act(x . w^T) without a gate and without bias: one kernel for few rows in bfloat16, else the matrix product
+    """act(x . w^T) without a gate and without bias: one kernel for few rows in bfloat16, and for many where that is the faster way, else the matrix product
     followed by ``activation_``. Either way the activation is taken in float and the result rounded once more than the
-    product alone (the fused kernel rounds once in all)."""
+    product alone (the fused kernels round once in all)."""
     _need(activation in PLAIN_ACTIVATIONS, lambda: f"activated_linear: {activation!r} is not known ({sorted(PLAIN_ACTIVATIONS)} are)")
     _need(x.dim() == 2 and w.dim() == 2 and x.shape[1] == w.shape[1],
           lambda: f"activated_linear: x {tuple(x.shape)} and w {tuple(w.shape)} do not fit")
