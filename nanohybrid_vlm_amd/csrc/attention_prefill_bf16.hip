@@ -598,7 +598,7 @@ static long long groups_of_tiles(int max_q_len, int G, bool two) {
 // them, gx to a request's. So: where the other way takes several blocks of all keys (G of 8 and more), or has two row tiles a wave and two waves
 // without any (53 and 53 where blocks meet, else 0.5 to 0.9), or where few blocks are spread over many units, heads of their own few blocks apart (G of 1: 5 tokens after 1,700 beside 500,
 // gx 8, 28.6 and 36.0). Measured over 2,500 sizes (1 to 200 tokens of heads of 64 and 128, groups of 1 to 16, after 17 to 30,000 keys beside 20 to 1,000 new ones): time over the other way's
-// 0.84 on average, the worst 1.03; taken everywhere 0.84, 1.26.
+// 0.85 on average, the worst 1.02; taken everywhere beyond 256 keys 0.83, 1.28.
 // Up to 448 keys groups of less than 4 gain nothing (1 to 25 tokens after 280 to 400: 0.96 to 1.1), and up to 256 larger ones at most 0.7 us (1 token after
 // 128: 6.3 and 6.4; 256: 7.6 and 7.2; groups of 8 of 64 6.1 and 5.4): there a token's sums keep the portions' order, so that a short
 // request's results hang less on how it is cut up (logits of sharpened scores 0.0190 apart, with the waves' sums 0.0204). Neither is further from 64

@@ -15,7 +15,7 @@
 // wave reads the next quarter's operands while it multiplies this one's. Of LDS' 128 bytes a clock the reads take 96 and the
 // loads 32, as long as the matrix instructions take. A block takes tile after tile (as many blocks as there are units), and the last quarters of one
 // ask for the first pieces of the next.
-// What bounds it is power: the matrix instructions take 74 % of the clocks, at 1.94 of 2.4 GHz (the library's 77 % at 1.93); of
+// What bounds it is power: the matrix instructions take 74 % of the clocks, at 1.82 to 1.94 of 2.4 GHz (the library's 77 % at 1.93 or 82 % at 1.69); of
 // zeros it is 222 us. That is why they are 16x16x32 ones: alone they run at 1,950 TFLOP/s, those of 32x32x16 at 1,720.
 // Measured and not kept: four waves of 128 x 128 (369 us; accumulators move between register files), a barrier a quarter (the same), loads
 // asked for at other places among the matrix instructions (the same), blocks at columns of their own (the same or up to 10 % more).
