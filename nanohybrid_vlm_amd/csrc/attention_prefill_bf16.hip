@@ -67,9 +67,10 @@ constexpr bool CH_POW2 = (CH & (CH - 1)) == 0;
 constexpr int KSWZ = CH_POW2 ? (CH < 16 ? CH : 16) - 1 : 0;
 // and at c ^ ((k & VSWZ) << 1) in the V tile, whose transposed reads take 32 bytes of 8 keys at once
 constexpr int VSWZ = CH_POW2 && CH >= 4 ? (CH / 2 < 8 ? CH / 2 : 8) - 1 : 0;
-// Requests whose rows are one tile get a path of their own (its tiles fit into that LDS). Not of heads of 80 and 96: of them three blocks share a unit, with 168
-// registers a wave, of which that path takes 200 (20 portions of 100 tokens, 16 on 4 heads of 80, 9.9 us, with two blocks 11.7; 2,000 tokens after 4,000, 24 on 8 of 96,
-// 143 and 174; with what is beyond 168 in memory the compiler also moves the portions' own).
+// Requests whose rows are one tile get a path of their own (its tiles fit into that LDS). Not of heads of 80 and 96: of them three blocks
+// share a unit, with 168 registers a wave, of which that path takes 200 (20 portions of 100 tokens, 16 on 4 heads of 80, 9.9 us, with two
+// blocks 11.7; 2,000 tokens after 4,000, 24 on 8 of 96, 143 and 174; with what is beyond 168 in memory the compiler also moves the
+// portions' own).
 constexpr bool ONE_TILE = D <= 64 || (D >= 112 && D <= 128);
 constexpr int MAX_RT = D <= 128 ? 2 : 1;    // row tiles per wave (template argument RT): all of them use every key and value
                                             // that the wave reads from LDS; two need the registers of head sizes up to 128
@@ -254,8 +255,9 @@ __device__ __forceinline__ void attend(Rows<RT>& w, int kb, KeyOperand key_opera
 // exp2 that overflows gives the limit 1; sink_l2 = sink log2(e), or -inf for none (sinks, may be null: one per head in
 // its place); gate (may be null). BIASED: slopes per head, slope_ratio = 1 / scale.
 //
-// Blocks a compute unit, four waves each, that the compiler is to leave registers for: as many as the tiles in LDS leave room for, where the portions' way
-// has no use for more (heads of 64, one row tile a wave: 125 of 128; left at two blocks it takes 130 to 140, for the one-tile path).
+// Blocks a compute unit, four waves each, that the compiler is to leave registers for: as many as the tiles in LDS leave room for, where
+// the portions' way has no use for more (heads of 64, one row tile a wave: 125 of 128; left at two blocks it takes 130 to 140, for the
+// one-tile path).
 template <int RT, bool PLAIN>
 constexpr int blocks_a_unit() { return RT == 1 && D <= 64 && PLAIN ? 4 : D <= 48 && PLAIN ? 3 : 2; }
 
@@ -593,16 +595,18 @@ static long long groups_of_tiles(int max_q_len, int G, bool two) {
 }
 
 // Beyond how many keys a request whose rows are one tile shares its keys out among the waves, where that is the faster way. Where two of
-// its blocks come to one unit it is not: loads of keys as operands touch sixteen rows at a time, of which a unit takes in less a ns (13 tokens after 1,700 keys of 32 on 8 heads
-// beside 50 new ones, 104 blocks on 64 units: 45 us, 53 so; with a unit each 39 and 32). Which units the blocks come to hangs on the empty ones between
-// them, gx to a request's. So: where the other way takes several blocks of all keys (G of 8 and more), or has two row tiles a wave and two waves
-// without any (53 and 53 where blocks meet, else 0.5 to 0.9), or where few blocks are spread over many units, heads of their own few blocks apart (G of 1: 5 tokens after 1,700 beside 500,
-// gx 8, 28.6 and 36.0). Measured over 2,500 sizes (1 to 200 tokens of heads of 64 and 128, groups of 1 to 16, after 17 to 30,000 keys beside 20 to 1,000 new ones): time over the other way's
-// 0.85 on average, the worst 1.02; taken everywhere beyond 256 keys 0.83, 1.28.
-// Up to 448 keys groups of less than 4 gain nothing (1 to 25 tokens after 280 to 400: 0.96 to 1.1), and up to 256 larger ones at most 0.7 us (1 token after
-// 128: 6.3 and 6.4; 256: 7.6 and 7.2; groups of 8 of 64 6.1 and 5.4): there a token's sums keep the portions' order, so that a short
-// request's results hang less on how it is cut up (logits of sharpened scores 0.0190 apart, with the waves' sums 0.0204). Neither is further from 64
-// bits: 0.0016 to 0.0024 of the results' size after 64 to 2,000 keys, the waves' sums up to a fifth closer at the fewest, the same at the most.
+// its blocks come to one unit it is not: loads of keys as operands touch sixteen rows at a time, of which a unit takes in less a ns (13
+// tokens after 1,700 keys of 32 on 8 heads beside 50 new ones, 104 blocks on 64 units: 45 us, 53 so; with a unit each 39 and 32). Which
+// units the blocks come to hangs on the empty ones between them, gx to a request's. So: where the other way takes several blocks of all
+// keys (G of 8 and more), or has two row tiles a wave and two waves without any (53 and 53 where blocks meet, else 0.5 to 0.9), or where
+// there are few blocks for the units (up to 64; of groups of less than 4 heads only with up to 4 blocks to a request, since with G of 1 and
+// gx of 8 they meet all the same: 5 tokens after 1,700 beside 500 28.6 and 36.0). Measured over 2,500 sizes (1 to 200 tokens of heads of 64
+// and 128, groups of 1 to 16, after 17 to 30,000 keys beside 20 to 1,000 new ones): time over the other way's 0.85 on average, the worst
+// 1.02; taken everywhere beyond 256 keys 0.83, 1.28. Up to 448 keys groups of less than 4 gain nothing (1 to 25 tokens after 280 to 400:
+// 0.96 to 1.1), and up to 256 larger ones at most 0.7 us (1 token after 128: 6.3 and 6.4; 256: 7.6 and 7.2; groups of 8 of 64 6.1 and 5.4):
+// there a token's sums keep the portions' order, so that a short request's results hang less on how it is cut up (logits of sharpened
+// scores 0.0190 apart, with the waves' sums 0.0204). Neither is further from 64 bits: 0.0016 to 0.0024 of the results' size after 64 to
+// 2,000 keys, the waves' sums up to a fifth closer at the fewest, the same at the most.
 static int one_tile_from_keys(int B, int G, int Hkv, bool two, long long gx) {
   if (!(G >= 8 || (two && G >= 4) || ((long long)B * Hkv <= 64 && (G >= 4 || gx <= 4)))) return 0x7fffffff;
   return G >= 4 ? 256 : 448;

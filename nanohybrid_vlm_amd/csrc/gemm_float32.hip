@@ -661,12 +661,12 @@ static Choice gated_tile(long long M, long long N, bool whole) {
   return best;
 }
 
-// Whether tiles of 128 x 128 rows of x and of w (gated: 64 outputs) are the faster ones: where tiles of 64 x 128 need twice the rounds of 256
-// blocks that these do. Measured over 9,700 sizes (90 to 2,048 rows, 700 to 8,200 outputs of 256 to 4,096
-// columns; time over that of the choice without them): 1 round 0.86 and 0.88 gated, the worst 1.01 and 1.03; 2 rounds 0.87 and 0.91,
-// 1.01; 3 0.89 and 0.91, 1.0; 4 and more 0.92, 1.08. Elsewhere 0.9 to 1.57 (2 rounds where the others need 2).
-// A second round of smaller ones that is hardly begun is little to save: of 257 to 300 blocks up to 1.17. And of few columns a tile's first pieces and its
-// sums are most of its time: 192 columns 0.97, 224 0.89, but 128 1.05, the worst 1.07 (1,004 x 2,592 12.2, 13.1 us).
+// Whether tiles of 128 x 128 rows of x and of w (gated: 64 outputs) are the faster ones: where tiles of 64 x 128 need twice the rounds of
+// 256 blocks that these do. Measured over 9,700 sizes (90 to 2,048 rows, 700 to 8,200 outputs of 256 to 4,096 columns; time over that of
+// the choice without them): 1 round 0.86 and 0.88 gated, the worst 1.01 and 1.03; 2 rounds 0.87 and 0.91, 1.01; 3 0.89 and 0.91, 1.0; 4 and
+// more 0.92, 1.08. Elsewhere 0.9 to 1.57 (2 rounds where the others need 2). A second round of smaller ones that is hardly begun is little
+// to save: of 257 to 300 blocks up to 1.17. And of few columns a tile's first pieces and its sums are most of its time: 192 columns 0.97,
+// 224 0.89, but 128 1.05, the worst 1.07 (1,004 x 2,592 12.2, 13.1 us).
 constexpr int BEGUN = 44, BIG_COLUMNS = 192;
 static bool big_tiles(long long M, long long N, int K, bool whole, bool gated) {
   const long long columns = gated ? 64 : 128, n = (N + columns - 1) / columns, blocks = (M + 127) / 128 * n, smaller = (M + 63) / 64 * n;

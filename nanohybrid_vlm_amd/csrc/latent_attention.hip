@@ -613,13 +613,13 @@ __global__ __launch_bounds__(256) void head_gemm_tile_kernel(const bf16_t* __res
   }
 }
 
-// The same where outputs are pieces of 16 bytes and the matrix nearly fills its tiles, or blocks are many (nhv_head_gemm_rows_pays). Bound by the bytes of x, y and the gate: a wave owns
-// 16 rows of one head, whose entries it holds as operands, and the head's matrix comes into LDS once a block (up to 64 KB at a time), as operands in
-// the order in which they are read. Two tiles of 16 outputs are 32 outputs side by side: tile t's line i is output
-// 8 (i / 4) + 4 t + i % 4, so that a lane ends up with eight outputs in a row and writes (and reads the gate) in pieces of
-// 16 bytes, with nothing but the matrix behind a barrier. 4,220 rows of 16 heads: 128 to 192 entries and 64 turned, 44 us as
-// blocks of 64 rows that walk over the outputs with the rows in LDS and the matrix from memory, 24 so; 192 to 128 with a gate
-// per entry 32 and 23 (these bytes at 5 TB/s: 12). Blocks of 4, 8 and 16 waves 27, 25 and 24.
+// The same where outputs are pieces of 16 bytes and the matrix nearly fills its tiles, or blocks are many (nhv_head_gemm_rows_pays). Bound
+// by the bytes of x, y and the gate: a wave owns 16 rows of one head, whose entries it holds as operands, and the head's matrix comes into
+// LDS once a block (up to 64 KB at a time), as operands in the order in which they are read. Two tiles of 16 outputs are 32 outputs side by
+// side: tile t's line i is output 8 (i / 4) + 4 t + i % 4, so that a lane ends up with eight outputs in a row and writes (and reads the
+// gate) in pieces of 16 bytes, with nothing but the matrix behind a barrier. 4,220 rows of 16 heads: 128 to 192 entries and 64 turned, 44
+// us as blocks of 64 rows that walk over the outputs with the rows in LDS and the matrix from memory, 24 so; 192 to 128 with a gate per
+// entry 32 and 23 (these bytes at 5 TB/s: 12). Blocks of 4, 8 and 16 waves 27, 25 and 24.
 #define HT_LDS 65536
 template <int KS, int WAVES>
 __global__ __launch_bounds__(64 * WAVES) void head_gemm_rows_kernel(const bf16_t* __restrict__ x, long long xs_t, long long xs_h,
@@ -713,11 +713,12 @@ __global__ __launch_bounds__(64 * WAVES) void head_gemm_rows_kernel(const bf16_t
   }
 }
 
-// Whether the matrix in LDS is the faster way for outputs in pieces of 16 bytes: of many blocks of 64 rows, or where at most a sixth of its tiles' products (64 outputs
-// by 128, 192, 256 or 512 entries) are for nothing, or heads are small. Measured over 845 such sizes (1 to 128 heads of 8 to 750 outputs of 8 to 512 entries, 65 to
-// 6,000 rows; time over the other way's): blocks from 700 on 0.65 on average, fewer and full tiles 0.90, small heads 0.84, the worst 1.07 (200 rows of 64 heads, 512 outputs
-// of 512 entries 38.1, 40.6 us); others 1.07, up to 1.24 (5 heads of 368 outputs of 288 entries 19.0, 23.3). Outputs of other lengths, or that begin elsewhere, can only
-// be stored entry by entry so: 321 sizes 1.03, up to 2.05 (2,038 rows of 16 heads, 64 to 300 entries, 22 us, 44).
+// Whether the matrix in LDS is the faster way for outputs in pieces of 16 bytes: of many blocks of 64 rows, or where at most a sixth of its
+// tiles' products (64 outputs by 128, 192, 256 or 512 entries) are for nothing, or heads are small. Measured over 845 such sizes (1 to 128
+// heads of 8 to 750 outputs of 8 to 512 entries, 65 to 6,000 rows; time over the other way's): blocks from 700 on 0.65 on average, fewer
+// and full tiles 0.90, small heads 0.84, the worst 1.07 (200 rows of 64 heads, 512 outputs of 512 entries 38.1, 40.6 us); others 1.07, up
+// to 1.24 (5 heads of 368 outputs of 288 entries 19.0, 23.3). Outputs of other lengths, or that begin elsewhere, can only be stored entry
+// by entry so: 321 sizes 1.03, up to 2.05 (2,038 rows of 16 heads, 64 to 300 entries, 22 us, 44).
 extern "C" int nhv_head_gemm_rows_pays(int rows, int H, int N, int K) {
   if (rows <= 64 || H <= 0 || N <= 0 || N % 8 || K <= 0 || K > HT_MAX_K) return 0;
   const long long blocks = (long long)H * ((rows + 63) / 64), tiles = (N + 63) / 64 * 64ll * (K <= 128 ? 128 : K <= 192 ? 192 : K <= 256 ? 256 : 512);

@@ -327,13 +327,14 @@ struct ChunkOperands {
   float a;
 };
 
-// What bounds it is the way to a chunk's operands, for which few chains wait at a time. Loads are whole kilobytes in the preparation's order, places go on by
-// additions, results are stored without a branch. us before and now, 16 heads of 128: 16 portions of 20 to 200 60, 48; 24 of 100 to 160 92, 72; 3 of 900 to 1,300 107, 90;
-// one of 3,000 137, 124. Of heads of 256 several long chains have gained nothing, and why they take longer is not known (1 head of 6,000 tokens with the preparation 435, 433;
-// 4 482, 488; 12 653, 697; 12 of 1,000 126, 138; 24 portions of 80, 12 heads, 240, 225).
-// AHEAD 2 leaves room for three waves a SIMD, AHEAD 3 for two (at least: with at most 256 registers a wave the products' sums stay in
-// ordinary registers); tiles of more than 32 rows a wave have room for 2 and two. Where there are more blocks than two a compute unit the third
-// counts for more, else the third chunk: 16 portions of 20 to 200 52, 48 us, 24 of 100 to 160 77, 72; 3 of 900 to 1,300 89, 91, one of 3,000 125, 130.
+// What bounds it is the way to a chunk's operands, for which few chains wait at a time. Loads are whole kilobytes in the preparation's
+// order, places go on by additions, results are stored without a branch. us before and now, 16 heads of 128: 16 portions of 20 to 200 60,
+// 48; 24 of 100 to 160 92, 72; 3 of 900 to 1,300 107, 90; one of 3,000 137, 124. Of heads of 256 several long chains have gained nothing,
+// and why they take longer is not known (1 head of 6,000 tokens with the preparation 435, 433; 4 482, 488; 12 653, 697; 12 of 1,000 126,
+// 138; 24 portions of 80, 12 heads, 240, 225). AHEAD 2 leaves room for three waves a SIMD, AHEAD 3 for two (at least: with at most 256
+// registers a wave the products' sums stay in ordinary registers); tiles of more than 32 rows a wave have room for 2 and two. Where there
+// are more blocks than two a compute unit the third counts for more, else the third chunk: 16 portions of 20 to 200 52, 48 us, 24 of 100 to
+// 160 77, 72; 3 of 900 to 1,300 89, 91, one of 3,000 125, 130.
 template <typename T, int TPW, bool EVEN, int AHEAD>
 __global__ __launch_bounds__(256, TPW <= 2 && AHEAD == 2 ? 3 : 2) void recurrence_chunks_kernel(const float* __restrict__ r_in, const float* __restrict__ k_in,
                                                                 const float* __restrict__ a_in, const float* __restrict__ decay_in,

@@ -60,10 +60,11 @@ __device__ __forceinline__ void store_entries(V* p, const float* in) {
   else *reinterpret_cast<float4*>(p) = make_float4(in[0], in[1], in[2], in[3]);
 }
 
-// Row ids[t] of a table times scale, as TO, by the whole block, eight entries a thread at a time (H a multiple of 8, table and rows 16 bytes aligned), in pieces of
-// 16 bytes of the result, neighbours' side by side: what a wave stores is in a row. (Eight floats a thread side by side: 2,048 rows of 4,096 floats 12.0 us, so 10.7,
-// entry by entry 11.4.) An id out of range gives a row of zeros. One trip to memory after the id's; entry by entry, a row of 4,096 in bfloat16 takes 256 threads 16
-// trips: 8 rows 8.9 us, so 3.8, 2,048 rows 16.6 and 11.5; 16 rows of 2,048 as floats 7.3 and 3.1.
+// Row ids[t] of a table times scale, as TO, by the whole block, eight entries a thread at a time (H a multiple of 8, table and rows 16
+// bytes aligned), in pieces of 16 bytes of the result, neighbours' side by side: what a wave stores is in a row. (Eight floats a thread
+// side by side: 2,048 rows of 4,096 floats 12.0 us, so 10.7, entry by entry 11.4.) An id out of range gives a row of zeros. One trip to
+// memory after the id's; entry by entry, a row of 4,096 in bfloat16 takes 256 threads 16 trips: 8 rows 8.9 us, so 3.8, 2,048 rows 16.6 and
+// 11.5; 16 rows of 2,048 as floats 7.3 and 3.1.
 template <typename T, typename TO>
 __device__ __forceinline__ void embed_row(const int* ids, const T* table, TO* out, int H, int V, float scale) {
   constexpr int E = 16 / sizeof(TO), P = 8 / E;

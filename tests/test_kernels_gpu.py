@@ -441,7 +441,8 @@ def test_float32_linear_in_all_its_tiles(ops, N, K):
         last = y
 
 
-@pytest.mark.parametrize("M,N,K,taken", [(300, 8000, 192, 1), (300, 7970, 224, 1), (417, 6144, 544, 1), (517, 6100, 288, 1), (517, 6144, 1024, 1), (577, 4130, 256, 1),
+@pytest.mark.parametrize("M,N,K,taken", [(300, 8000, 192, 1), (300, 7970, 224, 1), (417, 6144, 544, 1), (517, 6100, 288, 1),
+                                         (517, 6144, 1024, 1), (577, 4130, 256, 1),
                                          (1000, 6268, 352, 1), (1049, 3072, 1056, 1), (1100, 14400, 256, 1), (128, 20000, 256, 1),
                                          (300, 8000, 160, 0), (517, 7168, 288, 0), (300, 8000, 1200, 0), (545, 4130, 256, 0), (150, 2000, 256, 0)])
 def test_float32_linear_in_tiles_of_128_rows(ops, M, N, K, taken):
